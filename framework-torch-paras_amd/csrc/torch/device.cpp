@@ -4,8 +4,10 @@
 // 34-95, csrc/core/allocator.cpp:129-173) on top of the HIP-only context:
 // device i is HIP device i, one context stream per device (stream id 0), the
 // allocator hands out blocks of the binned HBM pool.
+#include <ATen/EmptyTensor.h>
 #include <ATen/detail/PrivateUse1HooksInterface.h>
 #include <c10/core/Allocator.h>
+#include <c10/core/DeviceGuard.h>
 #include <c10/core/impl/DeviceGuardImplInterface.h>
 #include <torch/version.h>
 
@@ -121,11 +123,15 @@ void* stream_for(c10::DeviceIndex index) {
 }
 
 at::Tensor empty_paras(c10::IntArrayRef sizes, c10::ScalarType dtype, c10::Device device) {
-    return at::empty(sizes, at::TensorOptions().dtype(dtype).device(device));
+    const c10::DeviceIndex prev = tl_device;        // the allocator serves the thread's current device
+    if (prev == device.index())
+        return at::detail::empty_generic(sizes, &g_allocator, c10::DispatchKeySet(c10::DispatchKey::PrivateUse1), dtype, std::nullopt);
+    const c10::DeviceGuard guard(device);
+    return at::detail::empty_generic(sizes, &g_allocator, c10::DispatchKeySet(c10::DispatchKey::PrivateUse1), dtype, std::nullopt);
 }
 
 at::Tensor workspace(size_t nbytes, c10::Device device) {
-    return at::empty({static_cast<int64_t>(nbytes > 0 ? nbytes : 1)}, at::TensorOptions().dtype(c10::kByte).device(device));
+    return empty_paras({static_cast<int64_t>(nbytes > 0 ? nbytes : 1)}, c10::kByte, device);
 }
 
 double narrow_scalar(double v, c10::ScalarType dtype) {

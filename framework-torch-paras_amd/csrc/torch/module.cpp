@@ -1,6 +1,7 @@
 // Python extension module `_C`: thin bindings over the C ABI, same function
 // names as the reference's module (csrc/python/module.cpp:30-78).
 #include <pybind11/pybind11.h>
+#include <torch/csrc/utils/pybind.h>
 
 #include <string>
 
@@ -61,6 +62,12 @@ PYBIND11_MODULE(_C, m) {
         check(paras_memory_stats(hip_device(index), &a, &c));
         return c;
     });
+    // what torch_paras.nn calls (differentiable)
+    const py::call_guard<py::gil_scoped_release> no_gil;
+    m.def("nn_rms_norm", &paras_torch::nn_rms_norm, no_gil);
+    m.def("nn_swiglu", &paras_torch::nn_swiglu, no_gil);
+    m.def("nn_rotate_half", &paras_torch::nn_rotate_half, no_gil);
+    m.def("nn_moe_layer", &paras_torch::nn_moe_layer, no_gil);
     m.def("is_bad_fork", [] { return paras_is_bad_fork() != 0; });
     m.def("abi_version", [] { return paras_abi_version(); });
 }

@@ -11,6 +11,8 @@
 //    _fused_sdp_choice: no weights are returned, so the MFMA flash / split-KV
 //    decode kernels serve every shape they accept (anything else still goes to
 //    the math-semantics kernel inside libparas_hip.so).
+#include <ATen/NativeFunctions.h>
+#include <ATen/TensorSubclassLikeUtils.h>
 #include <ATen/native/DispatchStub.h>
 #include <ATen/native/transformers/attention.h>
 #include <ATen/native/transformers/sdp_utils_cpp.h>
@@ -54,6 +56,7 @@ void prepare(const Tensor& query, const Tensor& key, const Tensor& value, const 
     auto to4 = [](const Tensor& t, c10::IntArrayRef lead) {
         std::vector<int64_t> full(lead.begin(), lead.end());
         full.insert(full.end(), t.sizes().end() - 3, t.sizes().end());
+        if (lead.size() == 1 && t.dim() == 4 && t.size(0) == lead[0]) return t;
         Tensor e = t.expand(full);
         int64_t batch = 1;                       // (spelled out: -1 cannot be inferred for an empty tensor)
         for (int64_t d : lead) batch *= d;
@@ -212,6 +215,32 @@ int64_t fused_sdp_choice(const Tensor& query, const Tensor& key, const Tensor& v
     return static_cast<int64_t>(fused ? sdp::SDPBackend::overrideable : sdp::SDPBackend::math);
 }
 
+// aten::scaled_dot_product_attention itself, registered above autograd.  What the composite would do
+// for an inference call on this device is turn a boolean mask into an additive one (zeros, logical_not,
+// masked_fill: none of them device ops here, so the mask crosses to the host and back, 90 us of a 98 us
+// call), ask fused_sdp_choice, and have the fused op fill nine results of which one is used.  The kernels
+// read a boolean mask as it is, so a call that would end in the fused op goes straight to them; anything
+// else -- gradients, dropout, operands the composite would refuse or convert -- is left to it.
+Tensor sdpa(const Tensor& query, const Tensor& key, const Tensor& value, const c10::optional<Tensor>& attn_mask, double dropout_p,
+            bool is_causal, c10::optional<double> scale, bool enable_gqa) {
+    const bool has_mask = attn_mask.has_value() && attn_mask->defined();
+    auto alike = [&](const Tensor& t) {
+        return is_paras(t) && t.device() == query.device() && t.scalar_type() == query.scalar_type() && t.dim() == query.dim() &&
+               !at::isTensorSubclassLike(t);
+    };
+    bool direct = dropout_p == 0.0 && query.dim() >= 3 && float_code(query.scalar_type()) >= 0 && alike(query) && alike(key) && alike(value) &&
+                  !needs_grad(query, key, value) && (enable_gqa || key.size(-3) == query.size(-3) || key.size(-3) == 1);
+    if (has_mask)
+        direct = direct && !is_causal && is_paras(*attn_mask) && attn_mask->device() == query.device() && !needs_grad(*attn_mask) &&
+                 attn_mask->dim() >= 2 && (attn_mask->scalar_type() == c10::kBool || attn_mask->scalar_type() == query.scalar_type());
+    if (!direct) return at::native::scaled_dot_product_attention(query, key, value, attn_mask, dropout_p, is_causal, scale, enable_gqa);
+    Prepared p;
+    prepare(query, key, value, attn_mask, is_causal, scale, /*enable_gqa=*/true, &p);
+    Tensor out;
+    run(&p, &out, nullptr, nullptr);
+    return out.sizes().equals(p.out_shape) ? out : out.reshape(p.out_shape);
+}
+
 }  // namespace
 }  // namespace paras_torch
 
@@ -222,4 +251,6 @@ REGISTER_PRIVATEUSE1_DISPATCH(_fused_sdp_choice_stub, &paras_torch::fused_sdp_ch
 TORCH_LIBRARY_IMPL(aten, PrivateUse1, m) {
     m.impl("aten::_scaled_dot_product_attention_math", &paras_torch::sdpa_math);
     m.impl("aten::_scaled_dot_product_fused_attention_overrideable", &paras_torch::sdpa_overrideable);
+    m.impl("aten::scaled_dot_product_attention", &paras_torch::sdpa);
 }
+TORCH_LIBRARY_IMPL(aten, AutogradPrivateUse1, m) { m.impl("aten::scaled_dot_product_attention", &paras_torch::sdpa); }

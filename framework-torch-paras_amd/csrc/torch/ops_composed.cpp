@@ -32,7 +32,7 @@ Tensor rms_norm(const Tensor& input, c10::IntArrayRef normalized_shape, const c1
     const bool fused_w = has_w && weight->scalar_type() == in.scalar_type();
     Tensor w;
     if (fused_w) w = weight->contiguous();
-    Tensor out = at::empty_like(in);
+    Tensor out = empty_paras_like(in);
     const int64_t rows = H > 0 ? in.numel() / H : 0;
     if (rows > 0 && H > 0)
         check(paras_rms_norm_composed_fwd(in.data_ptr(), fused_w ? w.data_ptr() : nullptr, out.data_ptr(), rows, H,
@@ -47,7 +47,7 @@ Tensor swiglu_device(const Tensor& x, const Tensor& gate) {
     require_same_device("paras swiglu", x, {{"gate", &gate}});
     auto shape = at::infer_size(x.sizes(), gate.sizes());
     Tensor xe = x.expand(shape).contiguous(), ge = gate.expand(shape).contiguous();
-    Tensor out = at::empty_like(xe);
+    Tensor out = empty_paras_like(xe);
     if (out.numel() == 0) return out;
     check(paras_swiglu_composed_fwd(xe.data_ptr(), ge.data_ptr(), out.data_ptr(), out.numel(),
                                     require_float_code(xe, "paras swiglu"), stream_for(xe)));

@@ -5,6 +5,8 @@
 // device pointers to libparas_hip.so.
 #include "paras_torch.h"
 
+#include <torch/csrc/autograd/custom_function.h>
+
 namespace paras_torch {
 namespace {
 
@@ -20,8 +22,8 @@ std::tuple<Tensor, Tensor> rms_norm(const Tensor& input, const Tensor& weight, d
     const int64_t rows = H > 0 ? in.numel() / H : 0;
     TORCH_CHECK(w.numel() == H, "paras rms_norm: weight size must match the last dimension");
     TORCH_CHECK(w.scalar_type() == in.scalar_type(), "paras rms_norm: weight dtype must match input dtype");
-    Tensor out = at::empty_like(in);
-    Tensor rstd = at::empty({rows}, in.options().dtype(c10::kFloat));
+    Tensor out = empty_paras_like(in);
+    Tensor rstd = empty_paras({rows}, c10::kFloat, in.device());
     if (rows == 0 || H == 0) return {out, rstd};
     check(paras_rms_norm_fwd(in.data_ptr(), w.data_ptr(), out.data_ptr(), rstd.data_ptr<float>(), rows, H, eps,
                              require_float_code(in, "paras rms_norm"), stream_for(in)));
@@ -38,9 +40,9 @@ std::tuple<Tensor, Tensor> rms_norm_backward(const Tensor& grad_out, const Tenso
     const int64_t rows = H > 0 ? in.numel() / H : 0;
     TORCH_CHECK(go.numel() == in.numel() && w.numel() == H && rs.numel() == rows && rs.scalar_type() == c10::kFloat,
                 "paras rms_norm_backward: shape mismatch");
-    Tensor grad_input = at::empty_like(in);
-    Tensor grad_weight = at::zeros({H}, w.options());
-    if (rows == 0 || H == 0) return {grad_input, grad_weight};
+    Tensor grad_input = empty_paras_like(in);
+    if (rows == 0 || H == 0) return {grad_input, at::zeros({H}, w.options())};
+    Tensor grad_weight = empty_paras({H}, w.scalar_type(), w.device());       // written whole by the kernels
     Tensor ws = workspace(paras_rms_norm_bwd_workspace(rows, H), in.device());
     check(paras_rms_norm_bwd(go.data_ptr(), in.data_ptr(), w.data_ptr(), rs.data_ptr<float>(), grad_input.data_ptr(),
                              grad_weight.data_ptr(), ws.data_ptr(), rows, H, require_float_code(in, "paras rms_norm_backward"),
@@ -54,7 +56,7 @@ Tensor swiglu(const Tensor& gate, const Tensor& up) {
     TORCH_CHECK(gate.scalar_type() == up.scalar_type(), "paras swiglu: gate and up must have the same dtype");
     require_same_device("paras swiglu", gate, {{"up", &up}});
     Tensor g = gate.contiguous(), u = up.contiguous();
-    Tensor out = at::empty_like(g);
+    Tensor out = empty_paras_like(g);
     if (out.numel() == 0) return out;
     check(paras_swiglu_fwd(g.data_ptr(), u.data_ptr(), out.data_ptr(), out.numel(), require_float_code(g, "paras swiglu"),
                            stream_for(g)));
@@ -66,7 +68,7 @@ std::tuple<Tensor, Tensor> swiglu_backward(const Tensor& grad_out, const Tensor&
     require_same_dtype("paras swiglu_backward", grad_out, {{"gate", &gate}, {"up", &up}});
     Tensor go = grad_out.contiguous(), g = gate.contiguous(), u = up.contiguous();
     TORCH_CHECK(go.numel() == g.numel() && g.numel() == u.numel(), "paras swiglu_backward: shape mismatch");
-    Tensor grad_gate = at::empty_like(g), grad_up = at::empty_like(u);
+    Tensor grad_gate = empty_paras_like(g), grad_up = empty_paras_like(u);
     if (go.numel() == 0) return {grad_gate, grad_up};
     check(paras_swiglu_bwd(go.data_ptr(), g.data_ptr(), u.data_ptr(), grad_gate.data_ptr(), grad_up.data_ptr(), go.numel(),
                            require_float_code(go, "paras swiglu_backward"), stream_for(go)));
@@ -80,7 +82,7 @@ Tensor rotate_half_impl(const Tensor& x, bool backward, const char* name) {
     const int64_t D = x.size(-1);
     TORCH_CHECK(D % 2 == 0, "paras ", name, ": last dimension must be even");
     Tensor in = x.contiguous();
-    Tensor out = at::empty_like(in);
+    Tensor out = empty_paras_like(in);
     if (out.numel() == 0) return out;
     check(paras_rotate_half(in.data_ptr(), out.data_ptr(), in.numel() / D, D, backward ? 1 : 0,
                             require_float_code(in, name), stream_for(in)));
@@ -97,10 +99,10 @@ std::tuple<Tensor, Tensor, Tensor, Tensor, Tensor, Tensor> moe_route(const Tenso
     const int64_t T = lg.size(0), E = lg.size(1);
     TORCH_CHECK(E >= 1 && E <= 256, "paras moe_route: expert count must be in [1, 256]");
     TORCH_CHECK(k >= 1 && k <= E, "paras topk: k out of range");
-    const auto i64 = lg.options().dtype(c10::kLong);
-    Tensor topi = at::empty({T, k}, i64), topw = at::empty({T, k}, lg.options().dtype(c10::kFloat));
-    Tensor order = at::empty({T * k}, i64), inv = at::empty({T * k}, i64);
-    Tensor counts = at::empty({E}, i64), offsets = at::empty({E + 1}, i64);
+    const auto dev = lg.device();
+    Tensor topi = empty_paras({T, k}, c10::kLong, dev), topw = empty_paras({T, k}, c10::kFloat, dev);
+    Tensor order = empty_paras({T * k}, c10::kLong, dev), inv = empty_paras({T * k}, c10::kLong, dev);
+    Tensor counts = empty_paras({E}, c10::kLong, dev), offsets = empty_paras({E + 1}, c10::kLong, dev);
     Tensor ws = workspace(paras_moe_route_workspace(T, E, k), lg.device());
     check(paras_moe_route(lg.data_ptr(), T, E, k, require_float_code(lg, "paras moe_route"), topi.data_ptr<int64_t>(),
                           topw.data_ptr<float>(), order.data_ptr<int64_t>(), inv.data_ptr<int64_t>(),
@@ -133,7 +135,7 @@ Tensor moe_ffn(const Tensor& x, const Tensor& w_gate, const Tensor& w_up, const 
     };
     Tensor xc = dense16(x), wg = dense16(w_gate), wu = dense16(w_up), wd = dense16(w_down);
     Tensor tw = topw.contiguous(), od = order.contiguous(), iv = inv_order.contiguous(), of = offsets.contiguous();
-    Tensor out = at::empty({T, H}, xc.options());
+    Tensor out = empty_paras({T, H}, xc.scalar_type(), xc.device());
     if (T == 0) return out;
     const int dt = require_float_code(xc, "paras moe_ffn");
     Tensor ws = workspace(paras_moe_ffn_workspace(T, k, H, I, dt), xc.device());
@@ -143,7 +145,91 @@ Tensor moe_ffn(const Tensor& x, const Tensor& w_gate, const Tensor& w_up, const 
     return out;
 }
 
+// ---- the differentiable forms.  Autograd nodes in C++: a node written in Python costs a trip into the
+// interpreter in each direction, which for a small tensor is more than the kernels behind it.  The ops are
+// reached through the dispatcher, so tensors of another device are refused as torch.ops.paras.* refuses them.
+template <typename Sig>
+c10::TypedOperatorHandle<Sig> find(const char* name) {
+    return c10::Dispatcher::singleton().findSchemaOrThrow(name, "").typed<Sig>();
+}
+std::tuple<Tensor, Tensor> call_rms_norm(const Tensor& x, const Tensor& w, double eps) {
+    static const auto op = find<std::tuple<Tensor, Tensor>(const Tensor&, const Tensor&, double)>("paras::rms_norm");
+    return op.call(x, w, eps);
+}
+std::tuple<Tensor, Tensor> call_rms_norm_backward(const Tensor& g, const Tensor& x, const Tensor& w, const Tensor& rstd) {
+    static const auto op = find<std::tuple<Tensor, Tensor>(const Tensor&, const Tensor&, const Tensor&, const Tensor&)>("paras::rms_norm_backward");
+    return op.call(g, x, w, rstd);
+}
+Tensor call_swiglu(const Tensor& gate, const Tensor& up) {
+    static const auto op = find<Tensor(const Tensor&, const Tensor&)>("paras::swiglu");
+    return op.call(gate, up);
+}
+std::tuple<Tensor, Tensor> call_swiglu_backward(const Tensor& g, const Tensor& gate, const Tensor& up) {
+    static const auto op = find<std::tuple<Tensor, Tensor>(const Tensor&, const Tensor&, const Tensor&)>("paras::swiglu_backward");
+    return op.call(g, gate, up);
+}
+Tensor call_rotate_half(const Tensor& x) {
+    static const auto op = find<Tensor(const Tensor&)>("paras::rotate_half");
+    return op.call(x);
+}
+Tensor call_rotate_half_backward(const Tensor& g) {
+    static const auto op = find<Tensor(const Tensor&)>("paras::rotate_half_backward");
+    return op.call(g);
+}
+
+using torch::autograd::AutogradContext;
+using torch::autograd::variable_list;
+
+struct RMSNormFunction : torch::autograd::Function<RMSNormFunction> {
+    static Tensor forward(AutogradContext* ctx, const Tensor& x, const Tensor& w, double eps) {
+        auto [out, rstd] = call_rms_norm(x, w, eps);
+        ctx->save_for_backward({x, w, rstd});
+        return out;
+    }
+    static variable_list backward(AutogradContext* ctx, const variable_list& grads) {
+        const auto saved = ctx->get_saved_variables();
+        auto [gx, gw] = call_rms_norm_backward(grads[0].contiguous(), saved[0], saved[1], saved[2]);
+        return {gx, gw, Tensor()};
+    }
+};
+struct SwiGLUFunction : torch::autograd::Function<SwiGLUFunction> {
+    static Tensor forward(AutogradContext* ctx, const Tensor& gate, const Tensor& up) {
+        ctx->save_for_backward({gate, up});
+        return call_swiglu(gate, up);
+    }
+    static variable_list backward(AutogradContext* ctx, const variable_list& grads) {
+        const auto saved = ctx->get_saved_variables();
+        auto [gg, gu] = call_swiglu_backward(grads[0].contiguous(), saved[0], saved[1]);
+        return {gg, gu};
+    }
+};
+struct RotateHalfFunction : torch::autograd::Function<RotateHalfFunction> {
+    static Tensor forward(AutogradContext*, const Tensor& x) { return call_rotate_half(x); }
+    static variable_list backward(AutogradContext*, const variable_list& grads) {
+        return {call_rotate_half_backward(grads[0].contiguous())};
+    }
+};
+
 }  // namespace
+
+Tensor nn_rms_norm(const Tensor& input, const Tensor& weight, double eps) {
+    if (needs_grad(input, weight)) return RMSNormFunction::apply(input, weight, eps);
+    return std::get<0>(call_rms_norm(input, weight, eps));
+}
+Tensor nn_swiglu(const Tensor& gate, const Tensor& up) {
+    return needs_grad(gate, up) ? SwiGLUFunction::apply(gate, up) : call_swiglu(gate, up);
+}
+Tensor nn_rotate_half(const Tensor& x) { return needs_grad(x) ? RotateHalfFunction::apply(x) : call_rotate_half(x); }
+
+Tensor nn_moe_layer(const Tensor& x, const Tensor& logits, const Tensor& w_gate, const Tensor& w_up, const Tensor& w_down, int64_t k) {
+    using Route = std::tuple<Tensor, Tensor, Tensor, Tensor, Tensor, Tensor>;
+    static const auto route = find<Route(const Tensor&, int64_t)>("paras::moe_route");
+    static const auto ffn = find<Tensor(const Tensor&, const Tensor&, const Tensor&, const Tensor&, const Tensor&, const Tensor&,
+                                        const Tensor&, const Tensor&, int64_t)>("paras::moe_ffn");
+    auto [topi, topw, order, inv, counts, offsets] = route.call(logits, k);
+    return ffn.call(x, w_gate, w_up, w_down, topw, order, inv, offsets, k);
+}
+
 }  // namespace paras_torch
 
 TORCH_LIBRARY(paras, m) {

@@ -49,7 +49,7 @@ Tensor run_gemm(const Tensor& a_in, const Tensor& mat2, const c10::optional<Tens
     Tensor a = as_rows(a_in, mfma), bt = as_nt_operand(mat2, mfma);
     const int64_t M = a.size(-2), K = a.size(-1), N = bt.size(-2);
     std::vector<int64_t> shape = batch >= 0 ? std::vector<int64_t>{batch, M, N} : std::vector<int64_t>{M, N};
-    Tensor out = at::empty(shape, a.options());
+    Tensor out = empty_paras(shape, a.scalar_type(), a.device());
     if (out.numel() == 0) return out;
     const void* add_ptr = nullptr;
     int64_t ld_add = 0, s_add = 0;
@@ -65,7 +65,7 @@ Tensor run_gemm(const Tensor& a_in, const Tensor& mat2, const c10::optional<Tens
     // few-row products (decode-time projections) run faster with a workspace for split partial sums
     const size_t ws_bytes = paras_gemm_nt_workspace(M, N, K, nb, code);
     Tensor ws;
-    if (ws_bytes > 0) ws = at::empty({static_cast<int64_t>(ws_bytes)}, a.options().dtype(c10::kByte));
+    if (ws_bytes > 0) ws = workspace(ws_bytes, a.device());
     check(paras_gemm_nt_ws(a.data_ptr(), bt.data_ptr(), add_ptr, out.data_ptr(), M, N, K, a.stride(-2), bt.stride(-2), N, ld_add,
                            nb, batch >= 0 ? a.stride(0) : 0, batch >= 0 ? bt.stride(0) : 0, M * N, s_add, alpha, beta, code,
                            ws_bytes > 0 ? ws.data_ptr() : nullptr, ws_bytes, stream_for(a)));

@@ -46,14 +46,21 @@ Tensor run(int op, const Tensor& self, const Tensor& other, double alpha, const 
         b = at::empty({}, self.options());
         b.fill_(other.to(self.scalar_type()).item());
     }
-    const std::vector<int64_t> shape = at::infer_size(self.sizes(), b.sizes());
+    const at::DimVector shape = self.sizes().equals(b.sizes()) ? at::DimVector(self.sizes()) : at::infer_size_dimvector(self.sizes(), b.sizes());
     TORCH_CHECK(shape.size() <= 8, "paras: tensor rank ", shape.size(), " exceeds kernel limit of 8");
-    const Tensor a = self.expand(shape), bb = b.expand(shape);
-    Tensor out = into != nullptr ? *into : at::empty(shape, self.options());
+    // the strides an expanded view would have (a view per operand costs more here than the launch)
+    auto strides_in = [&](const Tensor& t) {
+        at::DimVector st(shape.size(), 0);
+        const size_t lead = shape.size() - static_cast<size_t>(t.dim());
+        for (int64_t d = 0; d < t.dim(); ++d)
+            if (t.size(d) == shape[lead + d]) st[lead + d] = t.stride(d);     // (a size of 1 that is repeated: stride 0)
+        return st;
+    };
+    const at::DimVector as = strides_in(self), bs = strides_in(b);
+    Tensor out = into != nullptr ? *into : empty_paras(shape, self.scalar_type(), self.device());
     if (out.numel() == 0) return out;
-    check(paras_binary_strided(op, a.data_ptr(), bb.data_ptr(), out.data_ptr(), static_cast<int>(shape.size()), shape.data(),
-                               a.strides().data(), bb.strides().data(), alpha, require_float_code(self, "paras binary op"),
-                               stream_for(self)));
+    check(paras_binary_strided(op, self.data_ptr(), b.data_ptr(), out.data_ptr(), static_cast<int>(shape.size()), shape.data(),
+                               as.data(), bs.data(), alpha, require_float_code(self, "paras binary op"), stream_for(self)));
     return out;
 }
 

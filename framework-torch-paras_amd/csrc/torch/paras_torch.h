@@ -83,8 +83,22 @@ inline void* stream_for(const at::Tensor& t) { return stream_for(t.device().inde
 // Thread-local current device index (the device guard's state).
 c10::DeviceIndex current_device();
 
-// Fresh tensor on the `paras` device.
+// Fresh dense tensor on the `paras` device.  Built here, not through at::empty: the trip through the
+// dispatcher is a sixth of what a small op costs on the host, and every op makes at least one tensor.
 at::Tensor empty_paras(c10::IntArrayRef sizes, c10::ScalarType dtype, c10::Device device);
+
+inline at::Tensor empty_paras_like(const at::Tensor& t) { return empty_paras(t.sizes(), t.scalar_type(), t.device()); }
+
+// Whether autograd has to see an op with these inputs.
+template <typename... Ts>
+bool needs_grad(const Ts&... t) { return at::GradMode::is_enabled() && (... || (t.defined() && t.requires_grad())); }
+
+// Differentiable forms of the fused ops and the MoE layer, for torch_paras.nn.
+at::Tensor nn_rms_norm(const at::Tensor& input, const at::Tensor& weight, double eps);
+at::Tensor nn_swiglu(const at::Tensor& gate, const at::Tensor& up);
+at::Tensor nn_rotate_half(const at::Tensor& x);
+at::Tensor nn_moe_layer(const at::Tensor& x, const at::Tensor& logits, const at::Tensor& w_gate, const at::Tensor& w_up,
+                        const at::Tensor& w_down, int64_t k);
 
 // Device scratch memory for one op call (returned to the pool when it dies).
 at::Tensor workspace(size_t nbytes, c10::Device device);

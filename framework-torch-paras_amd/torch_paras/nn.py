@@ -1,68 +1,32 @@
 """Differentiable wrappers of the ``paras::`` fused ops, and the MoE layer.
 
 ``rms_norm``, ``swiglu`` and ``rotate_half`` keep the reference's signatures
-(python/torch_paras/nn.py:75-89); their backward passes call the explicit
-backward ops.  ``moe_route`` / ``moe_ffn`` / ``moe_layer`` are this build's
+(python/torch_paras/nn.py:75-89); their autograd nodes are C++ (csrc/torch/
+ops_fused.cpp) and call the explicit backward ops.  ``moe_route`` / ``moe_ffn`` / ``moe_layer`` are this build's
 additions (forward only).
 """
 from __future__ import annotations
 
 import torch
 
-from . import _C  # noqa: F401  (loading it registers the paras:: ops)
+from . import _C  # (loading it registers the paras:: ops)
 
 __all__ = ["rms_norm", "swiglu", "rotate_half", "moe_route", "moe_ffn", "moe_layer"]
 
 
-class _RMSNorm(torch.autograd.Function):
-    @staticmethod
-    def forward(ctx, x, weight, eps):
-        out, rstd = torch.ops.paras.rms_norm(x, weight, eps)
-        ctx.save_for_backward(x, weight, rstd)
-        return out
-
-    @staticmethod
-    def backward(ctx, grad):
-        x, weight, rstd = ctx.saved_tensors
-        gx, gw = torch.ops.paras.rms_norm_backward(grad.contiguous(), x, weight, rstd)
-        return gx, gw, None
-
-
-class _SwiGLU(torch.autograd.Function):
-    @staticmethod
-    def forward(ctx, gate, up):
-        ctx.save_for_backward(gate, up)
-        return torch.ops.paras.swiglu(gate, up)
-
-    @staticmethod
-    def backward(ctx, grad):
-        gate, up = ctx.saved_tensors
-        return torch.ops.paras.swiglu_backward(grad.contiguous(), gate, up)
-
-
-class _RotateHalf(torch.autograd.Function):
-    @staticmethod
-    def forward(ctx, x):
-        return torch.ops.paras.rotate_half(x)
-
-    @staticmethod
-    def backward(ctx, grad):
-        return torch.ops.paras.rotate_half_backward(grad.contiguous())
-
-
 def rms_norm(input: torch.Tensor, weight: torch.Tensor, eps: float = 1e-6) -> torch.Tensor:
     """Fused RMSNorm over the last dimension."""
-    return _RMSNorm.apply(input, weight, eps)
+    return _C.nn_rms_norm(input, weight, eps)
 
 
 def swiglu(gate: torch.Tensor, up: torch.Tensor) -> torch.Tensor:
     """Fused ``silu(gate) * up``."""
-    return _SwiGLU.apply(gate, up)
+    return _C.nn_swiglu(gate, up)
 
 
 def rotate_half(x: torch.Tensor) -> torch.Tensor:
     """RoPE helper ``cat(-x2, x1)`` with ``x1, x2 = x.chunk(2, -1)``."""
-    return _RotateHalf.apply(x)
+    return _C.nn_rotate_half(x)
 
 
 def moe_route(logits: torch.Tensor, k: int):
@@ -81,5 +45,4 @@ def moe_ffn(x, w_gate, w_up, w_down, topw, order, inv_order, offsets, k: int) ->
 def moe_layer(x, router_logits, w_gate, w_up, w_down, k: int = 2) -> torch.Tensor:
     """One MoE layer: ``x [T,H]``, ``router_logits [T,E]``, ``w_gate/w_up [E,I,H]``,
     ``w_down [E,H,I]``."""
-    topi, topw, order, inv_order, counts, offsets = moe_route(router_logits, k)
-    return moe_ffn(x, w_gate, w_up, w_down, topw, order, inv_order, offsets, k)
+    return _C.nn_moe_layer(x, router_logits, w_gate, w_up, w_down, k)
