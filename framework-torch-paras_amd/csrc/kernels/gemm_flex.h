@@ -1,0 +1,222 @@
+// Tile mainloop of the 16-bit products whose operands may lie either way round:
+// C tile = op(A) op(B)^T with fp32 accumulation on v_mfma_f32_16x16x32.
+//
+// An operand is a set of `rows` (rows of C for A, columns of C for B) times the contraction.  It is
+// either contiguous along the contraction ("K", what x W^T has) or contiguous along its rows ("R":
+// the weight of an input gradient, both operands of a weight gradient).  A "K" tile sits in LDS as
+// [row][64] and a fragment is one 16-byte read; an "R" tile sits as [64][rows], as it lies in memory,
+// and a fragment is two ds_read_b64_tr_b16 (the transposing LDS read: a group of 16 lanes reads 4
+// contraction steps x 16 rows and each lane receives the 4 steps of its row).  Transposing at the LDS
+// read instead of in memory saves a whole pass over each such operand.
+//
+// A workgroup is four waves, 2 x 2, one per SIMD at the large tiles; a wave computes MI x NJ blocks of
+// 16 x 16, so the tile is 32 MI x 32 NJ.  Tiles of 64 contraction steps go from memory straight to LDS
+// (buffer_load ... lds), two stages: no staging registers, no LDS stores, nothing in the loop but
+// MFMAs, LDS reads and one request per four MFMAs, which is what a single wave per SIMD can issue in the
+// shadow of its MFMAs.  One barrier per tile, before its last k-step: by then all of the tile's
+// fragments are in registers, so the tile after next can be requested into its stage right away and has
+// a tile's time to arrive, while the k-step's MFMAs run and the next tile's first fragments are read.
+//
+// Direct loads fill LDS in lane order, so rows cannot be padded apart; instead the 16-byte chunks of a
+// row (K) or the 32-byte units (R) are permuted by a function of the row, applied to the address a
+// lane fetches from and again where fragments are read, so that the lanes of one LDS access phase hit
+// distinct banks.  Loads are checked against the exact extent of the operand by the buffer unit: rows
+// past its end and contraction steps past K come back as zeros without a branch.
+#pragma once
+
+#include <hip/hip_runtime.h>
+
+#include "core/device_math.h"
+#include "kernels/gemm_tile.h"
+
+namespace paras {
+namespace flex {
+
+using gemm::i16x8;
+using gemm::quad16::float4v;
+
+// acc += b a, in place in the accumulation registers.  Written out because the compiler, given the
+// builtin, moves the 256 accumulators of the large tile from register to register on their way round the
+// loop (120 to 350 moves and some spills per 128 MFMAs).  Nothing here needs the wait states it would
+// insert: fragments come from LDS (a wait on the counter covers them), the next MFMA on the same
+// accumulator is a k-step away, and the loop ends with a pause before the accumulators are read.
+template <typename T> __device__ __forceinline__ void mma(float4v& acc, i16x8 b, i16x8 a);
+template <> __device__ __forceinline__ void mma<bf16_t>(float4v& acc, i16x8 b, i16x8 a) {
+    asm volatile("v_mfma_f32_16x16x32_bf16 %0, %1, %2, %0" : "+a"(acc) : "v"(b), "v"(a));
+}
+template <> __device__ __forceinline__ void mma<f16_t>(float4v& acc, i16x8 b, i16x8 a) {
+    asm volatile("v_mfma_f32_16x16x32_f16 %0, %1, %2, %0" : "+a"(acc) : "v"(b), "v"(a));
+}
+
+constexpr int kThreads = 256;
+constexpr int kBK = 64;
+constexpr std::uint32_t kOutOfRange = 0xF0000000u;       // a byte offset beyond any buffer extent used here
+constexpr long kMaxExtent = 0xE0000000L;
+constexpr long kMaxLd = 1L << 22;                        // elements: a tile's offsets stay far below kMaxExtent
+
+__device__ __forceinline__ int wave_id() { return __builtin_amdgcn_readfirstlane(static_cast<int>(threadIdx.x) >> 6); }
+
+// One operand as a workgroup fetches and reads it: W requests per wave and tile.
+template <int W, bool R> struct Operand {
+    static constexpr int kRows = 32 * W;
+    static constexpr int kElems = kRows * kBK;
+    static constexpr int kBases = R ? (W >= 4 ? 4 : W) : 2;     // lane offsets of fragment reads
+    const char* base;             // (first row of the tile, first contraction step of the part); uniform
+    long left;                    // bytes from there to the end of the operand; uniform
+    long step;                    // bytes from a tile to the next
+    std::uint32_t off[W];         // this lane's chunk of each request
+    int fb[kBases];
+
+    // 32-byte unit `u` of contraction step k of an R tile sits at unit u ^ unit_swizzle(k)
+    __device__ static __forceinline__ int unit_swizzle(int k) { return W >= 2 ? (k & 3) : ((k >> 1) & 1); }
+
+    __device__ __forceinline__ void init(const std::uint16_t* p, long ld, long rows, long row0, long k_first, long k_count, int w) {
+        const int lane = threadIdx.x & 63, l16 = lane & 15, kq = lane >> 4;
+        if constexpr (R) {
+            base = reinterpret_cast<const char*>(p + k_first * ld + row0);
+            left = ((k_count - 1) * ld + (rows - row0)) * 2;
+            step = kBK * ld * 2;
+#pragma unroll
+            for (int i = 0; i < W; ++i) {
+                const int c = (i * 4 + wave_id()) * 64 + lane;
+                const int k = c / (4 * W), slot = c % (4 * W);
+                off[i] = static_cast<std::uint32_t>(k * ld * 2 + (slot ^ (unit_swizzle(k) << 1)) * 16);
+            }
+            const int k = kq * 8 + (l16 >> 2);
+#pragma unroll
+            for (int b = 0; b < kBases; ++b) fb[b] = k * kRows + ((w * W + b) ^ unit_swizzle(k)) * 16 + 4 * (l16 & 3);
+        } else {
+            base = reinterpret_cast<const char*>(p + row0 * ld + k_first);
+            left = ((rows - row0 - 1) * ld + k_count) * 2;
+            step = kBK * 2;
+#pragma unroll
+            for (int i = 0; i < W; ++i)
+                off[i] = static_cast<std::uint32_t>(((i * 4 + wave_id()) * 8 + (lane >> 3)) * ld * 2 + ((lane & 7) ^ (lane >> 3)) * 16);
+#pragma unroll
+            for (int ks = 0; ks < 2; ++ks) fb[ks] = (w * 16 * W + l16) * kBK + ((ks * 4 + kq) ^ (l16 & 7)) * 8;
+        }
+    }
+    // From now on only the last tile is requested: its contraction steps past the end are not to be
+    // fetched (K: they are the next row's; R: the extent ends there anyway).
+    __device__ __forceinline__ void last_tile(int k_in_tile) {
+        if constexpr (!R) {
+            const int lane = threadIdx.x & 63;
+            const std::uint32_t gone = ((lane & 7) ^ (lane >> 3)) * 8 < k_in_tile ? 0u : kOutOfRange;
+#pragma unroll
+            for (int i = 0; i < W; ++i) off[i] |= gone;
+        }
+    }
+    __device__ __forceinline__ __amdgpu_buffer_rsrc_t rsrc(int kt, int k_tiles) const {
+        const long l = left - kt * step;
+        const long n = l < 0 || kt >= k_tiles ? 0 : (l > kMaxExtent ? kMaxExtent : l);
+        return __builtin_amdgcn_make_buffer_rsrc(const_cast<char*>(base + kt * step), 0, static_cast<int>(static_cast<std::uint32_t>(n)), 0x00020000);
+    }
+    __device__ __forceinline__ void request(__amdgpu_buffer_rsrc_t r, std::uint16_t* tile, int i) const {
+        typedef __attribute__((address_space(3))) void* lds_ptr;
+        __builtin_amdgcn_raw_ptr_buffer_load_lds(r, (lds_ptr)(tile + (i * 4 + wave_id()) * 512), 16, static_cast<int>(off[i]), 0, 0, 0);
+    }
+    __device__ __forceinline__ i16x8 frag(const std::uint16_t* tile, int blk, int ks) const {
+        if constexpr (R) {
+            typedef __attribute__((address_space(3))) i16x4 lds_i16x4;
+            const std::uint16_t* q = tile + fb[blk % kBases] + (blk / kBases) * kBases * 16 + ks * 32 * kRows;
+            const i16x4 lo = __builtin_amdgcn_ds_read_tr16_b64_v4i16((lds_i16x4*)(q));
+            const i16x4 hi = __builtin_amdgcn_ds_read_tr16_b64_v4i16((lds_i16x4*)(q + 4 * kRows));
+            return i16x8{lo[0], lo[1], lo[2], lo[3], hi[0], hi[1], hi[2], hi[3]};
+        } else {
+            return *reinterpret_cast<const i16x8*>(&tile[fb[ks] + blk * 16 * kBK]);
+        }
+    }
+};
+
+// acc[i][j]: the B fragment is the instruction's first operand, so lane (l16 = lane % 16, kq = lane / 16)
+// holds row i*16 + l16 of the wave's rows and columns j*16 + 4*kq .. + 3 of its columns.
+// (The stages are separate arrays named at compile time: an LDS read waits for every direct load in flight
+// that the compiler cannot prove to go elsewhere.)
+template <typename T, int MI, int NJ, bool AR, bool BR>
+__device__ __forceinline__ void mainloop(Operand<MI, AR>& oa, Operand<NJ, BR>& ob, int k_count, std::uint16_t* a0, std::uint16_t* a1,
+                                         std::uint16_t* b0, std::uint16_t* b1, float4v (&acc)[MI][NJ]) {
+    constexpr int C = MI + NJ;          // requests per wave and tile, and fragments per k-step
+    constexpr int S = MI * NJ;          // MFMAs per k-step
+    i16x8 af[2][MI], bf[2][NJ];
+    const int k_tiles = (k_count + kBK - 1) / kBK;
+    auto request_one = [&](__amdgpu_buffer_rsrc_t ra, __amdgpu_buffer_rsrc_t rb, std::uint16_t* ta, std::uint16_t* tb, int c) {
+        if (c < MI) oa.request(ra, ta, c);
+        else        ob.request(rb, tb, c - MI);
+    };
+    auto request_all = [&](int kt, std::uint16_t* ta, std::uint16_t* tb) {
+        if (kt == k_tiles - 1) {
+            oa.last_tile(k_count - kt * kBK);
+            ob.last_tile(k_count - kt * kBK);
+        }
+        const auto ra = oa.rsrc(kt, k_tiles);
+        const auto rb = ob.rsrc(kt, k_tiles);
+#pragma unroll
+        for (int c = 0; c < C; ++c) request_one(ra, rb, ta, tb, c);
+    };
+    auto read_frag = [&](const std::uint16_t* ta, const std::uint16_t* tb, int buf, int f, int ks) {
+        if (f < MI) af[buf][f] = oa.frag(ta, f, ks);
+        else        bf[buf][f - MI] = ob.frag(tb, f - MI, ks);
+    };
+    auto meet = [] {
+        __builtin_amdgcn_s_waitcnt(0x0070);     // vmcnt(0) lgkmcnt(0): this wave's part of the next tile has landed, its reads of this one are done
+        lds_barrier();
+    };
+#pragma unroll
+    for (int i = 0; i < MI; ++i)
+#pragma unroll
+        for (int j = 0; j < NJ; ++j) acc[i][j] = float4v{0.f, 0.f, 0.f, 0.f};
+    auto pin = [&] {          // orders the accumulators' other uses against the written-out MFMAs
+#pragma unroll
+        for (int i = 0; i < MI; ++i)
+#pragma unroll
+            for (int j = 0; j < NJ; ++j) asm volatile("" : "+a"(acc[i][j]));
+    };
+    pin();
+    // The requests for the tile after next are spread over the whole k-step that follows the barrier: bunched into
+    // its first half they come at twice the rate the CU's L1 takes them and hold up the MFMAs (8192^3 807 against
+    // 774 us), spread further into the next k-step the last of them are late at the barrier (788 us).
+    // Tile kt from stage (ca, cb); the next one is in (na, nb).  One body for every tile, the last ones included:
+    // a copy of it for them costs the accumulators their places (hundreds of spills), so requests past the end
+    // go to an empty extent, which fetches nothing and clears the stage.
+    auto tile = [&](int kt, std::uint16_t* ca, std::uint16_t* cb, std::uint16_t* na, std::uint16_t* nb) {
+        if (kt + 2 == k_tiles - 1) {
+            oa.last_tile(k_count - (kt + 2) * kBK);
+            ob.last_tile(k_count - (kt + 2) * kBK);
+        }
+        const auto ra = oa.rsrc(kt + 2, k_tiles);
+        const auto rb = ob.rsrc(kt + 2, k_tiles);
+#pragma unroll
+        for (int ks = 0; ks < 2; ++ks) {
+            if (ks == 1) meet();
+#pragma unroll
+            for (int j = 0; j < NJ; ++j)
+#pragma unroll
+                for (int i = 0; i < MI; ++i) {
+                    const int slot = j * MI + i;
+                    mma<T>(acc[i][j], bf[ks][j], af[ks][i]);
+#pragma unroll
+                    for (int c = 0; c < C; ++c) {
+                        if ((c * S * 7) / (8 * C) == slot) read_frag(ks == 0 ? ca : na, ks == 0 ? cb : nb, ks ^ 1, c, ks ^ 1);
+                        if (ks == 1 && (c * S) / C == slot) request_one(ra, rb, ca, cb, c);
+                    }
+                    __builtin_amdgcn_sched_barrier(0);
+                }
+        }
+    };
+    request_all(0, a0, b0);
+    request_all(1, a1, b1);
+    meet();
+#pragma unroll
+    for (int f = 0; f < C; ++f) read_frag(a0, b0, 0, f, 0);
+    // (In pairs, with one way out: an odd number of tiles multiplies a cleared one at the end.)
+    for (int kt = 0; kt < k_tiles; kt += 2) {
+        tile(kt, a0, b0, a1, b1);
+        tile(kt + 1, a1, b1, a0, b0);
+    }
+    asm volatile("s_nop 15\n\ts_nop 15" ::: "memory");      // the last products are on their way to the registers the epilogue reads
+    pin();
+    __builtin_amdgcn_s_waitcnt(0x0F70);         // vmcnt(0): no request may outlive the workgroup's LDS
+}
+
+}  // namespace flex
+}  // namespace paras

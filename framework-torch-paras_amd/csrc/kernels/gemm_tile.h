@@ -529,7 +529,6 @@ struct Tile128G {
     }
 };
 using Tile128 = Tile128G<2>;
-using Tile128x128 = Tile128G<1>;     // one column group: twice the workgroups for problems that would not fill the chip
 struct Tile256 {
     static constexpr int kBM = wide::kBM, kThreads = wide::kThreads, kBChunks = 2, kGroups = 2;
     using Lds = wide::TileLds;

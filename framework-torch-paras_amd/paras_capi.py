@@ -18,6 +18,13 @@ DT = {torch.float32: F32, torch.float16: F16, torch.bfloat16: BF16, torch.float6
 i64, vp, f64, i32, sz = C.c_int64, C.c_void_p, C.c_double, C.c_int, C.c_size_t
 
 
+class GemmArgs(C.Structure):
+    """paras_gemm_args of include/paras_hip.h."""
+    _fields_ = ([(n, C.c_void_p) for n in ("a", "b", "addend", "c")] +
+                [(n, C.c_int64) for n in ("M", "N", "K", "lda", "ldb", "ldc", "ld_add", "batch", "stride_a", "stride_b", "stride_c", "stride_add")] +
+                [("alpha", C.c_double), ("beta", C.c_double), ("dtype", C.c_int), ("a_rows", C.c_int), ("b_rows", C.c_int)])
+
+
 class SdpaArgs(C.Structure):
     _fields_ = [
         ("q", vp), ("k", vp), ("v", vp), ("out", vp), ("attn", vp), ("lse", vp), ("mask", vp),
@@ -71,6 +78,10 @@ SIGNATURES = {
     "paras_gemm_nt": (i32, [vp, vp, vp, vp] + [i64] * 12 + [f64, f64, i32, vp]),
     "paras_gemm_nt_workspace": (sz, [i64, i64, i64, i64, i32]),
     "paras_gemm_nt_ws": (i32, [vp, vp, vp, vp] + [i64] * 12 + [f64, f64, i32, vp, sz, vp]),
+    "paras_gemm_workspace": (sz, [C.POINTER(GemmArgs)]),
+    "paras_gemm": (i32, [C.POINTER(GemmArgs), vp, sz, vp]),
+    "paras_column_sum_workspace": (sz, [i64, i64, i32]),
+    "paras_column_sum": (i32, [vp, vp, i64, i64, i64, i32, vp, vp]),
     "paras_softmax_rows": (i32, [vp, vp, i64, i64, i32, i32, vp]),
     "paras_topk_rows": (i32, [vp, vp, vp, i64, i64, i64, i32, i32, vp]),
 }
@@ -294,3 +305,28 @@ def topk_rows(x, k, largest=True):
     indices = torch.empty(*x.shape[:-1], k, dtype=torch.int64, device=x.device)
     check(lib().paras_topk_rows(_ptr(x), _ptr(values), _ptr(indices), rows, n, k, 1 if largest else 0, DT[x.dtype], _stream()))
     return values, indices
+
+
+def gemm(a, b, addend=None, alpha=1.0, beta=1.0, workspace=True):
+    """C = alpha * a @ b^T (+ beta * addend), a [M, K], b [N, K], each contiguous along either dim
+    (paras_gemm); addend [N] or [M, N]."""
+    M, K = a.shape
+    N = b.shape[0]
+    c = torch.empty((M, N), dtype=a.dtype, device=a.device)
+    rows = [0 if t.stride(1) == 1 else 1 for t in (a, b)]
+    g = GemmArgs(_ptr(a), _ptr(b), _ptr(addend) if addend is not None else None, _ptr(c), M, N, K, 0, 0, N,
+                 addend.stride(0) if addend is not None and addend.dim() == 2 else 0, 1, 0, 0, 0, 0, alpha, beta, DT[a.dtype], *rows)
+    g.lda, g.ldb = a.stride(1 if rows[0] else 0), b.stride(1 if rows[1] else 0)
+    n = lib().paras_gemm_workspace(C.byref(g)) if workspace else 0
+    ws = torch.empty(max(n, 16), dtype=torch.uint8, device=a.device)
+    check(lib().paras_gemm(C.byref(g), _ptr(ws) if workspace else None, n, _stream()))
+    return c
+
+
+def column_sum(x):
+    """Sums of the columns of x [rows, cols] (paras_column_sum)."""
+    rows, cols = x.shape
+    out = torch.empty(cols, dtype=x.dtype, device=x.device)
+    ws = torch.empty(max(lib().paras_column_sum_workspace(rows, cols, DT[x.dtype]), 16), dtype=torch.uint8, device=x.device)
+    check(lib().paras_column_sum(_ptr(x), _ptr(out), rows, cols, x.stride(0), DT[x.dtype], _ptr(ws), _stream()))
+    return out

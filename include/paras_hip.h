@@ -369,6 +369,36 @@ PARAS_API int paras_gemm_nt_ws(const void* a, const void* b, const void* addend,
                                int64_t stride_b, int64_t stride_c, int64_t stride_add,
                                double alpha, double beta, int dtype, void* workspace,
                                size_t workspace_bytes, void* stream);
+/* The same product with operands either way round: an operand is contiguous   */
+/* along the contraction (row r, step k at r * ld + k) or, with a_rows / b_rows */
+/* set, along its rows (k * ld + r) -- dy W and dy^T x of a linear layer's      */
+/* backward without a transposed copy (the reference's LinearFunction::backward, */
+/* csrc/ops/vision_ops.cpp:280-309).  paras_gemm_workspace bytes (16-byte       */
+/* aligned) let the contraction be split over workgroups where there are few    */
+/* tiles, the parts being added in a fixed order; with fewer bytes or NULL it   */
+/* is not.  a_rows needs b_rows.  16-bit operands with a_rows or b_rows: 16-byte */
+/* aligned, leading dimensions and batch strides multiples of 8, and K a        */
+/* multiple of 8 unless both are set; fp32: any; fp64: neither may be set.      */
+typedef struct paras_gemm_args {
+    const void* a;
+    const void* b;
+    const void* addend;          /* may be NULL */
+    void* c;
+    int64_t M, N, K;
+    int64_t lda, ldb, ldc, ld_add;
+    int64_t batch, stride_a, stride_b, stride_c, stride_add;
+    double alpha, beta;
+    int dtype;
+    int a_rows, b_rows;
+} paras_gemm_args;
+PARAS_API size_t paras_gemm_workspace(const paras_gemm_args* args);
+PARAS_API int paras_gemm(const paras_gemm_args* args, void* workspace,
+                         size_t workspace_bytes, void* stream);
+/* out[c] = T(sum over the rows of x[r][c]), rows ld apart: a bias gradient (same */
+/* reference lines).  Any float dtype; paras_column_sum_workspace bytes.         */
+PARAS_API size_t paras_column_sum_workspace(int64_t rows, int64_t cols, int dtype);
+PARAS_API int paras_column_sum(const void* x, void* out, int64_t rows, int64_t cols,
+                               int64_t ld, int dtype, void* workspace, void* stream);
 
 /* ------------------------------------------------------------------------- */
 /* Row softmax and row top-k (replace softmax_out / topk_out,                  */

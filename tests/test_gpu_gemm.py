@@ -421,3 +421,44 @@ def test_gemm_nt_few_columns_and_many_rows(shape, dtype):
         ob = capi.gemm_nt(ab.cuda(), bb.cuda())
         for i in range(2):
             assert_gemm_close(ob[i, -3:], O.matmul_nt(ab[i, -3:], bb[i]), dtype)
+
+
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16, torch.float32])
+@pytest.mark.parametrize("shape", [(1, 64, 8), (33, 72, 64), (64, 136, 200), (200, 264, 72), (130, 1000, 1000), (520, 136, 4096), (3000, 520, 512),
+                                   (1000, 3000, 1032), (2048, 4096, 128)])
+def test_gemm_operands_either_way_round(shape, dtype):
+    """paras_gemm: both operands along the contraction, B along its rows (dy W), both along their rows
+    (dy^T x) -- tiles from 32 x 128 to 256 x 256, cut short in every direction, an odd and an even number of
+    contraction tiles, the contraction whole and in parts (in a fixed order: the same bits on every call)."""
+    M, N, K = shape
+    torch.manual_seed(M + N + K)
+    a = torch.randn(M, K).to(dtype)
+    b = (torch.randn(N, K) / math.sqrt(K)).to(dtype)
+    bias = torch.randn(N).to(dtype)
+    want = a.double() @ b.double().T
+    tol = {torch.bfloat16: 4e-3, torch.float16: 6e-4, torch.float32: 3e-6}[dtype]     # (fp32: a sequential sum of 4096 products)
+    rows16 = dtype != torch.float32
+    ac, bc = a.cuda(), b.cuda()
+    ar, br = a.T.contiguous().cuda().T, b.T.contiguous().cuda().T
+    if rows16 and N % 8:
+        pytest.skip("rows-contiguous 16-bit operands have leading dimensions that are multiples of 8")
+    for x, y in ((ac, bc), (ac, br), (ar, br)):
+        if rows16 and x is ar and M % 8:
+            continue
+        for ws in (False, True):
+            got = capi.gemm(x, y, workspace=ws)
+            assert ((got.cpu().double() - want).norm() / want.norm()).item() < tol
+            assert torch.equal(got, capi.gemm(x, y, workspace=ws))
+        got = capi.gemm(x, y, bias.cuda(), alpha=0.5, beta=2.0)
+        ref = 0.5 * want + 2.0 * bias.double()
+        assert ((got.cpu().double() - ref).norm() / ref.norm()).item() < tol
+
+
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16, torch.float32, torch.float64])
+@pytest.mark.parametrize("shape", [(1, 1), (7, 33), (9, 64), (3000, 4096), (65, 8200), (100000, 8)])
+def test_column_sum(shape, dtype):
+    x = torch.randn(*shape).to(dtype)
+    want = x.double().sum(0)
+    got = capi.column_sum(x.cuda()).cpu().double()
+    bound = {torch.bfloat16: 2.0 ** -8, torch.float16: 2.0 ** -11, torch.float32: 2.0 ** -23, torch.float64: 1e-14}[dtype]
+    assert bool(((got - want).abs() <= bound * want.abs() + 1e-5 * math.sqrt(shape[0]) * (1 if dtype.itemsize == 2 else 1e-2)).all())

@@ -878,3 +878,44 @@ def test_empty_and_degenerate_shapes_match_the_cpu(device):
     assert topi.shape == (0, 2) and counts.cpu().tolist() == [0] * 8 and offsets.cpu().tolist() == [0] * 9
     out, rstd = torch.ops.paras.rms_norm(torch.zeros(0, 64).to(device), torch.ones(64).to(device), 1e-6)
     assert out.shape == (0, 64) and rstd.numel() == 0
+
+
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float32])
+@pytest.mark.parametrize("lead,N,K,bias", [((5,), 64, 128, True), ((2, 7), 72, 64, True), ((3, 11, 2), 128, 200, False), ((1,), 8, 8, True)])
+def test_linear_gradients_in_one_node_match_the_cpu(device, lead, N, K, bias, dtype):
+    """F.linear's own autograd node: outputs and all gradients against the CPU in double, only the gradients
+    asked for, and a second differentiation of the first."""
+    torch.manual_seed(N + K)
+    x, w, b, dy = torch.randn(*lead, K).to(dtype), torch.randn(N, K).to(dtype), torch.randn(N).to(dtype), torch.randn(*lead, N).to(dtype)
+    ins = [x, w, b] if bias else [x, w]
+    dev = [t.to(device).requires_grad_() for t in ins]
+    ref = [t.double().requires_grad_() for t in ins]
+    y, yr = F.linear(*dev), F.linear(*ref)
+    tol = 8e-3 if dtype == torch.bfloat16 else 1e-5
+    pairs = zip([y, *torch.autograd.grad(y, dev, dy.to(device), retain_graph=True)], [yr, *torch.autograd.grad(yr, ref, dy.double(), retain_graph=True)])
+    for got, want in pairs:
+        assert got.shape == want.shape and ((got.detach().cpu().double() - want.detach()).norm() / want.detach().norm()).item() < tol
+    only, = torch.autograd.grad(y, dev[1:2], dy.to(device))
+    assert only.shape == w.shape
+    g, = torch.autograd.grad(F.linear(*dev), dev[0], dy.to(device), create_graph=True)
+    gw, = torch.autograd.grad(g, dev[1], torch.ones_like(g))
+    want = dy.double().reshape(-1, N).sum(0)[:, None].expand(N, K)
+    assert ((gw.cpu().double() - want).norm() / want.norm()).item() < tol
+
+
+@pytest.mark.parametrize("dtype", [torch.float16, torch.float32])
+@pytest.mark.parametrize("Lq,Lk,D,mask_shape", [(77, 77, 64, (2, 1, 1, 77)), (77, 77, 64, (2, 4, 77, 77)), (1, 200, 128, (2, 1, 1, 200)), (33, 50, 40, (50,)),
+                                                (33, 50, 64, (33, 50))])
+def test_boolean_masks_reach_the_kernels_as_they_are(device, Lq, Lk, D, mask_shape, dtype):
+    """A boolean mask gives what its additive form gives (0 / -inf, the composite op's conversion), masks the
+    direct route does not take (one-dimensional) included."""
+    torch.manual_seed(Lq + Lk + D)
+    q, k, v = (torch.randn(2, 4, n, D).to(dtype).to(device) for n in (Lq, Lk, Lk))
+    mask = torch.rand(*mask_shape) < 0.6
+    mask[..., 0] = True
+    add = torch.zeros(mask_shape).masked_fill(~mask, float("-inf")).to(dtype)
+    if len(mask_shape) == 1:
+        mask, add = mask.expand(Lq, Lk), add.expand(Lq, Lk)
+    got = F.scaled_dot_product_attention(q, k, v, attn_mask=mask.to(device))
+    want = F.scaled_dot_product_attention(q, k, v, attn_mask=add.to(device))
+    assert ((got - want).cpu().float().norm() / want.cpu().float().norm()).item() < (2e-3 if dtype == torch.float16 else 1e-6)
