@@ -1,0 +1,338 @@
+// Scaled-dot-product attention of fp32 tensors in one pass on the matrix cores (the output and the log-sum-exp;
+// returned weights are the composed route's or the general kernel's business).
+//
+// Before, small problems ran one workgroup per query row with scalar fp64 dot products formed three
+// times per score, every lane of a wavefront on a key row of its own (B1 H8 S128 D64: 44 us; B3 H64 S57
+// D128: 254 us), and large ones as two batched products around a row kernel with the scores in memory (B1 H2
+// S3737 D128: 740 us, of which 508 us one product with 60 workgroups).
+//
+// A workgroup takes 16 QB queries of one head; its four waves take the keys in turns of 32 (16 where
+// there are few keys or the registers are full) and meet at the end (running maximum, row sum, output: combined through LDS).  Per turn and wave:
+//   S^T = K Q^T      v_mfma 16x16x4, A = 16 keys, B = 16 queries
+//   online softmax   a lane holds one query and 4 keys of each 16 x 16 block
+//   O^T += V^T P^T   the accumulator layout of S^T is the B operand layout of this product: step t takes
+//                    register t of every lane, i.e. the keys that the instruction's row map puts there
+// so nothing passes through LDS or between lanes except the row maxima.  Operands come straight from memory
+// in 16-byte pieces, four MFMAs each: which contraction steps (QK) or head elements (PV) an instruction sees
+// is free as long as both operands agree, and O^T then ends up with 4 adjacent elements of a row in a lane.
+// K of the next turn and V of this one are requested before the turn's products.
+//
+// Acc = double: v_mfma_f64_16x16x4 (78 TFLOP/s published), softmax in fp64: what the general kernel
+// computes, for the problems that it served.  Acc = float: v_mfma_f32_16x16x4 (157 TFLOP/s), for the large
+// ones, which the batched products accumulated in fp32.  Scores are rounded to fp32 where the reference's
+// are (the product, the scaled product, the sum with an additive mask: attention_ops.cpp:101-128).
+// What bounds it: small problems the chain of one turn (two memory latencies, products, merge), large ones
+// the matrix cores and the L2 reads of K and V by every 16 QB queries.
+#include <hip/hip_runtime.h>
+
+#include <cmath>
+
+#include "core/device_math.h"
+#include "core/status.h"
+#include "kernels/sdpa_internal.h"
+
+namespace paras {
+namespace {
+
+constexpr int kWavesF = 4;
+constexpr std::uint32_t kOutOfRange = 0xF0000000u;
+
+struct F32Params {
+    const float* q; const float* k; const float* v; float* out; float* lse;
+    const void* mask;
+    int is_causal;
+    int Hq, Hkv, Lq, Lk, D, Dv;
+    int q_tiles;
+    long qs[3], ks[3], vs[3], ms[4];
+    double scale;
+};
+
+template <typename Acc> struct Mma;
+template <> struct Mma<double> {
+    typedef double vec __attribute__((ext_vector_type(4)));
+    __device__ static __forceinline__ vec run(float a, float b, vec c) {
+        return __builtin_amdgcn_mfma_f64_16x16x4f64(static_cast<double>(a), static_cast<double>(b), c, 0, 0, 0);
+    }
+    __device__ static __forceinline__ vec run(float a, double b, vec c) {
+        return __builtin_amdgcn_mfma_f64_16x16x4f64(static_cast<double>(a), b, c, 0, 0, 0);
+    }
+    __device__ static __forceinline__ int row(int g, int r) { return 4 * r + g; }       // row of register r in lane group g
+    __device__ static __forceinline__ double exp_of(double x) { return exp(x); }
+};
+template <> struct Mma<float> {
+    typedef float vec __attribute__((ext_vector_type(4)));
+    __device__ static __forceinline__ vec run(float a, float b, vec c) { return __builtin_amdgcn_mfma_f32_16x16x4f32(a, b, c, 0, 0, 0); }
+    __device__ static __forceinline__ int row(int g, int r) { return 4 * g + r; }
+    __device__ static __forceinline__ float exp_of(float x) { return __builtin_amdgcn_exp2f(x * 1.4426950408889634f); }
+};
+
+// DM: largest head size of this form (64, 128, 256); D and Dv are multiples of 4 up to it.
+// A turn is KB blocks of 16 keys.  kMask: 0 = none, 1 = bool (true = attend), 2 = additive.
+template <typename Acc, int DM, int QB, int KB, int kMask>
+__global__ __launch_bounds__(kWavesF * 64) void sdpa_f32_kernel(const F32Params p) {
+    using M = Mma<Acc>;
+    using vec = typename M::vec;
+    constexpr int DC = DM / 16, VC = DM / 64, kTurn = 16 * KB;
+    __shared__ Acc o_part[kWavesF][QB * VC * 4 * 256];
+    __shared__ Acc m_part[kWavesF][QB][16], l_part[kWavesF][QB][16];
+
+    // heaviest query tiles first under the causal rule
+    const int qt = p.is_causal ? p.q_tiles - 1 - static_cast<int>(blockIdx.x) : static_cast<int>(blockIdx.x);
+    const int h = blockIdx.y, b = blockIdx.z, hkv = h / (p.Hq / p.Hkv);
+    const int lane = threadIdx.x & 63, l16 = lane & 15, g = lane >> 4;
+    const int wave = __builtin_amdgcn_readfirstlane(static_cast<int>(threadIdx.x) >> 6);
+    const int q0 = qt * 16 * QB;
+
+    auto rsrc_of = [](const float* base, long rows, long ld, int width) {
+        return __builtin_amdgcn_make_buffer_rsrc(const_cast<float*>(base), 0, static_cast<int>(((rows - 1) * ld + width) * 4), 0x00020000);
+    };
+    const auto kr = rsrc_of(p.k + b * p.ks[0] + hkv * p.ks[1], p.Lk, p.ks[2], p.D);      // (< 2^31 bytes: checked by f32_supported)
+    const auto vr = rsrc_of(p.v + b * p.vs[0] + hkv * p.vs[1], p.Lk, p.vs[2], p.Dv);
+    auto load4 = [](__amdgpu_buffer_rsrc_t r, std::uint32_t off) {
+        return __builtin_bit_cast(float4_t, __builtin_amdgcn_raw_buffer_load_b128(r, static_cast<int>(off), 0, 0));
+    };
+    // (rows past the end come back as zeros; elements past the head size are kept out by an offset beyond the extent)
+    float4_t qf[QB][DC], kf[KB][DC], vf[KB][4][VC];
+    {
+        const auto qr = rsrc_of(p.q + b * p.qs[0] + h * p.qs[1], p.Lq, p.qs[2], p.D);
+#pragma unroll
+        for (int qb = 0; qb < QB; ++qb)
+#pragma unroll
+            for (int c = 0; c < DC; ++c) {
+                const int row = min(q0 + 16 * qb + l16, p.Lq - 1), d = 16 * c + 4 * g;
+                qf[qb][c] = load4(qr, d < p.D ? static_cast<std::uint32_t>(row * p.qs[2] + d) * 4u : kOutOfRange);
+            }
+    }
+    auto load_k = [&](int j0) {
+#pragma unroll
+        for (int kb = 0; kb < KB; ++kb)
+#pragma unroll
+            for (int c = 0; c < DC; ++c) {
+                const int key = j0 + 16 * kb + l16, d = 16 * c + 4 * g;
+                kf[kb][c] = load4(kr, d < p.D && key < p.Lk ? static_cast<std::uint32_t>(key * p.ks[2] + d) * 4u : kOutOfRange);
+            }
+    };
+    auto load_v = [&](int j0) {
+#pragma unroll
+        for (int kb = 0; kb < KB; ++kb)
+#pragma unroll
+            for (int t = 0; t < 4; ++t)
+#pragma unroll
+                for (int c = 0; c < VC; ++c) {
+                    const int key = j0 + 16 * kb + M::row(g, t), d = 64 * c + 4 * l16;
+                    vf[kb][t][c] = load4(vr, d < p.Dv && key < p.Lk ? static_cast<std::uint32_t>(key * p.vs[2] + d) * 4u : kOutOfRange);
+                }
+    };
+
+    vec o[QB][VC][4];
+    Acc m[QB], l[QB];
+#pragma unroll
+    for (int qb = 0; qb < QB; ++qb) {
+        m[qb] = -INFINITY;
+        l[qb] = 0;
+#pragma unroll
+        for (int c = 0; c < VC; ++c)
+#pragma unroll
+            for (int e = 0; e < 4; ++e) o[qb][c][e] = vec{0, 0, 0, 0};
+    }
+    const int keys = p.is_causal ? min(p.Lk, q0 + 16 * QB) : p.Lk;
+    const float scale = static_cast<float>(p.scale);         // (already rounded to fp32 by the caller, so this is exact)
+    // 32 keys of more than 128 elements leave no registers for operands ahead of time: they are requested where they are used
+    constexpr bool kAhead = DM <= 128 || sizeof(Acc) == 8;
+    if (kAhead && wave * kTurn < keys) load_k(wave * kTurn);
+    for (int j0 = wave * kTurn; j0 < keys; j0 += kWavesF * kTurn) {
+        // the mask ahead of everything else: a turn that no query of the tile sees is passed over
+        float mk[QB][KB][4];                          // additive values; bool: 0 where attended, -inf elsewhere
+        if constexpr (kMask != 0) {
+            bool any = false;
+#pragma unroll
+            for (int qb = 0; qb < QB; ++qb) {
+                const long mrow = b * p.ms[0] + h * p.ms[1] + static_cast<long>(min(q0 + 16 * qb + l16, p.Lq - 1)) * p.ms[2];
+#pragma unroll
+                for (int kb = 0; kb < KB; ++kb)
+#pragma unroll
+                    for (int r = 0; r < 4; ++r) {
+                        const long at = mrow + static_cast<long>(min(j0 + 16 * kb + M::row(g, r), p.Lk - 1)) * p.ms[3];
+                        if constexpr (kMask == 1) mk[qb][kb][r] = static_cast<const unsigned char*>(p.mask)[at] != 0 ? 0.0f : -INFINITY;
+                        else                      mk[qb][kb][r] = static_cast<const float*>(p.mask)[at];
+                        any = any || mk[qb][kb][r] != -INFINITY;
+                    }
+            }
+            if (__builtin_amdgcn_ballot_w64(any) == 0) {
+                if (kAhead && j0 + kWavesF * kTurn < keys) load_k(j0 + kWavesF * kTurn);
+                continue;
+            }
+        }
+        if constexpr (kAhead) load_v(j0);
+        else                  load_k(j0);
+        vec s[QB][KB];
+#pragma unroll
+        for (int qb = 0; qb < QB; ++qb)
+#pragma unroll
+            for (int kb = 0; kb < KB; ++kb) s[qb][kb] = vec{0, 0, 0, 0};
+#pragma unroll
+        for (int c = 0; c < DC; ++c)
+#pragma unroll
+            for (int e = 0; e < 4; ++e)
+#pragma unroll
+                for (int kb = 0; kb < KB; ++kb)
+#pragma unroll
+                    for (int qb = 0; qb < QB; ++qb) s[qb][kb] = M::run(kf[kb][c][e], qf[qb][c][e], s[qb][kb]);
+        if (kAhead && j0 + kWavesF * kTurn < keys) load_k(j0 + kWavesF * kTurn);
+        Acc pr[QB][KB][4];
+#pragma unroll
+        for (int qb = 0; qb < QB; ++qb) {
+            const int i = q0 + 16 * qb + l16;
+            float x[KB][4], mx = -INFINITY;
+#pragma unroll
+            for (int kb = 0; kb < KB; ++kb)
+#pragma unroll
+                for (int r = 0; r < 4; ++r) {
+                    const int j = j0 + 16 * kb + M::row(g, r);
+                    float y = static_cast<float>(s[qb][kb][r]) * scale;
+                    if constexpr (kMask != 0) y += mk[qb][kb][r];       // (bool: + 0 or - inf)
+                    if (j >= p.Lk || (p.is_causal && j > i)) y = -INFINITY;
+                    x[kb][r] = y;
+                    mx = fmaxf(mx, y);
+                }
+            mx = fmaxf(mx, __shfl_xor(mx, 16, 64));
+            mx = fmaxf(mx, __shfl_xor(mx, 32, 64));
+            const Acc m_new = static_cast<Acc>(mx) > m[qb] ? static_cast<Acc>(mx) : m[qb];
+            const Acc ref = m_new == -INFINITY ? static_cast<Acc>(0) : m_new;            // no visible key yet: any reference but -inf
+            if (__builtin_amdgcn_ballot_w64(m_new != m[qb]) != 0) {
+                const Acc f = M::exp_of(m[qb] - ref);
+                l[qb] *= f;
+#pragma unroll
+                for (int c = 0; c < VC; ++c)
+#pragma unroll
+                    for (int e = 0; e < 4; ++e) o[qb][c][e] *= f;
+                m[qb] = m_new;
+            }
+#pragma unroll
+            for (int kb = 0; kb < KB; ++kb)
+#pragma unroll
+                for (int r = 0; r < 4; ++r) {
+                    pr[qb][kb][r] = M::exp_of(static_cast<Acc>(x[kb][r]) - ref);
+                    l[qb] += pr[qb][kb][r];
+                }
+        }
+        if constexpr (!kAhead) load_v(j0);
+#pragma unroll
+        for (int kb = 0; kb < KB; ++kb)
+#pragma unroll
+            for (int t = 0; t < 4; ++t)
+#pragma unroll
+                for (int c = 0; c < VC; ++c)
+#pragma unroll
+                    for (int e = 0; e < 4; ++e)
+#pragma unroll
+                        for (int qb = 0; qb < QB; ++qb) o[qb][c][e] = M::run(vf[kb][t][c][e], pr[qb][kb][t], o[qb][c][e]);
+    }
+
+    // the waves meet
+#pragma unroll
+    for (int qb = 0; qb < QB; ++qb) {
+        l[qb] += __shfl_xor(l[qb], 16, 64);
+        l[qb] += __shfl_xor(l[qb], 32, 64);
+        if (g == 0) {
+            m_part[wave][qb][l16] = m[qb];
+            l_part[wave][qb][l16] = l[qb];
+        }
+#pragma unroll
+        for (int c = 0; c < VC; ++c)
+#pragma unroll
+            for (int e = 0; e < 4; ++e)
+#pragma unroll
+                for (int r = 0; r < 4; ++r) o_part[wave][((qb * VC + c) * 4 + e) * 256 + r * 64 + lane] = o[qb][c][e][r];
+    }
+    __syncthreads();
+    for (int item = wave; item < QB * VC * 4; item += kWavesF) {
+        const int r = item & 3, c = (item >> 2) % VC, qb = (item >> 2) / VC;
+        const int i = q0 + 16 * qb + l16, dv = 64 * c + 4 * M::row(g, r);
+        Acc mm = m_part[0][qb][l16];
+#pragma unroll
+        for (int w = 1; w < kWavesF; ++w) mm = m_part[w][qb][l16] > mm ? m_part[w][qb][l16] : mm;
+        const Acc ref = mm == -INFINITY ? static_cast<Acc>(0) : mm;
+        Acc sum = 0, val[4] = {0, 0, 0, 0};
+#pragma unroll
+        for (int w = 0; w < kWavesF; ++w) {
+            const Acc f = M::exp_of(m_part[w][qb][l16] - ref);
+            sum += f * l_part[w][qb][l16];
+#pragma unroll
+            for (int e = 0; e < 4; ++e) val[e] += f * o_part[w][((qb * VC + c) * 4 + e) * 256 + r * 64 + lane];
+        }
+        if (i >= p.Lq) continue;
+        const long row = (static_cast<long>(b) * p.Hq + h) * p.Lq + i;
+        if (dv < p.Dv) {
+            float4_t y;
+#pragma unroll
+            for (int e = 0; e < 4; ++e) y[e] = static_cast<float>(val[e] / sum);
+            *reinterpret_cast<float4_t*>(p.out + row * p.Dv + dv) = y;
+        }
+        if (p.lse != nullptr && c == 0 && r == 0 && g == 0) p.lse[row] = static_cast<float>(static_cast<double>(mm) + log(static_cast<double>(sum)));
+    }
+}
+
+template <typename Acc, int DM, int QB, int KB>
+void launch_form(F32Params p, const paras_sdpa_args& a, hipStream_t s) {
+    p.q_tiles = static_cast<int>((a.Lq + 16 * QB - 1) / (16 * QB));
+    const dim3 g(p.q_tiles, static_cast<unsigned>(a.Hq), static_cast<unsigned>(a.B)), t(kWavesF * 64);
+    if (a.mask_kind == 0)      hipLaunchKernelGGL((sdpa_f32_kernel<Acc, DM, QB, KB, 0>), g, t, 0, s, p);
+    else if (a.mask_kind == 1) hipLaunchKernelGGL((sdpa_f32_kernel<Acc, DM, QB, KB, 1>), g, t, 0, s, p);
+    else                       hipLaunchKernelGGL((sdpa_f32_kernel<Acc, DM, QB, KB, 2>), g, t, 0, s, p);
+}
+template <typename Acc, int DM>
+void launch_dm(const F32Params& p, const paras_sdpa_args& a, hipStream_t s) {
+    if constexpr (sizeof(Acc) == 8) {
+        // up to 64 keys turns of 16 give all four waves some; at 256 elements that is also all the registers hold
+        if constexpr (DM <= 128) {
+            if (a.Lk > 64) return launch_form<Acc, DM, 1, 2>(p, a, s);
+        }
+        launch_form<Acc, DM, 1, 1>(p, a, s);
+    } else {
+        // 32 queries per workgroup read K and V half as often; at 256 elements the registers do not hold them, and
+        // below two workgroups per CU 16 queries spread the work better
+        if constexpr (DM <= 128) {
+            if ((a.Lq + 31) / 32 * a.Hq * a.B >= 512) return launch_form<Acc, DM, 2, 2>(p, a, s);
+        }
+        launch_form<Acc, DM, 1, 2>(p, a, s);
+    }
+}
+
+}  // namespace
+
+bool f32_supported(const paras_sdpa_args& a) {
+    if (a.dtype != PARAS_F32) return false;
+    if (a.D < 4 || a.Dv < 4 || a.D > 256 || a.Dv > 256 || a.D % 4 != 0 || a.Dv % 4 != 0 || a.Lq < 1 || a.Lk < 1) return false;
+    if (a.Hq > 65535 || a.B > 65535 || a.Lq >= (1L << 30) || a.Lk >= (1L << 30)) return false;
+    if (a.q_strides[2] < 0 || a.k_strides[2] < 0 || a.v_strides[2] < 0) return false;
+    const long lim = (1L << 29) - 1;                       // elements: byte offsets below 2^31
+    return (a.Lq - 1) * a.q_strides[2] + a.D <= lim && (a.Lk - 1) * a.k_strides[2] + a.D <= lim && (a.Lk - 1) * a.v_strides[2] + a.Dv <= lim &&
+           (reinterpret_cast<uintptr_t>(a.out) & 15) == 0;
+}
+
+int launch_f32(const paras_sdpa_args& a, bool accumulate_f64, hipStream_t s) {
+    F32Params p{};
+    p.q = static_cast<const float*>(a.q); p.k = static_cast<const float*>(a.k); p.v = static_cast<const float*>(a.v);
+    p.out = static_cast<float*>(a.out); p.lse = a.lse; p.mask = a.mask;
+    p.is_causal = a.is_causal;
+    p.Hq = static_cast<int>(a.Hq); p.Hkv = static_cast<int>(a.Hkv);
+    p.Lq = static_cast<int>(a.Lq); p.Lk = static_cast<int>(a.Lk); p.D = static_cast<int>(a.D); p.Dv = static_cast<int>(a.Dv);
+    for (int i = 0; i < 3; ++i) { p.qs[i] = a.q_strides[i]; p.ks[i] = a.k_strides[i]; p.vs[i] = a.v_strides[i]; }
+    for (int i = 0; i < 4; ++i) p.ms[i] = a.mask_strides[i];
+    p.scale = a.scale;
+    const long dm = a.D > a.Dv ? a.D : a.Dv;
+    if (accumulate_f64) {
+        if (dm <= 64)       launch_dm<double, 64>(p, a, s);
+        else if (dm <= 128) launch_dm<double, 128>(p, a, s);
+        else                launch_dm<double, 256>(p, a, s);
+    } else {
+        if (dm <= 64)       launch_dm<float, 64>(p, a, s);
+        else if (dm <= 128) launch_dm<float, 128>(p, a, s);
+        else                launch_dm<float, 256>(p, a, s);
+    }
+    PARAS_HIP_TRY(hipGetLastError());
+    return PARAS_OK;
+}
+
+}  // namespace paras

@@ -12,7 +12,8 @@
 //   p  = T(exp(s - max) / sum exp)       _softmax, fp64 (pointwise_ops.cpp:954-977)
 //   o  = T(sum_j p*v)                    second bmm
 // All arithmetic is fp64 (78 TFLOP/s of it on this part; this path serves
-// small and unusual shapes, the large regular ones go to the MFMA kernels).
+// small and unusual shapes, the large regular ones go to the MFMA kernels, and
+// fp32 problems without returned weights to sdpa_f32.hip).
 //
 // One 256-thread workgroup per (batch, head, query) row.  Scores are not
 // stored: pass 1 finds the row max, pass 2 the denominator, pass 3 recomputes
@@ -153,6 +154,7 @@ __global__ __launch_bounds__(kBlock) void sdpa_generic_kernel(const GenericParam
 size_t generic_workspace(const paras_sdpa_args&) { return 0; }
 
 int launch_generic(const paras_sdpa_args& a, void*, hipStream_t s) {
+    if (a.attn == nullptr && f32_supported(a)) return launch_f32(a, /*accumulate_f64=*/true, s);
     if (a.D > kMaxD || a.Dv > kMaxD)
         return fail(PARAS_ERR_UNSUPPORTED, "paras sdpa: head dim %lld/%lld exceeds %d", (long long)a.D,
                     (long long)a.Dv, kMaxD);

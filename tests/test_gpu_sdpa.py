@@ -754,3 +754,40 @@ def test_composed_route_fp64_and_wide_16_bit_heads():
     assert name == "composed"
     want, wattn = O.sdpa_math(q, k, v, is_causal=True, gemm="aten")
     assert max_abs(out, want) <= ABS_16BIT and max_abs(attn, wattn) <= ABS_16BIT
+
+
+@pytest.mark.parametrize("kind", ["none", "causal", "bool", "additive"])
+@pytest.mark.parametrize("B,Hq,Hkv,Lq,Lk,D,Dv", [(1, 2, 1, 1, 1, 4, 4), (2, 4, 2, 17, 33, 64, 64), (1, 2, 2, 16, 64, 128, 128), (1, 3, 1, 50, 65, 40, 72),
+                                                 (1, 2, 2, 15, 130, 256, 256), (2, 8, 2, 300, 300, 64, 64), (1, 2, 1, 520, 700, 128, 96),
+                                                 (1, 1, 1, 260, 1000, 256, 200), (1, 8, 8, 2100, 129, 64, 128)])
+def test_fp32_one_pass_kernel(B, Hq, Hkv, Lq, Lk, D, Dv, kind):
+    """The fp32 kernel of the general and the composed route (fp64 and fp32 accumulation) against fp64: query and
+    key tiles cut short, every padded head size, grouped heads, each mask kind, a whole turn of keys masked out, a
+    query that sees no key (NaN, as in the reference), the log-sum-exp, and strided operands."""
+    torch.manual_seed(Lq + Lk + D)
+    q = torch.randn(B, Lq, Hq, D).transpose(1, 2)
+    k, v = torch.randn(B, Lk, Hkv, D).transpose(1, 2), torch.randn(B, Hkv, Lk, Dv)
+    mask, kw = None, {}
+    if kind == "causal":
+        kw = dict(is_causal=True)
+        mask = torch.zeros(Lq, Lk).masked_fill(torch.ones(Lq, Lk).tril() == 0, -math.inf)
+    elif kind == "bool":
+        keep = torch.rand(B, 1, Lq, Lk) < 0.7
+        keep[..., 64:192] = False
+        keep[..., 0] = True
+        if Lq > 1:
+            keep[0, 0, Lq // 2] = False
+        kw, mask = dict(mask=keep), torch.zeros(B, 1, Lq, Lk).masked_fill(~keep, -math.inf)
+    elif kind == "additive":
+        mask = torch.randn(1, Hq, 1, Lk)
+        kw = dict(mask=mask)
+    out, _, lse, _ = run(q, k, v, want_lse=True, **kw)
+    s = q.double() @ k.double().repeat_interleave(Hq // Hkv, 1).transpose(-1, -2) / math.sqrt(D)
+    if mask is not None:
+        s = s + mask.double()
+    want = s.softmax(-1) @ v.double().repeat_interleave(Hq // Hkv, 1)
+    ok = ~want.isnan()
+    assert torch.equal(out.cpu().isnan(), ~ok)
+    assert (out.cpu().double()[ok] - want[ok]).abs().max().item() <= 3e-6 * want[ok].abs().max().item()
+    want_lse = torch.logsumexp(s, -1)
+    assert torch.allclose(lse.cpu().double()[want_lse.isfinite()], want_lse[want_lse.isfinite()], rtol=1e-6, atol=2e-6)
