@@ -20,6 +20,7 @@
 #include "kernels/gemm_f32_host.h"
 #include "kernels/gemm_flex_host.h"
 #include "kernels/gemm_tile.h"
+#include "kernels/stream_rows.h"
 #include "paras_hip.h"
 
 namespace paras {
@@ -41,26 +42,84 @@ struct DenseParams {
                                 // result (row of a, row of b) belongs at c[row of b][row of a], and the addend likewise
 };
 
-// ---- few rows (M <= 128): the decode-time projections.  The product is bound by streaming the
-// weights once, so there is no tile and no LDS staging: a workgroup owns 16 weight rows, its eight
-// waves split the contraction (pieces of 64 dealt round-robin, so the eight read adjacent 128-byte
-// lines of each row), every wave feeds v_mfma_f32_16x16x32 straight from global memory (weights
-// as the row operand, with plain loads: non-temporal ones measured 5-18 % slower here, each
-// 128-byte line being touched by two instructions; the few activation rows from L2), and the eight partial
-// results meet in LDS in wave order.  Lane l of a 16x16 result holds activation row l%16 and
-// weight rows 4*(l/16) .. +3: four adjacent outputs, stored as one 8-byte piece when aligned.
-template <typename T> struct Mma16;
-template <> struct Mma16<bf16_t> {
-    __device__ static __forceinline__ float4_t run(u32x4 a, u32x4 b, float4_t c) {
-        return __builtin_amdgcn_mfma_f32_16x16x32_bf16(__builtin_bit_cast(bf16x8, a), __builtin_bit_cast(bf16x8, b), c, 0, 0, 0);
-    }
-};
-template <> struct Mma16<f16_t> {
-    __device__ static __forceinline__ float4_t run(u32x4 a, u32x4 b, float4_t c) {
-        return __builtin_amdgcn_mfma_f32_16x16x32_f16(__builtin_bit_cast(f16x8, a), __builtin_bit_cast(f16x8, b), c, 0, 0, 0);
-    }
-};
+// ---- up to 32 rows: the decode-time projections, bound by streaming the weights once.  A workgroup owns 16 NBG
+// weight rows and its eight waves split the contraction (stream_rows.h); 8 XQ activation rows at most.
+using stream::Mma16;
 
+template <typename T>
+__device__ __forceinline__ void few_rows_store(const DenseParams& p, std::uint16_t* C, const std::uint16_t* ADD, bool vec_ok, long row, long col, float4_t t) {
+    using El = Elem<T>;
+    if (row >= p.M) return;
+    if (p.swapped) {        // `row` is a column of the caller's result and `col + r` a row of it
+#pragma unroll
+        for (int r = 0; r < 4; ++r) {
+            if (col + r >= p.N) continue;
+            float v = p.alpha * t[r];
+            if (ADD) v = fmaf(p.beta, El::to_f32(ADD[(col + r) * p.ld_add + row]), v);
+            C[(col + r) * p.ldc + row] = El::from_f32(v);
+        }
+        return;
+    }
+    std::uint16_t o16[4];
+#pragma unroll
+    for (int r = 0; r < 4; ++r) {
+        float v = p.alpha * t[r];
+        if (ADD && col + r < p.N) v = fmaf(p.beta, El::to_f32(ADD[row * p.ld_add + col + r]), v);
+        o16[r] = El::from_f32(v);
+    }
+    if (vec_ok && col + 3 < p.N) {
+        u32x2 w2;
+        w2[0] = o16[0] | (static_cast<std::uint32_t>(o16[1]) << 16);
+        w2[1] = o16[2] | (static_cast<std::uint32_t>(o16[3]) << 16);
+        *reinterpret_cast<u32x2*>(C + row * p.ldc + col) = w2;
+    } else {
+#pragma unroll
+        for (int r = 0; r < 4; ++r)
+            if (col + r < p.N) C[row * p.ldc + col + r] = o16[r];
+    }
+}
+__device__ __forceinline__ bool few_rows_vec(const DenseParams& p) {
+    return (p.ldc % 4 == 0) && (p.sc % 4 == 0) && ((reinterpret_cast<uintptr_t>(p.c) & 7) == 0);
+}
+
+template <typename T, int NBG, int XQ>
+__global__ __launch_bounds__(stream::kThreads, 4) void stream_gemm_nt_kernel(const DenseParams p) {
+    using S = stream::Shape<1, NBG, XQ>;
+    constexpr int MB = S::kXBlocks;
+    __shared__ __attribute__((aligned(1024))) std::uint16_t lds[S::kLdsElems];
+    const long bidx = blockIdx.y;
+    const std::uint16_t* A = p.a + bidx * p.sa;
+    const int lane = threadIdx.x & 63;
+    const long n0 = static_cast<long>(blockIdx.x) * (16 * NBG);
+    const std::uint16_t* const w[1] = {p.b + bidx * p.sb + n0 * p.ldb};
+    std::uint32_t x_off[XQ];
+#pragma unroll
+    for (int q = 0; q < XQ; ++q) {
+        long xrow = q * 8 + (lane >> 3);
+        if (xrow >= p.M) xrow = p.M - 1;                    // clamped rows are computed but never stored
+        x_off[q] = static_cast<std::uint32_t>(xrow * p.lda * 2);
+    }
+    const long step = static_cast<long>(gridDim.x) * (16 * NBG);
+    const int count = static_cast<int>((p.N - n0 + step - 1) / step);
+    stream::products<T, 1, NBG, XQ>(w, p.ldb, p.N - n0, step, count, p.K, A, ((p.M - 1) * p.lda + p.K) * 2, x_off, lds,
+                                    [&](int j, const float4_t (&acc)[NBG][MB]) __attribute__((always_inline)) {
+        stream::share<NBG, MB>(lds, acc);
+        const int blk = stream::wave_id();                  // wave w finishes result block w
+        if (blk < NBG * MB) {
+            const float4_t t = stream::sum_of<NBG, MB>(lds, blk / MB, blk % MB);
+            if (XQ > 1 || (lane & 15) < 8)
+                few_rows_store<T>(p, p.c + bidx * p.sc, p.add ? p.add + bidx * p.sadd : nullptr, few_rows_vec(p), (blk % MB) * 16 + (lane & 15),
+                                  n0 + j * step + (blk / MB) * 16 + 4 * (lane >> 4), t);
+        }
+        lds_barrier();                                      // the LDS is free for the next block
+    });
+}
+
+// ---- 33 to 128 rows without a workspace: the same split, but with this many activation rows per weight row a trip
+// through LDS for each would cost more than it saves, so every wave feeds its MFMAs straight from memory (weights
+// as the row operand, with plain loads: non-temporal ones measured 5-18 % slower, each 128-byte line being touched by two
+// instructions; the activation rows from L2), and the eight partial results meet in LDS in wave order.  Lane l of
+// a 16x16 result holds activation row l%16 and weight rows 4*(l/16) .. +3.
 constexpr int kSkinnyWaves = 8;
 constexpr int kSkinnyMaxM = 128;
 constexpr int kFewRowsM = 32;            // with a workspace at hand the tile kernel with the contraction in parts takes over from here
@@ -155,9 +214,8 @@ __global__ __launch_bounds__(kSkinnyWaves * 64) void skinny_gemm_nt_kernel(const
     // wave w finishes result blocks w, w + 8, ...
     std::uint16_t* C = p.c + bidx * p.sc;
     const std::uint16_t* ADD = p.add ? p.add + bidx * p.sadd : nullptr;
-    const bool vec_ok = (p.ldc % 4 == 0) && (p.sc % 4 == 0) && ((reinterpret_cast<uintptr_t>(p.c) & 7) == 0);
+    const bool vec_ok = few_rows_vec(p);
     for (int blk = wave; blk < NB * MB; blk += kSkinnyWaves) {
-        const int nb = blk / MB, mb = blk % MB;
         float4_t t = part[0][blk][lane];
 #pragma unroll
         for (int w = 1; w < kSkinnyWaves; ++w) {
@@ -165,36 +223,7 @@ __global__ __launch_bounds__(kSkinnyWaves * 64) void skinny_gemm_nt_kernel(const
 #pragma unroll
             for (int r = 0; r < 4; ++r) t[r] += o[r];
         }
-        const long row = mb * 16 + r16;
-        const long col = n0 + nb * 16 + 4 * kg;
-        if (row >= p.M) continue;
-        if (p.swapped) {        // `row` is a column of the caller's result and `col + r` a row of it
-#pragma unroll
-            for (int r = 0; r < 4; ++r) {
-                if (col + r >= p.N) continue;
-                float v = p.alpha * t[r];
-                if (ADD) v = fmaf(p.beta, El::to_f32(ADD[(col + r) * p.ld_add + row]), v);
-                C[(col + r) * p.ldc + row] = El::from_f32(v);
-            }
-            continue;
-        }
-        std::uint16_t o16[4];
-#pragma unroll
-        for (int r = 0; r < 4; ++r) {
-            float v = p.alpha * t[r];
-            if (ADD && col + r < p.N) v = fmaf(p.beta, El::to_f32(ADD[row * p.ld_add + col + r]), v);
-            o16[r] = El::from_f32(v);
-        }
-        if (vec_ok && col + 3 < p.N) {
-            u32x2 w2;
-            w2[0] = o16[0] | (static_cast<std::uint32_t>(o16[1]) << 16);
-            w2[1] = o16[2] | (static_cast<std::uint32_t>(o16[3]) << 16);
-            *reinterpret_cast<u32x2*>(C + row * p.ldc + col) = w2;
-        } else {
-#pragma unroll
-            for (int r = 0; r < 4; ++r)
-                if (col + r < p.N) C[row * p.ldc + col + r] = o16[r];
-        }
+        few_rows_store<T>(p, C, ADD, vec_ok, (blk % MB) * 16 + r16, n0 + (blk / MB) * 16 + 4 * kg, t);
     }
 }
 
@@ -207,9 +236,11 @@ void launch_skinny(const DenseParams& p, long batch, hipStream_t s) {
     const dim3 g1(static_cast<unsigned>((p.N + 15) / 16), static_cast<unsigned>(batch));
     const dim3 g2(static_cast<unsigned>((p.N + 31) / 32), static_cast<unsigned>(batch));
     const bool two = mb > 1 && static_cast<long>(g2.x) * batch >= 256;
-    if (mb <= 1)      hipLaunchKernelGGL((skinny_gemm_nt_kernel<T, 1, 1>), g1, block, 0, s, p);
-    else if (mb <= 2) { if (two) hipLaunchKernelGGL((skinny_gemm_nt_kernel<T, 2, 2>), g2, block, 0, s, p);
-                        else     hipLaunchKernelGGL((skinny_gemm_nt_kernel<T, 2, 1>), g1, block, 0, s, p); }
+    const dim3 s1(stream::grid(p.N, 1, batch), static_cast<unsigned>(batch)), s2(stream::grid(p.N, 2, batch), static_cast<unsigned>(batch));
+    if (p.M <= 8)     hipLaunchKernelGGL((stream_gemm_nt_kernel<T, 1, 1>), s1, block, 0, s, p);
+    else if (mb <= 1) hipLaunchKernelGGL((stream_gemm_nt_kernel<T, 1, 2>), s1, block, 0, s, p);
+    else if (mb <= 2) { if (two) hipLaunchKernelGGL((stream_gemm_nt_kernel<T, 2, 4>), s2, block, 0, s, p);
+                        else     hipLaunchKernelGGL((stream_gemm_nt_kernel<T, 1, 4>), s1, block, 0, s, p); }
     else if (mb <= 4) { if (two) hipLaunchKernelGGL((skinny_gemm_nt_kernel<T, 4, 2>), g2, block, 0, s, p);
                         else     hipLaunchKernelGGL((skinny_gemm_nt_kernel<T, 4, 1>), g1, block, 0, s, p); }
     else              { if (two) hipLaunchKernelGGL((skinny_gemm_nt_kernel<T, 8, 2>), g2, block, 0, s, p);
@@ -557,8 +588,6 @@ Route route_of(const paras_gemm_args& g, bool may_split, bool nt_api, int causal
             }
             r.splits = splitk_plan(g.M, g.N, g.K, g.batch, &r.pieces);
         }
-    } else if (nt64 && may_split && g.M <= kFewRowsM) {
-        r.splits = splitk_plan(g.M, g.N, g.K, g.batch, &r.pieces);
     }
     if (r.splits >= 2) {
         r.kind = Route::FewRowsParts;

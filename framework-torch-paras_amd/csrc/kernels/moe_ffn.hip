@@ -33,6 +33,7 @@
 #include "core/device_math.h"
 #include "core/status.h"
 #include "kernels/gemm_tile.h"
+#include "kernels/stream_rows.h"
 #include "kernels/swiglu_math.h"
 
 namespace paras {
@@ -47,6 +48,7 @@ struct FfnGemmParams {
     std::uint16_t* c;           // [R, N]
     const long* order;          // gather index (routed row -> flat (token, slot)); null = direct rows
     const long* offsets;        // [E+1]
+    long a_bytes;               // extent of a (few-row kernels)
     long K, N, Nw, R;           // contraction, output columns, weight rows per expert, routed rows
     int E, k;
     int mt_total;               // upper bound on m-tiles
@@ -425,134 +427,80 @@ __global__ __launch_bounds__(quad16::kThreads, 1) void grouped_gemm_quad16_kerne
 // ---- few rows per expert (decode-time batches): the layer is bound by streaming every active
 // expert's weights once, which 128-row tiles with a handful of live rows do at half the memory
 // rate (and a single token, two active experts, at a fifth of it: its down-projection is 32
-// workgroups).  Here, as in the dense few-row kernel: a workgroup owns 16 weight rows of one expert
-// (for the gate-up GEMM the 16 gate rows and the 16 up rows of the same columns), its eight waves
-// split the contraction in pieces of 64 and feed v_mfma_f32_16x16x32 straight from global memory
-// (weights as the row operand; the expert's few routed rows, from L2, as the other), the eight
-// partial results meet in LDS in wave order.  An expert's rows are taken MB x 16 at a time, so any
-// count works (the weights of a second pass come from L2); experts without rows return at once.
-template <typename T> struct Mma16x16;
-template <> struct Mma16x16<bf16_t> {
-    __device__ static __forceinline__ float4_t run(u32x4 a, u32x4 b, float4_t c) {
-        return __builtin_amdgcn_mfma_f32_16x16x32_bf16(__builtin_bit_cast(bf16x8, a), __builtin_bit_cast(bf16x8, b), c, 0, 0, 0);
-    }
-};
-template <> struct Mma16x16<f16_t> {
-    __device__ static __forceinline__ float4_t run(u32x4 a, u32x4 b, float4_t c) {
-        return __builtin_amdgcn_mfma_f32_16x16x32_f16(__builtin_bit_cast(f16x8, a), __builtin_bit_cast(f16x8, b), c, 0, 0, 0);
-    }
-};
+// workgroups).  A workgroup owns 16 weight rows of one expert (for the gate-up GEMM the 16 gate rows and
+// the 16 up rows of the same columns) and its eight waves split the contraction (stream_rows.h).  An expert's
+// rows are taken up to 8, 16 or 32 at a time, whichever holds them, so any count works (the weights of a second
+// pass come from L2); experts without rows return at once.
+// (The SwiGLU of a workgroup's blocks waits until its last one: its fp64 tier would not fit into the registers beside
+// the requests under way.  Until then the sums stay in LDS, kFewBlocks blocks of them.)
+constexpr int kFewBlocks = 2;
 
-constexpr int kFewWaves = 8;
-
-template <typename T, bool kSwiglu, int MB>
-__global__ __launch_bounds__(kFewWaves * 64) void grouped_few_rows_kernel(const FfnGemmParams p) {
+template <typename T, bool kSwiglu, int XQ>
+__device__ __forceinline__ void few_rows(const FfnGemmParams& p, int e, long row_lo, long row_hi, std::uint16_t* lds, float4_t* kept) {
     using El = Elem<T>;
-    constexpr int NB = kSwiglu ? 2 : 1;                 // weight blocks: gate and up, or one
-    __shared__ float4_t part[kFewWaves][NB * MB][64];
-    const int e = blockIdx.y;
-    const long row_lo = p.offsets[e], row_hi = p.offsets[e + 1];
-    if (row_lo >= row_hi) return;                        // (uniform)
-    const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
-    const int r16 = lane & 15, kg = lane >> 4;
-    const long n0 = static_cast<long>(blockIdx.x) * 16;
-    long wrow = n0 + r16;
-    if (wrow >= p.Nw) wrow = p.Nw - 1;                   // clamped rows are computed but never stored
-    const std::uint16_t* wp[NB];
-    wp[0] = p.b + (static_cast<long>(e) * p.Nw + wrow) * p.K + kg * 16;
-    if constexpr (kSwiglu) wp[1] = p.b2 + (static_cast<long>(e) * p.Nw + wrow) * p.K + kg * 16;
-    const long pieces = p.K / 64;
-    // this wave's pieces of the contraction: wave, wave + 8, ...
-    const long mine = pieces > wave ? (pieces - wave + kFewWaves - 1) / kFewWaves : 0;
-
-    for (long chunk = row_lo; chunk < row_hi; chunk += MB * 16) {
-        const std::uint16_t* xp[MB];
+    using S = stream::Shape<(kSwiglu ? 2 : 1), 1, XQ>;
+    constexpr int NB = S::kBlocks, MB = S::kXBlocks;
+    const int lane = threadIdx.x & 63;
+    const long n0 = static_cast<long>(blockIdx.x) * 16, step = static_cast<long>(gridDim.x) * 16;
+    const int count = static_cast<int>((p.Nw - n0 + step - 1) / step);
+    const long first = (static_cast<long>(e) * p.Nw + n0) * p.K;
+    const std::uint16_t* w[NB];
+    w[0] = p.b + first;
+    if constexpr (kSwiglu) w[1] = p.b2 + first;
+    for (long chunk = row_lo; chunk < row_hi; chunk += XQ * 8) {
+        std::uint32_t x_off[XQ];
 #pragma unroll
-        for (int mb = 0; mb < MB; ++mb) {
-            long prow = chunk + mb * 16 + r16;
+        for (int q = 0; q < XQ; ++q) {
+            long prow = chunk + q * 8 + (lane >> 3);
             if (prow >= row_hi) prow = row_hi - 1;
             const long src = p.order ? static_cast<long>((static_cast<unsigned long long>(static_cast<unsigned>(p.order[prow])) * p.div_m) >> p.div_s) : prow;
-            xp[mb] = p.a + src * p.K + kg * 16;
+            x_off[q] = static_cast<std::uint32_t>(src * p.K * 2);
         }
-        float4_t acc[NB][MB];
-#pragma unroll
-        for (int nb = 0; nb < NB; ++nb)
-#pragma unroll
-            for (int mb = 0; mb < MB; ++mb) acc[nb][mb] = float4_t{0.f, 0.f, 0.f, 0.f};
-        // two pieces per trip, every load of the trip requested before its first MFMA; lane group kg
-        // supplies elements 16 kg .. + 7 of a piece to the first MFMA and the next eight to the
-        // second (any assignment works as long as both operands use the same one)
-        long t = 0;
-        for (; t + 2 <= mine; t += 2) {
-            u32x4 wv[2][2][NB], xv[2][2][MB];
-#pragma unroll
-            for (int u = 0; u < 2; ++u)
-#pragma unroll
-                for (int h = 0; h < 2; ++h) {
-                    const long kk = (wave + (t + u) * kFewWaves) * 64 + h * 8;
-#pragma unroll
-                    for (int nb = 0; nb < NB; ++nb) wv[u][h][nb] = load16(wp[nb] + kk);
-#pragma unroll
-                    for (int mb = 0; mb < MB; ++mb) xv[u][h][mb] = load16(xp[mb] + kk);
-                }
-#pragma unroll
-            for (int u = 0; u < 2; ++u)
-#pragma unroll
-                for (int h = 0; h < 2; ++h)
-#pragma unroll
-                    for (int mb = 0; mb < MB; ++mb)
-#pragma unroll
-                        for (int nb = 0; nb < NB; ++nb) acc[nb][mb] = Mma16x16<T>::run(wv[u][h][nb], xv[u][h][mb], acc[nb][mb]);
-        }
-        for (; t < mine; ++t) {
-#pragma unroll
-            for (int h = 0; h < 2; ++h) {
-                const long kk = (wave + t * kFewWaves) * 64 + h * 8;
-                u32x4 wv[NB];
-#pragma unroll
-                for (int nb = 0; nb < NB; ++nb) wv[nb] = load16(wp[nb] + kk);
-#pragma unroll
-                for (int mb = 0; mb < MB; ++mb) {
-                    const u32x4 xv = load16(xp[mb] + kk);
-#pragma unroll
-                    for (int nb = 0; nb < NB; ++nb) acc[nb][mb] = Mma16x16<T>::run(wv[nb], xv, acc[nb][mb]);
-                }
-            }
-        }
-#pragma unroll
-        for (int nb = 0; nb < NB; ++nb)
-#pragma unroll
-            for (int mb = 0; mb < MB; ++mb) part[wave][nb * MB + mb][lane] = acc[nb][mb];
-        __syncthreads();
-        // wave w finishes row block w, w + 8, ...: lane l holds routed row l % 16 of the block and the
-        // four weight rows (output columns) 4 (l / 16) .. + 3
-        for (int mb = wave; mb < MB; mb += kFewWaves) {
-            float4_t g = part[0][mb][lane], u = float4_t{0.f, 0.f, 0.f, 0.f};
-            if constexpr (kSwiglu) u = part[0][MB + mb][lane];
-#pragma unroll
-            for (int w = 1; w < kFewWaves; ++w) {
-                const float4_t o = part[w][mb][lane];
-#pragma unroll
-                for (int r = 0; r < 4; ++r) g[r] += o[r];
+        // value r of lane l in row block m of column block j: routed row l % 16 of the row block, column 4 (l / 16) + r
+        auto put = [&](int j, int m, int l, int r, float g, float u) __attribute__((always_inline)) {
+            const long prow = chunk + m * 16 + (l & 15), col = n0 + j * step + 4 * (l >> 4) + r;
+            if (prow >= row_hi || (XQ == 1 && (l & 15) >= 8) || col >= p.N) return;
+            if constexpr (kSwiglu) p.c[prow * p.N + col] = swiglu_from_acc<T>(g, u);
+            else                   p.c[prow * p.N + col] = El::from_f32(g);
+        };
+        stream::products<T, NB, 1, XQ>(w, p.K, p.Nw - n0, step, count, p.K, p.a, p.a_bytes, x_off, lds,
+                                       [&](int j, const float4_t (&acc)[NB][MB]) __attribute__((always_inline)) {
+            stream::share<NB, MB>(lds, acc);
+            const int m = stream::wave_id();             // wave m finishes row block m
+            if (m < MB) {
                 if constexpr (kSwiglu) {
-                    const float4_t o2 = part[w][MB + mb][lane];
 #pragma unroll
-                    for (int r = 0; r < 4; ++r) u[r] += o2[r];
+                    for (int b = 0; b < 2; ++b) kept[((j * MB + m) * 2 + b) * 64 + lane] = stream::sum_of<NB, MB>(lds, b, m);
+                } else {
+                    const float4_t g = stream::sum_of<NB, MB>(lds, 0, m);
+#pragma unroll
+                    for (int r = 0; r < 4; ++r) put(j, m, lane, r, g[r], 0.f);
                 }
             }
-            const long prow = chunk + mb * 16 + r16;
-            const long col = n0 + 4 * kg;
-            if (prow < row_hi) {
-#pragma unroll
-                for (int r = 0; r < 4; ++r) {
-                    if (col + r >= p.N) continue;
-                    if constexpr (kSwiglu) p.c[prow * p.N + col + r] = swiglu_from_acc<T>(g[r], u[r]);
-                    else                   p.c[prow * p.N + col + r] = El::from_f32(g[r]);
-                }
+            lds_barrier();                               // the LDS is free for the next block
+        });
+        if constexpr (kSwiglu) {
+            const float* v = reinterpret_cast<const float*>(kept);
+            for (int i = threadIdx.x; i < count * MB * 256; i += stream::kThreads) {
+                const int jm = i >> 8, in = i & 255;
+                put(jm / MB, jm % MB, in >> 2, in & 3, v[jm * 512 + in], v[jm * 512 + 256 + in]);
             }
+            lds_barrier();                               // the kept sums are free for the next rows
         }
-        __syncthreads();                                 // `part` is free for the next rows
     }
+}
+
+template <typename T, bool kSwiglu>
+__global__ __launch_bounds__(stream::kThreads, 4) void grouped_few_rows_kernel(const FfnGemmParams p) {
+    __shared__ __attribute__((aligned(1024))) std::uint16_t lds[stream::Shape<(kSwiglu ? 2 : 1), 1, 4>::kLdsElems];
+    __shared__ float4_t kept[kSwiglu ? kFewBlocks * 2 * 2 * 64 : 1];
+    const int e = blockIdx.y;
+    const long row_lo = p.offsets[e], row_hi = p.offsets[e + 1];
+    const int rows = __builtin_amdgcn_readfirstlane(static_cast<int>(row_hi - row_lo));
+    if (rows <= 0) return;
+    if (rows <= 8)       few_rows<T, kSwiglu, 1>(p, e, row_lo, row_hi, lds, kept);
+    else if (rows <= 16) few_rows<T, kSwiglu, 2>(p, e, row_lo, row_hi, lds, kept);
+    else                 few_rows<T, kSwiglu, 4>(p, e, row_lo, row_hi, lds, kept);
 }
 
 // out[t, :] = T( sum_slot T( y[inv[t*k+slot], :] * T(w[t, slot]) ) ), 8 columns per lane.
@@ -746,6 +694,10 @@ int run_ffn_few_rows(const void* x, const void* w_gate, const void* w_up, const 
                      const long* order, const long* inv_order, const long* offsets, void* out, void* workspace, long T_,
                      int E, int k, long H, long I, hipStream_t s) {
     const long R = T_ * k;
+    // Column blocks per workgroup: two save a start each where the rows of an expert take long to multiply (8 experts,
+    // 64 tokens 578 -> 557 us), one spreads better where they do not (2 tokens 203 -> 192, 5 tokens 430 -> 415).
+    const long each = R > 4L * E ? 2 : 1;
+    static_assert(kFewBlocks >= 2, "the sums a workgroup keeps");
     auto* h = static_cast<std::uint16_t*>(workspace);
     auto* y = reinterpret_cast<std::uint16_t*>(static_cast<char*>(workspace) + align_up(static_cast<size_t>(R) * I * 2, 256));
     FfnGemmParams g1{};
@@ -755,10 +707,11 @@ int run_ffn_few_rows(const void* x, const void* w_gate, const void* w_up, const 
     g1.c = h;
     g1.order = order;
     g1.offsets = offsets;
+    g1.a_bytes = T_ * H * 2;
     g1.K = H; g1.N = I; g1.Nw = I; g1.R = R; g1.E = E; g1.k = k;
     division_by(static_cast<unsigned>(k), &g1.div_m, &g1.div_s);
-    hipLaunchKernelGGL((grouped_few_rows_kernel<T, true, 2>), dim3(static_cast<unsigned>((I + 15) / 16), static_cast<unsigned>(E)),
-                       dim3(kFewWaves * 64), 0, s, g1);
+    hipLaunchKernelGGL((grouped_few_rows_kernel<T, true>), dim3(static_cast<unsigned>((I / 16 + each - 1) / each), static_cast<unsigned>(E)),
+                       dim3(stream::kThreads), 0, s, g1);
     PARAS_HIP_TRY(hipGetLastError());
     FfnGemmParams g2{};
     g2.a = h;
@@ -767,9 +720,10 @@ int run_ffn_few_rows(const void* x, const void* w_gate, const void* w_up, const 
     g2.c = y;
     g2.order = nullptr;
     g2.offsets = offsets;
+    g2.a_bytes = R * I * 2;
     g2.K = I; g2.N = H; g2.Nw = H; g2.R = R; g2.E = E; g2.k = k;
-    hipLaunchKernelGGL((grouped_few_rows_kernel<T, false, 2>), dim3(static_cast<unsigned>((H + 15) / 16), static_cast<unsigned>(E)),
-                       dim3(kFewWaves * 64), 0, s, g2);
+    hipLaunchKernelGGL((grouped_few_rows_kernel<T, false>), dim3(static_cast<unsigned>((H / 16 + each - 1) / each), static_cast<unsigned>(E)),
+                       dim3(stream::kThreads), 0, s, g2);
     PARAS_HIP_TRY(hipGetLastError());
     const long total = T_ * (H / 8);
     long blocks = (total + kThreads - 1) / kThreads;
@@ -790,11 +744,11 @@ int run_ffn(const void* x, const void* w_gate, const void* w_up, const void* w_d
     const long R = T_ * k;
     // Up to 16 routed rows per expert on average the few-row kernels (an expert with more than 32 rows
     // takes them 32 at a time).  8 experts, top-2, H = 4096, I = 14336, tiles against few-row kernels:
-    // 1 token 421 / 168 us, 8 tokens 615 / 397, 32 tokens 659 / 574, 64 tokens 663 / 667, 128 tokens
-    // 672 / 1124.  PARAS_MOE_FEW_ROWS = n moves the limit (0: never).
+    // 1 token 421 / 138 us, 16 tokens 630 / 484, 64 tokens 663 / 557 (128 tokens, where every expert's weights
+    // are read twice from L2: tiles, 672).  PARAS_MOE_FEW_ROWS = n moves the limit (0: never).
     static const char* few_env = std::getenv("PARAS_MOE_FEW_ROWS");
     const long few_limit = few_env != nullptr ? std::atol(few_env) : 16;
-    if (R <= few_limit * E && E <= 65535 && (I + 15) / 16 <= 0x7fffffffL)
+    if (R <= few_limit * E && E <= 65535 && T_ * H * 2 <= stream::kMaxExtent && R * I * 2 <= stream::kMaxExtent)
         return run_ffn_few_rows<T>(x, w_gate, w_up, w_down, topw, order, inv_order, offsets, out, workspace, T_, E, k, H, I, s);
     const long wide_tiles = (R / Tile256::kBM) * ((H + 2 * kBN - 1) / (2 * kBN));
     if (R / E >= 4 * Tile256::kBM && wide_tiles >= 128)

@@ -462,3 +462,35 @@ def test_column_sum(shape, dtype):
     got = capi.column_sum(x.cuda()).cpu().double()
     bound = {torch.bfloat16: 2.0 ** -8, torch.float16: 2.0 ** -11, torch.float32: 2.0 ** -23, torch.float64: 1e-14}[dtype]
     assert bool(((got - want).abs() <= bound * want.abs() + 1e-5 * math.sqrt(shape[0]) * (1 if dtype.itemsize == 2 else 1e-2)).all())
+
+
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])
+@pytest.mark.parametrize("M", [1, 8, 9, 16, 17, 32])
+def test_few_rows_streamed_through_lds(M, dtype):
+    """Products of up to 32 rows: one to four requests of activations per piece; a ragged last block of weight rows; fewer
+    pieces of the contraction than waves, one more than a multiple of them, several trips; workgroups with more than one
+    block (N = 17000); padded strides; an infinity that only some results may see."""
+    for (N, K) in [(40, 64), (23, 576), (264, 1024), (4096, 2624), (17000, 128)]:
+        torch.manual_seed(M + N + K)
+        a, b = torch.randn(M, K + 8).to(dtype), (torch.randn(N, K + 16) / math.sqrt(K)).to(dtype)
+        bias = torch.randn(N).to(dtype)
+        a[M // 2, 3] = float("inf")
+        b[N // 2, 3] = 0.25
+        got = capi.gemm_nt(a.cuda()[:, :K], b.cuda()[:, :K], bias.cuda()).cpu()
+        want = a[:, :K].double() @ b[:, :K].double().t() + bias.double()
+        special = ~torch.isfinite(want)
+        assert torch.equal(got.double()[special & ~want.isnan()], want[special & ~want.isnan()])
+        assert bool((got.isnan() == want.isnan()).all())
+        keep = [r for r in range(M) if r != M // 2]
+        if keep:            # fp32 sums of K products of size 1 / sqrt(K), then one rounding to the type: one ulp, or 1e-6 sqrt(K) where they cancel
+            err = (got[keep].double() - want[keep]).abs()
+            assert bool((err <= ulp16(want[keep], dtype) * 1.001 + 1e-6 * math.sqrt(K)).all())
+
+
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])
+def test_few_columns_streamed_through_lds(dtype):
+    """A router's logits: many rows and few columns, the operands in each other's place."""
+    for (M, N, K) in [(129, 1, 64), (300, 8, 704), (20000, 9, 128), (515, 32, 2048)]:
+        torch.manual_seed(M)
+        a, b = torch.randn(M, K).to(dtype), (torch.randn(N, K) / math.sqrt(K)).to(dtype)
+        assert_gemm_close(capi.gemm_nt(a.cuda(), b.cuda()), (a.double() @ b.double().t()).to(dtype), dtype)

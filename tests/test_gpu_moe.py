@@ -75,6 +75,23 @@ def test_ffn_few_rows_per_expert(T, dtype):
     assert_ffn_close(out, want, dtype)
 
 
+@pytest.mark.parametrize("rows", [1, 8, 9, 16, 17, 33])
+def test_ffn_few_rows_at_the_edges_of_the_activation_blocks(rows):
+    """An expert with exactly as many rows as one, two or four requests of activations hold, and one more; column counts
+    that leave workgroups with one or two blocks of weights; contractions shorter than the eight waves' share."""
+    for (H, I, E, dtype) in [(64, 320, 16, torch.bfloat16), (576, 192, 64, torch.float16)]:
+        torch.manual_seed(rows)
+        T, k = rows, 2
+        x = torch.randn(T, H).to(dtype)
+        wg, wu, wd = (0.05 * torch.randn(E, I, H)).to(dtype), (0.05 * torch.randn(E, I, H)).to(dtype), (0.05 * torch.randn(E, H, I)).to(dtype)
+        logits = torch.randn(T, E)
+        logits[:, 1] += 9.0                    # everybody's first choice: `rows` rows
+        topi, topw, order, inv, counts, offsets = capi.moe_route(logits.to(dtype).cuda(), k)
+        assert counts[1].item() == rows
+        out = capi.moe_ffn(x.cuda(), wg.cuda(), wu.cuda(), wd.cuda(), topw, order, inv, offsets, k)
+        assert_ffn_close(out, O.moe_ffn(x, wg, wu, wd, topw.cpu(), order.cpu(), inv.cpu(), offsets.cpu(), k), dtype)
+
+
 def test_route_errors_and_empty():
     with pytest.raises(capi.ParasError, match="k out of range"):
         capi.moe_route(torch.randn(4, 8, device="cuda"), 9)
