@@ -316,6 +316,35 @@ __global__ __launch_bounds__(kBlock) void binary_vec16_kernel(int op, const std:
     store16_nt(out + i * 8, o);
 }
 
+// 16-bit tensors whose rows are contiguous in both operands, in whole 16-byte pieces, whatever the other dims do (a
+// projection's heads seen as [B, h, S, D], times cos / sin repeated over them): eight elements per thread.  `s` as above with
+// the last dim counted in pieces.  An element at a time spends its time on 64-bit index divisions and 2-byte accesses:
+// [1, 32, 1500, 128] and [1, 8, 1500, 128] (transposed views) times [1500, 128], bf16, 32 us together; this way 15.
+template <typename T>
+__global__ __launch_bounds__(kBlock) void binary_rows_vec16_kernel(int op, const std::uint16_t* __restrict__ a,
+                                                                   const std::uint16_t* __restrict__ b, std::uint16_t* __restrict__ out,
+                                                                   unsigned nvec, const Strided s, double alpha) {
+    const unsigned i = blockIdx.x * kBlock + threadIdx.x;
+    if (i >= nvec) return;
+    const bool unit = alpha == 1.0;
+    unsigned left = i;
+    long ao = 0, bo = 0;
+    for (int d = s.ndim - 1; d >= 0; --d) {
+        const unsigned size = static_cast<unsigned>(s.sizes[d]), q = left / size, c = left - q * size;
+        left = q;
+        ao += c * s.src_strides[d];
+        bo += c * s.dst_strides[d];
+    }
+    const u32x4 av = load16(a + ao), bv = load16(b + bo);
+    const std::uint16_t* ae = reinterpret_cast<const std::uint16_t*>(&av);
+    const std::uint16_t* be = reinterpret_cast<const std::uint16_t*>(&bv);
+    u32x4 o;
+    std::uint16_t* oe = reinterpret_cast<std::uint16_t*>(&o);
+#pragma unroll
+    for (int j = 0; j < 8; ++j) oe[j] = binary_one<T>(op, ae[j], be[j], alpha, unit);
+    store16(out + static_cast<long>(i) * 8, o);
+}
+
 // ---- index_select along one dim of a dense tensor seen as [outer, n_src, inner]:
 // dst[o, i, :] = src[o, idx[i], :] (the reference's index_select, csrc/ops/indexing_ops.cpp:96-150;
 // embedding lookups arrive here as dim 0).  `inner` is counted in W-byte units.  An index outside
@@ -625,6 +654,22 @@ int paras_binary_strided(int op, const void* a, const void* b, void* out, int nd
                 hipLaunchKernelGGL((binary_vec16_kernel<bf16_t>), gv, blk, 0, st, op, static_cast<const uint16_t*>(a), static_cast<const uint16_t*>(b), static_cast<uint16_t*>(out), nvec, brow / 8, alpha);
             else
                 hipLaunchKernelGGL((binary_vec16_kernel<f16_t>), gv, blk, 0, st, op, static_cast<const uint16_t*>(a), static_cast<const uint16_t*>(b), static_cast<uint16_t*>(out), nvec, brow / 8, alpha);
+            PARAS_HIP_TRY(hipGetLastError());
+            return PARAS_OK;
+        }
+        const int last = s.ndim - 1;
+        bool rows = aligned && last >= 1 && n / 8 < (1L << 31) && s.src_strides[last] == 1 && s.dst_strides[last] == 1 && s.sizes[last] % 8 == 0;
+        for (int d = 0; rows && d < last; ++d) rows = s.src_strides[d] % 8 == 0 && s.dst_strides[d] % 8 == 0;
+        if (rows) {
+            Strided v = s;
+            v.sizes[last] /= 8;
+            v.src_strides[last] = v.dst_strides[last] = 8;
+            const unsigned nvec = static_cast<unsigned>(n / 8);
+            const dim3 gv((nvec + kBlock - 1) / kBlock);
+            if (dtype == PARAS_BF16)
+                hipLaunchKernelGGL((binary_rows_vec16_kernel<bf16_t>), gv, blk, 0, st, op, static_cast<const uint16_t*>(a), static_cast<const uint16_t*>(b), static_cast<uint16_t*>(out), nvec, v, alpha);
+            else
+                hipLaunchKernelGGL((binary_rows_vec16_kernel<f16_t>), gv, blk, 0, st, op, static_cast<const uint16_t*>(a), static_cast<const uint16_t*>(b), static_cast<uint16_t*>(out), nvec, v, alpha);
             PARAS_HIP_TRY(hipGetLastError());
             return PARAS_OK;
         }

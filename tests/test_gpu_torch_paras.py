@@ -919,3 +919,33 @@ def test_boolean_masks_reach_the_kernels_as_they_are(device, Lq, Lk, D, mask_sha
     got = F.scaled_dot_product_attention(q, k, v, attn_mask=mask.to(device))
     want = F.scaled_dot_product_attention(q, k, v, attn_mask=add.to(device))
     assert ((got - want).cpu().float().norm() / want.cpu().float().norm()).item() < (2e-3 if dtype == torch.float16 else 1e-6)
+
+
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])
+def test_binary_ops_on_views_with_contiguous_rows_match_the_host(dtype):
+    """Operands that are transposed or sliced, or repeat over some dims, with rows in whole 16-byte pieces -- and the ones just
+    beside that rule: a row of 12, a slice that starts 2 bytes off, a stride that is not a multiple of 8, columns repeated."""
+    torch.manual_seed(3)
+    base, other = torch.randn(2, 33, 5, 64).to(dtype), torch.randn(33, 64).to(dtype)
+    forms = [(lambda t: t.transpose(1, 2), lambda t: t),                                     # [2, 5, 33, 64] with [33, 64]
+             (lambda t: t.transpose(1, 2)[..., :24], lambda t: t[:, 8:32]),
+             (lambda t: t.transpose(1, 2)[..., :12], lambda t: t[:, :12]),
+             (lambda t: t.transpose(1, 2)[..., 1:17], lambda t: t[:, 1:17]),
+             (lambda t: t.transpose(1, 2)[..., :8], lambda t: t[:, :1]),
+             (lambda t: t.transpose(0, 2), lambda t: t[:, None, :][:, :, :].expand(33, 2, 64)),
+             (lambda t: t.reshape(2, 33, 320)[:, :, :63].transpose(0, 1), lambda t: t[:, None, :63]),
+             (lambda t: t[:, :1].transpose(1, 2), lambda t: t)]                                # the first operand repeats
+    for fa, fb in forms:
+        for name, f in (("mul", torch.mul), ("add", torch.add), ("sub", torch.sub), ("div", torch.div)):
+            x, y = fa(base.to("paras:0")), fb(other.to("paras:0"))
+            got = f(x, y)
+            if name == "div":       # (host: fp32 and then 16 bits; device: fp64 and then 16 bits, as for dense operands)
+                want = f(x.contiguous(), y.expand(got.shape).contiguous()).cpu()
+            else:
+                want = f(fa(base), fb(other))
+            assert got.shape == want.shape and torch.equal(got.cpu(), want), name
+    a = torch.randn(4, 3, 6, 16).to(dtype)
+    b = torch.randn(3, 1, 16).to(dtype)
+    got = a.to("paras:0")
+    got.mul_(b.to("paras:0"))
+    assert torch.equal(got.cpu(), a * b)
