@@ -344,6 +344,15 @@ __global__ __launch_bounds__(256, (D > 128 ? 1 : 2)) void flash_fwd_kernel(const
         std::uint32_t mr[MREGS];
 #pragma unroll
         for (int i = 0; i < MREGS; ++i) mr[i] = loaded[i];
+        if constexpr (kMask == 1) {
+            // Every key of the block open to every query of the wave, as in all but the last blocks of a row under a
+            // key-padding mask: nothing to swap and nothing to select (fp16 B6 H12 S777 D64 30.8 -> 29.9 us).
+            if (mask_whole_block(j) && __builtin_amdgcn_ballot_w64((mr[0] & mr[1] & mr[2] & mr[3]) != 0x01010101u) == 0) {
+#pragma unroll
+                for (int r = 0; r < 16; ++r) sc[r] = round_T(round_T(sc[r]) * p.score_scale);
+                return;
+            }
+        }
         if constexpr (kMask != 0) {
             if (mask_whole_block(j)) {
                 // registers as loaded: the lane's own sixteen keys.  Lower half: keeps its runs 0 and 2 (bool:

@@ -222,6 +222,26 @@ def test_flash_random_shapes_layouts_and_padding():
         assert bool(torch.isfinite(out).all()) and float((out.float() - want).abs().max()) <= ABS_16BIT, case_id
 
 
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])
+@pytest.mark.parametrize("D", [64, 128, 256])
+def test_flash_key_padding_masks_at_the_edges_of_a_block(dtype, D):
+    """Blocks of 32 keys that are open as a whole, closed as a whole or split, rows of keys that end inside a block; and a mask
+    with one closed key for one query only in an otherwise open block (not every lane of the wave sees the same)."""
+    lens, Lk, H = [1, 31, 32, 33, 64, 95, 190, 200], 200, 2
+    B = len(lens)
+    q, k, v = (torch.randn(B, H, n, D).to(dtype) for n in (77, Lk, Lk))
+    keep = (torch.arange(Lk)[None, :] < torch.tensor(lens)[:, None]).reshape(B, 1, 1, Lk)
+    one = torch.ones(1, 1, 77, Lk, dtype=torch.bool)
+    one[0, 0, 40, 70] = False
+    scale = O.round_to_dtype(1 / math.sqrt(D), dtype)
+    for mask in (keep, one):
+        out, _, _, kern = run(q, k, v, mask=mask, scale=scale)
+        want, _ = O.sdpa_math(q, k, v, attn_mask=mask, gemm="aten", scale=scale)
+        assert kern.startswith("flash_mfma")
+        err = (out.double().cpu() - want.double()).abs().max().item()
+        assert err <= (2.5e-2 if dtype == torch.bfloat16 else 4e-3), err     # a step of the type on values up to 4: 2^-7 x 2 (2^-10 x 2), and rounding of the weights
+
+
 MASK_SHAPES = [  # B, Hq, Hkv, Lq, Lk, D, mask shape
     (2, 4, 4, 200, 200, 128, (2, 1, 1, 200)),      # key-padding mask, broadcast over heads and queries
     (1, 4, 2, 130, 191, 64, (1, 1, 130, 191)),     # one [Lq, Lk] pattern for every head, ragged lengths
