@@ -132,14 +132,15 @@ template <int W, bool R> struct Operand {
 // holds row i*16 + l16 of the wave's rows and columns j*16 + 4*kq .. + 3 of its columns.
 // (The stages are separate arrays named at compile time: an LDS read waits for every direct load in flight
 // that the compiler cannot prove to go elsewhere.)
-template <typename T, int MI, int NJ, bool AR, bool BR>
-__device__ __forceinline__ void mainloop(Operand<MI, AR>& oa, Operand<NJ, BR>& ob, int k_count, std::uint16_t* a0, std::uint16_t* a1,
+// OA, OB: Operand or a type with its rsrc / request / frag / last_tile.
+template <typename T, int MI, int NJ, typename OA, typename OB>
+__device__ __forceinline__ void mainloop(OA& oa, OB& ob, int k_count, std::uint16_t* a0, std::uint16_t* a1,
                                          std::uint16_t* b0, std::uint16_t* b1, float4v (&acc)[MI][NJ]) {
     constexpr int C = MI + NJ;          // requests per wave and tile, and fragments per k-step
     constexpr int S = MI * NJ;          // MFMAs per k-step
     i16x8 af[2][MI], bf[2][NJ];
     const int k_tiles = (k_count + kBK - 1) / kBK;
-    auto request_one = [&](__amdgpu_buffer_rsrc_t ra, __amdgpu_buffer_rsrc_t rb, std::uint16_t* ta, std::uint16_t* tb, int c) {
+    auto request_one = [&](const auto& ra, const auto& rb, std::uint16_t* ta, std::uint16_t* tb, int c) {
         if (c < MI) oa.request(ra, ta, c);
         else        ob.request(rb, tb, c - MI);
     };

@@ -64,7 +64,7 @@ __global__ __launch_bounds__(kThreads, (MI * NJ >= 32 ? 1 : 2)) void gemm_flex_k
     oa.init(p.a + w.batch * p.sa, p.lda, p.M, row0, k_first, k_count, wave >> 1);
     ob.init(p.b + w.batch * p.sb, p.ldb, p.N, col0, k_first, k_count, wave & 1);
     float4v acc[MI][NJ];
-    mainloop<T, MI, NJ, AR, BR>(oa, ob, static_cast<int>(k_count), a0, a1, b0, b1, acc);
+    mainloop<T, MI, NJ>(oa, ob, static_cast<int>(k_count), a0, a1, b0, b1, acc);
 
     const int lane = threadIdx.x & 63;
     const int l16 = lane & 15, kq = lane >> 4;

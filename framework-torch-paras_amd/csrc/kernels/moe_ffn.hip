@@ -19,7 +19,7 @@
 // n0..n0+255 for GEMM 2), k-tile 64.  128 rows: waves arranged 2x2 with 64x64
 // per column group each (128 fp32 accumulators per lane).  256 rows, when the
 // experts hold enough rows for them: four waves with 128 x 128 each on
-// v_mfma_f32_16x16x32 (256 accumulators per lane; grouped_gemm_quad16_kernel).
+// v_mfma_f32_16x16x32 (256 accumulators per lane; grouped_gemm_direct_kernel).
 // Global -> registers -> LDS with the next
 // k-tile's loads in flight during the MFMAs.  Rows of one expert are contiguous
 // in the routed order; m-tiles never straddle experts (the grid is sized for the
@@ -32,6 +32,7 @@
 #include "core/device_context.h"
 #include "core/device_math.h"
 #include "core/status.h"
+#include "kernels/gemm_flex.h"
 #include "kernels/gemm_tile.h"
 #include "kernels/stream_rows.h"
 #include "kernels/swiglu_math.h"
@@ -48,7 +49,7 @@ struct FfnGemmParams {
     std::uint16_t* c;           // [R, N]
     const long* order;          // gather index (routed row -> flat (token, slot)); null = direct rows
     const long* offsets;        // [E+1]
-    long a_bytes;               // extent of a (few-row kernels)
+    long a_bytes;               // extent of a (few-row and direct kernels)
     long K, N, Nw, R;           // contraction, output columns, weight rows per expert, routed rows
     int E, k;
     int mt_total;               // upper bound on m-tiles
@@ -206,26 +207,63 @@ __device__ __forceinline__ void quad16_static_for(F&& f) {
     quad16_static_for_impl(std::make_integer_sequence<int, N>{}, static_cast<F&&>(f));
 }
 
-// A wave's queue of SwiGLU values that left the common tier (four of one lane per entry): laid over the
-// tile stages once the contraction is done.
+// A wave's queue of SwiGLU values that left the common tier (four of one lane per entry): laid over one
+// of the four tile stages once the contraction is done.
 struct SwigluQueue {
-    static constexpr unsigned kEntries = 1024;
+    static constexpr unsigned kEntries = 896;
     unsigned where[kEntries];       // (row in the tile) << 16 | column in the column unit
-    quad16::float4v gate[kEntries], up[kEntries];
+    flex::float4v gate[kEntries], up[kEntries];
 };
-static_assert(4 * sizeof(SwigluQueue) <= sizeof(quad16::TileLds), "four queues in the tile stages");
+constexpr int kStageElems = 256 * kBK;          // a stage of either operand: 256 rows of a k-tile
+static_assert(sizeof(SwigluQueue) <= kStageElems * 2, "a queue in a tile stage");
 
-// The same on the four-wave tile of v_mfma_f32_16x16x32 (gemm_tile.h, namespace quad16): what the layer
-// runs on when the experts are big enough for 256-row tiles.  Tile coordinates, the search for the
-// m-tile's expert and the staging offsets as above (a thread stages eight chunks of A and four per
-// column group of B); a lane of accumulator block (i, j) holds row i*16 + lane%16 and columns
-// 4*(lane/16) .. + 3 of column block j (group j / 4, columns wn*64 + (j % 4)*16 of it), so gate and
-// up of one output sit in blocks j and j + 4 of the same lane and an output row gets 8-byte stores.
+// The weight rows of a 256-column tile that come as two groups of 128: a wave's 128 rows of the LDS tile are 64 rows of
+// group 0 and the 64 rows of group 1 with the same index, so that the accumulators of a gate column and of its up
+// column belong to the same lane.  (An LDS tile row r: wave r / 128, block r % 128 / 16, of which four are group 0's.)
+struct TwoGroups : flex::Operand<8, false> {
+    const char* base2;
+    struct Rsrc { __amdgpu_buffer_rsrc_t g[2]; };
+    // b, b2: row 0 of the groups; rows_left[g] rows of group g exist (<= 0: none)
+    __device__ __forceinline__ void aim(const std::uint16_t* b, const std::uint16_t* b2, long K, long rows_left, long second, int w) {
+        const int lane = threadIdx.x & 63, l16 = lane & 15, kq = lane >> 4;
+        base = reinterpret_cast<const char*>(b);
+        base2 = reinterpret_cast<const char*>(b2);
+        left = rows_left * K * 2;
+        step = kBK * 2;
+#pragma unroll
+        for (int i = 0; i < 8; ++i) {
+            const int r = (i * 4 + flex::wave_id()) * 8 + (lane >> 3);
+            const long row = (r >> 7) * 64 + ((r >> 4) & 3) * 16 + (r & 15) + ((i & 2) ? second : 0);
+            off[i] = static_cast<std::uint32_t>(row * K * 2 + ((lane & 7) ^ (lane >> 3)) * 16);
+        }
+#pragma unroll
+        for (int ks = 0; ks < 2; ++ks) fb[ks] = (w * 128 + l16) * kBK + ((ks * 4 + kq) ^ (l16 & 7)) * 8;
+    }
+    __device__ __forceinline__ Rsrc rsrc(int kt, int k_tiles) const {
+        const long l = left - kt * step;
+        const int n = static_cast<int>(static_cast<std::uint32_t>(l < 0 || kt >= k_tiles ? 0 : (l > flex::kMaxExtent ? flex::kMaxExtent : l)));
+        return {{__builtin_amdgcn_make_buffer_rsrc(const_cast<char*>(base + kt * step), 0, n, 0x00020000),
+                 __builtin_amdgcn_make_buffer_rsrc(const_cast<char*>(base2 + kt * step), 0, n, 0x00020000)}};
+    }
+    __device__ __forceinline__ void request(const Rsrc& r, std::uint16_t* tile, int i) const {
+        flex::Operand<8, false>::request((i & 2) ? r.g[1] : r.g[0], tile, i);
+    }
+};
+
+// The same on the four-wave 256 x 256 tile of v_mfma_f32_16x16x32 whose loads go straight to LDS (gemm_flex.h): what the
+// layer runs on when the experts are big enough for 256-row tiles.  Tile coordinates and the search for the
+// m-tile's expert as above; the routed rows are gathered by the addresses the lanes fetch from.  A lane of accumulator
+// block (i, j) holds row i*16 + lane%16 and columns 4*(lane/16) .. + 3 of column block j (group j / 4, columns
+// wn*64 + (j % 4)*16 of it), so gate and up of one output sit in blocks j and j + 4 of the same lane and an output row
+// gets 8-byte stores.  Bound by the matrix cores' power and the LDS reads.
 template <typename T, bool kSwiglu>
-__global__ __launch_bounds__(quad16::kThreads, 1) void grouped_gemm_quad16_kernel(const FfnGemmParams p) {
+__global__ __launch_bounds__(flex::kThreads, 1) void grouped_gemm_direct_kernel(const FfnGemmParams p) {
     using El = Elem<T>;
-    constexpr int kBM = quad16::kBM;
-    __shared__ __attribute__((aligned(16))) quad16::TileLds lds;
+    constexpr int kBM = 256;
+    __shared__ __attribute__((aligned(1024))) std::uint16_t a0[kStageElems];
+    __shared__ __attribute__((aligned(1024))) std::uint16_t a1[kStageElems];
+    __shared__ __attribute__((aligned(1024))) std::uint16_t b0[kStageElems];
+    __shared__ __attribute__((aligned(1024))) std::uint16_t b1[kStageElems];
     int mt, nu;
     {
         const long L = blockIdx.x;
@@ -233,8 +271,9 @@ __global__ __launch_bounds__(quad16::kThreads, 1) void grouped_gemm_quad16_kerne
         const long j = L >> 3;
         const long per_group = static_cast<long>(p.mt_total) * p.ngt;
         const long g = j / per_group, rem = j % per_group;
-        mt = static_cast<int>(rem / p.ngt);
-        nu = static_cast<int>((g * 8 + xcd) * p.ngt + rem % p.ngt);
+        // (quotients come from vector arithmetic: what depends on them is to stay in scalar registers)
+        mt = __builtin_amdgcn_readfirstlane(static_cast<int>(rem / p.ngt));
+        nu = __builtin_amdgcn_readfirstlane(static_cast<int>((g * 8 + xcd) * p.ngt + rem % p.ngt));
         if (nu >= p.n_units) return;
     }
     int e = 0;
@@ -260,27 +299,30 @@ __global__ __launch_bounds__(quad16::kThreads, 1) void grouped_gemm_quad16_kerne
     const int l16 = lane & 15, kq = lane >> 4;
     const int wm = wave >> 1, wn = wave & 1;
 
-    unsigned a_off[8], b_off[2][4];
+    // W requests per wave of the routed rows: rows past the expert's last are not fetched (their results are not stored)
+    auto aim_rows = [&](auto& oa, int w) __attribute__((always_inline)) {
+        constexpr int W = sizeof(oa.off) / sizeof(oa.off[0]);
+        oa.base = reinterpret_cast<const char*>(p.order ? p.a : p.a + row0 * p.K);
+        oa.left = p.order ? p.a_bytes : (row_end - row0) * p.K * 2;
+        oa.step = kBK * 2;
 #pragma unroll
-    for (int i = 0; i < 8; ++i) {
-        const int c = tid + i * quad16::kThreads;
-        long prow = row0 + (c >> 3);
-        if (prow >= row_end) prow = row_end - 1;  // clamp: result rows beyond the expert are not stored
-        const long src = p.order ? static_cast<long>((static_cast<unsigned long long>(static_cast<unsigned>(p.order[prow])) * p.div_m) >> p.div_s) : prow;
-        a_off[i] = static_cast<unsigned>(src * p.K + (c & 7) * 8);
-    }
-    const std::uint16_t* const b_base[2] = {p.b + static_cast<long>(e) * p.Nw * p.K, p.b2 + static_cast<long>(e) * p.Nw * p.K};
-#pragma unroll
-    for (int g = 0; g < 2; ++g)
-#pragma unroll
-        for (int i = 0; i < 4; ++i) {
-            const int c = tid + i * quad16::kThreads;
-            long wrow = (kSwiglu ? n0 : n0 + g * kBN) + (c >> 3);
-            if (wrow >= p.Nw) wrow = p.Nw - 1;
-            b_off[g][i] = static_cast<unsigned>(wrow * p.K + (c & 7) * 8);
+        for (int i = 0; i < W; ++i) {
+            const long r = (i * 4 + flex::wave_id()) * 8 + (lane >> 3);
+            const bool live = row0 + r < row_end;
+            long src = r;
+            if (p.order) src = static_cast<long>((static_cast<unsigned long long>(static_cast<unsigned>(p.order[live ? row0 + r : row0])) * p.div_m) >> p.div_s);
+            oa.off[i] = live ? static_cast<std::uint32_t>(src * p.K * 2 + ((lane & 7) ^ (lane >> 3)) * 16) : flex::kOutOfRange;
         }
+#pragma unroll
+        for (int ks = 0; ks < 2; ++ks) oa.fb[ks] = (w * 16 * W + l16) * kBK + ((ks * 4 + kq) ^ (l16 & 7)) * 8;
+    };
+    TwoGroups ob;
+    {
+        const long first = (static_cast<long>(e) * p.Nw + n0) * p.K;
+        ob.aim(p.b + first, p.b2 + first, p.K, p.Nw - n0, kSwiglu ? 0 : kBN, wn);
+    }
     // four values of one output row: SwiGLU of the gate / up pairs, or the narrowed product
-    auto put4 = [&](long prow, long col, const quad16::float4v a0, const quad16::float4v a1, bool nan_here) __attribute__((always_inline)) {
+    auto put4 = [&](long prow, long col, const flex::float4v a0, const flex::float4v a1, bool nan_here) __attribute__((always_inline)) {
         if (prow >= row_end || col >= p.N) return;
         std::uint16_t o[4];
         if constexpr (kSwiglu) {
@@ -303,40 +345,44 @@ __global__ __launch_bounds__(quad16::kThreads, 1) void grouped_gemm_quad16_kerne
     auto any_nan = [&](float probe) { return __builtin_amdgcn_ballot_w64(probe != probe) != 0; };
 
     if (row_end - row0 <= 64) {     // an expert's last tile with few rows: the waves share them
-        quad16::float4v sacc[4][4];
-        quad16::short_tile_mainloop<T>(p.a, a_off, b_base, b_off, p.K, lds, sacc);
+        flex::Operand<2, false> oa;
+        aim_rows(oa, wm);
+        flex::float4v sacc[2][8];
+        flex::mainloop<T, 2, 8>(oa, ob, static_cast<int>(p.K), a0, a1, b0, b1, sacc);
 #pragma unroll
-        for (int i = 0; i < 4; ++i) {
-            const long prow = row0 + i * 16 + l16;
+        for (int i = 0; i < 2; ++i) {
+            const long prow = row0 + wm * 32 + i * 16 + l16;
             bool nan_here = false;
             if (!kSwiglu) {
                 float probe = 0.f;
 #pragma unroll
-                for (int jj = 0; jj < 4; ++jj)
+                for (int j = 0; j < 8; ++j)
 #pragma unroll
-                    for (int r = 0; r < 4; ++r) probe += sacc[i][jj][r];
+                    for (int r = 0; r < 4; ++r) probe += sacc[i][j][r];
                 nan_here = any_nan(probe);
             }
 #pragma unroll
-            for (int cb = 0; cb < 2; ++cb) {
-                const long col = n0 + wave * 32 + cb * 16 + 4 * kq;
+            for (int jb = 0; jb < 4; ++jb) {
+                const long col = n0 + wn * 64 + jb * 16 + 4 * kq;
                 if (kSwiglu) {
-                    put4(prow, col, sacc[i][cb], sacc[i][2 + cb], false);
+                    put4(prow, col, sacc[i][jb], sacc[i][4 + jb], false);
                 } else {
-                    put4(prow, col, sacc[i][cb], sacc[i][cb], nan_here);
-                    put4(prow, col + kBN, sacc[i][2 + cb], sacc[i][2 + cb], nan_here);
+                    put4(prow, col, sacc[i][jb], sacc[i][jb], nan_here);
+                    put4(prow, col + kBN, sacc[i][4 + jb], sacc[i][4 + jb], nan_here);
                 }
             }
         }
         return;
     }
-    quad16::float4v acc[8][8];
-    quad16::tile_mainloop<T>(p.a, a_off, b_base, b_off, p.K, lds, acc);
+    flex::Operand<8, false> oa;
+    aim_rows(oa, wm);
+    flex::float4v acc[8][8];
+    flex::mainloop<T, 8, 8>(oa, ob, static_cast<int>(p.K), a0, a1, b0, b1, acc);
     if constexpr (kSwiglu) {
         // About one value in a thousand leaves the common tier of SwiGLU, and where one lane of the 64 does,
         // the whole wave walks through the fp64 formula: at 128 values a lane that happened eight times a tile
         // and cost 4 % of the kernel.  A lane whose four values do not all pass queues them (the accumulators
-        // and where they go) in the wave's share of the tile stages, which nobody reads any more; after
+        // and where they go) in one of the tile stages, which nobody reads any more; after
         // the last row block (or when the next one might not fit) the wave works its queue off, one value per lane.
         __syncthreads();
         // (the lane's coordinates derived again, from a value the compiler cannot trace: none of this is to
@@ -344,7 +390,7 @@ __global__ __launch_bounds__(quad16::kThreads, 1) void grouped_gemm_quad16_kerne
         int t = threadIdx.x;
         asm volatile("" : "+v"(t));
         const int lane = t & 63, wave = t >> 6, l16 = t & 15, kq = (t >> 4) & 3, wm = t >> 7, wn = (t >> 6) & 1;
-        SwigluQueue& q = reinterpret_cast<SwigluQueue*>(&lds)[wave];
+        SwigluQueue& q = *reinterpret_cast<SwigluQueue*>(wave == 0 ? a0 : (wave == 1 ? a1 : (wave == 2 ? b0 : b1)));
         const unsigned long long lanes_below = (1ull << lane) - 1ull;
         unsigned queued = 0;      // uniform
         auto work_off = [&]() __attribute__((always_inline)) {
@@ -637,6 +683,7 @@ int run_ffn_shape(const void* x, const void* w_gate, const void* w_up, const voi
     g1.c = h;
     g1.order = order;
     g1.offsets = offsets;
+    g1.a_bytes = T_ * H * 2;
     g1.K = H; g1.N = I; g1.Nw = I; g1.R = R; g1.E = E; g1.k = k;
     g1.mt_total = mt_total;
     division_by(static_cast<unsigned>(k), &g1.div_m, &g1.div_s);
@@ -657,8 +704,10 @@ int run_ffn_shape(const void* x, const void* w_gate, const void* w_up, const voi
     // 32 x 32 x 16 ones, for measurements)
     static const bool eight_waves = std::getenv("PARAS_GEMM_EIGHT_WAVES") != nullptr;
     constexpr bool kBig = S::kBM == 256;
-    if (kBig && !eight_waves)
-        hipLaunchKernelGGL((grouped_gemm_quad16_kernel<T, true>), dim3(grid_of(g1)), dim3(quad16::kThreads), 0, s, g1);
+    // (its gathered rows are reached by 32-bit byte offsets from the start of x, its weight rows from the tile's first)
+    const bool direct = kBig && !eight_waves && T_ * H * 2 <= flex::kMaxExtent && H <= flex::kMaxLd && I <= flex::kMaxLd;
+    if (direct)
+        hipLaunchKernelGGL((grouped_gemm_direct_kernel<T, true>), dim3(grid_of(g1)), dim3(flex::kThreads), 0, s, g1);
     else
         hipLaunchKernelGGL((grouped_gemm_kernel<T, true, S>), dim3(grid_of(g1)), dim3(S::kThreads), 0, s, g1);
     PARAS_HIP_TRY(hipGetLastError());
@@ -674,8 +723,8 @@ int run_ffn_shape(const void* x, const void* w_gate, const void* w_up, const voi
     g2.mt_total = mt_total;
     g2.n_units = static_cast<int>((H + 2 * kBN - 1) / (2 * kBN));
     plan(g2);
-    if (kBig && !eight_waves)
-        hipLaunchKernelGGL((grouped_gemm_quad16_kernel<T, false>), dim3(grid_of(g2)), dim3(quad16::kThreads), 0, s, g2);
+    if (direct)
+        hipLaunchKernelGGL((grouped_gemm_direct_kernel<T, false>), dim3(grid_of(g2)), dim3(flex::kThreads), 0, s, g2);
     else
         hipLaunchKernelGGL((grouped_gemm_kernel<T, false, S>), dim3(grid_of(g2)), dim3(S::kThreads), 0, s, g2);
     PARAS_HIP_TRY(hipGetLastError());
