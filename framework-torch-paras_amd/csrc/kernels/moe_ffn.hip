@@ -214,6 +214,7 @@ struct SwigluQueue {
     unsigned where[kEntries];       // (row in the tile) << 16 | column in the column unit
     flex::float4v gate[kEntries], up[kEntries];
 };
+constexpr int kSuperM = 8, kSuperN = 4;
 constexpr int kStageElems = 256 * kBK;          // a stage of either operand: 256 rows of a k-tile
 static_assert(sizeof(SwigluQueue) <= kStageElems * 2, "a queue in a tile stage");
 
@@ -264,34 +265,41 @@ __global__ __launch_bounds__(flex::kThreads, 1) void grouped_gemm_direct_kernel(
     __shared__ __attribute__((aligned(1024))) std::uint16_t a1[kStageElems];
     __shared__ __attribute__((aligned(1024))) std::uint16_t b0[kStageElems];
     __shared__ __attribute__((aligned(1024))) std::uint16_t b1[kStageElems];
+    // Super-tiles of kSuperM row tiles x kSuperN column units, the 32 workgroups an XCD runs together: they fetch 8 panels of
+    // routed rows and 4 to 8 of weights between them (a sweep of all row tiles over two column units: 18 to 20).
+    // They are dealt to the XCDs one after the other, columns first, so that the XCDs share the rows' panels.
+    // (8192 tokens, 8 experts, H 4096, I 14336, the layer: 8 x 4 4675 us, 4 x 8 4750, 16 x 2 4760, 32 x 1 for the plain product 4820.)
     int mt, nu;
     {
-        const long L = blockIdx.x;
-        const int xcd = static_cast<int>(L & 7);
-        const long j = L >> 3;
-        const long per_group = static_cast<long>(p.mt_total) * p.ngt;
-        const long g = j / per_group, rem = j % per_group;
+        const unsigned xcd = blockIdx.x & 7, j = blockIdx.x >> 3;
+        const unsigned super = j / (kSuperM * kSuperN) * 8 + xcd, in = j % (kSuperM * kSuperN);
+        const unsigned across = (static_cast<unsigned>(p.n_units) + kSuperN - 1) / kSuperN;
         // (quotients come from vector arithmetic: what depends on them is to stay in scalar registers)
-        mt = __builtin_amdgcn_readfirstlane(static_cast<int>(rem / p.ngt));
-        nu = __builtin_amdgcn_readfirstlane(static_cast<int>((g * 8 + xcd) * p.ngt + rem % p.ngt));
+        const unsigned mb = static_cast<unsigned>(__builtin_amdgcn_readfirstlane(static_cast<int>(super / across)));
+        mt = static_cast<int>(mb * kSuperM + in % kSuperM);
+        nu = static_cast<int>((super - mb * across) * kSuperN + in / kSuperM);
         if (nu >= p.n_units) return;
     }
+    // m-tile -> (expert, first row): first every expert's tiles with more than 64 rows, then the short last ones, which
+    // take a fraction of the time and fill in at the end of every XCD's list
     int e = 0;
     long row0 = 0, row_end = 0;
     {
-        int tiles_before = 0;
+        int left = mt;
         bool found = false;
-        for (int i = 0; i < p.E; ++i) {
-            const long lo = p.offsets[i], hi = p.offsets[i + 1];
-            const int tiles = static_cast<int>((hi - lo + kBM - 1) / kBM);
-            if (!found && mt < tiles_before + tiles) {
-                e = i;
-                row0 = lo + static_cast<long>(mt - tiles_before) * kBM;
-                row_end = hi;
-                found = true;
+        for (int pass = 0; pass < 2 && !found; ++pass)
+            for (int i = 0; i < p.E && !found; ++i) {
+                const long lo = p.offsets[i], hi = p.offsets[i + 1];
+                const long full = (hi - lo) / kBM, over = (hi - lo) - full * kBM;
+                const int tiles = pass == 0 ? static_cast<int>(full) + (over > 64) : (over > 0 && over <= 64);
+                if (left < tiles) {
+                    e = i;
+                    row0 = lo + (pass == 0 ? left : full) * kBM;
+                    row_end = hi;
+                    found = true;
+                }
+                left -= tiles;
             }
-            tiles_before += tiles;
-        }
         if (!found) return;
     }
     const long n0 = static_cast<long>(nu) * (kSwiglu ? kBN : 2 * kBN);
@@ -699,6 +707,10 @@ int run_ffn_shape(const void* x, const void* w_gate, const void* w_up, const voi
         const long groups = (g.n_units + 8 * g.ngt - 1) / (8 * g.ngt);
         return static_cast<unsigned>(groups * 8 * g.ngt * g.mt_total);
     };
+    auto direct_grid_of = [](const FfnGemmParams& g) {
+        const long supers = static_cast<long>((g.mt_total + kSuperM - 1) / kSuperM) * ((g.n_units + kSuperN - 1) / kSuperN);
+        return static_cast<unsigned>((supers + 7) / 8 * 8 * kSuperM * kSuperN);
+    };
     plan(g1);
     // 256-row tiles: the four-wave tile of 16 x 16 x 32 MFMAs (PARAS_GEMM_EIGHT_WAVES: the eight-wave tile of
     // 32 x 32 x 16 ones, for measurements)
@@ -707,7 +719,7 @@ int run_ffn_shape(const void* x, const void* w_gate, const void* w_up, const voi
     // (its gathered rows are reached by 32-bit byte offsets from the start of x, its weight rows from the tile's first)
     const bool direct = kBig && !eight_waves && T_ * H * 2 <= flex::kMaxExtent && H <= flex::kMaxLd && I <= flex::kMaxLd;
     if (direct)
-        hipLaunchKernelGGL((grouped_gemm_direct_kernel<T, true>), dim3(grid_of(g1)), dim3(flex::kThreads), 0, s, g1);
+        hipLaunchKernelGGL((grouped_gemm_direct_kernel<T, true>), dim3(direct_grid_of(g1)), dim3(flex::kThreads), 0, s, g1);
     else
         hipLaunchKernelGGL((grouped_gemm_kernel<T, true, S>), dim3(grid_of(g1)), dim3(S::kThreads), 0, s, g1);
     PARAS_HIP_TRY(hipGetLastError());
@@ -724,7 +736,7 @@ int run_ffn_shape(const void* x, const void* w_gate, const void* w_up, const voi
     g2.n_units = static_cast<int>((H + 2 * kBN - 1) / (2 * kBN));
     plan(g2);
     if (direct)
-        hipLaunchKernelGGL((grouped_gemm_direct_kernel<T, false>), dim3(grid_of(g2)), dim3(flex::kThreads), 0, s, g2);
+        hipLaunchKernelGGL((grouped_gemm_direct_kernel<T, false>), dim3(direct_grid_of(g2)), dim3(flex::kThreads), 0, s, g2);
     else
         hipLaunchKernelGGL((grouped_gemm_kernel<T, false, S>), dim3(grid_of(g2)), dim3(S::kThreads), 0, s, g2);
     PARAS_HIP_TRY(hipGetLastError());
