@@ -381,8 +381,8 @@ def main() -> int:
             "workload": "bf16 MoE layer T=8192 H=4096 E=8 top-2 I=14336: routing + grouped expert FFN (configs[4])",
             "value": round(T / ms_all * 1e3, 1), "unit": "tokens/s", "ms_per_step": round(ms_all, 4), "steps": msteps,
             "route_ms": round(ms_route, 4), "ffn_ms": round(ms_ffn, 4), "ffn_tflops": round(tf, 2),
-            "kernel": "grouped_gemm_quad16_kernel<bf16> (gate-up+SwiGLU, down) + moe_combine_kernel",
-            "algorithmic_flops_per_launch": flops, "roofline": roofline("mfma", tf, "grouped_gemm_quad16_kernel"),
+            "kernel": "grouped_gemm_direct_kernel<bf16> (gate-up+SwiGLU, down) + moe_combine_kernel",
+            "algorithmic_flops_per_launch": flops, "roofline": roofline("mfma", tf, "grouped_gemm_direct_kernel"),
         }
         log(f"moe: route {ms_route * 1e3:.1f} us, ffn {ms_ffn * 1e3:.1f} us = {tf:.1f} TFLOP/s ({tf / MFMA_BF16_PEAK_TFLOPS:.1%}), "
             f"layer {ms_all * 1e3:.1f} us = {T / ms_all * 1e3:.0f} tokens/s")
@@ -423,8 +423,8 @@ def main() -> int:
         tf = flops / ms / 1e9
         results["linear"] = {
             "workload": "bf16 dense NT GEMM x W^T: M=16384 N=4096 K=4096 (nn.Linear of configs[2]'s tokens)",
-            "value": round(tf, 2), "unit": "TFLOP/s", "ms_per_step": round(ms, 4), "kernel": "dense_gemm_nt_quad16_kernel<bf16>",
-            "algorithmic_flops_per_launch": flops, "roofline": roofline("mfma", tf, "dense_gemm_nt_quad16_kernel"),
+            "value": round(tf, 2), "unit": "TFLOP/s", "ms_per_step": round(ms, 4), "kernel": "gemm_flex_kernel<bf16>",
+            "algorithmic_flops_per_launch": flops, "roofline": roofline("mfma", tf, "gemm_flex_kernel"),
         }
         log(f"linear: {ms * 1e3:.1f} us  {tf:.1f} TFLOP/s ({tf / MFMA_BF16_PEAK_TFLOPS:.1%})")
         lin_got = yc[M - 64:].cpu()

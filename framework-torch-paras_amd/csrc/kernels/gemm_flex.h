@@ -33,7 +33,7 @@ namespace paras {
 namespace flex {
 
 using gemm::i16x8;
-using gemm::quad16::float4v;
+typedef float float4v __attribute__((ext_vector_type(4)));
 
 // acc += b a, in place in the accumulation registers.  Written out because the compiler, given the
 // builtin, moves the 256 accumulators of the large tile from register to register on their way round the

@@ -14,18 +14,13 @@
 // contraction dim, which is exactly the 8-element-per-lane operand layout of
 // v_mfma_f32_32x32x16, so neither operand needs a transpose.
 //
-// Tiling (gemm_tile.h): a workgroup computes 128 or 256 routed rows x two
-// 128-column groups (gate and up columns n0..n0+127 for GEMM 1; columns
-// n0..n0+255 for GEMM 2), k-tile 64.  128 rows: waves arranged 2x2 with 64x64
-// per column group each (128 fp32 accumulators per lane).  256 rows, when the
-// experts hold enough rows for them: four waves with 128 x 128 each on
-// v_mfma_f32_16x16x32 (256 accumulators per lane; grouped_gemm_direct_kernel).
-// Global -> registers -> LDS with the next
-// k-tile's loads in flight during the MFMAs.  Rows of one expert are contiguous
-// in the routed order; m-tiles never straddle experts (the grid is sized for the
-// worst case and surplus workgroups exit).  The block index is unscrambled so
-// that the workgroups resident on one XCD cover all m-tiles of a few column
-// tiles: weight tiles are then shared through that XCD's L2.
+// Tiling: a workgroup computes 128 or 256 routed rows x two 128-column groups (gate and up columns
+// n0..n0+127 for GEMM 1; columns n0..n0+255 for GEMM 2), k-tile 64.  128 rows (gemm_tile.h): waves arranged
+// 2x2 with 64x64 per column group each (128 fp32 accumulators per lane), global -> registers -> LDS.  256
+// rows, when the experts hold enough rows for them: four waves with 128 x 128 each on v_mfma_f32_16x16x32
+// (256 accumulators per lane), loads straight to LDS (gemm_flex.h; grouped_gemm_direct_kernel).  Rows of one
+// expert are contiguous in the routed order; m-tiles never straddle experts (the grid is sized for the
+// worst case and surplus workgroups exit).
 #include <hip/hip_runtime.h>
 #include <cstdlib>
 
@@ -199,12 +194,12 @@ __global__ __launch_bounds__(S::kThreads, 2) void grouped_gemm_kernel(const FfnG
 
 // f(integral_constant<int, I>) for I = 0 .. N-1
 template <int... I, typename F>
-__device__ __forceinline__ void quad16_static_for_impl(std::integer_sequence<int, I...>, F&& f) {
+__device__ __forceinline__ void static_for_impl(std::integer_sequence<int, I...>, F&& f) {
     (f(std::integral_constant<int, I>{}), ...);
 }
 template <int N, typename F>
-__device__ __forceinline__ void quad16_static_for(F&& f) {
-    quad16_static_for_impl(std::make_integer_sequence<int, N>{}, static_cast<F&&>(f));
+__device__ __forceinline__ void static_for(F&& f) {
+    static_for_impl(std::make_integer_sequence<int, N>{}, static_cast<F&&>(f));
 }
 
 // A wave's queue of SwiGLU values that left the common tier (four of one lane per entry): laid over one
@@ -329,16 +324,12 @@ __global__ __launch_bounds__(flex::kThreads, 1) void grouped_gemm_direct_kernel(
         const long first = (static_cast<long>(e) * p.Nw + n0) * p.K;
         ob.aim(p.b + first, p.b2 + first, p.K, p.Nw - n0, kSwiglu ? 0 : kBN, wn);
     }
-    // four values of one output row: SwiGLU of the gate / up pairs, or the narrowed product
-    auto put4 = [&](long prow, long col, const flex::float4v a0, const flex::float4v a1, bool nan_here) __attribute__((always_inline)) {
+    // four values of one output row, narrowed
+    auto put4 = [&](long prow, long col, const flex::float4v v, bool nan_here) __attribute__((always_inline)) {
         if (prow >= row_end || col >= p.N) return;
         std::uint16_t o[4];
-        if constexpr (kSwiglu) {
-            swiglu4_from_acc<T>(a0, a1, o);
-        } else {
 #pragma unroll
-            for (int r = 0; r < 4; ++r) o[r] = __builtin_expect(nan_here, 0) ? El::from_f32(a0[r]) : El::from_f32_finite(a0[r]);
-        }
+        for (int r = 0; r < 4; ++r) o[r] = __builtin_expect(nan_here, 0) ? El::from_f32(v[r]) : El::from_f32_finite(v[r]);
         if (col + 3 < p.N) {        // (N is a multiple of 64 here and the rows are 16-byte aligned)
             u32x2 w2;
             w2[0] = o[0] | (static_cast<std::uint32_t>(o[1]) << 16);
@@ -352,40 +343,14 @@ __global__ __launch_bounds__(flex::kThreads, 1) void grouped_gemm_direct_kernel(
     };
     auto any_nan = [&](float probe) { return __builtin_amdgcn_ballot_w64(probe != probe) != 0; };
 
-    if (row_end - row0 <= 64) {     // an expert's last tile with few rows: the waves share them
-        flex::Operand<2, false> oa;
-        aim_rows(oa, wm);
-        flex::float4v sacc[2][8];
-        flex::mainloop<T, 2, 8>(oa, ob, static_cast<int>(p.K), a0, a1, b0, b1, sacc);
-#pragma unroll
-        for (int i = 0; i < 2; ++i) {
-            const long prow = row0 + wm * 32 + i * 16 + l16;
-            bool nan_here = false;
-            if (!kSwiglu) {
-                float probe = 0.f;
-#pragma unroll
-                for (int j = 0; j < 8; ++j)
-#pragma unroll
-                    for (int r = 0; r < 4; ++r) probe += sacc[i][j][r];
-                nan_here = any_nan(probe);
-            }
-#pragma unroll
-            for (int jb = 0; jb < 4; ++jb) {
-                const long col = n0 + wn * 64 + jb * 16 + 4 * kq;
-                if (kSwiglu) {
-                    put4(prow, col, sacc[i][jb], sacc[i][4 + jb], false);
-                } else {
-                    put4(prow, col, sacc[i][jb], sacc[i][jb], nan_here);
-                    put4(prow, col + kBN, sacc[i][4 + jb], sacc[i][4 + jb], nan_here);
-                }
-            }
-        }
-        return;
-    }
-    flex::Operand<8, false> oa;
+    // The tile with 32 MI of its rows: an expert's last tile takes the fewest that hold its rows, with the same sums in the
+    // same order (64 rows about a third of a full tile's time, 128 rows two thirds).
+    auto tile = [&](auto mi) __attribute__((always_inline)) {
+    constexpr int MI = decltype(mi)::value;
+    flex::Operand<MI, false> oa;
     aim_rows(oa, wm);
-    flex::float4v acc[8][8];
-    flex::mainloop<T, 8, 8>(oa, ob, static_cast<int>(p.K), a0, a1, b0, b1, acc);
+    flex::float4v acc[MI][8];
+    flex::mainloop<T, MI, 8>(oa, ob, static_cast<int>(p.K), a0, a1, b0, b1, acc);
     if constexpr (kSwiglu) {
         // About one value in a thousand leaves the common tier of SwiGLU, and where one lane of the 64 does,
         // the whole wave walks through the fp64 formula: at 128 values a lane that happened eight times a tile
@@ -412,9 +377,9 @@ __global__ __launch_bounds__(flex::kThreads, 1) void grouped_gemm_direct_kernel(
             }
             queued = 0;
         };
-        quad16_static_for<8>([&](auto I) __attribute__((always_inline)) {
+        static_for<MI>([&](auto I) __attribute__((always_inline)) {
             constexpr int i = decltype(I)::value;
-            const int trow = wm * 128 + i * 16 + l16;
+            const int trow = wm * 16 * MI + i * 16 + l16;
             const long prow = row0 + trow;
 #pragma unroll
             for (int jb = 0; jb < 4; ++jb) {
@@ -447,35 +412,34 @@ __global__ __launch_bounds__(flex::kThreads, 1) void grouped_gemm_direct_kernel(
                 }
             }
             // a row block queues 4 x 64 entries at most
-            if (i == 7 || queued > SwigluQueue::kEntries - 256) work_off();
+            if (i == MI - 1 || queued > SwigluQueue::kEntries - 256) work_off();
         });
         return;
     }
     // (row blocks as constants of the front end: the optimiser's unroller gives up on a loop of 128
     // SwiGLU values with their exact tier, and the accumulators would move to scratch memory)
-    quad16_static_for<8>([&](auto I) __attribute__((always_inline)) {
+    static_for<MI>([&](auto I) __attribute__((always_inline)) {
         constexpr int i = decltype(I)::value;
-        const long prow = row0 + wm * 128 + i * 16 + l16;
-        bool nan_here = false;
-        if (!kSwiglu) {
-            float probe = 0.f;
+        const long prow = row0 + wm * 16 * MI + i * 16 + l16;
+        float probe = 0.f;
 #pragma unroll
-            for (int j = 0; j < 8; ++j)
+        for (int j = 0; j < 8; ++j)
 #pragma unroll
-                for (int r = 0; r < 4; ++r) probe += acc[i][j][r];
-            nan_here = any_nan(probe);
-        }
+            for (int r = 0; r < 4; ++r) probe += acc[i][j][r];
+        const bool nan_here = any_nan(probe);
 #pragma unroll
         for (int jb = 0; jb < 4; ++jb) {
             const long col = n0 + wn * 64 + jb * 16 + 4 * kq;
-            if (kSwiglu) {
-                put4(prow, col, acc[i][jb], acc[i][4 + jb], false);
-            } else {
-                put4(prow, col, acc[i][jb], acc[i][jb], nan_here);
-                put4(prow, col + kBN, acc[i][4 + jb], acc[i][4 + jb], nan_here);
-            }
+            put4(prow, col, acc[i][jb], nan_here);
+            put4(prow, col + kBN, acc[i][4 + jb], nan_here);
         }
     });
+    };      // tile
+    const long rows = row_end - row0;
+    if (rows > 192)      tile(std::integral_constant<int, 8>{});
+    else if (rows > 128) tile(std::integral_constant<int, 6>{});
+    else if (rows > 64)  tile(std::integral_constant<int, 4>{});
+    else                 tile(std::integral_constant<int, 2>{});
 }
 
 // ---- few rows per expert (decode-time batches): the layer is bound by streaming every active

@@ -293,6 +293,32 @@ def test_ffn_rows_in_the_last_tile_of_every_expert(dtype):
     assert_ffn_close(out.cpu()[sel], ref, dtype)
 
 
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])
+@pytest.mark.parametrize("H", [2048, 2112])
+def test_ffn_last_tiles_at_the_edges_of_their_forms(H, dtype):
+    """Last tiles of 127, 128, 129, 192, 193 and 255 rows (they run with 128, 192 or 256 rows), a contraction of an odd number of
+    k-tiles (2112 = 33 x 64, which also leaves a ragged last column unit of the down-projection)."""
+    torch.manual_seed(12)
+    counts_wanted = [1151, 1152, 1153, 1216, 1217, 1279]
+    E, k, I = len(counts_wanted), 2, 320
+    T = sum(counts_wanted) // k
+    rows = torch.repeat_interleave(torch.arange(E), torch.tensor(counts_wanted))
+    logits = 0.1 * torch.randn(T, E)
+    logits[torch.arange(T), rows[:T]] += 5.0
+    logits[torch.arange(T), rows[T:]] += 4.0
+    logits = logits.to(dtype)
+    x = torch.randn(T, H).to(dtype)
+    wg, wu, wd = (0.03 * torch.randn(E, I, H)).to(dtype), (0.03 * torch.randn(E, I, H)).to(dtype), (0.05 * torch.randn(E, H, I)).to(dtype)
+    topi, topw, order, inv, counts, offsets = capi.moe_route(logits.cuda(), k)
+    assert counts.cpu().tolist() == counts_wanted
+    out = capi.moe_ffn(x.cuda(), wg.cuda(), wu.cuda(), wd.cuda(), topw, order, inv, offsets, k)
+    off, ordr = offsets.cpu().tolist(), order.cpu()
+    tails = [(ordr[off[e] + (counts_wanted[e] - 1) // 256 * 256: off[e + 1]] // k)[-40:] for e in range(E)]
+    sel = torch.unique(torch.cat(tails))
+    r = O.moe_route(logits[sel], k)
+    assert_ffn_close(out.cpu()[sel], O.moe_ffn(x[sel], wg, wu, wd, r[1], r[2], r[3], r[5], k, gemm="aten"), dtype)
+
+
 @pytest.mark.parametrize("shape", [(8192, 8, 2, torch.bfloat16), (5000, 64, 6, torch.float32), (700, 16, 4, torch.float16)])
 def test_route_when_the_workgroups_do_not_wait_for_each_other(shape, monkeypatch):
     """With a wait of one poll most workgroups of the one-kernel routing stop waiting for the others
