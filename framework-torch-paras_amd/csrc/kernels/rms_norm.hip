@@ -352,6 +352,123 @@ __global__ __launch_bounds__(kBlock) void rms_norm_bwd_dw_final(
     gw[j] = E::from_f64(acc);
 }
 
+// The same in one pass, for what the 16-byte kernels below do not take (fp32 tensors, 16-bit rows that are not whole aligned
+// 16-byte pieces): a workgroup holds a row of g and x in registers, V adjacent elements at a time, and keeps the column sums
+// of its rows there too, so that g and x are read once instead of three times and there is a partial sum per resident workgroup
+// instead of one per 16 rows.  The next row is requested before the current one is reduced.  Bound by memory and, at
+// fp32 16384 x 4096, by the fp64 arithmetic beside it: 329 -> 147 us (0.81 GB: 5.5 TB/s); 20000 x 1000 98 -> 45; bf16 16384 x 4001
+// 234 -> 120, 20000 x 777 63 -> 32.  From kBwdRowsSlabs slabs of 16 rows and kBwdRowsElems elements on: with less, most of the
+// chip idles behind the rows of a few workgroups (fp32 1024 x 1024 13.8 us in three kernels, 16.3 this way; 2048 x 768 15.6
+// and 18.0; 4000 x 8192 162 and 107).
+constexpr long kBwdRowsSlabs = 64, kBwdRowsElems = 3000000;
+template <typename T, int V, int NV, int BLOCK>
+__global__ __launch_bounds__(BLOCK, 4) void rms_norm_bwd_rows(
+    const typename Elem<T>::store_t* __restrict__ go, const typename Elem<T>::store_t* __restrict__ x,
+    const typename Elem<T>::store_t* __restrict__ w, const float* __restrict__ rstd,
+    typename Elem<T>::store_t* __restrict__ gx, double* __restrict__ partial, long rows, int H) {
+    using E = Elem<T>;
+    using S = typename E::store_t;
+    typedef S vec __attribute__((ext_vector_type(V)));
+    constexpr int kWaves = BLOCK / kWave;
+    __shared__ double slots[2][kWaves];
+    int at[NV];                      // first element of each piece; pieces past the row's end read its first one and are not stored
+    bool live[NV];
+    constexpr bool kHoldW = NV * V <= 4;
+    S wv[NV][V];
+    double dw[NV][V];
+    auto load = [](const S* p, S (&v)[V]) __attribute__((always_inline)) {
+        if constexpr (V == 1) {
+            v[0] = *p;
+        } else {
+            const vec t = *reinterpret_cast<const vec*>(p);
+#pragma unroll
+            for (int c = 0; c < V; ++c) v[c] = t[c];
+        }
+    };
+#pragma unroll
+    for (int i = 0; i < NV; ++i) {
+        const int j = (static_cast<int>(threadIdx.x) + i * BLOCK) * V;
+        live[i] = j < H;
+        at[i] = live[i] ? j : 0;
+        if constexpr (kHoldW) load(w + at[i], wv[i]);
+#pragma unroll
+        for (int c = 0; c < V; ++c) dw[i][c] = 0.0;
+    }
+    // (with eight elements per thread the weights come from L1 again for every row: they do not fit beside the rest)
+    auto weight = [&](int i, int c) __attribute__((always_inline)) {
+        if constexpr (kHoldW) return wv[i][c];
+        else                  return w[at[i] + c];
+    };
+    S gn[NV][V], xn[NV][V];
+    double rn = 0.0;
+    auto request = [&](long r) __attribute__((always_inline)) {
+#pragma unroll
+        for (int i = 0; i < NV; ++i) {
+            load(go + r * H + at[i], gn[i]);
+            load(x + r * H + at[i], xn[i]);
+        }
+        rn = static_cast<double>(rstd[r]);
+    };
+    long r = blockIdx.x;             // (the grid has no more workgroups than rows)
+    request(r);
+    int turn = 0;
+    for (; r < rows; r += gridDim.x, turn ^= 1) {
+        S g[NV][V], xx[NV][V];
+        const double rr = rn;
+#pragma unroll
+        for (int i = 0; i < NV; ++i)
+#pragma unroll
+            for (int c = 0; c < V; ++c) {
+                g[i][c] = gn[i][c];
+                xx[i][c] = xn[i][c];
+            }
+        request(r + gridDim.x < rows ? r + gridDim.x : r);
+        double dot = 0.0;
+#pragma unroll
+        for (int i = 0; i < NV; ++i)
+#pragma unroll
+            for (int c = 0; c < V; ++c) {
+                const double gj = E::to_f64(g[i][c]), xj = E::to_f64(xx[i][c]);
+                dw[i][c] += gj * xj * rr;
+                if (live[i]) dot += gj * E::to_f64(weight(i, c)) * xj;
+            }
+#pragma unroll
+        for (int o = kWave / 2; o > 0; o >>= 1) dot += __shfl_xor(dot, o, kWave);
+        if constexpr (kWaves > 1) {
+            if ((threadIdx.x & (kWave - 1)) == 0) slots[turn][threadIdx.x / kWave] = dot;
+            lds_barrier();           // (two sets of slots: the next row's sums do not meet a wave that still reads these)
+            dot = slots[turn][0];
+#pragma unroll
+            for (int v = 1; v < kWaves; ++v) dot += slots[turn][v];
+        }
+        const double coef = rr * rr * rr / static_cast<double>(H);
+#pragma unroll
+        for (int i = 0; i < NV; ++i) {
+            if (!live[i]) continue;
+            S o[V];
+#pragma unroll
+            for (int c = 0; c < V; ++c) {
+                const double gj = E::to_f64(g[i][c]), wj = E::to_f64(weight(i, c)), xj = E::to_f64(xx[i][c]);
+                o[c] = E::from_f64(gj * wj * rr - coef * xj * dot);
+            }
+            S* dst = gx + r * H + at[i];
+            if constexpr (V == 1) {
+                *dst = o[0];
+            } else {
+                vec t;
+#pragma unroll
+                for (int c = 0; c < V; ++c) t[c] = o[c];
+                *reinterpret_cast<vec*>(dst) = t;
+            }
+        }
+    }
+#pragma unroll
+    for (int i = 0; i < NV; ++i)
+        if (live[i])
+#pragma unroll
+            for (int c = 0; c < V; ++c) partial[static_cast<long>(blockIdx.x) * H + at[i] + c] = dw[i][c];
+}
+
 // ---- the row arithmetic of the one-pass backward kernels (one 16-byte vector of 8 elements) ----
 // First half: widen g and x, accumulate the row's dot product and the column sums.
 template <typename T>
@@ -983,6 +1100,45 @@ int launch_bwd(const void* go, const void* x, const void* w, const float* rstd, 
             else                     PARAS_BWD_LAUNCH(1024, false);
 #undef PARAS_BWD_LAUNCH_TEAMS
 #undef PARAS_BWD_LAUNCH
+            PARAS_HIP_TRY(hipGetLastError());
+            hipLaunchKernelGGL((rms_norm_bwd_dw_final_wide<T>), dim3(static_cast<unsigned>((H + kDwFinalCols - 1) / kDwFinalCols)), dim3(kDwFinalLanes * kDwFinalCols), 0, s,
+                               part, static_cast<S*>(gw), slabs, H);
+            PARAS_HIP_TRY(hipGetLastError());
+            return PARAS_OK;
+        }
+    }
+    if constexpr (sizeof(S) <= 4) {
+        if (slabs >= kBwdRowsSlabs && rows * H >= kBwdRowsElems && H <= 8192) {
+            int dev = 0;
+            (void)hipGetDevice(&dev);
+            auto* dst = DeviceContext::instance().device(dev);
+            const int block = H <= 1024 ? 256 : (H <= 2048 ? 512 : 1024);
+            const long resident = (dst ? dst->compute_units : 256) * (1024 / block);
+            if (slabs > resident) slabs = resident;          // a partial sum each: the workspace has one per 16 rows
+            const dim3 grid(static_cast<unsigned>(slabs));
+            auto* part = static_cast<double*>(workspace);
+            // pieces of 16 bytes where fp32 rows consist of them
+            const bool pieces = sizeof(S) == 4 && H % 4 == 0 &&
+                                ((reinterpret_cast<uintptr_t>(go) | reinterpret_cast<uintptr_t>(x) | reinterpret_cast<uintptr_t>(w) |
+                                  reinterpret_cast<uintptr_t>(gx)) & 15) == 0;
+#define PARAS_BWD_ROWS(V_, NV_, BLOCK_)                                                                              \
+    hipLaunchKernelGGL((rms_norm_bwd_rows<T, V_, NV_, BLOCK_>), grid, dim3(BLOCK_), 0, s, static_cast<const S*>(go), \
+                       static_cast<const S*>(x), static_cast<const S*>(w), rstd, static_cast<S*>(gx), part, rows, (int)H)
+            bool launched = false;
+            if constexpr (sizeof(S) == 4) {
+                launched = pieces;
+                if (!pieces)        {}
+                else if (H <= 1024) PARAS_BWD_ROWS(4, 1, 256);
+                else if (H <= 2048) PARAS_BWD_ROWS(4, 1, 512);
+                else if (H <= 4096) PARAS_BWD_ROWS(4, 1, 1024);
+                else                PARAS_BWD_ROWS(4, 2, 1024);
+            }
+            if (launched)       {}
+            else if (H <= 1024) PARAS_BWD_ROWS(1, 4, 256);
+            else if (H <= 2048) PARAS_BWD_ROWS(1, 4, 512);
+            else if (H <= 4096) PARAS_BWD_ROWS(1, 4, 1024);
+            else                PARAS_BWD_ROWS(1, 8, 1024);
+#undef PARAS_BWD_ROWS
             PARAS_HIP_TRY(hipGetLastError());
             hipLaunchKernelGGL((rms_norm_bwd_dw_final_wide<T>), dim3(static_cast<unsigned>((H + kDwFinalCols - 1) / kDwFinalCols)), dim3(kDwFinalLanes * kDwFinalCols), 0, s,
                                part, static_cast<S*>(gw), slabs, H);

@@ -375,3 +375,28 @@ def test_signed_zeros_infinities_and_nans_come_out_as_on_the_host(dtype):
             assert_bit_exact(got, want, f"rotate_half {dtype} backward={backward}")
         else:
             assert_same_bits_nan_aware(got, want, f"rotate_half {dtype} backward={backward}")
+
+
+@pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16, torch.float16])
+@pytest.mark.parametrize("shape", [(12000, 257), (3100, 1000), (3000, 1024), (3000, 1028), (1600, 2049), (1600, 2048), (1024, 4095),
+                                   (1024, 4100), (1024, 8191), (1024, 8192), (1024, 8193), (90000, 36), (1008, 3000)])
+def test_rms_norm_backward_rows_in_registers(shape, dtype):
+    """Enough rows for the one-pass kernel of fp32 tensors and of rows that are not whole 16-byte pieces: widths at the edges of its
+    block sizes, more rows than resident workgroups, and the sizes just outside it; an infinity and a NaN stay in their row and column."""
+    rows, H = shape
+    torch.manual_seed(rows + H)
+    x, w, go = torch.randn(rows, H).to(dtype), (1 + 0.1 * torch.randn(H)).to(dtype), torch.randn(rows, H).to(dtype)
+    _, rstd = O.rms_norm(x, w, 1e-6)
+    go[3, 0], go[rows - 1, H // 2] = float("inf"), float("nan")
+    gx, gw = capi.rms_norm_backward(dev(go), dev(x), dev(w), dev(rstd))
+    wgx, wgw = O.rms_norm_backward(go, x, w, rstd)
+    for got, want, what in ((gx, wgx, "grad_input"), (gw, wgw, "grad_weight")):
+        got = got.cpu()
+        assert torch.equal(got.isnan(), want.isnan()), what
+        ok = ~want.isnan()
+        # fp64 sums in another order, one rounding: a neighbouring value where the sum lies next to a boundary, else the same bits
+        err = (got[ok].double() - want[ok].double()).abs()
+        err[got[ok] == want[ok]] = 0.0
+        eps = {torch.float32: 2.0 ** -23, torch.bfloat16: 2.0 ** -7, torch.float16: 2.0 ** -10}[dtype]
+        assert bool((err <= eps * want[ok].double().abs() + 1e-12).all()), what
+        assert int((err > 0).sum()) <= 2 + want.numel() // 10000, what
