@@ -233,8 +233,8 @@ def test_flash_key_padding_masks_at_the_edges_of_a_block(dtype, D):
     keep = (torch.arange(Lk)[None, :] < torch.tensor(lens)[:, None]).reshape(B, 1, 1, Lk)
     one = torch.ones(1, 1, 77, Lk, dtype=torch.bool)
     one[0, 0, 40, 70] = False
-    scale = O.round_to_dtype(1 / math.sqrt(D), dtype)
-    for mask in (keep, one):
+    narrowed = O.round_to_dtype(1 / math.sqrt(D), dtype)
+    for mask, scale in ((keep, narrowed), (one, narrowed), (keep, 0.1013)):      # (0.1013 is no number of either type)
         out, _, _, kern = run(q, k, v, mask=mask, scale=scale)
         want, _ = O.sdpa_math(q, k, v, attn_mask=mask, gemm="aten", scale=scale)
         assert kern.startswith("flash_mfma")
