@@ -236,7 +236,12 @@ def test_flash_key_padding_masks_at_the_edges_of_a_block(dtype, D):
     narrowed = O.round_to_dtype(1 / math.sqrt(D), dtype)
     for mask, scale in ((keep, narrowed), (one, narrowed), (keep, 0.1013)):      # (0.1013 is no number of either type)
         out, _, _, kern = run(q, k, v, mask=mask, scale=scale)
-        want, _ = O.sdpa_math(q, k, v, attn_mask=mask, gemm="aten", scale=scale)
+        if scale == narrowed:
+            want, _ = O.sdpa_math(q, k, v, attn_mask=mask, gemm="aten", scale=scale)
+        else:       # (the oracle narrows the scale first; the C ABI takes it as it is: the same steps with the scale in fp32)
+            sc = (q.double() @ k.double().transpose(-1, -2)).to(dtype)
+            sc = (sc.float() * torch.tensor(scale, dtype=torch.float32)).to(dtype).double().masked_fill(~mask, -math.inf)
+            want = torch.softmax(sc, -1) @ v.double()
         assert kern.startswith("flash_mfma")
         err = (out.double().cpu() - want.double()).abs().max().item()
         assert err <= (2.5e-2 if dtype == torch.bfloat16 else 4e-3), err     # a step of the type on values up to 4: 2^-7 x 2 (2^-10 x 2), and rounding of the weights
