@@ -12,7 +12,6 @@
 //    decode kernels serve every shape they accept (anything else still goes to
 //    the math-semantics kernel inside libparas_hip.so).
 #include <ATen/NativeFunctions.h>
-#include <ATen/TensorSubclassLikeUtils.h>
 #include <ATen/native/DispatchStub.h>
 #include <ATen/native/transformers/attention.h>
 #include <ATen/native/transformers/sdp_utils_cpp.h>
@@ -220,13 +219,12 @@ int64_t fused_sdp_choice(const Tensor& query, const Tensor& key, const Tensor& v
 // masked_fill: none of them device ops here, so the mask crosses to the host and back, 90 us of a 98 us
 // call), ask fused_sdp_choice, and have the fused op fill nine results of which one is used.  The kernels
 // read a boolean mask as it is, so a call that would end in the fused op goes straight to them; anything
-// else -- gradients, dropout, operands the composite would refuse or convert -- is left to it.
+// else -- gradients, tangents, dropout, operands the composite would refuse or convert -- is left to it.
 Tensor sdpa(const Tensor& query, const Tensor& key, const Tensor& value, const c10::optional<Tensor>& attn_mask, double dropout_p,
             bool is_causal, c10::optional<double> scale, bool enable_gqa) {
     const bool has_mask = attn_mask.has_value() && attn_mask->defined();
     auto alike = [&](const Tensor& t) {
-        return is_paras(t) && t.device() == query.device() && t.scalar_type() == query.scalar_type() && t.dim() == query.dim() &&
-               !at::isTensorSubclassLike(t);
+        return is_paras(t) && t.device() == query.device() && t.scalar_type() == query.scalar_type() && t.dim() == query.dim() && plain(t);
     };
     bool direct = dropout_p == 0.0 && query.dim() >= 3 && float_code(query.scalar_type()) >= 0 && alike(query) && alike(key) && alike(value) &&
                   !needs_grad(query, key, value) && (enable_gqa || key.size(-3) == query.size(-3) || key.size(-3) == 1);

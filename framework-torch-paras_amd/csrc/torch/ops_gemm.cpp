@@ -7,7 +7,6 @@
 #include "paras_torch.h"
 
 #include <ATen/NativeFunctions.h>
-#include <ATen/TensorSubclassLikeUtils.h>
 #include <torch/csrc/autograd/custom_function.h>
 
 namespace paras_torch {
@@ -170,7 +169,7 @@ struct LinearFunction : torch::autograd::Function<LinearFunction> {
 Tensor linear(const Tensor& x, const Tensor& w, const c10::optional<Tensor>& bias_opt) {
     const Tensor bias = bias_opt.has_value() ? *bias_opt : Tensor();
     auto alike = [&](const Tensor& t) {
-        return is_paras(t) && t.device() == x.device() && t.scalar_type() == x.scalar_type() && !at::isTensorSubclassLike(t);
+        return is_paras(t) && t.device() == x.device() && t.scalar_type() == x.scalar_type() && plain(t);
     };
     const bool direct = x.dim() >= 1 && w.dim() == 2 && is_float(x) && alike(x) && alike(w) && x.size(-1) == w.size(1) && w.numel() > 0 &&
                         x.numel() > 0 && (!bias.defined() || (alike(bias) && bias.dim() == 1 && bias.size(0) == w.size(0)));

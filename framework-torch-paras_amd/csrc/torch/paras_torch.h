@@ -7,6 +7,7 @@
 
 #include <ATen/ATen.h>
 #include <c10/core/Device.h>
+#include <c10/core/impl/TorchDispatchModeTLS.h>
 #include <c10/util/Exception.h>
 #include <torch/library.h>
 
@@ -89,9 +90,22 @@ at::Tensor empty_paras(c10::IntArrayRef sizes, c10::ScalarType dtype, c10::Devic
 
 inline at::Tensor empty_paras_like(const at::Tensor& t) { return empty_paras(t.sizes(), t.scalar_type(), t.device()); }
 
-// Whether autograd has to see an op with these inputs.
+// Whether autograd has to see an op with these inputs: for their gradients, or for a tangent that one of them
+// carries (a dual tensor of forward-mode differentiation, whose requires_grad() is false as a rule).
+inline bool has_tangent(const at::Tensor& t) { return t.defined() && t._fw_grad(/*level=*/0).defined(); }
 template <typename... Ts>
-bool needs_grad(const Ts&... t) { return at::GradMode::is_enabled() && (... || (t.defined() && t.requires_grad())); }
+bool needs_grad(const Ts&... t) {
+    return (... || has_tangent(t)) || (at::GradMode::is_enabled() && (... || (t.defined() && t.requires_grad())));
+}
+
+// Whether an op registered above autograd may read t's memory and leave out the ops below it that its composite form
+// is made of: a dense `paras` tensor without a tangent that nothing wraps, batches, negates, names or watches
+// (no key in its set but the device's own, no dispatch mode active).
+inline bool plain(const at::Tensor& t) {
+    constexpr c10::DispatchKeySet own({c10::DispatchKey::PrivateUse1, c10::DispatchKey::AutogradPrivateUse1,
+                                       c10::DispatchKey::ADInplaceOrView, c10::DispatchKey::AutocastPrivateUse1});
+    return own.has_all(t.key_set()) && !has_tangent(t) && !c10::impl::dispatch_mode_enabled();
+}
 
 // Differentiable forms of the fused ops and the MoE layer, for torch_paras.nn.
 at::Tensor nn_rms_norm(const at::Tensor& input, const at::Tensor& weight, double eps);

@@ -7,6 +7,7 @@ import math
 
 import pytest
 import torch
+import torch.autograd.forward_ad as fwAD
 import torch.nn.functional as F
 
 import oracle as O
@@ -949,3 +950,41 @@ def test_binary_ops_on_views_with_contiguous_rows_match_the_host(dtype):
     got = a.to("paras:0")
     got.mul_(b.to("paras:0"))
     assert torch.equal(got.cpu(), a * b)
+
+
+@pytest.mark.parametrize("with_grad", [False, True])
+@pytest.mark.parametrize("which", [0, 1, 2])
+def test_linear_carries_forward_mode_tangents(device, which, with_grad):
+    """A dual input of F.linear (the input, the weight or the bias), with and without gradients asked for beside it: the
+    tangent of the output against the CPU's, and the gradient of what was computed from it."""
+    ins = [torch.randn(3, 5, 8), torch.randn(7, 8), torch.randn(7)]
+    tan = torch.randn_like(ins[which])
+
+    def both(place):
+        args = [t.to(place).requires_grad_(with_grad) for t in ins]
+        with fwAD.dual_level():
+            duals = list(args)
+            duals[which] = fwAD.make_dual(duals[which], tan.to(place))
+            y, t = fwAD.unpack_dual(F.linear(*duals))
+            assert t is not None, "the tangent was dropped"
+            return [y.detach(), t.detach(), *(torch.autograd.grad(y.sum(), args) if with_grad else [])]
+
+    for got, want in zip(both(device), both("cpu")):
+        assert_close(got, want)
+
+
+def test_forward_mode_is_refused_where_no_derivative_is_known(device):
+    """The fused ops and the fused attention have no forward-mode derivative: a dual input raises, whether or not it
+    asks for gradients as well, instead of coming out without its tangent."""
+    import torch_paras
+    nn = torch_paras.nn
+    x, w, q = torch.randn(3, 8), torch.randn(8), torch.randn(1, 2, 16, 64)
+    calls = {"rms_norm": (nn.rms_norm, x, w), "swiglu": (nn.swiglu, x, x), "rotate_half": (nn.rotate_half, x),
+             "attention": (F.scaled_dot_product_attention, q, q, q)}
+    for name, (f, *args) in calls.items():
+        for with_grad in (False, True) if name != "attention" else (False,):
+            for which in range(len(args)):
+                ins = [a.to(device).requires_grad_(with_grad) for a in args]
+                with fwAD.dual_level(), pytest.raises(RuntimeError, match="jvp|forward AD"):
+                    ins[which] = fwAD.make_dual(ins[which], torch.ones_like(args[which]).to(device))
+                    f(*ins)
