@@ -229,7 +229,7 @@ Tensor sdpa(const Tensor& query, const Tensor& key, const Tensor& value, const c
     bool direct = dropout_p == 0.0 && query.dim() >= 3 && float_code(query.scalar_type()) >= 0 && alike(query) && alike(key) && alike(value) &&
                   !needs_grad(query, key, value) && (enable_gqa || key.size(-3) == query.size(-3) || key.size(-3) == 1);
     if (has_mask)
-        direct = direct && !is_causal && is_paras(*attn_mask) && attn_mask->device() == query.device() && !needs_grad(*attn_mask) &&
+        direct = direct && !is_causal && is_paras(*attn_mask) && attn_mask->device() == query.device() && plain(*attn_mask) && !needs_grad(*attn_mask) &&
                  attn_mask->dim() >= 2 && (attn_mask->scalar_type() == c10::kBool || attn_mask->scalar_type() == query.scalar_type());
     if (!direct) return at::native::scaled_dot_product_attention(query, key, value, attn_mask, dropout_p, is_causal, scale, enable_gqa);
     Prepared p;

@@ -988,3 +988,30 @@ def test_forward_mode_is_refused_where_no_derivative_is_known(device):
                 with fwAD.dual_level(), pytest.raises(RuntimeError, match="jvp|forward AD"):
                     ins[which] = fwAD.make_dual(ins[which], torch.ones_like(args[which]).to(device))
                     f(*ins)
+
+
+class _Held(torch.Tensor):
+    """A wrapper subclass: it has a shape and a device but no memory of its own, only the tensor that it holds."""
+    @staticmethod
+    def __new__(cls, inner):
+        t = torch.Tensor._make_wrapper_subclass(cls, inner.shape, dtype=inner.dtype, device=inner.device)
+        t.inner = inner
+        return t
+
+    @classmethod
+    def __torch_dispatch__(cls, func, types, args=(), kwargs=None):
+        free = lambda t: t.inner if isinstance(t, cls) else t
+        tree_map = torch.utils._pytree.tree_map
+        return func(*tree_map(free, args), **tree_map(free, kwargs or {}))
+
+
+@pytest.mark.parametrize("held", ["q", "k", "v", "mask"])
+def test_attention_operands_that_wrap_another_tensor(device, held):
+    """A tensor subclass in the place of any operand, the mask included, is left to the composite op, which unwraps it."""
+    q, k, v, qd, kd, vd = _qkv(device, Lq=20, Lk=33, E=64)
+    mask = torch.rand(2, 1, 20, 33) < 0.7
+    mask[..., 0] = True
+    ops = dict(q=qd, k=kd, v=vd, mask=mask.to(device))
+    ops[held] = _Held(ops[held])
+    got = F.scaled_dot_product_attention(ops["q"], ops["k"], ops["v"], attn_mask=ops["mask"])
+    assert_close(got, F.scaled_dot_product_attention(q, k, v, attn_mask=mask))
