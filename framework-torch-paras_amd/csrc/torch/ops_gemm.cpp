@@ -153,7 +153,9 @@ struct LinearFunction : torch::autograd::Function<LinearFunction> {
         const bool want_x = ctx->needs_input_grad(0), want_w = ctx->needs_input_grad(1);
         const bool want_b = ctx->saved_data.count("bias") != 0 && ctx->needs_input_grad(2);
         Tensor gx, gw, gb;
-        if (at::GradMode::is_enabled()) {           // a graph of the backward is wanted: differentiable ops
+        // a graph of the backward is wanted, or a gradient is a batch of gradients, a dual tensor or wrapped: dispatcher ops
+        const bool composite = at::GradMode::is_enabled() || !plain(dy) || (want_x && !plain(w)) || (want_w && !plain(x));
+        if (composite) {
             if (want_x) gx = at::mm(dy, w).view(x_sizes);
             if (want_w) gw = at::mm(dy.t(), rows_of(x));
             if (want_b) gb = dy.sum(0);

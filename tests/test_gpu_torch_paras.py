@@ -1015,3 +1015,26 @@ def test_attention_operands_that_wrap_another_tensor(device, held):
     ops[held] = _Held(ops[held])
     got = F.scaled_dot_product_attention(ops["q"], ops["k"], ops["v"], attn_mask=ops["mask"])
     assert_close(got, F.scaled_dot_product_attention(q, k, v, attn_mask=mask))
+
+
+@pytest.mark.parametrize("lead", [(5,), (2, 7)])
+def test_linear_backward_of_gradients_that_are_not_plain_tensors(device, lead):
+    """The backward of F.linear under torch.autograd.grad(is_grads_batched=True), where the incoming gradient is a batch of
+    gradients, and with a dual tensor as incoming gradient (forward over reverse): against the CPU."""
+    ins = [torch.randn(*lead, 8), torch.randn(6, 8), torch.randn(6)]
+    dys, tan = torch.randn(4, *lead, 6), torch.randn(*lead, 6)
+
+    def both(place):
+        args = [t.to(place).requires_grad_() for t in ins]
+        y = F.linear(*args)
+        out = list(torch.autograd.grad(y, args, dys.to(place), is_grads_batched=True, retain_graph=True))
+        with fwAD.dual_level():
+            dual = fwAD.make_dual(dys[0].to(place), tan.to(place))
+            for g in torch.autograd.grad(y, args, dual):
+                out += list(fwAD.unpack_dual(g))
+        return out
+
+    got, want = both(device), both("cpu")
+    assert all(t is not None for t in got)
+    for g, w in zip(got, want):
+        assert_close(g, w)
