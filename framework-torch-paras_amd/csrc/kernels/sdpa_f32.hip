@@ -139,12 +139,32 @@ __global__ __launch_bounds__(kWavesF * 64) void sdpa_f32_kernel(const F32Params 
     const float scale = static_cast<float>(p.scale);         // (already rounded to fp32 by the caller, so this is exact)
     // 32 keys of more than 128 elements leave no registers for operands ahead of time: they are requested where they are used
     constexpr bool kAhead = DM <= 128 || sizeof(Acc) == 8;
+    // A turn that no query of the tile sees: its weights are zeros whatever its scores are, but zero times a value that is
+    // not finite is NaN, as in the reference's full product.  Each value times zero, then one product per block of the
+    // output (A = those, B = zeros) that carries a NaN to its column of every query and changes nothing else.
+    auto unseen_turn = [&](int j0) {
+        load_v(j0);
+#pragma unroll
+        for (int c = 0; c < VC; ++c)
+#pragma unroll
+            for (int e = 0; e < 4; ++e) {
+                float z = 0.0f;
+#pragma unroll
+                for (int kb = 0; kb < KB; ++kb)
+#pragma unroll
+                    for (int t = 0; t < 4; ++t) z = fmaf(vf[kb][t][c][e], 0.0f, z);
+#pragma unroll
+                for (int qb = 0; qb < QB; ++qb) o[qb][c][e] = M::run(z, static_cast<Acc>(0), o[qb][c][e]);
+            }
+    };
     if (kAhead && wave * kTurn < keys) load_k(wave * kTurn);
-    for (int j0 = wave * kTurn; j0 < keys; j0 += kWavesF * kTurn) {
-        // the mask ahead of everything else: a turn that no query of the tile sees is passed over
+    int j0 = wave * kTurn;
+    for (; j0 < keys; j0 += kWavesF * kTurn) {
+        // the mask ahead of everything else: a turn that a boolean mask closes to every query of the tile needs no scores (an
+        // additive mask does not close anything: a NaN or +inf score plus -inf is NaN)
         float mk[QB][KB][4];                          // additive values; bool: 0 where attended, -inf elsewhere
         if constexpr (kMask != 0) {
-            bool any = false;
+            bool any = kMask == 2;
 #pragma unroll
             for (int qb = 0; qb < QB; ++qb) {
                 const long mrow = b * p.ms[0] + h * p.ms[1] + static_cast<long>(min(q0 + 16 * qb + l16, p.Lq - 1)) * p.ms[2];
@@ -155,10 +175,11 @@ __global__ __launch_bounds__(kWavesF * 64) void sdpa_f32_kernel(const F32Params 
                         const long at = mrow + static_cast<long>(min(j0 + 16 * kb + M::row(g, r), p.Lk - 1)) * p.ms[3];
                         if constexpr (kMask == 1) mk[qb][kb][r] = static_cast<const unsigned char*>(p.mask)[at] != 0 ? 0.0f : -INFINITY;
                         else                      mk[qb][kb][r] = static_cast<const float*>(p.mask)[at];
-                        any = any || mk[qb][kb][r] != -INFINITY;
+                        if constexpr (kMask == 1) any = any || mk[qb][kb][r] == 0.0f;
                     }
             }
-            if (__builtin_amdgcn_ballot_w64(any) == 0) {
+            if (kMask == 1 && __builtin_amdgcn_ballot_w64(any) == 0) {
+                unseen_turn(j0);
                 if (kAhead && j0 + kWavesF * kTurn < keys) load_k(j0 + kWavesF * kTurn);
                 continue;
             }
@@ -190,7 +211,9 @@ __global__ __launch_bounds__(kWavesF * 64) void sdpa_f32_kernel(const F32Params 
                 for (int r = 0; r < 4; ++r) {
                     const int j = j0 + 16 * kb + M::row(g, r);
                     float y = static_cast<float>(s[qb][kb][r]) * scale;
-                    if constexpr (kMask != 0) y += mk[qb][kb][r];       // (bool: + 0 or - inf)
+                    // (selected where a mask is boolean: a NaN or infinite score of a masked key is no score)
+                    if constexpr (kMask == 1) y = mk[qb][kb][r] == 0.0f ? y : -INFINITY;
+                    if constexpr (kMask == 2) y += mk[qb][kb][r];
                     if (j >= p.Lk || (p.is_causal && j > i)) y = -INFINITY;
                     x[kb][r] = y;
                     mx = fmaxf(mx, y);
@@ -228,6 +251,10 @@ __global__ __launch_bounds__(kWavesF * 64) void sdpa_f32_kernel(const F32Params 
 #pragma unroll
                         for (int qb = 0; qb < QB; ++qb) o[qb][c][e] = M::run(vf[kb][t][c][e], pr[qb][kb][t], o[qb][c][e]);
     }
+
+    // what the causal rule hides from the whole tile
+    if constexpr (kMask == 0)
+        for (; j0 < p.Lk; j0 += kWavesF * kTurn) unseen_turn(j0);
 
     // the waves meet
 #pragma unroll

@@ -816,3 +816,36 @@ def test_fp32_one_pass_kernel(B, Hq, Hkv, Lq, Lk, D, Dv, kind):
     assert (out.cpu().double()[ok] - want[ok]).abs().max().item() <= 3e-6 * want[ok].abs().max().item()
     want_lse = torch.logsumexp(s, -1)
     assert torch.allclose(lse.cpu().double()[want_lse.isfinite()], want_lse[want_lse.isfinite()], rtol=1e-6, atol=2e-6)
+
+
+@pytest.mark.parametrize("kind", ["causal", "bool", "additive"])
+@pytest.mark.parametrize("H,Lq,Lk,D,Dv", [(2, 40, 200, 64, 64), (2, 70, 60, 128, 40), (2, 33, 260, 256, 128), (4, 512, 512, 64, 64), (4, 530, 700, 128, 128),
+                                          (2, 300, 400, 256, 256)])
+def test_fp32_values_that_are_not_finite_behind_a_mask(H, Lq, Lk, D, Dv, kind):
+    """NaN and infinity in keys and values that a mask hides from some queries or from all of them, small problems (fp64
+    sums) and large ones (fp32): NaN in the same outputs as the reference's composition -- the boolean mask and the causal
+    rule select, so a hidden key is no score; an additive -inf is added, so a hidden NaN stays; the weights multiply every
+    value, so zero times NaN is NaN -- and the other outputs right."""
+    q, k, v = torch.randn(1, H, Lq, D), torch.randn(1, H, Lk, D), torch.randn(1, H, Lk, Dv)
+    keep = torch.rand(1, 1, Lq, Lk) < 0.7
+    keep[..., 32:192] = False                                          # whole turns of keys that nobody sees
+    keep[..., 0] = True
+    if kind == "causal":
+        keep = torch.ones(Lq, Lk).tril().bool()[None, None]
+    add = torch.zeros(1, 1, Lq, Lk).masked_fill(~keep, -math.inf)
+    kw = dict(is_causal=True) if kind == "causal" else dict(mask=keep if kind == "bool" else add)
+
+    def want(k, v):
+        s = q.double() @ k.double().transpose(-1, -2) / math.sqrt(D)
+        s = s + add.double() if kind == "additive" else s.masked_fill(~keep, -math.inf)
+        return s.softmax(-1) @ v.double()
+
+    for what, row, col in (("k", 50, 3), ("k", Lk - 1, D - 1), ("k", 20, 0), ("v", 50, 3), ("v", Lk - 1, Dv - 1), ("v", 20, 0), ("v", 0, 7)):
+        for bad in (math.nan, math.inf, -math.inf):
+            k2, v2 = k.clone(), v.clone()
+            (k2 if what == "k" else v2)[0, 0, row, col] = bad
+            out, exp = run(q, k2, v2, **kw)[0].cpu().double(), want(k2, v2)
+            same = torch.equal(out.isnan(), exp.isnan()) and torch.equal(out.isinf(), exp.isinf())
+            assert same, f"{what}[{row}, {col}] = {bad}: {int(out.isnan().sum())} NaN outputs, {int(exp.isnan().sum())} expected"
+            ok = exp.isfinite()
+            assert (out[ok] - exp[ok]).abs().max().item() <= 3e-6 * exp[ok].abs().max().item()
