@@ -136,7 +136,6 @@ __global__ __launch_bounds__(kWavesF * 64) void sdpa_f32_kernel(const F32Params 
             for (int e = 0; e < 4; ++e) o[qb][c][e] = vec{0, 0, 0, 0};
     }
     const int keys = p.is_causal ? min(p.Lk, q0 + 16 * QB) : p.Lk;
-    const float scale = static_cast<float>(p.scale);         // (already rounded to fp32 by the caller, so this is exact)
     // 32 keys of more than 128 elements leave no registers for operands ahead of time: they are requested where they are used
     constexpr bool kAhead = DM <= 128 || sizeof(Acc) == 8;
     // A turn that no query of the tile sees: its weights are zeros whatever its scores are, but zero times a value that is
@@ -210,7 +209,8 @@ __global__ __launch_bounds__(kWavesF * 64) void sdpa_f32_kernel(const F32Params 
 #pragma unroll
                 for (int r = 0; r < 4; ++r) {
                     const int j = j0 + 16 * kb + M::row(g, r);
-                    float y = static_cast<float>(s[qb][kb][r]) * scale;
+                    // (the scale as it is given: in fp64, rounded once; the torch ops narrow it themselves)
+                    float y = static_cast<float>(static_cast<double>(static_cast<float>(s[qb][kb][r])) * p.scale);
                     // (selected where a mask is boolean: a NaN or infinite score of a masked key is no score)
                     if constexpr (kMask == 1) y = mk[qb][kb][r] == 0.0f ? y : -INFINITY;
                     if constexpr (kMask == 2) y += mk[qb][kb][r];

@@ -849,3 +849,22 @@ def test_fp32_values_that_are_not_finite_behind_a_mask(H, Lq, Lk, D, Dv, kind):
             assert same, f"{what}[{row}, {col}] = {bad}: {int(out.isnan().sum())} NaN outputs, {int(exp.isnan().sum())} expected"
             ok = exp.isfinite()
             assert (out[ok] - exp[ok]).abs().max().item() <= 3e-6 * exp[ok].abs().max().item()
+
+
+@pytest.mark.parametrize("S,H", [(128, 4), (512, 8)])
+def test_fp32_scale_is_taken_as_given(S, H):
+    """The scale of the C ABI is a double and multiplies the fp32 products exactly as given, in the small and in the large
+    form.  Products of small whole numbers are exact in fp32, so the log-sum-exp is off by the scaled scores' and its own
+    rounding to fp32 only, and lies nearer to the given scale's than to the narrowed one's (2^-24.5 of each score away)."""
+    q, k = (torch.randint(-8, 9, (1, H, S, 64)).float() for _ in range(2))
+    v = torch.randn(1, H, S, 64)
+    scale = 0.5 + 2.0 ** -25.5                                         # 0.5 in fp32
+    out, _, lse, _ = run(q, k, v, scale=scale, want_lse=True)
+    dots = q.double() @ k.double().transpose(-1, -2)
+
+    def lse_of(scale):
+        return torch.logsumexp((dots * scale).float().double(), -1)
+
+    got = lse.cpu().double()
+    assert (got - lse_of(scale)).norm().item() < 0.6 * (got - lse_of(0.5)).norm().item()
+    assert rel_err(out, (dots * scale).float().double().softmax(-1) @ v.double()) <= 1e-6
