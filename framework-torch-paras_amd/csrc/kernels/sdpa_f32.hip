@@ -17,9 +17,10 @@
 // is free as long as both operands agree, and O^T then ends up with 4 adjacent elements of a row in a lane.
 // K of the next turn and V of this one are requested before the turn's products.
 //
-// Acc = double: v_mfma_f64_16x16x4 (78 TFLOP/s published), softmax in fp64: what the general kernel
-// computes, for the problems that it served.  Acc = float: v_mfma_f32_16x16x4 (157 TFLOP/s), for the large
-// ones, which the batched products accumulated in fp32.  Scores are rounded to fp32 where the reference's
+// Acc = double: v_mfma_f64_16x16x4 (78 TFLOP/s published): what the general kernel computes, for the problems that it
+// served.  Acc = float: v_mfma_f32_16x16x4 (157 TFLOP/s), for the large ones, which the batched products
+// accumulated in fp32.  In both the softmax is fp64: exponentials and row sums unrounded, a weight rounded once, to
+// the type of the product that takes it.  Scores are rounded to fp32 where the reference's
 // are (the product, the scaled product, the sum with an additive mask: attention_ops.cpp:101-128).
 // What bounds it: small problems the chain of one turn (two memory latencies, products, merge), large ones
 // the matrix cores and the L2 reads of K and V by every 16 QB queries.
@@ -36,6 +37,7 @@ namespace {
 
 constexpr int kWavesF = 4;
 constexpr std::uint32_t kOutOfRange = 0xF0000000u;
+constexpr double kSlack = 8.0;
 
 struct F32Params {
     const float* q; const float* k; const float* v; float* out; float* lse;
@@ -57,13 +59,11 @@ template <> struct Mma<double> {
         return __builtin_amdgcn_mfma_f64_16x16x4f64(static_cast<double>(a), b, c, 0, 0, 0);
     }
     __device__ static __forceinline__ int row(int g, int r) { return 4 * r + g; }       // row of register r in lane group g
-    __device__ static __forceinline__ double exp_of(double x) { return exp(x); }
 };
 template <> struct Mma<float> {
     typedef float vec __attribute__((ext_vector_type(4)));
     __device__ static __forceinline__ vec run(float a, float b, vec c) { return __builtin_amdgcn_mfma_f32_16x16x4f32(a, b, c, 0, 0, 0); }
     __device__ static __forceinline__ int row(int g, int r) { return 4 * g + r; }
-    __device__ static __forceinline__ float exp_of(float x) { return __builtin_amdgcn_exp2f(x * 1.4426950408889634f); }
 };
 
 // DM: largest head size of this form (64, 128, 256); D and Dv are multiples of 4 up to it.
@@ -74,7 +74,7 @@ __global__ __launch_bounds__(kWavesF * 64) void sdpa_f32_kernel(const F32Params 
     using vec = typename M::vec;
     constexpr int DC = DM / 16, VC = DM / 64, kTurn = 16 * KB;
     __shared__ Acc o_part[kWavesF][QB * VC * 4 * 256];
-    __shared__ Acc m_part[kWavesF][QB][16], l_part[kWavesF][QB][16];
+    __shared__ double m_part[kWavesF][QB][16], l_part[kWavesF][QB][16];
 
     // heaviest query tiles first under the causal rule
     const int qt = p.is_causal ? p.q_tiles - 1 - static_cast<int>(blockIdx.x) : static_cast<int>(blockIdx.x);
@@ -125,7 +125,7 @@ __global__ __launch_bounds__(kWavesF * 64) void sdpa_f32_kernel(const F32Params 
     };
 
     vec o[QB][VC][4];
-    Acc m[QB], l[QB];
+    double m[QB], l[QB];                              // the exponentials' reference point; their sum, unrounded
 #pragma unroll
     for (int qb = 0; qb < QB; ++qb) {
         m[qb] = -INFINITY;
@@ -220,23 +220,28 @@ __global__ __launch_bounds__(kWavesF * 64) void sdpa_f32_kernel(const F32Params 
                 }
             mx = fmaxf(mx, __shfl_xor(mx, 16, 64));
             mx = fmaxf(mx, __shfl_xor(mx, 32, 64));
-            const Acc m_new = static_cast<Acc>(mx) > m[qb] ? static_cast<Acc>(mx) : m[qb];
-            const Acc ref = m_new == -INFINITY ? static_cast<Acc>(0) : m_new;            // no visible key yet: any reference but -inf
-            if (__builtin_amdgcn_ballot_w64(m_new != m[qb]) != 0) {
-                const Acc f = M::exp_of(m[qb] - ref);
+            // The reference point follows the running maximum with some slack and in steps of whole powers of two, so that
+            // the sums are rescaled seldom and exactly (a step beyond fp32's range takes them to nothing either way).
+            const bool raise = static_cast<double>(mx) > m[qb] + kSlack;
+            if (__builtin_amdgcn_ballot_w64(raise) != 0) {
+                const double to = static_cast<double>(mx), steps = ceil((to - m[qb]) * 1.4426950408889634);
+                const bool exact = steps < 128.0;
+                const double f = !raise ? 1.0 : exact ? ldexp(1.0, -static_cast<int>(steps)) : 0.0;
                 l[qb] *= f;
 #pragma unroll
                 for (int c = 0; c < VC; ++c)
 #pragma unroll
-                    for (int e = 0; e < 4; ++e) o[qb][c][e] *= f;
-                m[qb] = m_new;
+                    for (int e = 0; e < 4; ++e) o[qb][c][e] *= static_cast<Acc>(f);
+                m[qb] = !raise ? m[qb] : exact ? fma(steps, 0.6931471805599453, m[qb]) : to;
             }
+            const double ref = m[qb] == -INFINITY ? 0.0 : m[qb];                         // no visible key yet: any reference but -inf
 #pragma unroll
             for (int kb = 0; kb < KB; ++kb)
 #pragma unroll
                 for (int r = 0; r < 4; ++r) {
-                    pr[qb][kb][r] = M::exp_of(static_cast<Acc>(x[kb][r]) - ref);
-                    l[qb] += pr[qb][kb][r];
+                    const double w = exp(static_cast<double>(x[kb][r]) - ref);
+                    l[qb] += w;
+                    pr[qb][kb][r] = static_cast<Acc>(w);
                 }
         }
         if constexpr (!kAhead) load_v(j0);
@@ -276,17 +281,17 @@ __global__ __launch_bounds__(kWavesF * 64) void sdpa_f32_kernel(const F32Params 
     for (int item = wave; item < QB * VC * 4; item += kWavesF) {
         const int r = item & 3, c = (item >> 2) % VC, qb = (item >> 2) / VC;
         const int i = q0 + 16 * qb + l16, dv = 64 * c + 4 * M::row(g, r);
-        Acc mm = m_part[0][qb][l16];
+        double mm = m_part[0][qb][l16];
 #pragma unroll
         for (int w = 1; w < kWavesF; ++w) mm = m_part[w][qb][l16] > mm ? m_part[w][qb][l16] : mm;
-        const Acc ref = mm == -INFINITY ? static_cast<Acc>(0) : mm;
-        Acc sum = 0, val[4] = {0, 0, 0, 0};
+        const double ref = mm == -INFINITY ? 0.0 : mm;
+        double sum = 0, val[4] = {0, 0, 0, 0};
 #pragma unroll
         for (int w = 0; w < kWavesF; ++w) {
-            const Acc f = M::exp_of(m_part[w][qb][l16] - ref);
+            const double f = exp(m_part[w][qb][l16] - ref);
             sum += f * l_part[w][qb][l16];
 #pragma unroll
-            for (int e = 0; e < 4; ++e) val[e] += f * o_part[w][((qb * VC + c) * 4 + e) * 256 + r * 64 + lane];
+            for (int e = 0; e < 4; ++e) val[e] += f * static_cast<double>(o_part[w][((qb * VC + c) * 4 + e) * 256 + r * 64 + lane]);
         }
         if (i >= p.Lq) continue;
         const long row = (static_cast<long>(b) * p.Hq + h) * p.Lq + i;
@@ -296,7 +301,7 @@ __global__ __launch_bounds__(kWavesF * 64) void sdpa_f32_kernel(const F32Params 
             for (int e = 0; e < 4; ++e) y[e] = static_cast<float>(val[e] / sum);
             *reinterpret_cast<float4_t*>(p.out + row * p.Dv + dv) = y;
         }
-        if (p.lse != nullptr && c == 0 && r == 0 && g == 0) p.lse[row] = static_cast<float>(static_cast<double>(mm) + log(static_cast<double>(sum)));
+        if (p.lse != nullptr && c == 0 && r == 0 && g == 0) p.lse[row] = static_cast<float>(mm + log(sum));
     }
 }
 

@@ -868,3 +868,21 @@ def test_fp32_scale_is_taken_as_given(S, H):
     got = lse.cpu().double()
     assert (got - lse_of(scale)).norm().item() < 0.6 * (got - lse_of(0.5)).norm().item()
     assert rel_err(out, (dots * scale).float().double().softmax(-1) @ v.double()) <= 1e-6
+
+
+@pytest.mark.parametrize("Lq,H", [(16, 1), (512, 2)])
+@pytest.mark.parametrize("scale", [2.0 ** -8, 2.0 ** -6, 2.0 ** -4])
+def test_fp32_weights_are_rounded_once(Lq, H, scale):
+    """The softmax is formed in fp64 in the small and in the large form.  Scores that are exact in fp32 and values that
+    pick one weight each: an output is a weight rounded to fp32 and the quotient by the row sum rounded again, so no
+    further than two half units (2 x 2^-24) from fp64, whatever the order in which the maximum grew."""
+    q, k = (torch.randint(-3, 4, (1, H, n, 256)).float() for n in (Lq, 256))
+    k *= torch.linspace(0.25, 1.0, 256).mul(64).round().div(64)[:, None]            # (sixteen bits at most: still exact)
+    v = torch.eye(256).expand(1, H, 256, 256)
+    out, _, lse, _ = run(q, k, v, scale=scale, want_lse=True)
+    s = (q.double() @ k.double().transpose(-1, -2)) * scale
+    want = s.softmax(-1)
+    big = want > 1e-30                                                  # (below, fp32 itself runs out of exponents)
+    assert ((out.cpu().double() - want).abs()[big] / want[big]).max().item() <= 2 * 2.0 ** -24 * 1.001
+    ref = torch.logsumexp(s, -1)
+    assert (lse.cpu().double() - ref).abs().max().item() <= 2.0 ** -24 * ref.abs().max().item() * 1.001
