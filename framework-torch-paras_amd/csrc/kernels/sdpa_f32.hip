@@ -37,7 +37,7 @@ namespace {
 
 constexpr int kWavesF = 4;
 constexpr std::uint32_t kOutOfRange = 0xF0000000u;
-constexpr double kSlack = 8.0;
+constexpr double kSlack = 8.0;      // how far the running maximum may rise before the sums are rescaled
 
 struct F32Params {
     const float* q; const float* k; const float* v; float* out; float* lse;
@@ -47,6 +47,7 @@ struct F32Params {
     int q_tiles;
     long qs[3], ks[3], vs[3], ms[4];
     double scale;
+    double above;         // the exponentials' reference point lies this far above the (lagging) row maximum
 };
 
 template <typename Acc> struct Mma;
@@ -125,7 +126,7 @@ __global__ __launch_bounds__(kWavesF * 64) void sdpa_f32_kernel(const F32Params 
     };
 
     vec o[QB][VC][4];
-    double m[QB], l[QB];                              // the exponentials' reference point; their sum, unrounded
+    double m[QB], l[QB];                              // the maximum so far, up to kSlack behind; the sum of exponentials, unrounded
 #pragma unroll
     for (int qb = 0; qb < QB; ++qb) {
         m[qb] = -INFINITY;
@@ -220,7 +221,7 @@ __global__ __launch_bounds__(kWavesF * 64) void sdpa_f32_kernel(const F32Params 
                 }
             mx = fmaxf(mx, __shfl_xor(mx, 16, 64));
             mx = fmaxf(mx, __shfl_xor(mx, 32, 64));
-            // The reference point follows the running maximum with some slack and in steps of whole powers of two, so that
+            // m follows the running maximum with some slack and in steps of whole powers of two, so that
             // the sums are rescaled seldom and exactly (a step beyond fp32's range takes them to nothing either way).
             const bool raise = static_cast<double>(mx) > m[qb] + kSlack;
             if (__builtin_amdgcn_ballot_w64(raise) != 0) {
@@ -234,7 +235,7 @@ __global__ __launch_bounds__(kWavesF * 64) void sdpa_f32_kernel(const F32Params 
                     for (int e = 0; e < 4; ++e) o[qb][c][e] *= static_cast<Acc>(f);
                 m[qb] = !raise ? m[qb] : exact ? fma(steps, 0.6931471805599453, m[qb]) : to;
             }
-            const double ref = m[qb] == -INFINITY ? 0.0 : m[qb];                         // no visible key yet: any reference but -inf
+            const double ref = m[qb] == -INFINITY ? 0.0 : m[qb] + p.above;               // no visible key yet: any reference but -inf
 #pragma unroll
             for (int kb = 0; kb < KB; ++kb)
 #pragma unroll
@@ -301,7 +302,7 @@ __global__ __launch_bounds__(kWavesF * 64) void sdpa_f32_kernel(const F32Params 
             for (int e = 0; e < 4; ++e) y[e] = static_cast<float>(val[e] / sum);
             *reinterpret_cast<float4_t*>(p.out + row * p.Dv + dv) = y;
         }
-        if (p.lse != nullptr && c == 0 && r == 0 && g == 0) p.lse[row] = static_cast<float>(mm + log(sum));
+        if (p.lse != nullptr && c == 0 && r == 0 && g == 0) p.lse[row] = static_cast<float>(mm + p.above + log(sum));
     }
 }
 
@@ -353,6 +354,8 @@ int launch_f32(const paras_sdpa_args& a, bool accumulate_f64, hipStream_t s) {
     for (int i = 0; i < 3; ++i) { p.qs[i] = a.q_strides[i]; p.ks[i] = a.k_strides[i]; p.vs[i] = a.v_strides[i]; }
     for (int i = 0; i < 4; ++i) p.ms[i] = a.mask_strides[i];
     p.scale = a.scale;
+    // Lk weights of at most 1 / Lk: a weighted sum of values that fp32 holds is one that it holds
+    p.above = kSlack + std::log(static_cast<double>(a.Lk));
     const long dm = a.D > a.Dv ? a.D : a.Dv;
     if (accumulate_f64) {
         if (dm <= 64)       launch_dm<double, 64>(p, a, s);

@@ -886,3 +886,12 @@ def test_fp32_weights_are_rounded_once(Lq, H, scale):
     assert ((out.cpu().double() - want).abs()[big] / want[big]).max().item() <= 2 * 2.0 ** -24 * 1.001
     ref = torch.logsumexp(s, -1)
     assert (lse.cpu().double() - ref).abs().max().item() <= 2.0 ** -24 * ref.abs().max().item() * 1.001
+
+
+@pytest.mark.parametrize("Lq,Lk", [(20, 300), (512, 1000)])
+def test_fp32_values_near_the_end_of_the_range(Lq, Lk):
+    """Values of up to 3e38: their weighted mean is in fp32's range, and so are the sums on the way to it."""
+    q, k, v = torch.randn(1, 4, Lq, 64), torch.randn(1, 4, Lk, 64), torch.rand(1, 4, Lk, 64) * 2e38 + 1e38
+    s = q.double() @ k.double().transpose(-1, -2) / 8.0
+    assert rel_err(run(q, k, v)[0], s.softmax(-1) @ v.double()) <= 3e-6
+    assert rel_err(run(q * 20, k, v)[0], (s * 20).softmax(-1) @ v.double()) <= 3e-5      # (scores of up to a few hundred: 2^-24 of them)
