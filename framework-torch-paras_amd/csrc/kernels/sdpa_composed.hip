@@ -331,19 +331,13 @@ bool composed_supported(const paras_sdpa_args& a) {
 }
 
 size_t composed_workspace(const paras_sdpa_args& a) {
-    if (f32_supported(a) && a.attn == nullptr) return 0;
+    if (f32_supported(a)) return f32_workspace(a);
     const Plan pl = make_plan(a);
     return pl.vt_bytes + pl.score_bytes;
 }
 
 int launch_composed(const paras_sdpa_args& a, void* workspace, void* stream, hipStream_t s) {
-    // fp32: the output comes from the one-pass kernel, with or without the weights; the weights, when they are asked
-    // for, from the first product and the row kernel below.
-    const bool one_pass = f32_supported(a);
-    if (one_pass) {
-        const int rc = launch_f32(a, /*accumulate_f64=*/false, s);
-        if (rc != PARAS_OK || a.attn == nullptr) return rc;
-    }
+    if (f32_supported(a)) return launch_f32(a, /*accumulate_f64=*/false, workspace, s);
     PARAS_REQUIRE(workspace != nullptr, "paras sdpa: workspace is null");
     PARAS_REQUIRE((reinterpret_cast<uintptr_t>(workspace) & 255) == 0, "paras sdpa: the workspace must be 256-byte aligned");
     const Plan pl = make_plan(a);
@@ -353,7 +347,7 @@ int launch_composed(const paras_sdpa_args& a, void* workspace, void* stream, hip
     const long rep = a.Hq / a.Hkv;
 
     // v transposed once: the second product reads it along the keys
-    if (!one_pass) {
+    {
         const dim3 grid(static_cast<unsigned>((a.Lk + 31) / 32), static_cast<unsigned>((a.Dv + 31) / 32), static_cast<unsigned>(a.B * a.Hkv));
 #define PARAS_TRANSPOSE_V(S_)                                                                                                   \
     hipLaunchKernelGGL((transpose_v_kernel<S_>), grid, dim3(kBlock), 0, s, static_cast<const S_*>(a.v), reinterpret_cast<S_*>(vt), \
@@ -409,7 +403,6 @@ int launch_composed(const paras_sdpa_args& a, void* workspace, void* stream, hip
                 }
                 PARAS_HIP_TRY(hipGetLastError());
 
-                if (one_pass) continue;
                 const char* vp = vt + ((b * a.Hkv + hkv0) * a.Dv * a.Lk) * es;
                 char* op = static_cast<char*>(a.out) + (((b * a.Hq + h0) * a.Lq + i0) * a.Dv) * es;
                 rc = gemm_nt_causal(sc, vp, nullptr, op, nr, a.Dv, a.Lk, a.Lk, a.Lk, a.Dv, 0, nh, head_stride,

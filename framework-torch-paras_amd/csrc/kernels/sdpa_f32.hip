@@ -1,5 +1,5 @@
-// Scaled-dot-product attention of fp32 tensors in one pass on the matrix cores (the output and the log-sum-exp;
-// returned weights are the composed route's or the general kernel's business).
+// Scaled-dot-product attention of fp32 tensors in one pass on the matrix cores: the output, the log-sum-exp and, in
+// the form for large problems, the returned weights.
 //
 // Before, small problems ran one workgroup per query row with scalar fp64 dot products formed three
 // times per score, every lane of a wavefront on a key row of its own (B1 H8 S128 D64: 44 us; B3 H64 S57
@@ -41,10 +41,13 @@ constexpr double kSlack = 8.0;      // how far the running maximum may rise befo
 
 struct F32Params {
     const float* q; const float* k; const float* v; float* out; float* lse;
+    float* attn;          // [B, Hq, Lq, Lk] or null: takes the scaled and masked scores that were formed
+    double2* row_sums;    // with attn, [B * Hq * Lq]: each row's reference point and its sum of exponentials
     const void* mask;
     int is_causal;
     int Hq, Hkv, Lq, Lk, D, Dv;
     int q_tiles;
+    bool attn16;          // rows of attn are whole 16-byte pieces
     long qs[3], ks[3], vs[3], ms[4];
     double scale;
     double above;         // the exponentials' reference point lies this far above the (lagging) row maximum
@@ -139,6 +142,19 @@ __global__ __launch_bounds__(kWavesF * 64) void sdpa_f32_kernel(const F32Params 
     const int keys = p.is_causal ? min(p.Lk, q0 + 16 * QB) : p.Lk;
     // 32 keys of more than 128 elements leave no registers for operands ahead of time: they are requested where they are used
     constexpr bool kAhead = DM <= 128 || sizeof(Acc) == 8;
+    // The scores of a block for softmax_rows_kernel below: a lane holds 4 adjacent keys of one query.
+    auto keep_scores = [&](int qb, int j, const float (&x)[4]) {
+        const int i = q0 + 16 * qb + l16;
+        if (i >= p.Lq || j >= p.Lk) return;
+        float* at = p.attn + ((static_cast<long>(b) * p.Hq + h) * p.Lq + i) * p.Lk + j;
+        if (p.attn16) {
+            *reinterpret_cast<float4_t*>(at) = float4_t{x[0], x[1], x[2], x[3]};
+        } else {
+#pragma unroll
+            for (int r = 0; r < 4; ++r)
+                if (j + r < p.Lk) at[r] = x[r];
+        }
+    };
     // A turn that no query of the tile sees: its weights are zeros whatever its scores are, but zero times a value that is
     // not finite is NaN, as in the reference's full product.  Each value times zero, then one product per block of the
     // output (A = those, B = zeros) that carries a NaN to its column of every query and changes nothing else.
@@ -180,6 +196,14 @@ __global__ __launch_bounds__(kWavesF * 64) void sdpa_f32_kernel(const F32Params 
             }
             if (kMask == 1 && __builtin_amdgcn_ballot_w64(any) == 0) {
                 unseen_turn(j0);
+                if constexpr (sizeof(Acc) == 4)
+                    if (p.attn != nullptr) {
+                        const float hidden[4] = {-INFINITY, -INFINITY, -INFINITY, -INFINITY};
+#pragma unroll
+                        for (int qb = 0; qb < QB; ++qb)
+#pragma unroll
+                            for (int kb = 0; kb < KB; ++kb) keep_scores(qb, j0 + 16 * kb + M::row(g, 0), hidden);
+                    }
                 if (kAhead && j0 + kWavesF * kTurn < keys) load_k(j0 + kWavesF * kTurn);
                 continue;
             }
@@ -218,6 +242,11 @@ __global__ __launch_bounds__(kWavesF * 64) void sdpa_f32_kernel(const F32Params 
                     if (j >= p.Lk || (p.is_causal && j > i)) y = -INFINITY;
                     x[kb][r] = y;
                     mx = fmaxf(mx, y);
+                }
+            if constexpr (sizeof(Acc) == 4)
+                if (p.attn != nullptr) {
+#pragma unroll
+                    for (int kb = 0; kb < KB; ++kb) keep_scores(qb, j0 + 16 * kb + M::row(g, 0), x[kb]);
                 }
             mx = fmaxf(mx, __shfl_xor(mx, 16, 64));
             mx = fmaxf(mx, __shfl_xor(mx, 32, 64));
@@ -302,7 +331,47 @@ __global__ __launch_bounds__(kWavesF * 64) void sdpa_f32_kernel(const F32Params 
             for (int e = 0; e < 4; ++e) y[e] = static_cast<float>(val[e] / sum);
             *reinterpret_cast<float4_t*>(p.out + row * p.Dv + dv) = y;
         }
-        if (p.lse != nullptr && c == 0 && r == 0 && g == 0) p.lse[row] = static_cast<float>(mm + p.above + log(sum));
+        if (c == 0 && r == 0 && g == 0) {
+            if (p.lse != nullptr) p.lse[row] = static_cast<float>(mm + p.above + log(sum));
+            if (p.row_sums != nullptr) p.row_sums[row] = double2{mm == -INFINITY ? 0.0 : mm + p.above, sum};
+        }
+    }
+}
+
+// The returned weights, in place of the scores that sdpa_f32_kernel left: exp(score - reference) / sum in fp64, rounded
+// once; zeros for the keys that the causal rule hides (NaN where the row is).  A wave takes a row in pieces of W elements.
+// Bound by memory (one read and one write of the weights tensor); four pieces are on the way at a time.
+template <int W>
+__global__ __launch_bounds__(256) void softmax_rows_kernel(float* __restrict__ attn, const double2* __restrict__ row_sums, long rows, int Lq, int Lk, int is_causal) {
+    typedef float piece __attribute__((ext_vector_type(W)));
+    constexpr int kAtOnce = 4;
+    const long row = static_cast<long>(blockIdx.x) * 4 + (threadIdx.x >> 6);
+    if (row >= rows) return;
+    const int lane = threadIdx.x & 63;
+    const int seen = is_causal ? min(static_cast<int>(row % Lq) + 1, Lk) : Lk;
+    const double2 of = row_sums[row];
+    const double inv = 1.0 / of.y, none = 0.0 * inv;
+    float* const base = attn + row * Lk;
+    for (int j0 = 0; j0 < Lk; j0 += 64 * W * kAtOnce) {
+        piece x[kAtOnce];
+#pragma unroll
+        for (int t = 0; t < kAtOnce; ++t) {
+            const int j = j0 + (64 * t + lane) * W;
+            if (j < seen) x[t] = *reinterpret_cast<const piece*>(base + j);
+        }
+#pragma unroll
+        for (int t = 0; t < kAtOnce; ++t) {
+            const int j = j0 + (64 * t + lane) * W;
+            if (j >= Lk) continue;
+            piece y;
+#pragma unroll
+            for (int e = 0; e < W; ++e) y[e] = static_cast<float>(none);
+            if (j < seen)
+#pragma unroll
+                for (int e = 0; e < W; ++e)
+                    if (j + e < seen) y[e] = static_cast<float>(exp(static_cast<double>(x[t][e]) - of.x) * inv);
+            *reinterpret_cast<piece*>(base + j) = y;
+        }
     }
 }
 
@@ -344,7 +413,9 @@ bool f32_supported(const paras_sdpa_args& a) {
            (reinterpret_cast<uintptr_t>(a.out) & 15) == 0;
 }
 
-int launch_f32(const paras_sdpa_args& a, bool accumulate_f64, hipStream_t s) {
+size_t f32_workspace(const paras_sdpa_args& a) { return a.attn != nullptr ? static_cast<size_t>(a.B * a.Hq * a.Lq) * sizeof(double2) : 0; }
+
+int launch_f32(const paras_sdpa_args& a, bool accumulate_f64, void* workspace, hipStream_t s) {
     F32Params p{};
     p.q = static_cast<const float*>(a.q); p.k = static_cast<const float*>(a.k); p.v = static_cast<const float*>(a.v);
     p.out = static_cast<float*>(a.out); p.lse = a.lse; p.mask = a.mask;
@@ -353,6 +424,14 @@ int launch_f32(const paras_sdpa_args& a, bool accumulate_f64, hipStream_t s) {
     p.Lq = static_cast<int>(a.Lq); p.Lk = static_cast<int>(a.Lk); p.D = static_cast<int>(a.D); p.Dv = static_cast<int>(a.Dv);
     for (int i = 0; i < 3; ++i) { p.qs[i] = a.q_strides[i]; p.ks[i] = a.k_strides[i]; p.vs[i] = a.v_strides[i]; }
     for (int i = 0; i < 4; ++i) p.ms[i] = a.mask_strides[i];
+    if (a.attn != nullptr) {
+        PARAS_REQUIRE(!accumulate_f64, "paras sdpa: the fp64 form returns no weights");
+        PARAS_REQUIRE(workspace != nullptr, "paras sdpa: workspace is null");
+        PARAS_REQUIRE((reinterpret_cast<uintptr_t>(workspace) & 255) == 0, "paras sdpa: the workspace must be 256-byte aligned");
+        p.attn = static_cast<float*>(a.attn);
+        p.row_sums = static_cast<double2*>(workspace);
+        p.attn16 = a.Lk % 4 == 0 && (reinterpret_cast<uintptr_t>(a.attn) & 15) == 0;
+    }
     p.scale = a.scale;
     // Lk weights of at most 1 / Lk: a weighted sum of values that fp32 holds is one that it holds
     p.above = kSlack + std::log(static_cast<double>(a.Lk));
@@ -367,6 +446,13 @@ int launch_f32(const paras_sdpa_args& a, bool accumulate_f64, hipStream_t s) {
         else                launch_dm<float, 256>(p, a, s);
     }
     PARAS_HIP_TRY(hipGetLastError());
+    if (a.attn != nullptr) {
+        const long rows = a.B * a.Hq * a.Lq;
+        const dim3 grid(static_cast<unsigned>((rows + 3) / 4));
+        if (p.attn16) hipLaunchKernelGGL((softmax_rows_kernel<4>), grid, dim3(256), 0, s, p.attn, p.row_sums, rows, p.Lq, p.Lk, a.is_causal);
+        else          hipLaunchKernelGGL((softmax_rows_kernel<1>), grid, dim3(256), 0, s, p.attn, p.row_sums, rows, p.Lq, p.Lk, a.is_causal);
+        PARAS_HIP_TRY(hipGetLastError());
+    }
     return PARAS_OK;
 }
 

@@ -154,7 +154,7 @@ __global__ __launch_bounds__(kBlock) void sdpa_generic_kernel(const GenericParam
 size_t generic_workspace(const paras_sdpa_args&) { return 0; }
 
 int launch_generic(const paras_sdpa_args& a, void*, hipStream_t s) {
-    if (a.attn == nullptr && f32_supported(a)) return launch_f32(a, /*accumulate_f64=*/true, s);
+    if (a.attn == nullptr && f32_supported(a)) return launch_f32(a, /*accumulate_f64=*/true, nullptr, s);
     if (a.D > kMaxD || a.Dv > kMaxD)
         return fail(PARAS_ERR_UNSUPPORTED, "paras sdpa: head dim %lld/%lld exceeds %d", (long long)a.D,
                     (long long)a.Dv, kMaxD);

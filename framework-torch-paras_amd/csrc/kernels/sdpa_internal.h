@@ -43,10 +43,11 @@ int gemm_nt_causal(const void* a, const void* b, const void* addend, void* c, in
                    int64_t stride_b, int64_t stride_c, int64_t stride_add, double alpha, double beta, int dtype,
                    void* workspace, size_t workspace_bytes, void* stream, int causal_kind, long causal_first);
 
-// fp32 attention in one pass (no returned weights), products accumulated in fp64 (the general route's problems) or
+// fp32 attention in one pass, products accumulated in fp64 (the general route's problems, without returned weights) or
 // fp32 (the composed route's): head sizes of up to 256 that are multiples of 4.
-bool f32_supported(const paras_sdpa_args& a);
-int  launch_f32(const paras_sdpa_args& a, bool accumulate_f64, hipStream_t s);
+bool   f32_supported(const paras_sdpa_args& a);
+size_t f32_workspace(const paras_sdpa_args& a);
+int    launch_f32(const paras_sdpa_args& a, bool accumulate_f64, void* workspace, hipStream_t s);
 
 // Everything else (fp32/fp64, any head size, other layouts).
 size_t generic_workspace(const paras_sdpa_args& a);

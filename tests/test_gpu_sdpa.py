@@ -895,3 +895,41 @@ def test_fp32_values_near_the_end_of_the_range(Lq, Lk):
     s = q.double() @ k.double().transpose(-1, -2) / 8.0
     assert rel_err(run(q, k, v)[0], s.softmax(-1) @ v.double()) <= 3e-6
     assert rel_err(run(q * 20, k, v)[0], (s * 20).softmax(-1) @ v.double()) <= 3e-5      # (scores of up to a few hundred: 2^-24 of them)
+
+
+@pytest.mark.parametrize("kind", ["none", "causal", "bool", "additive"])
+@pytest.mark.parametrize("B,Hq,Hkv,Lq,Lk,D,Dv", [(1, 4, 2, 512, 512, 64, 64), (2, 2, 2, 333, 510, 128, 128), (1, 2, 2, 300, 701, 256, 64), (1, 4, 4, 700, 260, 40, 72)])
+def test_fp32_weights_of_the_one_pass_kernel(B, Hq, Hkv, Lq, Lk, D, Dv, kind):
+    """The weights returned for large fp32 problems: the scores of the one-pass kernel made into weights in place.  Rows
+    that are whole 16-byte pieces and others, rows longer than a wave's four pieces, turns that a mask closes, a query
+    that sees no key (NaN), a NaN key that everybody sees.  A weight is off by its score's rounding (products of 64 to 256
+    terms, 3e-6 of scores of a few units) and once more; the output does not depend on whether weights are asked for, nor
+    on what the weights tensor held."""
+    q, k, v = torch.randn(B, Hq, Lq, D), torch.randn(B, Hkv, Lk, D), torch.randn(B, Hkv, Lk, Dv)
+    keep = torch.rand(B, 1, Lq, Lk) < 0.7
+    keep[..., 32:192] = False
+    keep[..., 0] = True
+    keep[0, 0, Lq // 2] = False
+    add = torch.randn(1, Hq, 1, Lk)
+    kw = dict(none={}, causal=dict(is_causal=True), bool=dict(mask=keep), additive=dict(mask=add))[kind]
+    for nan_key in (False, True):
+        if nan_key:
+            k[0, 0, 0, 0] = math.nan
+        s = q.double() @ k.double().repeat_interleave(Hq // Hkv, 1).transpose(-1, -2) / math.sqrt(D)
+        if kind == "causal":
+            s = s.masked_fill(~torch.ones(Lq, Lk).tril().bool(), -math.inf)
+        elif kind == "bool":
+            s = s.masked_fill(~keep, -math.inf)
+        elif kind == "additive":
+            s = s + add.double()
+        want = s.softmax(-1)
+        out, attn, lse, name = run(q, k, v, want_attn=True, want_lse=True, **kw)
+        assert name == "composed"
+        attn = attn.cpu().double()
+        assert torch.equal(attn.isnan(), want.isnan())
+        ok = ~want.isnan()
+        assert ((attn - want).abs()[ok] <= 1e-5 * want[ok] + 1e-30).all()
+        assert torch.equal(attn[ok] == 0, want[ok].float() == 0)
+        again, _, lse2, _ = run(q, k, v, want_lse=True, **kw)
+        assert_bit_exact(out, again)
+        assert_bit_exact(lse, lse2)
