@@ -47,7 +47,7 @@ struct F32Params {
     int is_causal;
     int Hq, Hkv, Lq, Lk, D, Dv;
     int q_tiles;
-    bool attn16;          // rows of attn are whole 16-byte pieces
+    bool out16, attn16;   // rows of out / attn are whole 16-byte pieces
     long qs[3], ks[3], vs[3], ms[4];
     double scale;
     double above;         // the exponentials' reference point lies this far above the (lagging) row maximum
@@ -329,7 +329,13 @@ __global__ __launch_bounds__(kWavesF * 64) void sdpa_f32_kernel(const F32Params 
             float4_t y;
 #pragma unroll
             for (int e = 0; e < 4; ++e) y[e] = static_cast<float>(val[e] / sum);
-            *reinterpret_cast<float4_t*>(p.out + row * p.Dv + dv) = y;
+            float* const at = p.out + row * p.Dv + dv;
+            if (p.out16) {
+                *reinterpret_cast<float4_t*>(at) = y;
+            } else {
+#pragma unroll
+                for (int e = 0; e < 4; ++e) at[e] = y[e];
+            }
         }
         if (c == 0 && r == 0 && g == 0) {
             if (p.lse != nullptr) p.lse[row] = static_cast<float>(mm + p.above + log(sum));
@@ -403,14 +409,14 @@ void launch_dm(const F32Params& p, const paras_sdpa_args& a, hipStream_t s) {
 
 }  // namespace
 
+// (by sizes and strides alone: paras_sdpa_workspace may be asked before the pointers are known)
 bool f32_supported(const paras_sdpa_args& a) {
     if (a.dtype != PARAS_F32) return false;
     if (a.D < 4 || a.Dv < 4 || a.D > 256 || a.Dv > 256 || a.D % 4 != 0 || a.Dv % 4 != 0 || a.Lq < 1 || a.Lk < 1) return false;
     if (a.Hq > 65535 || a.B > 65535 || a.Lq >= (1L << 30) || a.Lk >= (1L << 30)) return false;
     if (a.q_strides[2] < 0 || a.k_strides[2] < 0 || a.v_strides[2] < 0) return false;
     const long lim = (1L << 29) - 1;                       // elements: byte offsets below 2^31
-    return (a.Lq - 1) * a.q_strides[2] + a.D <= lim && (a.Lk - 1) * a.k_strides[2] + a.D <= lim && (a.Lk - 1) * a.v_strides[2] + a.Dv <= lim &&
-           (reinterpret_cast<uintptr_t>(a.out) & 15) == 0;
+    return (a.Lq - 1) * a.q_strides[2] + a.D <= lim && (a.Lk - 1) * a.k_strides[2] + a.D <= lim && (a.Lk - 1) * a.v_strides[2] + a.Dv <= lim;
 }
 
 size_t f32_workspace(const paras_sdpa_args& a) { return a.attn != nullptr ? static_cast<size_t>(a.B * a.Hq * a.Lq) * sizeof(double2) : 0; }
@@ -419,6 +425,7 @@ int launch_f32(const paras_sdpa_args& a, bool accumulate_f64, void* workspace, h
     F32Params p{};
     p.q = static_cast<const float*>(a.q); p.k = static_cast<const float*>(a.k); p.v = static_cast<const float*>(a.v);
     p.out = static_cast<float*>(a.out); p.lse = a.lse; p.mask = a.mask;
+    p.out16 = (reinterpret_cast<uintptr_t>(a.out) & 15) == 0;
     p.is_causal = a.is_causal;
     p.Hq = static_cast<int>(a.Hq); p.Hkv = static_cast<int>(a.Hkv);
     p.Lq = static_cast<int>(a.Lq); p.Lk = static_cast<int>(a.Lk); p.D = static_cast<int>(a.D); p.Dv = static_cast<int>(a.Dv);

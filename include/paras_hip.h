@@ -231,7 +231,9 @@ typedef struct paras_sdpa_args {
     double      scale;          /* multiplies q k^T exactly as given          */
 } paras_sdpa_args;
 
-/* Scratch bytes the chosen kernel needs for these shapes (0 for most). */
+/* Scratch bytes the chosen kernel needs for these shapes (0 for most).  For fp32 and fp64 the sizes and
+ * strides decide, and whether attn is NULL; with 16-bit tensors the pointers' alignment to 16 bytes
+ * counts as well, so ask with the pointers of the call. */
 PARAS_API size_t paras_sdpa_workspace(const paras_sdpa_args* args);
 /* `workspace` may be NULL when paras_sdpa_workspace() returned 0. */
 PARAS_API int paras_sdpa_fwd(const paras_sdpa_args* args, void* workspace, void* stream);

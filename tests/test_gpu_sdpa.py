@@ -4,6 +4,7 @@ Bars: fp32 within 1e-5 relative (max |a-b| / max |b|); bf16 / fp16 within 2e-2
 absolute of the host-engine oracle; the generic kernel additionally reproduces
 the host engine's softmax weights bit for bit (it narrows at the same points).
 """
+import ctypes as C
 import math
 
 import pytest
@@ -933,3 +934,23 @@ def test_fp32_weights_of_the_one_pass_kernel(B, Hq, Hkv, Lq, Lk, D, Dv, kind):
         again, _, lse2, _ = run(q, k, v, want_lse=True, **kw)
         assert_bit_exact(out, again)
         assert_bit_exact(lse, lse2)
+
+
+@pytest.mark.parametrize("want_attn", [False, True])
+@pytest.mark.parametrize("Lq,Lk,D,Dv", [(33, 70, 64, 72), (512, 512, 64, 64), (300, 701, 128, 40)])
+def test_fp32_output_off_a_16_byte_boundary(Lq, Lk, D, Dv, want_attn):
+    """An output (and weights) that begin 4 bytes off: same kernel, same workspace, same bits."""
+    q, k, v = (torch.randn(1, 4, n, d).cuda() for n, d in ((Lq, D), (Lk, D), (Lk, Dv)))
+    want, wattn, _, name = capi.sdpa(q, k, v, want_attn=want_attn)
+    out = torch.full((want.numel() + 2,), math.inf, device="cuda")
+    attn = torch.full((4 * Lq * Lk + 2,), math.inf, device="cuda")
+    a = capi.sdpa_args(q, k, v, out[1:-1].view_as(want), attn[1:-1].view(1, 4, Lq, Lk) if want_attn else None)
+    n = capi.lib().paras_sdpa_workspace(C.byref(a))
+    ws = torch.empty(max(n, 1), dtype=torch.uint8, device="cuda")
+    assert capi.lib().paras_sdpa_kernel_name(C.byref(a)).decode() == name
+    capi.check(capi.lib().paras_sdpa_fwd(C.byref(a), ws.data_ptr() if n else None, torch.cuda.current_stream().cuda_stream))
+    assert_bit_exact(out[1:-1].view_as(want), want)
+    assert bool(out[[0, -1]].isinf().all())
+    if want_attn:
+        assert_bit_exact(attn[1:-1].view_as(wattn), wattn)
+        assert bool(attn[[0, -1]].isinf().all())
