@@ -140,8 +140,8 @@ __global__ __launch_bounds__(kWavesF * 64) void sdpa_f32_kernel(const F32Params 
             for (int e = 0; e < 4; ++e) o[qb][c][e] = vec{0, 0, 0, 0};
     }
     const int keys = p.is_causal ? min(p.Lk, q0 + 16 * QB) : p.Lk;
-    // 32 keys of more than 128 elements leave no registers for operands ahead of time: they are requested where they are used
-    constexpr bool kAhead = DM <= 128 || sizeof(Acc) == 8;
+    // more than 128 elements leave no registers for operands ahead of time: they are requested where they are used
+    constexpr bool kAhead = DM <= 128;
     // The scores of a block for softmax_rows_kernel below: a lane holds 4 adjacent keys of one query.
     auto keep_scores = [&](int qb, int j, const float (&x)[4]) {
         const int i = q0 + 16 * qb + l16;
@@ -173,29 +173,32 @@ __global__ __launch_bounds__(kWavesF * 64) void sdpa_f32_kernel(const F32Params 
                 for (int qb = 0; qb < QB; ++qb) o[qb][c][e] = M::run(z, static_cast<Acc>(0), o[qb][c][e]);
             }
     };
-    if (kAhead && wave * kTurn < keys) load_k(wave * kTurn);
-    int j0 = wave * kTurn;
-    for (; j0 < keys; j0 += kWavesF * kTurn) {
-        // the mask ahead of everything else: a turn that a boolean mask closes to every query of the tile needs no scores (an
-        // additive mask does not close anything: a NaN or +inf score plus -inf is NaN)
-        float mk[QB][KB][4];                          // additive values; bool: 0 where attended, -inf elsewhere
-        if constexpr (kMask != 0) {
-            bool any = kMask == 2;
+    // The mask of one query block's part of a turn at (kb, r).
+    auto mask_at = [&](int j0, int qb, int kb, int r) {
+        const long row = static_cast<long>(min(q0 + 16 * qb + l16, p.Lq - 1)), col = static_cast<long>(min(j0 + 16 * kb + M::row(g, r), p.Lk - 1));
+        return b * p.ms[0] + h * p.ms[1] + row * p.ms[2] + col * p.ms[3];
+    };
+    // A boolean mask's part of a turn, bit 4 kb + r; false: the turn is closed to every query of the tile.
+    auto open_bits = [&](int j0, unsigned (&open)[QB]) {
+        unsigned any = 0;
 #pragma unroll
-            for (int qb = 0; qb < QB; ++qb) {
-                const long mrow = b * p.ms[0] + h * p.ms[1] + static_cast<long>(min(q0 + 16 * qb + l16, p.Lq - 1)) * p.ms[2];
+        for (int qb = 0; qb < QB; ++qb) {
+            open[qb] = 0;
 #pragma unroll
-                for (int kb = 0; kb < KB; ++kb)
+            for (int kb = 0; kb < KB; ++kb)
 #pragma unroll
-                    for (int r = 0; r < 4; ++r) {
-                        const long at = mrow + static_cast<long>(min(j0 + 16 * kb + M::row(g, r), p.Lk - 1)) * p.ms[3];
-                        if constexpr (kMask == 1) mk[qb][kb][r] = static_cast<const unsigned char*>(p.mask)[at] != 0 ? 0.0f : -INFINITY;
-                        else                      mk[qb][kb][r] = static_cast<const float*>(p.mask)[at];
-                        if constexpr (kMask == 1) any = any || mk[qb][kb][r] == 0.0f;
-                    }
-            }
-            if (kMask == 1 && __builtin_amdgcn_ballot_w64(any) == 0) {
-                unseen_turn(j0);
+                for (int r = 0; r < 4; ++r) open[qb] |= static_cast<const unsigned char*>(p.mask)[mask_at(j0, qb, kb, r)] != 0 ? 1u << (4 * kb + r) : 0u;
+            any |= open[qb];
+        }
+        return __builtin_amdgcn_ballot_w64(any != 0) != 0;
+    };
+    // The first turn from j0 on that this wave has scores to form for.  One that a boolean mask closes needs none (an
+    // additive mask does not close anything: a NaN or +inf score plus -inf is NaN).
+    bool closed = false;                              // some turn of this wave is
+    auto next_open = [&](int j0, unsigned (&open)[QB]) {
+        if constexpr (kMask == 1)
+            for (; j0 < keys && !open_bits(j0, open); j0 += kWavesF * kTurn) {
+                closed = true;
                 if constexpr (sizeof(Acc) == 4)
                     if (p.attn != nullptr) {
                         const float hidden[4] = {-INFINITY, -INFINITY, -INFINITY, -INFINITY};
@@ -204,10 +207,21 @@ __global__ __launch_bounds__(kWavesF * 64) void sdpa_f32_kernel(const F32Params 
 #pragma unroll
                             for (int kb = 0; kb < KB; ++kb) keep_scores(qb, j0 + 16 * kb + M::row(g, 0), hidden);
                     }
-                if (kAhead && j0 + kWavesF * kTurn < keys) load_k(j0 + kWavesF * kTurn);
-                continue;
             }
-        }
+        return j0;
+    };
+    unsigned open[QB], open_next[QB];
+    int j0 = next_open(wave * kTurn, open);
+    if (kAhead && j0 < keys) load_k(j0);
+    while (j0 < keys) {
+        float mk[QB][KB][4];
+        if constexpr (kMask == 2)
+#pragma unroll
+            for (int qb = 0; qb < QB; ++qb)
+#pragma unroll
+                for (int kb = 0; kb < KB; ++kb)
+#pragma unroll
+                    for (int r = 0; r < 4; ++r) mk[qb][kb][r] = static_cast<const float*>(p.mask)[mask_at(j0, qb, kb, r)];
         if constexpr (kAhead) load_v(j0);
         else                  load_k(j0);
         vec s[QB][KB];
@@ -223,7 +237,8 @@ __global__ __launch_bounds__(kWavesF * 64) void sdpa_f32_kernel(const F32Params 
                 for (int kb = 0; kb < KB; ++kb)
 #pragma unroll
                     for (int qb = 0; qb < QB; ++qb) s[qb][kb] = M::run(kf[kb][c][e], qf[qb][c][e], s[qb][kb]);
-        if (kAhead && j0 + kWavesF * kTurn < keys) load_k(j0 + kWavesF * kTurn);
+        const int j_next = next_open(j0 + kWavesF * kTurn, open_next);
+        if (kAhead && j_next < keys) load_k(j_next);
         Acc pr[QB][KB][4];
 #pragma unroll
         for (int qb = 0; qb < QB; ++qb) {
@@ -237,7 +252,7 @@ __global__ __launch_bounds__(kWavesF * 64) void sdpa_f32_kernel(const F32Params 
                     // (the scale as it is given: in fp64, rounded once; the torch ops narrow it themselves)
                     float y = static_cast<float>(static_cast<double>(static_cast<float>(s[qb][kb][r])) * p.scale);
                     // (selected where a mask is boolean: a NaN or infinite score of a masked key is no score)
-                    if constexpr (kMask == 1) y = mk[qb][kb][r] == 0.0f ? y : -INFINITY;
+                    if constexpr (kMask == 1) y = (open[qb] >> (4 * kb + r) & 1u) != 0 ? y : -INFINITY;
                     if constexpr (kMask == 2) y += mk[qb][kb][r];
                     if (j >= p.Lk || (p.is_causal && j > i)) y = -INFINITY;
                     x[kb][r] = y;
@@ -285,11 +300,20 @@ __global__ __launch_bounds__(kWavesF * 64) void sdpa_f32_kernel(const F32Params 
                     for (int e = 0; e < 4; ++e)
 #pragma unroll
                         for (int qb = 0; qb < QB; ++qb) o[qb][c][e] = M::run(vf[kb][t][c][e], pr[qb][kb][t], o[qb][c][e]);
+        j0 = j_next;
+        if constexpr (kMask == 1)
+#pragma unroll
+            for (int qb = 0; qb < QB; ++qb) open[qb] = open_next[qb];
     }
 
-    // what the causal rule hides from the whole tile
+    // what the causal rule, or a boolean mask, hides from the whole tile
     if constexpr (kMask == 0)
         for (; j0 < p.Lk; j0 += kWavesF * kTurn) unseen_turn(j0);
+    if constexpr (kMask == 1)
+        if (closed)
+            for (j0 = wave * kTurn; j0 < keys; j0 += kWavesF * kTurn) {
+                if (!open_bits(j0, open)) unseen_turn(j0);
+            }
 
     // the waves meet
 #pragma unroll
