@@ -50,6 +50,7 @@ struct F32Params {
     bool out16, attn16;   // rows of out / attn are whole 16-byte pieces
     long qs[3], ks[3], vs[3], ms[4];
     double scale;
+    bool scale_is_float;
     double above;         // the exponentials' reference point lies this far above the (lagging) row maximum
 };
 
@@ -72,8 +73,9 @@ template <> struct Mma<float> {
 
 // DM: largest head size of this form (64, 128, 256); D and Dv are multiples of 4 up to it.
 // A turn is KB blocks of 16 keys.  kMask: 0 = none, 1 = bool (true = attend), 2 = additive.
+// (heads of up to 64 elements leave registers for two waves per SIMD)
 template <typename Acc, int DM, int QB, int KB, int kMask>
-__global__ __launch_bounds__(kWavesF * 64) void sdpa_f32_kernel(const F32Params p) {
+__global__ __launch_bounds__(kWavesF * 64, DM == 64 ? 2 : 1) void sdpa_f32_kernel(const F32Params p) {
     using M = Mma<Acc>;
     using vec = typename M::vec;
     constexpr int DC = DM / 16, VC = DM / 64, kTurn = 16 * KB;
@@ -107,25 +109,27 @@ __global__ __launch_bounds__(kWavesF * 64) void sdpa_f32_kernel(const F32Params 
                 qf[qb][c] = load4(qr, d < p.D ? static_cast<std::uint32_t>(row * p.qs[2] + d) * 4u : kOutOfRange);
             }
     }
+    // (byte offsets in 32 bits: in range below 2^31 up to the last row, and a row past it is not asked for)
+    const std::uint32_t kld = static_cast<std::uint32_t>(p.ks[2]) * 4u, vld = static_cast<std::uint32_t>(p.vs[2]) * 4u;
     auto load_k = [&](int j0) {
 #pragma unroll
-        for (int kb = 0; kb < KB; ++kb)
+        for (int kb = 0; kb < KB; ++kb) {
+            const int key = j0 + 16 * kb + l16;
+            const std::uint32_t row = key < p.Lk ? static_cast<std::uint32_t>(key) * kld + 16u * g : kOutOfRange;
 #pragma unroll
-            for (int c = 0; c < DC; ++c) {
-                const int key = j0 + 16 * kb + l16, d = 16 * c + 4 * g;
-                kf[kb][c] = load4(kr, d < p.D && key < p.Lk ? static_cast<std::uint32_t>(key * p.ks[2] + d) * 4u : kOutOfRange);
-            }
+            for (int c = 0; c < DC; ++c) kf[kb][c] = load4(kr, (16 * c + 4 * g < p.D ? row : kOutOfRange) + 64u * c);
+        }
     };
     auto load_v = [&](int j0) {
 #pragma unroll
         for (int kb = 0; kb < KB; ++kb)
 #pragma unroll
-            for (int t = 0; t < 4; ++t)
+            for (int t = 0; t < 4; ++t) {
+                const int key = j0 + 16 * kb + M::row(g, t);
+                const std::uint32_t row = key < p.Lk ? static_cast<std::uint32_t>(key) * vld + 16u * l16 : kOutOfRange;
 #pragma unroll
-                for (int c = 0; c < VC; ++c) {
-                    const int key = j0 + 16 * kb + M::row(g, t), d = 64 * c + 4 * l16;
-                    vf[kb][t][c] = load4(vr, d < p.Dv && key < p.Lk ? static_cast<std::uint32_t>(key * p.vs[2] + d) * 4u : kOutOfRange);
-                }
+                for (int c = 0; c < VC; ++c) vf[kb][t][c] = load4(vr, (64 * c + 4 * l16 < p.Dv ? row : kOutOfRange) + 256u * c);
+            }
     };
 
     vec o[QB][VC][4];
@@ -222,8 +226,12 @@ __global__ __launch_bounds__(kWavesF * 64) void sdpa_f32_kernel(const F32Params 
                 for (int kb = 0; kb < KB; ++kb)
 #pragma unroll
                     for (int r = 0; r < 4; ++r) mk[qb][kb][r] = static_cast<const float*>(p.mask)[mask_at(j0, qb, kb, r)];
-        if constexpr (kAhead) load_v(j0);
-        else                  load_k(j0);
+        if constexpr (kAhead) {
+            load_v(j0);
+        } else {
+            load_k(j0);
+            __builtin_amdgcn_sched_barrier(0);        // all of them on the way before the first is waited for
+        }
         vec s[QB][KB];
 #pragma unroll
         for (int qb = 0; qb < QB; ++qb)
@@ -244,20 +252,41 @@ __global__ __launch_bounds__(kWavesF * 64) void sdpa_f32_kernel(const F32Params 
         for (int qb = 0; qb < QB; ++qb) {
             const int i = q0 + 16 * qb + l16;
             float x[KB][4], mx = -INFINITY;
+            // (the scale as it is given, the product rounded once; the torch ops narrow it themselves, as the reference does,
+            // and the product of two floats needs no fp64)
+            if (p.scale_is_float) {
+                const float scale = static_cast<float>(p.scale);
+#pragma unroll
+                for (int kb = 0; kb < KB; ++kb)
+#pragma unroll
+                    for (int r = 0; r < 4; ++r) x[kb][r] = static_cast<float>(s[qb][kb][r]) * scale;
+            } else {
+#pragma unroll
+                for (int kb = 0; kb < KB; ++kb)
+#pragma unroll
+                    for (int r = 0; r < 4; ++r) x[kb][r] = static_cast<float>(static_cast<double>(static_cast<float>(s[qb][kb][r])) * p.scale);
+            }
+            // (selected where a mask is boolean: a NaN or infinite score of a masked key is no score)
+            if constexpr (kMask != 0)
+#pragma unroll
+                for (int kb = 0; kb < KB; ++kb)
+#pragma unroll
+                    for (int r = 0; r < 4; ++r) {
+                        if constexpr (kMask == 1) x[kb][r] = (open[qb] >> (4 * kb + r) & 1u) != 0 ? x[kb][r] : -INFINITY;
+                        else                      x[kb][r] += mk[qb][kb][r];
+                    }
+            if (j0 + kTurn > p.Lk || (p.is_causal && j0 + kTurn - 1 > q0 + 16 * qb))          // the last keys, the diagonal
+#pragma unroll
+                for (int kb = 0; kb < KB; ++kb)
+#pragma unroll
+                    for (int r = 0; r < 4; ++r) {
+                        const int j = j0 + 16 * kb + M::row(g, r);
+                        if (j >= p.Lk || (p.is_causal && j > i)) x[kb][r] = -INFINITY;
+                    }
 #pragma unroll
             for (int kb = 0; kb < KB; ++kb)
 #pragma unroll
-                for (int r = 0; r < 4; ++r) {
-                    const int j = j0 + 16 * kb + M::row(g, r);
-                    // (the scale as it is given: in fp64, rounded once; the torch ops narrow it themselves)
-                    float y = static_cast<float>(static_cast<double>(static_cast<float>(s[qb][kb][r])) * p.scale);
-                    // (selected where a mask is boolean: a NaN or infinite score of a masked key is no score)
-                    if constexpr (kMask == 1) y = (open[qb] >> (4 * kb + r) & 1u) != 0 ? y : -INFINITY;
-                    if constexpr (kMask == 2) y += mk[qb][kb][r];
-                    if (j >= p.Lk || (p.is_causal && j > i)) y = -INFINITY;
-                    x[kb][r] = y;
-                    mx = fmaxf(mx, y);
-                }
+                for (int r = 0; r < 4; ++r) mx = fmaxf(mx, x[kb][r]);
             if constexpr (sizeof(Acc) == 4)
                 if (p.attn != nullptr) {
 #pragma unroll
@@ -289,7 +318,10 @@ __global__ __launch_bounds__(kWavesF * 64) void sdpa_f32_kernel(const F32Params 
                     pr[qb][kb][r] = static_cast<Acc>(w);
                 }
         }
-        if constexpr (!kAhead) load_v(j0);
+        if constexpr (!kAhead) {
+            load_v(j0);
+            __builtin_amdgcn_sched_barrier(0);
+        }
 #pragma unroll
         for (int kb = 0; kb < KB; ++kb)
 #pragma unroll
@@ -464,6 +496,7 @@ int launch_f32(const paras_sdpa_args& a, bool accumulate_f64, void* workspace, h
         p.attn16 = a.Lk % 4 == 0 && (reinterpret_cast<uintptr_t>(a.attn) & 15) == 0;
     }
     p.scale = a.scale;
+    p.scale_is_float = static_cast<double>(static_cast<float>(a.scale)) == a.scale;
     // Lk weights of at most 1 / Lk: a weighted sum of values that fp32 holds is one that it holds
     p.above = kSlack + std::log(static_cast<double>(a.Lk));
     const long dm = a.D > a.Dv ? a.D : a.Dv;
