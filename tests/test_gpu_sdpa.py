@@ -954,3 +954,39 @@ def test_fp32_output_off_a_16_byte_boundary(Lq, Lk, D, Dv, want_attn):
     if want_attn:
         assert_bit_exact(attn[1:-1].view_as(wattn), wattn)
         assert bool(attn[[0, -1]].isinf().all())
+
+
+@pytest.mark.parametrize("cap", [None, 3 * 300 * 500, 50 * 1000])
+@pytest.mark.parametrize("kind", ["none", "causal", "bool", "additive"])
+@pytest.mark.parametrize("dtype,D,Dv,Lk", [(torch.float32, 66, 66, 500), (torch.float32, 260, 264, 512), (torch.float32, 64, 66, 4100), (torch.float64, 64, 64, 500)])
+def test_composed_route_of_problems_the_one_pass_kernel_does_not_take(dtype, D, Dv, Lk, kind, cap, monkeypatch):
+    """fp32 heads that are not multiples of 4 or beyond 256, and fp64: the batched products around the row kernels (rows
+    in 16-byte pieces, in registers, longer), whole and with the score bound lowered to a few heads or to blocks of rows."""
+    if cap is not None:
+        monkeypatch.setenv("PARAS_SDPA_SCORE_CAP", str(cap))
+    Lq = 300 if Lk < 4000 else 100
+    q, k, v = _composed_case(dtype, 2, 4, 2 if kind == "bool" else 4, Lq, Lk, D, Dv)
+    keep = torch.rand(2, 1, Lq, Lk) > 0.3
+    keep[..., 0] = True
+    keep[0, 0, 7] = False
+    kw = dict(none={}, causal=dict(is_causal=True), bool=dict(mask=keep), additive=dict(mask=torch.randn(1, 4, Lq, Lk).to(dtype)))[kind]
+    out, attn, lse, name = run(q, k, v, want_attn=True, want_lse=True, **kw)
+    assert name == "composed"
+    s = q.double() @ k.double().repeat_interleave(q.shape[1] // k.shape[1], 1).transpose(-1, -2) / math.sqrt(D)
+    if kind == "causal":
+        s = s.masked_fill(~torch.ones(Lq, Lk).tril().bool(), -math.inf)
+    elif kind == "bool":
+        s = s.masked_fill(~keep, -math.inf)
+    elif kind == "additive":
+        s = s + kw["mask"].double()
+    w = s.softmax(-1)
+    o = w @ v.double().repeat_interleave(q.shape[1] // v.shape[1], 1)
+    tol = REL_F32 if dtype == torch.float32 else 1e-12
+    for got, want in ((out, o), (attn, w), (lse, torch.logsumexp(s, -1))):
+        got, ok = got.cpu().double(), want.isfinite()
+        if got.dim() == 4:
+            assert torch.equal(got.isnan(), want.isnan())
+        bar = tol if got.dim() == 4 else 1e-6                           # (the log-sum-exp is fp32)
+        assert (got - want)[ok].abs().max().item() <= bar * want[ok].abs().max().item()
+    again = run(q, k, v, **kw)[0]                                       # scores in the workspace instead of the weights tensor
+    assert_bit_exact(out, again)
