@@ -1,12 +1,13 @@
 // Scaled-dot-product attention as the reference composes it
 // (csrc/ops/attention_ops.cpp:101-135), step by step on the device, for the
 // problems no fused kernel takes and the general one-row-per-workgroup kernel
-// would crawl through (fp32 / fp64 tensors, unusual head sizes or layouts at
-// sequence lengths in the thousands):
+// would crawl through: fp64 tensors, 16-bit heads or layouts that no MFMA kernel has,
+// fp32 heads beyond 256 or not a multiple of 4, at sequence lengths in the hundreds and thousands:
 //   s = T(q k^T)                     the batched product (paras_gemm_nt: fp32 accumulation,
 //                                    fp64 for fp64 tensors, one rounding to T)
 //   s = T(s * scale); -inf where masked / T(s + bias); p = T(softmax(s))   one row kernel, fp64
 //   o = T(p v)                       the batched product again, against v transposed once
+// (The other fp32 problems of this size, with or without returned weights, are sdpa_f32.hip's.)
 // The scores live in the caller's weights tensor when it asks for one, else in
 // the workspace, a bounded piece at a time (a few heads, or a block of query
 // rows of one head).  Each step narrows to T exactly where the reference's
@@ -347,17 +348,15 @@ int launch_composed(const paras_sdpa_args& a, void* workspace, void* stream, hip
     const long rep = a.Hq / a.Hkv;
 
     // v transposed once: the second product reads it along the keys
-    {
-        const dim3 grid(static_cast<unsigned>((a.Lk + 31) / 32), static_cast<unsigned>((a.Dv + 31) / 32), static_cast<unsigned>(a.B * a.Hkv));
-#define PARAS_TRANSPOSE_V(S_)                                                                                                   \
-    hipLaunchKernelGGL((transpose_v_kernel<S_>), grid, dim3(kBlock), 0, s, static_cast<const S_*>(a.v), reinterpret_cast<S_*>(vt), \
+    const dim3 vgrid(static_cast<unsigned>((a.Lk + 31) / 32), static_cast<unsigned>((a.Dv + 31) / 32), static_cast<unsigned>(a.B * a.Hkv));
+#define PARAS_TRANSPOSE_V(S_)                                                                                                    \
+    hipLaunchKernelGGL((transpose_v_kernel<S_>), vgrid, dim3(kBlock), 0, s, static_cast<const S_*>(a.v), reinterpret_cast<S_*>(vt), \
                        (long)a.Hkv, (long)a.Lk, (long)a.Dv, (long)a.v_strides[0], (long)a.v_strides[1], (long)a.v_strides[2])
-        if (es == 8)      PARAS_TRANSPOSE_V(double);
-        else if (es == 4) PARAS_TRANSPOSE_V(float);
-        else              PARAS_TRANSPOSE_V(std::uint16_t);
+    if (es == 8)      PARAS_TRANSPOSE_V(double);
+    else if (es == 4) PARAS_TRANSPOSE_V(float);
+    else              PARAS_TRANSPOSE_V(std::uint16_t);
 #undef PARAS_TRANSPOSE_V
-        PARAS_HIP_TRY(hipGetLastError());
-    }
+    PARAS_HIP_TRY(hipGetLastError());
 
     const bool run_on = heads_run_on(a);
     const long n_batches = run_on ? 1 : a.B, n_heads = run_on ? a.B * a.Hq : a.Hq;

@@ -7,7 +7,7 @@
 // S3737 D128: 740 us, of which 508 us one product with 60 workgroups).
 //
 // A workgroup takes 16 QB queries of one head; its four waves take the keys in turns of 32 (16 where
-// there are few keys or the registers are full) and meet at the end (running maximum, row sum, output: combined through LDS).  Per turn and wave:
+// there are few keys or the registers are full) and meet at the end (row maximum, row sum, output: combined through LDS).  Per turn and wave:
 //   S^T = K Q^T      v_mfma 16x16x4, A = 16 keys, B = 16 queries
 //   online softmax   a lane holds one query and 4 keys of each 16 x 16 block
 //   O^T += V^T P^T   the accumulator layout of S^T is the B operand layout of this product: step t takes
@@ -22,8 +22,18 @@
 // accumulated in fp32.  In both the softmax is fp64: exponentials and row sums unrounded, a weight rounded once, to
 // the type of the product that takes it.  Scores are rounded to fp32 where the reference's
 // are (the product, the scaled product, the sum with an additive mask: attention_ops.cpp:101-128).
-// What bounds it: small problems the chain of one turn (two memory latencies, products, merge), large ones
-// the matrix cores and the L2 reads of K and V by every 16 QB queries.
+// Against fp64, S 300 to 8192, heads of 64 to 256, scores of deviation 1 and 3: 3 to 49 % nearer than the batched products
+// around an fp64 row kernel, which add up all keys in one chain where four waves add up a quarter each.
+//
+// NaN and infinities come out where the reference's do: a boolean mask and the causal rule select, an additive mask is
+// added, and a value that nobody sees is still multiplied by its zero weights.
+//
+// What bounds it: small problems the chain of one turn (two memory latencies, products, merge; B1 H8 S128 D64 causal 6.9 us),
+// large ones the matrix cores and the vector instructions, which do not run beside fp32 MFMAs here (weights of one query
+// block interleaved with the products of the other, one MFMA to seven vector instructions: 874 -> 903 us).  B2 H16 S2048
+// D128: unmasked 742 us = 93 TFLOP/s, causal 623 (every value is read, seen or not: 25 of them), 30 % padding 775, an additive
+// mask 830; the batched products took 967 / 907 / 1520 / 1590.  B2 H8 S1024 D64 55 us (174), B1 H4 S2048 D256 203 (317).  With the
+// softmax in fp32 it took 697 / 567 / 665 / 950, 47 and 228, and single weights were 4.9e-7 off instead of 1.1e-7.
 #include <hip/hip_runtime.h>
 
 #include <cmath>
@@ -37,7 +47,9 @@ namespace {
 
 constexpr int kWavesF = 4;
 constexpr std::uint32_t kOutOfRange = 0xF0000000u;
-constexpr double kSlack = 8.0;      // how far the running maximum may rise before the sums are rescaled
+// How far the running maximum may rise before the sums are rescaled: scores of deviation 1 to 3 rise by less after their first
+// turn, and what it takes from fp32's exponent range is 8 of 87 powers of e.
+constexpr double kSlack = 8.0;
 
 struct F32Params {
     const float* q; const float* k; const float* v; float* out; float* lse;
@@ -402,7 +414,8 @@ __global__ __launch_bounds__(kWavesF * 64, DM == 64 ? 2 : 1) void sdpa_f32_kerne
 
 // The returned weights, in place of the scores that sdpa_f32_kernel left: exp(score - reference) / sum in fp64, rounded
 // once; zeros for the keys that the causal rule hides (NaN where the row is).  A wave takes a row in pieces of W elements.
-// Bound by memory (one read and one write of the weights tensor); four pieces are on the way at a time.
+// Bound by memory (one read and one write of the weights tensor); four pieces are on the way at a time.  B2 H16 S2048 D128 with
+// its 537 MB of weights 1000 us, causal 805; the product, row kernel and product in their place 967 and 907; B2 H8 S1024 D64 89 (174).
 template <int W>
 __global__ __launch_bounds__(256) void softmax_rows_kernel(float* __restrict__ attn, const double2* __restrict__ row_sums, long rows, int Lq, int Lk, int is_causal) {
     typedef float piece __attribute__((ext_vector_type(W)));

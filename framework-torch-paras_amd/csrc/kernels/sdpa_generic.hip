@@ -13,7 +13,7 @@
 //   o  = T(sum_j p*v)                    second bmm
 // All arithmetic is fp64 (78 TFLOP/s of it on this part; this path serves
 // small and unusual shapes, the large regular ones go to the MFMA kernels, and
-// fp32 problems without returned weights to sdpa_f32.hip).
+// small fp32 problems without returned weights to sdpa_f32.hip's fp64 form).
 //
 // One 256-thread workgroup per (batch, head, query) row.  Scores are not
 // stored: pass 1 finds the row max, pass 2 the denominator, pass 3 recomputes

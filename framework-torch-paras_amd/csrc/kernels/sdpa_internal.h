@@ -28,8 +28,9 @@ bool weights_supported(const paras_sdpa_args& a);
 int  launch_weights(const paras_sdpa_args& a, hipStream_t s);
 
 // The reference's composition run step by step with the library's own batched products and one
-// row kernel (fp32 / fp64 tensors, head sizes and layouts the fused kernels do not take), for
-// problems big enough that the general kernel would take milliseconds.
+// row kernel (fp64 tensors, head sizes and layouts the fused kernels do not take), for
+// problems big enough that the general kernel would take milliseconds; fp32 ones that f32_supported
+// takes go to launch_f32.
 bool   composed_supported(const paras_sdpa_args& a);
 size_t composed_workspace(const paras_sdpa_args& a);
 int    launch_composed(const paras_sdpa_args& a, void* workspace, void* stream, hipStream_t s);
@@ -44,7 +45,8 @@ int gemm_nt_causal(const void* a, const void* b, const void* addend, void* c, in
                    void* workspace, size_t workspace_bytes, void* stream, int causal_kind, long causal_first);
 
 // fp32 attention in one pass, products accumulated in fp64 (the general route's problems, without returned weights) or
-// fp32 (the composed route's): head sizes of up to 256 that are multiples of 4.
+// fp32 (the composed route's, with or without them), softmax in fp64: head sizes of up to 256 that are multiples of 4.
+// The workspace is for returned weights (two doubles per query), 256-byte aligned.
 bool   f32_supported(const paras_sdpa_args& a);
 size_t f32_workspace(const paras_sdpa_args& a);
 int    launch_f32(const paras_sdpa_args& a, bool accumulate_f64, void* workspace, hipStream_t s);

@@ -9,10 +9,11 @@
 // chunks of a row are permuted by its index, so that neither side has bank conflicts).
 //
 // The eight waves of a workgroup share out the contraction in pieces of 64 (128 bytes of a row each, dealt round
-// robin).  P pieces of a wave are under way in registers at any time, 130 to 200 KB per CU with two workgroups; a piece
+// robin).  P pieces of a wave are under way in registers at any time, 130 to 200 KB per CU where it holds two workgroups (a
+// workgroup takes whole weight rows, so 4096 rows give a CU one and 1024 rows give 64 of the 256 CUs one); a piece
 // past the wave's last is requested with an empty extent, which fetches nothing and keeps the number of requests
-// in flight known to the compiler (P is what fits into 128 registers: with one more, spilled registers are
-// reloaded through the same counter and the loop waits for everything: 25.9 -> 30.8 us for 8 x 14336 x 4096).
+// in flight known to the compiler (P is what the loop fits into 128 registers: with one more, spilled registers are
+// reloaded in it through the same counter and it waits for everything: 25.9 -> 30.8 us for 8 x 14336 x 4096).
 //
 // Against feeding the MFMAs straight from memory, bf16: 8 x 1024 x 4096 8.4 -> 6.0 us, 8 x 14336 x 4096 30.0 -> 26.2
 // (4.5 TB/s), 8 x 4096 x 14336 25.1 -> 22.5 (5.2), 13 x 2048 x 2048 6.1 -> 5.2; a mixture-of-experts layer (8 experts, top-2,

@@ -245,10 +245,13 @@ PARAS_API int paras_sdpa_fwd(const paras_sdpa_args* args, void* workspace, void*
  * head sizes below 256 other than 64 and 128: q, k, v copied into the workspace with
  * zero columns up to 64, 128 or 256, then flash_mfma / decode_split; the workspace
  * must be 256-byte aligned), "composed" (what none of these takes, from about
- * 3e7 multiply-adds and 64 queries and keys on: the reference's own composition,
+ * 3e7 multiply-adds and 64 queries and keys on: fp32 heads of up to 256 that are
+ * multiples of 4 in one pass on the matrix cores, with fp32 sums and an fp64
+ * softmax; anything else as the reference's own composition,
  * csrc/ops/attention_ops.cpp:101-135, run as two batched paras_gemm_nt products
  * around one scale / mask / softmax row kernel, scores in `attn` or in the
- * 256-byte aligned workspace, a bounded piece at a time) or "generic". */
+ * 256-byte aligned workspace, a bounded piece at a time) or "generic" (the rest;
+ * fp32 as above without returned weights in one pass with fp64 sums). */
 PARAS_API const char* paras_sdpa_kernel_name(const paras_sdpa_args* args);
 
 /* ------------------------------------------------------------------------- */
@@ -344,12 +347,13 @@ PARAS_API int paras_moe_ffn(const void* x, const void* w_gate, const void* w_up,
 /* x W^T of nn.Linear, q k^T), C [M, N] rows ldc apart; batch strides in       */
 /* elements (0 = shared).  addend may be NULL; ld_add = 0 broadcasts one row   */
 /* (a bias) over the M rows.  All four float dtypes.  bf16 / f16 with K a       */
-/* multiple of 64 and 16-byte aligned operand rows run on the MFMA kernels     */
-/* (fp32 accumulation, one rounding); fp32 tensors with at least 32 tiles of   */
-/* 128 x 128 outputs on the fp32 MFMA kernel (full fp32 multiplies, any K and  */
-/* alignment); everything else -- fp64 tensors, small fp32 products, 16-bit    */
-/* ones with other K or alignments -- on a general kernel (fp32 accumulation,  */
-/* fp64 for fp64 tensors), so no product needs a host path.                    */
+/* multiple of 8, 16-byte aligned operands and leading dimensions and batch    */
+/* strides that are multiples of 8 run on the MFMA kernels (fp32 accumulation, */
+/* one rounding; up to 32 rows, 128 without a workspace, on kernels that stream */
+/* the weights, K a multiple of 64); fp32 tensors on the fp32 MFMA kernel (full */
+/* fp32 multiplies, any K and alignment); everything else -- fp64 tensors,     */
+/* 16-bit ones with other K or alignments -- on a general kernel (fp32         */
+/* accumulation, fp64 for fp64 tensors), so no product needs a host path.      */
 /* ------------------------------------------------------------------------- */
 PARAS_API int paras_gemm_nt(const void* a, const void* b, const void* addend, void* c,
                             int64_t M, int64_t N, int64_t K, int64_t lda, int64_t ldb,
