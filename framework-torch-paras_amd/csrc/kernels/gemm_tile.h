@@ -1,6 +1,6 @@
-// Tile mainloops shared by the MFMA GEMM kernels (grouped expert GEMMs and the
-// dense NT GEMM): C tile = A[rows x K] * B[256 x K]^T with bf16/fp16 operands and
-// fp32 accumulation on v_mfma_f32_32x32x16.
+// Register-staged tile mainloops of the grouped expert GEMMs (128-row tiles, and 256-row ones that
+// gemm_flex.h's 32-bit offsets do not reach): C tile = A[rows x K] * B[256 x K]^T with bf16/fp16
+// operands and fp32 accumulation on v_mfma_f32_32x32x16.
 //
 // Both operands are read along their contiguous contraction dim, which is the
 // 8-element-per-lane operand layout of the MFMA, so neither needs a transpose.
