@@ -990,3 +990,27 @@ def test_composed_route_of_problems_the_one_pass_kernel_does_not_take(dtype, D, 
         assert (got - want)[ok].abs().max().item() <= bar * want[ok].abs().max().item()
     again = run(q, k, v, **kw)[0]                                       # scores in the workspace instead of the weights tensor
     assert_bit_exact(out, again)
+
+
+def test_fp32_weights_of_the_one_pass_kernel_in_a_captured_graph():
+    """The two launches that make outputs and returned weights, captured once and replayed on new inputs between eager
+    work: every replay equals the eager result, whatever the weights tensor held."""
+    q, k, v = (torch.randn(1, 4, n, 64, device="cuda") for n in (300, 500, 500))
+    out, attn = torch.empty(1, 4, 300, 64, device="cuda"), torch.empty(1, 4, 300, 500, device="cuda")
+    a = capi.sdpa_args(q, k, v, out, attn, is_causal=True)
+    ws = torch.empty(capi.lib().paras_sdpa_workspace(C.byref(a)), dtype=torch.uint8, device="cuda")
+    call = lambda: capi.check(capi.lib().paras_sdpa_fwd(C.byref(a), ws.data_ptr(), torch.cuda.current_stream().cuda_stream))
+    call()
+    torch.cuda.synchronize()
+    graph = torch.cuda.CUDAGraph()
+    with torch.cuda.graph(graph):
+        call()
+    for i in range(4):
+        for t in (q, k, v):
+            t.copy_(torch.randn_like(t))
+        attn.fill_(math.nan)
+        graph.replay()
+        torch.cuda.synchronize()
+        want, wattn, _, _ = capi.sdpa(q, k, v, is_causal=True, want_attn=True)
+        assert_bit_exact(out, want)
+        assert_bit_exact(attn, wattn)
