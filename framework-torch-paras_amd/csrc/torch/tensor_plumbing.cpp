@@ -12,6 +12,7 @@
 #include <ATen/native/CPUFallback.h>
 #include <ATen/native/Resize.h>
 #include <c10/core/DeviceGuard.h>
+#include <c10/core/impl/LocalDispatchKeySet.h>
 
 #include <cstring>
 #include <vector>
@@ -148,6 +149,17 @@ Tensor copy_from(const Tensor& self, const Tensor& dst, bool non_blocking) {
     TORCH_CHECK(false, "paras _copy_from: unsupported device pair ", self.device(), " -> ", dst.device());
 }
 
+// A copy from or into a view whose elements count negated (the flag of torch._neg_view and of imaginary parts of
+// conjugates).  Without a kernel for it the dispatcher resolves such a view by cloning it, which is a copy that
+// comes here again, and so on until the stack ends.  Here the memory is copied as it lies and negated if the two differ.
+Tensor copy_from_negated(const Tensor& self, const Tensor& dst, bool non_blocking) {
+    const bool differ = self.is_neg() != dst.is_neg();
+    const c10::impl::ExcludeDispatchKeyGuard as_it_lies(c10::DispatchKey::Negative);
+    at::_copy_from(self, dst, non_blocking);
+    if (differ) const_cast<Tensor&>(dst).neg_();
+    return dst;
+}
+
 Tensor copy_from_and_resize(const Tensor& self, const Tensor& dst) {
     if (dst.sizes() != self.sizes()) const_cast<Tensor&>(dst).resize_(self.sizes());
     return copy_from(self, dst, false);
@@ -244,6 +256,8 @@ TORCH_LIBRARY_IMPL(aten, PrivateUse1, m) {
     m.impl("aten::resize_", &resize_);
     m.impl("aten::_has_compatible_shallow_copy_type", &has_compatible_shallow_copy_type);
 }
+
+TORCH_LIBRARY_IMPL(aten, Negative, m) { m.impl("aten::_copy_from", &paras_torch::copy_from_negated); }
 
 TORCH_LIBRARY_IMPL(_, PrivateUse1, m) {
     m.fallback(torch::CppFunction::makeFromBoxedFunction<&paras_torch::cpu_fallback>());

@@ -1038,3 +1038,26 @@ def test_linear_backward_of_gradients_that_are_not_plain_tensors(device, lead):
     assert all(t is not None for t in got)
     for g, w in zip(got, want):
         assert_close(g, w)
+
+
+def test_negated_views_are_read_negated(device):
+    """Operands with the negative bit (torch._neg_view: the memory holds the opposite sign): projections, attention, the
+    fused ops and copies of them, against the CPU."""
+    import torch_paras
+    nn, neg = torch_paras.nn, torch._neg_view
+    x, w, b, q = torch.randn(5, 8), torch.randn(6, 8), torch.randn(6), torch.randn(1, 2, 16, 64)
+    calls = [(F.linear, x, w, b), (torch.mm, x, w.t().contiguous()), (F.scaled_dot_product_attention, q, q + 1, q - 1), (nn.swiglu, x, x + 1),
+             (torch.add, x, x + 2)]
+    for f, *args in calls:
+        for which in range(len(args)):
+            on = [a.to(device) for a in args]
+            plain, on[which] = [-a if i == which else a for i, a in enumerate(args)], neg(on[which])
+            want = f(*plain) if f is not nn.swiglu else F.silu(plain[0]) * plain[1]
+            assert_close(f(*on), want, f"{f} {which}")
+    assert torch.equal(neg(x.to(device)).cpu(), -x)
+    assert torch.equal(neg(x.to(device)).contiguous().cpu(), -x)
+    into = torch.zeros(5, 8).to(device)
+    neg(into).copy_(x.to(device))
+    assert torch.equal(into.cpu(), -x)
+    neg(into).copy_(x)
+    assert torch.equal(into.cpu(), -x)
