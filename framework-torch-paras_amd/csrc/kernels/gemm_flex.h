@@ -11,11 +11,17 @@
 //
 // A workgroup is four waves, 2 x 2, one per SIMD at the large tiles; a wave computes MI x NJ blocks of
 // 16 x 16, so the tile is 32 MI x 32 NJ.  Tiles of 64 contraction steps go from memory straight to LDS
-// (buffer_load ... lds), two stages: no staging registers, no LDS stores, nothing in the loop but
-// MFMAs, LDS reads and one request per four MFMAs, which is what a single wave per SIMD can issue in the
+// (buffer_load ... lds), ST stages: no staging registers, no LDS stores, nothing in the loop but
+// MFMAs, LDS reads and one request per few MFMAs, which is what a single wave per SIMD can issue in the
 // shadow of its MFMAs.  One barrier per tile, before its last k-step: by then all of the tile's
-// fragments are in registers, so the tile after next can be requested into its stage right away and has
-// a tile's time to arrive, while the k-step's MFMAs run and the next tile's first fragments are read.
+// fragments are in registers, so its stage can be requested anew right away, for the tile ST further on, and has
+// ST - 1 tiles' time to arrive, while the k-step's MFMAs run and the next tile's first fragments are read.
+//
+// What bounds it is the number of stages where a CU holds one or two workgroups of small tiles: a tile of 64 x 64 is 512
+// cycles of MFMA and LDS work, and its operands are 1500 cycles away.  Waits are for the next tile's requests only, the later ones stay
+// in flight (64 x 128 tiles, x W^T in bf16, two stages -> four: 1500 x 1024 x 4096 29.6 -> 23.1 us, 2040 x 1024 x 3584 29.5 -> 22.1,
+// 232 x 7168 x 2048 25.6 -> 17.8; 192 x 128, three stages: 1500 x 4096 x 4096 60.8 -> 50.2).  256-row tiles fill LDS with two stages and are
+// bound by the matrix cores' power.
 //
 // Direct loads fill LDS in lane order, so rows cannot be padded apart; instead the 16-byte chunks of a
 // row (K) or the 32-byte units (R) are permuted by a function of the row, applied to the address a
@@ -25,6 +31,8 @@
 #pragma once
 
 #include <hip/hip_runtime.h>
+
+#include <type_traits>
 
 #include "core/device_math.h"
 #include "kernels/gemm_tile.h"
@@ -130,14 +138,15 @@ template <int W, bool R> struct Operand {
 
 // acc[i][j]: the B fragment is the instruction's first operand, so lane (l16 = lane % 16, kq = lane / 16)
 // holds row i*16 + l16 of the wave's rows and columns j*16 + 4*kq .. + 3 of its columns.
-// (The stages are separate arrays named at compile time: an LDS read waits for every direct load in flight
+// (The ST stages are separate arrays named at compile time: an LDS read waits for every direct load in flight
 // that the compiler cannot prove to go elsewhere.)
 // OA, OB: Operand or a type with its rsrc / request / frag / last_tile.
-template <typename T, int MI, int NJ, typename OA, typename OB>
-__device__ __forceinline__ void mainloop(OA& oa, OB& ob, int k_count, std::uint16_t* a0, std::uint16_t* a1,
-                                         std::uint16_t* b0, std::uint16_t* b1, float4v (&acc)[MI][NJ]) {
+template <typename T, int MI, int NJ, int ST, typename OA, typename OB>
+__device__ __forceinline__ void mainloop(OA& oa, OB& ob, int k_count, std::uint16_t* const (&sa)[ST], std::uint16_t* const (&sb)[ST],
+                                         float4v (&acc)[MI][NJ]) {
     constexpr int C = MI + NJ;          // requests per wave and tile, and fragments per k-step
     constexpr int S = MI * NJ;          // MFMAs per k-step
+    static_assert(ST >= 2 && (ST - 1) * C < 64, "the tiles in flight have to fit the load counter");
     i16x8 af[2][MI], bf[2][NJ];
     const int k_tiles = (k_count + kBK - 1) / kBK;
     auto request_one = [&](const auto& ra, const auto& rb, std::uint16_t* ta, std::uint16_t* tb, int c) {
@@ -158,9 +167,11 @@ __device__ __forceinline__ void mainloop(OA& oa, OB& ob, int k_count, std::uint1
         if (f < MI) af[buf][f] = oa.frag(ta, f, ks);
         else        bf[buf][f - MI] = ob.frag(tb, f - MI, ks);
     };
-    auto meet = [] {
-        __builtin_amdgcn_s_waitcnt(0x0070);     // vmcnt(0) lgkmcnt(0): this wave's part of the next tile has landed, its reads of this one are done
-        lds_barrier();
+    // this wave's part of the next tile has landed (those of `ahead` tiles after it may be under way), its reads of this one are done
+    auto meet = [](auto ahead) {
+        constexpr int n = decltype(ahead)::value * C;
+        __builtin_amdgcn_s_waitcnt(0x0070 | (n & 15) | ((n >> 4) << 14));     // vmcnt(n) lgkmcnt(0)
+        asm volatile("s_barrier" ::: "memory");     // (a fence of the compiler's own would wait for every direct load in flight)
     };
 #pragma unroll
     for (int i = 0; i < MI; ++i)
@@ -173,22 +184,22 @@ __device__ __forceinline__ void mainloop(OA& oa, OB& ob, int k_count, std::uint1
             for (int j = 0; j < NJ; ++j) asm volatile("" : "+a"(acc[i][j]));
     };
     pin();
-    // The requests for the tile after next are spread over the whole k-step that follows the barrier: bunched into
+    // The requests for the next tile that goes into this stage are spread over the whole k-step that follows the barrier: bunched into
     // its first half they come at twice the rate the CU's L1 takes them and hold up the MFMAs (8192^3 807 against
     // 774 us), spread further into the next k-step the last of them are late at the barrier (788 us).
     // Tile kt from stage (ca, cb); the next one is in (na, nb).  One body for every tile, the last ones included:
     // a copy of it for them costs the accumulators their places (hundreds of spills), so requests past the end
     // go to an empty extent, which fetches nothing and clears the stage.
     auto tile = [&](int kt, std::uint16_t* ca, std::uint16_t* cb, std::uint16_t* na, std::uint16_t* nb) {
-        if (kt + 2 == k_tiles - 1) {
-            oa.last_tile(k_count - (kt + 2) * kBK);
-            ob.last_tile(k_count - (kt + 2) * kBK);
+        if (kt + ST == k_tiles - 1) {
+            oa.last_tile(k_count - (kt + ST) * kBK);
+            ob.last_tile(k_count - (kt + ST) * kBK);
         }
-        const auto ra = oa.rsrc(kt + 2, k_tiles);
-        const auto rb = ob.rsrc(kt + 2, k_tiles);
+        const auto ra = oa.rsrc(kt + ST, k_tiles);
+        const auto rb = ob.rsrc(kt + ST, k_tiles);
 #pragma unroll
         for (int ks = 0; ks < 2; ++ks) {
-            if (ks == 1) meet();
+            if (ks == 1) meet(std::integral_constant<int, ST - 2>{});
 #pragma unroll
             for (int j = 0; j < NJ; ++j)
 #pragma unroll
@@ -204,15 +215,15 @@ __device__ __forceinline__ void mainloop(OA& oa, OB& ob, int k_count, std::uint1
                 }
         }
     };
-    request_all(0, a0, b0);
-    request_all(1, a1, b1);
-    meet();
 #pragma unroll
-    for (int f = 0; f < C; ++f) read_frag(a0, b0, 0, f, 0);
-    // (In pairs, with one way out: an odd number of tiles multiplies a cleared one at the end.)
-    for (int kt = 0; kt < k_tiles; kt += 2) {
-        tile(kt, a0, b0, a1, b1);
-        tile(kt + 1, a1, b1, a0, b0);
+    for (int u = 0; u < ST; ++u) request_all(u, sa[u], sb[u]);
+    meet(std::integral_constant<int, ST - 1>{});
+#pragma unroll
+    for (int f = 0; f < C; ++f) read_frag(sa[0], sb[0], 0, f, 0);
+    // (In whole turns of the stages, with one way out: tiles past the last one multiply cleared stages.)
+    for (int kt = 0; kt < k_tiles; kt += ST) {
+#pragma unroll
+        for (int u = 0; u < ST; ++u) tile(kt + u, sa[u], sb[u], sa[(u + 1) % ST], sb[(u + 1) % ST]);
     }
     asm volatile("s_nop 15\n\ts_nop 15" ::: "memory");      // the last products are on their way to the registers the epilogue reads
     pin();

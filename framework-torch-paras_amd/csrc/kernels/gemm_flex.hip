@@ -51,13 +51,15 @@ __global__ __launch_bounds__(256) void gemm_flex_finish_kernel(const Params p) {
     }
 }
 
-// Per tile shape: rows, columns, workgroups a CU holds at once, and in us the time of one tile of 64
-// contraction steps on a CU that is full (`step`) and at least, on a CU with a single workgroup (`lat`: a
+// Per tile form: rows, columns, stages, workgroups a CU holds at once, and in us the time of one tile of 64
+// contraction steps on a CU that is full (`step`) and at least, on a CU with fewer workgroups (`lat`: a
 // barrier and the way from L2).
-struct Tile { int m, n, per_cu; double step, lat; };
-constexpr Tile kTiles[] = {{256, 256, 1, 1.39, 0.66}, {192, 256, 1, 1.09, 0.26}, {128, 256, 1, 0.93, 0.17}, {128, 128, 2, 0.86, 0.58},
-                           {64, 128, 3, 0.94, 0.39}, {64, 64, 4, 0.84, 0.20}, {32, 128, 3, 0.84, 0.26}};
-constexpr int kTileCount = 7;
+struct Tile { int m, n, stages, per_cu; double step, lat; };
+constexpr Tile kTiles[] = {{256, 256, 2, 1, 1.15, 0.36}, {192, 256, 2, 1, 0.94, 0.05}, {192, 192, 3, 1, 0.71, 0.34}, {192, 128, 3, 1, 0.55, 0.55},
+                           {128, 128, 2, 2, 0.84, 0.56}, {128, 128, 3, 1, 0.42, 0.34}, {64, 128, 2, 3, 0.90, 0.45}, {64, 128, 4, 1, 0.285, 0.30},
+                           {64, 64, 2, 4, 0.83, 0.36},   {64, 64, 3, 3, 0.545, 0.22},  {64, 64, 4, 2, 0.34, 0.21},  {32, 128, 4, 2, 0.43, 0.26}};
+constexpr int kTileCount = sizeof(kTiles) / sizeof(kTiles[0]);
+static_assert(kTiles[kTile128x128].m == 128 && kTiles[kTile128x128].n == 128 && kTiles[kTile128x128].stages == 2, "the tile that paras_gemm_nt_ws splits");
 constexpr int kCus = 256;
 
 }  // namespace
@@ -74,37 +76,38 @@ bool takes(const Problem& q) {
     return q.batch <= 65535 && tiles * q.batch < (1L << 25);
 }
 
-// The least estimated time over tile shapes and numbers of parts.  Rounds of workgroups times the time of
+// The least estimated time over tile forms and numbers of parts.  Rounds of workgroups times the time of
 // their share of the contraction and of their stores, plus the second kernel where the contraction is in
-// parts.  The constants were fitted to 6900 timings (1 to 16384 rows, 512 to 14336 columns, contractions of 8
-// to 14336, all three layouts): over those the choice is 1.9 % slower than the best one in the mean and 10 % at the
+// parts.  The constants were fitted to 55000 timings of 1250 problems (17 to 16384 rows, 64 to 14336 columns, contractions of
+// 18 to 14336, all three layouts): over those that take 8.5 us or more the choice is 1.1 % slower than the best one in the mean and 6 % at the
 // 95th percentile.  What the rule trades: a 256 x 256 tile reads half as much per flop as a 128 x 128 one
-// (16384 x 4096 x 4096 395 against 459 us), but with 192 of them for 256 CUs a quarter of the chip idles
-// (3000 x 4096 x 4096 98 us, with 256 tiles of 192 x 256 83 us); with few tiles the contraction is cut up
-// instead (8 x 14336 x 4096 41 us whole, 25 us in four parts).
+// (8192^3 757 us, 256 x 128 877), but with 192 of them for 256 CUs a quarter of the chip idles
+// (3000 x 4096 x 4096 94 us, with 256 tiles of 192 x 256 84 us); a small problem has few workgroups per CU, and then more
+// stages stand in for the other workgroups' loads (821 x 1024 x 3584 64 x 64: two stages in four parts 21 us, four stages 14.5 whole);
+// what is still too few tiles is cut up along the contraction (261 x 4096 x 14336 192 x 128: four parts 52 us).
 Plan plan(const Problem& q, bool may_split) {
     Plan best;
     double best_us = 1e30;
     const long k_tiles = (q.K + kBK - 1) / kBK;
     const double mn = static_cast<double>(q.M) * q.N * q.batch;
+    const double memory = static_cast<double>(q.M + q.N) * q.K * q.batch * 2 / 5.6e6 + 2.5;      // the operands' way from memory
     for (int t = 0; t < kTileCount; ++t) {
         const Tile& tl = kTiles[t];
-        if (t < 3 && q.K <= 512) continue;           // mostly stores: small tiles overlap them with other tiles' work
+        if (tl.m * tl.n > 128 * 128 && q.K <= 512) continue;     // mostly stores: small tiles overlap them with other tiles' work
         const long mt = (q.M + tl.m - 1) / tl.m, nt = (q.N + tl.n - 1) / tl.n, tiles = mt * nt * q.batch;
-        // the share of its panels that a workgroup is the first to ask for comes from further away than L2
-        const double first = (static_cast<double>(tl.n) / mt + static_cast<double>(tl.m) / nt) / (tl.m + tl.n);
-        const double lat = tl.lat + 0.54 * first, stores = tl.m * tl.n / 65536.0 * 4.7;
         for (int s = 1; s <= (may_split ? 32 : 1); s = s < 4 ? s + 1 : s + s / 2) {
             if (s > 1 && (s * 2 > k_tiles || tiles * s > 1600)) break;
-            const long per = (k_tiles + s - 1) / s, parts = (k_tiles + per - 1) / per, paired = per + (per & 1);
+            const long per = (k_tiles + s - 1) / s, parts = (k_tiles + per - 1) / per, turns = (per + tl.stages - 1) / tl.stages * tl.stages;
             const long wgs = tiles * parts, slots = static_cast<long>(kCus) * tl.per_cu, full = wgs / slots;
             const long rest = (wgs - full * slots + kCus - 1) / kCus;
+            const double stores = tl.m * tl.n / 65536.0 * (parts > 1 ? 8.9 : 7.5);
             auto round = [&](double n) {
                 const double c = tl.step * n / tl.per_cu;
-                return paired * (c > lat ? c : lat) + 2.3 + stores * n;
+                return turns * (c > tl.lat ? c : tl.lat) + 3.1 + stores * n;
             };
             double us = full * round(tl.per_cu) + (rest > 0 ? round(static_cast<double>(rest)) : 0.0);
-            if (parts > 1) us += 3.0 + mn * (8.0 * parts + 2.0) / 6.9e6;
+            if (us < memory) us = memory;
+            if (parts > 1) us += 4.0 + mn * (8.0 * parts + 2.0) / 6.9e6;
             if (us < best_us) {
                 best_us = us;
                 best.tile = t;

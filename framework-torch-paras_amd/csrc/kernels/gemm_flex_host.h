@@ -21,7 +21,7 @@ struct Problem {
     bool a_rows, b_rows;        // the operand is contiguous along its rows, not along the contraction (a_rows only with b_rows)
     bool bf16;
 };
-constexpr int kTile128x128 = 3;      // its index in the tile table
+constexpr int kTile128x128 = 4;      // the index of its two-stage form in the tile table
 struct Plan {
     int  tile = 0;              // index into the tile table
     int  splits = 1;            // parts of the contraction

@@ -45,15 +45,19 @@ __device__ __forceinline__ Work work_of(const Params& p, unsigned wg, unsigned t
             static_cast<int>(band * kBand + (in - nt * rows)), static_cast<int>(nt)};
 }
 
-template <typename T, int MI, int NJ, bool AR, bool BR>
-__global__ __launch_bounds__(kThreads, (MI * NJ >= 32 ? 1 : 2)) void gemm_flex_kernel(const Params p) {
+template <typename T, int MI, int NJ, int ST, bool AR, bool BR>
+__global__ __launch_bounds__(kThreads, (MI * NJ >= 32 || ST * (MI + NJ) > 20 ? 1 : 2)) void gemm_flex_kernel(const Params p) {
     using El = Elem<T>;
     using OA = Operand<MI, AR>;
     using OB = Operand<NJ, BR>;
     __shared__ __attribute__((aligned(1024))) std::uint16_t a0[OA::kElems];
     __shared__ __attribute__((aligned(1024))) std::uint16_t a1[OA::kElems];
+    __shared__ __attribute__((aligned(1024))) std::uint16_t a2[OA::kElems];     // (stages past ST are never named, and take no memory)
+    __shared__ __attribute__((aligned(1024))) std::uint16_t a3[OA::kElems];
     __shared__ __attribute__((aligned(1024))) std::uint16_t b0[OB::kElems];
     __shared__ __attribute__((aligned(1024))) std::uint16_t b1[OB::kElems];
+    __shared__ __attribute__((aligned(1024))) std::uint16_t b2[OB::kElems];
+    __shared__ __attribute__((aligned(1024))) std::uint16_t b3[OB::kElems];
     const Work w = work_of(p, blockIdx.x, gridDim.x);
     const long row0 = static_cast<long>(w.mt) * (32 * MI), col0 = static_cast<long>(w.nt) * (32 * NJ);
     const long k_first = static_cast<long>(w.split) * p.k_per_split;
@@ -64,7 +68,9 @@ __global__ __launch_bounds__(kThreads, (MI * NJ >= 32 ? 1 : 2)) void gemm_flex_k
     oa.init(p.a + w.batch * p.sa, p.lda, p.M, row0, k_first, k_count, wave >> 1);
     ob.init(p.b + w.batch * p.sb, p.ldb, p.N, col0, k_first, k_count, wave & 1);
     float4v acc[MI][NJ];
-    mainloop<T, MI, NJ>(oa, ob, static_cast<int>(k_count), a0, a1, b0, b1, acc);
+    if constexpr (ST == 2)      mainloop<T, MI, NJ, 2>(oa, ob, static_cast<int>(k_count), {a0, a1}, {b0, b1}, acc);
+    else if constexpr (ST == 3) mainloop<T, MI, NJ, 3>(oa, ob, static_cast<int>(k_count), {a0, a1, a2}, {b0, b1, b2}, acc);
+    else                        mainloop<T, MI, NJ, 4>(oa, ob, static_cast<int>(k_count), {a0, a1, a2, a3}, {b0, b1, b2, b3}, acc);
 
     const int lane = threadIdx.x & 63;
     const int l16 = lane & 15, kq = lane >> 4;
@@ -137,18 +143,23 @@ __global__ __launch_bounds__(kThreads, (MI * NJ >= 32 ? 1 : 2)) void gemm_flex_k
     }
 }
 
-// Tile shapes, largest first; kTiles in gemm_flex.hip describes them in the same order.
+// Tile forms, largest first; kTiles in gemm_flex.hip describes them in the same order.
 template <typename T, bool AR, bool BR>
 void launch_tile(int tile, const Params& p, unsigned grid, hipStream_t s) {
     const dim3 g(grid), t(kThreads);
     switch (tile) {
-        case 0: hipLaunchKernelGGL((gemm_flex_kernel<T, 8, 8, AR, BR>), g, t, 0, s, p); break;
-        case 1: hipLaunchKernelGGL((gemm_flex_kernel<T, 6, 8, AR, BR>), g, t, 0, s, p); break;
-        case 2: hipLaunchKernelGGL((gemm_flex_kernel<T, 4, 8, AR, BR>), g, t, 0, s, p); break;
-        case 3: hipLaunchKernelGGL((gemm_flex_kernel<T, 4, 4, AR, BR>), g, t, 0, s, p); break;
-        case 4: hipLaunchKernelGGL((gemm_flex_kernel<T, 2, 4, AR, BR>), g, t, 0, s, p); break;
-        case 5: hipLaunchKernelGGL((gemm_flex_kernel<T, 2, 2, AR, BR>), g, t, 0, s, p); break;
-        default: hipLaunchKernelGGL((gemm_flex_kernel<T, 1, 4, AR, BR>), g, t, 0, s, p); break;
+        case 0: hipLaunchKernelGGL((gemm_flex_kernel<T, 8, 8, 2, AR, BR>), g, t, 0, s, p); break;
+        case 1: hipLaunchKernelGGL((gemm_flex_kernel<T, 6, 8, 2, AR, BR>), g, t, 0, s, p); break;
+        case 2: hipLaunchKernelGGL((gemm_flex_kernel<T, 6, 6, 3, AR, BR>), g, t, 0, s, p); break;
+        case 3: hipLaunchKernelGGL((gemm_flex_kernel<T, 6, 4, 3, AR, BR>), g, t, 0, s, p); break;
+        case 4: hipLaunchKernelGGL((gemm_flex_kernel<T, 4, 4, 2, AR, BR>), g, t, 0, s, p); break;
+        case 5: hipLaunchKernelGGL((gemm_flex_kernel<T, 4, 4, 3, AR, BR>), g, t, 0, s, p); break;
+        case 6: hipLaunchKernelGGL((gemm_flex_kernel<T, 2, 4, 2, AR, BR>), g, t, 0, s, p); break;
+        case 7: hipLaunchKernelGGL((gemm_flex_kernel<T, 2, 4, 4, AR, BR>), g, t, 0, s, p); break;
+        case 8: hipLaunchKernelGGL((gemm_flex_kernel<T, 2, 2, 2, AR, BR>), g, t, 0, s, p); break;
+        case 9: hipLaunchKernelGGL((gemm_flex_kernel<T, 2, 2, 3, AR, BR>), g, t, 0, s, p); break;
+        case 10: hipLaunchKernelGGL((gemm_flex_kernel<T, 2, 2, 4, AR, BR>), g, t, 0, s, p); break;
+        default: hipLaunchKernelGGL((gemm_flex_kernel<T, 1, 4, 4, AR, BR>), g, t, 0, s, p); break;
     }
 }
 

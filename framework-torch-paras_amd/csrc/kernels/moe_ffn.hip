@@ -350,7 +350,7 @@ __global__ __launch_bounds__(flex::kThreads, 1) void grouped_gemm_direct_kernel(
     flex::Operand<MI, false> oa;
     aim_rows(oa, wm);
     flex::float4v acc[MI][8];
-    flex::mainloop<T, MI, 8>(oa, ob, static_cast<int>(p.K), a0, a1, b0, b1, acc);
+    flex::mainloop<T, MI, 8, 2>(oa, ob, static_cast<int>(p.K), {a0, a1}, {b0, b1}, acc);
     if constexpr (kSwiglu) {
         // About one value in a thousand leaves the common tier of SwiGLU, and where one lane of the 64 does,
         // the whole wave walks through the fp64 formula: at 128 values a lane that happened eight times a tile

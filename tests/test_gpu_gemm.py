@@ -495,3 +495,26 @@ def test_few_columns_streamed_through_lds(dtype):
         torch.manual_seed(M)
         a, b = torch.randn(M, K).to(dtype), (torch.randn(N, K) / math.sqrt(K)).to(dtype)
         assert_gemm_close(capi.gemm_nt(a.cuda(), b.cuda()), (a.double() @ b.double().t()).to(dtype), dtype)
+
+
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])
+@pytest.mark.parametrize("shape", [(81, 64, 40), (105, 80, 968), (63, 968, 1768), (232, 4136, 960), (72, 752, 2880), (1056, 1016, 232), (40, 2808, 2656),
+                                   (1224, 2560, 136), (1816, 2264, 552), (1816, 2264, 768), (2792, 2216, 584), (57, 112, 2632)])
+def test_gemm_tiles_with_several_stages(shape, dtype):
+    """Tiles whose operands are requested two or three tiles ahead: one tile of contraction to forty, numbers of them that do
+    and do not come in whole turns of the stages, rows and columns cut short, whole and in parts, all three layouts.  Every
+    element against fp64 (bar: the rounding of the result plus 4 sqrt(K) fp32 roundings of a sum of K terms near 1 / sqrt(K))."""
+    M, N, K = shape
+    torch.manual_seed(M + 3 * N + K)
+    a = torch.randn(M, K).to(dtype).cuda()
+    b = (torch.randn(N, K) / math.sqrt(K)).to(dtype).cuda()
+    want = a.double() @ b.double().T
+    half_ulp = {torch.bfloat16: 2.0 ** -8, torch.float16: 2.0 ** -11}[dtype]      # of a value just above a power of two: 8 and 11 significant bits
+    bar = half_ulp * 1.01 * want.abs() + 4 * math.sqrt(K) * 2.0 ** -24 + 2.0 ** -24
+    ar, br = a.T.contiguous().T, b.T.contiguous().T
+    for x, y in ((a, b), (a, br), (ar, br)):
+        if x is ar and M % 8:
+            continue
+        for ws in (False, True):
+            got = capi.gemm(x, y, workspace=ws)
+            assert bool(((got.double() - want).abs() <= bar).all())
