@@ -38,6 +38,7 @@ struct DenseParams {
     long sa, sb, sc, sadd;      // batch strides (elements)
     float alpha, beta;
     double alpha64, beta64;     // the same, for fp64 tensors
+    long rows_each;             // streaming few-row kernel only: weight rows per workgroup
     int  swapped;               // few-row kernels only: a and b have changed places (few output COLUMNS, many rows), so a
                                 // result (row of a, row of b) belongs at c[row of b][row of a], and the addend likewise
 };
@@ -47,13 +48,13 @@ struct DenseParams {
 using stream::Mma16;
 
 template <typename T>
-__device__ __forceinline__ void few_rows_store(const DenseParams& p, std::uint16_t* C, const std::uint16_t* ADD, bool vec_ok, long row, long col, float4_t t) {
+__device__ __forceinline__ void few_rows_store(const DenseParams& p, std::uint16_t* C, const std::uint16_t* ADD, bool vec_ok, long row, long col, long cols, float4_t t) {
     using El = Elem<T>;
     if (row >= p.M) return;
     if (p.swapped) {        // `row` is a column of the caller's result and `col + r` a row of it
 #pragma unroll
         for (int r = 0; r < 4; ++r) {
-            if (col + r >= p.N) continue;
+            if (col + r >= cols) continue;
             float v = p.alpha * t[r];
             if (ADD) v = fmaf(p.beta, El::to_f32(ADD[(col + r) * p.ld_add + row]), v);
             C[(col + r) * p.ldc + row] = El::from_f32(v);
@@ -64,10 +65,10 @@ __device__ __forceinline__ void few_rows_store(const DenseParams& p, std::uint16
 #pragma unroll
     for (int r = 0; r < 4; ++r) {
         float v = p.alpha * t[r];
-        if (ADD && col + r < p.N) v = fmaf(p.beta, El::to_f32(ADD[row * p.ld_add + col + r]), v);
+        if (ADD && col + r < cols) v = fmaf(p.beta, El::to_f32(ADD[row * p.ld_add + col + r]), v);
         o16[r] = El::from_f32(v);
     }
-    if (vec_ok && col + 3 < p.N) {
+    if (vec_ok && col + 3 < cols) {
         u32x2 w2;
         w2[0] = o16[0] | (static_cast<std::uint32_t>(o16[1]) << 16);
         w2[1] = o16[2] | (static_cast<std::uint32_t>(o16[3]) << 16);
@@ -75,7 +76,7 @@ __device__ __forceinline__ void few_rows_store(const DenseParams& p, std::uint16
     } else {
 #pragma unroll
         for (int r = 0; r < 4; ++r)
-            if (col + r < p.N) C[row * p.ldc + col + r] = o16[r];
+            if (col + r < cols) C[row * p.ldc + col + r] = o16[r];
     }
 }
 __device__ __forceinline__ bool few_rows_vec(const DenseParams& p) {
@@ -90,7 +91,7 @@ __global__ __launch_bounds__(stream::kThreads, 4) void stream_gemm_nt_kernel(con
     const long bidx = blockIdx.y;
     const std::uint16_t* A = p.a + bidx * p.sa;
     const int lane = threadIdx.x & 63;
-    const long n0 = static_cast<long>(blockIdx.x) * (16 * NBG);
+    const long n0 = blockIdx.x * p.rows_each, rows = p.N - n0 < p.rows_each ? p.N - n0 : p.rows_each;
     const std::uint16_t* const w[1] = {p.b + bidx * p.sb + n0 * p.ldb};
     std::uint32_t x_off[XQ];
 #pragma unroll
@@ -99,9 +100,9 @@ __global__ __launch_bounds__(stream::kThreads, 4) void stream_gemm_nt_kernel(con
         if (xrow >= p.M) xrow = p.M - 1;                    // clamped rows are computed but never stored
         x_off[q] = static_cast<std::uint32_t>(xrow * p.lda * 2);
     }
-    const long step = static_cast<long>(gridDim.x) * (16 * NBG);
-    const int count = static_cast<int>((p.N - n0 + step - 1) / step);
-    stream::products<T, 1, NBG, XQ>(w, p.ldb, p.N - n0, step, count, p.K, A, ((p.M - 1) * p.lda + p.K) * 2, x_off, lds,
+    constexpr int step = 16 * NBG;
+    const int count = static_cast<int>((rows + step - 1) / step);
+    stream::products<T, 1, NBG, XQ, true>(w, p.ldb, rows, step, count, p.K, A, ((p.M - 1) * p.lda + p.K) * 2, x_off, lds,
                                     [&](int j, const float4_t (&acc)[NBG][MB]) __attribute__((always_inline)) {
         stream::share<NBG, MB>(lds, acc);
         const int blk = stream::wave_id();                  // wave w finishes result block w
@@ -109,7 +110,7 @@ __global__ __launch_bounds__(stream::kThreads, 4) void stream_gemm_nt_kernel(con
             const float4_t t = stream::sum_of<NBG, MB>(lds, blk / MB, blk % MB);
             if (XQ > 1 || (lane & 15) < 8)
                 few_rows_store<T>(p, p.c + bidx * p.sc, p.add ? p.add + bidx * p.sadd : nullptr, few_rows_vec(p), (blk % MB) * 16 + (lane & 15),
-                                  n0 + j * step + (blk / MB) * 16 + 4 * (lane >> 4), t);
+                                  n0 + j * step + (blk / MB) * 16 + 4 * (lane >> 4), n0 + rows, t);
         }
         lds_barrier();                                      // the LDS is free for the next block
     });
@@ -223,28 +224,43 @@ __global__ __launch_bounds__(kSkinnyWaves * 64) void skinny_gemm_nt_kernel(const
 #pragma unroll
             for (int r = 0; r < 4; ++r) t[r] += o[r];
         }
-        few_rows_store<T>(p, C, ADD, vec_ok, (blk % MB) * 16 + r16, n0 + (blk / MB) * 16 + 4 * kg, t);
+        few_rows_store<T>(p, C, ADD, vec_ok, (blk % MB) * 16 + r16, n0 + (blk / MB) * 16 + 4 * kg, p.N, t);
     }
 }
 
-// Two blocks of weight rows per workgroup when that still leaves a workgroup for every CU: every
+// Up to 32 rows: the weight rows are dealt out evenly, one workgroup per CU or two where a CU's share is more than 32 of them,
+// in blocks of 16 rows, or of 32 from a share of 17 on (the activations are read once per block).  The last block of a workgroup is cut
+// short where its share ends: rows past it are requested with an empty extent.  Whole blocks of 16 for everyone left 64 of 256
+// CUs with one block where the others had two (8 x 14336 x 4096 27.0 us, 28 rows each 21.8; 16 x 7168 x 2048 9.3 -> 7.8),
+// and shares below eight rows ask for less than a request holds (8 x 4096 x 4096 16 / 8 / 4 rows each: 9.6 / 11.0 / 17.3 us; 1024
+// rows 6.1 / 5.9 / 5.9).
+// More rows than 32: two blocks of weight rows per workgroup when that still leaves a workgroup for every CU: every
 // activation fragment then feeds two MFMAs, which halves the reads of the activations from L2.
 template <typename T>
-void launch_skinny(const DenseParams& p, long batch, hipStream_t s) {
+void launch_skinny(DenseParams p, long batch, hipStream_t s) {
     const dim3 block(kSkinnyWaves * 64);
     const int mb = static_cast<int>((p.M + 15) / 16);
+    if (mb <= 2) {
+        constexpr long kCus = 256;
+        auto share = [&](long workgroups) { return ((p.N * batch + workgroups - 1) / workgroups + 3) / 4 * 4; };
+        const bool two = share(kCus) > 16;
+        p.rows_each = share(kCus) > 32 ? share(2 * kCus) : (share(kCus) > 8 ? share(kCus) : 8);
+        const dim3 g(static_cast<unsigned>((p.N + p.rows_each - 1) / p.rows_each), static_cast<unsigned>(batch));
+        if (p.M <= 8)     { if (two) hipLaunchKernelGGL((stream_gemm_nt_kernel<T, 2, 1>), g, block, 0, s, p);
+                            else     hipLaunchKernelGGL((stream_gemm_nt_kernel<T, 1, 1>), g, block, 0, s, p); }
+        else if (mb <= 1) { if (two) hipLaunchKernelGGL((stream_gemm_nt_kernel<T, 2, 2>), g, block, 0, s, p);
+                            else     hipLaunchKernelGGL((stream_gemm_nt_kernel<T, 1, 2>), g, block, 0, s, p); }
+        else              { if (two) hipLaunchKernelGGL((stream_gemm_nt_kernel<T, 2, 4>), g, block, 0, s, p);
+                            else     hipLaunchKernelGGL((stream_gemm_nt_kernel<T, 1, 4>), g, block, 0, s, p); }
+        return;
+    }
     const dim3 g1(static_cast<unsigned>((p.N + 15) / 16), static_cast<unsigned>(batch));
     const dim3 g2(static_cast<unsigned>((p.N + 31) / 32), static_cast<unsigned>(batch));
-    const bool two = mb > 1 && static_cast<long>(g2.x) * batch >= 256;
-    const dim3 s1(stream::grid(p.N, 1, batch), static_cast<unsigned>(batch)), s2(stream::grid(p.N, 2, batch), static_cast<unsigned>(batch));
-    if (p.M <= 8)     hipLaunchKernelGGL((stream_gemm_nt_kernel<T, 1, 1>), s1, block, 0, s, p);
-    else if (mb <= 1) hipLaunchKernelGGL((stream_gemm_nt_kernel<T, 1, 2>), s1, block, 0, s, p);
-    else if (mb <= 2) { if (two) hipLaunchKernelGGL((stream_gemm_nt_kernel<T, 2, 4>), s2, block, 0, s, p);
-                        else     hipLaunchKernelGGL((stream_gemm_nt_kernel<T, 1, 4>), s1, block, 0, s, p); }
-    else if (mb <= 4) { if (two) hipLaunchKernelGGL((skinny_gemm_nt_kernel<T, 4, 2>), g2, block, 0, s, p);
-                        else     hipLaunchKernelGGL((skinny_gemm_nt_kernel<T, 4, 1>), g1, block, 0, s, p); }
-    else              { if (two) hipLaunchKernelGGL((skinny_gemm_nt_kernel<T, 8, 2>), g2, block, 0, s, p);
-                        else     hipLaunchKernelGGL((skinny_gemm_nt_kernel<T, 8, 1>), g1, block, 0, s, p); }
+    const bool two = static_cast<long>(g2.x) * batch >= 256;
+    if (mb <= 4) { if (two) hipLaunchKernelGGL((skinny_gemm_nt_kernel<T, 4, 2>), g2, block, 0, s, p);
+                   else     hipLaunchKernelGGL((skinny_gemm_nt_kernel<T, 4, 1>), g1, block, 0, s, p); }
+    else         { if (two) hipLaunchKernelGGL((skinny_gemm_nt_kernel<T, 8, 2>), g2, block, 0, s, p);
+                   else     hipLaunchKernelGGL((skinny_gemm_nt_kernel<T, 8, 1>), g1, block, 0, s, p); }
 }
 
 // ---- few rows with a workspace: the same product with the activations read once per 128 weight

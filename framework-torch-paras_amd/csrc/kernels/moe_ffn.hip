@@ -481,7 +481,7 @@ __device__ __forceinline__ void few_rows(const FfnGemmParams& p, int e, long row
             if constexpr (kSwiglu) p.c[prow * p.N + col] = swiglu_from_acc<T>(g, u);
             else                   p.c[prow * p.N + col] = El::from_f32(g);
         };
-        stream::products<T, NB, 1, XQ>(w, p.K, p.Nw - n0, step, count, p.K, p.a, p.a_bytes, x_off, lds,
+        stream::products<T, NB, 1, XQ, false>(w, p.K, p.Nw - n0, step, count, p.K, p.a, p.a_bytes, x_off, lds,
                                        [&](int j, const float4_t (&acc)[NB][MB]) __attribute__((always_inline)) {
             stream::share<NB, MB>(lds, acc);
             const int m = stream::wave_id();             // wave m finishes row block m

@@ -9,14 +9,13 @@
 // chunks of a row are permuted by its index, so that neither side has bank conflicts).
 //
 // The eight waves of a workgroup share out the contraction in pieces of 64 (128 bytes of a row each, dealt round
-// robin).  P pieces of a wave are under way in registers at any time, 130 to 200 KB per CU where it holds two workgroups (a
-// workgroup takes whole weight rows, so 4096 rows give a CU one and 1024 rows give 64 of the 256 CUs one); a piece
+// robin).  P pieces of a wave are under way in registers at any time, 130 to 200 KB per CU where it holds two workgroups; a piece
 // past the wave's last is requested with an empty extent, which fetches nothing and keeps the number of requests
 // in flight known to the compiler (P is what the loop fits into 128 registers: with one more, spilled registers are
 // reloaded in it through the same counter and it waits for everything: 25.9 -> 30.8 us for 8 x 14336 x 4096).
 //
-// Against feeding the MFMAs straight from memory, bf16: 8 x 1024 x 4096 8.4 -> 6.0 us, 8 x 14336 x 4096 30.0 -> 26.2
-// (4.5 TB/s), 8 x 4096 x 14336 25.1 -> 22.5 (5.2), 13 x 2048 x 2048 6.1 -> 5.2; a mixture-of-experts layer (8 experts, top-2,
+// Against feeding the MFMAs straight from memory, bf16: 8 x 1024 x 4096 8.4 -> 5.9 us, 8 x 14336 x 4096 30.0 -> 21.8
+// (5.4 TB/s), 8 x 4096 x 14336 25.1 -> 22.0 (5.3), 13 x 2048 x 2048 6.1 -> 5.2; a mixture-of-experts layer (8 experts, top-2,
 // H 4096, I 14336) of 1 / 2 / 5 / 16 tokens 160 / 250 / 470 / 557 -> 138 / 192 / 415 / 484 us (5 tokens: 6.1 TB/s).
 #pragma once
 
@@ -47,12 +46,13 @@ constexpr long kMaxExtent = 0xE0000000L;
 constexpr long kMaxLd = 1L << 22;                        // elements between weight rows
 
 // G matrices with the same rows and stride (gate and up), NBG blocks of 16 of their rows, up to 8 XQ activation rows.
-template <int G, int NBG, int XQ> struct Shape {
+// kLone: the only such loop of its kernel, for which the compiler then finds registers for one more piece in two of the forms.
+template <int G, int NBG, int XQ, bool kLone = false> struct Shape {
     static constexpr int kBlocks = G * NBG;              // weight blocks
     static constexpr int kXBlocks = (XQ + 1) / 2;        // activation blocks of 16 rows
     static constexpr int kRequests = 2 * kBlocks + XQ;   // 1 KB each per piece
     static constexpr int kWaveElems = kRequests * 512;   // LDS per wave
-    static constexpr int kP = kRequests <= 3 ? 5 : (kRequests <= 4 ? 4 : (kRequests <= 5 ? 3 : 2));
+    static constexpr int kP = kRequests <= 3 ? 5 : (kRequests <= 4 ? (kLone ? 5 : 4) : (kRequests <= (kLone ? 6 : 5) ? 3 : 2));
     static constexpr int kPartElems = kWaves * kBlocks * kXBlocks * 512;     // the waves' results, laid over the same LDS
     static constexpr int kLdsElems = kWaves * kWaveElems > kPartElems ? kWaves * kWaveElems : kPartElems;
 };
@@ -67,10 +67,10 @@ __device__ __forceinline__ int wave_id() { return __builtin_amdgcn_readfirstlane
 // next one's weights are on their way.  store(j, acc) is called by all waves after the block's last piece, with
 // acc[b][m]: lane (r16 = lane % 16, kg = lane / 16) holds this wave's part for activation row 16 m + r16 and weight rows
 // 4 kg .. + 3 of block b (blocks of w[0] first).
-template <typename T, int G, int NBG, int XQ, typename Store>
+template <typename T, int G, int NBG, int XQ, bool kLone, typename Store>
 __device__ __forceinline__ void products(const std::uint16_t* const (&w)[G], long ld, long rows, long step, int count, long K,
                                          const std::uint16_t* x, long x_bytes, const std::uint32_t (&x_off)[XQ], std::uint16_t* lds, Store&& store) {
-    using S = Shape<G, NBG, XQ>;
+    using S = Shape<G, NBG, XQ, kLone>;
     constexpr int P = S::kP, NB = S::kBlocks, MB = S::kXBlocks;
     const int lane = threadIdx.x & 63, wave = wave_id();
     const int r16 = lane & 15, kg = lane >> 4;
@@ -176,15 +176,6 @@ __device__ __forceinline__ void products(const std::uint16_t* const (&w)[G], lon
         }
         store(j, acc);
     }
-}
-
-// Workgroups for N weight rows in blocks of 16 nbg, `others` such products side by side: no more than are resident (two
-// per CU) if every one can take the same number of blocks or one less.  (14336 x 4096 bf16, 8 rows: 26.2 us, a block each 27.)
-inline unsigned grid(long N, int nbg, long others) {
-    const long blocks = (N + 16 * nbg - 1) / (16 * nbg), slots = 512;
-    long each = (blocks * others + slots - 1) / slots;
-    if (each > blocks) each = blocks;
-    return static_cast<unsigned>((blocks + each - 1) / each);
 }
 
 // The waves' sums meet in LDS; block (b, m) is then sum_of(...) for the wave that takes it, in wave order.

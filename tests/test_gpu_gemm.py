@@ -489,6 +489,22 @@ def test_few_rows_streamed_through_lds(M, dtype):
 
 
 @pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])
+@pytest.mark.parametrize("M", [1, 8, 16, 32])
+def test_few_rows_dealt_out_evenly(M, dtype):
+    """Shares of weight rows per workgroup from 8 to more than 32 rows that are no whole blocks of 16 or 32: every element,
+    and nothing beside the result (rows of the output wider than it)."""
+    for (N, K) in [(2052, 192), (3000, 64), (4100, 576), (7172, 128), (8192, 64), (8196, 64), (14333, 128), (21000, 64)]:
+        torch.manual_seed(M + N)
+        a, b = torch.randn(M, K).to(dtype).cuda(), (torch.randn(N, K) / math.sqrt(K)).to(dtype).cuda()
+        out = torch.full((M + 1, N + 8), 7.0, dtype=dtype, device="cuda")
+        capi.check(capi.lib().paras_gemm_nt(a.data_ptr(), b.data_ptr(), None, out.data_ptr(), M, N, K, K, K, N + 8, 0, 1, 0, 0, 0, 0, 1.0, 0.0,
+                                            capi.DT[dtype], capi._stream()))
+        want = a.double() @ b.double().t()
+        assert bool(((out[:M, :N].double() - want).abs() <= ulp16(want, dtype) * 1.001 + 1e-6 * math.sqrt(K)).all())
+        assert bool((out[M:] == 7.0).all()) and bool((out[:, N:] == 7.0).all())
+
+
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])
 def test_few_columns_streamed_through_lds(dtype):
     """A router's logits: many rows and few columns, the operands in each other's place."""
     for (M, N, K) in [(129, 1, 64), (300, 8, 704), (20000, 9, 128), (515, 32, 2048)]:
