@@ -613,6 +613,7 @@ __global__ __launch_bounds__(256, (D > 128 ? 1 : 2)) void flash_fwd_kernel(const
         mask_load(0, m0);
         finish_scores(0, s_a, mx, m0);
     }
+    lds_reads_done_barrier();              // K tile 2 goes where S(0) was read from
     // One tile of the main loop (`par` = parity of t, a compile-time name for the buffers; two
     // tiles per trip).  The tile's first block also requests the next tile pair (= stage_pair(t + 1)).
     auto tile = [&](int t, auto par) {

@@ -515,6 +515,7 @@ __global__ __launch_bounds__(256, 1) void flash_wide_kernel(const FlashParams p)
                 raise_at[qb] = m_run[qb] + lazy_margin;
             }
         }
+        lds_reads_done_barrier();          // K tile 2 goes where the scores and the fragments above were read from
         for (int t = 0; t < wave_tiles; t += 2) {
             tile(t, Par0{});
             if (t + 1 >= wave_tiles) break;
