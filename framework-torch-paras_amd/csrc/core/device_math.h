@@ -152,13 +152,6 @@ __device__ __forceinline__ void lds_barrier() {
     __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "workgroup", "local");
 }
 
-// The same for a workgroup that has direct-to-LDS loads in flight: the fences above wait for all of those.  This wave's LDS
-// reads are done (lgkmcnt(0)), and no access moves across.
-__device__ __forceinline__ void lds_reads_done_barrier() {
-    __builtin_amdgcn_s_waitcnt(0xC07F);
-    asm volatile("s_barrier" ::: "memory");
-}
-
 // ---- 16-byte global access ---------------------------------------------------
 __device__ __forceinline__ u32x4 load16(const void* p) {
     return *reinterpret_cast<const u32x4*>(p);

@@ -67,7 +67,8 @@ bool plan_padded(const paras_sdpa_args& a, PaddedPlan* plan) {
     pl.inner.q = fake; pl.inner.k = fake; pl.inner.v = fake; pl.inner.out = fake;
     size_t inner_ws = 0;
     if (decode_supported(pl.inner)) inner_ws = decode_workspace(pl.inner);
-    else if (!flash_supported(pl.inner)) return false;
+    else if (flash_supported(pl.inner)) inner_ws = flash_workspace(pl.inner);
+    else return false;
     pl.total = off + up256(inner_ws);
     if (plan) *plan = pl;
     return true;
@@ -103,7 +104,7 @@ int launch_padded(const paras_sdpa_args& a, void* workspace, void* stream, hipSt
     if ((rc = copy_in(a.k, a.k_strides, const_cast<void*>(in.k), a.Hkv, a.Lk)) != PARAS_OK) return rc;
     if ((rc = copy_in(a.v, a.v_strides, const_cast<void*>(in.v), a.Hkv, a.Lk)) != PARAS_OK) return rc;
     if (decode_supported(in)) rc = launch_decode(in, ws + pl.inner_off, s);
-    else                      rc = launch_flash(in, s);
+    else                      rc = launch_flash(in, ws + pl.inner_off, s);
     if (rc != PARAS_OK) return rc;
     const int64_t sizes[4] = {a.B, a.Hq, a.Lq, a.D}, ss[4] = {a.Hq * a.Lq * Dp, a.Lq * Dp, Dp, 1},
                   ds[4] = {a.Hq * a.Lq * a.D, a.Lq * a.D, a.D, 1};
@@ -132,6 +133,7 @@ size_t paras_sdpa_workspace(const paras_sdpa_args* args) {
     using namespace paras;
     if (validate(args) != PARAS_OK || empty_output(*args)) return 0;
     switch (choose(*args)) {
+        case SdpaKernel::Flash:   return flash_workspace(*args);
         case SdpaKernel::Decode:  return decode_workspace(*args);
         case SdpaKernel::Generic: return generic_workspace(*args);
         case SdpaKernel::Composed: return composed_workspace(*args);
@@ -162,7 +164,7 @@ int paras_sdpa_fwd(const paras_sdpa_args* args, void* workspace, void* stream) {
         return paras_fill_strided(a.out, 1, &n, &one, esz, 0, stream);
     }
     switch (choose(a)) {
-        case SdpaKernel::Flash: return launch_flash(a, s);
+        case SdpaKernel::Flash: return launch_flash(a, workspace, s);
         case SdpaKernel::Weights: return launch_weights(a, s);
         case SdpaKernel::Padded: return launch_padded(a, workspace, stream, s);
         case SdpaKernel::Composed: return launch_composed(a, workspace, stream, s);

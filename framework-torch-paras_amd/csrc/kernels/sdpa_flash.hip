@@ -44,7 +44,7 @@
 //
 // so the matrix pipe has independent work in flight under the softmax VALU
 // work of the same wave.  K is staged half a tile ahead of V: K tile u holds
-// keys [64u-32, 64u+32), so the two blocks whose scores are computed during V
+// keys [64u-32, 64u+32) (tile 0 only 0 .. 31, in a buffer of its own), so the two blocks whose scores are computed during V
 // tile t (blocks 2t+1, 2t+2) both live in K tile t+1, and K and V need only two
 // LDS buffers each with a single barrier per tile.  The operand fragments run
 // through a register ring that carries across the two blocks of a tile, and a
@@ -65,6 +65,9 @@
 // -inf and contribute zeros; a query with no visible key at all ends as 0/0 = NaN,
 // like the reference's softmax.
 //
+// A problem with fewer query tiles than CUs shares its keys out as well: two halves per workgroup or parts of the keys in
+// workgroups of their own (plan_shares).
+//
 // v_mfma_f32_32x32x16_{bf16,f16}: 32 MFMAs per wave per 64-key tile at D=128.
 #include <hip/hip_runtime.h>
 
@@ -84,9 +87,47 @@ using namespace flash;
 
 constexpr int kBM = 128;   // queries per workgroup: 4 waves x 32
 
+// Tiles of keys that the queries of a tile see.
+template <bool kCausal>
+__device__ __forceinline__ int tiles_of(const FlashParams& p, int qblock) {
+    const int keys = kCausal ? min(min(qblock * kBM + kBM, p.Lq), p.Lk) : p.Lk;
+    return (keys + kBN - 1) / kBN;
+}
+
+// The weight of a share of the keys whose maximum is m beside one with M >= m.  A share in which the query saw no key counts
+// with weight zero (and hands on a NaN that its values left there, as 0 x NaN does in the product).
+__device__ __forceinline__ float weight_of(float m, float M, float scale_log2) {
+    return m == -INFINITY ? 0.f : __builtin_amdgcn_exp2f((m - M) * scale_log2);
+}
+
+// One query's outputs from its lanes (half lh of the lanes holds, of each 32 columns, 8 g + 4 lh .. + 3) divided by the sum
+// of its weights, and the logarithm of that sum where it is asked for; columns d0 .. d0 + 32 DBLK.
+template <typename T, int D, int DBLK>
+__device__ __forceinline__ void store_rows(const FlashParams& p, int b, int hq, int my_q, int lh, const float16_t (&oacc)[DBLK], float m, float l, int d0 = 0) {
+    if (my_q >= p.Lq) return;
+    const float inv_l = 1.0f / l;
+    std::uint16_t* op = p.out + ((static_cast<long>(b) * p.Hq + hq) * p.Lq + my_q) * D + d0;
+#pragma unroll
+    for (int db = 0; db < DBLK; ++db)
+#pragma unroll
+        for (int g = 0; g < 4; ++g) {
+            const int d = db * 32 + g * 8 + 4 * lh;
+            u32x2 w;
+            w[0] = Mma<T>::pack2(oacc[db][4 * g + 0] * inv_l, oacc[db][4 * g + 1] * inv_l);
+            w[1] = Mma<T>::pack2(oacc[db][4 * g + 2] * inv_l, oacc[db][4 * g + 3] * inv_l);
+            *reinterpret_cast<u32x2*>(op + d) = w;
+        }
+    if (p.lse != nullptr && lh == 0) p.lse[(static_cast<long>(b) * p.Hq + hq) * p.Lq + my_q] = m * p.scale + logf(l);
+}
+
 // kMask: 0 none, 1 bytes (nonzero = attend), 2 additive values of type T.
-template <typename T, int D, bool kCausal, int kMask>
-__global__ __launch_bounds__(256, (D > 128 ? 1 : 2)) void flash_fwd_kernel(const FlashParams p) {
+// kHalves = 2: a workgroup is eight waves, four for the first half of the keys and four for the second, each half with tiles of its
+// own; the second half's unnormalised outputs, maxima and sums reach the first through LDS at the end.
+// kParts: the keys of a query tile are shared out to several workgroups, p.part_tiles tiles each, which leave their
+// unnormalised outputs, maxima and sums to flash_combine_kernel.
+// A wave sees its keys as keys 0 .. Lk - 1.
+template <typename T, int D, bool kCausal, int kMask, bool kParts, int kHalves>
+__global__ __launch_bounds__(256 * kHalves, (D > 128 || kHalves > 1 ? 1 : 2)) void flash_fwd_kernel(const FlashParams p) {
     static_assert(!(kCausal && kMask != 0), "a mask and the causal rule are mutually exclusive");
     // 32-query blocks per wave.  The code is written for any QB; 2 halves the LDS operand
     // traffic per query but needs one wave per SIMD and measured 30 % slower (nothing hides
@@ -103,34 +144,41 @@ __global__ __launch_bounds__(256, (D > 128 ? 1 : 2)) void flash_fwd_kernel(const
     auto ksw = [](int row) { return D >= 128 ? (row & 15) : ((row >> 1) & 7); };
     auto vsw = [](int row) { return D >= 128 ? ((row & 3) << 2) : (((row >> 1) & 1) << 2); };
 
-    // LDS: two tiles each of K and V (4 x 16 KiB per workgroup at D = 128, two workgroups per
+    // LDS: two tiles each of K and V and the first half tile of K (72 KiB per workgroup at D = 128, two workgroups per
     // CU).  They are four separate arrays on purpose: the compiler makes an LDS read wait for
     // every direct-to-LDS load in flight unless it can prove from the variables involved that the
     // two do not overlap, and the point of the double buffer is to read one tile while the next
     // one streams in.  The main loop therefore names its buffers at compile time (`Par`), the
     // rarely taken paths pick them at run time (`AnyPar`) and accept the wait.
-    __shared__ __attribute__((aligned(1024))) std::uint16_t k_lds0[kBN * D];
-    __shared__ __attribute__((aligned(1024))) std::uint16_t k_lds1[kBN * D];
-    __shared__ __attribute__((aligned(1024))) std::uint16_t v_lds0[kBN * D];
-    __shared__ __attribute__((aligned(1024))) std::uint16_t v_lds1[kBN * D];
+    __shared__ __attribute__((aligned(1024))) std::uint16_t k_lds0[kHalves * kBN * D];
+    __shared__ __attribute__((aligned(1024))) std::uint16_t k_lds1[kHalves * kBN * D];
+    __shared__ __attribute__((aligned(1024))) std::uint16_t v_lds0[kHalves * kBN * D];
+    __shared__ __attribute__((aligned(1024))) std::uint16_t v_lds1[kHalves * kBN * D];
+    // Keys 0..31, whose scores come before the loop.  (Not the upper half of K tile 0: K tile 2 is requested into that buffer
+    // while another wave may still read them, and a barrier in between costs a problem of two tiles 5 %.)
+    __shared__ __attribute__((aligned(1024))) std::uint16_t k_first[kHalves * 32 * D];
     using Par0 = std::integral_constant<int, 0>;
     using Par1 = std::integral_constant<int, 1>;
     struct AnyPar { int value; };
+    const int tid = threadIdx.x, lane = tid & 63;
+    const int half = kHalves == 1 ? 0 : __builtin_amdgcn_readfirstlane(tid >> 8);
+    const int wave = __builtin_amdgcn_readfirstlane(kHalves == 1 ? tid >> 6 : (tid >> 6) & 3);      // within its half
+    const int own = half * kBN * D;            // where this half's tiles are in the arrays
     // buffer of tile index parity `par`; `flip` selects the other one
     auto kbuf = [&](auto par, bool flip) -> std::uint16_t* {
-        if constexpr (std::is_same<decltype(par), AnyPar>::value) return ((par.value ^ (flip ? 1 : 0)) & 1) ? k_lds1 : k_lds0;
-        else return (decltype(par)::value != 0) != flip ? k_lds1 : k_lds0;
+        if constexpr (std::is_same<decltype(par), AnyPar>::value) return (((par.value ^ (flip ? 1 : 0)) & 1) ? k_lds1 : k_lds0) + own;
+        else return ((decltype(par)::value != 0) != flip ? k_lds1 : k_lds0) + own;
     };
     auto vbuf = [&](auto par, bool flip) -> std::uint16_t* {
-        if constexpr (std::is_same<decltype(par), AnyPar>::value) return ((par.value ^ (flip ? 1 : 0)) & 1) ? v_lds1 : v_lds0;
-        else return (decltype(par)::value != 0) != flip ? v_lds1 : v_lds0;
+        if constexpr (std::is_same<decltype(par), AnyPar>::value) return (((par.value ^ (flip ? 1 : 0)) & 1) ? v_lds1 : v_lds0) + own;
+        else return ((decltype(par)::value != 0) != flip ? v_lds1 : v_lds0) + own;
     };
 
     const int nq = p.n_qblocks;
     const int BH = p.B * p.Hq;
     int bh, qi;
     {
-        const int idx = blockIdx.x;
+        const int idx = kParts ? blockIdx.x % (BH * nq) : blockIdx.x;
         if (BH % 16 == 0) {
             const int xcd = idx & 7, j = idx >> 3;
             const int g = j / (2 * nq), r = j % (2 * nq);
@@ -140,19 +188,37 @@ __global__ __launch_bounds__(256, (D > 128 ? 1 : 2)) void flash_fwd_kernel(const
             const int xcd = idx & 7, j = idx >> 3;
             bh = (j / nq) * 8 + xcd;
             qi = j % nq;
+        } else if (kCausal) {        // the longest tiles of all heads first (B10 H1 S5121 D128: 102 -> 86 us; head by head the last heads' longest start late)
+            bh = idx % BH;
+            qi = idx / BH;
         } else {
             bh = idx / nq;
             qi = idx % nq;
         }
     }
     const int qblock = nq - 1 - qi;
+    int n_tiles = tiles_of<kCausal>(p, qblock);
+    int first = 0;                             // this wave's first tile of keys
+    const bool whole = !kParts || n_tiles <= p.part_tiles;
+    const int part = kParts ? static_cast<int>(blockIdx.x) / (BH * nq) : 0;
+    if constexpr (kParts) {
+        first = part * p.part_tiles;
+        if (first >= n_tiles) return;
+        n_tiles = min(n_tiles - first, p.part_tiles);
+    }
+    const int turns = kHalves == 1 ? n_tiles : (n_tiles + 1) / 2;       // tiles between the workgroup's barriers
+    if constexpr (kHalves == 2) {
+        first += half * turns;
+        n_tiles = half == 0 ? turns : n_tiles - turns;                  // (the second half of a single tile has none)
+    }
+    const int key0 = first * kBN;
+    const int Lk = kParts || kHalves == 2 ? min(p.Lk - key0, n_tiles * kBN) : p.Lk;
     const int b = bh / p.Hq, hq = bh % p.Hq;
     const int hkv = hq / (p.Hq / p.Hkv);
 
-    const int tid = threadIdx.x, lane = tid & 63;
-    const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
     const int lq = lane & 31, lh = lane >> 5;
     const int q0 = qblock * kBM + wave * WQ;   // first query of this wave; query block qb starts at q0 + 32 qb
+    const int q0k = q0 - key0;                 // the same, counted from this workgroup's first key (the causal rule)
 
     i16x8 qreg[QB][KSTEPS];
 #pragma unroll
@@ -164,19 +230,14 @@ __global__ __launch_bounds__(256, (D > 128 ? 1 : 2)) void flash_fwd_kernel(const
         for (int ks = 0; ks < KSTEPS; ++ks) qreg[qb][ks] = *reinterpret_cast<const i16x8*>(qp + ks * 16 + lh * 8);
     }
 
-    const std::uint16_t* kbase = p.k + b * p.ks_b + hkv * p.ks_h;
-    const std::uint16_t* vbase = p.v + b * p.vs_b + hkv * p.vs_h;
-
-    int n_tiles = (p.Lk + kBN - 1) / kBN;
-    if (kCausal) {
-        const int last_q = min(qblock * kBM + kBM, p.Lq) - 1;
-        n_tiles = (min(last_q + 1, p.Lk) + kBN - 1) / kBN;
-    }
-    const int wave_tiles = kCausal ? min(n_tiles, (q0 + WQ - 1) / kBN + 1) : n_tiles;
+    const std::uint16_t* kbase = p.k + b * p.ks_b + hkv * p.ks_h + static_cast<long>(key0) * p.ks_l;
+    const std::uint16_t* vbase = p.v + b * p.vs_b + hkv * p.vs_h + static_cast<long>(key0) * p.vs_l;
+    // (keys may lie wholly beyond a wave's last query: no tiles, and zeros with a maximum of -inf)
+    const int wave_tiles = !kCausal ? n_tiles : ((kParts || kHalves == 2) && q0k + WQ - 1 < 0 ? 0 : min(n_tiles, (q0k + WQ - 1) / kBN + 1));
 
     // ---- staging: 64 LDS rows <- global rows first .. first+63, straight from memory into LDS
     // with buffer loads.  The buffer descriptor spans rows [0, Lk) of this (batch, kv head), so
-    // rows outside it (before the first key in K tile 0, past the end of K in the last tiles)
+    // rows outside it (past the end of K in the last tiles)
     // arrive as zeros without a branch: the hardware range-checks every dword of every lane.
     const int srow = wave * RPI + lane / CHUNKS;
     const int slot = lane % CHUNKS;
@@ -190,7 +251,7 @@ __global__ __launch_bounds__(256, (D > 128 ? 1 : 2)) void flash_fwd_kernel(const
     static_assert((RPI * NW) % 16 == 0 || (RPI * NW == 8 && D == 256), "the staging swizzle assumes whole groups of 16 (or 8) rows per request");
     typedef __attribute__((address_space(3))) void* lptr_t;
     auto make_rsrc = [&](const std::uint16_t* base, int row_bytes) {
-        const int bytes = (p.Lk - 1) * row_bytes + D * 2;           // < 2^31: checked by flash_supported
+        const int bytes = kHalves == 2 && Lk <= 0 ? 0 : (Lk - 1) * row_bytes + D * 2;           // < 2^31: checked by flash_supported
         return __builtin_amdgcn_make_buffer_rsrc(const_cast<std::uint16_t*>(base), 0, bytes, 0x00020000);
     };
     const __amdgpu_buffer_rsrc_t k_rsrc = make_rsrc(kbase, k_row_bytes);
@@ -233,7 +294,8 @@ __global__ __launch_bounds__(256, (D > 128 ? 1 : 2)) void flash_fwd_kernel(const
             for (int r = 0; r < 16; ++r) oacc[qb][i][r] = 0.f;
     }
 
-    stage_rows(k_rsrc, OfK{}, k_row_bytes, -32, k_lds0);   // K tile 0: keys 0..31 in its upper half
+#pragma unroll
+    for (int i = 0; i < NI / 2; ++i) stage_one(k_rsrc, OfK{}, k_row_bytes, 0, k_first + half * 32 * D, i);
     stage_pair(0, Par0{});
     publish();
 
@@ -249,10 +311,10 @@ __global__ __launch_bounds__(256, (D > 128 ? 1 : 2)) void flash_fwd_kernel(const
     }
     const float lazy_margin = 8.0f / p.scale_log2;
 
-    auto needs_mask = [&](int j, int qb) { return (kCausal && j * 32 + 31 > q0 + 32 * qb) || j * 32 + 32 > p.Lk; };
+    auto needs_mask = [&](int j, int qb) { return (kCausal && j * 32 + 31 > q0k + 32 * qb) || j * 32 + 32 > Lk; };
     auto apply_mask = [&](int j, int qb, float16_t& sc) {
-        const int my_q = q0 + 32 * qb + lq;
-        const int last_visible = kCausal ? min(my_q, p.Lk - 1) : p.Lk - 1;
+        const int my_q = q0k + 32 * qb + lq;
+        const int last_visible = kCausal ? min(my_q, Lk - 1) : Lk - 1;
         const int rel = last_visible - j * 32 - 4 * lh;
 #pragma unroll
         for (int r = 0; r < 16; ++r)
@@ -266,7 +328,7 @@ __global__ __launch_bounds__(256, (D > 128 ? 1 : 2)) void flash_fwd_kernel(const
     if constexpr (kMask != 0) {
         const int my_q = q0 + lq;
         const long qrow = my_q < p.Lq ? my_q : p.Lq - 1;
-        mrow = p.mask + (static_cast<long>(b) * p.ms_b + static_cast<long>(hq) * p.ms_h + qrow * p.ms_q) * (kMask == 1 ? 1 : 2);
+        mrow = p.mask + (static_cast<long>(b) * p.ms_b + static_cast<long>(hq) * p.ms_h + qrow * p.ms_q + key0 * p.ms_k) * (kMask == 1 ? 1 : 2);
     }
     // A mask that is contiguous along the keys, with Lk >= 4: a run that hangs over the end of the
     // row is read from the row's last four elements and shifted down, so no load leaves the row and
@@ -279,8 +341,8 @@ __global__ __launch_bounds__(256, (D > 128 ? 1 : 2)) void flash_fwd_kernel(const
     // the block's 32 (bool) or 64 (additive: two pieces) bytes of its query's row: half lh holds keys
     // 16 lh .. 16 lh + 15 and needs keys 8 g + 4 lh .. + 3, so the two halves of a query swap every
     // other run when the mask is applied (v_permlane32_swap: lanes l and l + 32).
-    const bool mask_runs = p.ms_k == 1 && p.Lk >= 4;       // uniform
-    auto mask_whole_block = [&](int j) { return mask_runs && j * 32 + 32 <= p.Lk; };      // uniform
+    const bool mask_runs = p.ms_k == 1 && Lk >= 4;       // uniform
+    auto mask_whole_block = [&](int j) { return mask_runs && j * 32 + 32 <= Lk; };      // uniform
     auto mask_load = [&](int j, std::uint32_t (&mr)[MREGS]) {
         if constexpr (kMask != 0) {
             typedef std::uint32_t u32_any __attribute__((aligned(1)));
@@ -303,7 +365,7 @@ __global__ __launch_bounds__(256, (D > 128 ? 1 : 2)) void flash_fwd_kernel(const
                     std::uint32_t e[4];
 #pragma unroll
                     for (int i = 0; i < 4; ++i) {
-                        const int key = min(j * 32 + 8 * g + 4 * lh + i, p.Lk - 1);   // (keys past the end: any value, the end-of-K rule masks them)
+                        const int key = min(j * 32 + 8 * g + 4 * lh + i, Lk - 1);   // (keys past the end: any value, the end-of-K rule masks them)
                         const unsigned char* at = mrow + static_cast<long>(key) * p.ms_k * ES;
                         if constexpr (kMask == 1) e[i] = *at;
                         else                      e[i] = *reinterpret_cast<const std::uint16_t*>(at);
@@ -320,7 +382,7 @@ __global__ __launch_bounds__(256, (D > 128 ? 1 : 2)) void flash_fwd_kernel(const
 #pragma unroll
             for (int g = 0; g < 4; ++g) {
                 const int key = j * 32 + 8 * g + 4 * lh;
-                const int at = min(key, p.Lk - 4);
+                const int at = min(key, Lk - 4);
                 const unsigned sh = static_cast<unsigned>(key - at);          // 0 unless the run hangs over
                 if constexpr (kMask == 1) {
                     const std::uint32_t w = *reinterpret_cast<const u32_any*>(mrow + at);
@@ -598,7 +660,7 @@ __global__ __launch_bounds__(256, (D > 128 ? 1 : 2)) void flash_fwd_kernel(const
 
     float16_t s_a[QB], s_b[QB];
     if (wave_tiles > 0) {
-        // S(0): keys 0..31 = rows 32..63 of K tile 0
+        // S(0): keys 0..31
         float mx[QB];
 #pragma unroll
         for (int qb = 0; qb < QB; ++qb) {
@@ -606,14 +668,13 @@ __global__ __launch_bounds__(256, (D > 128 ? 1 : 2)) void flash_fwd_kernel(const
             for (int r = 0; r < 16; ++r) s_a[qb][r] = 0.f;
 #pragma unroll
             for (int ks = 0; ks < KSTEPS; ++ks)
-                s_a[qb] = Mma<T>::run(*reinterpret_cast<const i16x8*>(&k_lds0[32 * D + k_rd[ks]]), qreg[qb][ks], s_a[qb]);
+                s_a[qb] = Mma<T>::run(*reinterpret_cast<const i16x8*>(&k_first[half * 32 * D + k_rd[ks]]), qreg[qb][ks], s_a[qb]);
             mx[qb] = lane_max(s_a[qb]);
         }
         std::uint32_t m0[MREGS];
         mask_load(0, m0);
         finish_scores(0, s_a, mx, m0);
     }
-    lds_reads_done_barrier();              // K tile 2 goes where S(0) was read from
     // One tile of the main loop (`par` = parity of t, a compile-time name for the buffers; two
     // tiles per trip).  The tile's first block also requests the next tile pair (= stage_pair(t + 1)).
     auto tile = [&](int t, auto par) {
@@ -639,7 +700,7 @@ __global__ __launch_bounds__(256, (D > 128 ? 1 : 2)) void flash_fwd_kernel(const
         // The tile's second block contributes nothing when it starts past the end of K or, for a
         // causal wave, past the wave's last query (every other wave's diagonal tile).
         const int second0 = (2 * t + 1) * 32;
-        if (second0 >= p.Lk || (kCausal && second0 > q0 + WQ - 1)) {
+        if (second0 >= Lk || (kCausal && second0 > q0k + WQ - 1)) {
             first_fetches(2 * t, VFirst{}, par);
             block(2 * t, s_a, s_b, No{}, NoTail{}, par, No{});
         } else {
@@ -649,43 +710,128 @@ __global__ __launch_bounds__(256, (D > 128 ? 1 : 2)) void flash_fwd_kernel(const
         }
         publish();
     }
-    for (int t = wave_tiles; t < n_tiles; ++t) {           // done early (causal): keep staging for the other waves
+    for (int t = wave_tiles; t < turns; ++t) {             // done early (causal): keep staging for the other waves
         if (t + 1 < n_tiles) stage_pair(t + 1, AnyPar{t + 1});
         publish();
     }
 
+    float l_tot[QB];
 #pragma unroll
-    for (int qb = 0; qb < QB; ++qb) {
-        const int my_q = q0 + 32 * qb + lq;
-        const float l_tot = half_swap_sum(l_run[qb]);
-        const float inv_l = 1.0f / l_tot;
-        if (my_q < p.Lq) {
-            std::uint16_t* op = p.out + ((static_cast<long>(b) * p.Hq + hq) * p.Lq + my_q) * D;
+    for (int qb = 0; qb < QB; ++qb) l_tot[qb] = half_swap_sum(l_run[qb]);
+    if constexpr (kHalves == 2) {
+        static_assert(QB == 1 && kHalves * kBN * D * 2 >= DBLK * 4 * 64 * 16, "a wave's outputs fit one of the arrays, whose tiles are done with");
+        __shared__ float ml[NW][2][64];
+        std::uint16_t* const mine = wave == 0 ? k_lds0 : (wave == 1 ? k_lds1 : (wave == 2 ? v_lds0 : v_lds1));
+        float4_t* const po = reinterpret_cast<float4_t*>(mine) + lane;
+        if (half == 1) {
 #pragma unroll
-            for (int db = 0; db < DBLK; ++db)
+            for (int i = 0; i < DBLK * 4; ++i)
+                po[i * 64] = float4_t{oacc[0][i / 4][4 * (i % 4)], oacc[0][i / 4][4 * (i % 4) + 1], oacc[0][i / 4][4 * (i % 4) + 2], oacc[0][i / 4][4 * (i % 4) + 3]};
+            ml[wave][0][lane] = m_run[0];
+            ml[wave][1][lane] = l_tot[0];
+        }
+        __syncthreads();
+        if (half == 1) return;
+        const float m1 = ml[wave][0][lane], l1 = ml[wave][1][lane], M = fmaxf(m_run[0], m1);
+        const float f0 = weight_of(m_run[0], M, p.scale_log2), f1 = weight_of(m1, M, p.scale_log2);
 #pragma unroll
-                for (int g = 0; g < 4; ++g) {
-                    const int d = db * 32 + g * 8 + 4 * lh;
-                    u32x2 w;
-                    w[0] = Mma<T>::pack2(oacc[qb][db][4 * g + 0] * inv_l, oacc[qb][db][4 * g + 1] * inv_l);
-                    w[1] = Mma<T>::pack2(oacc[qb][db][4 * g + 2] * inv_l, oacc[qb][db][4 * g + 3] * inv_l);
-                    *reinterpret_cast<u32x2*>(op + d) = w;
-                }
-            if (p.lse != nullptr && lh == 0)
-                p.lse[(static_cast<long>(b) * p.Hq + hq) * p.Lq + my_q] = m_run[qb] * p.scale + logf(l_tot);
+        for (int i = 0; i < DBLK * 4; ++i) {
+            const float4_t v = po[i * 64];
+#pragma unroll
+            for (int r = 0; r < 4; ++r) oacc[0][i / 4][4 * (i % 4) + r] = fmaf(f1, v[r], f0 * oacc[0][i / 4][4 * (i % 4) + r]);
+        }
+        l_tot[0] = fmaf(f1, l1, f0 * l_tot[0]);
+        m_run[0] = M;
+    }
+    if constexpr (kParts) {
+        if (!whole) {
+            static_assert(QB == 1, "one query block per wave in a slot");
+            const long slot = (static_cast<long>(bh) * nq + qblock) * p.n_parts + part;
+            float4_t* po = reinterpret_cast<float4_t*>(p.part_o) + (slot * NW + wave) * (DBLK * 4 * 64) + lane;
+#pragma unroll
+            for (int i = 0; i < DBLK * 4; ++i)
+                po[i * 64] = float4_t{oacc[0][i / 4][4 * (i % 4)], oacc[0][i / 4][4 * (i % 4) + 1], oacc[0][i / 4][4 * (i % 4) + 2], oacc[0][i / 4][4 * (i % 4) + 3]};
+            float* ml = p.part_ml + (slot * NW + wave) * 64;
+            ml[lane] = lh == 0 ? m_run[0] : l_tot[0];
+            return;
         }
     }
+#pragma unroll
+    for (int qb = 0; qb < QB; ++qb) store_rows<T, D, DBLK>(p, b, hq, q0 + 32 * qb + lq, lh, oacc[qb], m_run[qb], l_tot[qb]);
+}
+
+// The parts of a query tile brought together: O = sum of exp(m_s - M) O_s over sum of exp(m_s - M) l_s, in part order.
+// A workgroup takes 32 columns of a tile's 128 queries, lane for lane as the parts were stored.
+template <typename T, int D, bool kCausal>
+__global__ __launch_bounds__(256) void flash_combine_kernel(const FlashParams p) {
+    constexpr int DBLK = D / 32, NW = 4, kAhead = 4;
+    const int tile = blockIdx.x / DBLK, db = blockIdx.x % DBLK;
+    const int bh = tile / p.n_qblocks, qblock = tile % p.n_qblocks;
+    const int parts = (tiles_of<kCausal>(p, qblock) + p.part_tiles - 1) / p.part_tiles;
+    if (parts <= 1) return;
+    const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6, lq = lane & 31, lh = lane >> 5;
+    const long slot = static_cast<long>(tile) * p.n_parts;
+    const float* ml = p.part_ml + (slot * NW + wave) * 64;
+    const float4_t* po = reinterpret_cast<const float4_t*>(p.part_o) + (slot * NW + wave) * (DBLK * 4 * 64) + db * 256 + lane;
+    float M = -INFINITY;
+#pragma unroll 8
+    for (int s = 0; s < parts; ++s) M = fmaxf(M, ml[s * (NW * 64) + lq]);
+    float L = 0.f;
+    float16_t o;
+#pragma unroll
+    for (int r = 0; r < 16; ++r) o[r] = 0.f;
+    for (int s0 = 0; s0 < parts; s0 += kAhead) {        // four parts in flight
+        float4_t v[kAhead][4];
+        float m[kAhead], l[kAhead];
+#pragma unroll
+        for (int u = 0; u < kAhead; ++u) {
+            const int s = min(s0 + u, parts - 1);
+            m[u] = ml[s * (NW * 64) + lq];
+            l[u] = ml[s * (NW * 64) + 32 + lq];
+#pragma unroll
+            for (int g = 0; g < 4; ++g) v[u][g] = po[static_cast<long>(s) * (NW * DBLK * 4 * 64) + g * 64];
+        }
+#pragma unroll
+        for (int u = 0; u < kAhead; ++u) {
+            if (s0 + u >= parts) break;
+            const float f = weight_of(m[u], M, p.scale_log2);
+            L = fmaf(f, l[u], L);
+#pragma unroll
+            for (int g = 0; g < 4; ++g)
+#pragma unroll
+                for (int r = 0; r < 4; ++r) o[4 * g + r] = fmaf(f, v[u][g][r], o[4 * g + r]);
+        }
+    }
+    const int b = bh / p.Hq, hq = bh % p.Hq;
+    const float16_t oacc[1] = {o};
+    FlashParams q = p;
+    if (db != 0) q.lse = nullptr;                       // (one workgroup of the tile writes it)
+    store_rows<T, D, 1>(q, b, hq, qblock * kBM + wave * 32 + lq, lh, oacc, M, L, db * 32);
+}
+
+template <typename T, int D, bool kParts, int kHalves>
+void launch_mask(const FlashParams& p, bool causal, int mask_kind, hipStream_t s) {
+    const dim3 grid(static_cast<unsigned>(static_cast<long>(p.B) * p.Hq * p.n_qblocks * (kParts ? p.n_parts : 1))), wg(256 * kHalves);
+    if (causal)              hipLaunchKernelGGL((flash_fwd_kernel<T, D, true, 0, kParts, kHalves>), grid, wg, 0, s, p);
+    else if (mask_kind == 1) hipLaunchKernelGGL((flash_fwd_kernel<T, D, false, 1, kParts, kHalves>), grid, wg, 0, s, p);
+    else if (mask_kind == 2) hipLaunchKernelGGL((flash_fwd_kernel<T, D, false, 2, kParts, kHalves>), grid, wg, 0, s, p);
+    else                     hipLaunchKernelGGL((flash_fwd_kernel<T, D, false, 0, kParts, kHalves>), grid, wg, 0, s, p);
 }
 
 template <typename T, int D>
-int launch_t(FlashParams p, bool causal, int mask_kind, hipStream_t s) {
+int launch_t(FlashParams p, bool causal, int mask_kind, bool halves, hipStream_t s) {
+    constexpr int kHalves = D > 128 ? 1 : 2;           // (the tiles of two halves of 256-element heads do not fit LDS)
     p.n_qblocks = (p.Lq + kBM - 1) / kBM;
-    const long blocks = static_cast<long>(p.B) * p.Hq * p.n_qblocks;
-    const dim3 grid(static_cast<unsigned>(blocks)), wg(256);
-    if (causal)              hipLaunchKernelGGL((flash_fwd_kernel<T, D, true, 0>), grid, wg, 0, s, p);
-    else if (mask_kind == 1) hipLaunchKernelGGL((flash_fwd_kernel<T, D, false, 1>), grid, wg, 0, s, p);
-    else if (mask_kind == 2) hipLaunchKernelGGL((flash_fwd_kernel<T, D, false, 2>), grid, wg, 0, s, p);
-    else                     hipLaunchKernelGGL((flash_fwd_kernel<T, D, false, 0>), grid, wg, 0, s, p);
+    if (p.n_parts <= 1) {
+        if (halves) launch_mask<T, D, false, kHalves>(p, causal, mask_kind, s);
+        else        launch_mask<T, D, false, 1>(p, causal, mask_kind, s);
+    } else {
+        launch_mask<T, D, true, 1>(p, causal, mask_kind, s);
+        PARAS_HIP_TRY(hipGetLastError());
+        const dim3 grid(static_cast<unsigned>(static_cast<long>(p.B) * p.Hq * p.n_qblocks * (D / 32)));
+        if (causal) hipLaunchKernelGGL((flash_combine_kernel<T, D, true>), grid, dim3(256), 0, s, p);
+        else        hipLaunchKernelGGL((flash_combine_kernel<T, D, false>), grid, dim3(256), 0, s, p);
+    }
     PARAS_HIP_TRY(hipGetLastError());
     return PARAS_OK;
 }
@@ -717,12 +863,59 @@ bool flash_supported(const paras_sdpa_args& a) {
     return true;
 }
 
+namespace {
+
+// How the keys of a problem with few query tiles are shared out (launch_flash).  A workgroup of four waves uses a CU's arithmetic
+// to the full, so nothing is gained where every CU has one; the rule trades idle CUs against the parts' way through memory.
+//   Parts: up to 128 query tiles (head size 256: any number), as many parts as give every CU one (causal: 320 in all, half of which
+// have keys), four tiles of keys at least (two), if the tiles a workgroup is spared, in us, are more than the second
+// kernel's 4.5 us and the parts' way out and in.  In bf16 and fp16, B1 H2 S4393 D64: none 43.8 -> 24.9, causal 50.0 -> 23.4, key-padding
+// mask 89 -> 34; D128 59 -> 36, 64 -> 28, 115 -> 47; D256 B1 H2 S2000 56 -> 29, 59 -> 29, 74 -> 34.  (B2 H8 S963, 128 tiles, D128 none: 18.5
+// whole, 25.7 in two parts.)
+//   Halves within a workgroup, D <= 128: two waves per SIMD help where a wave waits or works outside the matrix cores, and under the causal
+// rule they shorten the last tiles; without mask and rule they cost as much as they give.  B12 H1 S1499 D64, mask 35.3 -> 27.0; B3 H4 S2377
+// D128, mask 63 -> 56; B1 H8 S8192 D128, causal 159 -> 137; B1 H32 S512 D64, mask 13.9 -> 12.7, D128, causal 13.4 -> 14.9 (eight
+// tiles: whole).
+struct Shares {
+    int  parts = 1, part_tiles = 0;
+    bool halves = false;
+};
+Shares plan_shares(const paras_sdpa_args& a) {
+    Shares r;
+    const bool causal = a.is_causal != 0, masked = a.mask_kind != 0;
+    const long W = static_cast<long>(a.B * a.Hq) * ((a.Lq + kBM - 1) / kBM);
+    const long tiles = ((causal && a.Lq < a.Lk ? a.Lq : a.Lk) + kBN - 1) / kBN;      // of the query tile that sees the most
+    const long least = a.D > 128 ? 2 : 4;
+    if (W < 1 || W > 512 || tiles <= least) return r;
+    const double tile_us = a.D == 64 ? (masked ? 1.15 : causal ? 0.65 : 0.6) : a.D == 128 ? (masked ? 1.45 : 0.85) : (masked ? 2.6 : causal ? 1.55 : 1.65);
+    const long parts = (causal ? 320 : 256) / W;
+    if (parts > 1 && (W <= 128 || a.D > 128)) {
+        const long t = (tiles + parts - 1) / parts > least ? (tiles + parts - 1) / parts : least, n = (tiles + t - 1) / t;
+        if (n > 1 && tile_us * (tiles - t) > 4.5 + static_cast<double>(W * n * a.D) / (causal ? 8000 : 4000)) {
+            r.parts = static_cast<int>(n);
+            r.part_tiles = static_cast<int>(t);
+            return r;
+        }
+    }
+    r.halves = a.D <= 128 && ((masked && W <= 256 && tiles >= 8) || (causal && ((W <= 256 && tiles >= 12) || (W <= 512 && tiles >= 24))));
+    return r;
+}
+
+}  // namespace
+
+size_t flash_workspace(const paras_sdpa_args& a) {
+    const Shares r = plan_shares(a);
+    if (r.parts <= 1 || flash_uses_wide(a)) return 0;
+    const size_t slots = static_cast<size_t>(a.B * a.Hq) * ((a.Lq + kBM - 1) / kBM) * r.parts;
+    return slots * (kBM * a.D + 2 * kBM) * sizeof(float);
+}
+
 bool flash_uses_wide(const paras_sdpa_args& a) {
     return flash::wide_supported(a.B, a.Hq, a.Lq, a.Lk, static_cast<int>(a.D), a.mask_kind, a.is_causal != 0);
 }
 
-int launch_flash(const paras_sdpa_args& a, hipStream_t s) {
-    FlashParams p;
+int launch_flash(const paras_sdpa_args& a, void* workspace, hipStream_t s) {
+    FlashParams p{};
     p.q = static_cast<const std::uint16_t*>(a.q);
     p.k = static_cast<const std::uint16_t*>(a.k);
     p.v = static_cast<const std::uint16_t*>(a.v);
@@ -745,10 +938,17 @@ int launch_flash(const paras_sdpa_args& a, hipStream_t s) {
     }
     const bool causal = a.is_causal != 0;
     const int mk = a.mask_kind;
+    const Shares r = plan_shares(a);
+    if (r.parts > 1 && workspace != nullptr) {
+        p.n_parts = r.parts;
+        p.part_tiles = r.part_tiles;
+        p.part_o = static_cast<float*>(workspace);
+        p.part_ml = p.part_o + static_cast<size_t>(a.B * a.Hq) * ((a.Lq + kBM - 1) / kBM) * r.parts * kBM * a.D;
+    }
     if (flash_uses_wide(a)) return launch_flash_wide(p, causal, a.dtype == PARAS_BF16, s);
     if (a.dtype == PARAS_BF16)
-        return a.D == 256 ? launch_t<bf16_t, 256>(p, causal, mk, s) : a.D == 128 ? launch_t<bf16_t, 128>(p, causal, mk, s) : launch_t<bf16_t, 64>(p, causal, mk, s);
-    return a.D == 256 ? launch_t<f16_t, 256>(p, causal, mk, s) : a.D == 128 ? launch_t<f16_t, 128>(p, causal, mk, s) : launch_t<f16_t, 64>(p, causal, mk, s);
+        return a.D == 256 ? launch_t<bf16_t, 256>(p, causal, mk, r.halves, s) : a.D == 128 ? launch_t<bf16_t, 128>(p, causal, mk, r.halves, s) : launch_t<bf16_t, 64>(p, causal, mk, r.halves, s);
+    return a.D == 256 ? launch_t<f16_t, 256>(p, causal, mk, r.halves, s) : a.D == 128 ? launch_t<f16_t, 128>(p, causal, mk, r.halves, s) : launch_t<f16_t, 64>(p, causal, mk, r.halves, s);
 }
 
 }  // namespace paras

@@ -35,6 +35,11 @@ struct FlashParams {
     const unsigned char* mask;
     long ms_b, ms_h, ms_q, ms_k;
     float score_scale; // the caller's scale as given; the masked variants apply it themselves and run with scale = 1
+    // keys of a query tile shared out to n_parts workgroups, part_tiles tiles each (sdpa_flash.hip): [B Hq, n_qblocks, n_parts] slots
+    // of 128 x D outputs as the lanes hold them, and of each wave's 32 maxima and 32 sums
+    int    n_parts, part_tiles;
+    float* part_o;
+    float* part_ml;
     unsigned magic_nq, magic_hq, magic_rep;   // ceil(2^32 / d) for d = n_qblocks, Hq, Hq / Hkv (set by the wide kernel's launcher)
 };
 

@@ -88,6 +88,8 @@ __global__ __launch_bounds__(256, 1) void flash_wide_kernel(const FlashParams p)
     __shared__ __attribute__((aligned(1024))) std::uint16_t k_lds1[kBN * D];
     __shared__ __attribute__((aligned(1024))) std::uint16_t v_lds0[kBN * D];
     __shared__ __attribute__((aligned(1024))) std::uint16_t v_lds1[kBN * D];
+    // K tile 0 of an item, read before the loop.  (Not in k_lds0: K tile 2 is requested into it while another wave may still read.)
+    __shared__ __attribute__((aligned(1024))) std::uint16_t k_first[kBN * D];
     // A wavefront's 64 x 128 outputs pass through LDS on their way out (16 KB each, its own region:
     // no barrier), so that the global stores write whole rows.
     constexpr int OROW = D + 8;   // row pitch of that region in elements: 16 bytes of padding spread the rows over the banks
@@ -209,7 +211,7 @@ __global__ __launch_bounds__(256, 1) void flash_wide_kernel(const FlashParams p)
     float m_run[QB], l_run[QB];
     // The first tiles of an item: K tiles 0 and 1, V tile 0 (the loop stages the rest).
     auto stage_first = [&]() {
-        stage_rows(k_rsrc, k_lane, k_row_bytes, 0, k_lds0);
+        stage_rows(k_rsrc, k_lane, k_row_bytes, 0, k_first);
         stage_rows(k_rsrc, k_lane, k_row_bytes, kBN, k_lds1);
         stage_rows(v_rsrc, v_lane, v_row_bytes, 0, v_lds0);
     };
@@ -495,7 +497,7 @@ __global__ __launch_bounds__(256, 1) void flash_wide_kernel(const FlashParams p)
         {
             // S(0) from the first half of K tile 0, then the keys of block 1 for block 0's score MFMAs
 #pragma unroll
-            for (int ks = 0; ks < KSTEPS; ++ks) fetch_k(k_lds0, ks);
+            for (int ks = 0; ks < KSTEPS; ++ks) fetch_k(k_first, ks);
 #pragma unroll
             for (int ks = 0; ks < KSTEPS; ++ks)
 #pragma unroll
@@ -505,7 +507,7 @@ __global__ __launch_bounds__(256, 1) void flash_wide_kernel(const FlashParams p)
                 }
             asm volatile("s_nop 15\n\ts_nop 15" : "+v"(s_a[0]), "+v"(s_a[1]));   // MFMA results the compiler cannot see coming
 #pragma unroll
-            for (int ks = 0; ks < KSTEPS; ++ks) fetch_k(k_lds0 + 32 * D, ks);
+            for (int ks = 0; ks < KSTEPS; ++ks) fetch_k(k_first + 32 * D, ks);
             // The first reference point is the maximum of block 0 itself: nothing to rescale yet.
             // (Every query sees key 0, so the maximum is finite.)
 #pragma unroll
@@ -515,7 +517,6 @@ __global__ __launch_bounds__(256, 1) void flash_wide_kernel(const FlashParams p)
                 raise_at[qb] = m_run[qb] + lazy_margin;
             }
         }
-        lds_reads_done_barrier();          // K tile 2 goes where the scores and the fragments above were read from
         for (int t = 0; t < wave_tiles; t += 2) {
             tile(t, Par0{});
             if (t + 1 >= wave_tiles) break;
@@ -593,10 +594,11 @@ bool wide_supported(long B, long Hq, long Lq, long Lk, int head, int mask_kind, 
     // One workgroup per CU and 256 queries per item: it needs a few items per CU to keep them all
     // busy and, under the causal rule, long rows for the items' fixed cost to pay off (measured
     // against the 32-queries-per-wavefront kernel: ahead from 4096 causal / 1024 unmasked queries on).
+    const long least = causal ? 4096 : 1024;
+    if (Lq < least || Lk < least) return false;        // (before the runtime is asked: small calls are bound by the host)
     int dev = 0, cus = 0;
     if (hipGetDevice(&dev) != hipSuccess || hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, dev) != hipSuccess) return false;
-    if (bh * nq < 2ull * static_cast<unsigned long long>(cus)) return false;
-    return causal ? (Lq >= 4096 && Lk >= 4096) : (Lq >= 1024 && Lk >= 1024);
+    return bh * nq >= 2ull * static_cast<unsigned long long>(cus);
 }
 
 int launch_flash_wide(FlashParams p, bool causal, bool is_bf16, hipStream_t s) {

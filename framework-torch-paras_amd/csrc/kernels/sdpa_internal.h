@@ -10,8 +10,11 @@ namespace paras {
 
 // MFMA flash forward: bf16/f16, D == Dv in {64, 128}, no explicit mask
 // (causal or none), no attention weights returned.
-bool flash_supported(const paras_sdpa_args& a);
-int  launch_flash(const paras_sdpa_args& a, hipStream_t s);
+bool   flash_supported(const paras_sdpa_args& a);
+// Workspace for the parts of a problem with too few query tiles to fill the chip; without it (null) launch_flash does not share
+// out the keys.
+size_t flash_workspace(const paras_sdpa_args& a);
+int    launch_flash(const paras_sdpa_args& a, void* workspace, hipStream_t s);
 // Whether launch_flash takes its 64-queries-per-wavefront form (head size 128, no mask, enough
 // long rows to fill the chip with one workgroup per CU); only meaningful when flash_supported.
 bool flash_uses_wide(const paras_sdpa_args& a);

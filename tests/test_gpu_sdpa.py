@@ -123,6 +123,52 @@ def test_flash_matches_oracle(dtype, shape):
 
 
 @pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])
+@pytest.mark.parametrize("kind", ["none", "causal", "bool", "additive"])
+@pytest.mark.parametrize("D", [64, 128, 256])
+def test_flash_with_the_keys_shared_out(D, kind, dtype):
+    """Few query tiles: parts of the keys in workgroups of their own (their number known from the workspace), and two halves within a
+    workgroup; parts and halves that end inside a tile, that lie wholly beyond a query (causal) and in which a mask leaves nothing.
+    Against the host engine; rows without any key are NaN, a NaN in V behind a mask reaches every query; the log-sum-exp where
+    no mask narrows the scores: fp32 sums, 1e-4."""
+    causal, masked = kind == "causal", kind in ("bool", "additive")
+    shapes = [(1, 2, 1, 1300, 1300), (2, 2, 2, 130, 1301)] if causal else [(1, 2, 1, 300, 2500), (1, 1, 1, 33, 897), (2, 1, 1, 200, 1023)]
+    if D < 256:
+        shapes += [(3, 8, 8, 900, 837)] if causal else [(4, 8, 8, 500, 577)]
+    seen_parts = False
+    for B, Hq, Hkv, Lq, Lk in shapes:
+        torch.manual_seed(Lq + D)
+        q, k, v = torch.randn(B, Hq, Lq, D).to(dtype), torch.randn(B, Hkv, Lk, D).to(dtype), torch.randn(B, Hkv, Lk, D).to(dtype)
+        kw, empty = dict(scale=O.round_to_dtype(1 / math.sqrt(D), dtype)), None      # (the host engine narrows the scale to the type)
+        if masked:
+            m = torch.rand(B, 1, Lq, Lk) < 0.4
+            m[:, :, : Lq // 2, Lk // 3:] = False               # whole shares without a visible key
+            m[:, :, Lq // 2:, : Lk // 2] = False
+            empty = Lq // 3
+            m[0, 0, empty] = False
+            kw["mask"] = m if kind == "bool" else torch.where(m, torch.randn(B, 1, Lq, Lk), torch.tensor(-math.inf)).to(dtype)
+        out, _, lse, kern = run(q, k, v, is_causal=causal, want_lse=True, **kw)
+        assert kern == "flash_mfma"
+        mask = kw.get("mask")
+        a = capi.sdpa_args(q, k, v, torch.empty_like(q), mask=mask, is_causal=causal)
+        seen_parts |= capi.lib().paras_sdpa_workspace(C.byref(a)) > 0
+        want, _ = O.sdpa_math(q, k, v, is_causal=causal, enable_gqa=True, gemm="aten", scale=kw["scale"], attn_mask=mask)
+        out = out.cpu()
+        assert bool((out.isnan() == want.isnan()).all()) and (empty is None or bool(out[0, :, empty].isnan().all()))
+        # a step of the type on values up to 4, 2^-7 x 2 (2^-10 x 2), and the rounding of the weights
+        assert max_abs(out.nan_to_num(), want.nan_to_num()) <= (2.5e-2 if dtype == torch.bfloat16 else 4e-3), (B, Hq, Lq, Lk)
+        if not masked:
+            s = (q.float() @ k.float().repeat_interleave(Hq // Hkv, 1).transpose(-1, -2)) * kw["scale"]
+            if causal:
+                s = s.masked_fill(~torch.ones(Lq, Lk).tril().bool(), -math.inf)
+            assert max_abs(lse, torch.logsumexp(s, -1)) <= 1e-4
+        else:
+            v[0, 0, Lk // 2 + 1, 3] = math.nan                  # hidden from the first half of the queries, open to some of the others
+            bad = run(q, k, v, **kw)[0].cpu()
+            assert bool(bad[0, : Hq // Hkv, :, 3].isnan().all()) and bool((bad[0, :, :, 4].isnan() == want[0, :, :, 4].isnan()).all())
+    assert seen_parts
+
+
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])
 def test_flash_accuracy_with_large_scores(dtype):
     """Inputs twice and four times the usual magnitude (score spread x4 / x16): the error against
     the exact fp64 result must stay that of rounding P and O to the operand type.  Rounding a
