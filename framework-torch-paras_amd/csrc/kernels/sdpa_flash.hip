@@ -94,6 +94,61 @@ __device__ __forceinline__ int tiles_of(const FlashParams& p, int qblock) {
     return (keys + kBN - 1) / kBN;
 }
 
+// The keys of (batch, head) up to the last one that a mask shared by all queries opens, to the next 16 or so; all of them if the
+// mask is not of that kind or the row is so short that the look at it costs more than it saves (S91 D128 7.6 -> 7.9 us, S424 16.2 ->
+// 15.6).  From the end of the row, 1024 bytes at a time.
+__device__ __forceinline__ int open_keys(const FlashParams& p, int b, int hq, int lane) {
+    if (p.ms_q != 0 || p.ms_k != 1 || p.Lk <= 256) return p.Lk;
+    typedef u32x4 u32x4_any __attribute__((aligned(1)));
+    const unsigned char* row = p.mask + static_cast<long>(b) * p.ms_b + static_cast<long>(hq) * p.ms_h;
+    for (int k0 = (p.Lk - 1) / 1024 * 1024; k0 >= 0; k0 -= 1024) {
+        const int at = k0 + 16 * lane;
+        std::uint32_t any = 0;
+        if (at < p.Lk) {
+            const u32x4 w = *reinterpret_cast<const u32x4_any*>(row + min(at, p.Lk - 16));
+            any = w[0] | w[1] | w[2] | w[3];
+        }
+        const unsigned long long lanes = __builtin_amdgcn_ballot_w64(any != 0);
+        if (lanes != 0) return min(p.Lk, k0 + 16 * (64 - __builtin_clzll(lanes)));
+    }
+    return 0;
+}
+
+// Keys first .. last - 1 are closed to every query: their weights are 0, and so is their share of the outputs, but for the columns
+// in which a value is an infinity or a NaN, since 0 times those is NaN.  All the workgroup's threads look (8 columns each); it has finished
+// its tiles.  (What it saves is arithmetic, scores, narrowings and exponentials: with lengths from half to all of the longest, fp16 B6 H12
+// S777 D64 26.7 -> 24.0 us, bf16 B13 H4 S1837 D128 134 -> 106, B4 H16 S5283 D64 738 -> 532, the same bits.)
+template <typename T, int D, int DBLK, int kThreads>
+__device__ __forceinline__ void close_columns(const FlashParams& p, const std::uint16_t* v, int first, int last, int* flags, int lh, float16_t (&oacc)[DBLK]) {
+    constexpr std::uint32_t kExp = std::is_same<T, bf16_t>::value ? 0x7F807F80u : 0x7C007C00u, kUnit = std::is_same<T, bf16_t>::value ? 0x00800080u : 0x04000400u;
+    constexpr int kChunks = D / 8, kRows = kThreads / kChunks;
+    const int tid = threadIdx.x, col = tid % kChunks;
+    const std::uint16_t* at = v + col * 8;
+    u32x4 bad = {0, 0, 0, 0};
+#pragma unroll 4
+    for (int r = first + tid / kChunks; r < last; r += kRows) {
+        const u32x4 w = *reinterpret_cast<const u32x4*>(at + static_cast<long>(r) * p.vs_l);
+#pragma unroll
+        for (int i = 0; i < 4; ++i) bad[i] |= (w[i] & kExp) + kUnit;       // an exponent of all ones carries into the sign's place
+    }
+#pragma unroll
+    for (int i = 0; i < 4; ++i) bad[i] &= 0x80008000u;
+    if (__builtin_expect(__syncthreads_or((bad[0] | bad[1] | bad[2] | bad[3]) != 0), 0)) {
+        for (int i = tid; i < D; i += kThreads) flags[i] = 0;
+        __syncthreads();
+#pragma unroll
+        for (int i = 0; i < 8; ++i)
+            if ((bad[i / 2] >> (16 * (i & 1) + 15)) & 1u) flags[col * 8 + i] = 1;
+        __syncthreads();
+#pragma unroll
+        for (int db = 0; db < DBLK; ++db)
+#pragma unroll
+            for (int r = 0; r < 16; ++r)
+                if (flags[db * 32 + (r >> 2) * 8 + 4 * lh + (r & 3)] != 0) oacc[db][r] = __builtin_nanf("");
+        __syncthreads();                       // the flags' place may be written again
+    }
+}
+
 // The weight of a share of the keys whose maximum is m beside one with M >= m.  A share in which the query saw no key counts
 // with weight zero (and hands on a NaN that its values left there, as 0 x NaN does in the product).
 __device__ __forceinline__ float weight_of(float m, float M, float scale_log2) {
@@ -197,6 +252,7 @@ __global__ __launch_bounds__(256 * kHalves, (D > 128 || kHalves > 1 ? 1 : 2)) vo
         }
     }
     const int qblock = nq - 1 - qi;
+    const int b = bh / p.Hq, hq = bh % p.Hq;
     int n_tiles = tiles_of<kCausal>(p, qblock);
     int first = 0;                             // this wave's first tile of keys
     const bool whole = !kParts || n_tiles <= p.part_tiles;
@@ -206,14 +262,23 @@ __global__ __launch_bounds__(256 * kHalves, (D > 128 || kHalves > 1 ? 1 : 2)) vo
         if (first >= n_tiles) return;
         n_tiles = min(n_tiles - first, p.part_tiles);
     }
+    // A key-padding mask: the tiles past the last open key of the sequence are left out of the loop (close_columns).  Not for
+    // heads of 256: the registers it takes are spilled there (B14 H1 S117 13.9 -> 17.1 us, B1 H4 S2402 48 -> 55).
+    constexpr bool kLeaveOut = kMask == 1 && D <= 128;
+    int closed0 = 0, closed1 = 0;              // keys of this workgroup that are left out
+    if constexpr (kLeaveOut) {
+        const int open = max(min((open_keys(p, b, hq, lane) + kBN - 1) / kBN - first, n_tiles), 0);
+        closed0 = (first + open) * kBN;
+        closed1 = min(p.Lk, (first + n_tiles) * kBN);
+        n_tiles = open;
+    }
     const int turns = kHalves == 1 ? n_tiles : (n_tiles + 1) / 2;       // tiles between the workgroup's barriers
     if constexpr (kHalves == 2) {
         first += half * turns;
         n_tiles = half == 0 ? turns : n_tiles - turns;                  // (the second half of a single tile has none)
     }
     const int key0 = first * kBN;
-    const int Lk = kParts || kHalves == 2 ? min(p.Lk - key0, n_tiles * kBN) : p.Lk;
-    const int b = bh / p.Hq, hq = bh % p.Hq;
+    const int Lk = kParts || kHalves == 2 || kLeaveOut ? min(p.Lk - key0, n_tiles * kBN) : p.Lk;
     const int hkv = hq / (p.Hq / p.Hkv);
 
     const int lq = lane & 31, lh = lane >> 5;
@@ -251,7 +316,7 @@ __global__ __launch_bounds__(256 * kHalves, (D > 128 || kHalves > 1 ? 1 : 2)) vo
     static_assert((RPI * NW) % 16 == 0 || (RPI * NW == 8 && D == 256), "the staging swizzle assumes whole groups of 16 (or 8) rows per request");
     typedef __attribute__((address_space(3))) void* lptr_t;
     auto make_rsrc = [&](const std::uint16_t* base, int row_bytes) {
-        const int bytes = kHalves == 2 && Lk <= 0 ? 0 : (Lk - 1) * row_bytes + D * 2;           // < 2^31: checked by flash_supported
+        const int bytes = (kHalves == 2 || kLeaveOut) && Lk <= 0 ? 0 : (Lk - 1) * row_bytes + D * 2;           // < 2^31: checked by flash_supported
         return __builtin_amdgcn_make_buffer_rsrc(const_cast<std::uint16_t*>(base), 0, bytes, 0x00020000);
     };
     const __amdgpu_buffer_rsrc_t k_rsrc = make_rsrc(kbase, k_row_bytes);
@@ -715,6 +780,9 @@ __global__ __launch_bounds__(256 * kHalves, (D > 128 || kHalves > 1 ? 1 : 2)) vo
         publish();
     }
 
+    if constexpr (kLeaveOut) {
+        if (closed0 < closed1) close_columns<T, D, DBLK, 256 * kHalves>(p, p.v + b * p.vs_b + hkv * p.vs_h, closed0, closed1, reinterpret_cast<int*>(k_first), lh, oacc[0]);
+    }
     float l_tot[QB];
 #pragma unroll
     for (int qb = 0; qb < QB; ++qb) l_tot[qb] = half_swap_sum(l_run[qb]);

@@ -169,6 +169,41 @@ def test_flash_with_the_keys_shared_out(D, kind, dtype):
 
 
 @pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])
+@pytest.mark.parametrize("D", [64, 128, 256])
+def test_flash_key_padding_leaves_out_closed_tiles(D, dtype):
+    """Keys past a sequence's last one: whole tiles of them, ends at, before and after a tile's, no key at all, rows shorter and longer
+    than one look at the mask (1024 keys), whole, in halves and in parts.  What lies in V there does not change a bit unless it is
+    an infinity or a NaN, which makes its column NaN for every query (0 x NaN, as in the host engine's product)."""
+    for H, Lq, Lk, lens in [(2, 130, 290, [0, 1, 63, 64, 65, 255, 256, 290]), (1, 40, 1500, [1499, 16, 700, 1025, 1024, 0]), (8, 140, 900, [512, 530, 900, 0, 64, 100]),
+                            (1, 20, 15, [3, 0, 15])]:
+        B = len(lens)
+        torch.manual_seed(Lk + D)
+        q, k, v = (torch.randn(B, n, L, D).to(dtype) for n, L in ((2 * H, Lq), (H, Lk), (H, Lk)))
+        keep = (torch.arange(Lk)[None, :] < torch.tensor(lens)[:, None]).reshape(B, 1, 1, Lk)
+        scale = O.round_to_dtype(1 / math.sqrt(D), dtype)
+        out = run(q, k, v, mask=keep, scale=scale)[0].cpu()
+        want, _ = O.sdpa_math(q, k, v, attn_mask=keep, enable_gqa=True, gemm="aten", scale=scale)
+        assert bool((out.isnan() == want.isnan()).all())
+        # a step of the type on values up to 4, and the rounding of the weights
+        assert max_abs(out.nan_to_num(), want.nan_to_num()) <= (2.5e-2 if dtype == torch.bfloat16 else 4e-3), (Lk, lens)
+        full = run(q, k, v, mask=keep.expand(B, 1, Lq, Lk).contiguous(), scale=scale)[0].cpu()      # a mask of every query's own: nothing is left out
+        bar = 2.5e-2 if dtype == torch.bfloat16 else 4e-3
+        # (halves and parts divide the open keys in the one case and all keys in the other, and sum in another order)
+        assert max_abs(out.nan_to_num(), full.nan_to_num()) <= (0.0 if Lk <= 290 else bar)
+        v2, poisoned = v.clone(), torch.zeros(B, 2 * H, D, dtype=torch.bool)
+        for b, n in enumerate(lens):
+            if n < Lk:
+                v2[b, :, n:] *= 3
+                for at, d, x in ((n, 5, math.nan), (Lk - 1, 31, math.inf), ((n + Lk) // 2, D - 1, -math.inf)):
+                    v2[b, 0, at, d] = x
+                    poisoned[b, :2, d] = True
+        got = run(q, k, v2, mask=keep, scale=scale)[0].cpu()
+        assert bool((got.isnan() == (out.isnan() | poisoned[:, :, None, :])).all())
+        clean = ~poisoned[:, :, None, :].expand_as(out)
+        assert torch.equal(got[clean].nan_to_num(), out[clean].nan_to_num())
+
+
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])
 def test_flash_accuracy_with_large_scores(dtype):
     """Inputs twice and four times the usual magnitude (score spread x4 / x16): the error against
     the exact fp64 result must stay that of rounding P and O to the operand type.  Rounding a
