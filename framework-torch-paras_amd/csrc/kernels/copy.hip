@@ -27,8 +27,21 @@ struct Strided {
     long dst_strides[kMaxDims];
 };
 
-__device__ __forceinline__ void offsets(const Strided& s, long flat, long* so, long* d_o) {
+// (`small`: the whole index fits 32 bits, uniform.  A 64-bit division is some hundred instructions.)
+__device__ __forceinline__ void offsets(const Strided& s, long flat, bool small, long* so, long* d_o) {
     long a = 0, b = 0;
+    if (small) {
+        unsigned left = static_cast<unsigned>(flat);
+        for (int d = s.ndim - 1; d >= 0; --d) {
+            const unsigned size = static_cast<unsigned>(s.sizes[d]), q = left / size, c = left - q * size;
+            left = q;
+            a += c * s.src_strides[d];
+            b += c * s.dst_strides[d];
+        }
+        *so = a;
+        *d_o = b;
+        return;
+    }
     for (int d = s.ndim - 1; d >= 0; --d) {
         const long c = flat % s.sizes[d];
         flat /= s.sizes[d];
@@ -44,7 +57,7 @@ __global__ __launch_bounds__(kBlock) void copy_same_kernel(const W* __restrict__
                                                            const Strided s) {
     for (long i = static_cast<long>(blockIdx.x) * kBlock + threadIdx.x; i < n; i += static_cast<long>(gridDim.x) * kBlock) {
         long a, b;
-        offsets(s, i, &a, &b);
+        offsets(s, i, n <= 0xFFFFFFFFL, &a, &b);
         dst[b] = src[a];
     }
 }
@@ -57,7 +70,7 @@ __global__ __launch_bounds__(kBlock) void copy_convert_kernel(const typename Ele
                                                               const Strided s) {
     for (long i = static_cast<long>(blockIdx.x) * kBlock + threadIdx.x; i < n; i += static_cast<long>(gridDim.x) * kBlock) {
         long a, b;
-        offsets(s, i, &a, &b);
+        offsets(s, i, n <= 0xFFFFFFFFL, &a, &b);
         if constexpr (sizeof(typename Elem<TS>::store_t) == 8)
             dst[b] = Elem<TD>::from_f64(Elem<TS>::to_f64(src[a]));
         else
@@ -69,7 +82,7 @@ template <typename W>
 __global__ __launch_bounds__(kBlock) void fill_kernel(W* __restrict__ dst, long n, const Strided s, W value) {
     for (long i = static_cast<long>(blockIdx.x) * kBlock + threadIdx.x; i < n; i += static_cast<long>(gridDim.x) * kBlock) {
         long a, b;
-        offsets(s, i, &a, &b);
+        offsets(s, i, n <= 0xFFFFFFFFL, &a, &b);
         dst[b] = value;
     }
 }
@@ -285,7 +298,7 @@ __global__ __launch_bounds__(kBlock) void binary_strided_kernel(int op, const ty
     const bool unit = alpha == 1.0;
     for (long i = static_cast<long>(blockIdx.x) * kBlock + threadIdx.x; i < n; i += static_cast<long>(gridDim.x) * kBlock) {
         long ao, bo;
-        offsets(s, i, &ao, &bo);
+        offsets(s, i, n <= 0xFFFFFFFFL, &ao, &bo);
         out[i] = binary_one<T>(op, a[ao], b[bo], alpha, unit);
     }
 }
@@ -305,7 +318,7 @@ __global__ __launch_bounds__(kBlock) void binary_vec16_kernel(int op, const std:
         const std::uint32_t w = b[0] | (static_cast<std::uint32_t>(b[0]) << 16);
         bv = u32x4{w, w, w, w};
     } else {
-        bv = brow == nvec ? load16_nt(b + i * 8) : load16(b + (i % brow) * 8);
+        bv = brow == nvec ? load16_nt(b + i * 8) : load16(b + (nvec <= 0xFFFFFFFFL ? static_cast<unsigned>(i) % static_cast<unsigned>(brow) : i % brow) * 8);
     }
     const std::uint16_t* ae = reinterpret_cast<const std::uint16_t*>(&av);
     const std::uint16_t* be = reinterpret_cast<const std::uint16_t*>(&bv);

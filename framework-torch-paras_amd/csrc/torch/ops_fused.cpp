@@ -81,9 +81,18 @@ Tensor rotate_half_impl(const Tensor& x, bool backward, const char* name) {
     TORCH_CHECK(x.dim() <= 8, "paras ", name, ": rank exceeds kernel limit");
     const int64_t D = x.size(-1);
     TORCH_CHECK(D % 2 == 0, "paras ", name, ": last dimension must be even");
-    Tensor in = x.contiguous();
-    Tensor out = empty_paras_like(in);
+    Tensor out = empty_paras_like(x);
     if (out.numel() == 0) return out;
+    // rows that the kernel can read where they are: no copy to bring them together
+    bool rows = !x.is_contiguous() && !x.is_neg() && (x.scalar_type() == c10::kBFloat16 || x.scalar_type() == c10::kHalf) && D % 16 == 0 && x.stride(-1) == 1 &&
+                (reinterpret_cast<uintptr_t>(x.data_ptr()) & 15) == 0 && x.numel() / 8 < (1L << 31);
+    for (int64_t d = 0; rows && d + 1 < x.dim(); ++d) rows = x.stride(d) % 8 == 0;
+    if (rows) {
+        check(paras_rotate_half_strided(x.data_ptr(), out.data_ptr(), static_cast<int>(x.dim()), x.sizes().data(), x.strides().data(), backward ? 1 : 0,
+                                        require_float_code(x, name), stream_for(x)));
+        return out;
+    }
+    Tensor in = x.contiguous();
     check(paras_rotate_half(in.data_ptr(), out.data_ptr(), in.numel() / D, D, backward ? 1 : 0,
                             require_float_code(in, name), stream_for(in)));
     return out;

@@ -61,6 +61,7 @@ SIGNATURES = {
     "paras_rms_norm_bwd": (i32, [vp, vp, vp, vp, vp, vp, vp, i64, i64, i32, vp]),
     "paras_swiglu_fwd": (i32, [vp, vp, vp, i64, i32, vp]),
     "paras_swiglu_bwd": (i32, [vp, vp, vp, vp, vp, i64, i32, vp]),
+    "paras_rotate_half_strided": (i32, [vp, vp, i32, C.POINTER(i64), C.POINTER(i64), i32, i32, vp]),
     "paras_rotate_half": (i32, [vp, vp, i64, i64, i32, i32, vp]),
     "paras_sdpa_workspace": (sz, [C.POINTER(SdpaArgs)]),
     "paras_sdpa_fwd": (i32, [C.POINTER(SdpaArgs), vp, vp]),

@@ -195,6 +195,10 @@ PARAS_API int paras_swiglu_composed_fwd(const void* x, const void* gate, void* o
 /* ------------------------------------------------------------------------- */
 PARAS_API int paras_rotate_half(const void* x, void* out, int64_t rows, int64_t D,
                                 int backward, int dtype, void* stream);
+/* The same for 16-bit x of any layout whose rows are D contiguous elements, D a multiple of 16, each on a   */
+/* 16-byte boundary (a transposed view of a projection's heads); strides in elements, out dense, < 2^34 elements. */
+PARAS_API int paras_rotate_half_strided(const void* x, void* out, int ndim, const int64_t* sizes, const int64_t* strides, int backward,
+                                        int dtype, void* stream);
 
 /* ------------------------------------------------------------------------- */
 /* Scaled dot-product attention forward                                       */

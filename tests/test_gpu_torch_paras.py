@@ -1061,3 +1061,23 @@ def test_negated_views_are_read_negated(device):
     assert torch.equal(into.cpu(), -x)
     neg(into).copy_(x)
     assert torch.equal(into.cpu(), -x)
+
+
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])
+def test_rotate_half_of_views_is_that_of_their_copies(dtype, device):
+    """Rows that lie anywhere (a projection's heads, slices of a fused one, repeated rows, one dimension of many) are read where they
+    are; NaNs, infinities and zeros keep the host's bits; views the kernel cannot read that way are copied as before."""
+    from torch_paras import nn as paras_nn
+    base = torch.randn(2, 9, 6 * 64).to(dtype)
+    base[0, 3, 5], base[1, 2, 40], base[1, 8, 100], base[0, 0, 7] = math.nan, math.inf, -math.inf, 0.0
+    p = base.to(device)
+    views = [lambda t: t.view(2, 9, 6, 64).transpose(1, 2), lambda t: t.view(2, 9, 3, 128).transpose(1, 2), lambda t: t[:, :, 64:192],
+             lambda t: t.view(2, 9, 24, 16).permute(2, 0, 1, 3), lambda t: t[:, :1].expand(2, 5, 384), lambda t: t[1, ::2, :32],
+             lambda t: t.view(2, 9, 6, 64)[:, :, 2:3].transpose(1, 2), lambda t: t[:, :, 4:36], lambda t: t.transpose(1, 2)[:, 3:5].transpose(1, 2),
+             lambda t: t.view(2, 9, 32, 12).transpose(1, 2)]
+    for i, view in enumerate(views):
+        got, want = paras_nn.rotate_half(view(p)), paras_nn.rotate_half(view(base).contiguous().to("paras:0"))
+        assert got.is_contiguous() and got.shape == want.shape
+        assert torch.equal(got.cpu().view(torch.int16), want.cpu().view(torch.int16)), i
+        gb = torch.ops.paras.rotate_half_backward(view(p)).cpu()
+        assert torch.equal(gb.view(torch.int16), torch.ops.paras.rotate_half_backward(view(base).contiguous().to("paras:0")).cpu().view(torch.int16)), i
