@@ -57,7 +57,11 @@ __global__ __launch_bounds__(256) void gemm_flex_finish_kernel(const Params p) {
 struct Tile { int m, n, stages, per_cu; double step, lat; };
 constexpr Tile kTiles[] = {{256, 256, 2, 1, 1.15, 0.36}, {192, 256, 2, 1, 0.94, 0.05}, {192, 192, 3, 1, 0.71, 0.34}, {192, 128, 3, 1, 0.55, 0.55},
                            {128, 128, 2, 2, 0.84, 0.56}, {128, 128, 3, 1, 0.42, 0.34}, {64, 128, 2, 3, 0.90, 0.45}, {64, 128, 4, 1, 0.285, 0.30},
-                           {64, 64, 2, 4, 0.83, 0.36},   {64, 64, 3, 3, 0.545, 0.22},  {64, 64, 4, 2, 0.34, 0.21},  {32, 128, 4, 2, 0.43, 0.26}};
+                           {64, 64, 2, 4, 0.83, 0.36},   {64, 64, 3, 3, 0.545, 0.22},  {64, 64, 4, 2, 0.34, 0.21},  {32, 128, 4, 2, 0.43, 0.26},
+                           {256, 224, 2, 1, 0.985, 0.30}, {224, 224, 2, 1, 0.92, 0.30}, {192, 224, 2, 1, 0.85, 0.30}};
+// The last three, for both operands along the contraction only, come in whole rounds of workgroups where the others do not
+// (1500 x 14336 x 4096 in bf16: 448 tiles of 192 x 256 in two rounds 165 us, 512 of 192 x 224 154; 5566 x 7104 x 2624 256 x 256 197, 256 x 224 177).
+constexpr int kAlongContraction = 12;
 constexpr int kTileCount = sizeof(kTiles) / sizeof(kTiles[0]);
 static_assert(kTiles[kTile128x128].m == 128 && kTiles[kTile128x128].n == 128 && kTiles[kTile128x128].stages == 2, "the tile that paras_gemm_nt_ws splits");
 constexpr int kCus = 256;
@@ -93,6 +97,7 @@ Plan plan(const Problem& q, bool may_split) {
     const double memory = static_cast<double>(q.M + q.N) * q.K * q.batch * 2 / 5.6e6 + 2.5;      // the operands' way from memory
     for (int t = 0; t < kTileCount; ++t) {
         const Tile& tl = kTiles[t];
+        if (t >= kAlongContraction && (q.a_rows || q.b_rows)) break;
         if (tl.m * tl.n > 128 * 128 && q.K <= 512) continue;     // mostly stores: small tiles overlap them with other tiles' work
         const long mt = (q.M + tl.m - 1) / tl.m, nt = (q.N + tl.n - 1) / tl.n, tiles = mt * nt * q.batch;
         for (int s = 1; s <= (may_split ? 32 : 1); s = s < 4 ? s + 1 : s + s / 2) {

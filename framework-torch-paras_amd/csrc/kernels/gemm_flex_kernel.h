@@ -143,10 +143,17 @@ __global__ __launch_bounds__(kThreads, (MI * NJ >= 32 || ST * (MI + NJ) > 20 ? 1
     }
 }
 
-// Tile forms, largest first; kTiles in gemm_flex.hip describes them in the same order.
+// Tile forms; kTiles in gemm_flex.hip describes them in the same order.
 template <typename T, bool AR, bool BR>
 void launch_tile(int tile, const Params& p, unsigned grid, hipStream_t s) {
     const dim3 g(grid), t(kThreads);
+    if constexpr (!AR && !BR) {          // (the permuted units of a tile that lies along its rows need widths of 64 or 128)
+        switch (tile) {
+            case 12: hipLaunchKernelGGL((gemm_flex_kernel<T, 8, 7, 2, AR, BR>), g, t, 0, s, p); return;
+            case 13: hipLaunchKernelGGL((gemm_flex_kernel<T, 7, 7, 2, AR, BR>), g, t, 0, s, p); return;
+            case 14: hipLaunchKernelGGL((gemm_flex_kernel<T, 6, 7, 2, AR, BR>), g, t, 0, s, p); return;
+        }
+    }
     switch (tile) {
         case 0: hipLaunchKernelGGL((gemm_flex_kernel<T, 8, 8, 2, AR, BR>), g, t, 0, s, p); break;
         case 1: hipLaunchKernelGGL((gemm_flex_kernel<T, 6, 8, 2, AR, BR>), g, t, 0, s, p); break;

@@ -515,7 +515,8 @@ def test_few_columns_streamed_through_lds(dtype):
 
 @pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])
 @pytest.mark.parametrize("shape", [(81, 64, 40), (105, 80, 968), (63, 968, 1768), (232, 4136, 960), (72, 752, 2880), (1056, 1016, 232), (40, 2808, 2656),
-                                   (1224, 2560, 136), (1816, 2264, 552), (1816, 2264, 768), (2792, 2216, 584), (57, 112, 2632)])
+                                   (1224, 2560, 136), (1816, 2264, 552), (1816, 2264, 768), (2792, 2216, 584), (57, 112, 2632),
+                                   (1500, 14336, 520), (3900, 3576, 1032), (1336, 8056, 584)])
 def test_gemm_tiles_with_several_stages(shape, dtype):
     """Tiles whose operands are requested two or three tiles ahead: one tile of contraction to forty, numbers of them that do
     and do not come in whole turns of the stages, rows and columns cut short, whole and in parts, all three layouts.  Every
