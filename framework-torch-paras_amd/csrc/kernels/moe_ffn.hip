@@ -22,7 +22,9 @@
 // expert are contiguous in the routed order; m-tiles never straddle experts (the grid is sized for the
 // worst case and surplus workgroups exit).
 #include <hip/hip_runtime.h>
+#include <cmath>
 #include <cstdlib>
+#include <type_traits>
 
 #include "core/device_context.h"
 #include "core/device_math.h"
@@ -442,6 +444,175 @@ __global__ __launch_bounds__(flex::kThreads, 1) void grouped_gemm_direct_kernel(
     else                 tile(std::integral_constant<int, 2>{});
 }
 
+// ---- experts of a few dozen to a few hundred rows: tiles of 32 MI rows on the staged mainloop of gemm_flex.h, with enough
+// stages in flight that one or two workgroups per CU do not wait for each tile's way from L2, which is what bounds these sizes (the
+// register-staged 128-row tiles that they replace had one tile under way).
+// The weight rows of a tile are 32 NJ columns of the result or, for gate and up, 16 NJ of each: of a wave's NJ blocks of 16 the
+// first half are gate rows and the second half the up rows of the same columns, so that both accumulators of an output belong to one lane.
+template <int NJ> struct GateUp : flex::Operand<NJ, false> {
+    const char* base2;
+    struct Rsrc { __amdgpu_buffer_rsrc_t g[2]; };
+    __device__ __forceinline__ void aim(const std::uint16_t* gate, const std::uint16_t* up, long K, long rows_left, int w) {
+        static_assert(NJ % 4 == 0, "a request of 32 rows belongs to one of the two");
+        const int lane = threadIdx.x & 63, l16 = lane & 15, kq = lane >> 4;
+        this->base = reinterpret_cast<const char*>(gate);
+        base2 = reinterpret_cast<const char*>(up);
+        this->left = rows_left * K * 2;
+        this->step = kBK * 2;
+#pragma unroll
+        for (int i = 0; i < NJ; ++i) {
+            const int r = (i * 4 + flex::wave_id()) * 8 + (lane >> 3), block = (r >> 4) % NJ;
+            const long row = ((r >> 4) / NJ * (NJ / 2) + block % (NJ / 2)) * 16 + (r & 15);
+            this->off[i] = static_cast<std::uint32_t>(row * K * 2 + ((lane & 7) ^ (lane >> 3)) * 16);
+        }
+#pragma unroll
+        for (int ks = 0; ks < 2; ++ks) this->fb[ks] = (w * 16 * NJ + l16) * kBK + ((ks * 4 + kq) ^ (l16 & 7)) * 8;
+    }
+    __device__ __forceinline__ Rsrc rsrc(int kt, int k_tiles) const {
+        const long l = this->left - kt * this->step;
+        const int n = static_cast<int>(static_cast<std::uint32_t>(l < 0 || kt >= k_tiles ? 0 : (l > flex::kMaxExtent ? flex::kMaxExtent : l)));
+        return {{__builtin_amdgcn_make_buffer_rsrc(const_cast<char*>(this->base + kt * this->step), 0, n, 0x00020000),
+                 __builtin_amdgcn_make_buffer_rsrc(const_cast<char*>(base2 + kt * this->step), 0, n, 0x00020000)}};
+    }
+    __device__ __forceinline__ void request(const Rsrc& r, std::uint16_t* tile, int i) const {
+        flex::Operand<NJ, false>::request((2 * i) % NJ >= NJ / 2 ? r.g[1] : r.g[0], tile, i);
+    }
+};
+
+// The m-tile's expert and rows, m-tiles of kBM rows counted expert by expert: every lane looks at one expert (64 at a time; one
+// after the other the offsets of 64 experts are 64 round trips before a workgroup's first load).  False: past the last tile.
+__device__ __forceinline__ bool find_tile(const FfnGemmParams& p, int mt, int kBM, int* e, long* row0, long* row_end) {
+    const int lane = threadIdx.x & 63;
+    int before = 0;
+    for (int e0 = 0; e0 < p.E; e0 += 64) {
+        const int i = e0 + lane;
+        const int lo = i < p.E ? static_cast<int>(p.offsets[i]) : 0, hi = i < p.E ? static_cast<int>(p.offsets[i + 1]) : 0;
+        const int tiles = (hi - lo + kBM - 1) / kBM;
+        int sum = tiles;
+#pragma unroll
+        for (int d = 1; d < 64; d <<= 1) {
+            const int o = __shfl_up(sum, d, 64);
+            if (lane >= d) sum += o;
+        }
+        const int first = before + sum - tiles;
+        const unsigned long long here = __builtin_amdgcn_ballot_w64(mt >= first && mt < first + tiles);
+        if (here != 0) {
+            const int l = __builtin_ctzll(here);
+            *e = e0 + l;
+            *row_end = __builtin_amdgcn_readlane(hi, l);
+            *row0 = __builtin_amdgcn_readlane(lo, l) + static_cast<long>(mt - __builtin_amdgcn_readlane(first, l)) * kBM;
+            return true;
+        }
+        before += __builtin_amdgcn_readlane(sum, 63);
+    }
+    return false;
+}
+
+__device__ __forceinline__ unsigned scalar_of(unsigned v) { return static_cast<unsigned>(__builtin_amdgcn_readfirstlane(static_cast<int>(v))); }
+constexpr int kTileBand = 8;        // m-tiles whose column units an XCD walks through together: they share the experts' weights in its L2
+
+template <typename T, bool kSwiglu, int MI, int NJ, int ST>
+__global__ __launch_bounds__(flex::kThreads, (MI * NJ >= 32 || ST * (MI + NJ) > 20 ? 1 : 2)) void grouped_tile_kernel(const FfnGemmParams p) {
+    using El = Elem<T>;
+    using OA = flex::Operand<MI, false>;
+    using OB = typename std::conditional<kSwiglu, GateUp<NJ>, flex::Operand<NJ, false>>::type;
+    constexpr int kBM = 32 * MI, kCols = kSwiglu ? 16 * NJ : 32 * NJ;
+    __shared__ __attribute__((aligned(1024))) std::uint16_t a0[OA::kElems];
+    __shared__ __attribute__((aligned(1024))) std::uint16_t a1[OA::kElems];
+    __shared__ __attribute__((aligned(1024))) std::uint16_t a2[OA::kElems];     // (stages past ST are never named, and take no memory)
+    __shared__ __attribute__((aligned(1024))) std::uint16_t a3[OA::kElems];
+    __shared__ __attribute__((aligned(1024))) std::uint16_t b0[OB::kElems];
+    __shared__ __attribute__((aligned(1024))) std::uint16_t b1[OB::kElems];
+    __shared__ __attribute__((aligned(1024))) std::uint16_t b2[OB::kElems];
+    __shared__ __attribute__((aligned(1024))) std::uint16_t b3[OB::kElems];
+    // Workgroup w runs on XCD w % 8: every XCD takes a contiguous run of the list of tiles
+    int mt, nu;
+    {
+        const unsigned total = gridDim.x, q = total / 8, r = total % 8, x = blockIdx.x % 8;
+        const unsigned lin = x * q + (x < r ? x : r) + blockIdx.x / 8;
+        const unsigned band = scalar_of(lin / (kTileBand * static_cast<unsigned>(p.n_units))), in = lin - band * kTileBand * static_cast<unsigned>(p.n_units);
+        const unsigned left = static_cast<unsigned>(p.mt_total) - band * kTileBand, rows = left < kTileBand ? left : kTileBand;
+        nu = static_cast<int>(scalar_of(in / rows));
+        mt = static_cast<int>(band * kTileBand + (in - static_cast<unsigned>(nu) * rows));
+    }
+    int e = 0;
+    long row0 = 0, row_end = 0;
+    if (!find_tile(p, mt, kBM, &e, &row0, &row_end)) return;
+    const long n0 = static_cast<long>(nu) * kCols;
+    const int lane = threadIdx.x & 63, wave = flex::wave_id(), l16 = lane & 15, kq = lane >> 4;
+    const int wm = wave >> 1, wn = wave & 1;
+
+    OA oa;          // rows past the expert's last are not fetched (their results are not stored)
+    oa.base = reinterpret_cast<const char*>(p.order ? p.a : p.a + row0 * p.K);
+    oa.left = p.order ? p.a_bytes : (row_end - row0) * p.K * 2;
+    oa.step = kBK * 2;
+#pragma unroll
+    for (int i = 0; i < MI; ++i) {
+        const long r = (i * 4 + wave) * 8 + (lane >> 3);
+        const bool live = row0 + r < row_end;
+        long src = r;
+        if (p.order) src = static_cast<long>((static_cast<unsigned long long>(static_cast<unsigned>(p.order[live ? row0 + r : row0])) * p.div_m) >> p.div_s);
+        oa.off[i] = live ? static_cast<std::uint32_t>(src * p.K * 2 + ((lane & 7) ^ (lane >> 3)) * 16) : flex::kOutOfRange;
+    }
+#pragma unroll
+    for (int ks = 0; ks < 2; ++ks) oa.fb[ks] = (wm * 16 * MI + l16) * kBK + ((ks * 4 + kq) ^ (l16 & 7)) * 8;
+    OB ob;
+    const long first = static_cast<long>(e) * p.Nw * p.K;
+    if constexpr (kSwiglu) ob.aim(p.b + first + n0 * p.K, p.b2 + first + n0 * p.K, p.K, p.Nw - n0, wn);
+    else                   ob.init(p.b + first, p.K, p.Nw, n0, 0, p.K, wn);
+    flex::float4v acc[MI][NJ];
+    const int K = static_cast<int>(p.K);
+    if constexpr (ST == 2)      flex::mainloop<T, MI, NJ, 2>(oa, ob, K, {a0, a1}, {b0, b1}, acc);
+    else if constexpr (ST == 3) flex::mainloop<T, MI, NJ, 3>(oa, ob, K, {a0, a1, a2}, {b0, b1, b2}, acc);
+    else                        flex::mainloop<T, MI, NJ, 4>(oa, ob, K, {a0, a1, a2, a3}, {b0, b1, b2, b3}, acc);
+
+    auto put = [&](long prow, long col, const std::uint16_t (&o)[4]) __attribute__((always_inline)) {
+        if (prow >= row_end || col >= p.N) return;          // (N is a multiple of 64 here and the rows are 16-byte aligned)
+        u32x2 w2;
+        w2[0] = o[0] | (static_cast<std::uint32_t>(o[1]) << 16);
+        w2[1] = o[2] | (static_cast<std::uint32_t>(o[3]) << 16);
+        *reinterpret_cast<u32x2*>(p.c + prow * p.N + col) = w2;
+    };
+#pragma unroll
+    for (int i = 0; i < MI; ++i) {
+        const long prow = row0 + wm * 16 * MI + i * 16 + l16;
+        if constexpr (kSwiglu) {
+#pragma unroll
+            for (int j = 0; j < NJ / 2; ++j) {
+                std::uint16_t o[4];
+                const bool ok = swiglu4_common_tier<T>(acc[i][j], acc[i][NJ / 2 + j], o);
+                if (!ok && prow < row_end) {
+#pragma unroll 1
+                    for (int r = 0; r < 4; ++r) {
+                        const float g = r < 2 ? (r == 0 ? acc[i][j][0] : acc[i][j][1]) : (r == 2 ? acc[i][j][2] : acc[i][j][3]);
+                        const float u = r < 2 ? (r == 0 ? acc[i][NJ / 2 + j][0] : acc[i][NJ / 2 + j][1]) : (r == 2 ? acc[i][NJ / 2 + j][2] : acc[i][NJ / 2 + j][3]);
+                        const std::uint16_t v = swiglu_from_acc<T>(g, u);
+                        o[0] = r == 0 ? v : o[0];
+                        o[1] = r == 1 ? v : o[1];
+                        o[2] = r == 2 ? v : o[2];
+                        o[3] = r == 3 ? v : o[3];
+                    }
+                }
+                put(prow, n0 + wn * 8 * NJ + j * 16 + 4 * kq, o);
+            }
+        } else {
+            float probe = 0.f;
+#pragma unroll
+            for (int j = 0; j < NJ; ++j)
+#pragma unroll
+                for (int r = 0; r < 4; ++r) probe += acc[i][j][r];
+            const bool nan_here = __builtin_amdgcn_ballot_w64(probe != probe) != 0;      // (an infinity minus an infinity counts as well)
+#pragma unroll
+            for (int j = 0; j < NJ; ++j) {
+                std::uint16_t o[4];
+#pragma unroll
+                for (int r = 0; r < 4; ++r) o[r] = __builtin_expect(nan_here, 0) ? El::from_f32(acc[i][j][r]) : El::from_f32_finite(acc[i][j][r]);
+                put(prow, n0 + wn * 16 * NJ + j * 16 + 4 * kq, o);
+            }
+        }
+    }
+}
+
 // ---- few rows per expert (decode-time batches): the layer is bound by streaming every active
 // expert's weights once, which 128-row tiles with a handful of live rows do at half the memory
 // rate (and a single token, two active experts, at a fifth of it: its down-projection is 32
@@ -639,6 +810,70 @@ int run_ffn_any(const void* x, const void* w_gate, const void* w_up, const void*
     return PARAS_OK;
 }
 
+// The tiles of a grouped product: rows, weight rows, stages, workgroups a CU holds, and for the gate-up product and the plain one the time
+// in us of 64 contraction steps on a CU that is full (`step`) and at least (`lat`).  The last is grouped_gemm_direct_kernel.
+struct GroupedForm { int m, n, stages, per_cu; double step[2], lat[2]; };
+constexpr GroupedForm kForms[] = {{128, 128, 2, 2, {1.165, 0.99}, {0.68, 0.48}}, {128, 128, 3, 1, {0.66, 0.38}, {0.29, 0.02}}, {64, 128, 2, 3, {0.96, 0.90}, {0.53, 0.42}},
+                                  {64, 128, 4, 1, {0.43, 0.26}, {0.43, 0.26}},  {32, 128, 4, 2, {0.38, 0.33}, {0.16, 0.07}}, {256, 256, 2, 1, {1.22, 1.02}, {0.30, 0.30}}};
+constexpr int kFormCount = sizeof(kForms) / sizeof(kForms[0]), kDirectForm = kFormCount - 1;
+
+// The least estimated time: rounds of workgroups times their contraction and stores, or the way of the weights from memory, or
+// that of all tiles' operands from the caches, whichever is longest.  (How the rows are spread over the experts is known on the device only: half
+// an empty tile per expert, one tile where an expert has less than two thirds of one.)  Fitted to 1900 timings of 160 layers (8 to 8192
+// tokens, 4 to 64 experts, H 512 to 4096, I 512 to 14336), over which the choice is 3 % (gate-up) and 4 % (down) slower than the best form in the
+// mean.  Against 128-row tiles staged through registers, and 256-row tiles from 1024 rows per expert on, as before: gate-up 1.4 times and down
+// 1.8 times as fast in the mean; T 1202, 8 experts, top-2, H 576, I 12416: 160 -> @a us and 247 -> @b.
+int grouped_form(bool swiglu, long E, long R, long N, long K) {
+    const int w = swiglu ? 0 : 1;
+    const double start = swiglu ? 3.7 : 1.8, store = swiglu ? 19.5 : 9.9, rows = static_cast<double>(R) / E, used = R < E ? R : E;
+    const double memory = used * N * K * (swiglu ? 4.0 / 4.42e6 : 2.0 / 4.02e6) + (swiglu ? 2.4 : 0.9), cached = swiglu ? 15.2e6 : 12.9e6;
+    int best = 0;
+    double best_us = 1e30;
+    for (int f = 0; f < kFormCount; ++f) {
+        const GroupedForm& t = kForms[f];
+        const long cols = swiglu ? t.n / 2 : t.n, units = (N + cols - 1) / cols, k_tiles = K / kBK, turns = (k_tiles + t.stages - 1) / t.stages * t.stages;
+        const double m_tiles = rows < 0.7 * t.m ? used : E * (rows / t.m + 0.5), tiles = m_tiles * units;
+        auto round = [&](double n) {
+            const double c = t.step[w] * n / t.per_cu;
+            return turns * (c > t.lat[w] ? c : t.lat[w]) + start + store * t.m * cols / 65536.0 * n;
+        };
+        double us;
+        if (f == kDirectForm) {          // super-tiles of 32 workgroups, dealt to the 8 XCDs
+            us = std::ceil(std::ceil(m_tiles / kSuperM) * std::ceil(static_cast<double>(units) / kSuperN) / 8) * round(1.0);
+        } else {
+            const double slots = 256.0 * t.per_cu, full = std::floor(tiles / slots), rest = std::ceil((tiles - full * slots) / 256.0);
+            us = full * round(t.per_cu) + (rest > 0 ? round(rest) : 0.0);
+        }
+        const double traffic = tiles * (t.m + t.n) * K * 2.0 / cached;
+        us = us > memory ? us : memory;
+        us = us > traffic ? us : traffic;
+        if (us < best_us) {
+            best_us = us;
+            best = f;
+        }
+    }
+    return best;
+}
+
+template <typename T, bool kSwiglu>
+void launch_form(int form, FfnGemmParams g, hipStream_t s) {
+    const GroupedForm f = kForms[form];
+    const long cols = kSwiglu ? f.n / 2 : f.n;
+    g.mt_total = static_cast<int>((g.R + f.m - 1) / f.m + (g.R < g.E ? g.R : g.E));      // an upper bound: workgroups past the last tile return
+    g.n_units = static_cast<int>((g.N + cols - 1) / cols);
+    const dim3 block(flex::kThreads), grid(static_cast<unsigned>(static_cast<long>(g.mt_total) * g.n_units));
+    const long supers = static_cast<long>((g.mt_total + kSuperM - 1) / kSuperM) * ((g.n_units + kSuperN - 1) / kSuperN);
+    switch (form) {
+        case 0: hipLaunchKernelGGL((grouped_tile_kernel<T, kSwiglu, 4, 4, 2>), grid, block, 0, s, g); break;
+        case 1: hipLaunchKernelGGL((grouped_tile_kernel<T, kSwiglu, 4, 4, 3>), grid, block, 0, s, g); break;
+        case 2: hipLaunchKernelGGL((grouped_tile_kernel<T, kSwiglu, 2, 4, 2>), grid, block, 0, s, g); break;
+        case 3: hipLaunchKernelGGL((grouped_tile_kernel<T, kSwiglu, 2, 4, 4>), grid, block, 0, s, g); break;
+        case 4: hipLaunchKernelGGL((grouped_tile_kernel<T, kSwiglu, 1, 4, 4>), grid, block, 0, s, g); break;
+        default:
+            hipLaunchKernelGGL((grouped_gemm_direct_kernel<T, kSwiglu>), dim3(static_cast<unsigned>((supers + 7) / 8 * 8 * kSuperM * kSuperN)), block, 0, s, g);
+    }
+}
+
 template <typename T, typename S>
 int run_ffn_shape(const void* x, const void* w_gate, const void* w_up, const void* w_down, const float* topw,
             const long* order, const long* inv_order, const long* offsets, void* out, void* workspace, long T_,
@@ -671,19 +906,12 @@ int run_ffn_shape(const void* x, const void* w_gate, const void* w_up, const voi
         const long groups = (g.n_units + 8 * g.ngt - 1) / (8 * g.ngt);
         return static_cast<unsigned>(groups * 8 * g.ngt * g.mt_total);
     };
-    auto direct_grid_of = [](const FfnGemmParams& g) {
-        const long supers = static_cast<long>((g.mt_total + kSuperM - 1) / kSuperM) * ((g.n_units + kSuperN - 1) / kSuperN);
-        return static_cast<unsigned>((supers + 7) / 8 * 8 * kSuperM * kSuperN);
-    };
     plan(g1);
-    // 256-row tiles: the four-wave tile of 16 x 16 x 32 MFMAs (PARAS_GEMM_EIGHT_WAVES: the eight-wave tile of
-    // 32 x 32 x 16 ones, for measurements)
+    // By form (grouped_form), unless rows or weights are out of a 32-bit byte offset's reach, from the start of x and from a
+    // tile's first weight row (PARAS_GEMM_EIGHT_WAVES: the eight-wave tile of 32 x 32 x 16 MFMAs where it applies, for measurements).
     static const bool eight_waves = std::getenv("PARAS_GEMM_EIGHT_WAVES") != nullptr;
-    constexpr bool kBig = S::kBM == 256;
-    // (its gathered rows are reached by 32-bit byte offsets from the start of x, its weight rows from the tile's first)
-    const bool direct = kBig && !eight_waves && T_ * H * 2 <= flex::kMaxExtent && H <= flex::kMaxLd && I <= flex::kMaxLd;
-    if (direct)
-        hipLaunchKernelGGL((grouped_gemm_direct_kernel<T, true>), dim3(direct_grid_of(g1)), dim3(flex::kThreads), 0, s, g1);
+    const bool by_form = !(eight_waves && S::kBM == 256) && T_ * H * 2 <= flex::kMaxExtent && H <= flex::kMaxLd && I <= flex::kMaxLd;
+    if (by_form) launch_form<T, true>(grouped_form(true, E, R, I, H), g1, s);
     else
         hipLaunchKernelGGL((grouped_gemm_kernel<T, true, S>), dim3(grid_of(g1)), dim3(S::kThreads), 0, s, g1);
     PARAS_HIP_TRY(hipGetLastError());
@@ -699,8 +927,7 @@ int run_ffn_shape(const void* x, const void* w_gate, const void* w_up, const voi
     g2.mt_total = mt_total;
     g2.n_units = static_cast<int>((H + 2 * kBN - 1) / (2 * kBN));
     plan(g2);
-    if (direct)
-        hipLaunchKernelGGL((grouped_gemm_direct_kernel<T, false>), dim3(direct_grid_of(g2)), dim3(flex::kThreads), 0, s, g2);
+    if (by_form) launch_form<T, false>(grouped_form(false, E, R, H, I), g2, s);
     else
         hipLaunchKernelGGL((grouped_gemm_kernel<T, false, S>), dim3(grid_of(g2)), dim3(S::kThreads), 0, s, g2);
     PARAS_HIP_TRY(hipGetLastError());
@@ -767,12 +994,12 @@ int run_ffn(const void* x, const void* w_gate, const void* w_up, const void* w_d
             const long* order, const long* inv_order, const long* offsets, void* out, void* workspace, long T_,
             int E, int k, long H, long I, hipStream_t s) {
     const long R = T_ * k;
-    // Up to 16 routed rows per expert on average the few-row kernels (an expert with more than 32 rows
-    // takes them 32 at a time).  8 experts, top-2, H = 4096, I = 14336, tiles against few-row kernels:
-    // 1 token 421 / 138 us, 16 tokens 630 / 484, 64 tokens 663 / 557 (128 tokens, where every expert's weights
-    // are read twice from L2: tiles, 672).  PARAS_MOE_FEW_ROWS = n moves the limit (0: never).
+    // Few routed rows per expert on average: the few-row kernels (an expert with more than 32 rows takes them 32 at a time).  Up to 8, and
+    // up to 16 where the weights are long enough for their stream to decide.  Few-row kernels / tiles: 8 experts, top-2, H 4096,
+    // I 14336 40 tokens 480 / 551 us, 64 tokens 528 / 544, 128 tokens 823 / 602; H 1216, I 512 57 tokens 16 / 8; 64 experts, top-6, H 576,
+    // I 10944 133 tokens 587 / 516; 16 experts H 832, I 3776 61 tokens (8 rows each) 68 / 60.  PARAS_MOE_FEW_ROWS = n moves the limit (0: never).
     static const char* few_env = std::getenv("PARAS_MOE_FEW_ROWS");
-    const long few_limit = few_env != nullptr ? std::atol(few_env) : 16;
+    const long few_limit = few_env != nullptr ? std::atol(few_env) : (H * I >= 20'000'000L ? 16 : 8);
     if (R <= few_limit * E && E <= 65535 && T_ * H * 2 <= stream::kMaxExtent && R * I * 2 <= stream::kMaxExtent)
         return run_ffn_few_rows<T>(x, w_gate, w_up, w_down, topw, order, inv_order, offsets, out, workspace, T_, E, k, H, I, s);
     const long wide_tiles = (R / Tile256::kBM) * ((H + 2 * kBN - 1) / (2 * kBN));

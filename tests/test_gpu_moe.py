@@ -418,3 +418,39 @@ def test_route_recorded_into_a_graph_and_replayed():
         for name, g, e, w in zip(NAMES, recorded, eager, want):
             assert_bit_exact(g, w, f"replay {trial}: moe_route {name}")
             assert_bit_exact(e, w, f"eager call {trial}: moe_route {name}")
+
+
+# (gate-up and down between them run on every tile form: 128-row ones with two and three stages, 64-row ones with two and four, 32- and 256-row ones)
+TILE_SHAPES = [(1843, 70, 6, 192, 256), (2055, 32, 4, 192, 192), (1188, 70, 6, 192, 192), (2555, 70, 6, 128, 192), (395, 70, 6, 640, 192), (167, 32, 4, 704, 384),
+               (727, 70, 6, 576, 192), (163, 70, 6, 192, 128), (159, 70, 6, 320, 768), (2778, 70, 6, 960, 448), (45, 4, 1, 256, 320), (2769, 70, 6, 192, 512)]
+
+
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])
+@pytest.mark.parametrize("shape", TILE_SHAPES)
+def test_ffn_tiles_of_every_form(shape, dtype):
+    """Experts of a few to a few hundred rows, uneven: one that most tokens choose, some that nobody does, more experts than a
+    wave has lanes; gates far from zero (SwiGLU's exact tier), a NaN, an infinite and an all-zero token.  Sampled tokens against the
+    oracle, and no other token touched by the NaN."""
+    T, E, k, H, I = shape
+    torch.manual_seed(T + E)
+    logits = torch.randn(T, E)
+    logits[:, E // 2] += 3.0
+    logits[:, E - 1] -= 20.0
+    logits[:, 0] -= 20.0 if k < E - 2 else 0.0
+    logits = logits.to(dtype)
+    x = torch.randn(T, H).to(dtype)
+    x[5, 3], x[T // 2, 10], x[T - 2] = float("nan"), float("inf"), 0
+    wg, wu = (0.4 * torch.randn(E, I, H)).to(dtype), (0.05 * torch.randn(E, I, H)).to(dtype)
+    wd = (0.02 * torch.randn(E, H, I)).to(dtype)
+    topi, topw, order, inv, counts, offsets = capi.moe_route(logits.cuda(), k)
+    out = capi.moe_ffn(x.cuda(), wg.cuda(), wu.cuda(), wd.cuda(), topw, order, inv, offsets, k).cpu()
+    sel = torch.cat([torch.tensor([0, 5, T // 2, T - 2, T - 1]), torch.randperm(T)[:40]])
+    r = O.moe_route(logits[sel], k)
+    ref = O.moe_ffn(x[sel], wg, wu, wd, r[1], r[2], r[3], r[5], k, gemm="aten")
+    got = out[sel]
+    assert torch.equal(got.isnan(), ref.isnan()) and torch.equal(got[3], torch.zeros(H, dtype=dtype))
+    fin = ref.isfinite().all(dim=1)
+    assert int(fin.sum()) >= 35
+    assert_ffn_close(got[fin], ref[fin], dtype)
+    bad = set((~out.isfinite()).any(dim=1).nonzero().flatten().tolist())
+    assert {5} <= bad <= {5, T // 2}
