@@ -248,6 +248,54 @@ struct TwoGroups : flex::Operand<8, false> {
     }
 };
 
+// The experts' m-tiles, counted expert by expert: every lane looks at one expert (64 at a time; one after the other the offsets of
+// 64 experts are 64 round trips before a workgroup's first load).  `tiles_of(rows)`: the tiles of an expert with that many.
+struct ExpertTiles {
+    int lo, hi, tiles, upto;        // of 64 experts, by lane: rows [lo, hi), tiles, and those of the 64 up to this one
+    template <typename Tiles> __device__ __forceinline__ void look(const FfnGemmParams& p, int e0, Tiles tiles_of) {
+        const int lane = threadIdx.x & 63, i = e0 + lane;
+        lo = i < p.E ? static_cast<int>(p.offsets[i]) : 0;
+        hi = i < p.E ? static_cast<int>(p.offsets[i + 1]) : 0;
+        count(tiles_of);
+    }
+    template <typename Tiles> __device__ __forceinline__ void count(Tiles tiles_of) {
+        tiles = tiles_of(hi - lo);
+        upto = tiles;
+#pragma unroll
+        for (int d = 1; d < 64; d <<= 1) {
+            const int o = __shfl_up(upto, d, 64);
+            if (static_cast<int>(threadIdx.x & 63) >= d) upto += o;
+        }
+    }
+    __device__ __forceinline__ int all() const { return __builtin_amdgcn_readlane(upto, 63); }
+};
+
+// `head`: experts 0 to 63
+template <typename Tiles> __device__ __forceinline__ int count_tiles(const FfnGemmParams& p, const ExpertTiles& head, Tiles tiles_of) {
+    int n = head.all();
+    for (int e0 = 64; e0 < p.E; e0 += 64) {
+        ExpertTiles more;
+        more.look(p, e0, tiles_of);
+        n += more.all();
+    }
+    return n;
+}
+
+// m-tile `mt`, one of those counted: its expert, that expert's rows and which of its tiles it is
+struct TileOf { int e, lo, hi, nth; };
+template <typename Tiles> __device__ __forceinline__ TileOf find_tile(const FfnGemmParams& p, int mt, const ExpertTiles& head, Tiles tiles_of) {
+    ExpertTiles at = head;
+    int before = 0, e0 = 0;
+    while (e0 + 64 < p.E && mt >= before + at.all()) {
+        before += at.all();
+        e0 += 64;
+        at.look(p, e0, tiles_of);
+    }
+    const int first = before + at.upto - at.tiles;
+    const int l = __builtin_ctzll(__builtin_amdgcn_ballot_w64(mt >= first && mt < first + at.tiles) | 1ull << 63);
+    return {e0 + l, __builtin_amdgcn_readlane(at.lo, l), __builtin_amdgcn_readlane(at.hi, l), mt - __builtin_amdgcn_readlane(first, l)};
+}
+
 // The same on the four-wave 256 x 256 tile of v_mfma_f32_16x16x32 whose loads go straight to LDS (gemm_flex.h): what the
 // layer runs on when the experts are big enough for 256-row tiles.  Tile coordinates and the search for the
 // m-tile's expert as above; the routed rows are gathered by the addresses the lanes fetch from.  A lane of accumulator
@@ -279,25 +327,26 @@ __global__ __launch_bounds__(flex::kThreads, 1) void grouped_gemm_direct_kernel(
     }
     // m-tile -> (expert, first row): first every expert's tiles with more than 64 rows, then the short last ones, which
     // take a fraction of the time and fill in at the end of every XCD's list
-    int e = 0;
-    long row0 = 0, row_end = 0;
+    int e;
+    long row0, row_end;
     {
-        int left = mt;
-        bool found = false;
-        for (int pass = 0; pass < 2 && !found; ++pass)
-            for (int i = 0; i < p.E && !found; ++i) {
-                const long lo = p.offsets[i], hi = p.offsets[i + 1];
-                const long full = (hi - lo) / kBM, over = (hi - lo) - full * kBM;
-                const int tiles = pass == 0 ? static_cast<int>(full) + (over > 64) : (over > 0 && over <= 64);
-                if (left < tiles) {
-                    e = i;
-                    row0 = lo + (pass == 0 ? left : full) * kBM;
-                    row_end = hi;
-                    found = true;
-                }
-                left -= tiles;
-            }
-        if (!found) return;
+        auto whole = [](int rows) { return rows / kBM + (rows % kBM > 64); };
+        auto ends = [](int rows) { return static_cast<int>(rows % kBM > 0 && rows % kBM <= 64); };
+        ExpertTiles head;
+        head.look(p, 0, whole);
+        const int n_whole = count_tiles(p, head, whole);
+        TileOf at;
+        if (mt < n_whole) {
+            at = find_tile(p, mt, head, whole);
+        } else {
+            head.count(ends);
+            if (mt - n_whole >= count_tiles(p, head, ends)) return;
+            at = find_tile(p, mt - n_whole, head, ends);
+            at.nth = (at.hi - at.lo) / kBM;
+        }
+        e = at.e;
+        row0 = at.lo + static_cast<long>(at.nth) * kBM;
+        row_end = at.hi;
     }
     const long n0 = static_cast<long>(nu) * (kSwiglu ? kBN : 2 * kBN);
     const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
@@ -479,35 +528,6 @@ template <int NJ> struct GateUp : flex::Operand<NJ, false> {
     }
 };
 
-// The m-tile's expert and rows, m-tiles of kBM rows counted expert by expert: every lane looks at one expert (64 at a time; one
-// after the other the offsets of 64 experts are 64 round trips before a workgroup's first load).  False: past the last tile.
-__device__ __forceinline__ bool find_tile(const FfnGemmParams& p, int mt, int kBM, int* e, long* row0, long* row_end) {
-    const int lane = threadIdx.x & 63;
-    int before = 0;
-    for (int e0 = 0; e0 < p.E; e0 += 64) {
-        const int i = e0 + lane;
-        const int lo = i < p.E ? static_cast<int>(p.offsets[i]) : 0, hi = i < p.E ? static_cast<int>(p.offsets[i + 1]) : 0;
-        const int tiles = (hi - lo + kBM - 1) / kBM;
-        int sum = tiles;
-#pragma unroll
-        for (int d = 1; d < 64; d <<= 1) {
-            const int o = __shfl_up(sum, d, 64);
-            if (lane >= d) sum += o;
-        }
-        const int first = before + sum - tiles;
-        const unsigned long long here = __builtin_amdgcn_ballot_w64(mt >= first && mt < first + tiles);
-        if (here != 0) {
-            const int l = __builtin_ctzll(here);
-            *e = e0 + l;
-            *row_end = __builtin_amdgcn_readlane(hi, l);
-            *row0 = __builtin_amdgcn_readlane(lo, l) + static_cast<long>(mt - __builtin_amdgcn_readlane(first, l)) * kBM;
-            return true;
-        }
-        before += __builtin_amdgcn_readlane(sum, 63);
-    }
-    return false;
-}
-
 __device__ __forceinline__ unsigned scalar_of(unsigned v) { return static_cast<unsigned>(__builtin_amdgcn_readfirstlane(static_cast<int>(v))); }
 constexpr int kTileBand = 8;        // m-tiles whose column units an XCD walks through together: they share the experts' weights in its L2
 
@@ -525,19 +545,26 @@ __global__ __launch_bounds__(flex::kThreads, (MI * NJ >= 32 || ST * (MI + NJ) > 
     __shared__ __attribute__((aligned(1024))) std::uint16_t b1[OB::kElems];
     __shared__ __attribute__((aligned(1024))) std::uint16_t b2[OB::kElems];
     __shared__ __attribute__((aligned(1024))) std::uint16_t b3[OB::kElems];
-    // Workgroup w runs on XCD w % 8: every XCD takes a contiguous run of the list of tiles
+    // Workgroup w runs on XCD w % 8: every XCD takes a contiguous run of the list of tiles.  Of the tiles that there are: the grid has room for
+    // any spread of the rows, and with runs of that room the last XCDs have nothing
+    // (64 experts, 150 layers: 1.15 to 1.2 times the time; 8 experts: 1.07 to 1.1 times).
+    auto tiles_of = [](int rows) { return (rows + kBM - 1) / kBM; };
+    ExpertTiles head;
+    head.look(p, 0, tiles_of);
+    const unsigned m_tiles = static_cast<unsigned>(count_tiles(p, head, tiles_of)), units = static_cast<unsigned>(p.n_units);
     int mt, nu;
     {
-        const unsigned total = gridDim.x, q = total / 8, r = total % 8, x = blockIdx.x % 8;
-        const unsigned lin = x * q + (x < r ? x : r) + blockIdx.x / 8;
-        const unsigned band = scalar_of(lin / (kTileBand * static_cast<unsigned>(p.n_units))), in = lin - band * kTileBand * static_cast<unsigned>(p.n_units);
-        const unsigned left = static_cast<unsigned>(p.mt_total) - band * kTileBand, rows = left < kTileBand ? left : kTileBand;
+        const unsigned total = m_tiles * units, q = total / 8, r = total % 8, x = blockIdx.x % 8, i = blockIdx.x / 8;
+        if (i >= q + (x < r ? 1 : 0)) return;
+        const unsigned lin = x * q + (x < r ? x : r) + i;
+        const unsigned band = scalar_of(lin / (kTileBand * units)), in = lin - band * kTileBand * units;
+        const unsigned left = m_tiles - band * kTileBand, rows = left < kTileBand ? left : kTileBand;
         nu = static_cast<int>(scalar_of(in / rows));
         mt = static_cast<int>(band * kTileBand + (in - static_cast<unsigned>(nu) * rows));
     }
-    int e = 0;
-    long row0 = 0, row_end = 0;
-    if (!find_tile(p, mt, kBM, &e, &row0, &row_end)) return;
+    const TileOf at = find_tile(p, mt, head, tiles_of);
+    const int e = at.e;
+    const long row0 = at.lo + static_cast<long>(at.nth) * kBM, row_end = at.hi;
     const long n0 = static_cast<long>(nu) * kCols;
     const int lane = threadIdx.x & 63, wave = flex::wave_id(), l16 = lane & 15, kq = lane >> 4;
     const int wm = wave >> 1, wn = wave & 1;
@@ -813,22 +840,22 @@ int run_ffn_any(const void* x, const void* w_gate, const void* w_up, const void*
 // The tiles of a grouped product: rows, weight rows, stages, workgroups a CU holds, and for the gate-up product and the plain one the time
 // in us of 64 contraction steps on a CU that is full (`step`) and at least (`lat`).  The last is grouped_gemm_direct_kernel.
 struct GroupedForm { int m, n, stages, per_cu; double step[2], lat[2]; };
-constexpr GroupedForm kForms[] = {{128, 128, 2, 2, {1.165, 0.99}, {0.68, 0.48}}, {128, 128, 3, 1, {0.66, 0.38}, {0.29, 0.02}}, {64, 128, 2, 3, {0.96, 0.90}, {0.53, 0.42}},
-                                  {64, 128, 4, 1, {0.43, 0.26}, {0.43, 0.26}},  {32, 128, 4, 2, {0.38, 0.33}, {0.16, 0.07}}, {256, 256, 2, 1, {1.22, 1.02}, {0.30, 0.30}}};
+constexpr GroupedForm kForms[] = {{128, 128, 2, 2, {0.91, 0.78}, {0.66, 0.47}}, {128, 128, 3, 1, {0.54, 0.36}, {0.13, 0.02}}, {64, 128, 2, 3, {0.74, 0.33}, {0.51, 0.42}},
+                                  {64, 128, 4, 1, {0.19, 0.24}, {0.35, 0.23}}, {32, 128, 4, 2, {0.30, 0.07}, {0.15, 0.16}}, {256, 256, 2, 1, {1.13, 0.97}, {0.32, 0.30}}};
 constexpr int kFormCount = sizeof(kForms) / sizeof(kForms[0]), kDirectForm = kFormCount - 1;
 
-// The least estimated time: rounds of workgroups times their contraction and stores, or the way of the weights from memory, or
-// that of all tiles' operands from the caches, whichever is longest.  (How the rows are spread over the experts is known on the device only: half
-// an empty tile per expert, one tile where an expert has less than two thirds of one.)  Fitted to 1900 timings of 160 layers (8 to 8192
-// tokens, 4 to 64 experts, H 512 to 4096, I 512 to 14336), over which the choice is 3 % (gate-up) and 4 % (down) slower than the best form in the
-// mean.  Against 128-row tiles staged through registers, and 256-row tiles from 1024 rows per expert on, as before: gate-up 1.4 times and down
-// 1.8 times as fast in the mean; T 1202, 8 experts, top-2, H 576, I 12416: 160 -> @a us and 247 -> @b.
+// The least estimated time, from three that overlap for the most part (the fourth root of the sum of their fourth powers): rounds of
+// workgroups times their contraction and stores, the way of the weights from memory, and that of all tiles' operands from the caches.  (How
+// the rows are spread over the experts is known on the device only: half an empty tile per expert, one tile where an expert has less than two
+// thirds of one.)  Fitted to 1800 timings of 150 layers (8 to 8192 tokens, 4 to 64 experts, H 512 to 4096, I 512 to 14336), over which the
+// choice is 2 % (gate-up) and 5 % (down) slower than the best form in the mean; always the same form is 15 % and 22 % at the least.
 int grouped_form(bool swiglu, long E, long R, long N, long K) {
     const int w = swiglu ? 0 : 1;
-    const double start = swiglu ? 3.7 : 1.8, store = swiglu ? 19.5 : 9.9, rows = static_cast<double>(R) / E, used = R < E ? R : E;
-    const double memory = used * N * K * (swiglu ? 4.0 / 4.42e6 : 2.0 / 4.02e6) + (swiglu ? 2.4 : 0.9), cached = swiglu ? 15.2e6 : 12.9e6;
+    const double start = swiglu ? 3.9 : 1.3, store = swiglu ? 15.4 : 9.4, rows = static_cast<double>(R) / E, used = R < E ? R : E;
+    const double memory = used * N * K * (swiglu ? 4.0 / 5.34e6 : 2.0 / 5.37e6), cached = swiglu ? 16.4e6 : 14.1e6;
+    auto fourth = [](double v) { return v * v * v * v; };
     int best = 0;
-    double best_us = 1e30;
+    double best_cost = 1e300;
     for (int f = 0; f < kFormCount; ++f) {
         const GroupedForm& t = kForms[f];
         const long cols = swiglu ? t.n / 2 : t.n, units = (N + cols - 1) / cols, k_tiles = K / kBK, turns = (k_tiles + t.stages - 1) / t.stages * t.stages;
@@ -845,10 +872,9 @@ int grouped_form(bool swiglu, long E, long R, long N, long K) {
             us = full * round(t.per_cu) + (rest > 0 ? round(rest) : 0.0);
         }
         const double traffic = tiles * (t.m + t.n) * K * 2.0 / cached;
-        us = us > memory ? us : memory;
-        us = us > traffic ? us : traffic;
-        if (us < best_us) {
-            best_us = us;
+        const double cost = fourth(us) + fourth(memory) + fourth(traffic);
+        if (cost < best_cost) {
+            best_cost = cost;
             best = f;
         }
     }
