@@ -5,6 +5,7 @@ unit in the last place of the 16-bit result where that is larger (|y| >= 4 for
 bf16: a GEMM whose fp32 summation order differs from ATen's flips the final
 rounding of a few outputs, by exactly one ulp)."""
 import ctypes as C
+import math
 
 import pytest
 import torch
@@ -52,6 +53,28 @@ def test_route_quantised_logits_many_ties_and_skew():
     for name, g, w in zip(NAMES, got, want):
         assert_bit_exact(g, w, f"moe_route {name}")
     assert got[4][2].item() == 0 and got[4][5].item() == 3000
+
+
+@pytest.mark.parametrize("shape", [(1, 16, 8), (63, 9, 1), (65, 64, 8), (300, 33, 5), (515, 64, 6), (4099, 32, 4)])
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float32])
+def test_route_of_rows_with_ties_infinities_and_nans(shape, dtype):
+    """Rows held in registers: equal values go to the lower expert, -0 is 0, and a NaN behind the first expert is chosen as little as -inf
+    behind the others (the rows with one go through another selection, in the same wave)."""
+    T, E, k = shape
+    g = torch.Generator().manual_seed(T)
+    logits = torch.randint(-2, 3, (T, E), generator=g).float()
+    logits[torch.rand(T, E, generator=g) < 0.2] = -0.0
+    logits[::3, : E - k] = -math.inf
+    logits[1::5, 0] = math.inf
+    plain = logits.clone().to(dtype)
+    odd = plain.clone()
+    odd[::6, : E - k][:, 1:] = math.nan
+    got = capi.moe_route(odd.cuda(), k)
+    for name, a, b in zip(NAMES, got, O.moe_route(plain, k)):
+        if name == "topw":          # inf - inf
+            assert torch.equal(torch.isnan(a.cpu()), torch.isnan(b))
+            a, b = a.nan_to_num(), b.nan_to_num()
+        assert_bit_exact(a, b, f"moe_route {name} T{T} E{E} k{k} {dtype}")
 
 
 @pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])
