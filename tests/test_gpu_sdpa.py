@@ -656,6 +656,36 @@ def test_decode_with_masks_matches_oracle(dtype):
     assert max_abs(out[[0, 2]], want[[0, 2]]) <= ABS_16BIT
 
 
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])
+@pytest.mark.parametrize("D", [64, 128, 256])
+@pytest.mark.parametrize("shape", [(1, 2, 1, 70001), (3, 4, 4, 515), (2, 3, 3, 161), (5, 1, 1, 33), (1, 1, 1, 2048)])
+def test_decode_of_many_splits_and_of_masks_in_any_layout(dtype, D, shape):
+    """Splits beyond what the combining workgroup holds at once and in numbers that do not divide its groups; mask rows at odd
+    addresses, masks whose keys are strided, one row for all keys, and a ragged last tile (its mask is read element by element)."""
+    B, Hq, Hkv, Lk = shape
+    g = torch.Generator().manual_seed(Lk + D)
+    q, k, v = (torch.randn(B, h, n, D, generator=g).to(dtype) for h, n in ((Hq, 1), (Hkv, Lk), (Hkv, Lk)))
+    rows = torch.rand(B, 1, 1, Lk, generator=g) > 0.4
+    rows[..., -1] = True
+    bias = torch.randn(B, Hq, 1, Lk, generator=g).to(dtype)
+    strided = torch.rand(Lk, B, generator=g).gt(0.4)
+    strided[0] = True
+    masks = [None, rows, bias, strided.t()[:, None, None, :], bias.transpose(0, 3).contiguous().transpose(0, 3), bias[..., :1].expand(B, Hq, 1, Lk)]
+    # The weights and the result are narrowed once each, by at most u of their size; scores and sums are fp32.
+    u = 2.0 ** -8 if dtype == torch.bfloat16 else 2.0 ** -11
+    kd, vd = (x.double().repeat_interleave(Hq // Hkv, 1) for x in (k, v))
+    for i, mask in enumerate(masks):
+        out, _, lse, kern = run(q, k, v, mask=mask, want_lse=True)
+        s = (q.double() @ kd.transpose(-1, -2)) / math.sqrt(D)
+        if mask is not None:
+            s = s.masked_fill(~mask, -math.inf) if mask.dtype == torch.bool else s + mask.double()
+        w = s.softmax(-1)
+        want, size = w @ vd, w @ vd.abs()
+        assert kern == "decode_split"
+        assert bool(((out.double().cpu() - want).abs() <= 1.02 * u * (size + want.abs()) + 1e-5).all()), i
+        assert torch.allclose(lse.double().cpu(), torch.logsumexp(s, -1), rtol=1e-5, atol=1e-4), i
+
+
 def test_generic_handles_odd_heads_masks_and_all_masked_rows():
     q, k, v = torch.randn(1, 3, 5, 24), torch.randn(1, 3, 9, 24), torch.randn(1, 3, 9, 40)
     out, attn, _, kern = run(q, k, v, want_attn=True)                # Dv != D
