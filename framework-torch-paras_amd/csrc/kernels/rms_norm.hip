@@ -71,6 +71,40 @@ __device__ __forceinline__ double rsqrt_f64(double v) {
     return r;
 }
 
+// A 16-byte vector of a row of fp32 values.  kAny: rows of any width at any address of an element; of the row's last vector only the
+// `left` elements that there are (the others read as zeros, which add nothing to a sum of squares).  A 16-byte access to an address that is
+// a multiple of 4 runs at full rate; one that is only a multiple of 2 does not: with rows of 16-bit elements this way 6506 x 9685 took
+// 141 us, 1.8 TB/s, and 2667 x 14377 85 where element by element takes 78.
+typedef std::uint32_t u32x4_any __attribute__((ext_vector_type(4), aligned(4)));
+template <bool kAny, typename S> __device__ __forceinline__ u32x4 load_vec(const S* p, int left) {
+    if constexpr (!kAny) {
+        return load16_nt(p);
+    } else {
+        static_assert(sizeof(S) == 4, "16-bit elements lie at odd addresses of two bytes");
+        if (left >= 4) return __builtin_nontemporal_load(reinterpret_cast<const u32x4_any*>(p));
+        u32x4 v = {0u, 0u, 0u, 0u};
+#pragma unroll
+        for (int j = 0; j < 3; ++j)
+            if (j < left) v[j] = __builtin_bit_cast(std::uint32_t, p[j]);
+        return v;
+    }
+}
+template <bool kAny, typename S> __device__ __forceinline__ void store_vec(S* p, u32x4 v, int left) {
+    if constexpr (!kAny) {
+        store16_nt(p, v);
+    } else {
+        if (left >= 4) {
+            __builtin_nontemporal_store(u32x4_any(v), reinterpret_cast<u32x4_any*>(p));
+            return;
+        }
+#pragma unroll
+        for (int j = 0; j < 3; ++j) {
+            const std::uint32_t e = v[j];        // (a copy: the cast takes an element of a vector for its first one)
+            if (j < left) p[j] = __builtin_bit_cast(S, e);
+        }
+    }
+}
+
 // Register-resident row: H == vectors per row * kVec, vectors per row <= BLOCK*NV.  The workgroup is
 // sized to the row (128 threads for a row of 1024 16-bit elements, 1024 for one of 16384), at most two
 // vectors per thread: four need more than the 64 registers that eight waves per SIMD leave.
@@ -86,7 +120,8 @@ constexpr int fwd_waves_per_simd() {
     if (!PIPE || NV < 2 || __is_same(T, bf16_t)) return 8;
     return __is_same(T, f16_t) ? 6 : 4;
 }
-template <typename T, int NV, int BLOCK, bool PIPE = false>
+// kAny: fp32 rows of any width and alignment.
+template <typename T, int NV, int BLOCK, bool PIPE = false, bool kAny = false>
 __global__ __launch_bounds__((BLOCK == 0 ? 1024 : BLOCK), (fwd_waves_per_simd<T, NV, PIPE>())) void rms_norm_fwd_vec(
     const typename Elem<T>::store_t* __restrict__ x, const typename Elem<T>::store_t* __restrict__ w,
     typename Elem<T>::store_t* __restrict__ out, float* __restrict__ rstd, long rows, int H,
@@ -97,12 +132,16 @@ __global__ __launch_bounds__((BLOCK == 0 ? 1024 : BLOCK), (fwd_waves_per_simd<T,
     __shared__ double slots[2 * ((BLOCK == 0 ? 1024 : BLOCK) / kWave)];
     const int block = BLOCK == 0 ? static_cast<int>(blockDim.x) : BLOCK;
 
-    const int nvec = H / V;  // 16-byte vectors per row
+    const int nvec = kAny ? (H + V - 1) / V : H / V;  // 16-byte vectors per row
     u32x4 wv[NV];
 #pragma unroll
     for (int i = 0; i < NV; ++i) {
         const int c = threadIdx.x + i * block;
-        if (c < nvec) wv[i] = load16(w + static_cast<long>(c) * V);  // shared by every row: an L2 hit
+        if constexpr (kAny) {
+            if (c < nvec) wv[i] = load_vec<true>(w + static_cast<long>(c) * V, H - c * V);
+        } else {
+            if (c < nvec) wv[i] = load16(w + static_cast<long>(c) * V);  // shared by every row: an L2 hit
+        }
     }
     // A NaN result must come out as the host's 16-bit types write it, which the fast tier's
     // conversion instructions do not do, and its range test does not see a NaN (min / max skip
@@ -129,7 +168,7 @@ __global__ __launch_bounds__((BLOCK == 0 ? 1024 : BLOCK), (fwd_waves_per_simd<T,
 #pragma unroll
         for (int i = 0; i < NV; ++i) {
             const int c = threadIdx.x + i * block;
-            if (c < nvec) dst[i] = load16_nt(xr + static_cast<long>(c) * V);
+            if (c < nvec) dst[i] = load_vec<kAny>(xr + static_cast<long>(c) * V, H - c * V);
         }
     };
     u32x4 xv[NV], xn[NV];
@@ -185,7 +224,7 @@ __global__ __launch_bounds__((BLOCK == 0 ? 1024 : BLOCK), (fwd_waves_per_simd<T,
                     S* oe = reinterpret_cast<S*>(&o);
 #pragma unroll
                     for (int j = 0; j < V; ++j) oe[j] = scale_one<T>(e[j], rs32, rs, we[j]);
-                    store16_nt(outr + static_cast<long>(c) * V, o);
+                    store_vec<kAny>(outr + static_cast<long>(c) * V, o, H - c * V);
                 }
             }
         }
@@ -937,6 +976,10 @@ int grid_for_rows(long rows) {
     return static_cast<int>(rows < cap ? rows : cap);
 }
 
+// fp32 rows of any width and alignment from here on take the 16-byte kernel (21787 x 994 and 15646 x 3610, forward and backward:
+// 116 -> 92 us and 280 -> 207); in shorter ones half of its smallest workgroup would be idle.
+constexpr long kAnyWidth = 256;
+
 template <typename T>
 int launch_fwd(const void* x, const void* w, void* out, float* rstd, long rows, long H,
                double eps, hipStream_t s) {
@@ -1001,7 +1044,20 @@ int launch_fwd(const void* x, const void* w, void* out, float* rstd, long rows, 
                                1.0 / static_cast<double>(H));
     }
 #undef PARAS_RMS_FWD
-    else
+    else if (sizeof(S) == 4 && H >= kAnyWidth && H <= 2048 * V) {
+        if constexpr (sizeof(S) == 4) {
+            const long any_vecs = (H + V - 1) / V, waves = pipe_cap / 16 * 4 * fwd_waves_per_simd<T, 2, true>();        // resident, with two vectors per thread
+#define PARAS_RMS_FWD_ANY(NV_, BLOCK_, RESIDENT_)                                                                                              \
+    hipLaunchKernelGGL((rms_norm_fwd_vec<T, NV_, BLOCK_, true, true>), dim3(static_cast<unsigned>(rows < (RESIDENT_) ? rows : (RESIDENT_))), \
+                       dim3(BLOCK_), 0, s, xs, ws, os, rstd, rows, (int)H, eps, 1.0 / static_cast<double>(H))
+            if (any_vecs <= 128)       PARAS_RMS_FWD_ANY(1, 128, pipe_cap);
+            else if (any_vecs <= 256)  PARAS_RMS_FWD_ANY(1, 256, pipe_cap);
+            else if (any_vecs <= 512)  PARAS_RMS_FWD_ANY(2, 256, waves / 4);
+            else if (any_vecs <= 1024) PARAS_RMS_FWD_ANY(2, 512, waves / 8);
+            else                       PARAS_RMS_FWD_ANY(2, 1024, waves / 16);
+#undef PARAS_RMS_FWD_ANY
+        }
+    } else
         hipLaunchKernelGGL((rms_norm_fwd_any<T>), dim3(grid), dim3(kBlock), 0, s, xs, ws, os, rstd, rows, H, eps);
     PARAS_HIP_TRY(hipGetLastError());
     return PARAS_OK;

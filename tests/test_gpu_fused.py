@@ -378,6 +378,43 @@ def test_signed_zeros_infinities_and_nans_come_out_as_on_the_host(dtype):
 
 
 @pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16, torch.float16])
+@pytest.mark.parametrize("shape", [(1100, 4097), (1030, 4095), (7, 255), (5, 257), (9000, 511), (9000, 513), (1600, 1023), (1600, 1025), (1600, 2047),
+                                   (1040, 2049), (700, 8189), (3, 8191), (3, 8193), (1100, 4096)])
+def test_rms_norm_of_rows_of_any_width_and_alignment(shape, dtype):
+    """Rows that are not whole aligned 16-byte vectors: widths one off those that fill a workgroup's vectors, last vectors of one to
+    three elements, rows and weights that start one element past a 16-byte boundary, an infinity and a NaN."""
+    rows, H = shape
+    g = torch.Generator().manual_seed(rows + H)
+    x, w, go = (torch.randn(n, generator=g).to(dtype) for n in ((rows, H), (H,), (rows, H)))
+    x[1, H - 1], x[2, 0] = float("inf"), float("nan")
+
+    def off_by_one(t):
+        flat = torch.empty(t.numel() + 1, dtype=dtype, device="cuda")[1:]
+        return flat.copy_(t.reshape(-1)).view(t.shape)
+
+    out, rstd = capi.rms_norm(off_by_one(x), off_by_one(w), 1e-6)
+    wout, wrstd = O.rms_norm(x, w, 1e-6)
+    if dtype == torch.float32:      # the fp64 sum's order moves rstd by up to H 2^-53: past a rounding boundary of fp32 once in 2^29 / H elements or rarer
+        got, same = out.cpu(), wout.isnan()
+        assert torch.equal(got.isnan(), same)
+        off = (got != wout) & ~same
+        assert bool(((got - wout)[off].abs() <= 2.0 ** -23 * wout[off].abs()).all()) and int(off.sum()) <= 2 + out.numel() * H // 2 ** 29
+    else:
+        assert_same_bits_nan_aware(out, wout, "rms_norm")
+    assert torch.allclose(rstd.cpu(), wrstd, rtol=2.0 ** -23, atol=0, equal_nan=True)
+    x[1, H - 1], x[2, 0] = 1.0, -1.0
+    _, wrstd = O.rms_norm(x, w, 1e-6)
+    gx, gw = capi.rms_norm_backward(off_by_one(go), off_by_one(x), off_by_one(w), dev(wrstd))
+    for got, want, what in zip((gx, gw), O.rms_norm_backward(go, x, w, wrstd), ("grad_input", "grad_weight")):
+        # fp64 sums in another order, one rounding: a neighbouring value where the sum lies next to a boundary, else the same bits
+        err = (got.cpu().double() - want.double()).abs()
+        eps = {torch.float32: 2.0 ** -23, torch.bfloat16: 2.0 ** -7, torch.float16: 2.0 ** -10}[dtype]
+        tiny = {torch.float32: 2.0 ** -149, torch.bfloat16: 2.0 ** -133, torch.float16: 2.0 ** -24}[dtype]
+        assert bool((err <= eps * want.double().abs() + tiny).all()), what
+        assert float((err > 0).double().mean()) <= 1e-3, what
+
+
+@pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16, torch.float16])
 @pytest.mark.parametrize("shape", [(12000, 257), (3100, 1000), (3000, 1024), (3000, 1028), (1600, 2049), (1600, 2048), (1024, 4095),
                                    (1024, 4100), (1024, 8191), (1024, 8192), (1024, 8193), (90000, 36), (1008, 3000)])
 def test_rms_norm_backward_rows_in_registers(shape, dtype):
