@@ -18,9 +18,9 @@ namespace paras {
 namespace {
 
 constexpr int kBlock  = 256;
-constexpr int kUnroll = 4;  // 16-byte vectors per stream per lane per iteration
 
-template <typename T>
+// kUnroll: 16-byte vectors per stream per lane per iteration.
+template <typename T, int kUnroll>
 __global__ __launch_bounds__(kBlock) void swiglu_fwd_vec(
     const typename Elem<T>::store_t* __restrict__ gate, const typename Elem<T>::store_t* __restrict__ up,
     typename Elem<T>::store_t* __restrict__ out, long nvec) {
@@ -252,10 +252,16 @@ int launch_swiglu_fwd(const void* gate, const void* up, void* out, long n, hipSt
                            reinterpret_cast<uintptr_t>(out)) % 16) == 0;
     long done = 0;
     if (aligned && n >= V) {
+        // Four vectors per lane keep enough bytes under way where there are waves enough; with fewer the arithmetic of one vector
+        // after the other decides, for longer where it is the two tiers of 16-bit results (bf16, four / one: 14336 vectors 5.3 / 2.9 us,
+        // 131072 6.5 / 4.0, 524288 8.4 / 7.1; fp32: 14336 3.4 / 2.3, 262144 4.9 / 4.6, 672000 8.3 / 8.8).
         const long nvec = n / V;
-        long blocks = (nvec + kBlock * kUnroll - 1) / (kBlock * kUnroll);
+        const int unroll = nvec <= (sizeof(S) == 2 ? 1 << 20 : 1 << 18) ? 1 : 4;
+        long blocks = (nvec + kBlock * unroll - 1) / (kBlock * unroll);
         if (blocks > 0x7fffffffL) blocks = 0x7fffffffL;  // the kernel grid-strides beyond that
-        hipLaunchKernelGGL((swiglu_fwd_vec<T>), dim3(static_cast<unsigned>(blocks)), dim3(kBlock), 0, s, g, u, o, nvec);
+        const dim3 grid(static_cast<unsigned>(blocks));
+        if (unroll == 1) hipLaunchKernelGGL((swiglu_fwd_vec<T, 1>), grid, dim3(kBlock), 0, s, g, u, o, nvec);
+        else             hipLaunchKernelGGL((swiglu_fwd_vec<T, 4>), grid, dim3(kBlock), 0, s, g, u, o, nvec);
         PARAS_HIP_TRY(hipGetLastError());
         done = nvec * V;
     }

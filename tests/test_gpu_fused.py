@@ -80,6 +80,15 @@ def test_swiglu_matches_oracle(dtype, n):
     assert_bit_exact(capi.swiglu(dev(gate), dev(up)), O.swiglu(gate, up), f"swiglu {dtype} n={n}")
 
 
+@pytest.mark.parametrize("dtype, vec, few", [(torch.float32, 4, 1 << 18), (torch.bfloat16, 8, 1 << 20), (torch.float16, 8, 1 << 20)])
+@pytest.mark.parametrize("vecs", [0, 1, 255, 257])
+def test_swiglu_around_the_change_of_vectors_per_lane(dtype, vec, few, vecs):
+    """The last count of 16-byte vectors at which a lane takes one, those just above it, where it takes four, and elements left over."""
+    n = (few + vecs) * vec + 3
+    gate, up = (3 * torch.randn(n)).to(dtype), torch.randn(n).to(dtype)
+    assert_bit_exact(capi.swiglu(dev(gate), dev(up)), O.swiglu(gate, up), f"swiglu {dtype} n={n}")
+
+
 def test_swiglu_extreme_gates_take_the_exact_tier():
     """Gates outside the range of the fp32 fast path, zeros, infinities, NaN."""
     vals = [0.0, -0.0, 1e-30, -1e-30, -8.0, -8.5, -20.0, -60.0, -100.0, -700.0, 8.0, 60.0, 61.0, 100.0, 3e38,
