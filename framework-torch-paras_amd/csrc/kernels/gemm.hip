@@ -116,14 +116,14 @@ __global__ __launch_bounds__(stream::kThreads, 4) void stream_gemm_nt_kernel(con
     });
 }
 
-// ---- 33 to 128 rows without a workspace: the same split, but with this many activation rows per weight row a trip
+// ---- 33 to 128 rows, as few_rows_up_to says: the same split, but with this many activation rows per weight row a trip
 // through LDS for each would cost more than it saves, so every wave feeds its MFMAs straight from memory (weights
 // as the row operand, with plain loads: non-temporal ones measured 5-18 % slower, each 128-byte line being touched by two
 // instructions; the activation rows from L2), and the eight partial results meet in LDS in wave order.  Lane l of
 // a 16x16 result holds activation row l%16 and weight rows 4*(l/16) .. +3.
 constexpr int kSkinnyWaves = 8;
 constexpr int kSkinnyMaxM = 128;
-constexpr int kFewRowsM = 32;            // with a workspace at hand the tile kernel with the contraction in parts takes over from here
+constexpr int kFewRowsM = 32;            // the staged tiles take over from here (few_rows_up_to)
 
 template <typename T, int MB, int NB>   // MB = 16-row blocks of activations, NB = 16-row blocks of weights per workgroup
 __global__ __launch_bounds__(kSkinnyWaves * 64) void skinny_gemm_nt_kernel(const DenseParams p) {
@@ -404,6 +404,16 @@ bool few_rows_by_tiles(long M, long N, long batch) {
     return M > 32 && M <= kSkinnyMaxM && (N + gemm::kBN - 1) / gemm::kBN * batch >= 192;
 }
 
+// From 33 rows on the staged tiles are faster but for short contractions of few weight rows, where their start is most of
+// the call: few-row kernels / tiles, 33 x 512 x 512 4.3 / 4.9 us, 48 x 3072 x 512 4.8 / 5.2, 64 x 1024 x 512 5.0 / 5.1, 64 x 4096 x 256 4.1 / 4.4;
+// 64 x 4096 x 512 5.7 / 5.4, 40 x 2048 x 1024 7.0 / 6.7, 64 x 1024 x 1024 7.2 / 6.5, 33 x 6144 x 512 6.5 / 5.3, 56 x 4384 x 256 4.9 / 4.4,
+// 63 x 7192 x 1024 12.5 / 7.0, 108 x 7456 x 6656 110 / 36.  Where the tiles want the contraction in parts and the caller has no workspace for
+// them, and for paras_gemm_nt, the few-row kernels stay up to kSkinnyMaxM rows.
+bool few_rows_up_to(long M, long N, long K, long batch, bool parts_or_whole) {
+    if (M <= kFewRowsM) return true;
+    return parts_or_whole ? M <= 64 && M * K <= 36000 && N * batch <= 4096 : M <= kSkinnyMaxM;
+}
+
 // Few output columns and many rows: the few-row kernels with the operands in each other's place.  Up to
 // 32 columns (every workgroup re-reads the short operand, and from 48 rows of it on the tile kernel with
 // the contraction in parts is faster: M = 16384, N = 128, K = 4096 80 us this way).
@@ -610,7 +620,7 @@ Route route_of(const paras_gemm_args& g, bool may_split, bool nt_api, int causal
         r.workspace = static_cast<size_t>(r.splits) * g.batch * g.M * g.N * sizeof(float);
         return r;
     }
-    if (nt64 && g.M <= (may_split && !nt_api ? kFewRowsM : kSkinnyMaxM) && !few_rows_by_tiles(g.M, g.N, g.batch) && g.batch <= 65535) {
+    if (nt64 && few_rows_up_to(g.M, g.N, g.K, g.batch, may_split && !nt_api) && !few_rows_by_tiles(g.M, g.N, g.batch) && g.batch <= 65535) {
         r.kind = Route::FewRows;
         return r;
     }
@@ -631,15 +641,33 @@ int check_args(const paras_gemm_args& g) {
     return PARAS_OK;
 }
 
-int run(const paras_gemm_args& g, void* workspace, size_t workspace_bytes, void* stream, bool nt_api, int causal_kind, long causal_first) {
+// Where a product's partial sums go: memory that the caller has, or a way to ask it for some.
+struct Scratch {
+    void* p = nullptr;
+    size_t bytes = 0;
+    paras_scratch_fn ask = nullptr;
+    void* ctx = nullptr;
+};
+
+// The route is found once.  It is the one that paras_gemm_workspace answers for, and only where it wants more than the caller has
+// another one is taken.
+int run(const paras_gemm_args& g, const Scratch& scratch, void* stream, bool nt_api, int causal_kind, long causal_first) {
     int rc = check_args(g);
     if (rc != PARAS_OK || g.M == 0 || g.N == 0 || g.batch == 0) return rc;
     hipStream_t s = nullptr;
     rc = resolve_stream(stream, &s);
     if (rc != PARAS_OK) return rc;
-    const bool ws_ok = workspace != nullptr && (reinterpret_cast<uintptr_t>(workspace) & 15) == 0;
-    Route r = route_of(g, ws_ok, nt_api, causal_kind, causal_first);
-    if (r.workspace > workspace_bytes) r = route_of(g, false, nt_api, causal_kind, causal_first);
+    Route r = route_of(g, /*may_split=*/true, nt_api, causal_kind, causal_first);
+    void* workspace = scratch.p;
+    if (r.workspace > 0) {
+        if (scratch.ask != nullptr) {
+            workspace = scratch.ask(scratch.ctx, r.workspace);
+            PARAS_REQUIRE(workspace != nullptr && (reinterpret_cast<uintptr_t>(workspace) & 15) == 0,
+                          "paras_gemm_scratch: no memory for %zu bytes on a 16-byte boundary", r.workspace);
+        } else if (workspace == nullptr || (reinterpret_cast<uintptr_t>(workspace) & 15) != 0 || r.workspace > scratch.bytes) {
+            r = route_of(g, false, nt_api, causal_kind, causal_first);
+        }
+    }
     if (r.kind == Route::F32) return f32::launch(f32_problem(g, causal_kind, causal_first), r.f32, workspace, s);
     if (r.kind == Route::Flex) return flex::launch(flex_problem(g), r.flex, workspace, s);
     PARAS_REQUIRE(!g.a_rows && !g.b_rows, "paras_gemm: these sizes or alignments need operands that are contiguous along the contraction");
@@ -710,7 +738,7 @@ int gemm_nt_causal(const void* a, const void* b, const void* addend, void* c, in
     g.lda = lda; g.ldb = ldb; g.ldc = ldc; g.ld_add = ld_add;
     g.batch = batch; g.stride_a = stride_a; g.stride_b = stride_b; g.stride_c = stride_c; g.stride_add = stride_add;
     g.alpha = alpha; g.beta = beta; g.dtype = dtype;
-    return run(g, workspace, workspace_bytes, stream, /*nt_api=*/true, causal_kind, causal_first);
+    return run(g, {workspace, workspace_bytes}, stream, /*nt_api=*/true, causal_kind, causal_first);
 }
 }  // namespace paras
 
@@ -751,7 +779,12 @@ size_t paras_gemm_workspace(const paras_gemm_args* args) {
 
 int paras_gemm(const paras_gemm_args* args, void* workspace, size_t workspace_bytes, void* stream) {
     PARAS_REQUIRE(args != nullptr, "paras_gemm: null argument block");
-    return paras::run(*args, workspace, workspace_bytes, stream, /*nt_api=*/false, 0, 0);
+    return paras::run(*args, {workspace, workspace_bytes}, stream, /*nt_api=*/false, 0, 0);
+}
+
+int paras_gemm_scratch(const paras_gemm_args* args, paras_scratch_fn scratch, void* ctx, void* stream) {
+    PARAS_REQUIRE(args != nullptr && scratch != nullptr, "paras_gemm_scratch: null argument");
+    return paras::run(*args, {nullptr, 0, scratch, ctx}, stream, /*nt_api=*/false, 0, 0);
 }
 
 }  // extern "C"

@@ -3,6 +3,8 @@
 // parts, and the launch.
 #include <hip/hip_runtime.h>
 
+#include <utility>
+
 #include "core/device_context.h"
 #include "core/status.h"
 #include "kernels/gemm_flex_host.h"
@@ -89,39 +91,84 @@ bool takes(const Problem& q) {
 // (3000 x 4096 x 4096 94 us, with 256 tiles of 192 x 256 84 us); a small problem has few workgroups per CU, and then more
 // stages stand in for the other workgroups' loads (821 x 1024 x 3584 64 x 64: two stages in four parts 21 us, four stages 14.5 whole);
 // what is still too few tiles is cut up along the contraction (261 x 4096 x 14336 192 x 128: four parts 52 us).
-Plan plan(const Problem& q, bool may_split) {
+//
+// The search is on the way of every call, and a small product's launch costs a few us: the forms' constants are the compiler's
+// (no division by a variable but two per number of parts), and forms and numbers of parts are left out whose least possible time is no
+// better than one found.  The same plan as the search through all of them; host time of that and of this: 48 x 1024 x 1024 1.4 and 0.17 us,
+// 128 x 2048 x 2048 2.0 and 0.41, 1024 x 1024 x 4096 2.1 and 0.19, 8192^3 0.37 and 0.05.
+namespace {
+
+struct Search {
+    int M, N, batch, k_tiles;
+    bool may_split;
+    double mn, memory;                          // elements of the result; us for the operands' way from memory
+    int per[9], parts[9];                       // of the contraction, for 1, 2, 3, 4, 6, 9, 13, 19, 28 parts wanted
+    int known = 0;
+    double best_us = 1e30, found = 1e30;        // of `best`; of any form looked at
     Plan best;
-    double best_us = 1e30;
-    const long k_tiles = (q.K + kBK - 1) / kBK;
-    const double mn = static_cast<double>(q.M) * q.N * q.batch;
-    const double memory = static_cast<double>(q.M + q.N) * q.K * q.batch * 2 / 5.6e6 + 2.5;      // the operands' way from memory
-    for (int t = 0; t < kTileCount; ++t) {
-        const Tile& tl = kTiles[t];
-        if (t >= kAlongContraction && (q.a_rows || q.b_rows)) break;
-        if (tl.m * tl.n > 128 * 128 && q.K <= 512) continue;     // mostly stores: small tiles overlap them with other tiles' work
-        const long mt = (q.M + tl.m - 1) / tl.m, nt = (q.N + tl.n - 1) / tl.n, tiles = mt * nt * q.batch;
-        for (int s = 1; s <= (may_split ? 32 : 1); s = s < 4 ? s + 1 : s + s / 2) {
-            if (s > 1 && (s * 2 > k_tiles || tiles * s > 1600)) break;
-            const long per = (k_tiles + s - 1) / s, parts = (k_tiles + per - 1) / per, turns = (per + tl.stages - 1) / tl.stages * tl.stages;
-            const long wgs = tiles * parts, slots = static_cast<long>(kCus) * tl.per_cu, full = wgs / slots;
-            const long rest = (wgs - full * slots + kCus - 1) / kCus;
-            const double stores = tl.m * tl.n / 65536.0 * (parts > 1 ? 8.9 : 7.5);
+
+    void want(int i, int wanted) {
+        if (i < known) return;
+        per[i] = static_cast<unsigned>(k_tiles + wanted - 1) / static_cast<unsigned>(wanted);
+        parts[i] = static_cast<unsigned>(k_tiles + per[i] - 1) / static_cast<unsigned>(per[i]);
+        known = i + 1;
+    }
+    template <int t, bool record> void consider() {
+        constexpr Tile tl = kTiles[t];
+        constexpr int slots = kCus * tl.per_cu;
+        constexpr double area = tl.m * tl.n / 65536.0, each = tl.step / tl.per_cu;
+        const int tiles = (static_cast<unsigned>(M) + (tl.m - 1)) / tl.m * ((static_cast<unsigned>(N) + (tl.n - 1)) / tl.n) * batch;     // below 2^25
+        // no less than the CUs' arithmetic and stores, shared out evenly, take
+        const double least = (3.1 + tiles * (k_tiles * each + area * 7.5) / kCus) * kBelow;
+        if (least >= found) return;
+        for (int i = 0, wanted = 1; wanted <= (may_split ? 32 : 1); ++i, wanted = wanted < 4 ? wanted + 1 : wanted + wanted / 2) {
+            if (wanted > 1 && (wanted * 2 > k_tiles || tiles * wanted > 1600)) break;
+            want(i, wanted);
+            const int n_parts = parts[i], turns = static_cast<unsigned>(per[i] + (tl.stages - 1)) / tl.stages * tl.stages;
+            const double finish = n_parts > 1 ? 4.0 + mn * (8.0 * n_parts + 2.0) / 6.9e6 : 0.0;
+            if (least + finish >= found) break;
+            if ((turns * tl.lat + 3.1) * kBelow + finish >= found) continue;
+            const int wgs = tiles * n_parts, full = static_cast<unsigned>(wgs) / slots;
+            const int rest = static_cast<unsigned>(wgs - full * slots + kCus - 1) / kCus;
+            const double stores = area * (n_parts > 1 ? 8.9 : 7.5);
             auto round = [&](double n) {
                 const double c = tl.step * n / tl.per_cu;
                 return turns * (c > tl.lat ? c : tl.lat) + 3.1 + stores * n;
             };
-            double us = full * round(tl.per_cu) + (rest > 0 ? round(static_cast<double>(rest)) : 0.0);
+            double us = full * round(tl.per_cu) + (rest > 0 ? round(rest) : 0.0);
             if (us < memory) us = memory;
-            if (parts > 1) us += 4.0 + mn * (8.0 * parts + 2.0) / 6.9e6;
-            if (us < best_us) {
+            us += finish;
+            if (us * kAbove < found) found = us * kAbove;
+            if (record && us < best_us) {
                 best_us = us;
                 best.tile = t;
-                best.splits = static_cast<int>(parts);
-                best.k_per_split = per * kBK;
+                best.splits = n_parts;
+                best.k_per_split = static_cast<long>(per[i]) * kBK;
             }
         }
     }
-    return best;
+    template <int... t> void consider_all(std::integer_sequence<int, t...>, bool large, bool along_contraction) {
+        consider<kUsual, false>();              // (so that the others have something to be measured against)
+        // (best_us <= memory: nothing is better)
+        (void)((best_us <= memory ||
+                ((t < kAlongContraction || along_contraction) && (kTiles[t].m * kTiles[t].n <= 128 * 128 || large) ? consider<t, true>() : void(), false)) || ...);
+    }
+    static constexpr int kUsual = 9;                                        // 64 x 64, three stages: a third of all choices
+    static constexpr double kBelow = 1.0 - 1e-9, kAbove = 1.0 + 1e-9;       // the bounds are other sums than the estimate
+};
+
+}  // namespace
+
+Plan plan(const Problem& q, bool may_split) {
+    Search s;
+    s.M = static_cast<int>(q.M); s.N = static_cast<int>(q.N); s.batch = static_cast<int>(q.batch);       // (takes(): below 2^30, 2^31 and 2^16)
+    s.k_tiles = static_cast<int>((q.K + kBK - 1) / kBK);
+    s.may_split = may_split;
+    s.mn = static_cast<double>(q.M) * q.N * q.batch;
+    s.memory = static_cast<double>(q.M + q.N) * q.K * q.batch * 2 / 5.6e6 + 2.5;
+    // (K <= 512: mostly stores, and small tiles overlap them with other tiles' work)
+    s.consider_all(std::make_integer_sequence<int, kTileCount>{}, q.K > 512, !q.a_rows && !q.b_rows);
+    return s.best;
 }
 
 int launch(const Problem& q, const Plan& plan, void* workspace, hipStream_t s) {

@@ -9,6 +9,8 @@
 #include <ATen/NativeFunctions.h>
 #include <torch/csrc/autograd/custom_function.h>
 
+#include <exception>
+
 namespace paras_torch {
 namespace {
 
@@ -52,6 +54,24 @@ Operand operand(const Tensor& t, bool swap, bool may_be_rows) {
     return {c, c.data_ptr(), R > 1 ? K : up8(K), batched ? R * K : 0, false};
 }
 
+// Memory for a product's partial sums, allocated when the library says how much; what the allocator throws does not
+// pass through the library.
+struct Partials {
+    Tensor hold;
+    c10::Device device;
+    std::exception_ptr failed;
+    static void* allocate(void* self, size_t nbytes) noexcept {
+        auto* p = static_cast<Partials*>(self);
+        try {
+            p->hold = workspace(nbytes, p->device);
+            return p->hold.data_ptr();
+        } catch (...) {
+            p->failed = std::current_exception();
+            return nullptr;
+        }
+    }
+};
+
 // out[b] = alpha * a[b] mat2[b] + beta * addend[b], a [.., M, K], into a dense tensor of `shape`.  mat2 is
 // [.., K, N], or [.., N, K] with `mat2_nk`; a is [.., K, M] with `a_km`.
 Tensor run_gemm(const Tensor& a_in, bool a_km, const Tensor& mat2, bool mat2_nk, const Tensor* addend, double alpha, double beta, int64_t batch,
@@ -84,10 +104,10 @@ Tensor run_gemm(const Tensor& a_in, bool a_km, const Tensor& mat2, bool mat2_nk,
     g.alpha = alpha; g.beta = beta; g.dtype = code;
     g.a_rows = a.rows; g.b_rows = b.rows;
     // products with few tiles run faster with a workspace for the partial sums of a split contraction
-    const size_t ws_bytes = paras_gemm_workspace(&g);
-    Tensor ws;
-    if (ws_bytes > 0) ws = workspace(ws_bytes, a_in.device());
-    check(paras_gemm(&g, ws_bytes > 0 ? ws.data_ptr() : nullptr, ws_bytes, stream_for(a_in)));
+    Partials partials{Tensor(), a_in.device(), nullptr};
+    const int rc = paras_gemm_scratch(&g, &Partials::allocate, &partials, stream_for(a_in));
+    if (partials.failed) std::rethrow_exception(partials.failed);
+    check(rc);
     return out;
 }
 

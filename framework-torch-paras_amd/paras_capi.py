@@ -34,6 +34,8 @@ class SdpaArgs(C.Structure):
         ("scale", f64),
     ]
 
+SCRATCH_FN = C.CFUNCTYPE(vp, vp, sz)          # paras_scratch_fn
+
 
 # name -> (restype, argtypes); the list is also what the symbol-export test walks.
 SIGNATURES = {
@@ -81,6 +83,7 @@ SIGNATURES = {
     "paras_gemm_nt_ws": (i32, [vp, vp, vp, vp] + [i64] * 12 + [f64, f64, i32, vp, sz, vp]),
     "paras_gemm_workspace": (sz, [C.POINTER(GemmArgs)]),
     "paras_gemm": (i32, [C.POINTER(GemmArgs), vp, sz, vp]),
+    "paras_gemm_scratch": (i32, [C.POINTER(GemmArgs), SCRATCH_FN, vp, vp]),
     "paras_column_sum_workspace": (sz, [i64, i64, i32]),
     "paras_column_sum": (i32, [vp, vp, i64, i64, i64, i32, vp, vp]),
     "paras_softmax_rows": (i32, [vp, vp, i64, i64, i32, i32, vp]),
@@ -322,6 +325,22 @@ def gemm(a, b, addend=None, alpha=1.0, beta=1.0, workspace=True):
     ws = torch.empty(max(n, 16), dtype=torch.uint8, device=a.device)
     check(lib().paras_gemm(C.byref(g), _ptr(ws) if workspace else None, n, _stream()))
     return c
+
+
+def gemm_scratch(a, b, allocate):
+    """paras_gemm_scratch on a [M, K], b [N, K]; allocate(nbytes) -> tensor or None.  Returns C (filled with sevens before the
+    call), what paras_gemm_workspace answers, and the status."""
+    (M, K), N = a.shape, b.shape[0]
+    c = torch.full((M, N), 7, dtype=a.dtype, device=a.device)
+    g = GemmArgs(_ptr(a), _ptr(b), None, _ptr(c), M, N, K, a.stride(0), b.stride(0), N, 0, 1, 0, 0, 0, 0, 1.0, 0.0, DT[a.dtype], 0, 0)
+    held = []
+
+    def ask(_, nbytes):
+        held.append(allocate(nbytes))
+        return None if held[-1] is None else held[-1].data_ptr()
+
+    rc = lib().paras_gemm_scratch(C.byref(g), SCRATCH_FN(ask), None, _stream())
+    return c, lib().paras_gemm_workspace(C.byref(g)), rc
 
 
 def column_sum(x):

@@ -353,7 +353,7 @@ PARAS_API int paras_moe_ffn(const void* x, const void* w_gate, const void* w_up,
 /* (a bias) over the M rows.  All four float dtypes.  bf16 / f16 with K a       */
 /* multiple of 8, 16-byte aligned operands and leading dimensions and batch    */
 /* strides that are multiples of 8 run on the MFMA kernels (fp32 accumulation, */
-/* one rounding; up to 32 rows, 128 without a workspace, on kernels that stream */
+/* one rounding; up to 32 rows, 128 by paras_gemm_nt, on kernels that stream    */
 /* the weights, K a multiple of 64); fp32 tensors on the fp32 MFMA kernel (full */
 /* fp32 multiplies, any K and alignment); everything else -- fp64 tensors,     */
 /* 16-bit ones with other K or alignments -- on a general kernel (fp32         */
@@ -404,6 +404,15 @@ typedef struct paras_gemm_args {
 PARAS_API size_t paras_gemm_workspace(const paras_gemm_args* args);
 PARAS_API int paras_gemm(const paras_gemm_args* args, void* workspace,
                          size_t workspace_bytes, void* stream);
+/* paras_gemm for callers that allocate the workspace when they learn its size: */
+/* scratch(ctx, nbytes) is called at most once, before anything is launched, with */
+/* the size paras_gemm_workspace would answer (not at all where that is 0), and   */
+/* returns nbytes of device memory on a 16-byte boundary.  NULL or another       */
+/* boundary: PARAS_ERR_INVALID, nothing is launched.  It must not throw.  How the */
+/* product is carried out is settled once, not once per entry point.             */
+typedef void* (*paras_scratch_fn)(void* ctx, size_t nbytes);
+PARAS_API int paras_gemm_scratch(const paras_gemm_args* args, paras_scratch_fn scratch,
+                                 void* ctx, void* stream);
 /* out[c] = T(sum over the rows of x[r][c]), rows ld apart: a bias gradient (same */
 /* reference lines).  Any float dtype; paras_column_sum_workspace bytes.         */
 PARAS_API size_t paras_column_sum_workspace(int64_t rows, int64_t cols, int dtype);

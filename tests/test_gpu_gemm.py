@@ -535,3 +535,28 @@ def test_gemm_tiles_with_several_stages(shape, dtype):
         for ws in (False, True):
             got = capi.gemm(x, y, workspace=ws)
             assert bool(((got.double() - want).abs() <= bar).all())
+
+
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16, torch.float32])
+@pytest.mark.parametrize("shape", [(8, 512, 1024), (33, 512, 512), (64, 4096, 512), (65, 512, 512), (64, 4104, 512), (64, 512, 576), (128, 2048, 2048), (700, 24, 512),
+                                   (96, 1000, 72), (300, 136, 14336)])
+def test_scratch_is_asked_for_once_and_the_route_is_the_planned_one(shape, dtype):
+    """paras_gemm_scratch: the size that paras_gemm_workspace answers, once, or no question where that is 0, and the bits of
+    paras_gemm -- with that workspace, and without any where none is wanted: the route is one choice.  Either side of the rules
+    for 33 to 64 rows (512 x 64 and 4096 weight rows), few columns, other contractions, parts.  No memory: an error before
+    anything is launched."""
+    M, N, K = shape
+    torch.manual_seed(M + N + K)
+    a, b = torch.randn(M, K).to(dtype).cuda(), (torch.randn(N, K) / math.sqrt(K)).to(dtype).cuda()
+    want = a.double() @ b.double().T
+    asked = []
+    c, n, rc = capi.gemm_scratch(a, b, lambda size: asked.append(size) or torch.empty(size, dtype=torch.uint8, device="cuda"))
+    assert rc == 0 and asked == ([n] if n else [])
+    assert torch.equal(c, capi.gemm(a, b))
+    if n == 0:
+        assert torch.equal(c, capi.gemm(a, b, workspace=False))
+    assert ((c.double() - want).norm() / want.norm()).item() < {torch.bfloat16: 4e-3, torch.float16: 6e-4, torch.float32: 3e-6}[dtype]
+    if n:
+        c, _, rc = capi.gemm_scratch(a, b, lambda size: None)
+        assert rc == -1 and bool((c == 7).all())
+    assert n > 0 or shape != (300, 136, 14336)

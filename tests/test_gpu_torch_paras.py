@@ -450,6 +450,15 @@ def test_linear_mm_bmm_addmm_on_device(device, dtype):
     _one_ulp(torch.matmul(q.to(device), k.to(device).transpose(-1, -2)), torch.matmul(q, k.transpose(-1, -2)), dtype)
 
 
+@pytest.mark.parametrize("shape", [(48, 1024, 1024), (40, 3000, 512), (96, 4096, 1024), (128, 7168, 512), (128, 2048, 2048)])
+def test_linear_runs_the_route_that_is_planned(device, shape):
+    """33 to 128 rows: F.linear gives the bits of paras_gemm with the workspace that it asks for, whether that is any or none."""
+    M, N, K = shape
+    x, w = torch.randn(M, K).bfloat16(), (torch.randn(N, K) / math.sqrt(K)).bfloat16()
+    import capi
+    assert_bit_exact(F.linear(x.to(device), w.to(device)).cpu(), capi.gemm(x.cuda(), w.cuda()).cpu())
+
+
 def test_gemm_other_dtypes_and_shapes_stay_on_the_device(device):
     """fp32 / fp64 products and contraction sizes the MFMA kernels do not take run on the general
     device kernel (reference tolerance against torch-CPU; fp32 accumulation and one rounding for the
