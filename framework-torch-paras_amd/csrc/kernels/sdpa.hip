@@ -3,6 +3,7 @@
 #include <hip/hip_runtime.h>
 
 #include <cmath>
+#include <cstdint>
 
 #include "core/device_context.h"
 #include "core/status.h"
@@ -83,12 +84,13 @@ SdpaKernel choose(const paras_sdpa_args& a) {
     return SdpaKernel::Generic;
 }
 
-int launch_padded(const paras_sdpa_args& a, void* workspace, void* stream, hipStream_t s) {
+int launch_padded(const paras_sdpa_args& a, Scratch scratch, void* stream, hipStream_t s) {
     PaddedPlan pl;
     PARAS_REQUIRE(plan_padded(a, &pl), "paras sdpa: not a shape for the padded route");
-    PARAS_REQUIRE(workspace != nullptr, "paras sdpa: workspace is null");
-    PARAS_REQUIRE((reinterpret_cast<uintptr_t>(workspace) & 255) == 0, "paras sdpa: the workspace must be 256-byte aligned");
-    char* ws = static_cast<char*>(workspace);
+    PARAS_REQUIRE(scratch.p != nullptr, "paras sdpa: workspace is null");
+    PARAS_REQUIRE((reinterpret_cast<uintptr_t>(scratch.p) & 255) == 0, "paras sdpa: the workspace must be 256-byte aligned");
+    PARAS_REQUIRE(scratch.has(pl.total), "paras sdpa: a workspace of %zu bytes, %zu needed", scratch.bytes, pl.total);
+    char* ws = static_cast<char*>(scratch.p);
     paras_sdpa_args in = pl.inner;
     in.q = ws + pl.q_off; in.k = ws + pl.k_off; in.v = ws + pl.v_off; in.out = ws + pl.out_off;
     const int64_t Dp = in.D, one = 1;
@@ -103,12 +105,52 @@ int launch_padded(const paras_sdpa_args& a, void* workspace, void* stream, hipSt
     if ((rc = copy_in(a.q, a.q_strides, const_cast<void*>(in.q), a.Hq, a.Lq)) != PARAS_OK) return rc;
     if ((rc = copy_in(a.k, a.k_strides, const_cast<void*>(in.k), a.Hkv, a.Lk)) != PARAS_OK) return rc;
     if ((rc = copy_in(a.v, a.v_strides, const_cast<void*>(in.v), a.Hkv, a.Lk)) != PARAS_OK) return rc;
-    if (decode_supported(in)) rc = launch_decode(in, ws + pl.inner_off, s);
-    else                      rc = launch_flash(in, ws + pl.inner_off, s);
+    if (decode_supported(in)) rc = launch_decode(in, scratch.past(pl.inner_off), s);
+    else                      rc = launch_flash(in, scratch.past(pl.inner_off), s);
     if (rc != PARAS_OK) return rc;
     const int64_t sizes[4] = {a.B, a.Hq, a.Lq, a.D}, ss[4] = {a.Hq * a.Lq * Dp, a.Lq * Dp, Dp, 1},
                   ds[4] = {a.Hq * a.Lq * a.D, a.Lq * a.D, a.D, 1};
     return paras_copy_strided(in.out, a.out, 4, sizes, ss, ds, 2, a.dtype, a.dtype, stream);
+}
+
+// `bytes`: how large the workspace is, or null where the caller does not say.  Then it is taken to be what paras_sdpa_workspace
+// answers, but nothing is written to it where the kernels that share keys out could do without: a caller of a problem that needs no
+// scratch memory may have passed any.
+int run(const paras_sdpa_args* args, void* workspace, const size_t* bytes, void* stream) {
+    int rc = validate(args);
+    if (rc != PARAS_OK) return rc;
+    const paras_sdpa_args& a = *args;
+    if (empty_output(a)) return PARAS_OK;
+    PARAS_REQUIRE(a.out != nullptr, "paras sdpa: null output pointer");
+    PARAS_REQUIRE(a.Lk == 0 || (a.q && a.k && a.v), "paras sdpa: null tensor pointer");   // (empty k / v have no storage)
+    hipStream_t s = nullptr;
+    rc = resolve_stream(stream, &s);
+    if (rc != PARAS_OK) return rc;
+    if (a.Lk == 0) {
+        // softmax over nothing, then a product with an empty inner dim: zeros.
+        // (a fill kernel rather than hipMemsetAsync: callers may be capturing this stream into a graph)
+        const int esz = a.dtype == PARAS_F64 ? 8 : a.dtype == PARAS_F32 ? 4 : 2;
+        const int64_t n = a.B * a.Hq * a.Lq * a.Dv, one = 1;
+        return paras_fill_strided(a.out, 1, &n, &one, esz, 0, stream);
+    }
+    const Scratch given{workspace, bytes != nullptr ? *bytes : SIZE_MAX};
+    switch (choose(a)) {
+        case SdpaKernel::Flash: return launch_flash(a, bytes != nullptr ? given : Scratch{}, s);
+        case SdpaKernel::Weights: return launch_weights(a, s);
+        case SdpaKernel::Padded: return launch_padded(a, given, stream, s);
+        case SdpaKernel::Composed:
+            if (bytes != nullptr) {
+                const size_t need = composed_workspace(a);
+                PARAS_REQUIRE(need == 0 || given.has(need), "paras sdpa: a workspace of %zu bytes, %zu needed", workspace != nullptr ? given.bytes : 0, need);
+            }
+            return launch_composed(a, workspace, stream, s);
+        case SdpaKernel::Decode:
+            if (bytes != nullptr) return launch_decode(a, given, s);
+            if (decode_fills_chip(a)) return launch_decode(a, {}, s);
+            PARAS_REQUIRE(workspace != nullptr || decode_workspace(a) == 0, "paras sdpa: workspace is null");
+            return launch_decode(a, given, s);
+        default: return launch_generic(a, workspace, s);
+    }
 }
 
 }  // namespace
@@ -146,33 +188,11 @@ size_t paras_sdpa_workspace(const paras_sdpa_args* args) {
 }
 
 int paras_sdpa_fwd(const paras_sdpa_args* args, void* workspace, void* stream) {
-    using namespace paras;
-    int rc = validate(args);
-    if (rc != PARAS_OK) return rc;
-    const paras_sdpa_args& a = *args;
-    if (empty_output(a)) return PARAS_OK;
-    PARAS_REQUIRE(a.out != nullptr, "paras sdpa: null output pointer");
-    PARAS_REQUIRE(a.Lk == 0 || (a.q && a.k && a.v), "paras sdpa: null tensor pointer");   // (empty k / v have no storage)
-    hipStream_t s = nullptr;
-    rc = resolve_stream(stream, &s);
-    if (rc != PARAS_OK) return rc;
-    if (a.Lk == 0) {
-        // softmax over nothing, then a product with an empty inner dim: zeros.
-        // (a fill kernel rather than hipMemsetAsync: callers may be capturing this stream into a graph)
-        const int esz = a.dtype == PARAS_F64 ? 8 : a.dtype == PARAS_F32 ? 4 : 2;
-        const int64_t n = a.B * a.Hq * a.Lq * a.Dv, one = 1;
-        return paras_fill_strided(a.out, 1, &n, &one, esz, 0, stream);
-    }
-    switch (choose(a)) {
-        case SdpaKernel::Flash: return launch_flash(a, workspace, s);
-        case SdpaKernel::Weights: return launch_weights(a, s);
-        case SdpaKernel::Padded: return launch_padded(a, workspace, stream, s);
-        case SdpaKernel::Composed: return launch_composed(a, workspace, stream, s);
-        case SdpaKernel::Decode:
-            PARAS_REQUIRE(workspace != nullptr || decode_workspace(a) == 0, "paras sdpa: workspace is null");
-            return launch_decode(a, workspace, s);
-        default: return launch_generic(a, workspace, s);
-    }
+    return paras::run(args, workspace, nullptr, stream);
+}
+
+int paras_sdpa_fwd_ws(const paras_sdpa_args* args, void* workspace, size_t workspace_bytes, void* stream) {
+    return paras::run(args, workspace, &workspace_bytes, stream);
 }
 
 }  // extern "C"

@@ -431,17 +431,20 @@ int combine_threads(int splits, long D) {
 bool aligned16(const void* ptr) { return (reinterpret_cast<uintptr_t>(ptr) & 15) == 0; }
 bool mult8(const int64_t* s) { return s[0] % 8 == 0 && s[1] % 8 == 0 && s[2] % 8 == 0; }
 
+long compute_units() {
+    int dev = 0;
+    (void)hipGetDevice(&dev);
+    auto* st = DeviceContext::instance().device(dev);
+    return st ? st->compute_units : 256;
+}
+
 // Split count: whole rounds of workgroups over the CUs (a few workgroups more than that are a round of their own), one to eight of
 // them, or no split at all; the one of least estimated time: that of all bytes from memory, of a CU's bytes, and of the tiles
 // that follow each other in a wave, plus the merging of the splits where there are any.  Fitted to 70 problems (1 to 128 sequences, 64 to 32768
 // keys, 1 to 8 KV heads, D 64 and 128): the choice is within 1 % of the best count in the mean, two workgroups per CU, rounded up,
 // 5 % (42 KV heads of 16260 keys: 13 splits 79.1 us, 12 65.0; 144 heads of 298 keys: 2 splits 15.6, 1 11.1; 288 of 14555, D 64: 213 and 172).
-void plan(const paras_sdpa_args& a, int* splits, int* chunk) {
-    int dev = 0;
-    (void)hipGetDevice(&dev);
-    auto* st = DeviceContext::instance().device(dev);
-    const long cus = st ? st->compute_units : 256;
-    const long pairs = a.B * a.Hkv, rows = pairs * (a.Hq / a.Hkv) * a.Lq;
+void plan(const paras_sdpa_args& a, bool may_split, int* splits, int* chunk) {
+    const long cus = compute_units(), pairs = a.B * a.Hkv, rows = pairs * (a.Hq / a.Hkv) * a.Lq;
     const long unit = kWaves * kTile;                        // 128 keys: one tile per wave
     long max_splits = (a.Lk + 2 * unit - 1) / (2 * unit);    // >= 2 tiles per wave
     if (max_splits > kMaxSplits) max_splits = kMaxSplits;
@@ -450,7 +453,7 @@ void plan(const paras_sdpa_args& a, int* splits, int* chunk) {
     auto fourth = [](double v) { return v * v * v * v; };
     double best = 1e300;
     long last = 0;
-    for (long round = 0; round <= 8; ++round) {
+    for (long round = 0; round <= (may_split ? 8 : 0); ++round) {
         long want = round == 0 ? 1 : cus * round / pairs;
         want = want < 1 ? 1 : (want > max_splits ? max_splits : want);
         if (want == last) continue;
@@ -466,6 +469,12 @@ void plan(const paras_sdpa_args& a, int* splits, int* chunk) {
             *chunk = static_cast<int>(steps * unit);
         }
     }
+}
+
+size_t workspace_of(const paras_sdpa_args& a, int splits) {
+    if (splits == 1) return 0;
+    const size_t slots = static_cast<size_t>(a.B * a.Hkv) * splits;
+    return slots * (kMaxRows * a.D + 2 * kMaxRows) * sizeof(float);
 }
 
 }  // namespace
@@ -487,13 +496,13 @@ bool decode_supported(const paras_sdpa_args& a) {
 
 size_t decode_workspace(const paras_sdpa_args& a) {
     int splits = 1, chunk = 0;
-    plan(a, &splits, &chunk);
-    if (splits == 1) return 0;
-    const size_t slots = static_cast<size_t>(a.B * a.Hkv) * splits;
-    return slots * (kMaxRows * a.D + 2 * kMaxRows) * sizeof(float);
+    plan(a, true, &splits, &chunk);
+    return workspace_of(a, splits);
 }
 
-int launch_decode(const paras_sdpa_args& a, void* workspace, hipStream_t s) {
+bool decode_fills_chip(const paras_sdpa_args& a) { return a.B * a.Hkv >= 2 * compute_units(); }
+
+int launch_decode(const paras_sdpa_args& a, Scratch scratch, hipStream_t s) {
     DecodeParams p;
     p.q = static_cast<const std::uint16_t*>(a.q);
     p.k = static_cast<const std::uint16_t*>(a.k);
@@ -506,11 +515,12 @@ int launch_decode(const paras_sdpa_args& a, void* workspace, hipStream_t s) {
     p.B = (int)a.B; p.Hq = (int)a.Hq; p.Hkv = (int)a.Hkv; p.Lq = (int)a.Lq; p.Lk = (int)a.Lk;
     p.G = (int)(a.Hq / a.Hkv);
     p.R = p.G * p.Lq;
-    plan(a, &p.splits, &p.chunk);
+    plan(a, scratch.p != nullptr && aligned16(scratch.p), &p.splits, &p.chunk);
+    if (p.splits > 1 && !scratch.has(workspace_of(a, p.splits))) plan(a, false, &p.splits, &p.chunk);
     p.scale = static_cast<float>(a.scale);
     p.scale_log2 = static_cast<float>(a.scale * 1.4426950408889634);
     const size_t slots = static_cast<size_t>(a.B * a.Hkv) * p.splits;
-    p.part_o = static_cast<float*>(workspace);
+    p.part_o = static_cast<float*>(scratch.p);
     p.part_ml = p.part_o ? p.part_o + slots * kMaxRows * a.D : nullptr;
     const dim3 grid(p.splits, static_cast<unsigned>(a.B * a.Hkv));
     p.mask = static_cast<const unsigned char*>(a.mask);

@@ -982,7 +982,7 @@ bool flash_uses_wide(const paras_sdpa_args& a) {
     return flash::wide_supported(a.B, a.Hq, a.Lq, a.Lk, static_cast<int>(a.D), a.mask_kind, a.is_causal != 0);
 }
 
-int launch_flash(const paras_sdpa_args& a, void* workspace, hipStream_t s) {
+int launch_flash(const paras_sdpa_args& a, Scratch scratch, hipStream_t s) {
     FlashParams p{};
     p.q = static_cast<const std::uint16_t*>(a.q);
     p.k = static_cast<const std::uint16_t*>(a.k);
@@ -1007,10 +1007,10 @@ int launch_flash(const paras_sdpa_args& a, void* workspace, hipStream_t s) {
     const bool causal = a.is_causal != 0;
     const int mk = a.mask_kind;
     const Shares r = plan_shares(a);
-    if (r.parts > 1 && workspace != nullptr) {
+    if (r.parts > 1 && scratch.has(flash_workspace(a)) && aligned16(scratch.p)) {
         p.n_parts = r.parts;
         p.part_tiles = r.part_tiles;
-        p.part_o = static_cast<float*>(workspace);
+        p.part_o = static_cast<float*>(scratch.p);
         p.part_ml = p.part_o + static_cast<size_t>(a.B * a.Hq) * ((a.Lq + kBM - 1) / kBM) * r.parts * kBM * a.D;
     }
     if (flash_uses_wide(a)) return launch_flash_wide(p, causal, a.dtype == PARAS_BF16, s);

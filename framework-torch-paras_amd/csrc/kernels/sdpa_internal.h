@@ -8,22 +8,34 @@
 
 namespace paras {
 
-// MFMA flash forward: bf16/f16, D == Dv in {64, 128}, no explicit mask
-// (causal or none), no attention weights returned.
+// Device memory that a caller brings, and how much of it there is.
+struct Scratch {
+    void*  p = nullptr;
+    size_t bytes = 0;
+    bool has(size_t n) const { return p != nullptr && bytes >= n; }
+    // what is left of it past the first n bytes
+    Scratch past(size_t n) const { return has(n) ? Scratch{static_cast<char*>(p) + n, bytes - n} : Scratch{}; }
+};
+
+// MFMA flash forward: bf16/f16, D == Dv in {64, 128, 256}, causal or with a boolean or additive mask,
+// no attention weights returned.
 bool   flash_supported(const paras_sdpa_args& a);
-// Workspace for the parts of a problem with too few query tiles to fill the chip; without it (null) launch_flash does not share
-// out the keys.
+// Workspace for the parts of a problem with too few query tiles to fill the chip; without it, or with less, launch_flash does not
+// share out the keys.
 size_t flash_workspace(const paras_sdpa_args& a);
-int    launch_flash(const paras_sdpa_args& a, void* workspace, hipStream_t s);
+int    launch_flash(const paras_sdpa_args& a, Scratch scratch, hipStream_t s);
 // Whether launch_flash takes its 64-queries-per-wavefront form (head size 128, no mask, enough
 // long rows to fill the chip with one workgroup per CU); only meaningful when flash_supported.
 bool flash_uses_wide(const paras_sdpa_args& a);
 
 // Split-KV decode: short query (Lq * Hq/Hkv <= 16), long K/V, bf16/f16,
-// D == Dv in {64, 128}, optional bool / additive mask, not causal.
+// D == Dv in {64, 128, 256}, optional bool / additive mask, not causal.
 bool   decode_supported(const paras_sdpa_args& a);
+// Workspace for the splits of the keys; without it, or with less, launch_decode does not split them.
 size_t decode_workspace(const paras_sdpa_args& a);
-int    launch_decode(const paras_sdpa_args& a, void* workspace, hipStream_t s);
+// Enough KV heads for two workgroups per CU without a split.
+bool   decode_fills_chip(const paras_sdpa_args& a);
+int    launch_decode(const paras_sdpa_args& a, Scratch scratch, hipStream_t s);
 
 // MFMA attention that also returns the softmax weights (the math op): bf16/f16,
 // D == Dv in {64, 128}, causal / bool / additive masks contiguous along the keys.

@@ -151,7 +151,7 @@ void run(Prepared* p, Tensor* out, Tensor* attn, Tensor* lse) {
     const size_t nws = paras_sdpa_workspace(&a);
     Tensor ws;
     if (nws > 0) ws = workspace(nws, p->q.device());
-    check(paras_sdpa_fwd(&a, nws > 0 ? ws.data_ptr() : nullptr, st));
+    check(paras_sdpa_fwd_ws(&a, nws > 0 ? ws.data_ptr() : nullptr, nws, st));
 }
 
 std::tuple<Tensor, Tensor> sdpa_math(const Tensor& query, const Tensor& key, const Tensor& value,

@@ -67,6 +67,7 @@ SIGNATURES = {
     "paras_rotate_half": (i32, [vp, vp, i64, i64, i32, i32, vp]),
     "paras_sdpa_workspace": (sz, [C.POINTER(SdpaArgs)]),
     "paras_sdpa_fwd": (i32, [C.POINTER(SdpaArgs), vp, vp]),
+    "paras_sdpa_fwd_ws": (i32, [C.POINTER(SdpaArgs), vp, sz, vp]),
     "paras_sdpa_kernel_name": (C.c_char_p, [C.POINTER(SdpaArgs)]),
     "paras_moe_route_workspace": (sz, [i64, i64, i64]),
     "paras_moe_route": (i32, [vp, i64, i64, i64, i32, vp, vp, vp, vp, vp, vp, vp, vp]),
@@ -213,7 +214,7 @@ def sdpa(q, k, v, mask=None, is_causal=False, scale=None, want_attn=False, want_
     name = lib().paras_sdpa_kernel_name(C.byref(a)).decode()
     nws = lib().paras_sdpa_workspace(C.byref(a))
     ws = torch.empty(nws, dtype=torch.uint8, device=q.device) if nws else None
-    check(lib().paras_sdpa_fwd(C.byref(a), _ptr(ws), _stream()))
+    check(lib().paras_sdpa_fwd_ws(C.byref(a), _ptr(ws), nws, _stream()))
     return out, attn, lse, name
 
 

@@ -239,7 +239,13 @@ typedef struct paras_sdpa_args {
  * strides decide, and whether attn is NULL; with 16-bit tensors the pointers' alignment to 16 bytes
  * counts as well, so ask with the pointers of the call. */
 PARAS_API size_t paras_sdpa_workspace(const paras_sdpa_args* args);
-/* `workspace` may be NULL when paras_sdpa_workspace() returned 0. */
+/* The flash and decode kernels share a head's keys out over workgroups where that is faster and
+ * `workspace_bytes` are at least what paras_sdpa_workspace() answers, 16-byte aligned; with less, or NULL, they
+ * do not.  The other kernels cannot do without what they ask for: PARAS_ERR_INVALID. */
+PARAS_API int paras_sdpa_fwd_ws(const paras_sdpa_args* args, void* workspace, size_t workspace_bytes, void* stream);
+/* The same from a caller that does not say how much memory `workspace` is.  Nothing is written to it by the
+ * flash kernels, nor by the decode kernel where there are two KV heads per CU (B * Hkv, 512 on MI355X): they
+ * share no keys out.  Otherwise it holds paras_sdpa_workspace() bytes, and may be NULL where that is 0. */
 PARAS_API int paras_sdpa_fwd(const paras_sdpa_args* args, void* workspace, void* stream);
 /* Name of the kernel paras_sdpa_fwd would pick: "flash_mfma" (bf16 / f16 heads of
  * 64, 128 or 256 elements; "flash_mfma_wide" where its 64-queries-per-wavefront

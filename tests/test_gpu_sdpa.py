@@ -168,6 +168,69 @@ def test_flash_with_the_keys_shared_out(D, kind, dtype):
     assert seen_parts
 
 
+@pytest.mark.parametrize("kind", ["none", "causal", "bool", "additive", "decode", "decode-bool"])
+@pytest.mark.parametrize("dtype,D", [(torch.bfloat16, 64), (torch.float16, 128), (torch.bfloat16, 256)])
+def test_scratch_memory_is_written_within_its_size_only(dtype, D, kind):
+    """Problems whose keys are shared out where there is room for it.  Without a size (paras_sdpa_fwd), with none, too small a
+    one or one off 16 bytes: not shared out and not one byte written, the same bits each way.  With the size asked for: that many bytes
+    and no more.  Both forms against fp64 (a few steps of the type on sums of unit variance)."""
+    decode = kind.startswith("decode")
+    B, Hq, Hkv, Lq, Lk = (65, 16, 8, 1, 2000) if decode else (1, 2, 1, 1300, 1300) if kind == "causal" else (1, 2, 1, 300, 2500)
+    q, k, v = (torch.randn(B, h, n, D, device="cuda").to(dtype) for h, n in ((Hq, Lq), (Hkv, Lk), (Hkv, Lk)))
+    mask = None
+    if kind.endswith("bool"):
+        mask = torch.rand(B, 1, 1 if decode else Lq, Lk, device="cuda") < 0.7
+        mask[..., 0] = True
+    elif kind == "additive":
+        mask = torch.randn(B, 1, Lq, Lk, device="cuda").to(dtype)
+    out = torch.empty_like(q)
+    a = capi.sdpa_args(q, k, v, out, mask=mask, is_causal=kind == "causal", scale=O.round_to_dtype(1 / math.sqrt(D), dtype))
+    L, st = capi.lib(), torch.cuda.current_stream().cuda_stream
+    need = L.paras_sdpa_workspace(C.byref(a))
+    assert need > 0 and L.paras_sdpa_kernel_name(C.byref(a)) == (b"decode_split" if decode else b"flash_mfma")
+    room = torch.full((need + 4096,), 0xA5, dtype=torch.uint8, device="cuda")
+    p = room.data_ptr()
+
+    def result(call):
+        out.fill_(math.nan)
+        capi.check(call())
+        return out.clone()
+
+    whole = result(lambda: L.paras_sdpa_fwd(C.byref(a), None, st))
+    for call in (lambda: L.paras_sdpa_fwd(C.byref(a), p, st), lambda: L.paras_sdpa_fwd_ws(C.byref(a), None, 0, st), lambda: L.paras_sdpa_fwd_ws(C.byref(a), None, need, st),
+                 lambda: L.paras_sdpa_fwd_ws(C.byref(a), p, need - 1, st), lambda: L.paras_sdpa_fwd_ws(C.byref(a), p + 8, need, st)):
+        assert_bit_exact(result(call), whole)
+        assert bool((room == 0xA5).all())
+    shared = result(lambda: L.paras_sdpa_fwd_ws(C.byref(a), p, need, st))
+    assert bool((room[need:] == 0xA5).all()) and not bool((room[:need] == 0xA5).all())
+    for b in range(0, B, 13):
+        s = q[b].double() @ k[b].double().repeat_interleave(Hq // Hkv, 0).transpose(-1, -2).contiguous() * a.scale
+        if kind == "causal":
+            s = s.masked_fill(~torch.ones(Lq, Lk, device="cuda").tril().bool(), -math.inf)
+        elif mask is not None:
+            s = s.masked_fill(~mask[b], -math.inf) if mask.dtype == torch.bool else s + mask[b].double()
+        want = s.softmax(-1) @ v[b].double().repeat_interleave(Hq // Hkv, 0)
+        for got in (whole[b], shared[b]):
+            assert (got.double() - want).abs().max().item() <= (2.5e-2 if dtype == torch.bfloat16 else 4e-3)
+
+
+@pytest.mark.parametrize("dtype,D,Lq", [(torch.bfloat16, 80, 300), (torch.float64, 64, 512), (torch.float32, 66, 512)])
+def test_kernels_that_need_their_scratch_memory_refuse_less(dtype, D, Lq):
+    """The padded and the composed route with one byte too few, or none: an error, and neither output nor scratch written."""
+    q, k, v = (torch.randn(1, 4, Lq, D, device="cuda").to(dtype) for _ in range(3))
+    out = torch.full_like(q, 7)
+    a = capi.sdpa_args(q, k, v, out)
+    L, st = capi.lib(), torch.cuda.current_stream().cuda_stream
+    need = L.paras_sdpa_workspace(C.byref(a))
+    room = torch.full((need,), 0xA5, dtype=torch.uint8, device="cuda")
+    assert need > 0
+    for p, n in ((room.data_ptr(), need - 1), (None, need), (room.data_ptr(), 0)):
+        assert L.paras_sdpa_fwd_ws(C.byref(a), p, n, st) == -1
+    assert bool((room == 0xA5).all()) and bool((out == 7).all())
+    capi.check(L.paras_sdpa_fwd_ws(C.byref(a), room.data_ptr(), need, st))
+    assert not bool((out == 7).all())
+
+
 @pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])
 @pytest.mark.parametrize("D", [64, 128, 256])
 def test_flash_key_padding_leaves_out_closed_tiles(D, dtype):
