@@ -1,15 +1,12 @@
-// Register-staged tile mainloops of the grouped expert GEMMs (128-row tiles, and 256-row ones that
-// gemm_flex.h's 32-bit offsets do not reach): C tile = A[rows x K] * B[256 x K]^T with bf16/fp16
-// operands and fp32 accumulation on v_mfma_f32_32x32x16.
+// Register-staged tile mainloop of the grouped expert GEMMs, for rows that gemm_flex.h's 32-bit byte offsets do not
+// reach: C tile = A[256 rows x K] * B[256 x K]^T with bf16/fp16 operands and fp32 accumulation on v_mfma_f32_32x32x16.
 //
 // Both operands are read along their contiguous contraction dim, which is the
 // 8-element-per-lane operand layout of the MFMA, so neither needs a transpose.
 // The 256 B rows come as two groups of 128 (gate / up weights, or two adjacent
-// column blocks) and each wave owns 64x64 of each group: 128 fp32 accumulators
-// per lane.  k-tile 64, global -> registers -> LDS with the next k-tile's loads
-// in flight during the MFMAs.  Two shapes: 128 rows with 4 waves arranged 2x2
-// (two workgroups per CU, each with a single LDS stage), and 256 rows with 8
-// waves arranged 4x2 (one workgroup per CU, two LDS stages, namespace wide).
+// column blocks).  Eight waves arranged 4 x 2, each with 64 x 64 of both groups: 128 fp32 accumulators
+// per lane.  k-tile 64, global -> registers -> LDS, two LDS stages, one workgroup per CU.  Offsets are in
+// elements from 64-bit bases.
 #pragma once
 
 #include <hip/hip_runtime.h>
@@ -22,8 +19,8 @@ namespace paras {
 namespace gemm {
 
 constexpr int kThreads = 256;
-constexpr int kBM = 128;
-constexpr int kBN = 128;          // columns per group; a workgroup computes two groups
+constexpr int kBM = 128;          // the dense 128 x 128 tile (paras_gemm_nt_ws)
+constexpr int kBN = 128;          // its columns, and those of a group here; a workgroup computes two groups
 constexpr int kBK = 64;
 constexpr int kLS = kBK + 8;      // LDS row stride (elements): 16 consecutive rows hit distinct banks.  (Unpadded rows
                                   // with an XOR swizzle of the chunks measured no faster.)
@@ -42,108 +39,6 @@ template <> struct MmaT<f16_t> {
     }
 };
 
-
-template <int G>     // G column groups of 128
-struct TileLdsG {
-    std::uint16_t a[kBM * kLS];
-    std::uint16_t b[G][kBN * kLS];
-};
-using TileLds = TileLdsG<2>;
-
-// a_off[i] / b_off[g][i]: element offsets (from the uniform bases a_base / b_base[g]) of this
-// thread's four 16-byte chunks per operand row set at k = 0 (chunk c = tid + i*256 -> tile row
-// c/8, column (c%8)*8).  32-bit offsets against a scalar base keep the addressing out of the
-// vector registers; callers check that every operand spans fewer than 2^32 elements.
-// Accumulates into acc[g][mi][ni]; lane (column lr = lane%32, half lh = lane/32) of
-// block (mi, ni) ends up holding rows (r/4)*8 + 4*lh + r%4, r = 0..15.
-template <typename T, int G>
-__device__ __forceinline__ void tile_mainloop(const std::uint16_t* a_base, const unsigned (&a_off)[4],
-                                              const std::uint16_t* const (&b_base)[G], const unsigned (&b_off)[G][4],
-                                              long K, TileLdsG<G>& lds, float16_t (&acc)[G][2][2]) {
-    const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
-    const int lr = lane & 31, lh = lane >> 5;
-    const int wm = wave >> 1, wn = wave & 1;
-    std::uint16_t* a_lds = lds.a;
-    std::uint16_t (*b_lds)[kBN * kLS] = lds.b;
-    u32x4 a_st[4], b_st[G][4];
-    auto load_tile = [&](long k0) {
-#pragma unroll
-        for (int i = 0; i < 4; ++i) a_st[i] = load16(a_base + k0 + a_off[i]);
-#pragma unroll
-        for (int g = 0; g < G; ++g)
-#pragma unroll
-            for (int i = 0; i < 4; ++i) b_st[g][i] = load16(b_base[g] + k0 + b_off[g][i]);
-    };
-    auto store_tile = [&]() {
-#pragma unroll
-        for (int i = 0; i < 4; ++i) {
-            const int c = tid + i * kThreads;
-            const int off = (c >> 3) * kLS + (c & 7) * 8;
-            *reinterpret_cast<u32x4*>(&a_lds[off]) = a_st[i];
-#pragma unroll
-            for (int g = 0; g < G; ++g) *reinterpret_cast<u32x4*>(&b_lds[g][off]) = b_st[g][i];
-        }
-    };
-
-#pragma unroll
-    for (int g = 0; g < G; ++g)
-#pragma unroll
-        for (int mi = 0; mi < 2; ++mi)
-#pragma unroll
-            for (int ni = 0; ni < 2; ++ni)
-#pragma unroll
-                for (int r = 0; r < 16; ++r) acc[g][mi][ni][r] = 0.f;
-
-    const int a_off0 = (wm * 64 + lr) * kLS + lh * 8;
-    const int b_off0 = (wn * 64 + lr) * kLS + lh * 8;
-    const long k_tiles = K / kBK;
-    load_tile(0);
-    store_tile();
-    __syncthreads();
-    for (long kt = 0; kt < k_tiles; ++kt) {
-        if (kt + 1 < k_tiles) load_tile((kt + 1) * kBK);
-        // Fixed issue order, fenced slot by slot: one MFMA per slot, the fragments of the next
-        // k-step requested while the current one computes (A into a second register pair right
-        // away, each B fragment back into its own registers as soon as its two MFMAs have
-        // issued), so an operand is asked for about six MFMAs before it is used.
-        constexpr int Q = 2 * G;               // B fragments per k-step
-        i16x8 af[2][2], bf[Q];
-        auto read_a = [&](int buf, int ks) {
-#pragma unroll
-            for (int mi = 0; mi < 2; ++mi)
-                af[buf][mi] = *reinterpret_cast<const i16x8*>(&a_lds[a_off0 + mi * 32 * kLS + ks * 16]);
-        };
-        auto read_b = [&](int q, int ks) {   // q = 2*g + ni
-            bf[q] = *reinterpret_cast<const i16x8*>(&b_lds[q >> 1][b_off0 + (q & 1) * 32 * kLS + ks * 16]);
-        };
-        read_a(0, 0);
-#pragma unroll
-        for (int q = 0; q < Q; ++q) read_b(q, 0);
-#pragma unroll
-        for (int ks = 0; ks < kBK / 16; ++ks) {
-            const int cur = ks & 1;
-            const bool more = ks + 1 < kBK / 16;
-#pragma unroll
-            for (int q = 0; q < Q; ++q)
-#pragma unroll
-                for (int mi = 0; mi < 2; ++mi) {
-                    acc[q >> 1][mi][q & 1] = MmaT<T>::run(af[cur][mi], bf[q], acc[q >> 1][mi][q & 1]);
-                    if (more && q == 0 && mi == 0) read_a(cur ^ 1, ks + 1);
-                    if (more && mi == 1) read_b(q, ks + 1);
-                    __builtin_amdgcn_sched_barrier(0);
-                }
-        }
-        __syncthreads();
-        if (kt + 1 < k_tiles) {
-            store_tile();
-            __syncthreads();
-        }
-    }
-
-}
-
-// The same per-wave work (64 x 64 of each column group) with eight waves arranged 4 x 2 over a
-// 256 x (2 x 128) tile: a third fewer global loads and LDS stores per flop than the 128-row tile.
 // The eight waves move in step (one barrier per k-tile), so LDS is double buffered and a k-tile is
 // in registers for a whole tile time before it is stored.
 namespace wide {
@@ -159,8 +54,11 @@ struct TileLds {
     StageLds st[2];
 };
 
-// a_off[i]: chunk c = tid + i*512 -> tile row c/8, column (c%8)*8 (i < 4); b_off[g][i]: the same
-// for the 128 rows of column group g (i < 2).
+// a_off[i] / b_off[g][i]: element offsets (from the uniform bases a_base / b_base[g]) of this thread's 16-byte chunks at
+// k = 0: chunk c = tid + i*512 -> tile row c/8, column (c%8)*8 (i < 4; for the 128 rows of column group g i < 2).  32-bit
+// offsets against a scalar base keep the addressing out of the vector registers; callers check that every operand spans
+// fewer than 2^32 elements.  Accumulates into acc[g][mi][ni]; lane (column lr = lane%32, half lh = lane/32) of block
+// (mi, ni) ends up holding rows (r/4)*8 + 4*lh + r%4, r = 0..15.
 template <typename T>
 __device__ __forceinline__ void tile_mainloop(const std::uint16_t* a_base, const unsigned (&a_off)[4],
                                               const std::uint16_t* const (&b_base)[2], const unsigned (&b_off)[2][2],
@@ -344,38 +242,6 @@ __device__ __forceinline__ void narrow_block(const float16_t& a, std::uint16_t (
         for (int r = 0; r < 16; ++r) o[r] = Elem<T>::from_f32(a[r]);
     }
 }
-
-// The two tile shapes as a kernel sees them.
-template <int G>
-struct Tile128G {
-    static constexpr int kBM = gemm::kBM, kThreads = gemm::kThreads, kBChunks = 4, kGroups = G;
-    static constexpr int kShortRows = 0;    // no short-tile form
-    using Lds = TileLdsG<G>;
-    template <typename T>
-    __device__ static __forceinline__ void mainloop(const std::uint16_t* a_base, const unsigned (&a_off)[4],
-                                                    const std::uint16_t* const (&b_base)[G], const unsigned (&b_off)[G][4],
-                                                    long K, Lds& lds, float16_t (&acc)[G][2][2]) {
-        tile_mainloop<T, G>(a_base, a_off, b_base, b_off, K, lds, acc);
-    }
-};
-using Tile128 = Tile128G<2>;
-struct Tile256 {
-    static constexpr int kBM = wide::kBM, kThreads = wide::kThreads, kBChunks = 2, kGroups = 2;
-    using Lds = wide::TileLds;
-    template <typename T>
-    __device__ static __forceinline__ void mainloop(const std::uint16_t* a_base, const unsigned (&a_off)[4],
-                                                    const std::uint16_t* const (&b_base)[2], const unsigned (&b_off)[2][2],
-                                                    long K, Lds& lds, float16_t (&acc)[2][2][2]) {
-        wide::tile_mainloop<T>(a_base, a_off, b_base, b_off, K, lds, acc);
-    }
-    static constexpr int kShortRows = 64;   // a tile with no more valid rows than this can take short_mainloop
-    template <typename T>
-    __device__ static __forceinline__ void short_mainloop(const std::uint16_t* a_base, unsigned a_off0,
-                                                          const std::uint16_t* const (&b_base)[2], const unsigned (&b_off)[2][2],
-                                                          long K, Lds& lds, float16_t (&acc)[2]) {
-        wide::short_tile_mainloop<T>(a_base, a_off0, b_base, b_off, K, lds, acc);
-    }
-};
 
 }  // namespace gemm
 }  // namespace paras

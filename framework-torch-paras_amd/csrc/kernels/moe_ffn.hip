@@ -14,11 +14,10 @@
 // contraction dim, which is exactly the 8-element-per-lane operand layout of
 // v_mfma_f32_32x32x16, so neither operand needs a transpose.
 //
-// Tiling: a workgroup computes 128 or 256 routed rows x two 128-column groups (gate and up columns
-// n0..n0+127 for GEMM 1; columns n0..n0+255 for GEMM 2), k-tile 64.  128 rows (gemm_tile.h): waves arranged
-// 2x2 with 64x64 per column group each (128 fp32 accumulators per lane), global -> registers -> LDS.  256
-// rows, when the experts hold enough rows for them: four waves with 128 x 128 each on v_mfma_f32_16x16x32
-// (256 accumulators per lane), loads straight to LDS (gemm_flex.h; grouped_gemm_direct_kernel).  Rows of one
+// Tiling: 32 to 256 routed rows x 128 or 256 weight rows (gate and up rows of the same columns for GEMM 1), k-tile 64, four
+// waves on v_mfma_f32_16x16x32 with loads straight to LDS (gemm_flex.h; grouped_tile_kernel, grouped_gemm_direct_kernel), the
+// tile chosen by an estimate (grouped_form); few rows per expert on kernels that stream the weights (grouped_few_rows_kernel); an x
+// beyond a 32-bit byte offset on register-staged 256-row tiles (gemm_tile.h; grouped_gemm_kernel).  Rows of one
 // expert are contiguous in the routed order; m-tiles never straddle experts (the grid is sized for the
 // worst case and surplus workgroups exit).
 #include <hip/hip_runtime.h>
@@ -65,11 +64,14 @@ inline void division_by(unsigned d, unsigned* m, int* s) {
     *m = static_cast<unsigned>(((1ull << *s) + d - 1) / d);
 }
 
-template <typename T, bool kSwiglu, typename S>
-__global__ __launch_bounds__(S::kThreads, 2) void grouped_gemm_kernel(const FfnGemmParams p) {
+// ---- register-staged 256-row tiles, for an x whose rows are out of a 32-bit byte offset's reach (from 3.76 GB; also
+// PARAS_GEMM_EIGHT_WAVES).  8 experts, top-2, H 4096: 8192 tokens, I 14336 5149 us, on the other tiles 4956; 65536 tokens, I 1792
+// 5834 and 5620; H 2048, I 4096, 1024 tokens 206 and 200.
+template <typename T, bool kSwiglu>
+__global__ __launch_bounds__(wide::kThreads, 2) void grouped_gemm_kernel(const FfnGemmParams p) {
     using El = Elem<T>;
-    constexpr int kBM = S::kBM;
-    __shared__ __attribute__((aligned(16))) typename S::Lds lds;
+    constexpr int kBM = wide::kBM, kThreads = wide::kThreads, kShortRows = 64;
+    __shared__ __attribute__((aligned(16))) wide::TileLds lds;
 
     // ---- tile coordinates.  Linear id L: xcd = L % 8 (hardware round-robin);
     // within an XCD walk (column group, m-tile, column-in-group).
@@ -110,10 +112,10 @@ __global__ __launch_bounds__(S::kThreads, 2) void grouped_gemm_kernel(const FfnG
     const int wm = wave >> 1, wn = wave & 1;
 
     // ---- global -> register staging: 16-byte chunks, 8 per row of a k-tile
-    unsigned a_off[4], b_off[2][S::kBChunks];
+    unsigned a_off[4], b_off[2][2];
 #pragma unroll
     for (int i = 0; i < 4; ++i) {
-        const int c = tid + i * S::kThreads;
+        const int c = tid + i * kThreads;
         long prow = row0 + (c >> 3);
         if (prow >= row_end) prow = row_end - 1;  // clamp: result rows beyond the expert are not stored
         const long src = p.order ? static_cast<long>((static_cast<unsigned long long>(static_cast<unsigned>(p.order[prow])) * p.div_m) >> p.div_s) : prow;
@@ -124,35 +126,33 @@ __global__ __launch_bounds__(S::kThreads, 2) void grouped_gemm_kernel(const FfnG
 #pragma unroll
     for (int g = 0; g < 2; ++g)
 #pragma unroll
-        for (int i = 0; i < S::kBChunks; ++i) {
-            const int c = tid + i * S::kThreads;
+        for (int i = 0; i < 2; ++i) {
+            const int c = tid + i * kThreads;
             long wrow = (kSwiglu ? n0 : n0 + g * kBN) + (c >> 3);
             if (wrow >= p.Nw) wrow = p.Nw - 1;
             b_off[g][i] = static_cast<unsigned>(wrow * p.K + (c & 7) * 8);
         }
     // An expert's last tile with few rows: the waves share those rows (same sums, a fraction of
     // the time) instead of most of them idling through the contraction.
-    if constexpr (S::kShortRows > 0) {
-        if (row_end - row0 <= S::kShortRows) {
-            float16_t sacc[2];
-            S::template short_mainloop<T>(p.a, a_off[0], b_base, b_off, p.K, lds, sacc);
-            const long col = n0 + (wave & 3) * 32 + lr;
+    if (row_end - row0 <= kShortRows) {
+        float16_t sacc[2];
+        wide::short_tile_mainloop<T>(p.a, a_off[0], b_base, b_off, p.K, lds, sacc);
+        const long col = n0 + (wave & 3) * 32 + lr;
 #pragma unroll
-            for (int r = 0; r < 16; ++r) {
-                const long prow = row0 + (wave >> 2) * 32 + (r >> 2) * 8 + 4 * lh + (r & 3);
-                if (prow >= row_end) continue;
-                if (kSwiglu) {
-                    if (col < p.N) p.c[prow * p.N + col] = swiglu_from_acc<T>(sacc[0][r], sacc[1][r]);
-                } else {
-                    if (col < p.N) p.c[prow * p.N + col] = El::from_f32(sacc[0][r]);
-                    if (col + kBN < p.N) p.c[prow * p.N + col + kBN] = El::from_f32(sacc[1][r]);
-                }
+        for (int r = 0; r < 16; ++r) {
+            const long prow = row0 + (wave >> 2) * 32 + (r >> 2) * 8 + 4 * lh + (r & 3);
+            if (prow >= row_end) continue;
+            if (kSwiglu) {
+                if (col < p.N) p.c[prow * p.N + col] = swiglu_from_acc<T>(sacc[0][r], sacc[1][r]);
+            } else {
+                if (col < p.N) p.c[prow * p.N + col] = El::from_f32(sacc[0][r]);
+                if (col + kBN < p.N) p.c[prow * p.N + col + kBN] = El::from_f32(sacc[1][r]);
             }
-            return;
         }
+        return;
     }
     float16_t acc[2][2][2];
-    S::template mainloop<T>(p.a, a_off, b_base, b_off, p.K, lds, acc);
+    wide::tile_mainloop<T>(p.a, a_off, b_base, b_off, p.K, lds, acc);
 
     // ---- epilogue.  Accumulator lane (column lr, half lh) holds rows (r/4)*8 + 4*lh + r%4.
     // One uniform base, a 32-bit byte offset per lane (the launcher sends output rows of 2^22
@@ -900,14 +900,29 @@ void launch_form(int form, FfnGemmParams g, hipStream_t s) {
     }
 }
 
-template <typename T, typename S>
-int run_ffn_shape(const void* x, const void* w_gate, const void* w_up, const void* w_down, const float* topw,
+// The register-staged tiles' grid: an XCD sweeps up to two column units together (one expert's weight panel for them is
+// 4 MB at K = 4096, the size of an XCD's L2; 4 units measured 8 % slower), fewer when there are not enough units to keep all 8
+// XCDs busy.
+template <typename T, bool kSwiglu>
+void launch_register_staged(FfnGemmParams g, hipStream_t s) {
+    const long cols = kSwiglu ? kBN : 2 * kBN;
+    g.mt_total = static_cast<int>((g.R + wide::kBM - 1) / wide::kBM) + g.E;
+    g.n_units = static_cast<int>((g.N + cols - 1) / cols);
+    g.ngt = g.n_units < 16 ? 1 : 2;
+    const long groups = (g.n_units + 8 * g.ngt - 1) / (8 * g.ngt);
+    hipLaunchKernelGGL((grouped_gemm_kernel<T, kSwiglu>), dim3(static_cast<unsigned>(groups * 8 * g.ngt * g.mt_total)), dim3(wide::kThreads), 0, s, g);
+}
+
+template <typename T>
+int run_ffn_tiles(const void* x, const void* w_gate, const void* w_up, const void* w_down, const float* topw,
             const long* order, const long* inv_order, const long* offsets, void* out, void* workspace, long T_,
             int E, int k, long H, long I, hipStream_t s) {
     const long R = T_ * k;
     auto* h = static_cast<std::uint16_t*>(workspace);
     auto* y = reinterpret_cast<std::uint16_t*>(static_cast<char*>(workspace) + align_up(static_cast<size_t>(R) * I * 2, 256));
-    const int mt_total = static_cast<int>((R + S::kBM - 1) / S::kBM) + E;
+    // By form, unless x is out of a 32-bit byte offset's reach (weights are aimed at from a tile's first row: paras_moe_ffn's limit on H and I
+    // is theirs).  PARAS_GEMM_EIGHT_WAVES: the register-staged tiles whatever the size, for tests and measurements; looked up per call.
+    const bool by_form = T_ * H * 2 <= flex::kMaxExtent && std::getenv("PARAS_GEMM_EIGHT_WAVES") == nullptr;
 
     FfnGemmParams g1{};
     g1.a = static_cast<const std::uint16_t*>(x);
@@ -918,44 +933,21 @@ int run_ffn_shape(const void* x, const void* w_gate, const void* w_up, const voi
     g1.offsets = offsets;
     g1.a_bytes = T_ * H * 2;
     g1.K = H; g1.N = I; g1.Nw = I; g1.R = R; g1.E = E; g1.k = k;
-    g1.mt_total = mt_total;
     division_by(static_cast<unsigned>(k), &g1.div_m, &g1.div_s);
-    g1.n_units = static_cast<int>((I + kBN - 1) / kBN);
-    // Column units an XCD sweeps together: up to 2 (one expert's weight panel for them is
-    // 4 MB at K = 4096, the size of an XCD's L2; 4 units measured 8 % slower), fewer when
-    // there are not enough units to keep all 8 XCDs busy.
-    auto plan = [](FfnGemmParams& g) {
-        int ngt = g.n_units / 8;
-        g.ngt = ngt < 1 ? 1 : (ngt > 2 ? 2 : ngt);
-    };
-    auto grid_of = [&](const FfnGemmParams& g) {
-        const long groups = (g.n_units + 8 * g.ngt - 1) / (8 * g.ngt);
-        return static_cast<unsigned>(groups * 8 * g.ngt * g.mt_total);
-    };
-    plan(g1);
-    // By form (grouped_form), unless rows or weights are out of a 32-bit byte offset's reach, from the start of x and from a
-    // tile's first weight row (PARAS_GEMM_EIGHT_WAVES: the eight-wave tile of 32 x 32 x 16 MFMAs where it applies, for measurements).
-    static const bool eight_waves = std::getenv("PARAS_GEMM_EIGHT_WAVES") != nullptr;
-    const bool by_form = !(eight_waves && S::kBM == 256) && T_ * H * 2 <= flex::kMaxExtent && H <= flex::kMaxLd && I <= flex::kMaxLd;
     if (by_form) launch_form<T, true>(grouped_form(true, E, R, I, H), g1, s);
-    else
-        hipLaunchKernelGGL((grouped_gemm_kernel<T, true, S>), dim3(grid_of(g1)), dim3(S::kThreads), 0, s, g1);
+    else         launch_register_staged<T, true>(g1, s);
     PARAS_HIP_TRY(hipGetLastError());
 
     FfnGemmParams g2{};
     g2.a = h;
     g2.b = static_cast<const std::uint16_t*>(w_down);
-    g2.b2 = g2.b;  // column group 1 = the next 128 weight rows, selected through the row index
+    g2.b2 = g2.b;  // (register-staged) column group 1 = the next 128 weight rows, selected through the row index
     g2.c = y;
     g2.order = nullptr;
     g2.offsets = offsets;
     g2.K = I; g2.N = H; g2.Nw = H; g2.R = R; g2.E = E; g2.k = k;
-    g2.mt_total = mt_total;
-    g2.n_units = static_cast<int>((H + 2 * kBN - 1) / (2 * kBN));
-    plan(g2);
     if (by_form) launch_form<T, false>(grouped_form(false, E, R, H, I), g2, s);
-    else
-        hipLaunchKernelGGL((grouped_gemm_kernel<T, false, S>), dim3(grid_of(g2)), dim3(S::kThreads), 0, s, g2);
+    else         launch_register_staged<T, false>(g2, s);
     PARAS_HIP_TRY(hipGetLastError());
 
     const long total = T_ * (H / 8);
@@ -1012,9 +1004,6 @@ int run_ffn_few_rows(const void* x, const void* w_gate, const void* w_up, const 
     return PARAS_OK;
 }
 
-// 256-row tiles when the experts are big enough for them: an expert's last tile is half empty on
-// average, so the rows per expert should be many times the tile, and there must be tiles for at
-// least half the CUs.
 template <typename T>
 int run_ffn(const void* x, const void* w_gate, const void* w_up, const void* w_down, const float* topw,
             const long* order, const long* inv_order, const long* offsets, void* out, void* workspace, long T_,
@@ -1028,10 +1017,7 @@ int run_ffn(const void* x, const void* w_gate, const void* w_up, const void* w_d
     const long few_limit = few_env != nullptr ? std::atol(few_env) : (H * I >= 20'000'000L ? 16 : 8);
     if (R <= few_limit * E && E <= 65535 && T_ * H * 2 <= stream::kMaxExtent && R * I * 2 <= stream::kMaxExtent)
         return run_ffn_few_rows<T>(x, w_gate, w_up, w_down, topw, order, inv_order, offsets, out, workspace, T_, E, k, H, I, s);
-    const long wide_tiles = (R / Tile256::kBM) * ((H + 2 * kBN - 1) / (2 * kBN));
-    if (R / E >= 4 * Tile256::kBM && wide_tiles >= 128)
-        return run_ffn_shape<T, Tile256>(x, w_gate, w_up, w_down, topw, order, inv_order, offsets, out, workspace, T_, E, k, H, I, s);
-    return run_ffn_shape<T, Tile128>(x, w_gate, w_up, w_down, topw, order, inv_order, offsets, out, workspace, T_, E, k, H, I, s);
+    return run_ffn_tiles<T>(x, w_gate, w_up, w_down, topw, order, inv_order, offsets, out, workspace, T_, E, k, H, I, s);
 }
 
 }  // namespace
@@ -1059,7 +1045,7 @@ int paras_moe_ffn(const void* x, const void* w_gate, const void* w_up, const voi
     // tensors; anything else goes to the general kernels (any size, any alignment).
     const bool aligned = ((reinterpret_cast<uintptr_t>(x) | reinterpret_cast<uintptr_t>(w_gate) | reinterpret_cast<uintptr_t>(w_up) |
                            reinterpret_cast<uintptr_t>(w_down) | reinterpret_cast<uintptr_t>(out) | reinterpret_cast<uintptr_t>(workspace)) & 15) == 0;
-    const bool tiles = H % kBK == 0 && I % kBK == 0 && aligned && H < (1LL << 22) && I < (1LL << 22);   // (the tiles' stores use 32-bit byte offsets within a tile)
+    const bool tiles = H % kBK == 0 && I % kBK == 0 && aligned && H < flex::kMaxLd && I < flex::kMaxLd;   // (the tiles' loads and stores use 32-bit byte offsets within a tile)
     PARAS_REQUIRE(T * k <= 0x3fffffffLL, "paras_moe_ffn: too many routed rows");
     if (T * H >= (1LL << 32) || T * k * I >= (1LL << 32) || I * H >= (1LL << 32))
         return fail(PARAS_ERR_UNSUPPORTED, "paras_moe_ffn: an operand (x, the routed intermediate, or one expert's weight matrix) spans 2^32 elements or more");

@@ -478,3 +478,36 @@ def test_ffn_tiles_of_every_form(shape, dtype):
     assert_ffn_close(got[fin], ref[fin], dtype)
     bad = set((~out.isfinite()).any(dim=1).nonzero().flatten().tolist())
     assert {5} <= bad <= {5, T // 2}
+
+
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])
+@pytest.mark.parametrize("shape", [(1843, 70, 6, 192, 256), (395, 70, 6, 640, 192), (2756, 4, 1, 768, 320), (2581, 8, 2, 320, 256)])
+def test_ffn_register_staged_tiles(shape, dtype, monkeypatch):
+    """The tiles of an x beyond a 32-bit byte offset, at sizes where rows, columns and experts end inside them: the same uneven
+    layers as above, and last tiles of a row to a whole tile."""
+    monkeypatch.setenv("PARAS_GEMM_EIGHT_WAVES", "1")
+    test_ffn_tiles_of_every_form(shape, dtype)
+    if shape[1] == 8:
+        test_ffn_rows_in_the_last_tile_of_every_expert(dtype)
+        test_ffn_last_tiles_at_the_edges_of_their_forms(2112, dtype)
+
+
+def test_ffn_tokens_beyond_a_32_bit_byte_offset():
+    """x of more than 3.76 GB (the extent that a byte offset of the direct loads covers): the first and last tokens and some
+    between against fp64 on the device, each narrowed where the layer narrows."""
+    T, E, k, H, I, dt = 459_000, 8, 1, 4096, 64, torch.bfloat16
+    assert T * H * 2 > 0xE0000000
+    torch.manual_seed(3)
+    logits = torch.randn(T, E, device="cuda").to(dt)
+    x = torch.randn(T, H, device="cuda", dtype=dt)
+    wg, wu, wd = (0.02 * torch.randn(E, I, H, device="cuda")).to(dt), (0.02 * torch.randn(E, I, H, device="cuda")).to(dt), (0.1 * torch.randn(E, H, I, device="cuda")).to(dt)
+    route = [t.cuda() for t in O.moe_route(logits.cpu(), k)]
+    out = capi.moe_ffn(x, wg, wu, wd, route[1], route[2], route[3], route[5], k)
+    sel = torch.cat([torch.arange(8), torch.arange(T - 200, T), torch.randperm(T)[:64]]).cuda()
+    for t in sel.tolist():
+        e, v = int(route[0][t, 0]), x[t].double()
+        g, u = (v @ wg[e].double().T.contiguous()).to(dt).double(), (v @ wu[e].double().T.contiguous()).to(dt).double()
+        h = (g / (1 + torch.exp(-g)) * u).to(dt).double()
+        want = (h @ wd[e].double().T.contiguous()).to(dt).double()
+        # (fp32 sums may round a gate, an up value or a result the other way: a step of 2^-8 of it, a few of 64 terms)
+        assert (out[t].double() - want).norm().item() <= 1e-2 * want.norm().item(), t
