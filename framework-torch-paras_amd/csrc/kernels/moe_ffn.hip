@@ -1009,13 +1009,17 @@ int run_ffn(const void* x, const void* w_gate, const void* w_up, const void* w_d
             const long* order, const long* inv_order, const long* offsets, void* out, void* workspace, long T_,
             int E, int k, long H, long I, hipStream_t s) {
     const long R = T_ * k;
-    // Few routed rows per expert on average: the few-row kernels (an expert with more than 32 rows takes them 32 at a time).  Up to 8, and
-    // up to 16 where the weights are long enough for their stream to decide.  Few-row kernels / tiles: 8 experts, top-2, H 4096,
-    // I 14336 40 tokens 480 / 551 us, 64 tokens 528 / 544, 128 tokens 823 / 602; H 1216, I 512 57 tokens 16 / 8; 64 experts, top-6, H 576,
-    // I 10944 133 tokens 587 / 516; 16 experts H 832, I 3776 61 tokens (8 rows each) 68 / 60.  PARAS_MOE_FEW_ROWS = n moves the limit (0: never).
-    static const char* few_env = std::getenv("PARAS_MOE_FEW_ROWS");
-    const long few_limit = few_env != nullptr ? std::atol(few_env) : (H * I >= 20'000'000L ? 16 : 8);
-    if (R <= few_limit * E && E <= 65535 && T_ * H * 2 <= stream::kMaxExtent && R * I * 2 <= stream::kMaxExtent)
+    // The few-row kernels (an expert with more than 32 rows takes them 32 at a time) spend a workgroup's start on every 16 weight rows
+    // of every expert, and a row's products on all of them; the tiles' down-projection is E H / 128 workgroups that walk the whole of I each.
+    // So: the fewer rows and experts and the longer I.  1410 layers (1 to 64 experts, 0.4 to 64 rows each, H 512 to 4096, I 512 to 14336): this rule
+    // costs 1.1 % over the better of the two in the mean and 8 % at the 95th percentile, the best limit on rows per expert alone 3.4 % and 21 %.
+    // Few-row kernels / tiles: 4 experts of 11 rows, H 1280, I 9920 81 / 105 us; 8 of 10, 704 x 3072 38 / 45; 8 experts, top-2, 4096 x 14336, 1 token
+    // 128 / 168, 5 tokens 369 / 380, 64 tokens 507 / 479, 128 tokens 757 / 509; 64 of 4, 768 x 1472 118 / 94; 32 of 13, 704 x 3200 115 / 97.  Beyond
+    // 16 rows on average some experts have more than 32: 4 of 30, 1088 x 2176 46 / 28.
+    // PARAS_MOE_FEW_ROWS = n: up to n rows per expert instead (0: never); looked up per call.
+    const char* env = std::getenv("PARAS_MOE_FEW_ROWS");
+    const bool few = env != nullptr ? R <= std::atol(env) * E : 4 * R * E <= I && R <= 16L * E;
+    if (few && E <= 65535 && T_ * H * 2 <= stream::kMaxExtent && R * I * 2 <= stream::kMaxExtent)
         return run_ffn_few_rows<T>(x, w_gate, w_up, w_down, topw, order, inv_order, offsets, out, workspace, T_, E, k, H, I, s);
     return run_ffn_tiles<T>(x, w_gate, w_up, w_down, topw, order, inv_order, offsets, out, workspace, T_, E, k, H, I, s);
 }

@@ -511,3 +511,25 @@ def test_ffn_tokens_beyond_a_32_bit_byte_offset():
         want = (h @ wd[e].double().T.contiguous()).to(dt).double()
         # (fp32 sums may round a gate, an up value or a result the other way: a step of 2^-8 of it, a few of 64 terms)
         assert (out[t].double() - want).norm().item() <= 1e-2 * want.norm().item(), t
+
+
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])
+@pytest.mark.parametrize("T", [40, 64])
+def test_ffn_few_rows_per_expert_at_any_size(T, dtype, monkeypatch):
+    """The few-row kernels where tiles would be chosen: experts with more than 32 rows, and rows at the edges of their blocks."""
+    monkeypatch.setenv("PARAS_MOE_FEW_ROWS", "1000")
+    test_ffn_few_rows_per_expert(T, dtype)
+    for rows in (8, 9, 16, 17, 33):
+        test_ffn_few_rows_at_the_edges_of_the_activation_blocks(rows)
+
+
+@pytest.mark.parametrize("T,E,k,I", [(16, 4, 1, 256), (17, 4, 1, 256), (64, 4, 1, 1024), (65, 4, 1, 1088), (64, 8, 2, 4096), (65, 8, 2, 4224), (3, 1, 1, 64)])
+def test_ffn_either_side_of_the_limits_for_few_rows(T, E, k, I):
+    """4 R E <= I, and 16 rows per expert: whole and one more."""
+    H, dt = 192, torch.bfloat16
+    torch.manual_seed(T)
+    x = torch.randn(T, H).to(dt)
+    wg, wu, wd = (0.07 * torch.randn(E, I, H)).to(dt), (0.07 * torch.randn(E, I, H)).to(dt), (0.02 * torch.randn(E, H, I)).to(dt)
+    topi, topw, order, inv, counts, offsets = capi.moe_route(torch.randn(T, E).to(dt).cuda(), k)
+    out = capi.moe_ffn(x.cuda(), wg.cuda(), wu.cuda(), wd.cuda(), topw, order, inv, offsets, k)
+    assert_ffn_close(out, O.moe_ffn(x, wg, wu, wd, topw.cpu(), order.cpu(), inv.cpu(), offsets.cpu(), k), dt)
