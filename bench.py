@@ -3,19 +3,19 @@
 
     python bench.py [--gpus 1] [--steps K] [--warmup W] [--workload NAME] [--no-cpu]
 
-Prints ONE JSON line.  The headline value is BASELINE.json's first metric:
-bf16 causal flash-attention forward at B=4, H=32, S=4096, D=128 (configs[2]) in
+Prints ONE JSON line.  The headline value is that of
+bf16 causal flash-attention forward at B=4, H=32, S=4096, D=128 in
 TFLOP/s, counted with the causal-halved figure 4*B*H*S^2*D/2.  The same line
 carries, under "workloads", the other configurations the metric names
-(RMSNorm and SwiGLU of configs[1] in GB/s, the GQA decode of configs[3], the
-MoE layer of configs[4]), the dense projection GEMM and the backward / RoPE
+(RMSNorm 16384x4096 and SwiGLU 16384x14336 in GB/s, the GQA decode of 64 sequences over 8192 keys,
+the MoE layer of 8192 tokens and 8 experts), the dense projection GEMM and the backward / RoPE
 helper ops that sit either side of the path, each with its own roofline object.
 
 A step is one pass of the workload's kernels over one batch of synthetic
 inputs that are resident in HBM before the timed region.  Inputs are drawn the
 way the reference's tests draw theirs: torch.manual_seed(0) at the start of
-each workload, torch-CPU randn (N(0,1) / N(1,0.02) / N(0,0.02) as BASELINE.json
-states), then moved to the device.  Kernels are called through the C ABI of
+each workload, torch-CPU randn (N(0,1) / N(1,0.02) / N(0,0.02)),
+then moved to the device.  Kernels are called through the C ABI of
 libparas_hip.so on torch's current stream; per-launch durations come from HIP
 events recorded on that same stream.  Every workload first makes untimed
 launches for a fixed wall time (SETTLE_MS / SETTLE_MFMA_MS, whatever --warmup
@@ -175,7 +175,7 @@ def main() -> int:
             t += mean
         return t.to(dtype)
 
-    # ------------------------------------------------------------------ configs[2]
+    # ------------------------------------------------------------------ causal prefill attention
     if want("sdpa_prefill"):
         torch.manual_seed(0)
         B, H, S, D = 4, 32, 4096, 128
@@ -190,7 +190,7 @@ def main() -> int:
         flops = 4 * B * H * S * S * D / 2          # causal-halved
         tf = flops / ms / 1e9
         results["sdpa_prefill"] = {
-            "workload": "bf16 causal flash-attention fwd B=4 H=32 S=4096 D=128 (configs[2])",
+            "workload": "bf16 causal flash-attention fwd B=4 H=32 S=4096 D=128",
             "value": round(tf, 2), "unit": "TFLOP/s", "ms_per_step": round(ms, 4), "wall_ms_per_step": round(wall, 4),
             "kernel": "flash_wide_kernel<bf16,causal>" if wide else "flash_fwd_kernel<bf16,128,causal>",
             "algorithmic_flops_per_launch": flops,
@@ -262,7 +262,7 @@ def main() -> int:
         checks["sdpa_weights"] = check_weights
         del q, k, v, out, attn
 
-    # ------------------------------------------------------------------ configs[1]
+    # ------------------------------------------------------------------ RMSNorm, then SwiGLU
     if want("rmsnorm_swiglu"):
         torch.manual_seed(0)
         rows, Hd, I = 16384, 4096, 14336
@@ -292,7 +292,7 @@ def main() -> int:
         bytes_s = 3 * n * 2
         gbs_s = bytes_s / ms_s / 1e6
         results["rmsnorm_swiglu"] = {
-            "workload": "bf16 fused RMSNorm 16384x4096 (eps 1e-6) then SwiGLU 16384x14336 (configs[1])",
+            "workload": "bf16 fused RMSNorm 16384x4096 (eps 1e-6) then SwiGLU 16384x14336",
             "value": round((bytes_r + bytes_s) / (ms_r + ms_s) / 1e6, 1), "unit": "GB/s",
             "ms_per_step": round(ms_r + ms_s, 4),
             "rms_norm": {"ms": round(ms_r, 4), "algorithmic_bytes_per_launch": bytes_r, "kernel": "rms_norm_fwd_vec<bf16,2>",
@@ -315,7 +315,7 @@ def main() -> int:
         checks["rmsnorm_swiglu"] = check_rs
         del gate, up, so, xc, gc_, uc
 
-    # ------------------------------------------------------------------ configs[3]
+    # ------------------------------------------------------------------ decode attention
     if want("sdpa_decode"):
         torch.manual_seed(0)
         B, Hq, Hkv, Lk, D = 64, 32, 8, 8192, 128
@@ -330,7 +330,7 @@ def main() -> int:
         nbytes = 2 * B * Hkv * Lk * D * 2 + 2 * B * Hq * D * 2
         gbs = nbytes / ms / 1e6
         results["sdpa_decode"] = {
-            "workload": "bf16 GQA decode SDPA B=64 Hq=32 Hkv=8 Lq=1 Lk=8192 D=128 (configs[3])",
+            "workload": "bf16 GQA decode SDPA B=64 Hq=32 Hkv=8 Lq=1 Lk=8192 D=128",
             "value": round(gbs, 1), "unit": "GB/s", "ms_per_step": round(ms, 4),
             "tokens_per_s": round(B / ms * 1e3, 1), "kernel": "decode_split_kernel<bf16> + decode_combine_kernel",
             "algorithmic_bytes_per_launch": nbytes, "roofline": roofline("hbm", gbs, "decode_split_kernel"),
@@ -346,7 +346,7 @@ def main() -> int:
         checks["sdpa_decode"] = check_decode
         del q, k, v, out, ws, qc, kc, vc
 
-    # ------------------------------------------------------------------ configs[4]
+    # ------------------------------------------------------------------ MoE layer
     if want("moe"):
         torch.manual_seed(0)
         T, Hd, E, kk, I = 8192, 4096, 8, 2, 14336
@@ -378,7 +378,7 @@ def main() -> int:
         flops = T * kk * 3 * 2 * Hd * I
         tf = flops / ms_ffn / 1e9
         results["moe"] = {
-            "workload": "bf16 MoE layer T=8192 H=4096 E=8 top-2 I=14336: routing + grouped expert FFN (configs[4])",
+            "workload": "bf16 MoE layer T=8192 H=4096 E=8 top-2 I=14336: routing + grouped expert FFN",
             "value": round(T / ms_all * 1e3, 1), "unit": "tokens/s", "ms_per_step": round(ms_all, 4), "steps": msteps,
             "route_ms": round(ms_route, 4), "ffn_ms": round(ms_ffn, 4), "ffn_tflops": round(tf, 2),
             "kernel": "grouped_gemm_direct_kernel<bf16> (gate-up+SwiGLU, down) + moe_combine_kernel",
@@ -422,7 +422,7 @@ def main() -> int:
         flops = 2 * M * N * K
         tf = flops / ms / 1e9
         results["linear"] = {
-            "workload": "bf16 dense NT GEMM x W^T: M=16384 N=4096 K=4096 (nn.Linear of configs[2]'s tokens)",
+            "workload": "bf16 dense NT GEMM x W^T: M=16384 N=4096 K=4096 (nn.Linear over 16384 tokens)",
             "value": round(tf, 2), "unit": "TFLOP/s", "ms_per_step": round(ms, 4), "kernel": "gemm_flex_kernel<bf16>",
             "algorithmic_flops_per_launch": flops, "roofline": roofline("mfma", tf, "gemm_flex_kernel"),
         }

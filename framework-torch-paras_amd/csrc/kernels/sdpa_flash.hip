@@ -939,7 +939,8 @@ namespace {
 // have keys), four tiles of keys at least (two), if the tiles a workgroup is spared, in us, are more than the second
 // kernel's 4.5 us and the parts' way out and in.  In bf16 and fp16, B1 H2 S4393 D64: none 43.8 -> 24.9, causal 50.0 -> 23.4, key-padding
 // mask 89 -> 34; D128 59 -> 36, 64 -> 28, 115 -> 47; D256 B1 H2 S2000 56 -> 29, 59 -> 29, 74 -> 34.  (B2 H8 S963, 128 tiles, D128 none: 18.5
-// whole, 25.7 in two parts.)
+// whole, 25.7 in two parts.)  Of 150 drawn problems that it shares out none is slower than whole, 1.70 times as fast in the mean; the nearest
+// to the line: fp16 D128 none B1 H4 S1050 19.1 -> 18.5, D256 additive B1 H8 S824 37.3 -> 36.2, causal D64 B5 H1 S868 13.5 -> 12.6.
 //   Halves within a workgroup, D <= 128: two waves per SIMD help where a wave waits or works outside the matrix cores, and under the causal
 // rule they shorten the last tiles; without mask and rule they cost as much as they give.  B12 H1 S1499 D64, mask 35.3 -> 27.0; B3 H4 S2377
 // D128, mask 63 -> 56; B1 H8 S8192 D128, causal 159 -> 137; B1 H32 S512 D64, mask 13.9 -> 12.7, D128, causal 13.4 -> 14.9 (eight

@@ -192,7 +192,7 @@ for t in (out, y):
 
 
 def test_256_row_tiles_on_eight_waves_give_the_same_bits():
-    """PARAS_GEMM_EIGHT_WAVES=1 (read once per process, hence the child process) sends the 256-row tiles of the
+    """PARAS_GEMM_EIGHT_WAVES=1 sends the tiles of the
     expert FFN to the eight-wave kernel on 32 x 32 x 16 MFMAs.  It adds the same products in the same order as the
     four-wave kernel on 16 x 16 x 32: identical outputs, compared by digest.  (The dense product, which has no such
     form, is along as the control: the switch leaves it alone.)"""

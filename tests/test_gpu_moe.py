@@ -192,7 +192,7 @@ def test_operands_that_are_not_16_byte_aligned(dtype):
 
 
 def test_config5_routing_exact_and_sampled_tokens():
-    """BASELINE config 5 (T=8192 H=4096 E=8 top-2 I=14336 bf16) at full size:
+    """The benchmark's layer (T=8192 H=4096 E=8 top-2 I=14336 bf16) at full size:
     routing bit-exact on all tokens, the FFN on 48 sampled tokens against the
     oracle (a token's output depends only on its own row and routing)."""
     T, H, E, k, I = 8192, 4096, 8, 2, 14336
@@ -203,7 +203,7 @@ def test_config5_routing_exact_and_sampled_tokens():
     got = capi.moe_route(logits.cuda(), k)
     want = O.moe_route(logits, k)
     for name, g, w in zip(NAMES, got, want):
-        assert_bit_exact(g, w, f"config 5 moe_route {name}")
+        assert_bit_exact(g, w, f"full-size moe_route {name}")
     topi, topw, order, inv, counts, offsets = got
     out = capi.moe_ffn(x.cuda(), wg.cuda(), wu.cuda(), wd.cuda(), topw, order, inv, offsets, k)
     assert not bool(out.isnan().any())

@@ -34,7 +34,7 @@ def max_abs(a, b):
 
 
 def test_config1_fp32_causal():
-    """B=1 H=8 S=128 D=64 fp32, N(0,1), seed 0, scale 1/sqrt(D)."""
+    """The reference's own test size: B=1 H=8 S=128 D=64 fp32, N(0,1), seed 0, scale 1/sqrt(D)."""
     q, k, v = torch.randn(1, 8, 128, 64), torch.randn(1, 8, 128, 64), torch.randn(1, 8, 128, 64)
     out, attn, lse, name = run(q, k, v, is_causal=True, want_attn=True, want_lse=True)
     want, wattn = O.sdpa_math(q, k, v, is_causal=True, gemm="aten")
@@ -779,7 +779,7 @@ def test_error_conventions():
 
 
 def test_config3_shape_properties_and_slice():
-    """BASELINE config 3 (bf16 causal B=4 H=32 S=4096 D=128) at full size: a
+    """The benchmark's prefill (bf16 causal B=4 H=32 S=4096 D=128) at full size: a
     slice against the oracle, the whole output through properties."""
     B, H, S, D = 4, 32, 4096, 128
     q, k, v = torch.randn(B, H, S, D).bfloat16(), torch.randn(B, H, S, D).bfloat16(), torch.randn(B, H, S, D).bfloat16()
@@ -838,7 +838,7 @@ def test_flash_wide_kernel_matches_oracle(B, Hq, Hkv, Lq, Lk, causal, dtype):
 
 
 def test_config4_shape_slice_and_gqa_equivalence():
-    """BASELINE config 4 (bf16 GQA decode B=64 Hq=32 Hkv=8 Lk=8192 D=128)."""
+    """The benchmark's decode (bf16 GQA decode B=64 Hq=32 Hkv=8 Lk=8192 D=128)."""
     B, Hq, Hkv, Lk = 64, 32, 8, 8192
     q = torch.randn(B, Hq, 1, 128).bfloat16()
     k, v = torch.randn(B, Hkv, Lk, 128).bfloat16(), torch.randn(B, Hkv, Lk, 128).bfloat16()

@@ -22,7 +22,7 @@ from ffn_bar import assert_ffn_close
 
 
 def test_two_host_evaluations_of_the_expert_ffn_differ_by_one_step_beyond_2e_2():
-    """64 tokens of BASELINE config 5's shape (H 4096, I 14336, top-2, weights 0.02 N(0,1), bf16; two
+    """64 tokens of the benchmark's MoE layer (H 4096, I 14336, top-2, weights 0.02 N(0,1), bf16; two
     experts so that the weights fit in seconds): ATen's GEMM against the oracle's C GEMM."""
     torch.manual_seed(0)
     T, H, E, k, I = 64, 4096, 2, 2, 14336
