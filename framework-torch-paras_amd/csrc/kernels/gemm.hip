@@ -407,11 +407,12 @@ bool few_rows_by_tiles(long M, long N, long batch) {
 // From 33 rows on the staged tiles are faster but for short contractions of few weight rows, where their start is most of
 // the call: few-row kernels / tiles, 33 x 512 x 512 4.3 / 4.9 us, 48 x 3072 x 512 4.8 / 5.2, 64 x 1024 x 512 5.0 / 5.1, 64 x 4096 x 256 4.1 / 4.4;
 // 64 x 4096 x 512 5.7 / 5.4, 40 x 2048 x 1024 7.0 / 6.7, 64 x 1024 x 1024 7.2 / 6.5, 33 x 6144 x 512 6.5 / 5.3, 56 x 4384 x 256 4.9 / 4.4,
-// 63 x 7192 x 1024 12.5 / 7.0, 108 x 7456 x 6656 110 / 36.  Where the tiles want the contraction in parts and the caller has no workspace for
+// 63 x 7192 x 1024 12.5 / 7.0, 108 x 7456 x 6656 110 / 36; 128 products of 64 x 64 x 64 3.7 / 4.2, two of 100 x 512 x 64 3.7 / 4.1,
+// eight of 128 x 512 x 64 4.1 / 4.3; two of 100 x 128 x 128 4.0 / 4.0, 128 of 33 x 512 x 64 6.0 / 6.0.  Where the tiles want the contraction in parts and the caller has no workspace for
 // them, and for paras_gemm_nt, the few-row kernels stay up to kSkinnyMaxM rows.
 bool few_rows_up_to(long M, long N, long K, long batch, bool parts_or_whole) {
     if (M <= kFewRowsM) return true;
-    return parts_or_whole ? M <= 64 && M * K <= 36000 && N * batch <= 4096 : M <= kSkinnyMaxM;
+    return M <= kSkinnyMaxM && (!parts_or_whole || (K <= 64 && M * N * batch <= 1 << 19) || (M <= 64 && M * K <= 36000 && N * batch <= 4096));
 }
 
 // Few output columns and many rows: the few-row kernels with the operands in each other's place.  Up to

@@ -538,12 +538,12 @@ def test_gemm_tiles_with_several_stages(shape, dtype):
 
 
 @pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16, torch.float32])
-@pytest.mark.parametrize("shape", [(8, 512, 1024), (33, 512, 512), (64, 4096, 512), (65, 512, 512), (64, 4104, 512), (64, 512, 576), (128, 2048, 2048), (700, 24, 512),
+@pytest.mark.parametrize("shape", [(8, 512, 1024), (33, 512, 512), (64, 4096, 512), (65, 512, 512), (64, 4104, 512), (64, 512, 576), (128, 4096, 64), (128, 4104, 64), (65, 256, 128), (128, 2048, 2048), (700, 24, 512),
                                    (96, 1000, 72), (300, 136, 14336)])
 def test_scratch_is_asked_for_once_and_the_route_is_the_planned_one(shape, dtype):
     """paras_gemm_scratch: the size that paras_gemm_workspace answers, once, or no question where that is 0, and the bits of
     paras_gemm -- with that workspace, and without any where none is wanted: the route is one choice.  Either side of the rules
-    for 33 to 64 rows (512 x 64 and 4096 weight rows), few columns, other contractions, parts.  No memory: an error before
+    for 33 to 64 rows (and for 65 to 128 with a contraction of 64), few columns, other contractions, parts.  No memory: an error before
     anything is launched."""
     M, N, K = shape
     torch.manual_seed(M + N + K)
