@@ -394,8 +394,6 @@ __global__ __launch_bounds__(256) void skinny_splitk_finish_kernel(const DensePa
     (p.c + bidx * p.sc)[row * p.ldc + col] = El::from_f32(v);
 }
 
-// Splits of the contraction for the workspace kernel (0 = it does not apply): enough workgroups to
-// fill the chip twice, at least two slabs each.
 // Few rows but many columns (a vocabulary projection, a fused gate-up projection at M = 64 ... 128):
 // from about 200 tiles of 128 x 128 the tile kernel streams the weights faster than the few-row
 // kernels do (M = 128, N = 128256, K = 4096: 267 against 649 us; N = 28672: 75 against 106 us; at
@@ -444,6 +442,8 @@ int tile_splitk_plan(long M, long N, long K, long batch, long* k_per_split) {
     return static_cast<int>(splits);
 }
 
+// Splits of the contraction for the workspace kernel (0 = it does not apply): enough workgroups to
+// fill the chip twice, at least two slabs each.
 int splitk_plan(long M, long N, long K, long batch, int* pieces_per_split) {
     if (M < 32 || M > kSkinnyMaxM || K % 64 != 0 || N < 512) return 0;   // up to 16 rows the activations are no load
     if (few_rows_by_tiles(M, N, batch)) return 0;
