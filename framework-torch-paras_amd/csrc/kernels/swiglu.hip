@@ -19,14 +19,54 @@ namespace {
 
 constexpr int kBlock  = 256;
 
-// kUnroll: 16-byte vectors per stream per lane per iteration.
+// One 16-byte vector of results.  16-bit types: every element through the fp32 tier, without a branch; the few whose value is next to a
+// rounding boundary (or outside the tier's range) are redone in fp64 in a loop that runs as often as the lane with the most of
+// them needs.  A wave of eight elements a lane then comes to the fp64 formula 0.3 (bf16) or 0.7 (fp16) times instead of 0.5 or 3.2.
+template <typename T>
+__device__ __forceinline__ u32x4 swiglu_vec(u32x4 gv, u32x4 uv) {
+    using E = Elem<T>;
+    using S = typename E::store_t;
+    const S* ge = reinterpret_cast<const S*>(&gv);
+    const S* ue = reinterpret_cast<const S*>(&uv);
+    u32x4 o;
+    S* oe = reinterpret_cast<S*>(&o);
+    if constexpr (sizeof(S) == 2) {
+        unsigned redo = 0;
+        S r[8];
+#pragma unroll
+        for (int j = 0; j < 8; ++j) {
+            bool ok;
+            r[j] = swiglu_fast<T>(ge[j], ue[j], ok);
+            redo |= ok ? 0u : (1u << j);
+        }
+        while (redo != 0) {
+            const int j = __builtin_ctz(redo);
+            redo &= redo - 1;
+            S g16 = 0, u16 = 0;
+#pragma unroll
+            for (int k = 0; k < 8; ++k)
+                if (k == j) { g16 = ge[k]; u16 = ue[k]; }
+            const S x = swiglu_exact<T>(E::to_f32(g16), E::to_f32(u16));
+#pragma unroll
+            for (int k = 0; k < 8; ++k)
+                if (k == j) r[k] = x;
+        }
+#pragma unroll
+        for (int j = 0; j < 4; ++j) o[j] = r[2 * j] | (static_cast<std::uint32_t>(r[2 * j + 1]) << 16);
+    } else {
+#pragma unroll
+        for (int j = 0; j < E::kVec; ++j) oe[j] = swiglu_one<T>(ge[j], ue[j]);
+    }
+    return o;
+}
+
+// kUnroll: 16-byte vectors per stream per lane per iteration.  `tail`: elements past the last whole vector, the last workgroup's (a launch
+// of their own cost 4.5 us behind 43 M elements, and as much of the host's time as the first).
 template <typename T, int kUnroll>
 __global__ __launch_bounds__(kBlock) void swiglu_fwd_vec(
     const typename Elem<T>::store_t* __restrict__ gate, const typename Elem<T>::store_t* __restrict__ up,
-    typename Elem<T>::store_t* __restrict__ out, long nvec) {
-    using E = Elem<T>;
-    using S = typename E::store_t;
-    constexpr int V = E::kVec;
+    typename Elem<T>::store_t* __restrict__ out, long nvec, int tail) {
+    constexpr int V = Elem<T>::kVec;
     const long stride = static_cast<long>(gridDim.x) * kBlock * kUnroll;
     for (long base = static_cast<long>(blockIdx.x) * kBlock * kUnroll + threadIdx.x; base < nvec;
          base += stride) {
@@ -42,25 +82,21 @@ __global__ __launch_bounds__(kBlock) void swiglu_fwd_vec(
 #pragma unroll
         for (int k = 0; k < kUnroll; ++k) {
             const long i = base + static_cast<long>(k) * kBlock;
-            if (i < nvec) {
-                const S* ge = reinterpret_cast<const S*>(&gv[k]);
-                const S* ue = reinterpret_cast<const S*>(&uv[k]);
-                u32x4 o;
-                S* oe = reinterpret_cast<S*>(&o);
-#pragma unroll
-                for (int j = 0; j < V; ++j) oe[j] = swiglu_one<T>(ge[j], ue[j]);
-                store16_nt(out + i * V, o);
-            }
+            if (i < nvec) store16_nt(out + i * V, swiglu_vec<T>(gv[k], uv[k]));
         }
+    }
+    if (blockIdx.x + 1 == gridDim.x && static_cast<int>(threadIdx.x) < tail) {
+        const long i = nvec * V + threadIdx.x;
+        out[i] = swiglu_one<T>(gate[i], up[i]);
     }
 }
 
 template <typename T>
 __global__ __launch_bounds__(kBlock) void swiglu_fwd_any(
     const typename Elem<T>::store_t* __restrict__ gate, const typename Elem<T>::store_t* __restrict__ up,
-    typename Elem<T>::store_t* __restrict__ out, long first, long n) {
+    typename Elem<T>::store_t* __restrict__ out, long n) {
     const long stride = static_cast<long>(gridDim.x) * kBlock;
-    for (long i = first + static_cast<long>(blockIdx.x) * kBlock + threadIdx.x; i < n; i += stride)
+    for (long i = static_cast<long>(blockIdx.x) * kBlock + threadIdx.x; i < n; i += stride)
         out[i] = swiglu_one<T>(gate[i], up[i]);
 }
 
@@ -92,7 +128,7 @@ __global__ __launch_bounds__(kBlock) void swiglu_bwd_vec(const std::uint16_t* __
                                                          const std::uint16_t* __restrict__ gate,
                                                          const std::uint16_t* __restrict__ up,
                                                          std::uint16_t* __restrict__ ggate,
-                                                         std::uint16_t* __restrict__ gup, long nvec) {
+                                                         std::uint16_t* __restrict__ gup, long nvec, int tail) {
     using E = Elem<T>;
     for (long i = static_cast<long>(blockIdx.x) * kBlock + threadIdx.x; i < nvec; i += static_cast<long>(gridDim.x) * kBlock) {
         const u32x4 dv = load16_nt(go + i * 8), gv = load16_nt(gate + i * 8), uv = load16_nt(up + i * 8);
@@ -131,6 +167,10 @@ __global__ __launch_bounds__(kBlock) void swiglu_bwd_vec(const std::uint16_t* __
         }
         store16_nt(ggate + i * 8, wg);
         store16_nt(gup + i * 8, wu);
+    }
+    if (blockIdx.x + 1 == gridDim.x && static_cast<int>(threadIdx.x) < tail) {        // (past the last whole vector)
+        const long i = nvec * 8 + threadIdx.x;
+        swiglu_bwd_exact<T>(E::to_f32(go[i]), E::to_f32(gate[i]), E::to_f32(up[i]), ggate[i], gup[i]);
     }
 }
 
@@ -250,7 +290,6 @@ int launch_swiglu_fwd(const void* gate, const void* up, void* out, long n, hipSt
     auto* o = static_cast<S*>(out);
     const bool aligned = ((reinterpret_cast<uintptr_t>(gate) | reinterpret_cast<uintptr_t>(up) |
                            reinterpret_cast<uintptr_t>(out)) % 16) == 0;
-    long done = 0;
     if (aligned && n >= V) {
         // Four vectors per lane keep enough bytes under way where there are waves enough; with fewer the arithmetic of one vector
         // after the other decides, for longer where it is the two tiers of 16-bit results (bf16, four / one: 14336 vectors 5.3 / 2.9 us,
@@ -260,16 +299,13 @@ int launch_swiglu_fwd(const void* gate, const void* up, void* out, long n, hipSt
         long blocks = (nvec + kBlock * unroll - 1) / (kBlock * unroll);
         if (blocks > 0x7fffffffL) blocks = 0x7fffffffL;  // the kernel grid-strides beyond that
         const dim3 grid(static_cast<unsigned>(blocks));
-        if (unroll == 1) hipLaunchKernelGGL((swiglu_fwd_vec<T, 1>), grid, dim3(kBlock), 0, s, g, u, o, nvec);
-        else             hipLaunchKernelGGL((swiglu_fwd_vec<T, 4>), grid, dim3(kBlock), 0, s, g, u, o, nvec);
-        PARAS_HIP_TRY(hipGetLastError());
-        done = nvec * V;
+        const int tail = static_cast<int>(n - nvec * V);
+        if (unroll == 1) hipLaunchKernelGGL((swiglu_fwd_vec<T, 1>), grid, dim3(kBlock), 0, s, g, u, o, nvec, tail);
+        else             hipLaunchKernelGGL((swiglu_fwd_vec<T, 4>), grid, dim3(kBlock), 0, s, g, u, o, nvec, tail);
+    } else {
+        hipLaunchKernelGGL((swiglu_fwd_any<T>), dim3(stream_grid(kBlock, n)), dim3(kBlock), 0, s, g, u, o, n);
     }
-    if (done < n) {
-        hipLaunchKernelGGL((swiglu_fwd_any<T>), dim3(stream_grid(kBlock, n - done)), dim3(kBlock), 0, s, g,
-                           u, o, done, n);
-        PARAS_HIP_TRY(hipGetLastError());
-    }
+    PARAS_HIP_TRY(hipGetLastError());
     return PARAS_OK;
 }
 
@@ -282,7 +318,6 @@ int launch_swiglu_bwd(const void* go, const void* gate, const void* up, void* gg
     const auto* u = static_cast<const S*>(up);
     auto* og = static_cast<S*>(ggate);
     auto* ou = static_cast<S*>(gup);
-    long done = 0;
     if constexpr (sizeof(S) == 2) {
         const bool aligned = ((reinterpret_cast<uintptr_t>(go) | reinterpret_cast<uintptr_t>(gate) | reinterpret_cast<uintptr_t>(up) |
                                reinterpret_cast<uintptr_t>(ggate) | reinterpret_cast<uintptr_t>(gup)) % 16) == 0;
@@ -290,16 +325,14 @@ int launch_swiglu_bwd(const void* go, const void* gate, const void* up, void* gg
             const long nvec = n / 8;
             long blocks = (nvec + kBlock - 1) / kBlock;
             if (blocks > 0x7fffffffL) blocks = 0x7fffffffL;  // the kernel grid-strides beyond that
-            hipLaunchKernelGGL((swiglu_bwd_vec<T>), dim3(static_cast<unsigned>(blocks)), dim3(kBlock), 0, s, d, g, u, og, ou, nvec);
+            hipLaunchKernelGGL((swiglu_bwd_vec<T>), dim3(static_cast<unsigned>(blocks)), dim3(kBlock), 0, s, d, g, u, og, ou, nvec,
+                               static_cast<int>(n - nvec * 8));
             PARAS_HIP_TRY(hipGetLastError());
-            done = nvec * 8;
+            return PARAS_OK;
         }
     }
-    if (done < n) {
-        hipLaunchKernelGGL((swiglu_bwd_any<T>), dim3(stream_grid(kBlock, n - done)), dim3(kBlock), 0, s, d + done, g + done,
-                           u + done, og + done, ou + done, n - done);
-        PARAS_HIP_TRY(hipGetLastError());
-    }
+    hipLaunchKernelGGL((swiglu_bwd_any<T>), dim3(stream_grid(kBlock, n)), dim3(kBlock), 0, s, d, g, u, og, ou, n);
+    PARAS_HIP_TRY(hipGetLastError());
     return PARAS_OK;
 }
 

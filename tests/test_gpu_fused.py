@@ -299,6 +299,32 @@ def test_swiglu_backward_every_gate_value(dtype):
 
 
 @pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])
+def test_swiglu_tiers_for_every_gate_and_many_values(dtype):
+    """The error bounds of the fp32 tier hold for every gate: each one with 24 random up and grad_out values of many magnitudes, so that
+    every distance from a rounding boundary turns up (any element that stood with a wrong rounding differs by a bit)."""
+    g = torch.Generator().manual_seed(23)
+    gate = torch.arange(-32768, 32768, dtype=torch.int32).to(torch.int16).view(dtype).repeat(24)
+    gate = gate[gate.isfinite()]
+    up, dy = ((torch.randn(gate.numel(), generator=g) * 2.0 ** torch.randint(-6, 7, (gate.numel(),), generator=g)).to(dtype) for _ in range(2))
+    assert_bit_exact(capi.swiglu(dev(gate), dev(up)), O.swiglu(gate, up), "swiglu")
+    gg, gu = capi.swiglu_backward(dev(dy), dev(gate), dev(up))
+    wgg, wgu = O.swiglu_backward(dy, gate, up)
+    assert_bit_exact(gg, wgg, "grad_gate")
+    assert_bit_exact(gu, wgu, "grad_up")
+
+
+@pytest.mark.parametrize("dtype", EXACT)
+@pytest.mark.parametrize("n", [9, 15, 8 * 256 + 1, 8 * 1024 + 7, (8 << 20) + 8 * 1025 + 5])
+def test_swiglu_elements_past_the_last_whole_vector(dtype, n):
+    gate, up, dy = (2 * torch.randn(n)).to(dtype), torch.randn(n).to(dtype), torch.randn(n).to(dtype)
+    assert_bit_exact(capi.swiglu(dev(gate), dev(up)), O.swiglu(gate, up), f"swiglu n={n}")
+    gg, gu = capi.swiglu_backward(dev(dy), dev(gate), dev(up))
+    wgg, wgu = O.swiglu_backward(dy, gate, up)
+    assert_bit_exact(gg, wgg, f"grad_gate n={n}")
+    assert_bit_exact(gu, wgu, f"grad_up n={n}")
+
+
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])
 def test_swiglu_backward_random_and_ragged(dtype):
     torch.manual_seed(17)
     for n, scale in ((8, 1.0), (1000003, 1.0), (4099, 6.0), (65536, 0.05)):
