@@ -44,6 +44,18 @@ def test_route_matches_oracle(shape, dtype):
         assert_bit_exact(g, w, f"moe_route {name} T{T} E{E} k{k} {dtype}")
 
 
+@pytest.mark.parametrize("T", [2, 8, 9, 64, 127, 128, 129])
+@pytest.mark.parametrize("E,k", [(1, 1), (8, 8), (9, 2), (17, 3), (33, 7), (64, 6), (64, 8)])
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float32])
+def test_route_few_tokens(T, E, k, dtype):
+    """Either side of the number of tokens that one workgroup takes with eight lanes to a token, and of its forms by experts."""
+    logits = torch.randn(T, E, generator=torch.Generator().manual_seed(100 * T + E)).to(dtype)
+    logits[T // 2] = logits[T // 2, 0]
+    got = capi.moe_route(logits.cuda(), k)
+    for name, g, w in zip(NAMES, got, O.moe_route(logits, k)):
+        assert_bit_exact(g, w, f"moe_route {name} T{T} E{E} k{k} {dtype}")
+
+
 def test_route_quantised_logits_many_ties_and_skew():
     logits = torch.randint(-2, 3, (3000, 8)).float().bfloat16()     # 5 distinct values: ties everywhere
     logits[:, 5] += 5                                                 # one hot expert: skewed counts
