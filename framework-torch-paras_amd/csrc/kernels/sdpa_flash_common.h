@@ -28,6 +28,10 @@ struct FlashParams {
     long vs_b, vs_h, vs_l;
     int  B, Hq, Hkv, Lq, Lk;
     int  n_qblocks;
+    int  head_group;   // heads whose query tiles an XCD (or, not dealt to XCDs, the chip) goes through together
+    // (what places a workgroup stands together: it is fetched before anything else can be)
+    int rep;           // Hq / Hkv (sdpa_flash.hip)
+    unsigned magic_group, magic_heads, magic_hq, magic_rep;   // for quotients by head_group n_qblocks (or what else places a workgroup), head_group, Hq, Hq / Hkv
     float scale_log2;  // scale * log2(e)
     float scale;
     // optional mask over [B, Hq, Lq, Lk] (element strides; 0 = broadcast): bytes (nonzero = attend)
@@ -40,8 +44,15 @@ struct FlashParams {
     int    n_parts, part_tiles;
     float* part_o;
     float* part_ml;
-    unsigned magic_nq, magic_hq, magic_rep;   // ceil(2^32 / d) for d = n_qblocks, Hq, Hq / Hkv (set by the wide kernel's launcher)
 };
+
+// x / d for 0 <= x < 2^31: the high half of a product with floor(2^32 / d) is the quotient or one less.  The quotients that place a workgroup
+// are a chain in front of its first load, and the code of six divisions is fetched on the way.
+inline unsigned magic_of(long d) { return d == 1 ? 0xFFFFFFFFu : static_cast<unsigned>((1L << 32) / d); }
+__device__ __forceinline__ int quotient(int x, int d, unsigned magic) {
+    const int q = static_cast<int>(__umulhi(static_cast<unsigned>(x), magic));
+    return q + (x - q * d >= d ? 1 : 0);
+}
 
 template <typename T> struct Mma;
 template <> struct Mma<bf16_t> {

@@ -120,9 +120,9 @@ __global__ __launch_bounds__(256, 1) void flash_wide_kernel(const FlashParams p)
     // normalised and stored.
     //   Workgroup w runs on XCD w % 8 (round-robin dispatch), so with a head count that divides
     // by 8 the heads are dealt to the XCDs and the workgroups of an XCD share the K / V of few
-    // heads at a time in its L2.  Within such a pool the items are numbered head by head, longest
-    // query tile first under the causal rule, and dealt in rounds of one item per workgroup, every
-    // other round in reverse order, which evens out the triangle (tile i then tile n-1-i).
+    // heads at a time in its L2.  Within such a pool the items are numbered by groups of heads, longest
+    // query tiles first under the causal rule, and dealt in rounds of one item per workgroup, every
+    // other round in reverse order, which evens out the triangle (tile i then tile n-1-i; head_group_of chooses the groups).
     const int nq = p.n_qblocks;
     const int BH = p.B * p.Hq;
     const int n_wg = static_cast<int>(gridDim.x), wg_id = static_cast<int>(blockIdx.x);
@@ -135,7 +135,8 @@ __global__ __launch_bounds__(256, 1) void flash_wide_kernel(const FlashParams p)
     auto item_at = [&](int round, int& bh, int& qblock) {
         const int i = round * pool_wgs + ((round & 1) ? pool_wgs - 1 - pool_pos : pool_pos);
         if (i >= pool_items) return false;
-        const int head = nq == 1 ? i : fast_div(i, p.magic_nq), pos = i - head * nq;
+        const int span = p.head_group * nq, group = span == 1 ? i : fast_div(i, p.magic_group), in = i - group * span;
+        const int pos = p.head_group == 1 ? in : fast_div(in, p.magic_heads), head = group * p.head_group + in - pos * p.head_group;
         bh = by_xcd ? head * 8 + (wg_id & 7) : head;
         qblock = kCausal ? nq - 1 - pos : pos;
         return true;
@@ -560,6 +561,43 @@ __global__ __launch_bounds__(256, 1) void flash_wide_kernel(const FlashParams p)
     }
 }
 
+// Heads whose query tiles are dealt out together, longest first, under the causal rule: the smallest group (its keys and values share the L2)
+// with which no workgroup has over 3 % more than its share of tiles, or else the one that comes nearest.  One head at a time is even where the
+// query tiles of whole heads fill the rounds; elsewhere a workgroup may come to long tiles every time (5 sequences of 6175, 8 heads: 25
+// query tiles for 32 workgroups, one of which had 1.4 times its share; 444 -> 369 us; 2 of 7777, 16 heads 681 -> 436; 7 of 5000, 4 heads 280 -> 183).
+int head_group_of(long BH, long nq, long blocks) {
+    const bool by_xcd = BH % 8 == 0 && blocks % 8 == 0;
+    const long heads = by_xcd ? BH / 8 : BH, wgs = by_xcd ? blocks / 8 : blocks, items = heads * nq;
+    constexpr long kWgs = 512;
+    if (wgs > kWgs || items > 4096) return 1;         // (many rounds are even enough)
+    const double share = static_cast<double>(heads) * (nq * (nq + 1) / 2) / wgs;
+    long best = 1, least = 0x7fffffffffffL;
+    for (long G = 1; G <= heads; ++G) {
+        if (heads % G != 0) continue;
+        long load[kWgs] = {};
+        long most = 0, w = 0, way = 1;
+        for (long i = 0, pos = 0, at = 0; i < items; ++i) {           // item i: nq - pos tiles' worth, of the group's head `at`
+            load[w] += nq - pos;
+            if (load[w] > most) most = load[w];
+            w += way;
+            if (w < 0 || w == wgs) {                                  // the next round, the other way
+                way = -way;
+                w += way;
+            }
+            if (++at == G) {
+                at = 0;
+                if (++pos == nq) pos = 0;
+            }
+        }
+        if (most < least) {
+            least = most;
+            best = G;
+        }
+        if (most <= 1.03 * share) break;
+    }
+    return static_cast<int>(best);
+}
+
 template <typename T>
 int launch_t(FlashParams p, bool causal, hipStream_t s) {
     p.n_qblocks = (p.Lq + kWideBM - 1) / kWideBM;
@@ -569,11 +607,13 @@ int launch_t(FlashParams p, bool causal, hipStream_t s) {
     PARAS_HIP_TRY(hipGetDevice(&dev));
     PARAS_HIP_TRY(hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, dev));
     auto magic = [](long d) { return static_cast<unsigned>(((1ull << 32) + static_cast<unsigned long long>(d) - 1) / static_cast<unsigned long long>(d)); };
-    p.magic_nq = magic(p.n_qblocks);
     p.magic_hq = magic(p.Hq);
     p.magic_rep = magic(p.Hq / p.Hkv);
     long blocks = items < cus ? items : cus;
     if (blocks >= 8 && (static_cast<long>(p.B) * p.Hq) % 8 == 0) blocks -= blocks % 8;
+    p.head_group = causal ? head_group_of(static_cast<long>(p.B) * p.Hq, p.n_qblocks, blocks) : 1;
+    p.magic_group = magic(static_cast<long>(p.head_group) * p.n_qblocks);
+    p.magic_heads = magic(p.head_group);
     const dim3 grid(static_cast<unsigned>(blocks)), wg(256);
     if (causal) hipLaunchKernelGGL((flash_wide_kernel<T, true>), grid, wg, 0, s, p);
     else        hipLaunchKernelGGL((flash_wide_kernel<T, false>), grid, wg, 0, s, p);

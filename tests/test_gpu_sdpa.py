@@ -941,6 +941,36 @@ def test_composed_route_gqa_masks_and_pieces(cap, monkeypatch):
     assert rel_err(out, want) <= REL_F32
 
 
+@pytest.mark.parametrize("B,H,Hkv,S,D", [(1, 8, 8, 300, 64), (3, 8, 2, 200, 64), (2, 8, 8, 640, 64), (7, 8, 8, 130, 64), (7, 8, 4, 300, 128), (3, 16, 16, 200, 256),
+                                         (5, 3, 3, 300, 64), (25, 8, 8, 129, 64)])
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])
+def test_flash_causal_groups_of_heads(B, H, Hkv, S, D, dtype):
+    """Every query tile of every head is computed once, whatever number of heads an XCD goes through together (1, 2, 3, 5, 6, 7 or
+    25 to an XCD here, and heads that are not dealt to XCDs), with one query tile per head and several."""
+    torch.manual_seed(B * S)
+    q, k, v = torch.randn(B, H, S, D).to(dtype), torch.randn(B, Hkv, S, D).to(dtype), torch.randn(B, Hkv, S, D).to(dtype)
+    out, _, _, name = run(q, k, v, is_causal=True)
+    assert name.startswith("flash_mfma")
+    kf, vf = (t.float().repeat_interleave(H // Hkv, 1) for t in (k, v))
+    want = torch.nn.functional.scaled_dot_product_attention(q.float(), kf, vf, is_causal=True)
+    assert max_abs(out, want) <= ABS_16BIT
+
+
+@pytest.mark.parametrize("B,H,S", [(5, 8, 6175), (3, 16, 5000), (7, 5, 4200), (2, 32, 4096)])
+def test_flash_wide_kernel_deals_every_query_tile(B, H, S):
+    """Long causal prompts whose query tiles are dealt out by groups of heads: the same as sequence by sequence, which is the kernel
+    of 32 queries per wavefront (both round 16-bit weights and results: the bar of either against the oracle)."""
+    g = torch.Generator(device="cuda").manual_seed(S)
+    q, k, v = (torch.randn(B, H, S, 128, generator=g, device="cuda", dtype=torch.bfloat16) for _ in range(3))
+    out, _, _, name = capi.sdpa(q, k, v, is_causal=True)
+    assert name == "flash_mfma_wide"
+    for b in range(B):
+        for h in range(0, H, 4):
+            want, _, _, other = capi.sdpa(q[b:b + 1, h:h + 4].contiguous(), k[b:b + 1, h:h + 4].contiguous(), v[b:b + 1, h:h + 4].contiguous(), is_causal=True)
+            assert other != name
+            assert (out[b:b + 1, h:h + 4].float() - want.float()).abs().max().item() <= ABS_16BIT
+
+
 def test_composed_route_fp64_and_wide_16_bit_heads():
     torch.manual_seed(5)
     q, k, v = _composed_case(torch.float64, 1, 4, 4, 2048, 2048, 32)
