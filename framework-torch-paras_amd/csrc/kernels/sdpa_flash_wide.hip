@@ -565,13 +565,18 @@ __global__ __launch_bounds__(256, 1) void flash_wide_kernel(const FlashParams p)
 // with which no workgroup has over 3 % more than its share of tiles, or else the one that comes nearest.  One head at a time is even where the
 // query tiles of whole heads fill the rounds; elsewhere a workgroup may come to long tiles every time (5 sequences of 6175, 8 heads: 25
 // query tiles for 32 workgroups, one of which had 1.4 times its share; 444 -> 369 us; 2 of 7777, 16 heads 681 -> 436; 7 of 5000, 4 heads 280 -> 183).
-int head_group_of(long BH, long nq, long blocks) {
+struct Deal {
+    int    group = 1;
+    double even = 1.0;               // a workgroup's share of the work, of what the one with the most has
+};
+Deal deal_of(long BH, long nq, long blocks) {
+    Deal d;
     const bool by_xcd = BH % 8 == 0 && blocks % 8 == 0;
     const long heads = by_xcd ? BH / 8 : BH, wgs = by_xcd ? blocks / 8 : blocks, items = heads * nq;
     constexpr long kWgs = 512;
-    if (wgs > kWgs || items > 4096) return 1;         // (many rounds are even enough)
+    if (wgs > kWgs || items > 1024) return d;         // (many rounds are even enough)
     const double share = static_cast<double>(heads) * (nq * (nq + 1) / 2) / wgs;
-    long best = 1, least = 0x7fffffffffffL;
+    long least = 0x7fffffffffffL;
     for (long G = 1; G <= heads; ++G) {
         if (heads % G != 0) continue;
         long load[kWgs] = {};
@@ -591,11 +596,18 @@ int head_group_of(long BH, long nq, long blocks) {
         }
         if (most < least) {
             least = most;
-            best = G;
+            d.group = static_cast<int>(G);
         }
         if (most <= 1.03 * share) break;
     }
-    return static_cast<int>(best);
+    d.even = share / least;
+    return d;
+}
+
+// One workgroup per CU, or fewer, and a whole number per XCD where the heads are dealt to them
+long workgroups_for(long BH, long items, long cus) {
+    const long blocks = items < cus ? items : cus;
+    return blocks >= 8 && BH % 8 == 0 ? blocks - blocks % 8 : blocks;
 }
 
 template <typename T>
@@ -609,9 +621,8 @@ int launch_t(FlashParams p, bool causal, hipStream_t s) {
     auto magic = [](long d) { return static_cast<unsigned>(((1ull << 32) + static_cast<unsigned long long>(d) - 1) / static_cast<unsigned long long>(d)); };
     p.magic_hq = magic(p.Hq);
     p.magic_rep = magic(p.Hq / p.Hkv);
-    long blocks = items < cus ? items : cus;
-    if (blocks >= 8 && (static_cast<long>(p.B) * p.Hq) % 8 == 0) blocks -= blocks % 8;
-    p.head_group = causal ? head_group_of(static_cast<long>(p.B) * p.Hq, p.n_qblocks, blocks) : 1;
+    const long BH = static_cast<long>(p.B) * p.Hq, blocks = workgroups_for(BH, items, cus);
+    p.head_group = causal ? deal_of(BH, p.n_qblocks, blocks).group : 1;
     p.magic_group = magic(static_cast<long>(p.head_group) * p.n_qblocks);
     p.magic_heads = magic(p.head_group);
     const dim3 grid(static_cast<unsigned>(blocks)), wg(256);
@@ -631,14 +642,24 @@ bool wide_supported(long B, long Hq, long Lq, long Lk, int head, int mask_kind, 
     const unsigned long long bh = static_cast<unsigned long long>(B) * static_cast<unsigned long long>(Hq);
     if (bh * nq * nq >= (1ull << 32) || bh * static_cast<unsigned long long>(Hq) >= (1ull << 32)) return false;
     if (forced >= 0) return forced != 0;
-    // One workgroup per CU and 256 queries per item: it needs a few items per CU to keep them all
-    // busy and, under the causal rule, long rows for the items' fixed cost to pay off (measured
-    // against the 32-queries-per-wavefront kernel: ahead from 4096 causal / 1024 unmasked queries on).
-    const long least = causal ? 4096 : 1024;
+    // Against the kernel of 32 queries per wavefront (W query tiles of 128, two to a CU), measured for 110 problems of 900 to 8000 queries:
+    //   Unmasked: both come in rounds, this one of a CU's 256 queries, that one of 128 for the first of a CU and again for the second, and a
+    // round here takes 1.82 of those.  So wherever the last of that kernel's is a second one, and from two items to a CU on (2 to 5 % behind at worst)
+    // (the other / this: B1 H8 S5524 135 / 119 us, W 352; B2 H8 S6249 341 / 300, W 784; B2 H8 S3992 127 / 120, W 512; B2 H8 S5432 237 / 260,
+    // W 688; B1 H16 S1661 30 / 40, W 208; B6 H16 S4585 897 / 825).
+    //   Causal: 5 % ahead where its workgroups come out even and its query tiles of 256 pad no more than those of 128 (B4 H16 S4563 352 / 333;
+    // B13 H8 S2011 138 / 131; B5 H16 S1487 62 / 60; a ninth more of padded triangle: B9 H32 S2372 460 / 524; uneven, 0.78: B2 H8 S6079 153 / 156).
+    // Of the 110, the slower one is taken 6 times, by 0.5 to 6 % (with the limits of before, 4096 causal or 1024 unmasked queries and two query tiles of
+    // 256 per CU, 2.3 % in the mean over all, up to 15 %).
+    const long least = causal ? 1400 : 896;
     if (Lq < least || Lk < least) return false;        // (before the runtime is asked: small calls are bound by the host)
     int dev = 0, cus = 0;
     if (hipGetDevice(&dev) != hipSuccess || hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, dev) != hipSuccess) return false;
-    return bh * nq >= 2ull * static_cast<unsigned long long>(cus);
+    const long BH = static_cast<long>(bh), items = BH * static_cast<long>(nq), tiles = (Lq + 127) / 128;
+    if (!causal) return (items >= 2 * cus && Lq >= 1024) || 1.82 * static_cast<double>((items + cus - 1) / cus) < static_cast<double>((BH * tiles + cus - 1) / cus);
+    const double rows = static_cast<double>(nq * kWideBM) / static_cast<double>(tiles * 128), padded = 0.94 * rows * rows;
+    if (items < cus || padded >= 1.0) return false;
+    return padded < deal_of(BH, static_cast<long>(nq), workgroups_for(BH, items, cus)).even + 0.1;
 }
 
 int launch_flash_wide(FlashParams p, bool causal, bool is_bf16, hipStream_t s) {

@@ -971,6 +971,19 @@ def test_flash_wide_kernel_deals_every_query_tile(B, H, S):
             assert (out[b:b + 1, h:h + 4].float() - want.float()).abs().max().item() <= ABS_16BIT
 
 
+@pytest.mark.parametrize("B,H,S,causal,wide", [(1, 8, 4200, False, True), (1, 8, 4096, False, False), (6, 16, 1024, False, False), (7, 16, 1024, False, True), (2, 32, 896, False, True),
+                                               (2, 32, 895, False, False), (5, 16, 1500, True, True), (5, 16, 1408, True, False), (5, 16, 1399, True, False), (2, 8, 6079, True, False)])
+def test_flash_either_side_of_the_limits_of_the_wide_kernel(B, H, S, causal, wide):
+    """By rounds of query tiles over the CUs, and under the causal rule by padding and by how evenly the tiles are dealt out (256 CUs)."""
+    torch.manual_seed(S)
+    q, k, v = (torch.randn(B, H, S, 128, device="cuda", dtype=torch.bfloat16) for _ in range(3))
+    out, _, _, name = capi.sdpa(q, k, v, is_causal=causal)
+    assert (name == "flash_mfma_wide") == wide, name
+    for b, h in ((0, 0), (B - 1, H - 1), (B // 2, H // 2)):
+        want = torch.nn.functional.scaled_dot_product_attention(*(t[b:b + 1, h:h + 1].float().cpu() for t in (q, k, v)), is_causal=causal)
+        assert max_abs(out[b:b + 1, h:h + 1], want) <= ABS_16BIT
+
+
 def test_composed_route_fp64_and_wide_16_bit_heads():
     torch.manual_seed(5)
     q, k, v = _composed_case(torch.float64, 1, 4, 4, 2048, 2048, 32)
