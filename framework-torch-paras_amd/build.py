@@ -41,6 +41,7 @@ HIP_FLAGS = [
     "-O3", f"--offload-arch={ARCH}", "-fPIC", "-std=c++17", "-fvisibility=hidden",
     # Packed-fp32 VALU forms are kept out of every kernel of this library.
     "-Xclang", "-target-feature", "-Xclang", "-packed-fp32-ops",
+    "-mllvm", "-amdgpu-kernarg-preload-count=16",
     "-Wno-unused-command-line-argument", "-Wno-option-ignored",
     f"-I{INCLUDE}", f"-I{CSRC}",
 ]
