@@ -41,6 +41,8 @@ HIP_FLAGS = [
     "-O3", f"--offload-arch={ARCH}", "-fPIC", "-std=c++17", "-fvisibility=hidden",
     # Packed-fp32 VALU forms are kept out of every kernel of this library.
     "-Xclang", "-target-feature", "-Xclang", "-packed-fp32-ops",
+    # Arguments that are not structures are in scalar registers when a wave starts (up to 16 words with what else stands there) instead of
+    # being fetched in front of the first load: 0.2 to 0.35 us of each small kernel.
     "-mllvm", "-amdgpu-kernarg-preload-count=16",
     "-Wno-unused-command-line-argument", "-Wno-option-ignored",
     f"-I{INCLUDE}", f"-I{CSRC}",

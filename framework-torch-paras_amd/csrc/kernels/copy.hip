@@ -8,6 +8,7 @@
 #include <hip/hip_runtime.h>
 
 #include <cmath>
+#include <type_traits>
 
 #include "core/device_context.h"
 #include "core/device_math.h"
@@ -50,6 +51,34 @@ __device__ __forceinline__ void offsets(const Strided& s, long flat, bool small,
     }
     *so = a;
     *d_o = b;
+}
+
+// Up to four dimensions and 2^32 elements, in 112 bytes: a launch whose arguments take more costs the host 0.7 us more, 3.4 for 2.7 (a decode step's
+// new keys and values written into the cache).  Strides in elements of W.
+struct FewDims {
+    const void* src;
+    void* dst;
+    unsigned n;
+    int ndim;
+    unsigned sizes[4];
+    long src_strides[4], dst_strides[4];
+};
+static_assert(sizeof(FewDims) <= 112, "see above");
+bool few_dims(const Strided& s, long n) { return s.ndim <= 4 && n <= 0xFFFFFFFFL; }
+
+template <typename W>
+__global__ __launch_bounds__(kBlock) void copy_few_dims_kernel(const FewDims s) {
+    for (unsigned long i = static_cast<unsigned long>(blockIdx.x) * kBlock + threadIdx.x; i < s.n; i += static_cast<unsigned long>(gridDim.x) * kBlock) {
+        unsigned left = static_cast<unsigned>(i);
+        long a = 0, b = 0;
+        for (int d = s.ndim - 1; d >= 0; --d) {
+            const unsigned q = left / s.sizes[d], c = left - q * s.sizes[d];
+            left = q;
+            a += c * s.src_strides[d];
+            b += c * s.dst_strides[d];
+        }
+        static_cast<W*>(s.dst)[b] = static_cast<const W*>(s.src)[a];
+    }
 }
 
 template <typename W>
@@ -330,32 +359,41 @@ __global__ __launch_bounds__(kBlock) void binary_vec16_kernel(int op, const std:
 }
 
 // 16-bit tensors whose rows are contiguous in both operands, in whole 16-byte pieces, whatever the other dims do (a
-// projection's heads seen as [B, h, S, D], times cos / sin repeated over them): eight elements per thread.  `s` as above with
-// the last dim counted in pieces.  An element at a time spends its time on 64-bit index divisions and 2-byte accesses:
+// projection's heads seen as [B, h, S, D], times cos / sin repeated over them): eight elements per thread.  An element at a time spends its time on 64-bit index divisions and 2-byte accesses:
 // [1, 32, 1500, 128] and [1, 8, 1500, 128] (transposed views) times [1500, 128], bf16, 32 us together; this way 15.
-template <typename T>
-__global__ __launch_bounds__(kBlock) void binary_rows_vec16_kernel(int op, const std::uint16_t* __restrict__ a,
-                                                                   const std::uint16_t* __restrict__ b, std::uint16_t* __restrict__ out,
-                                                                   unsigned nvec, const Strided s, double alpha) {
+template <int ND> struct BinaryRows {       // (four dimensions: 112 bytes, as FewDims; the last one is the pieces of a row)
+    const std::uint16_t* a;
+    const std::uint16_t* b;
+    std::uint16_t* out;
+    unsigned nvec;
+    int op, ndim;
+    unsigned sizes[ND];
+    long a_strides[ND - 1], b_strides[ND - 1];
+    double alpha;
+};
+static_assert(sizeof(BinaryRows<4>) <= 112, "see above");
+template <typename T, int ND>
+__global__ __launch_bounds__(kBlock) void binary_rows_vec16_kernel(const BinaryRows<ND> s) {
     const unsigned i = blockIdx.x * kBlock + threadIdx.x;
-    if (i >= nvec) return;
-    const bool unit = alpha == 1.0;
-    unsigned left = i;
-    long ao = 0, bo = 0;
-    for (int d = s.ndim - 1; d >= 0; --d) {
-        const unsigned size = static_cast<unsigned>(s.sizes[d]), q = left / size, c = left - q * size;
+    if (i >= s.nvec) return;
+    const bool unit = s.alpha == 1.0;
+    unsigned left = i / s.sizes[s.ndim - 1];
+    const unsigned col = i - left * s.sizes[s.ndim - 1];
+    long ao = col * 8L, bo = ao;
+    for (int d = s.ndim - 2; d >= 0; --d) {
+        const unsigned q = left / s.sizes[d], c = left - q * s.sizes[d];
         left = q;
-        ao += c * s.src_strides[d];
-        bo += c * s.dst_strides[d];
+        ao += c * s.a_strides[d];
+        bo += c * s.b_strides[d];
     }
-    const u32x4 av = load16(a + ao), bv = load16(b + bo);
+    const u32x4 av = load16(s.a + ao), bv = load16(s.b + bo);
     const std::uint16_t* ae = reinterpret_cast<const std::uint16_t*>(&av);
     const std::uint16_t* be = reinterpret_cast<const std::uint16_t*>(&bv);
     u32x4 o;
     std::uint16_t* oe = reinterpret_cast<std::uint16_t*>(&o);
 #pragma unroll
-    for (int j = 0; j < 8; ++j) oe[j] = binary_one<T>(op, ae[j], be[j], alpha, unit);
-    store16(out + static_cast<long>(i) * 8, o);
+    for (int j = 0; j < 8; ++j) oe[j] = binary_one<T>(s.op, ae[j], be[j], s.alpha, unit);
+    store16(s.out + static_cast<long>(i) * 8, o);
 }
 
 // ---- index_select along one dim of a dense tensor seen as [outer, n_src, inner]:
@@ -378,6 +416,22 @@ unsigned grid_for(long n) {
     long g = (n + kBlock - 1) / kBlock;
     if (g > 65536) g = 65536;
     return static_cast<unsigned>(g < 1 ? 1 : g);
+}
+
+template <typename W>
+void copy_same(const void* src, void* dst, long n, const Strided& s, hipStream_t st) {
+    const dim3 g(grid_for(n)), b(kBlock);
+    if (few_dims(s, n)) {
+        FewDims f{src, dst, static_cast<unsigned>(n), s.ndim, {}, {}, {}};
+        for (int d = 0; d < s.ndim; ++d) {
+            f.sizes[d] = static_cast<unsigned>(s.sizes[d]);
+            f.src_strides[d] = s.src_strides[d];
+            f.dst_strides[d] = s.dst_strides[d];
+        }
+        hipLaunchKernelGGL((copy_few_dims_kernel<W>), g, b, 0, st, f);
+        return;
+    }
+    hipLaunchKernelGGL((copy_same_kernel<W>), g, b, 0, st, static_cast<const W*>(src), static_cast<W*>(dst), n, s);
 }
 
 // Launches the register-resident kernel if the row shape allows it; false = use the general one.
@@ -559,18 +613,16 @@ int paras_copy_strided(const void* src, void* dst, int ndim, const int64_t* size
                 w.sizes[s.ndim - 1] /= per;
                 for (int d = 0; d + 1 < s.ndim; ++d) { w.src_strides[d] /= per; w.dst_strides[d] /= per; }
                 const long nw = n / per;
-                hipLaunchKernelGGL((copy_same_kernel<u32x4>), dim3(grid_for(nw)), b, 0, st, static_cast<const u32x4*>(src),
-                                   static_cast<u32x4*>(dst), nw, w);
+                copy_same<u32x4>(src, dst, nw, w, st);
                 PARAS_HIP_TRY(hipGetLastError());
                 return PARAS_OK;
             }
         }
-        const dim3 g(grid_for(n));
         switch (elem_size) {
-            case 1: hipLaunchKernelGGL((copy_same_kernel<uint8_t>), g, b, 0, st, static_cast<const uint8_t*>(src), static_cast<uint8_t*>(dst), n, s); break;
-            case 2: hipLaunchKernelGGL((copy_same_kernel<uint16_t>), g, b, 0, st, static_cast<const uint16_t*>(src), static_cast<uint16_t*>(dst), n, s); break;
-            case 4: hipLaunchKernelGGL((copy_same_kernel<uint32_t>), g, b, 0, st, static_cast<const uint32_t*>(src), static_cast<uint32_t*>(dst), n, s); break;
-            case 8: hipLaunchKernelGGL((copy_same_kernel<uint64_t>), g, b, 0, st, static_cast<const uint64_t*>(src), static_cast<uint64_t*>(dst), n, s); break;
+            case 1: copy_same<uint8_t>(src, dst, n, s, st); break;
+            case 2: copy_same<uint16_t>(src, dst, n, s, st); break;
+            case 4: copy_same<uint32_t>(src, dst, n, s, st); break;
+            case 8: copy_same<uint64_t>(src, dst, n, s, st); break;
             default: return fail(PARAS_ERR_UNSUPPORTED, "paras_copy_strided: element size %d", elem_size);
         }
         PARAS_HIP_TRY(hipGetLastError());
@@ -674,15 +726,21 @@ int paras_binary_strided(int op, const void* a, const void* b, void* out, int nd
         bool rows = aligned && last >= 1 && n / 8 < (1L << 31) && s.src_strides[last] == 1 && s.dst_strides[last] == 1 && s.sizes[last] % 8 == 0;
         for (int d = 0; rows && d < last; ++d) rows = s.src_strides[d] % 8 == 0 && s.dst_strides[d] % 8 == 0;
         if (rows) {
-            Strided v = s;
-            v.sizes[last] /= 8;
-            v.src_strides[last] = v.dst_strides[last] = 8;
             const unsigned nvec = static_cast<unsigned>(n / 8);
-            const dim3 gv((nvec + kBlock - 1) / kBlock);
-            if (dtype == PARAS_BF16)
-                hipLaunchKernelGGL((binary_rows_vec16_kernel<bf16_t>), gv, blk, 0, st, op, static_cast<const uint16_t*>(a), static_cast<const uint16_t*>(b), static_cast<uint16_t*>(out), nvec, v, alpha);
-            else
-                hipLaunchKernelGGL((binary_rows_vec16_kernel<f16_t>), gv, blk, 0, st, op, static_cast<const uint16_t*>(a), static_cast<const uint16_t*>(b), static_cast<uint16_t*>(out), nvec, v, alpha);
+            auto launch = [&](auto dims) {
+                constexpr int ND = decltype(dims)::value;
+                BinaryRows<ND> v{static_cast<const uint16_t*>(a), static_cast<const uint16_t*>(b), static_cast<uint16_t*>(out), nvec, op, s.ndim, {}, {}, {}, alpha};
+                for (int d = 0; d < s.ndim; ++d) v.sizes[d] = static_cast<unsigned>(d < last ? s.sizes[d] : s.sizes[d] / 8);
+                for (int d = 0; d < last; ++d) {
+                    v.a_strides[d] = s.src_strides[d];
+                    v.b_strides[d] = s.dst_strides[d];
+                }
+                const dim3 gv((nvec + kBlock - 1) / kBlock);
+                if (dtype == PARAS_BF16) hipLaunchKernelGGL((binary_rows_vec16_kernel<bf16_t, ND>), gv, blk, 0, st, v);
+                else                     hipLaunchKernelGGL((binary_rows_vec16_kernel<f16_t, ND>), gv, blk, 0, st, v);
+            };
+            if (s.ndim <= 4) launch(std::integral_constant<int, 4>{});
+            else             launch(std::integral_constant<int, kMaxDims>{});
             PARAS_HIP_TRY(hipGetLastError());
             return PARAS_OK;
         }

@@ -38,7 +38,6 @@ struct DenseParams {
     long sa, sb, sc, sadd;      // batch strides (elements)
     float alpha, beta;
     double alpha64, beta64;     // the same, for fp64 tensors
-    long rows_each;             // streaming few-row kernel only: weight rows per workgroup
     int  swapped;               // few-row kernels only: a and b have changed places (few output COLUMNS, many rows), so a
                                 // result (row of a, row of b) belongs at c[row of b][row of a], and the addend likewise
 };
@@ -47,8 +46,22 @@ struct DenseParams {
 // weight rows and its eight waves split the contraction (stream_rows.h); 8 XQ activation rows at most.
 using stream::Mma16;
 
-template <typename T>
-__device__ __forceinline__ void few_rows_store(const DenseParams& p, std::uint16_t* C, const std::uint16_t* ADD, bool vec_ok, long row, long col, long cols, float4_t t) {
+// What the streaming kernel needs of DenseParams, in 112 bytes: a launch whose arguments take more costs the host 0.7 us more, 3.4 for 2.7.
+struct FewParams {
+    const std::uint16_t* a;
+    const std::uint16_t* b;
+    const std::uint16_t* add;
+    std::uint16_t* c;
+    long sa, sb, sc, sadd;
+    int  M, N, K;
+    int  lda, ldb, ldc, ld_add;
+    float alpha, beta;
+    int  rows_each, swapped;
+};
+static_assert(sizeof(FewParams) <= 112, "see above");
+
+template <typename T, typename P>
+__device__ __forceinline__ void few_rows_store(const P& p, std::uint16_t* C, const std::uint16_t* ADD, bool vec_ok, long row, long col, long cols, float4_t t) {
     using El = Elem<T>;
     if (row >= p.M) return;
     if (p.swapped) {        // `row` is a column of the caller's result and `col + r` a row of it
@@ -79,19 +92,20 @@ __device__ __forceinline__ void few_rows_store(const DenseParams& p, std::uint16
             if (col + r < cols) C[row * p.ldc + col + r] = o16[r];
     }
 }
-__device__ __forceinline__ bool few_rows_vec(const DenseParams& p) {
+template <typename P>
+__device__ __forceinline__ bool few_rows_vec(const P& p) {
     return (p.ldc % 4 == 0) && (p.sc % 4 == 0) && ((reinterpret_cast<uintptr_t>(p.c) & 7) == 0);
 }
 
 template <typename T, int NBG, int XQ>
-__global__ __launch_bounds__(stream::kThreads, 4) void stream_gemm_nt_kernel(const DenseParams p) {
+__global__ __launch_bounds__(stream::kThreads, 4) void stream_gemm_nt_kernel(const FewParams p) {
     using S = stream::Shape<1, NBG, XQ>;
     constexpr int MB = S::kXBlocks;
     __shared__ __attribute__((aligned(1024))) std::uint16_t lds[S::kLdsElems];
     const long bidx = blockIdx.y;
     const std::uint16_t* A = p.a + bidx * p.sa;
     const int lane = threadIdx.x & 63;
-    const long n0 = blockIdx.x * p.rows_each, rows = p.N - n0 < p.rows_each ? p.N - n0 : p.rows_each;
+    const long n0 = static_cast<long>(blockIdx.x) * p.rows_each, rows = p.N - n0 < p.rows_each ? p.N - n0 : p.rows_each;
     const std::uint16_t* const w[1] = {p.b + bidx * p.sb + n0 * p.ldb};
     std::uint32_t x_off[XQ];
 #pragma unroll
@@ -102,7 +116,7 @@ __global__ __launch_bounds__(stream::kThreads, 4) void stream_gemm_nt_kernel(con
     }
     constexpr int step = 16 * NBG;
     const int count = static_cast<int>((rows + step - 1) / step);
-    stream::products<T, 1, NBG, XQ, true>(w, p.ldb, rows, step, count, p.K, A, ((p.M - 1) * p.lda + p.K) * 2, x_off, lds,
+    stream::products<T, 1, NBG, XQ, true>(w, p.ldb, rows, step, count, p.K, A, (static_cast<long>(p.M - 1) * p.lda + p.K) * 2, x_off, lds,
                                     [&](int j, const float4_t (&acc)[NBG][MB]) __attribute__((always_inline)) {
         stream::share<NBG, MB>(lds, acc);
         const int blk = stream::wave_id();                  // wave w finishes result block w
@@ -237,21 +251,25 @@ __global__ __launch_bounds__(kSkinnyWaves * 64) void skinny_gemm_nt_kernel(const
 // More rows than 32: two blocks of weight rows per workgroup when that still leaves a workgroup for every CU: every
 // activation fragment then feeds two MFMAs, which halves the reads of the activations from L2.
 template <typename T>
-void launch_skinny(DenseParams p, long batch, hipStream_t s) {
+void launch_skinny(const DenseParams& p, long batch, hipStream_t s) {
     const dim3 block(kSkinnyWaves * 64);
     const int mb = static_cast<int>((p.M + 15) / 16);
-    if (mb <= 2) {
+    auto fits = [](long v) { return v <= 0x7fffffffL; };
+    if (mb <= 2 && fits(p.N) && fits(p.K) && fits(p.lda) && fits(p.ldb) && fits(p.ldc) && (p.add == nullptr || fits(p.ld_add))) {
         constexpr long kCus = 256;
         auto share = [&](long workgroups) { return ((p.N * batch + workgroups - 1) / workgroups + 3) / 4 * 4; };
         const bool two = share(kCus) > 16;
-        p.rows_each = share(kCus) > 32 ? share(2 * kCus) : (share(kCus) > 8 ? share(kCus) : 8);
-        const dim3 g(static_cast<unsigned>((p.N + p.rows_each - 1) / p.rows_each), static_cast<unsigned>(batch));
-        if (p.M <= 8)     { if (two) hipLaunchKernelGGL((stream_gemm_nt_kernel<T, 2, 1>), g, block, 0, s, p);
-                            else     hipLaunchKernelGGL((stream_gemm_nt_kernel<T, 1, 1>), g, block, 0, s, p); }
-        else if (mb <= 1) { if (two) hipLaunchKernelGGL((stream_gemm_nt_kernel<T, 2, 2>), g, block, 0, s, p);
-                            else     hipLaunchKernelGGL((stream_gemm_nt_kernel<T, 1, 2>), g, block, 0, s, p); }
-        else              { if (two) hipLaunchKernelGGL((stream_gemm_nt_kernel<T, 2, 4>), g, block, 0, s, p);
-                            else     hipLaunchKernelGGL((stream_gemm_nt_kernel<T, 1, 4>), g, block, 0, s, p); }
+        const long even = share(kCus) > 32 ? share(2 * kCus) : (share(kCus) > 8 ? share(kCus) : 8), rows_each = even < p.N ? even : p.N;
+        const dim3 g(static_cast<unsigned>((p.N + rows_each - 1) / rows_each), static_cast<unsigned>(batch));
+        auto narrow = [](long v) { return static_cast<int>(v); };
+        const FewParams f{p.a, p.b, p.add, p.c, p.sa, p.sb, p.sc, p.sadd, narrow(p.M), narrow(p.N), narrow(p.K), narrow(p.lda), narrow(p.ldb), narrow(p.ldc),
+                          p.add != nullptr ? narrow(p.ld_add) : 0, p.alpha, p.beta, narrow(rows_each), p.swapped};
+        if (p.M <= 8)     { if (two) hipLaunchKernelGGL((stream_gemm_nt_kernel<T, 2, 1>), g, block, 0, s, f);
+                            else     hipLaunchKernelGGL((stream_gemm_nt_kernel<T, 1, 1>), g, block, 0, s, f); }
+        else if (mb <= 1) { if (two) hipLaunchKernelGGL((stream_gemm_nt_kernel<T, 2, 2>), g, block, 0, s, f);
+                            else     hipLaunchKernelGGL((stream_gemm_nt_kernel<T, 1, 2>), g, block, 0, s, f); }
+        else              { if (two) hipLaunchKernelGGL((stream_gemm_nt_kernel<T, 2, 4>), g, block, 0, s, f);
+                            else     hipLaunchKernelGGL((stream_gemm_nt_kernel<T, 1, 4>), g, block, 0, s, f); }
         return;
     }
     const dim3 g1(static_cast<unsigned>((p.N + 15) / 16), static_cast<unsigned>(batch));

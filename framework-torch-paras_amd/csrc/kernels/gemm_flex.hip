@@ -16,8 +16,16 @@ namespace flex {
 namespace {
 
 // Adds the parts in order and applies the epilogue; V columns per thread.
+struct FinishParams {
+    const float* partial;
+    const std::uint16_t* add;
+    std::uint16_t* c;
+    long M, N, sc, sadd;
+    int  ldc, ld_add, splits;
+    float alpha, beta;
+};
 template <typename T, int V>
-__global__ __launch_bounds__(256) void gemm_flex_finish_kernel(const Params p) {
+__global__ __launch_bounds__(256) void gemm_flex_finish_kernel(const FinishParams p) {
     using El = Elem<T>;
     typedef float vec __attribute__((ext_vector_type(V)));
     const long mn = p.M * p.N, i = (static_cast<long>(blockIdx.x) * 256 + threadIdx.x) * V;
@@ -78,7 +86,9 @@ bool takes(const Problem& q) {
     if (!aligned(q.a, q.lda, q.sa) || !aligned(q.b, q.ldb, q.sb)) return false;
     // (a chunk of 8 contraction steps is in or out as a whole)
     if (q.K <= 0 || q.K >= (1L << 30) || (!(q.a_rows && q.b_rows) && q.K % 8 != 0)) return false;
-    const long tiles = ((q.M + 31) / 32) * ((q.N + 63) / 64);
+    constexpr long kInt = 0x7fffffffL;
+    if (q.ldc > kInt || (q.add != nullptr && q.ld_add > kInt)) return false;       // (flex::Params)
+    const long tiles = ((q.M + 31) / 32) * ((q.N + 63) / 64);          // (below 2^25: M and N fit as well)
     return q.batch <= 65535 && tiles * q.batch < (1L << 25);
 }
 
@@ -172,19 +182,18 @@ Plan plan(const Problem& q, bool may_split) {
 }
 
 int launch(const Problem& q, const Plan& plan, void* workspace, hipStream_t s) {
+    auto narrow = [](long v) { return static_cast<int>(v); };       // (takes())
     Params p{};
-    p.a = q.a; p.b = q.b; p.add = q.add; p.c = q.c;
-    p.M = q.M; p.N = q.N; p.K = q.K;
-    p.lda = q.lda; p.ldb = q.ldb; p.ldc = q.ldc; p.ld_add = q.ld_add;
+    p.a = q.a; p.b = q.b; p.add = q.add;
+    p.out = plan.splits > 1 ? workspace : q.c;
+    p.M = narrow(q.M); p.N = narrow(q.N); p.K = narrow(q.K);
+    p.lda = narrow(q.lda); p.ldb = narrow(q.ldb); p.ldc = narrow(q.ldc); p.ld_add = q.add != nullptr ? narrow(q.ld_add) : 0;
     p.sa = q.sa; p.sb = q.sb; p.sc = q.sc; p.sadd = q.sadd;
     p.alpha = q.alpha; p.beta = q.beta;
     const Tile t = kTiles[plan.tile];
-    p.m_tiles = static_cast<int>((q.M + t.m - 1) / t.m);
-    p.n_tiles = static_cast<int>((q.N + t.n - 1) / t.n);
     p.splits = plan.splits;
-    p.k_per_split = plan.k_per_split;
-    p.partial = static_cast<float*>(workspace);
-    const long wgs = static_cast<long>(p.m_tiles) * p.n_tiles * plan.splits * q.batch;
+    p.k_per_split = narrow(plan.k_per_split);
+    const long wgs = (q.M + t.m - 1) / t.m * ((q.N + t.n - 1) / t.n) * plan.splits * q.batch;
     const unsigned grid = static_cast<unsigned>(wgs);
     if (q.a_rows)      launch_rr(q.bf16, plan.tile, p, grid, s);
     else if (q.b_rows) launch_kr(q.bf16, plan.tile, p, grid, s);
@@ -193,11 +202,12 @@ int launch(const Problem& q, const Plan& plan, void* workspace, hipStream_t s) {
     if (plan.splits > 1) {
         const bool vec = q.N % 4 == 0 && q.ldc % 4 == 0 && q.sc % 4 == 0 && (reinterpret_cast<uintptr_t>(q.c) & 7) == 0;
         const long n = (q.M * q.N + (vec ? 1023 : 255)) / (vec ? 1024 : 256);
+        const FinishParams f{static_cast<const float*>(workspace), q.add, q.c, q.M, q.N, q.sc, q.sadd, p.ldc, p.ld_add, plan.splits, q.alpha, q.beta};
         const dim3 g(static_cast<unsigned>(n), static_cast<unsigned>(q.batch));
-        if (q.bf16) { if (vec) hipLaunchKernelGGL((gemm_flex_finish_kernel<bf16_t, 4>), g, dim3(256), 0, s, p);
-                      else     hipLaunchKernelGGL((gemm_flex_finish_kernel<bf16_t, 1>), g, dim3(256), 0, s, p); }
-        else        { if (vec) hipLaunchKernelGGL((gemm_flex_finish_kernel<f16_t, 4>), g, dim3(256), 0, s, p);
-                      else     hipLaunchKernelGGL((gemm_flex_finish_kernel<f16_t, 1>), g, dim3(256), 0, s, p); }
+        if (q.bf16) { if (vec) hipLaunchKernelGGL((gemm_flex_finish_kernel<bf16_t, 4>), g, dim3(256), 0, s, f);
+                      else     hipLaunchKernelGGL((gemm_flex_finish_kernel<bf16_t, 1>), g, dim3(256), 0, s, f); }
+        else        { if (vec) hipLaunchKernelGGL((gemm_flex_finish_kernel<f16_t, 4>), g, dim3(256), 0, s, f);
+                      else     hipLaunchKernelGGL((gemm_flex_finish_kernel<f16_t, 1>), g, dim3(256), 0, s, f); }
         PARAS_HIP_TRY(hipGetLastError());
     }
     return PARAS_OK;

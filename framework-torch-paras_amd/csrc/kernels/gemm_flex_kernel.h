@@ -7,20 +7,21 @@
 namespace paras {
 namespace flex {
 
+// (112 bytes: a launch whose arguments take more than that costs the host 0.7 us more, 3.4 for 2.7.  Sizes and row strides that do not fit are
+// refused by takes().)
 struct Params {
     const std::uint16_t* a;
     const std::uint16_t* b;
     const std::uint16_t* add;   // may be null
-    std::uint16_t* c;
-    long M, N, K;
-    long lda, ldb, ldc, ld_add;
+    void* out;                  // splits == 1: the result; otherwise fp32 [batch][split][M][N]
     long sa, sb, sc, sadd;      // batch strides (elements)
-    int  m_tiles, n_tiles;
+    int  M, N, K;
+    int  lda, ldb, ldc, ld_add;
     int  splits;                // parts of the contraction, one workgroup each per tile
-    long k_per_split;           // contraction steps per part (a multiple of 64)
-    float* partial;             // splits > 1: [batch][split][M][N]
+    int  k_per_split;           // contraction steps per part (a multiple of 64)
     float alpha, beta;
 };
+static_assert(sizeof(Params) <= 112, "see above");
 
 // Workgroup w runs on XCD w % 8, each with an L2 of its own: every XCD takes a contiguous run of the
 // work list, and the list walks the tiles in bands of kBand row tiles, so that the 32 workgroups an XCD
@@ -31,17 +32,17 @@ constexpr int kXcds = 8, kBand = 4;
 // them -- buffer descriptors, loop bounds -- would be held per lane.)
 struct Work { int batch, split, mt, nt; };
 __device__ __forceinline__ unsigned scalar(unsigned v) { return static_cast<unsigned>(__builtin_amdgcn_readfirstlane(static_cast<int>(v))); }
-__device__ __forceinline__ Work work_of(const Params& p, unsigned wg, unsigned total) {
+__device__ __forceinline__ Work work_of(unsigned m_tiles, unsigned n_tiles, unsigned splits, unsigned wg, unsigned total) {
     const unsigned q = total / kXcds, r = total % kXcds, x = wg % kXcds;
     const unsigned lin = x * q + (x < r ? x : r) + wg / kXcds;
-    const unsigned tiles = static_cast<unsigned>(p.m_tiles) * static_cast<unsigned>(p.n_tiles);
+    const unsigned tiles = m_tiles * n_tiles;
     const unsigned outer = scalar(lin / tiles);
     const unsigned t = lin - outer * tiles;
-    const unsigned per_band = kBand * static_cast<unsigned>(p.n_tiles);
+    const unsigned per_band = kBand * n_tiles;
     const unsigned band = scalar(t / per_band), in = t - band * per_band;
-    const unsigned left = static_cast<unsigned>(p.m_tiles) - band * kBand, rows = left < kBand ? left : kBand;
-    const unsigned nt = scalar(in / rows), batch = scalar(outer / static_cast<unsigned>(p.splits));
-    return {static_cast<int>(batch), static_cast<int>(outer - batch * static_cast<unsigned>(p.splits)),
+    const unsigned left = m_tiles - band * kBand, rows = left < kBand ? left : kBand;
+    const unsigned nt = scalar(in / rows), batch = scalar(outer / splits);
+    return {static_cast<int>(batch), static_cast<int>(outer - batch * splits),
             static_cast<int>(band * kBand + (in - nt * rows)), static_cast<int>(nt)};
 }
 
@@ -58,7 +59,8 @@ __global__ __launch_bounds__(kThreads, (MI * NJ >= 32 || ST * (MI + NJ) > 20 ? 1
     __shared__ __attribute__((aligned(1024))) std::uint16_t b1[OB::kElems];
     __shared__ __attribute__((aligned(1024))) std::uint16_t b2[OB::kElems];
     __shared__ __attribute__((aligned(1024))) std::uint16_t b3[OB::kElems];
-    const Work w = work_of(p, blockIdx.x, gridDim.x);
+    const Work w = work_of((static_cast<unsigned>(p.M) + 32 * MI - 1) / (32 * MI), (static_cast<unsigned>(p.N) + 32 * NJ - 1) / (32 * NJ),
+                           static_cast<unsigned>(p.splits), blockIdx.x, gridDim.x);
     const long row0 = static_cast<long>(w.mt) * (32 * MI), col0 = static_cast<long>(w.nt) * (32 * NJ);
     const long k_first = static_cast<long>(w.split) * p.k_per_split;
     const long k_count = p.K - k_first < p.k_per_split ? p.K - k_first : p.k_per_split;
@@ -76,7 +78,7 @@ __global__ __launch_bounds__(kThreads, (MI * NJ >= 32 || ST * (MI + NJ) > 20 ? 1
     const int l16 = lane & 15, kq = lane >> 4;
     const long wrow = row0 + (wave >> 1) * 16 * MI + l16, wcol = col0 + (wave & 1) * 16 * NJ + 4 * kq;
     if (p.splits > 1) {
-        float* dst = p.partial + (w.batch * p.splits + w.split) * (p.M * p.N);
+        float* dst = static_cast<float*>(p.out) + static_cast<long>(w.batch * p.splits + w.split) * (static_cast<long>(p.M) * p.N);
         const bool vec = p.N % 4 == 0;
 #pragma unroll
         for (int i = 0; i < MI; ++i) {
@@ -96,11 +98,11 @@ __global__ __launch_bounds__(kThreads, (MI * NJ >= 32 || ST * (MI + NJ) > 20 ? 1
         }
         return;
     }
-    std::uint16_t* C = p.c + w.batch * p.sc;
+    std::uint16_t* C = static_cast<std::uint16_t*>(p.out) + w.batch * p.sc;
     const std::uint16_t* ADD = p.add ? p.add + w.batch * p.sadd : nullptr;
     // plain product into rows of 8-byte aligned pieces: the conversion instruction, four columns per store; a
     // row block in which a NaN turns up takes the software narrowing (which writes NaNs as the host's types do)
-    const bool plain = p.alpha == 1.0f && ADD == nullptr && p.ldc % 4 == 0 && p.sc % 4 == 0 && (reinterpret_cast<uintptr_t>(p.c) & 7) == 0;
+    const bool plain = p.alpha == 1.0f && ADD == nullptr && p.ldc % 4 == 0 && p.sc % 4 == 0 && (reinterpret_cast<uintptr_t>(p.out) & 7) == 0;
 #pragma unroll
     for (int i = 0; i < MI; ++i) {
         const long row = wrow + i * 16;

@@ -20,6 +20,7 @@
 
 #include <cmath>
 #include <cstdlib>
+#include <type_traits>
 
 #include "core/device_context.h"
 #include "core/device_math.h"
@@ -39,23 +40,32 @@ constexpr int kMaxRows = 16;        // query rows per KV head (MFMA N)
 typedef short i16x8 __attribute__((ext_vector_type(8)));
 typedef __attribute__((address_space(3))) i16x4 lds_i16x4;
 
+// (112 bytes without a mask: a launch whose arguments take more costs the host 0.7 us more, 3.4 for 2.7, and a call is two of them.)
 struct DecodeParams {
     const std::uint16_t* q;
     const std::uint16_t* k;
     const std::uint16_t* v;
     std::uint16_t* out;
     float* lse;
-    float* part_o;   // [pairs, splits, 16, D]
-    float* part_ml;  // [pairs, splits, 2, 16]
-    long qs_b, qs_h, qs_l, ks_b, ks_h, ks_l, vs_b, vs_h, vs_l;
-    int B, Hq, Hkv, Lq, Lk, G, R;
-    int splits, chunk;  // keys per workgroup
+    float* part;     // [pairs, splits]: 16 maxima, 16 sums, 16 x D outputs
+    int q8_b, q8_h, q8_l, k8_b, k8_h, k8_l, v8_b, v8_h, v8_l;     // strides in eights of elements (decode_supported)
+    int Hkv, Lk;
+    int chunk;       // keys per workgroup
+    std::uint32_t shape;          // splits | Lq << 16 | G << 24
     float scale_log2, scale;
-    // optional mask (element strides; 0 = broadcast): bytes that are zero / non-zero, or additive values of the tensor dtype
+    __device__ int splits() const { return static_cast<int>(shape & 0xffff); }
+    __device__ int Lq() const { return static_cast<int>(shape >> 16 & 0xff); }
+    __device__ int G() const { return static_cast<int>(shape >> 24); }
+};
+static_assert(sizeof(DecodeParams) <= 112, "see above");
+// optional mask (element strides; 0 = broadcast): bytes that are zero / non-zero, or additive values of the tensor dtype
+struct DecodeMaskParams : DecodeParams {
     const unsigned char* mask;
     long ms_b, ms_h, ms_q, ms_k;
     float inv_scale;    // the scores are kept unscaled: an additive mask value m enters as m / scale
 };
+
+__host__ __device__ constexpr long slot_floats(long D) { return kMaxRows * (D + 2); }
 
 template <typename T> struct Mma16;
 template <> struct Mma16<bf16_t> {
@@ -93,7 +103,7 @@ __device__ __forceinline__ float group_sum(float x) {
 
 // kMask: 0 = none, 1 = bool (true = attend), 2 = additive values of dtype T
 template <typename T, int D, int kMask>
-__global__ __launch_bounds__(kThreads, (D > 128 ? 1 : 2)) void decode_split_kernel(const DecodeParams p) {
+__global__ __launch_bounds__(kThreads, (D > 128 ? 1 : 2)) void decode_split_kernel(const typename std::conditional<kMask == 0, DecodeParams, DecodeMaskParams>::type p) {
     constexpr int kD = D, kVS = D + 16;
     constexpr int KS = D / 32;           // 32-wide contraction steps of q k^T
     constexpr int DB = D / 16;           // 16-wide output blocks of O^T
@@ -102,7 +112,7 @@ __global__ __launch_bounds__(kThreads, (D > 128 ? 1 : 2)) void decode_split_kern
     __shared__ __attribute__((aligned(16))) std::uint16_t v_lds[kWaves][2][kTile * (D + 16)];
     __shared__ float m_lds[kWaves][kMaxRows], l_lds[kWaves][kMaxRows];
 
-    const int split = blockIdx.x, pair = blockIdx.y;
+    const int split = blockIdx.x, pair = blockIdx.y, Lq = p.Lq(), G = p.G(), R = G * Lq;
     const int b = pair / p.Hkv, hkv = pair % p.Hkv;
     const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
     const int lq = lane & 15, lg = lane >> 4;
@@ -110,9 +120,9 @@ __global__ __launch_bounds__(kThreads, (D > 128 ? 1 : 2)) void decode_split_kern
     // ---- the query rows of this KV head: row r = gi*Lq + i  (head hkv*G+gi, position i)
     i16x8 qreg[KS];
     {
-        const bool live = lq < p.R;
-        const int gi = live ? lq / p.Lq : 0, qi = live ? lq % p.Lq : 0;
-        const std::uint16_t* qp = p.q + b * p.qs_b + static_cast<long>(hkv * p.G + gi) * p.qs_h + static_cast<long>(qi) * p.qs_l;
+        const bool live = lq < R;
+        const int gi = live ? lq / Lq : 0, qi = live ? lq % Lq : 0;
+        const std::uint16_t* qp = p.q + 8 * (static_cast<long>(b) * p.q8_b + static_cast<long>(hkv * G + gi) * p.q8_h + static_cast<long>(qi) * p.q8_l);
 #pragma unroll
         for (int ks = 0; ks < KS; ++ks) {
             i16x8 z = {0, 0, 0, 0, 0, 0, 0, 0};
@@ -123,9 +133,9 @@ __global__ __launch_bounds__(kThreads, (D > 128 ? 1 : 2)) void decode_split_kern
     // ---- this lane's mask row (query row lq): the 8 keys it scores per tile are 4 lg .. 4 lg + 3 of each 16-key block
     const unsigned char* mrow = nullptr;
     if constexpr (kMask != 0) {
-        const bool live = lq < p.R;
-        const int gi = live ? lq / p.Lq : 0, qi = live ? lq % p.Lq : 0;
-        mrow = p.mask + (static_cast<long>(b) * p.ms_b + static_cast<long>(hkv * p.G + gi) * p.ms_h + static_cast<long>(qi) * p.ms_q) * (kMask == 1 ? 1 : 2);
+        const bool live = lq < R;
+        const int gi = live ? lq / Lq : 0, qi = live ? lq % Lq : 0;
+        mrow = p.mask + (static_cast<long>(b) * p.ms_b + static_cast<long>(hkv * G + gi) * p.ms_h + static_cast<long>(qi) * p.ms_q) * (kMask == 1 ? 1 : 2);
     }
 
     // ---- this wave's key range
@@ -136,8 +146,9 @@ __global__ __launch_bounds__(kThreads, (D > 128 ? 1 : 2)) void decode_split_kern
     const int k_end = min(k_begin + wlen, chunk1);
     const int n_tiles = k_end > k_begin ? (k_end - k_begin + kTile - 1) / kTile : 0;
 
-    const std::uint16_t* kbase = p.k + b * p.ks_b + hkv * p.ks_h;
-    const std::uint16_t* vbase = p.v + b * p.vs_b + hkv * p.vs_h;
+    const std::uint16_t* kbase = p.k + 8 * (static_cast<long>(b) * p.k8_b + static_cast<long>(hkv) * p.k8_h);
+    const long k_row = 8L * p.k8_l, v_row = 8L * p.v8_l;
+    const std::uint16_t* vbase = p.v + 8 * (static_cast<long>(b) * p.v8_b + static_cast<long>(hkv) * p.v8_h);
 
     i16x8 kcur[2][KS], knext[2][KS];
     u32x4 vst[VCH];
@@ -146,7 +157,7 @@ __global__ __launch_bounds__(kThreads, (D > 128 ? 1 : 2)) void decode_split_kern
         for (int kb = 0; kb < 2; ++kb) {
             int key = k_begin + t * kTile + kb * 16 + lq;
             key = key < p.Lk ? key : p.Lk - 1;  // masked later; keep the load in bounds
-            const std::uint16_t* kp = kbase + static_cast<long>(key) * p.ks_l + 8 * lg;
+            const std::uint16_t* kp = kbase + static_cast<long>(key) * k_row + 8 * lg;
 #pragma unroll
             for (int ks = 0; ks < KS; ++ks) dst[kb][ks] = __builtin_bit_cast(i16x8, load16_nt(kp + 32 * ks));  // read once: keep it out of the caches
         }
@@ -157,7 +168,7 @@ __global__ __launch_bounds__(kThreads, (D > 128 ? 1 : 2)) void decode_split_kern
             const int c = lane + i * 64;  // 16-byte chunk of the 32 x D tile
             const int row = c / (D / 8), col = (c % (D / 8)) * 8;
             const int key = k_begin + t * kTile + row;
-            vst[i] = key < k_end ? load16_nt(vbase + static_cast<long>(key) * p.vs_l + col) : u32x4{0, 0, 0, 0};
+            vst[i] = key < k_end ? load16_nt(vbase + static_cast<long>(key) * v_row + col) : u32x4{0, 0, 0, 0};
         }
     };
     auto store_v = [&](int buf) {
@@ -314,7 +325,7 @@ __global__ __launch_bounds__(kThreads, (D > 128 ? 1 : 2)) void decode_split_kern
     __syncthreads();  // everyone is done with the V tiles
     float* o_lds = reinterpret_cast<float*>(&v_lds[0][0][0]);  // [wave][16][D] floats: 32 KB / 16 KB, inside the V tiles' space
     static_assert(sizeof(float) * kWaves * kMaxRows * D <= sizeof(std::uint16_t) * kWaves * 2 * kTile * kVS, "merge space");
-    if (lq < p.R) {
+    if (lq < R) {
 #pragma unroll
         for (int db = 0; db < DB; ++db)
 #pragma unroll
@@ -325,7 +336,7 @@ __global__ __launch_bounds__(kThreads, (D > 128 ? 1 : 2)) void decode_split_kern
         }
     }
     __syncthreads();
-    for (int idx = tid; idx < p.R * kD; idx += kThreads) {
+    for (int idx = tid; idx < R * kD; idx += kThreads) {
         const int r = idx / kD, d = idx % kD;
         float M = -INFINITY;
 #pragma unroll
@@ -338,18 +349,18 @@ __global__ __launch_bounds__(kThreads, (D > 128 ? 1 : 2)) void decode_split_kern
             L += l_lds[w][r] * f;
             O += o_lds[(w * kMaxRows + r) * kD + d] * f;
         }
-        if (p.splits == 1) {
-            const int gi = r / p.Lq, qi = r % p.Lq;
-            const long orow = (static_cast<long>(b) * p.Hq + hkv * p.G + gi) * p.Lq + qi;
+        if (p.splits() == 1) {
+            const int gi = r / Lq, qi = r % Lq;
+            const long orow = ((static_cast<long>(b) * p.Hkv + hkv) * G + gi) * Lq + qi;
             const float val = O / L;
             p.out[orow * kD + d] = static_cast<std::uint16_t>(Mma16<T>::pack2(val, 0.f) & 0xffffu);
             if (p.lse && d == 0) p.lse[orow] = M * p.scale + logf(L);
         } else {
-            const long slot = static_cast<long>(pair) * p.splits + split;
-            p.part_o[(slot * kMaxRows + r) * kD + d] = O;
+            float* slot = p.part + (static_cast<long>(pair) * p.splits() + split) * slot_floats(kD);
+            slot[2 * kMaxRows + r * kD + d] = O;
             if (d == 0) {
-                p.part_ml[(slot * 2 + 0) * kMaxRows + r] = M;
-                p.part_ml[(slot * 2 + 1) * kMaxRows + r] = L;
+                slot[r] = M;
+                slot[kMaxRows + r] = L;
             }
         }
     }
@@ -369,18 +380,18 @@ __global__ __launch_bounds__(kCombine) void decode_combine_kernel(const DecodePa
     __shared__ float4_t o_lds[kCombine];
     const int pair = blockIdx.x, r = blockIdx.y, tid = threadIdx.x, threads = blockDim.x, waves = threads / kWave;
     const int group = tid / kLanes, groups = threads / kLanes, d0 = tid % kLanes * 4;
-    const int b = pair / p.Hkv, hkv = pair % p.Hkv;
-    const long slot0 = static_cast<long>(pair) * p.splits;
-    auto part = [&](int s) { return *reinterpret_cast<const f32x4_any*>(p.part_o + ((slot0 + s) * kMaxRows + r) * D + d0); };
+    const int splits = p.splits(), Lq = p.Lq(), G = p.G();
+    const float* slot0 = p.part + static_cast<long>(pair) * splits * slot_floats(D);
+    auto part = [&](int s) { return *reinterpret_cast<const f32x4_any*>(slot0 + s * slot_floats(D) + 2 * kMaxRows + r * D + d0); };
     float4_t ahead[kAhead];
 #pragma unroll
     for (int i = 0; i < kAhead; ++i) {
         const int s = group + i * groups;
-        ahead[i] = s < p.splits ? float4_t(part(s)) : float4_t{0.f, 0.f, 0.f, 0.f};
+        ahead[i] = s < splits ? float4_t(part(s)) : float4_t{0.f, 0.f, 0.f, 0.f};
     }
     float M = -INFINITY;
-    for (int s = tid; s < p.splits; s += threads) {
-        const float* ml = p.part_ml + (slot0 + s) * 2 * kMaxRows + r;
+    for (int s = tid; s < splits; s += threads) {
+        const float* ml = slot0 + s * slot_floats(D) + r;
         m_lds[s] = ml[0];
         l_lds[s] = ml[kMaxRows];
         M = fmaxf(M, m_lds[s]);
@@ -391,7 +402,7 @@ __global__ __launch_bounds__(kCombine) void decode_combine_kernel(const DecodePa
     __syncthreads();
     for (int w = 0; w < waves; ++w) M = fmaxf(M, wave_m[w]);
     float L = 0.f;
-    for (int s = tid; s < p.splits; s += threads) {
+    for (int s = tid; s < splits; s += threads) {
         const float f = m_lds[s] == -INFINITY ? 0.f : __builtin_amdgcn_exp2f((m_lds[s] - M) * p.scale_log2);
         m_lds[s] = f;
         L += l_lds[s] * f;
@@ -406,16 +417,16 @@ __global__ __launch_bounds__(kCombine) void decode_combine_kernel(const DecodePa
 #pragma unroll
     for (int i = 0; i < kAhead; ++i) {
         const int s = group + i * groups;
-        if (s < p.splits) O += ahead[i] * m_lds[s];
+        if (s < splits) O += ahead[i] * m_lds[s];
     }
 #pragma unroll 4
-    for (int s = group + kAhead * groups; s < p.splits; s += groups) O += float4_t(part(s)) * m_lds[s];
+    for (int s = group + kAhead * groups; s < splits; s += groups) O += float4_t(part(s)) * m_lds[s];
     o_lds[tid] = O;
     __syncthreads();
     if (group != 0) return;
     for (int g = 1; g < groups; ++g) O += o_lds[g * kLanes + tid];
-    const int gi = r / p.Lq, qi = r % p.Lq;
-    const long orow = (static_cast<long>(b) * p.Hq + hkv * p.G + gi) * p.Lq + qi;
+    const int gi = r / Lq, qi = r % Lq;
+    const long orow = (static_cast<long>(pair) * G + gi) * Lq + qi;
 #pragma unroll
     for (int i = 0; i < 4; ++i) p.out[orow * D + d0 + i] = static_cast<std::uint16_t>(Mma16<T>::pack2(O[i] / L, 0.f) & 0xffffu);
     if (p.lse && tid == 0) p.lse[orow] = M * p.scale + logf(L);
@@ -474,7 +485,7 @@ void plan(const paras_sdpa_args& a, bool may_split, int* splits, int* chunk) {
 size_t workspace_of(const paras_sdpa_args& a, int splits) {
     if (splits == 1) return 0;
     const size_t slots = static_cast<size_t>(a.B * a.Hkv) * splits;
-    return slots * (kMaxRows * a.D + 2 * kMaxRows) * sizeof(float);
+    return slots * slot_floats(a.D) * sizeof(float);
 }
 
 }  // namespace
@@ -491,6 +502,9 @@ bool decode_supported(const paras_sdpa_args& a) {
     if (!(a.scale > 0.0) || !std::isfinite(a.scale)) return false;
     if (!aligned16(a.q) || !aligned16(a.k) || !aligned16(a.v)) return false;
     if (!mult8(a.q_strides) || !mult8(a.k_strides) || !mult8(a.v_strides)) return false;
+    for (const int64_t* st : {a.q_strides, a.k_strides, a.v_strides})
+        for (int i = 0; i < 3; ++i)
+            if (st[i] / 8 != static_cast<int>(st[i] / 8)) return false;          // (DecodeParams)
     return true;
 }
 
@@ -503,40 +517,41 @@ size_t decode_workspace(const paras_sdpa_args& a) {
 bool decode_fills_chip(const paras_sdpa_args& a) { return a.B * a.Hkv >= 2 * compute_units(); }
 
 int launch_decode(const paras_sdpa_args& a, Scratch scratch, hipStream_t s) {
-    DecodeParams p;
+    DecodeMaskParams p;
     p.q = static_cast<const std::uint16_t*>(a.q);
     p.k = static_cast<const std::uint16_t*>(a.k);
     p.v = static_cast<const std::uint16_t*>(a.v);
     p.out = static_cast<std::uint16_t*>(a.out);
     p.lse = a.lse;
-    p.qs_b = a.q_strides[0]; p.qs_h = a.q_strides[1]; p.qs_l = a.q_strides[2];
-    p.ks_b = a.k_strides[0]; p.ks_h = a.k_strides[1]; p.ks_l = a.k_strides[2];
-    p.vs_b = a.v_strides[0]; p.vs_h = a.v_strides[1]; p.vs_l = a.v_strides[2];
-    p.B = (int)a.B; p.Hq = (int)a.Hq; p.Hkv = (int)a.Hkv; p.Lq = (int)a.Lq; p.Lk = (int)a.Lk;
-    p.G = (int)(a.Hq / a.Hkv);
-    p.R = p.G * p.Lq;
-    plan(a, scratch.p != nullptr && aligned16(scratch.p), &p.splits, &p.chunk);
-    if (p.splits > 1 && !scratch.has(workspace_of(a, p.splits))) plan(a, false, &p.splits, &p.chunk);
+    auto eights = [](int64_t stride) { return static_cast<int>(stride / 8); };
+    p.q8_b = eights(a.q_strides[0]); p.q8_h = eights(a.q_strides[1]); p.q8_l = eights(a.q_strides[2]);
+    p.k8_b = eights(a.k_strides[0]); p.k8_h = eights(a.k_strides[1]); p.k8_l = eights(a.k_strides[2]);
+    p.v8_b = eights(a.v_strides[0]); p.v8_h = eights(a.v_strides[1]); p.v8_l = eights(a.v_strides[2]);
+    p.Hkv = (int)a.Hkv; p.Lk = (int)a.Lk;
+    const int G = (int)(a.Hq / a.Hkv), R = G * (int)a.Lq;
+    int splits = 1;
+    plan(a, scratch.p != nullptr && aligned16(scratch.p), &splits, &p.chunk);
+    if (splits > 1 && !scratch.has(workspace_of(a, splits))) plan(a, false, &splits, &p.chunk);
+    p.shape = static_cast<std::uint32_t>(splits) | static_cast<std::uint32_t>(a.Lq) << 16 | static_cast<std::uint32_t>(G) << 24;
     p.scale = static_cast<float>(a.scale);
     p.scale_log2 = static_cast<float>(a.scale * 1.4426950408889634);
-    const size_t slots = static_cast<size_t>(a.B * a.Hkv) * p.splits;
-    p.part_o = static_cast<float*>(scratch.p);
-    p.part_ml = p.part_o ? p.part_o + slots * kMaxRows * a.D : nullptr;
-    const dim3 grid(p.splits, static_cast<unsigned>(a.B * a.Hkv));
+    p.part = static_cast<float*>(scratch.p);
+    const dim3 grid(splits, static_cast<unsigned>(a.B * a.Hkv));
     p.mask = static_cast<const unsigned char*>(a.mask);
     p.ms_b = a.mask_strides[0]; p.ms_h = a.mask_strides[1]; p.ms_q = a.mask_strides[2]; p.ms_k = a.mask_strides[3];
     p.inv_scale = static_cast<float>(1.0 / a.scale);
+    const DecodeParams& plain = p;
     const bool bf = a.dtype == PARAS_BF16;
     const dim3 block(kThreads);
-    const dim3 g2(static_cast<unsigned>(a.B * a.Hkv), p.R);
+    const dim3 g2(static_cast<unsigned>(a.B * a.Hkv), R);
 #define PARAS_DECODE_LAUNCH(T_, D_)                                                                        \
     do {                                                                                                   \
-        if (a.mask_kind == 0)      hipLaunchKernelGGL((decode_split_kernel<T_, D_, 0>), grid, block, 0, s, p); \
+        if (a.mask_kind == 0)      hipLaunchKernelGGL((decode_split_kernel<T_, D_, 0>), grid, block, 0, s, plain); \
         else if (a.mask_kind == 1) hipLaunchKernelGGL((decode_split_kernel<T_, D_, 1>), grid, block, 0, s, p); \
         else                       hipLaunchKernelGGL((decode_split_kernel<T_, D_, 2>), grid, block, 0, s, p); \
         PARAS_HIP_TRY(hipGetLastError());                                                                  \
-        if (p.splits > 1) {                                                                                \
-            hipLaunchKernelGGL((decode_combine_kernel<T_, D_>), g2, dim3(combine_threads(p.splits, D_)), 0, s, p);                    \
+        if (splits > 1) {                                                                                  \
+            hipLaunchKernelGGL((decode_combine_kernel<T_, D_>), g2, dim3(combine_threads(splits, D_)), 0, s, plain);                  \
             PARAS_HIP_TRY(hipGetLastError());                                                              \
         }                                                                                                  \
     } while (0)

@@ -246,15 +246,21 @@ __global__ __launch_bounds__(kBlock) void rotate_half_vec16(const std::uint16_t*
 
 // The same for rows of D contiguous elements that lie anywhere: a projection's heads seen as [B, h, S, D], which were copied
 // together first (bf16 [1, 32, 1500, 128] and [1, 8, 1500, 128], transposed views: 22.3 us, 12.6 this way).
-struct RowDims {
+// (Up to four dimensions: the arguments stay within 112 bytes; more cost a launch 0.7 us more of the host's time, 3.4 for 2.7.)
+template <int ND> struct RowDims {
+    const std::uint16_t* x;
+    std::uint16_t* out;
+    unsigned nvec;
     int ndim;                    // the last dim is the row, in vectors
-    unsigned sizes[8];
-    long strides[8];             // elements
+    int backward, nan_kind;
+    unsigned sizes[ND];
+    long strides[ND];            // elements
 };
-__global__ __launch_bounds__(kBlock) void rotate_half_rows_vec16(const std::uint16_t* __restrict__ x, std::uint16_t* __restrict__ out,
-                                                                 unsigned nvec, const RowDims s, int backward, int nan_kind) {
+static_assert(sizeof(RowDims<4>) <= 112, "see above");
+template <int ND>
+__global__ __launch_bounds__(kBlock) void rotate_half_rows_vec16(const RowDims<ND> s) {
     const unsigned i = blockIdx.x * kBlock + threadIdx.x;
-    if (i >= nvec) return;
+    if (i >= s.nvec) return;
     const unsigned half = s.sizes[s.ndim - 1] / 2;
     unsigned left = i / s.sizes[s.ndim - 1];
     const unsigned col = i - left * s.sizes[s.ndim - 1];
@@ -265,9 +271,9 @@ __global__ __launch_bounds__(kBlock) void rotate_half_rows_vec16(const std::uint
         at += static_cast<long>(left - q * s.sizes[d]) * s.strides[d];
         left = q;
     }
-    u32x4 v = load16(x + at);
-    rotate_piece(v, backward ? !first : first, nan_kind);
-    store16(out + static_cast<long>(i) * 8, v);
+    u32x4 v = load16(s.x + at);
+    rotate_piece(v, s.backward ? !first : first, s.nan_kind);
+    store16(s.out + static_cast<long>(i) * 8, v);
 }
 
 int stream_grid(long work_items_per_block_iter, long total) {
@@ -422,7 +428,7 @@ int paras_rotate_half_strided(const void* x, void* out, int ndim, const int64_t*
     PARAS_REQUIRE(dtype == PARAS_BF16 || dtype == PARAS_F16, "paras_rotate_half_strided: 16-bit dtypes only");
     PARAS_REQUIRE(ndim >= 1 && ndim <= 8 && sizes && strides, "paras_rotate_half_strided: 1 to 8 dimensions");
     PARAS_REQUIRE(sizes[ndim - 1] % 16 == 0 && strides[ndim - 1] == 1, "paras_rotate_half_strided: rows of a multiple of 16 contiguous elements");
-    RowDims d{};
+    RowDims<8> d{};
     long n = 1;
     for (int k = 0; k < ndim; ++k) {
         PARAS_REQUIRE(sizes[k] >= 0 && (k == ndim - 1 || strides[k] % 8 == 0), "paras_rotate_half_strided: rows that begin on 16 bytes");
@@ -443,9 +449,22 @@ int paras_rotate_half_strided(const void* x, void* out, int ndim, const int64_t*
     hipStream_t s = nullptr;
     int rc = resolve_stream(stream, &s);
     if (rc != PARAS_OK) return rc;
-    const unsigned nvec = static_cast<unsigned>(n / 8);
-    hipLaunchKernelGGL(rotate_half_rows_vec16, dim3((nvec + kBlock - 1) / kBlock), dim3(kBlock), 0, s, static_cast<const uint16_t*>(x),
-                       static_cast<uint16_t*>(out), nvec, d, backward, dtype == PARAS_BF16 ? 1 : 2);
+    d.x = static_cast<const uint16_t*>(x);
+    d.out = static_cast<uint16_t*>(out);
+    d.nvec = static_cast<unsigned>(n / 8);
+    d.backward = backward;
+    d.nan_kind = dtype == PARAS_BF16 ? 1 : 2;
+    const dim3 grid((d.nvec + kBlock - 1) / kBlock), block(kBlock);
+    if (d.ndim <= 4) {
+        RowDims<4> few{d.x, d.out, d.nvec, d.ndim, d.backward, d.nan_kind, {}, {}};
+        for (int k = 0; k < d.ndim; ++k) {
+            few.sizes[k] = d.sizes[k];
+            few.strides[k] = d.strides[k];
+        }
+        hipLaunchKernelGGL((rotate_half_rows_vec16<4>), grid, block, 0, s, few);
+    } else {
+        hipLaunchKernelGGL((rotate_half_rows_vec16<8>), grid, block, 0, s, d);
+    }
     PARAS_HIP_TRY(hipGetLastError());
     return PARAS_OK;
 }
