@@ -31,8 +31,9 @@
 // What bounds it: small problems the chain of one turn (two memory latencies, products, merge; B1 H8 S128 D64 causal 6.9 us),
 // large ones the matrix cores and the vector instructions, which do not run beside fp32 MFMAs here (weights of one query
 // block interleaved with the products of the other, one MFMA to seven vector instructions: 874 -> 903 us).  B2 H16 S2048
-// D128: unmasked 742 us = 93 TFLOP/s, causal 623 (every value is read, seen or not: 25 of them), 30 % padding 775, an additive
-// mask 830; the batched products took 967 / 907 / 1520 / 1590.  B2 H8 S1024 D64 55 us (174), B1 H4 S2048 D256 203 (317).  With the
+// D128: unmasked 696-705 us = 98 TFLOP/s, causal 512-520 (every value is read, seen or not: 25 of them), 30 % padding 731, an additive
+// mask 834; the batched products took 967 / 907 / 1520 / 1590.  B2 H8 S1024 D64 57 us (174), B1 H4 S2048 D256 206 (317).  (With blocks of 32 queries
+// at 64 and 128 elements, turns of 32 keys and the softmax in fp64 742 / 623 / 775 / 830, 55 and 203.)  With those and the
 // softmax in fp32 it took 697 / 567 / 665 / 950, 47 and 228, and single weights were 4.9e-7 off instead of 1.1e-7.
 #include <hip/hip_runtime.h>
 
@@ -87,7 +88,7 @@ template <> struct Mma<float> {
 // A turn is KB blocks of 16 keys.  kMask: 0 = none, 1 = bool (true = attend), 2 = additive.
 // (heads of up to 64 elements leave registers for two waves per SIMD)
 template <typename Acc, int DM, int QB, int KB, int kMask>
-__global__ __launch_bounds__(kWavesF * 64, DM == 64 ? 2 : 1) void sdpa_f32_kernel(const F32Params p) {
+__global__ __launch_bounds__(kWavesF * 64, DM == 64 || (DM == 128 && KB == 1 && sizeof(Acc) == 4) ? 2 : 1) void sdpa_f32_kernel(const F32Params p) {
     using M = Mma<Acc>;
     using vec = typename M::vec;
     constexpr int DC = DM / 16, VC = DM / 64, kTurn = 16 * KB;
@@ -415,7 +416,7 @@ __global__ __launch_bounds__(kWavesF * 64, DM == 64 ? 2 : 1) void sdpa_f32_kerne
 // The returned weights, in place of the scores that sdpa_f32_kernel left: exp(score - reference) / sum in fp64, rounded
 // once; zeros for the keys that the causal rule hides (NaN where the row is).  A wave takes a row in pieces of W elements.
 // Bound by memory (one read and one write of the weights tensor); four pieces are on the way at a time.  B2 H16 S2048 D128 with
-// its 537 MB of weights 1000 us, causal 805; the product, row kernel and product in their place 967 and 907; B2 H8 S1024 D64 89 (174).
+// its 537 MB of weights 988 us, causal 719; the product, row kernel and product in their place 967 and 907; B2 H8 S1024 D64 89 (174).
 template <int W>
 __global__ __launch_bounds__(256) void softmax_rows_kernel(float* __restrict__ attn, const double2* __restrict__ row_sums, long rows, int Lq, int Lk, int is_causal) {
     typedef float piece __attribute__((ext_vector_type(W)));
@@ -467,12 +468,19 @@ void launch_dm(const F32Params& p, const paras_sdpa_args& a, hipStream_t s) {
         }
         launch_form<Acc, DM, 1, 1>(p, a, s);
     } else {
-        // 32 queries per workgroup read K and V half as often; at 256 elements the registers do not hold them, and
-        // below two workgroups per CU 16 queries spread the work better
-        if constexpr (DM <= 128) {
-            if ((a.Lq + 31) / 32 * a.Hq * a.B >= 512) return launch_form<Acc, DM, 2, 2>(p, a, s);
+        // Turns of 16 keys for 16 queries take the fewest registers, and what they leave room for, two workgroups per CU at 128 elements and
+        // four at 64, is worth more than the operands that larger blocks share (us, 16 queries x 16 keys / 16 x 32 / 32 x 32: D128 B3 H8 S145 causal
+        // 10.5 / 12.5 / 21.1, B1 H64 S300 46.7 / 69.6 / 72.8, B2 H16 S2048 696 / 831 / 742; D64 B9 H16 S66 9.1 / 11.0 / 13.3, B1 H64 S300
+        // 27.8 / 30.8 / 34.4; D256 B2 H16 S600 140 / 152).  With 64 elements and more keys than a few turns each the larger turns are ahead, for
+        // they wait for half as many row maxima (B1 H4 S4000 causal 196 / 153 / 188, B1 H1 S3000 51 / 47 / 83), and, without mask or causal rule, blocks
+        // of 32 queries where they fill the chip (B2 H16 S2048 400 / 400 / 385).
+        if constexpr (DM == 64) {
+            if (a.Lk > 320) {
+                if (a.mask_kind == 0 && !a.is_causal && (a.Lq + 31) / 32 * a.Hq * a.B >= 448) return launch_form<Acc, DM, 2, 2>(p, a, s);
+                return launch_form<Acc, DM, 1, 2>(p, a, s);
+            }
         }
-        launch_form<Acc, DM, 1, 2>(p, a, s);
+        launch_form<Acc, DM, 1, 1>(p, a, s);
     }
 }
 

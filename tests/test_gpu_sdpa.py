@@ -984,6 +984,19 @@ def test_flash_either_side_of_the_limits_of_the_wide_kernel(B, H, S, causal, wid
         assert max_abs(out[b:b + 1, h:h + 1], want) <= ABS_16BIT
 
 
+@pytest.mark.parametrize("B,H,S,D", [(8, 8, 320, 64), (8, 8, 321, 64), (4, 8, 449, 64), (4, 8, 417, 64), (9, 16, 66, 128), (4, 8, 333, 128), (3, 8, 200, 256), (8, 4, 100, 96)])
+@pytest.mark.parametrize("kind", ["none", "causal", "padding"])
+def test_fp32_attention_either_side_of_its_forms(B, H, S, D, kind):
+    """Turns of 16 or 32 keys, blocks of 16 or 32 queries, by head size, keys, mask and number of query blocks: against fp64 to the bar of the
+    one-pass kernel (3e-6 relative)."""
+    torch.manual_seed(S)
+    q, k, v = torch.randn(B, H, S, D), torch.randn(B, H, S, D), torch.randn(B, H, S, D)
+    mask = (torch.arange(S)[None, :] < torch.randint(S // 2, S + 1, (B, 1))).reshape(B, 1, 1, S).expand(B, H, S, S) if kind == "padding" else None
+    out, _, _, _ = run(q, k, v, is_causal=kind == "causal", **({"mask": mask} if mask is not None else {}))
+    want = torch.nn.functional.scaled_dot_product_attention(q.double(), k.double(), v.double(), attn_mask=mask, is_causal=kind == "causal")
+    assert rel_err(out, want) <= 3e-6
+
+
 def test_composed_route_fp64_and_wide_16_bit_heads():
     torch.manual_seed(5)
     q, k, v = _composed_case(torch.float64, 1, 4, 4, 2048, 2048, 32)
