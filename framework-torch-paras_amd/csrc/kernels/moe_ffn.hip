@@ -50,7 +50,7 @@ struct FfnGemmParams {
     int E, k;
     int mt_total;               // upper bound on m-tiles
     int n_units;                // column units (128 output columns for GEMM 1, 256 for GEMM 2)
-    int ngt;                    // column units an XCD sweeps together
+    int ngt;                    // column units an XCD sweeps together (register-staged tiles); 256 x 256 tiles: 1 = dealt one by one
     unsigned div_m;             // flat (token, slot) index / k as a multiplication: (x * div_m) >> div_s
     int div_s;                  // for every x < 2^30 (a 64-bit division per gathered row is ~150 instructions)
 };
@@ -211,6 +211,8 @@ struct SwigluQueue {
     unsigned where[kEntries];       // (row in the tile) << 16 | column in the column unit
     flex::float4v gate[kEntries], up[kEntries];
 };
+__device__ __forceinline__ unsigned scalar_of(unsigned v) { return static_cast<unsigned>(__builtin_amdgcn_readfirstlane(static_cast<int>(v))); }
+constexpr int kTileBand = 8;        // m-tiles whose column units an XCD walks through together: they share the experts' weights in its L2
 constexpr int kSuperM = 8, kSuperN = 4;
 constexpr int kStageElems = 256 * kBK;          // a stage of either operand: 256 rows of a k-tile
 static_assert(sizeof(SwigluQueue) <= kStageElems * 2, "a queue in a tile stage");
@@ -314,35 +316,52 @@ __global__ __launch_bounds__(flex::kThreads, 1) void grouped_gemm_direct_kernel(
     // routed rows and 4 to 8 of weights between them (a sweep of all row tiles over two column units: 18 to 20).
     // They are dealt to the XCDs one after the other, columns first, so that the XCDs share the rows' panels.
     // (8192 tokens, 8 experts, H 4096, I 14336, the layer: 8 x 4 4675 us, 4 x 8 4750, 16 x 2 4760, 32 x 1 for the plain product 4820.)
-    int mt, nu;
-    {
-        const unsigned xcd = blockIdx.x & 7, j = blockIdx.x >> 3;
-        const unsigned super = j / (kSuperM * kSuperN) * 8 + xcd, in = j % (kSuperM * kSuperN);
-        const unsigned across = (static_cast<unsigned>(p.n_units) + kSuperN - 1) / kSuperN;
-        // (quotients come from vector arithmetic: what depends on them is to stay in scalar registers)
-        const unsigned mb = static_cast<unsigned>(__builtin_amdgcn_readfirstlane(static_cast<int>(super / across)));
-        mt = static_cast<int>(mb * kSuperM + in % kSuperM);
-        nu = static_cast<int>((super - mb * across) * kSuperN + in / kSuperM);
-        if (nu >= p.n_units) return;
-    }
     // m-tile -> (expert, first row): first every expert's tiles with more than 64 rows, then the short last ones, which
     // take a fraction of the time and fill in at the end of every XCD's list
+    int mt, nu;
     int e;
     long row0, row_end;
     {
-        auto whole = [](int rows) { return rows / kBM + (rows % kBM > 64); };
-        auto ends = [](int rows) { return static_cast<int>(rows % kBM > 0 && rows % kBM <= 64); };
         ExpertTiles head;
-        head.look(p, 0, whole);
-        const int n_whole = count_tiles(p, head, whole);
         TileOf at;
-        if (mt < n_whole) {
-            at = find_tile(p, mt, head, whole);
+        if (p.ngt != 0) {
+            // A few rounds of tiles: a contiguous run of the tiles that there are for every XCD, as grouped_tile_kernel deals them, since a few
+            // super-tiles, some of them half empty, are not the same number for all (down in bf16, 5595 tokens, top-2, 8 experts, H 2112,
+            // I 5760: 368 us in super-tiles, 272; gate-up in fp16, 1668 tokens, top-1, 4 experts, 832 x 3264, less than a round: 61 on tiles of
+            // 128 x 128, 41).  Expert by expert: with the short tiles at the end of the list one XCD has most of them (3056 tokens, top-6,
+            // 64 experts, 1472 x 768, the layer: 290, and 271 so).
+            auto tiles_of = [](int rows) { return (rows + kBM - 1) / kBM; };
+            head.look(p, 0, tiles_of);
+            const unsigned m_tiles = static_cast<unsigned>(count_tiles(p, head, tiles_of)), units = static_cast<unsigned>(p.n_units);
+            const unsigned total = m_tiles * units, q = total / 8, r = total % 8, x = blockIdx.x % 8, i = blockIdx.x / 8;
+            if (i >= q + (x < r ? 1 : 0)) return;
+            const unsigned lin = x * q + (x < r ? x : r) + i;
+            const unsigned band = scalar_of(lin / (kTileBand * units)), in = lin - band * kTileBand * units;
+            const unsigned left = m_tiles - band * kTileBand, rows = left < kTileBand ? left : kTileBand;
+            nu = static_cast<int>(scalar_of(in / rows));
+            mt = static_cast<int>(band * kTileBand + (in - static_cast<unsigned>(nu) * rows));
+            at = find_tile(p, mt, head, tiles_of);
         } else {
-            head.count(ends);
-            if (mt - n_whole >= count_tiles(p, head, ends)) return;
-            at = find_tile(p, mt - n_whole, head, ends);
-            at.nth = (at.hi - at.lo) / kBM;
+            const unsigned xcd = blockIdx.x & 7, j = blockIdx.x >> 3;
+            const unsigned super = j / (kSuperM * kSuperN) * 8 + xcd, in = j % (kSuperM * kSuperN);
+            const unsigned across = (static_cast<unsigned>(p.n_units) + kSuperN - 1) / kSuperN;
+            // (quotients come from vector arithmetic: what depends on them is to stay in scalar registers)
+            const unsigned mb = static_cast<unsigned>(__builtin_amdgcn_readfirstlane(static_cast<int>(super / across)));
+            mt = static_cast<int>(mb * kSuperM + in % kSuperM);
+            nu = static_cast<int>((super - mb * across) * kSuperN + in / kSuperM);
+            if (nu >= p.n_units) return;
+            auto whole = [](int rows) { return rows / kBM + (rows % kBM > 64); };
+            auto ends = [](int rows) { return static_cast<int>(rows % kBM > 0 && rows % kBM <= 64); };
+            head.look(p, 0, whole);
+            const int n_whole = count_tiles(p, head, whole);
+            if (mt < n_whole) {
+                at = find_tile(p, mt, head, whole);
+            } else {
+                head.count(ends);
+                if (mt - n_whole >= count_tiles(p, head, ends)) return;
+                at = find_tile(p, mt - n_whole, head, ends);
+                at.nth = (at.hi - at.lo) / kBM;
+            }
         }
         e = at.e;
         row0 = at.lo + static_cast<long>(at.nth) * kBM;
@@ -527,9 +546,6 @@ template <int NJ> struct GateUp : flex::Operand<NJ, false> {
         flex::Operand<NJ, false>::request((2 * i) % NJ >= NJ / 2 ? r.g[1] : r.g[0], tile, i);
     }
 };
-
-__device__ __forceinline__ unsigned scalar_of(unsigned v) { return static_cast<unsigned>(__builtin_amdgcn_readfirstlane(static_cast<int>(v))); }
-constexpr int kTileBand = 8;        // m-tiles whose column units an XCD walks through together: they share the experts' weights in its L2
 
 template <typename T, bool kSwiglu, int MI, int NJ, int ST>
 __global__ __launch_bounds__(flex::kThreads, (MI * NJ >= 32 || ST * (MI + NJ) > 20 ? 1 : 2)) void grouped_tile_kernel(const FfnGemmParams p) {
@@ -838,17 +854,30 @@ int run_ffn_any(const void* x, const void* w_gate, const void* w_up, const void*
 }
 
 // The tiles of a grouped product: rows, weight rows, stages, workgroups a CU holds, and for the gate-up product and the plain one the time
-// in us of 64 contraction steps on a CU that is full (`step`) and at least (`lat`).  The last is grouped_gemm_direct_kernel.
+// in us of 64 contraction steps on a CU that is full (`step`) and at least (`lat`).  The last two are grouped_gemm_direct_kernel, its tiles dealt in
+// super-tiles or one by one.
 struct GroupedForm { int m, n, stages, per_cu; double step[2], lat[2]; };
 constexpr GroupedForm kForms[] = {{128, 128, 2, 2, {0.91, 0.78}, {0.66, 0.47}}, {128, 128, 3, 1, {0.54, 0.36}, {0.13, 0.02}}, {64, 128, 2, 3, {0.74, 0.33}, {0.51, 0.42}},
-                                  {64, 128, 4, 1, {0.19, 0.24}, {0.35, 0.23}}, {32, 128, 4, 2, {0.30, 0.07}, {0.15, 0.16}}, {256, 256, 2, 1, {1.13, 0.97}, {0.32, 0.30}}};
-constexpr int kFormCount = sizeof(kForms) / sizeof(kForms[0]), kDirectForm = kFormCount - 1;
+                                  {64, 128, 4, 1, {0.19, 0.24}, {0.35, 0.23}}, {32, 128, 4, 2, {0.30, 0.07}, {0.15, 0.16}}, {256, 256, 2, 1, {1.13, 0.97}, {0.32, 0.30}},
+                                  {256, 256, 2, 1, {1.13, 0.97}, {0.32, 0.30}}};
+constexpr int kFormCount = sizeof(kForms) / sizeof(kForms[0]), kDirectForm = kFormCount - 2, kOneByOne = kFormCount - 1;
+
+// Tiles of 256 rows where each of E experts has R / E rows on average and each row is sent on its own (a normal distribution).
+double tiles_256(long E, long R) {
+    const double rows = static_cast<double>(R) / E, spread = std::sqrt(2.0 * rows);
+    double n = 1.0 - std::exp(-rows);
+    for (double j = 256; j < rows + 3 * spread; j += 256) n += 0.5 * std::erfc((j + 0.5 - rows) / spread);
+    return E * n;
+}
 
 // The least estimated time, from three that overlap for the most part (the fourth root of the sum of their fourth powers): rounds of
 // workgroups times their contraction and stores, the way of the weights from memory, and that of all tiles' operands from the caches.  (How
 // the rows are spread over the experts is known on the device only: half an empty tile per expert, one tile where an expert has less than two
 // thirds of one.)  Fitted to 1800 timings of 150 layers (8 to 8192 tokens, 4 to 64 experts, H 512 to 4096, I 512 to 14336), over which the
-// choice is 2 % (gate-up) and 5 % (down) slower than the best form in the mean; always the same form is 15 % and 22 % at the least.
+// choice is 2 % (gate-up) and 5 % (down) slower than the best form in the mean; always the same form is 15 % and 22 % at the least.  (256 x 256 tiles one
+// by one came later, for up to three rounds: of more the last is a small part.  One tile too many is a round, so their number is estimated by the
+// spread of the rows, with 3 % more, and a round is taken 5 % and 6 us longer than the contraction and stores, which is what separates 33 products near
+// the line: none over 4 % slower than the other forms would be, the mean 8 % faster.  36 layers of 500 to 8192 tokens: 0.3 % slower to 34 % faster, the mean 6 %.)
 int grouped_form(bool swiglu, long E, long R, long N, long K) {
     const int w = swiglu ? 0 : 1;
     const double start = swiglu ? 3.9 : 1.3, store = swiglu ? 15.4 : 9.4, rows = static_cast<double>(R) / E, used = R < E ? R : E;
@@ -859,7 +888,8 @@ int grouped_form(bool swiglu, long E, long R, long N, long K) {
     for (int f = 0; f < kFormCount; ++f) {
         const GroupedForm& t = kForms[f];
         const long cols = swiglu ? t.n / 2 : t.n, units = (N + cols - 1) / cols, k_tiles = K / kBK, turns = (k_tiles + t.stages - 1) / t.stages * t.stages;
-        const double m_tiles = rows < 0.7 * t.m ? used : E * (rows / t.m + 0.5), tiles = m_tiles * units;
+        if (f == kOneByOne && static_cast<double>(R) / 256 * units > 3 * 256) continue;
+        const double m_tiles = f == kOneByOne ? tiles_256(E, R) : rows < 0.7 * t.m ? used : E * (rows / t.m + 0.5), tiles = m_tiles * units;
         auto round = [&](double n) {
             const double c = t.step[w] * n / t.per_cu;
             return turns * (c > t.lat[w] ? c : t.lat[w]) + start + store * t.m * cols / 65536.0 * n;
@@ -867,6 +897,8 @@ int grouped_form(bool swiglu, long E, long R, long N, long K) {
         double us;
         if (f == kDirectForm) {          // super-tiles of 32 workgroups, dealt to the 8 XCDs
             us = std::ceil(std::ceil(m_tiles / kSuperM) * std::ceil(static_cast<double>(units) / kSuperN) / 8) * round(1.0);
+        } else if (f == kOneByOne) {
+            us = 1.05 * std::ceil(1.03 * tiles / 256) * (round(1.0) + 6.0);
         } else {
             const double slots = 256.0 * t.per_cu, full = std::floor(tiles / slots), rest = std::ceil((tiles - full * slots) / 256.0);
             us = full * round(t.per_cu) + (rest > 0 ? round(rest) : 0.0);
@@ -895,8 +927,11 @@ void launch_form(int form, FfnGemmParams g, hipStream_t s) {
         case 2: hipLaunchKernelGGL((grouped_tile_kernel<T, kSwiglu, 2, 4, 2>), grid, block, 0, s, g); break;
         case 3: hipLaunchKernelGGL((grouped_tile_kernel<T, kSwiglu, 2, 4, 4>), grid, block, 0, s, g); break;
         case 4: hipLaunchKernelGGL((grouped_tile_kernel<T, kSwiglu, 1, 4, 4>), grid, block, 0, s, g); break;
-        default:
-            hipLaunchKernelGGL((grouped_gemm_direct_kernel<T, kSwiglu>), dim3(static_cast<unsigned>((supers + 7) / 8 * 8 * kSuperM * kSuperN)), block, 0, s, g);
+        default: {
+            g.ngt = form == kOneByOne ? 1 : 0;
+            const long wgs = form == kOneByOne ? (static_cast<long>(g.mt_total) * g.n_units + 7) / 8 * 8 : (supers + 7) / 8 * 8 * kSuperM * kSuperN;
+            hipLaunchKernelGGL((grouped_gemm_direct_kernel<T, kSwiglu>), dim3(static_cast<unsigned>(wgs)), block, 0, s, g);
+        }
     }
 }
 

@@ -455,10 +455,12 @@ def test_route_recorded_into_a_graph_and_replayed():
             assert_bit_exact(e, w, f"eager call {trial}: moe_route {name}")
 
 
-# (gate-up and down between them run on every tile form: 128-row ones with two and three stages, 64-row ones with two and four, 32- and 256-row ones)
+# (gate-up and down between them run on every tile form: 128-row ones with two and three stages, 64-row ones with two and four,
+# 32- and 256-row ones, the last of them dealt in super-tiles and one by one)
 TILE_SHAPES = [(1843, 70, 6, 192, 256), (2055, 32, 4, 192, 192), (1188, 70, 6, 192, 192), (2555, 70, 6, 128, 192), (395, 70, 6, 640, 192), (167, 32, 4, 704, 384),
                (727, 70, 6, 576, 192), (163, 70, 6, 192, 128), (159, 70, 6, 320, 768), (2778, 70, 6, 960, 448), (45, 4, 1, 256, 320), (2769, 70, 6, 192, 512),
-               (2756, 4, 1, 768, 320), (2978, 8, 2, 960, 128), (2581, 8, 2, 320, 256), (2861, 32, 4, 960, 128)]
+               (2756, 4, 1, 768, 320), (2978, 8, 2, 960, 128), (2581, 8, 2, 320, 256), (2861, 32, 4, 960, 128), (1834, 32, 4, 192, 896),
+               (2006, 70, 6, 704, 384), (1796, 32, 4, 1472, 576)]
 
 
 @pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])
