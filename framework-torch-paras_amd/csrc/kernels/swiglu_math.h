@@ -146,8 +146,12 @@ __device__ __forceinline__ void swiglu4_from_acc(const V a0, const V a1, typenam
 // q crosses zero near g = -1.278: rho grows without bound there and those elements take the exact
 // tier.  One more unit for the last product; a relative error of E units is less than E fp32 ulps of the result,
 // which is what narrow_is_safe takes.  (The bounds by analysis were three times as wide, and so was the share of the elements
-// that came to the fp64 tier: 8192 x 14336 in fp16 272 us, with these 237; bf16, where few did, 186 and 183.)
-constexpr std::uint32_t kSwigluBwdUlps = 10;
+// that came to the fp64 tier: 8192 x 14336 in fp16 272 us, with these 237.)  bf16, with 32 times fewer elements near a
+// boundary, keeps bounds of that width: the kernel is bound by memory, and with hardly a wave going to the fp64 tier the
+// waves of a CU stay in step and a forward and backward in turn take longer, 309 us at 8192 x 14336 for 293 with these (188.7 and 182.5
+// at 6553 x 11008).
+template <typename T> struct SwigluBwdUlps { static constexpr std::uint32_t kAll = 10, kGate = 12; static constexpr float kPerRho = 2.5f; };
+template <> struct SwigluBwdUlps<bf16_t> { static constexpr std::uint32_t kAll = 36, kGate = 36; static constexpr float kPerRho = 10.0f; };
 
 template <typename T>
 __device__ __forceinline__ void swiglu_bwd_exact(float dy, float g, float u, typename Elem<T>::store_t& dgate,
@@ -170,8 +174,8 @@ __device__ __forceinline__ void swiglu_bwd_fast(float dy, float g, float u, floa
     yg = (dy * u) * (r * q);
     const float rho = fabsf(ger) * __builtin_amdgcn_rcpf(fabsf(q));
     const bool in_range = (fabsf(g - 26.0f) <= 34.0f) && (rho < 4096.0f);     // -8 <= g <= 60, q well away from zero; false for NaN
-    const std::uint32_t ulps_g = static_cast<std::uint32_t>(fmaf(2.5f, in_range ? rho : 0.0f, 12.0f));
-    ok_u = in_range && narrow_is_safe<T>(yu, kSwigluBwdUlps);
+    const std::uint32_t ulps_g = static_cast<std::uint32_t>(fmaf(SwigluBwdUlps<T>::kPerRho, in_range ? rho : 0.0f, SwigluBwdUlps<T>::kGate));
+    ok_u = in_range && narrow_is_safe<T>(yu, SwigluBwdUlps<T>::kAll);
     ok_g = in_range && narrow_is_safe<T>(yg, ulps_g);
     // exact signed zeros need no fp64 (zero padding stays on the fast tier)
     ok_u = ok_u || (yu == 0.0f && (dy == 0.0f || g == 0.0f));
