@@ -9,6 +9,8 @@
 // than a persistent grid-stride loop).
 #include <hip/hip_runtime.h>
 
+#include <type_traits>
+
 #include "core/device_context.h"
 #include "core/device_math.h"
 #include "core/status.h"
@@ -19,9 +21,10 @@ namespace {
 
 constexpr int kBlock  = 256;
 
-// One 16-byte vector of results.  16-bit types: every element through the fp32 tier, without a branch; the few whose value is next to a
+// One 16-byte vector of results.  fp16: every element through the fp32 tier, without a branch; the few whose value is next to a
 // rounding boundary (or outside the tier's range) are redone in fp64 in a loop that runs as often as the lane with the most of
-// them needs.  A wave of eight elements a lane then comes to the fp64 formula 0.3 (bf16) or 0.7 (fp16) times instead of 0.5 or 3.2.
+// them needs.  A wave of eight elements a lane then comes to the fp64 formula 0.7 times instead of 3.2.  bf16, where that is 0.3 for 0.5,
+// branches element by element: a forward and backward of 8192 x 14336 take 301 us with the loop, 297 without.
 template <typename T>
 __device__ __forceinline__ u32x4 swiglu_vec(u32x4 gv, u32x4 uv) {
     using E = Elem<T>;
@@ -30,7 +33,7 @@ __device__ __forceinline__ u32x4 swiglu_vec(u32x4 gv, u32x4 uv) {
     const S* ue = reinterpret_cast<const S*>(&uv);
     u32x4 o;
     S* oe = reinterpret_cast<S*>(&o);
-    if constexpr (sizeof(S) == 2) {
+    if constexpr (std::is_same_v<T, f16_t>) {
         unsigned redo = 0;
         S r[8];
 #pragma unroll
