@@ -998,7 +998,7 @@ size_t flash_workspace(const paras_sdpa_args& a) {
 }
 
 bool flash_uses_wide(const paras_sdpa_args& a) {
-    return flash::wide_supported(a.B, a.Hq, a.Lq, a.Lk, static_cast<int>(a.D), a.mask_kind, a.is_causal != 0);
+    return flash::wide_supported(a.B, a.Hq, a.Hkv, a.Lq, a.Lk, static_cast<int>(a.D), a.mask_kind, a.is_causal != 0);
 }
 
 int launch_flash(const paras_sdpa_args& a, Scratch scratch, hipStream_t s) {

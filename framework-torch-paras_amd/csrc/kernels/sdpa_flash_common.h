@@ -148,7 +148,7 @@ __device__ __forceinline__ void map_workgroup(int idx, int BH, int nq, int& bh, 
 
 // 64 queries per wavefront (sdpa_flash_wide.hip): head size 128, causal or unmasked.
 constexpr int kWideBM = 256;   // queries per workgroup of that kernel
-bool wide_supported(long B, long Hq, long Lq, long Lk, int D, int mask_kind, bool causal);
+bool wide_supported(long B, long Hq, long Hkv, long Lq, long Lk, int D, int mask_kind, bool causal);
 int  launch_flash_wide(FlashParams p, bool causal, bool is_bf16, hipStream_t s);
 
 }  // namespace flash

@@ -51,6 +51,7 @@
 #include "core/device_math.h"
 #include "core/status.h"
 #include "kernels/sdpa_flash_common.h"
+#include "kernels/sdpa_flash_deal.h"
 
 namespace paras {
 namespace flash {
@@ -122,7 +123,7 @@ __global__ __launch_bounds__(256, 1) void flash_wide_kernel(const FlashParams p)
     // by 8 the heads are dealt to the XCDs and the workgroups of an XCD share the K / V of few
     // heads at a time in its L2.  Within such a pool the items are numbered by groups of heads, longest
     // query tiles first under the causal rule, and dealt in rounds of one item per workgroup, every
-    // other round in reverse order, which evens out the triangle (tile i then tile n-1-i; head_group_of chooses the groups).
+    // other round in reverse order, which evens out the triangle (tile i then tile n-1-i; deal_of chooses the groups).
     const int nq = p.n_qblocks;
     const int BH = p.B * p.Hq;
     const int n_wg = static_cast<int>(gridDim.x), wg_id = static_cast<int>(blockIdx.x);
@@ -130,13 +131,13 @@ __global__ __launch_bounds__(256, 1) void flash_wide_kernel(const FlashParams p)
     const int pool_wgs = by_xcd ? n_wg >> 3 : n_wg;
     const int pool_pos = by_xcd ? wg_id >> 3 : wg_id;
     const int pool_items = (by_xcd ? BH >> 3 : BH) * nq;
-    // (x / d as a multiply-high by ceil(2^32 / d): exact while x * d < 2^32, which the launcher checks)
+    // (x / d as a multiply-high by ceil(2^32 / d): exact while x * d < 2^32, which wide_supported checks for bh / Hq; a group may be all the items)
     auto fast_div = [](int x, unsigned magic) { return static_cast<int>(__umulhi(static_cast<unsigned>(x), magic)); };
     auto item_at = [&](int round, int& bh, int& qblock) {
         const int i = round * pool_wgs + ((round & 1) ? pool_wgs - 1 - pool_pos : pool_pos);
         if (i >= pool_items) return false;
-        const int span = p.head_group * nq, group = span == 1 ? i : fast_div(i, p.magic_group), in = i - group * span;
-        const int pos = p.head_group == 1 ? in : fast_div(in, p.magic_heads), head = group * p.head_group + in - pos * p.head_group;
+        const int span = p.head_group * nq, group = quotient(i, span, p.magic_group), in = i - group * span;
+        const int pos = quotient(in, p.head_group, p.magic_heads), head = group * p.head_group + in - pos * p.head_group;
         bh = by_xcd ? head * 8 + (wg_id & 7) : head;
         qblock = kCausal ? nq - 1 - pos : pos;
         return true;
@@ -561,54 +562,14 @@ __global__ __launch_bounds__(256, 1) void flash_wide_kernel(const FlashParams p)
     }
 }
 
-// Heads whose query tiles are dealt out together, longest first, under the causal rule: the smallest group (its keys and values share the L2)
-// with which no workgroup has over 3 % more than its share of tiles, or else the one that comes nearest.  One head at a time is even where the
-// query tiles of whole heads fill the rounds; elsewhere a workgroup may come to long tiles every time (5 sequences of 6175, 8 heads: 25
-// query tiles for 32 workgroups, one of which had 1.4 times its share; 444 -> 369 us; 2 of 7777, 16 heads 681 -> 436; 7 of 5000, 4 heads 280 -> 183).
-struct Deal {
-    int    group = 1;
-    double even = 1.0;               // a workgroup's share of the work, of what the one with the most has
-};
-Deal deal_of(long BH, long nq, long blocks) {
-    Deal d;
-    const bool by_xcd = BH % 8 == 0 && blocks % 8 == 0;
-    const long heads = by_xcd ? BH / 8 : BH, wgs = by_xcd ? blocks / 8 : blocks, items = heads * nq;
-    constexpr long kWgs = 512;
-    if (wgs > kWgs || items > 1024) return d;         // (many rounds are even enough)
-    const double share = static_cast<double>(heads) * (nq * (nq + 1) / 2) / wgs;
-    long least = 0x7fffffffffffL;
-    for (long G = 1; G <= heads; ++G) {
-        if (heads % G != 0) continue;
-        long load[kWgs] = {};
-        long most = 0, w = 0, way = 1;
-        for (long i = 0, pos = 0, at = 0; i < items; ++i) {           // item i: nq - pos tiles' worth, of the group's head `at`
-            load[w] += nq - pos;
-            if (load[w] > most) most = load[w];
-            w += way;
-            if (w < 0 || w == wgs) {                                  // the next round, the other way
-                way = -way;
-                w += way;
-            }
-            if (++at == G) {
-                at = 0;
-                if (++pos == nq) pos = 0;
-            }
-        }
-        if (most < least) {
-            least = most;
-            d.group = static_cast<int>(G);
-        }
-        if (most <= 1.03 * share) break;
-    }
-    d.even = share / least;
-    return d;
-}
-
 // One workgroup per CU, or fewer, and a whole number per XCD where the heads are dealt to them
 long workgroups_for(long BH, long items, long cus) {
     const long blocks = items < cus ? items : cus;
     return blocks >= 8 && BH % 8 == 0 ? blocks - blocks % 8 : blocks;
 }
+
+// Keys and values per query head
+double head_bytes(long Hq, long Hkv, long Lk) { return static_cast<double>(Lk) * (2 * D * 2) * static_cast<double>(Hkv) / static_cast<double>(Hq); }
 
 template <typename T>
 int launch_t(FlashParams p, bool causal, hipStream_t s) {
@@ -622,9 +583,9 @@ int launch_t(FlashParams p, bool causal, hipStream_t s) {
     p.magic_hq = magic(p.Hq);
     p.magic_rep = magic(p.Hq / p.Hkv);
     const long BH = static_cast<long>(p.B) * p.Hq, blocks = workgroups_for(BH, items, cus);
-    p.head_group = causal ? deal_of(BH, p.n_qblocks, blocks).group : 1;
-    p.magic_group = magic(static_cast<long>(p.head_group) * p.n_qblocks);
-    p.magic_heads = magic(p.head_group);
+    p.head_group = causal ? deal_of(BH, p.n_qblocks, blocks, head_bytes(p.Hq, p.Hkv, p.Lk)).group : 1;
+    p.magic_group = magic_of(static_cast<long>(p.head_group) * p.n_qblocks);
+    p.magic_heads = magic_of(p.head_group);
     const dim3 grid(static_cast<unsigned>(blocks)), wg(256);
     if (causal) hipLaunchKernelGGL((flash_wide_kernel<T, true>), grid, wg, 0, s, p);
     else        hipLaunchKernelGGL((flash_wide_kernel<T, false>), grid, wg, 0, s, p);
@@ -634,10 +595,10 @@ int launch_t(FlashParams p, bool causal, hipStream_t s) {
 
 }  // namespace
 
-bool wide_supported(long B, long Hq, long Lq, long Lk, int head, int mask_kind, bool causal) {
+bool wide_supported(long B, long Hq, long Hkv, long Lq, long Lk, int head, int mask_kind, bool causal) {
     static const int forced = [] { const char* e = std::getenv("PARAS_FLASH_WIDE"); return e ? std::atoi(e) : -1; }();
     if (head != D || mask_kind != 0) return false;
-    // the item arithmetic divides by multiply-high: exact while dividend * divisor < 2^32
+    // (the item arithmetic divides by multiply-high: bh / Hq is exact while dividend * divisor < 2^32; no one has run more tiles than the other bound)
     const unsigned long long nq = (static_cast<unsigned long long>(Lq) + kWideBM - 1) / kWideBM;
     const unsigned long long bh = static_cast<unsigned long long>(B) * static_cast<unsigned long long>(Hq);
     if (bh * nq * nq >= (1ull << 32) || bh * static_cast<unsigned long long>(Hq) >= (1ull << 32)) return false;
@@ -647,19 +608,24 @@ bool wide_supported(long B, long Hq, long Lq, long Lk, int head, int mask_kind, 
     // round here takes 1.82 of those.  So wherever the last of that kernel's is a second one, and from two items to a CU on (2 to 5 % behind at worst)
     // (the other / this: B1 H8 S5524 135 / 119 us, W 352; B2 H8 S6249 341 / 300, W 784; B2 H8 S3992 127 / 120, W 512; B2 H8 S5432 237 / 260,
     // W 688; B1 H16 S1661 30 / 40, W 208; B6 H16 S4585 897 / 825).
-    //   Causal: 5 % ahead where its workgroups come out even and its query tiles of 256 pad no more than those of 128 (B4 H16 S4563 352 / 333;
-    // B13 H8 S2011 138 / 131; B5 H16 S1487 62 / 60; a ninth more of padded triangle: B9 H32 S2372 460 / 524; uneven, 0.78: B2 H8 S6079 153 / 156).
-    // Of the 110, the slower one is taken 6 times, by 0.5 to 6 % (with the limits of before, 4096 causal or 1024 unmasked queries and two query tiles of
-    // 256 per CU, 2.3 % in the mean over all, up to 15 %).
+    //   Causal: by the cost of the deal (deal_of; 1 is an even one) times how much more of the triangle query tiles of 256 pad than those of 128 do, where that is
+    // under 6 %.  How much it may be goes with the length (an item's fixed cost: cost 1.04, B10 H16 S1536 109 / 116 us, B5 H24 S2048 138 / 135; 1.07, B1 H40
+    // S4608 228 / 205), is more where the other kernel's tiles are few rounds and so come out ill themselves (1.08, B2 H32 S1536 51 / 49) and more where the heads
+    // are not dealt to XCDs, whose caches do not help that kernel then (1.05, B3 H28 S1792 82 / 86, B5 H28 S2048 186 / 173; 1.09, B7 H36 S2558 523 / 446).
+    // Over 172 problems of 1400 to 8200 queries 2.3 % less than with a deal taken to be even wherever there were over 1024 items, 7.5 % less than with one head at a
+    // time and limits of 4096 queries and two items to a CU; none over 3 % slower than either.
     const long least = causal ? 1400 : 896;
     if (Lq < least || Lk < least) return false;        // (before the runtime is asked: small calls are bound by the host)
     int dev = 0, cus = 0;
     if (hipGetDevice(&dev) != hipSuccess || hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, dev) != hipSuccess) return false;
     const long BH = static_cast<long>(bh), items = BH * static_cast<long>(nq), tiles = (Lq + 127) / 128;
     if (!causal) return (items >= 2 * cus && Lq >= 1024) || 1.82 * static_cast<double>((items + cus - 1) / cus) < static_cast<double>((BH * tiles + cus - 1) / cus);
-    const double rows = static_cast<double>(nq * kWideBM) / static_cast<double>(tiles * 128), padded = 0.94 * rows * rows;
-    if (items < cus || padded >= 1.0) return false;
-    return padded < deal_of(BH, static_cast<long>(nq), workgroups_for(BH, items, cus)).even + 0.1;
+    const double rows = static_cast<double>(nq * kWideBM) / static_cast<double>(tiles * 128), padding = rows * rows;
+    if (items < cus || padding >= 1.064) return false;
+    const long blocks = workgroups_for(BH, items, cus);
+    const double cost = padding * deal_of(BH, static_cast<long>(nq), blocks, head_bytes(Hq, Hkv, Lk)).cost, thousands = 1e-3 * static_cast<double>(Lq);
+    if (BH % 8 == 0 && blocks % 8 == 0) return cost < std::fmin(0.94 + 0.0475 * thousands, 1.07) + (items < 2 * cus ? 0.07 : items < 3 * cus && Lq >= 4096 ? 0.05 : 0.0);
+    return cost < std::fmin(0.93 + 0.065 * thousands, 1.13) + (items > 4 * cus ? 0.06 : 0.0);
 }
 
 int launch_flash_wide(FlashParams p, bool causal, bool is_bf16, hipStream_t s) {

@@ -971,6 +971,22 @@ def test_flash_wide_kernel_deals_every_query_tile(B, H, S):
             assert (out[b:b + 1, h:h + 4].float() - want.float()).abs().max().item() <= ABS_16BIT
 
 
+@pytest.mark.parametrize("B,H,Hkv,S", [(7, 12, 12, 3840), (15, 4, 4, 5120), (3, 28, 28, 1500), (5, 28, 4, 2048), (9, 36, 36, 1536), (7, 36, 36, 2558)])
+def test_flash_wide_kernel_deals_heads_that_belong_to_no_xcd(B, H, Hkv, S):
+    """The same with head counts that do not divide by 8, most of them with over 1024 items: dealt out over all heads at once, or one by one."""
+    g = torch.Generator(device="cuda").manual_seed(S)
+    q, k, v = (torch.randn(B, h, S, 128, generator=g, device="cuda", dtype=torch.bfloat16) for h in (H, Hkv, Hkv))
+    out, _, _, name = capi.sdpa(q, k, v, is_causal=True)
+    assert name == "flash_mfma_wide"
+    rep = H // Hkv
+    for b in range(B):
+        for h in range(0, Hkv, 2):
+            some = slice(h * rep, min(h + 2, Hkv) * rep)
+            want, _, _, other = capi.sdpa(q[b:b + 1, some].contiguous(), k[b:b + 1, h:h + 2].contiguous(), v[b:b + 1, h:h + 2].contiguous(), is_causal=True)
+            assert other != name
+            assert (out[b:b + 1, some].float() - want.float()).abs().max().item() <= ABS_16BIT
+
+
 @pytest.mark.parametrize("B,H,S,causal,wide", [(1, 8, 4200, False, True), (1, 8, 4096, False, False), (6, 16, 1024, False, False), (7, 16, 1024, False, True), (2, 32, 896, False, True),
                                                (2, 32, 895, False, False), (5, 16, 1500, True, True), (5, 16, 1408, True, False), (5, 16, 1399, True, False), (2, 8, 6079, True, False)])
 def test_flash_either_side_of_the_limits_of_the_wide_kernel(B, H, S, causal, wide):

@@ -1,5 +1,7 @@
 """What paras_sdpa_workspace and paras_sdpa_kernel_name answer (host code only: nothing is launched)."""
 import ctypes as C
+import random
+import subprocess
 
 import pytest
 import torch
@@ -22,3 +24,60 @@ def test_workspace_of_wide_types_does_not_depend_on_the_pointers(dtype, with_att
         a.attn = (base or 4096) if with_attn else None
         seen.add((capi.lib().paras_sdpa_kernel_name(C.byref(a)), capi.lib().paras_sdpa_workspace(C.byref(a))))
     assert len(seen) == 1, seen
+
+
+@pytest.fixture(scope="module")
+def deal(tmp_path_factory):
+    """sdpa_flash_deal.h as a library of its own (plain C++, no HIP)."""
+    where = tmp_path_factory.mktemp("deal")
+    (where / "deal.cpp").write_text('''#include "kernels/sdpa_flash_deal.h"
+using namespace paras::flash;
+extern "C" long by_runs(long heads, long nq, long wgs, long G) { return most_by_runs(heads, nq, wgs, G); }
+extern "C" long by_places(long heads, long nq, long wgs, long G) { return most_by_places(heads, nq, wgs, G); }
+extern "C" int group(long BH, long nq, long blocks, double bytes) { return deal_of(BH, nq, blocks, bytes).group; }
+extern "C" double cost(long BH, long nq, long blocks, double bytes) { return deal_of(BH, nq, blocks, bytes).cost; }
+''')
+    subprocess.run(["g++", "-O2", "-std=c++17", "-shared", "-fPIC", f"-I{capi.PKG / 'csrc'}", str(where / "deal.cpp"), "-o", str(where / "deal.so")], check=True)
+    lib = C.CDLL(str(where / "deal.so"))
+    for f in (lib.by_runs, lib.by_places):
+        f.restype, f.argtypes = C.c_long, [C.c_long] * 4
+    lib.group.restype, lib.cost.restype = C.c_int, C.c_double
+    lib.group.argtypes = lib.cost.argtypes = [C.c_long] * 3 + [C.c_double]
+    return lib
+
+
+def most_one_by_one(heads, nq, wgs, G):
+    """The kernel's numbering of items, item by item: what the workgroup with the most gets, in tiles of keys."""
+    load = [0] * wgs
+    for i in range(heads * nq):
+        turn, x = divmod(i, wgs)
+        load[wgs - 1 - x if turn % 2 else x] += nq - i % (G * nq) // G
+    return max(load)
+
+
+def test_the_most_a_workgroup_gets_is_what_dealing_item_by_item_gives(deal):
+    rng = random.Random(5)
+    cases = [(1, 1, 1, 1), (8, 6, 32, 8), (252, 10, 256, 1), (7, 33, 32, 7), (3, 2, 300, 1), (64, 16, 256, 64), (5, 25, 32, 5)]
+    for n in range(400):
+        G = rng.randint(1, 12)
+        cases.append((G * rng.randint(1, 20), rng.randint(1, 40), rng.randint(1, 40 if n % 2 else 300), G))
+    for c in cases:
+        want = most_one_by_one(*c)
+        assert deal.by_runs(*c) == want and deal.by_places(*c) == want, c
+
+
+@pytest.mark.parametrize("B,H,S", [(3, 36, 2560), (9, 12, 2560), (3, 28, 3584), (15, 4, 5120), (5, 28, 2048), (9, 4, 8192), (1, 36, 8192), (7, 12, 3840), (5, 14, 3840), (13, 12, 1792),
+                                   (3, 28, 1500), (3, 28, 4096), (5, 8, 6175), (6, 8, 5376), (4, 32, 4096)])
+def test_causal_query_tiles_are_dealt_evenly(deal, B, H, S):
+    """No workgroup has over a tenth more than its share (one head at a time it is 1.3 to 2 times for most of these), whether the heads are dealt to the
+    XCDs or not and however many items there are; and the cost that is reported is that of the deal."""
+    nq, BH = -(-S // 256), B * H
+    blocks = min(256, BH * nq)
+    blocks -= blocks % 8 if BH % 8 == 0 else 0
+    heads, wgs = (BH // 8, blocks // 8) if BH % 8 == 0 else (BH, blocks)
+    G = deal.group(BH, nq, blocks, 512.0 * S)
+    assert heads % G == 0
+    uneven = most_one_by_one(heads, nq, wgs, G) / (heads * nq * (nq + 1) / 2 / wgs)
+    assert uneven <= 1.1, (G, uneven)
+    fits = G * S * 512 * (8 if BH % 8 == 0 else 1) <= 128e6
+    assert deal.cost(BH, nq, blocks, 512.0 * S) >= 0.45 + 0.55 * uneven - 1e-9 and (not fits or deal.cost(BH, nq, blocks, 512.0 * S) <= 0.45 + 0.55 * uneven + 1e-9)
