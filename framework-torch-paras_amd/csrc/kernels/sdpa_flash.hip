@@ -997,9 +997,11 @@ size_t flash_workspace(const paras_sdpa_args& a) {
     return slots * (kBM * a.D + 2 * kBM) * sizeof(float);
 }
 
-bool flash_uses_wide(const paras_sdpa_args& a) {
-    return flash::wide_supported(a.B, a.Hq, a.Hkv, a.Lq, a.Lk, static_cast<int>(a.D), a.mask_kind, a.is_causal != 0);
+static int wide_group_of(const paras_sdpa_args& a) {
+    return flash::wide_group(a.B, a.Hq, a.Hkv, a.Lq, a.Lk, static_cast<int>(a.D), a.mask_kind, a.is_causal != 0);
 }
+
+bool flash_uses_wide(const paras_sdpa_args& a) { return wide_group_of(a) != 0; }
 
 int launch_flash(const paras_sdpa_args& a, Scratch scratch, hipStream_t s) {
     FlashParams p{};
@@ -1032,7 +1034,7 @@ int launch_flash(const paras_sdpa_args& a, Scratch scratch, hipStream_t s) {
         p.part_o = static_cast<float*>(scratch.p);
         p.part_ml = p.part_o + static_cast<size_t>(a.B * a.Hq) * ((a.Lq + kBM - 1) / kBM) * r.parts * kBM * a.D;
     }
-    if (flash_uses_wide(a)) return launch_flash_wide(p, causal, a.dtype == PARAS_BF16, s);
+    if (const int group = wide_group_of(a); group != 0) return launch_flash_wide(p, group, causal, a.dtype == PARAS_BF16, s);
     if (a.dtype == PARAS_BF16)
         return a.D == 256 ? launch_t<bf16_t, 256>(p, causal, mk, r.halves, s) : a.D == 128 ? launch_t<bf16_t, 128>(p, causal, mk, r.halves, s) : launch_t<bf16_t, 64>(p, causal, mk, r.halves, s);
     return a.D == 256 ? launch_t<f16_t, 256>(p, causal, mk, r.halves, s) : a.D == 128 ? launch_t<f16_t, 128>(p, causal, mk, r.halves, s) : launch_t<f16_t, 64>(p, causal, mk, r.halves, s);

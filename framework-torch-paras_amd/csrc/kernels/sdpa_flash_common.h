@@ -148,8 +148,10 @@ __device__ __forceinline__ void map_workgroup(int idx, int BH, int nq, int& bh, 
 
 // 64 queries per wavefront (sdpa_flash_wide.hip): head size 128, causal or unmasked.
 constexpr int kWideBM = 256;   // queries per workgroup of that kernel
-bool wide_supported(long B, long Hq, long Hkv, long Lq, long Lk, int D, int mask_kind, bool causal);
-int  launch_flash_wide(FlashParams p, bool causal, bool is_bf16, hipStream_t s);
+// The heads whose query tiles it deals out together (causal; 1 otherwise), or 0 where the problem is not for it.  Asked once per launch: the deal is worked
+// out on the way to either answer.
+int wide_group(long B, long Hq, long Hkv, long Lq, long Lk, int D, int mask_kind, bool causal);
+int launch_flash_wide(FlashParams p, int group, bool causal, bool is_bf16, hipStream_t s);
 
 }  // namespace flash
 }  // namespace paras

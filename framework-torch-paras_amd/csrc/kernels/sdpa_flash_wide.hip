@@ -131,7 +131,7 @@ __global__ __launch_bounds__(256, 1) void flash_wide_kernel(const FlashParams p)
     const int pool_wgs = by_xcd ? n_wg >> 3 : n_wg;
     const int pool_pos = by_xcd ? wg_id >> 3 : wg_id;
     const int pool_items = (by_xcd ? BH >> 3 : BH) * nq;
-    // (x / d as a multiply-high by ceil(2^32 / d): exact while x * d < 2^32, which wide_supported checks for bh / Hq; a group may be all the items)
+    // (x / d as a multiply-high by ceil(2^32 / d): exact while x * d < 2^32, which wide_group checks for bh / Hq; a group may be all the items)
     auto fast_div = [](int x, unsigned magic) { return static_cast<int>(__umulhi(static_cast<unsigned>(x), magic)); };
     auto item_at = [&](int round, int& bh, int& qblock) {
         const int i = round * pool_wgs + ((round & 1) ? pool_wgs - 1 - pool_pos : pool_pos);
@@ -572,7 +572,7 @@ long workgroups_for(long BH, long items, long cus) {
 double head_bytes(long Hq, long Hkv, long Lk) { return static_cast<double>(Lk) * (2 * D * 2) * static_cast<double>(Hkv) / static_cast<double>(Hq); }
 
 template <typename T>
-int launch_t(FlashParams p, bool causal, hipStream_t s) {
+int launch_t(FlashParams p, int group, bool causal, hipStream_t s) {
     p.n_qblocks = (p.Lq + kWideBM - 1) / kWideBM;
     const long items = static_cast<long>(p.B) * p.Hq * p.n_qblocks;
     // one workgroup per CU (that is all its LDS and registers hold), each walking its share of the items
@@ -583,7 +583,7 @@ int launch_t(FlashParams p, bool causal, hipStream_t s) {
     p.magic_hq = magic(p.Hq);
     p.magic_rep = magic(p.Hq / p.Hkv);
     const long BH = static_cast<long>(p.B) * p.Hq, blocks = workgroups_for(BH, items, cus);
-    p.head_group = causal ? deal_of(BH, p.n_qblocks, blocks, head_bytes(p.Hq, p.Hkv, p.Lk)).group : 1;
+    p.head_group = group;
     p.magic_group = magic_of(static_cast<long>(p.head_group) * p.n_qblocks);
     p.magic_heads = magic_of(p.head_group);
     const dim3 grid(static_cast<unsigned>(blocks)), wg(256);
@@ -595,14 +595,13 @@ int launch_t(FlashParams p, bool causal, hipStream_t s) {
 
 }  // namespace
 
-bool wide_supported(long B, long Hq, long Hkv, long Lq, long Lk, int head, int mask_kind, bool causal) {
+int wide_group(long B, long Hq, long Hkv, long Lq, long Lk, int head, int mask_kind, bool causal) {
     static const int forced = [] { const char* e = std::getenv("PARAS_FLASH_WIDE"); return e ? std::atoi(e) : -1; }();
-    if (head != D || mask_kind != 0) return false;
+    if (head != D || mask_kind != 0 || forced == 0) return 0;
     // (the item arithmetic divides by multiply-high: bh / Hq is exact while dividend * divisor < 2^32; no one has run more tiles than the other bound)
     const unsigned long long nq = (static_cast<unsigned long long>(Lq) + kWideBM - 1) / kWideBM;
     const unsigned long long bh = static_cast<unsigned long long>(B) * static_cast<unsigned long long>(Hq);
-    if (bh * nq * nq >= (1ull << 32) || bh * static_cast<unsigned long long>(Hq) >= (1ull << 32)) return false;
-    if (forced >= 0) return forced != 0;
+    if (bh * nq * nq >= (1ull << 32) || bh * static_cast<unsigned long long>(Hq) >= (1ull << 32)) return 0;
     // Against the kernel of 32 queries per wavefront (W query tiles of 128, two to a CU), measured for 110 problems of 900 to 8000 queries:
     //   Unmasked: both come in rounds, this one of a CU's 256 queries, that one of 128 for the first of a CU and again for the second, and a
     // round here takes 1.82 of those.  So wherever the last of that kernel's is a second one, and from two items to a CU on (2 to 5 % behind at worst)
@@ -613,23 +612,25 @@ bool wide_supported(long B, long Hq, long Hkv, long Lq, long Lk, int head, int m
     // S4608 228 / 205), is more where the other kernel's tiles are few rounds and so come out ill themselves (1.08, B2 H32 S1536 51 / 49) and more where the heads
     // are not dealt to XCDs, whose caches do not help that kernel then (1.05, B3 H28 S1792 82 / 86, B5 H28 S2048 186 / 173; 1.09, B7 H36 S2558 523 / 446).
     // Over 172 problems of 1400 to 8200 queries 2.3 % less than with a deal taken to be even wherever there were over 1024 items, 7.5 % less than with one head at a
-    // time and limits of 4096 queries and two items to a CU; none over 3 % slower than either.
+    // time and limits of 4096 queries and two items to a CU; none over 1 % slower than either in repeated runs.
     const long least = causal ? 1400 : 896;
-    if (Lq < least || Lk < least) return false;        // (before the runtime is asked: small calls are bound by the host)
+    if (forced < 0 && (Lq < least || Lk < least)) return 0;        // (before the runtime is asked: small calls are bound by the host)
     int dev = 0, cus = 0;
-    if (hipGetDevice(&dev) != hipSuccess || hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, dev) != hipSuccess) return false;
+    if (hipGetDevice(&dev) != hipSuccess || hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, dev) != hipSuccess) return 0;
     const long BH = static_cast<long>(bh), items = BH * static_cast<long>(nq), tiles = (Lq + 127) / 128;
-    if (!causal) return (items >= 2 * cus && Lq >= 1024) || 1.82 * static_cast<double>((items + cus - 1) / cus) < static_cast<double>((BH * tiles + cus - 1) / cus);
+    if (!causal) return forced > 0 || (items >= 2 * cus && Lq >= 1024) || 1.82 * static_cast<double>((items + cus - 1) / cus) < static_cast<double>((BH * tiles + cus - 1) / cus);
     const double rows = static_cast<double>(nq * kWideBM) / static_cast<double>(tiles * 128), padding = rows * rows;
-    if (items < cus || padding >= 1.064) return false;
+    if (forced < 0 && (items < cus || padding >= 1.064)) return 0;
     const long blocks = workgroups_for(BH, items, cus);
-    const double cost = padding * deal_of(BH, static_cast<long>(nq), blocks, head_bytes(Hq, Hkv, Lk)).cost, thousands = 1e-3 * static_cast<double>(Lq);
-    if (BH % 8 == 0 && blocks % 8 == 0) return cost < std::fmin(0.94 + 0.0475 * thousands, 1.07) + (items < 2 * cus ? 0.07 : items < 3 * cus && Lq >= 4096 ? 0.05 : 0.0);
-    return cost < std::fmin(0.93 + 0.065 * thousands, 1.13) + (items > 4 * cus ? 0.06 : 0.0);
+    const Deal deal = deal_of(BH, static_cast<long>(nq), blocks, head_bytes(Hq, Hkv, Lk));
+    const double cost = padding * deal.cost, thousands = 1e-3 * static_cast<double>(Lq);
+    const double most = BH % 8 == 0 && blocks % 8 == 0 ? std::fmin(0.94 + 0.0475 * thousands, 1.07) + (items < 2 * cus ? 0.07 : items < 3 * cus && Lq >= 4096 ? 0.05 : 0.0)
+                                                       : std::fmin(0.93 + 0.065 * thousands, 1.13) + (items > 4 * cus ? 0.06 : 0.0);
+    return forced > 0 || cost < most ? deal.group : 0;
 }
 
-int launch_flash_wide(FlashParams p, bool causal, bool is_bf16, hipStream_t s) {
-    return is_bf16 ? launch_t<bf16_t>(p, causal, s) : launch_t<f16_t>(p, causal, s);
+int launch_flash_wide(FlashParams p, int group, bool causal, bool is_bf16, hipStream_t s) {
+    return is_bf16 ? launch_t<bf16_t>(p, group, causal, s) : launch_t<f16_t>(p, group, causal, s);
 }
 
 }  // namespace flash

@@ -31,9 +31,16 @@ def deal(tmp_path_factory):
     """sdpa_flash_deal.h as a library of its own (plain C++, no HIP)."""
     where = tmp_path_factory.mktemp("deal")
     (where / "deal.cpp").write_text('''#include "kernels/sdpa_flash_deal.h"
+#include <chrono>
 using namespace paras::flash;
 extern "C" long by_runs(long heads, long nq, long wgs, long G) { return most_by_runs(heads, nq, wgs, G); }
 extern "C" long by_places(long heads, long nq, long wgs, long G) { return most_by_places(heads, nq, wgs, G); }
+extern "C" double seconds(long BH, long nq, long blocks, double bytes, int times) {
+    const auto start = std::chrono::steady_clock::now();
+    volatile double sink = 0;
+    for (int i = 0; i < times; ++i) sink = sink + deal_of(BH, nq, blocks, bytes).cost;
+    return std::chrono::duration<double>(std::chrono::steady_clock::now() - start).count();
+}
 extern "C" int group(long BH, long nq, long blocks, double bytes) { return deal_of(BH, nq, blocks, bytes).group; }
 extern "C" double cost(long BH, long nq, long blocks, double bytes) { return deal_of(BH, nq, blocks, bytes).cost; }
 ''')
@@ -41,6 +48,7 @@ extern "C" double cost(long BH, long nq, long blocks, double bytes) { return dea
     lib = C.CDLL(str(where / "deal.so"))
     for f in (lib.by_runs, lib.by_places):
         f.restype, f.argtypes = C.c_long, [C.c_long] * 4
+    lib.seconds.restype, lib.seconds.argtypes = C.c_double, [C.c_long] * 3 + [C.c_double, C.c_int]
     lib.group.restype, lib.cost.restype = C.c_int, C.c_double
     lib.group.argtypes = lib.cost.argtypes = [C.c_long] * 3 + [C.c_double]
     return lib
@@ -81,3 +89,11 @@ def test_causal_query_tiles_are_dealt_evenly(deal, B, H, S):
     assert uneven <= 1.1, (G, uneven)
     fits = G * S * 512 * (8 if BH % 8 == 0 else 1) <= 128e6
     assert deal.cost(BH, nq, blocks, 512.0 * S) >= 0.45 + 0.55 * uneven - 1e-9 and (not fits or deal.cost(BH, nq, blocks, 512.0 * S) <= 0.45 + 0.55 * uneven + 1e-9)
+
+
+@pytest.mark.parametrize("B,H,S", [(3, 28, 1500), (7, 12, 1500), (5, 28, 1500), (5, 12, 2048), (1, 36, 4096), (15, 4, 1500), (5, 16, 1500), (4, 32, 4096), (1, 97, 8192)])
+def test_a_deal_is_worked_out_in_a_microsecond(deal, B, H, S):
+    """0.2 to 1.2 us, once per call; a walk over every item of every group took 10 to 60, twice."""
+    nq, BH = -(-S // 256), B * H
+    blocks = min(256, BH * nq) // 8 * 8 if BH % 8 == 0 else min(256, BH * nq)
+    assert min(deal.seconds(BH, nq, blocks, 512.0 * S, 100) for _ in range(200)) / 100 <= 4e-6
