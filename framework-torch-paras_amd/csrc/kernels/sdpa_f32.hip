@@ -6,8 +6,7 @@
 // D128: 254 us), and large ones as two batched products around a row kernel with the scores in memory (B1 H2
 // S3737 D128: 740 us, of which 508 us one product with 60 workgroups).
 //
-// A workgroup takes 16 QB queries of one head; its four waves take the keys in turns of 32 (16 where
-// there are few keys or the registers are full) and meet at the end (row maximum, row sum, output: combined through LDS).  Per turn and wave:
+// A workgroup takes 16 QB queries of one head; its four waves take the keys in turns of 16 or 32 (form_of) and meet at the end (row maximum, row sum, output: combined through LDS).  Per turn and wave:
 //   S^T = K Q^T      v_mfma 16x16x4, A = 16 keys, B = 16 queries
 //   online softmax   a lane holds one query and 4 keys of each 16 x 16 block
 //   O^T += V^T P^T   the accumulator layout of S^T is the B operand layout of this product: step t takes
@@ -32,7 +31,7 @@
 // large ones the matrix cores and the vector instructions, which do not run beside fp32 MFMAs here (weights of one query
 // block interleaved with the products of the other, one MFMA to seven vector instructions: 874 -> 903 us).  B2 H16 S2048
 // D128: unmasked 696-705 us = 98 TFLOP/s, causal 512-520 (every value is read, seen or not: 25 of them), 30 % padding 731, an additive
-// mask 834; the batched products took 967 / 907 / 1520 / 1590.  B2 H8 S1024 D64 57 us (174), B1 H4 S2048 D256 206 (317).  (With blocks of 32 queries
+// mask 831; the batched products took 967 / 907 / 1520 / 1590.  B2 H8 S1024 D64 55 us (174), B1 H4 S2048 D256 203 (317).  (With blocks of 32 queries
 // at 64 and 128 elements, turns of 32 keys and the softmax in fp64 742 / 623 / 775 / 830, 55 and 203.)  With those and the
 // softmax in fp32 it took 697 / 567 / 665 / 950, 47 and 228, and single weights were 4.9e-7 off instead of 1.1e-7.
 #include <hip/hip_runtime.h>
@@ -159,11 +158,23 @@ __global__ __launch_bounds__(kWavesF * 64, DM == 64 || (DM == 128 && KB == 1 && 
     const int keys = p.is_causal ? min(p.Lk, q0 + 16 * QB) : p.Lk;
     // more than 128 elements leave no registers for operands ahead of time: they are requested where they are used
     constexpr bool kAhead = DM <= 128;
+    // (where a mask takes what registers these leave, places in the mask and the weights are worked out where they are used instead of being held)
+    constexpr bool kTight = sizeof(Acc) == 4 && DM == 128 && QB == 2 && KB == 1 && kMask != 0;
     // The scores of a block for softmax_rows_kernel below: a lane holds 4 adjacent keys of one query.
     auto keep_scores = [&](int qb, int j, const float (&x)[4]) {
-        const int i = q0 + 16 * qb + l16;
-        if (i >= p.Lq || j >= p.Lk) return;
-        float* at = p.attn + ((static_cast<long>(b) * p.Hq + h) * p.Lq + i) * p.Lk + j;
+        float* at;
+        if constexpr (kTight) {
+            // (bytes in 32 bits past the tile's first row: there are 64 queries and 2^31 weights to a head, at least and at most)
+            int query = 16 * qb + l16;
+            asm volatile("" : "+v"(query));
+            if (q0 + query >= p.Lq || j >= p.Lk) return;
+            float* const tile = p.attn + ((static_cast<long>(b) * p.Hq + h) * p.Lq + q0) * p.Lk;
+            at = reinterpret_cast<float*>(reinterpret_cast<char*>(tile) + (static_cast<std::uint32_t>(query) * static_cast<std::uint32_t>(p.Lk) + static_cast<std::uint32_t>(j)) * 4u);
+        } else {
+            const int i = q0 + 16 * qb + l16;
+            if (i >= p.Lq || j >= p.Lk) return;
+            at = p.attn + ((static_cast<long>(b) * p.Hq + h) * p.Lq + i) * p.Lk + j;
+        }
         if (p.attn16) {
             *reinterpret_cast<float4_t*>(at) = float4_t{x[0], x[1], x[2], x[3]};
         } else {
@@ -195,18 +206,39 @@ __global__ __launch_bounds__(kWavesF * 64, DM == 64 || (DM == 128 && KB == 1 && 
         const long row = static_cast<long>(min(q0 + 16 * qb + l16, p.Lq - 1)), col = static_cast<long>(min(j0 + 16 * kb + M::row(g, r), p.Lk - 1));
         return b * p.ms[0] + h * p.ms[1] + row * p.ms[2] + col * p.ms[3];
     };
+    // The same for all of a turn, element(qb, kb, r, place).
+    auto each_mask_place = [&](int j0, auto&& element) {
+        if constexpr (kTight) {
+            int key = j0 + M::row(g, 0);
+            asm volatile("" : "+v"(key));
+            long col[4];
+#pragma unroll
+            for (int r = 0; r < 4; ++r) col[r] = static_cast<long>(min(key + r, p.Lk - 1)) * p.ms[3];
+#pragma unroll
+            for (int qb = 0; qb < QB; ++qb) {
+                int query = q0 + 16 * qb + l16;
+                asm volatile("" : "+v"(query));
+                const long row = b * p.ms[0] + h * p.ms[1] + static_cast<long>(min(query, p.Lq - 1)) * p.ms[2];
+#pragma unroll
+                for (int r = 0; r < 4; ++r) element(qb, 0, r, row + col[r]);
+            }
+        } else {
+#pragma unroll
+            for (int qb = 0; qb < QB; ++qb)
+#pragma unroll
+                for (int kb = 0; kb < KB; ++kb)
+#pragma unroll
+                    for (int r = 0; r < 4; ++r) element(qb, kb, r, mask_at(j0, qb, kb, r));
+        }
+    };
     // A boolean mask's part of a turn, bit 4 kb + r; false: the turn is closed to every query of the tile.
     auto open_bits = [&](int j0, unsigned (&open)[QB]) {
         unsigned any = 0;
 #pragma unroll
-        for (int qb = 0; qb < QB; ++qb) {
-            open[qb] = 0;
+        for (int qb = 0; qb < QB; ++qb) open[qb] = 0;
+        each_mask_place(j0, [&](int qb, int kb, int r, long place) { open[qb] |= static_cast<const unsigned char*>(p.mask)[place] != 0 ? 1u << (4 * kb + r) : 0u; });
 #pragma unroll
-            for (int kb = 0; kb < KB; ++kb)
-#pragma unroll
-                for (int r = 0; r < 4; ++r) open[qb] |= static_cast<const unsigned char*>(p.mask)[mask_at(j0, qb, kb, r)] != 0 ? 1u << (4 * kb + r) : 0u;
-            any |= open[qb];
-        }
+        for (int qb = 0; qb < QB; ++qb) any |= open[qb];
         return __builtin_amdgcn_ballot_w64(any != 0) != 0;
     };
     // The first turn from j0 on that this wave has scores to form for.  One that a boolean mask closes needs none (an
@@ -232,13 +264,7 @@ __global__ __launch_bounds__(kWavesF * 64, DM == 64 || (DM == 128 && KB == 1 && 
     if (kAhead && j0 < keys) load_k(j0);
     while (j0 < keys) {
         float mk[QB][KB][4];
-        if constexpr (kMask == 2)
-#pragma unroll
-            for (int qb = 0; qb < QB; ++qb)
-#pragma unroll
-                for (int kb = 0; kb < KB; ++kb)
-#pragma unroll
-                    for (int r = 0; r < 4; ++r) mk[qb][kb][r] = static_cast<const float*>(p.mask)[mask_at(j0, qb, kb, r)];
+        if constexpr (kMask == 2) each_mask_place(j0, [&](int qb, int kb, int r, long place) { mk[qb][kb][r] = static_cast<const float*>(p.mask)[place]; });
         if constexpr (kAhead) {
             load_v(j0);
         } else {
@@ -416,7 +442,7 @@ __global__ __launch_bounds__(kWavesF * 64, DM == 64 || (DM == 128 && KB == 1 && 
 // The returned weights, in place of the scores that sdpa_f32_kernel left: exp(score - reference) / sum in fp64, rounded
 // once; zeros for the keys that the causal rule hides (NaN where the row is).  A wave takes a row in pieces of W elements.
 // Bound by memory (one read and one write of the weights tensor); four pieces are on the way at a time.  B2 H16 S2048 D128 with
-// its 537 MB of weights 988 us, causal 719; the product, row kernel and product in their place 967 and 907; B2 H8 S1024 D64 89 (174).
+// its 537 MB of weights 925 us, causal 714; the product, row kernel and product in their place 967 and 907; B2 H8 S1024 D64 88 (174).
 template <int W>
 __global__ __launch_bounds__(256) void softmax_rows_kernel(float* __restrict__ attn, const double2* __restrict__ row_sums, long rows, int Lq, int Lk, int is_causal) {
     typedef float piece __attribute__((ext_vector_type(W)));
@@ -451,13 +477,65 @@ __global__ __launch_bounds__(256) void softmax_rows_kernel(float* __restrict__ a
     }
 }
 
-template <typename Acc, int DM, int QB, int KB>
-void launch_form(F32Params p, const paras_sdpa_args& a, hipStream_t s) {
+template <typename Acc, int DM, int QB, int KB, int kMask>
+void launch_masked(F32Params p, const paras_sdpa_args& a, hipStream_t s) {
     p.q_tiles = static_cast<int>((a.Lq + 16 * QB - 1) / (16 * QB));
     const dim3 g(p.q_tiles, static_cast<unsigned>(a.Hq), static_cast<unsigned>(a.B)), t(kWavesF * 64);
-    if (a.mask_kind == 0)      hipLaunchKernelGGL((sdpa_f32_kernel<Acc, DM, QB, KB, 0>), g, t, 0, s, p);
-    else if (a.mask_kind == 1) hipLaunchKernelGGL((sdpa_f32_kernel<Acc, DM, QB, KB, 1>), g, t, 0, s, p);
-    else                       hipLaunchKernelGGL((sdpa_f32_kernel<Acc, DM, QB, KB, 2>), g, t, 0, s, p);
+    hipLaunchKernelGGL((sdpa_f32_kernel<Acc, DM, QB, KB, kMask>), g, t, 0, s, p);
+}
+template <typename Acc, int DM, int QB, int KB>
+void launch_form(const F32Params& p, const paras_sdpa_args& a, hipStream_t s) {
+    if (a.mask_kind == 0)      launch_masked<Acc, DM, QB, KB, 0>(p, a, s);
+    else if (a.mask_kind == 1) launch_masked<Acc, DM, QB, KB, 1>(p, a, s);
+    else                       launch_masked<Acc, DM, QB, KB, 2>(p, a, s);
+}
+
+// Queries by keys of a turn in the fp32 form.  Turns of 16 keys for 16 queries take the fewest registers, and what they leave room for, two workgroups per CU at 128
+// elements and four at 64, is worth more than the operands that larger blocks share, but not everywhere.  The figures are us of 16 x 16 / 16 x 32 / 32 x 32 keys, from 90
+// problems, each without a mask, causal, with 30 % of the keys padded and with an additive mask, with the weights returned and without.
+//   Whether weights are returned changes the queries of a block at most, and not the keys of a turn, so the output is the same bits either way.
+enum class Form { k16x16, k32x16, k16x32, k32x32 };
+template <int DM>
+Form form_of(const paras_sdpa_args& a) {
+    const long heads = a.B * a.Hq, blocks = (a.Lq + 15) / 16 * heads, pairs = (a.Lq + 31) / 32 * heads;
+    const bool causal = a.is_causal != 0, padded = a.mask_kind == 1, added = a.mask_kind == 2;
+    const double scores = static_cast<double>(heads) * static_cast<double>(a.Lq) * static_cast<double>(a.Lk);
+    if (DM == 64) {
+        // Four workgroups of 16 x 16 per CU are ahead up to a few turns each; beyond, turns of 32 keys wait for half as many row maxima (B1 H4 S4000 causal 192 /
+        // 150 / 184, B1 H1 S3000 49 / 47 / 81).  Blocks of 32 queries, two per CU, where they come in whole rounds: unmasked B2 H16 S2048 397 / 398 / 382; with an
+        // additive mask, B2 H16 S2048 519 / 531 / 449, B1 H8 S2048 (one round) 137 / 137 / 125, B1 H64 S600 106 / 111 / 100; between whole rounds B1 H16
+        // S1500 134 / 141 / 135, B2 H16 S600 57 / 59 / 64.
+        if (a.Lk <= 320) return Form::k16x16;
+        if (added && (pairs >= 1000 || (pairs >= 448 && pairs <= 512 && a.Lk >= 1000))) return Form::k32x32;
+        if (added && pairs > 512 && a.Lk <= 2000) return Form::k16x16;
+        if (!padded && !added && !causal && pairs >= 448) return Form::k32x32;
+        if (causal && pairs >= 448 && a.Lk <= 640) return Form::k16x16;              // (B8 H16 S512 109 / 113 / 109)
+        return Form::k16x32;
+    }
+    if (DM == 128) {
+        // Two workgroups of 16 x 16 per CU: B2 H16 S2048 695 / 833 / 746, B1 H64 S300 46 / 70 / 73, B3 H8 S145 causal 10 / 12 / 21.  One per CU and larger turns
+        // where there is no second one for most CUs: masks, B1 H1 S3000 padded 85 / 82 / 136, additive 95 / 84 / 162; causal, where the second ones are the
+        // longest tiles of the next head, on the CUs that have the longest of the first: B1 H2 S3000 112 / 80 / 134, B1 H3 S2000 88 / 72 / 93, B2 H2 S1100
+        // 39 / 33 / 56 (but B1 H3 S2500, 471 blocks, 97 / 105 / 115; B1 H5 S1200 49 / 52 / 61).  Causal S8192: B1 H2 489 / 481 / 433, B1 H4 883 / 960 / 864, B1 H8 1706 /
+        // 1909 / 1734.
+        if ((padded || added) && blocks <= 256 && a.Lk >= (added ? 900 : 1200)) return Form::k16x32;
+        if (causal && blocks > 256 && (blocks <= 300 || (blocks <= 448 && heads <= 3)) && a.Lk >= 900) return Form::k16x32;
+        if (causal && a.Lk >= 8192 && a.Lk % 1024 == 0 && blocks <= 2048) return Form::k32x32;
+        // 32 queries by 16 keys read K and V half as often, in the registers of two workgroups per CU still.  Where more weights are written than the last-level cache holds
+        // (16 x 16 / 32 x 16 / 32 x 32: B2 H16 S2048 unmasked 990 / 925 / 981, padded 1051 / 950 / 1021, additive 1103 / 998 / 1067; B1 H8 S4096 995 / 926 / 961, 1064 /
+        // 960 / 993, 1111 / 999 / 1042; but B1 H7 S4000, 875 pairs, 815 / 855: over one to a CU and not two in the last round), and for long rows of an additive
+        // mask (B1 H8 S4096 818 / 730 / 793, B1 H2 S8192 831 / 731 / 806).
+        const bool ragged = pairs < 1536 && pairs % 512 > 256 && pairs % 512 < 448;
+        if (a.attn != nullptr && !causal && scores >= 96e6 && !ragged) return Form::k32x16;
+        if (added && a.Lk >= 4096) return Form::k32x16;
+        return Form::k16x16;
+    }
+    // 256 elements, one workgroup per CU: 16 x 16 leaves the registers for what is requested ahead, 16 x 32 waits for half as many row maxima, which counts over
+    // many turns, and reads and writes rows of weights in longer pieces: B2 H16 S600 179 / 188, S2048 1629 / 1609, with the weights 2010 / 1838, B4 H16 S2048
+    // 3463 / 3215, B1 H1 S5000 484 / 463; B1 H32 S1500 931 / 931, with the weights 1119 / 1055.  Up to 80 keys one wave would take a second turn of 16 for the
+    // last of them (B9 H16 S66 37 / 35, additive 39 / 36; a mask or the causal rule may close that one: 35 / 38 padded).
+    if (a.Lk >= (causal ? 4000 : 2000) || (!causal && scores >= 64e6) || (a.Lk > 64 && a.Lk <= 80 && !causal && !padded)) return Form::k16x32;
+    return Form::k16x16;
 }
 template <typename Acc, int DM>
 void launch_dm(const F32Params& p, const paras_sdpa_args& a, hipStream_t s) {
@@ -468,19 +546,15 @@ void launch_dm(const F32Params& p, const paras_sdpa_args& a, hipStream_t s) {
         }
         launch_form<Acc, DM, 1, 1>(p, a, s);
     } else {
-        // Turns of 16 keys for 16 queries take the fewest registers, and what they leave room for, two workgroups per CU at 128 elements and
-        // four at 64, is worth more than the operands that larger blocks share (us, 16 queries x 16 keys / 16 x 32 / 32 x 32: D128 B3 H8 S145 causal
-        // 10.5 / 12.5 / 21.1, B1 H64 S300 46.7 / 69.6 / 72.8, B2 H16 S2048 696 / 831 / 742; D64 B9 H16 S66 9.1 / 11.0 / 13.3, B1 H64 S300
-        // 27.8 / 30.8 / 34.4; D256 B2 H16 S600 140 / 152).  With 64 elements and more keys than a few turns each the larger turns are ahead, for
-        // they wait for half as many row maxima (B1 H4 S4000 causal 196 / 153 / 188, B1 H1 S3000 51 / 47 / 83), and, without mask or causal rule, blocks
-        // of 32 queries where they fill the chip (B2 H16 S2048 400 / 400 / 385).
-        if constexpr (DM == 64) {
-            if (a.Lk > 320) {
-                if (a.mask_kind == 0 && !a.is_causal && (a.Lq + 31) / 32 * a.Hq * a.B >= 448) return launch_form<Acc, DM, 2, 2>(p, a, s);
-                return launch_form<Acc, DM, 1, 2>(p, a, s);
-            }
+        const Form form = form_of<DM>(a);
+        if (form == Form::k16x16) return launch_form<Acc, DM, 1, 1>(p, a, s);
+        if constexpr (DM == 64) {               // (no boolean mask takes 32 x 32 there)
+            if (form == Form::k32x32) return a.mask_kind == 0 ? launch_masked<Acc, DM, 2, 2, 0>(p, a, s) : launch_masked<Acc, DM, 2, 2, 2>(p, a, s);
+        } else if constexpr (DM == 128) {       // (only the causal rule takes 32 x 32 there)
+            if (form == Form::k32x32) return launch_masked<Acc, DM, 2, 2, 0>(p, a, s);
+            if (form == Form::k32x16) return launch_form<Acc, DM, 2, 1>(p, a, s);
         }
-        launch_form<Acc, DM, 1, 1>(p, a, s);
+        launch_form<Acc, DM, 1, 2>(p, a, s);
     }
 }
 

@@ -1013,6 +1013,40 @@ def test_fp32_attention_either_side_of_its_forms(B, H, S, D, kind):
     assert rel_err(out, want) <= 3e-6
 
 
+@pytest.mark.parametrize("B,H,S,D,kind", [(8, 16, 512, 64, "additive"), (1, 15, 1024, 64, "additive"), (1, 18, 1024, 64, "additive"), (1, 15, 1000, 64, "none"), (8, 16, 512, 64, "causal"), (1, 16, 700, 64, "padding"),
+                                          (1, 1, 1000, 128, "additive"), (1, 1, 1000, 128, "padding"), (2, 2, 1100, 128, "causal"), (1, 3, 2000, 128, "causal"), (1, 4, 8192, 128, "causal"), (1, 2, 4100, 128, "additive"),
+                                          (2, 12, 2048, 128, "none"), (2, 12, 2048, 128, "padding"), (2, 12, 2048, 128, "additive"), (1, 5, 4500, 128, "none"),
+                                          (1, 1, 2001, 256, "padding"), (2, 16, 1500, 256, "none"), (9, 16, 66, 256, "additive"), (9, 16, 80, 256, "none"), (9, 16, 81, 256, "padding")])
+def test_fp32_attention_forms_by_mask_size_and_weights(B, H, S, D, kind):
+    """The forms that masks, the causal rule, long rows and returned weights choose, against fp64 (to the one-pass kernel's bar) for some of the heads.  The output is the
+    same bits whether the weights are asked for or not, also where their number alone makes blocks of 32 queries of those of 16."""
+    g = torch.Generator(device="cuda").manual_seed(S + D)
+    q, k, v = (torch.randn(B, H, S, D, generator=g, device="cuda") for _ in range(3))
+    mask = None
+    if kind == "padding":
+        mask = (torch.arange(S, device="cuda")[None, :] < torch.randint(S // 2, S + 1, (B, 1), generator=g, device="cuda")).reshape(B, 1, 1, S).expand(B, H, S, S)
+    elif kind == "additive":
+        mask = torch.randn(1, 1, S, S, generator=g, device="cuda").expand(B, H, S, S)
+    kw = dict(is_causal=kind == "causal", mask=mask)
+    out, _, lse, name = capi.sdpa(q, k, v, want_lse=True, **kw)
+    assert name == "composed"
+    again, attn, lse2, _ = capi.sdpa(q, k, v, want_attn=True, want_lse=True, **kw)
+    assert_bit_exact(again, out)
+    assert_bit_exact(lse2, lse)
+    for b, h in {(0, 0), (B // 2, H // 2), (B - 1, H - 1)}:
+        one = lambda t: t[b, h].double().cpu()
+        s = one(q) @ one(k).T / math.sqrt(D)
+        if kind == "causal":
+            s = s.masked_fill(~torch.ones(S, S, dtype=torch.bool).tril(), -math.inf)
+        elif kind == "padding":
+            s = s.masked_fill(~mask[b, h].cpu(), -math.inf)
+        elif kind == "additive":
+            s = s + one(mask)
+        w = s.softmax(-1)
+        assert rel_err(out[b, h], w @ one(v)) <= 3e-6
+        assert ((one(attn) - w).abs() <= 1e-5 * w + 1e-30).all()           # (as test_fp32_weights_of_the_one_pass_kernel)
+
+
 def test_composed_route_fp64_and_wide_16_bit_heads():
     torch.manual_seed(5)
     q, k, v = _composed_case(torch.float64, 1, 4, 4, 2048, 2048, 32)
