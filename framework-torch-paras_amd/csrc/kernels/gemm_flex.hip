@@ -20,8 +20,8 @@ struct FinishParams {
     const float* partial;
     const std::uint16_t* add;
     std::uint16_t* c;
-    long M, N, sc, sadd;
-    int  ldc, ld_add, splits;
+    long M, N, sc, sadd, ldc, ld_add;
+    int  splits;
     float alpha, beta;
 };
 template <typename T, int V>
@@ -202,7 +202,7 @@ int launch(const Problem& q, const Plan& plan, void* workspace, hipStream_t s) {
     if (plan.splits > 1) {
         const bool vec = q.N % 4 == 0 && q.ldc % 4 == 0 && q.sc % 4 == 0 && (reinterpret_cast<uintptr_t>(q.c) & 7) == 0;
         const long n = (q.M * q.N + (vec ? 1023 : 255)) / (vec ? 1024 : 256);
-        const FinishParams f{static_cast<const float*>(workspace), q.add, q.c, q.M, q.N, q.sc, q.sadd, p.ldc, p.ld_add, plan.splits, q.alpha, q.beta};
+        const FinishParams f{static_cast<const float*>(workspace), q.add, q.c, q.M, q.N, q.sc, q.sadd, q.ldc, q.ld_add, plan.splits, q.alpha, q.beta};
         const dim3 g(static_cast<unsigned>(n), static_cast<unsigned>(q.batch));
         if (q.bf16) { if (vec) hipLaunchKernelGGL((gemm_flex_finish_kernel<bf16_t, 4>), g, dim3(256), 0, s, f);
                       else     hipLaunchKernelGGL((gemm_flex_finish_kernel<bf16_t, 1>), g, dim3(256), 0, s, f); }

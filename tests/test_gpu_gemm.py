@@ -6,6 +6,7 @@ in double and rounds once.  Bar: every element within one 16-bit ulp of the
 oracle (summation order is the only difference), and torch-CPU addmm / linear
 as the library check for the epilogue.
 """
+import ctypes as C
 import math
 
 import pytest
@@ -560,3 +561,19 @@ def test_scratch_is_asked_for_once_and_the_route_is_the_planned_one(shape, dtype
         c, _, rc = capi.gemm_scratch(a, b, lambda size: None)
         assert rc == -1 and bool((c == 7).all())
     assert n > 0 or shape != (300, 136, 14336)
+
+
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])
+def test_addend_rows_far_apart_in_a_product_in_parts(dtype):
+    """The kernel that adds the parts reads the addend: 1100 rows of 2^22 elements, the last of them beyond 2^32 elements.  Bar as in
+    test_gemm_tiles_with_several_stages, with a rounding of the addend's size more."""
+    M, N, K, ld = 1100, 64, 8192, 1 << 22
+    g = torch.Generator(device="cuda").manual_seed(3)
+    a, b = torch.randn(M, K, generator=g, device="cuda").to(dtype), (torch.randn(N, K, generator=g, device="cuda") / math.sqrt(K)).to(dtype)
+    add = torch.empty(M, ld, device="cuda", dtype=dtype)[:, :N]
+    add.copy_(torch.randn(M, N, generator=g, device="cuda"))
+    problem = capi.GemmArgs(a.data_ptr(), b.data_ptr(), add.data_ptr(), a.data_ptr(), M, N, K, K, K, N, ld, 1, 0, 0, 0, 0, 1.0, 1.0, capi.DT[dtype], 0, 0)
+    assert capi.lib().paras_gemm_workspace(C.byref(problem)) > 0
+    want = a.double() @ b.double().T + add.double()
+    half_ulp = {torch.bfloat16: 2.0 ** -8, torch.float16: 2.0 ** -11}[dtype]
+    assert bool(((capi.gemm(a, b, add).double() - want).abs() <= half_ulp * 1.01 * want.abs() + (4 * math.sqrt(K) + 8) * 2.0 ** -24).all())
