@@ -86,8 +86,6 @@ bool takes(const Problem& q) {
     if (!aligned(q.a, q.lda, q.sa) || !aligned(q.b, q.ldb, q.sb)) return false;
     // (a chunk of 8 contraction steps is in or out as a whole)
     if (q.K <= 0 || q.K >= (1L << 30) || (!(q.a_rows && q.b_rows) && q.K % 8 != 0)) return false;
-    constexpr long kInt = 0x7fffffffL;
-    if (q.ldc > kInt || (q.add != nullptr && q.ld_add > kInt)) return false;       // (flex::Params)
     const long tiles = ((q.M + 31) / 32) * ((q.N + 63) / 64);          // (below 2^25: M and N fit as well)
     return q.batch <= 65535 && tiles * q.batch < (1L << 25);
 }
@@ -187,11 +185,11 @@ int launch(const Problem& q, const Plan& plan, void* workspace, hipStream_t s) {
     p.a = q.a; p.b = q.b; p.add = q.add;
     p.out = plan.splits > 1 ? workspace : q.c;
     p.M = narrow(q.M); p.N = narrow(q.N); p.K = narrow(q.K);
-    p.lda = narrow(q.lda); p.ldb = narrow(q.ldb); p.ldc = narrow(q.ldc); p.ld_add = q.add != nullptr ? narrow(q.ld_add) : 0;
+    p.lda = static_cast<std::uint32_t>(q.lda); p.ldb = narrow(q.ldb); p.ldc = q.ldc; p.ld_add = q.ld_add;
     p.sa = q.sa; p.sb = q.sb; p.sc = q.sc; p.sadd = q.sadd;
     p.alpha = q.alpha; p.beta = q.beta;
     const Tile t = kTiles[plan.tile];
-    p.splits = plan.splits;
+    p.splits = static_cast<std::uint32_t>(plan.splits);
     p.k_per_split = narrow(plan.k_per_split);
     const long wgs = (q.M + t.m - 1) / t.m * ((q.N + t.n - 1) / t.n) * plan.splits * q.batch;
     const unsigned grid = static_cast<unsigned>(wgs);

@@ -7,20 +7,22 @@
 namespace paras {
 namespace flex {
 
-// (112 bytes: a launch whose arguments take more than that costs the host 0.7 us more, 3.4 for 2.7.  Sizes and row strides that do not fit are
-// refused by takes().)
+// (112 bytes: a launch whose arguments take more than that costs the host 0.7 us more, 3.4 for 2.7.)
 struct Params {
     const std::uint16_t* a;
     const std::uint16_t* b;
     const std::uint16_t* add;   // may be null
     void* out;                  // splits == 1: the result; otherwise fp32 [batch][split][M][N]
     long sa, sb, sc, sadd;      // batch strides (elements)
+    long ldc, ld_add;
     int  M, N, K;
-    int  lda, ldb, ldc, ld_add;
-    int  splits;                // parts of the contraction, one workgroup each per tile
+    int  ldb;
+    std::uint32_t lda : 23;     // (up to kMaxLd, as ldb)
+    std::uint32_t splits : 9;   // parts of the contraction, one workgroup each per tile (up to 384)
     int  k_per_split;           // contraction steps per part (a multiple of 64)
     float alpha, beta;
 };
+static_assert(kMaxLd < (1L << 23), "Params::lda");
 static_assert(sizeof(Params) <= 112, "see above");
 
 // Workgroup w runs on XCD w % 8, each with an L2 of its own: every XCD takes a contiguous run of the
@@ -59,8 +61,9 @@ __global__ __launch_bounds__(kThreads, (MI * NJ >= 32 || ST * (MI + NJ) > 20 ? 1
     __shared__ __attribute__((aligned(1024))) std::uint16_t b1[OB::kElems];
     __shared__ __attribute__((aligned(1024))) std::uint16_t b2[OB::kElems];
     __shared__ __attribute__((aligned(1024))) std::uint16_t b3[OB::kElems];
+    asm volatile("" ::"s"(p.ldc), "s"(p.ld_add));          // (fetched with the rest: left to itself the compiler does it in front of the stores)
     const Work w = work_of((static_cast<unsigned>(p.M) + 32 * MI - 1) / (32 * MI), (static_cast<unsigned>(p.N) + 32 * NJ - 1) / (32 * NJ),
-                           static_cast<unsigned>(p.splits), blockIdx.x, gridDim.x);
+                           p.splits, blockIdx.x, gridDim.x);
     const long row0 = static_cast<long>(w.mt) * (32 * MI), col0 = static_cast<long>(w.nt) * (32 * NJ);
     const long k_first = static_cast<long>(w.split) * p.k_per_split;
     const long k_count = p.K - k_first < p.k_per_split ? p.K - k_first : p.k_per_split;
@@ -78,7 +81,7 @@ __global__ __launch_bounds__(kThreads, (MI * NJ >= 32 || ST * (MI + NJ) > 20 ? 1
     const int l16 = lane & 15, kq = lane >> 4;
     const long wrow = row0 + (wave >> 1) * 16 * MI + l16, wcol = col0 + (wave & 1) * 16 * NJ + 4 * kq;
     if (p.splits > 1) {
-        float* dst = static_cast<float*>(p.out) + static_cast<long>(w.batch * p.splits + w.split) * (static_cast<long>(p.M) * p.N);
+        float* dst = static_cast<float*>(p.out) + static_cast<long>(w.batch * static_cast<int>(p.splits) + w.split) * (static_cast<long>(p.M) * p.N);
         const bool vec = p.N % 4 == 0;
 #pragma unroll
         for (int i = 0; i < MI; ++i) {

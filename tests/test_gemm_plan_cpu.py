@@ -38,3 +38,11 @@ def test_parts_of_the_contraction_by_size(a_rows, b_rows):
                            (1 << 20, 64, 64, False), (64, 1 << 20, 64, False)]:
         n = capi.lib().paras_gemm_workspace(C.byref(args(M, N, K, a_rows=a_rows, b_rows=b_rows)))
         assert n % (4 * M * N) == 0 and (n > 0) == split and n != 4 * M * N, (M, N, K, n)
+
+
+@pytest.mark.parametrize("a_rows,b_rows", [(0, 0), (0, 1), (1, 1)])
+def test_the_route_does_not_depend_on_how_far_apart_the_rows_of_the_result_are(a_rows, b_rows):
+    for ld in (512, 1 << 22, (1 << 31) - 1, 1 << 31, 1 << 33):
+        g = args(256, 512, 14336, a_rows=a_rows, b_rows=b_rows)
+        g.addend, g.ldc, g.ld_add = 4096, ld, ld
+        assert capi.lib().paras_gemm_workspace(C.byref(g)) == capi.lib().paras_gemm_workspace(C.byref(args(256, 512, 14336, a_rows=a_rows, b_rows=b_rows))) > 0, ld

@@ -577,3 +577,28 @@ def test_addend_rows_far_apart_in_a_product_in_parts(dtype):
     want = a.double() @ b.double().T + add.double()
     half_ulp = {torch.bfloat16: 2.0 ** -8, torch.float16: 2.0 ** -11}[dtype]
     assert bool(((capi.gemm(a, b, add).double() - want).abs() <= half_ulp * 1.01 * want.abs() + (4 * math.sqrt(K) + 8) * 2.0 ** -24).all())
+
+
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])
+@pytest.mark.parametrize("K,a_rows,b_rows", [(128, 0, 0), (72, 0, 0), (8200, 0, 0), (72, 0, 1), (72, 1, 1), (8192, 1, 1)])
+def test_rows_of_result_and_addend_beyond_31_bits(K, a_rows, b_rows, dtype):
+    """Two rows more than 2^31 elements apart, in the result and in the addend: the few-row kernel, tiles of each layout, whole and in parts.
+    Bar as in test_addend_rows_far_apart_in_a_product_in_parts."""
+    M, N, ldc, ld_add = 2, 100, (1 << 31) + 8, (1 << 31) + 20
+    g = torch.Generator(device="cuda").manual_seed(K)
+    a, b = torch.randn(K, 8, generator=g, device="cuda").to(dtype), (torch.randn(K, 104, generator=g, device="cuda") / math.sqrt(K)).to(dtype)
+    x, y = a[:, :M].T, b[:, :N].T
+    a, b = a if a_rows else x.contiguous(), b if b_rows else y.contiguous()
+    c, add = torch.empty(M, ldc, device="cuda", dtype=dtype)[:, :N + 4], torch.empty(M, ld_add, device="cuda", dtype=dtype)[:, :N]
+    c.fill_(7)
+    add.copy_(torch.randn(M, N, generator=g, device="cuda"))
+    problem = capi.GemmArgs(a.data_ptr(), b.data_ptr(), add.data_ptr(), c.data_ptr(), M, N, K, a.stride(0), b.stride(0), ldc, ld_add, 1, 0, 0, 0, 0, 1.0, 1.0,
+                            capi.DT[dtype], a_rows, b_rows)
+    n = capi.lib().paras_gemm_workspace(C.byref(problem))
+    assert (n > 0) == (K > 8000)
+    ws = torch.empty(max(n, 16), dtype=torch.uint8, device="cuda")
+    capi.check(capi.lib().paras_gemm(C.byref(problem), ws.data_ptr(), n, torch.cuda.current_stream().cuda_stream))
+    want = x.double().contiguous() @ y.double().T + add.double()
+    half_ulp = {torch.bfloat16: 2.0 ** -8, torch.float16: 2.0 ** -11}[dtype]
+    assert bool(((c[:, :N].double() - want).abs() <= half_ulp * 1.01 * want.abs() + (4 * math.sqrt(K) + 8) * 2.0 ** -24).all())
+    assert bool((c[:, N:] == 7).all())
