@@ -48,7 +48,8 @@ struct DecodeParams {
     std::uint16_t* out;
     float* lse;
     float* part;     // [pairs, splits]: 16 maxima, 16 sums, 16 x D outputs
-    int q8_b, q8_h, q8_l, k8_b, k8_h, k8_l, v8_b, v8_h, v8_l;     // strides in eights of elements (decode_supported)
+    int q8_b, q8_h, q8_l, k8_b, k8_h, k8_l, v8_b, v8_h, v8_l;     // strides in eights of elements (decode_supported); between sequences 2^far eights
+    int far;
     int Hkv, Lk;
     int chunk;       // keys per workgroup
     std::uint32_t shape;          // splits | Lq << 16 | G << 24
@@ -122,7 +123,7 @@ __global__ __launch_bounds__(kThreads, (D > 128 ? 1 : 2)) void decode_split_kern
     {
         const bool live = lq < R;
         const int gi = live ? lq / Lq : 0, qi = live ? lq % Lq : 0;
-        const std::uint16_t* qp = p.q + 8 * (static_cast<long>(b) * p.q8_b + static_cast<long>(hkv * G + gi) * p.q8_h + static_cast<long>(qi) * p.q8_l);
+        const std::uint16_t* qp = p.q + 8 * ((static_cast<long>(b) * p.q8_b << p.far) + static_cast<long>(hkv * G + gi) * p.q8_h + static_cast<long>(qi) * p.q8_l);
 #pragma unroll
         for (int ks = 0; ks < KS; ++ks) {
             i16x8 z = {0, 0, 0, 0, 0, 0, 0, 0};
@@ -146,9 +147,9 @@ __global__ __launch_bounds__(kThreads, (D > 128 ? 1 : 2)) void decode_split_kern
     const int k_end = min(k_begin + wlen, chunk1);
     const int n_tiles = k_end > k_begin ? (k_end - k_begin + kTile - 1) / kTile : 0;
 
-    const std::uint16_t* kbase = p.k + 8 * (static_cast<long>(b) * p.k8_b + static_cast<long>(hkv) * p.k8_h);
+    const std::uint16_t* kbase = p.k + 8 * ((static_cast<long>(b) * p.k8_b << p.far) + static_cast<long>(hkv) * p.k8_h);
     const long k_row = 8L * p.k8_l, v_row = 8L * p.v8_l;
-    const std::uint16_t* vbase = p.v + 8 * (static_cast<long>(b) * p.v8_b + static_cast<long>(hkv) * p.v8_h);
+    const std::uint16_t* vbase = p.v + 8 * ((static_cast<long>(b) * p.v8_b << p.far) + static_cast<long>(hkv) * p.v8_h);
 
     i16x8 kcur[2][KS], knext[2][KS];
     u32x4 vst[VCH];
@@ -488,6 +489,15 @@ size_t workspace_of(const paras_sdpa_args& a, int splits) {
     return slots * slot_floats(a.D) * sizeof(float);
 }
 
+// DecodeParams::far: 0 but for sequences 2^34 elements apart and more (a cache that holds all layers of a sequence together); -1: no power of two does.
+int far_of(const paras_sdpa_args& a) {
+    const int64_t q = a.q_strides[0] / 8, k = a.k_strides[0] / 8, v = a.v_strides[0] / 8;
+    auto fits = [](int64_t n) { return n == static_cast<int>(n); };
+    int far = 0;
+    while (!(fits(q >> far) && fits(k >> far) && fits(v >> far))) ++far;
+    return ((q | k | v) & ((int64_t{1} << far) - 1)) == 0 ? far : -1;
+}
+
 }  // namespace
 
 bool decode_supported(const paras_sdpa_args& a) {
@@ -503,9 +513,9 @@ bool decode_supported(const paras_sdpa_args& a) {
     if (!aligned16(a.q) || !aligned16(a.k) || !aligned16(a.v)) return false;
     if (!mult8(a.q_strides) || !mult8(a.k_strides) || !mult8(a.v_strides)) return false;
     for (const int64_t* st : {a.q_strides, a.k_strides, a.v_strides})
-        for (int i = 0; i < 3; ++i)
+        for (int i = 1; i < 3; ++i)
             if (st[i] / 8 != static_cast<int>(st[i] / 8)) return false;          // (DecodeParams)
-    return true;
+    return far_of(a) >= 0;
 }
 
 size_t decode_workspace(const paras_sdpa_args& a) {
@@ -524,9 +534,11 @@ int launch_decode(const paras_sdpa_args& a, Scratch scratch, hipStream_t s) {
     p.out = static_cast<std::uint16_t*>(a.out);
     p.lse = a.lse;
     auto eights = [](int64_t stride) { return static_cast<int>(stride / 8); };
-    p.q8_b = eights(a.q_strides[0]); p.q8_h = eights(a.q_strides[1]); p.q8_l = eights(a.q_strides[2]);
-    p.k8_b = eights(a.k_strides[0]); p.k8_h = eights(a.k_strides[1]); p.k8_l = eights(a.k_strides[2]);
-    p.v8_b = eights(a.v_strides[0]); p.v8_h = eights(a.v_strides[1]); p.v8_l = eights(a.v_strides[2]);
+    p.far = far_of(a);
+    auto between = [&](int64_t stride) { return static_cast<int>(stride / 8 >> p.far); };
+    p.q8_b = between(a.q_strides[0]); p.q8_h = eights(a.q_strides[1]); p.q8_l = eights(a.q_strides[2]);
+    p.k8_b = between(a.k_strides[0]); p.k8_h = eights(a.k_strides[1]); p.k8_l = eights(a.k_strides[2]);
+    p.v8_b = between(a.v_strides[0]); p.v8_h = eights(a.v_strides[1]); p.v8_l = eights(a.v_strides[2]);
     p.Hkv = (int)a.Hkv; p.Lk = (int)a.Lk;
     const int G = (int)(a.Hq / a.Hkv), R = G * (int)a.Lq;
     int splits = 1;

@@ -1294,3 +1294,20 @@ def test_fp32_weights_of_the_one_pass_kernel_in_a_captured_graph():
         want, wattn, _, _ = capi.sdpa(q, k, v, is_causal=True, want_attn=True)
         assert_bit_exact(out, want)
         assert_bit_exact(attn, wattn)
+
+
+@pytest.mark.parametrize("masked", [False, True])
+def test_one_token_attention_over_sequences_far_apart(masked):
+    """Keys and values of two sequences more than 2^34 elements apart: the same bits as side by side."""
+    Hkv, L, D, apart = 2, 300, 128, (1 << 34) + 4096
+    g = torch.Generator(device="cuda").manual_seed(9)
+    q, k, v = (torch.randn(2, h, l, D, generator=g, device="cuda", dtype=torch.bfloat16) for h, l in ((8, 1), (Hkv, L), (Hkv, L)))
+    mask = (torch.rand(2, 1, 1, L, generator=g, device="cuda") < 0.7).expand(2, 8, 1, L) if masked else None
+    far = torch.empty(apart + 2 * Hkv * L * D, device="cuda", dtype=torch.bfloat16)
+    fk, fv = (torch.as_strided(far, (2, Hkv, L, D), (apart, L * D, D, 1), i * Hkv * L * D) for i in (0, 1))
+    fk.copy_(k)
+    fv.copy_(v)
+    out, _, _, name = capi.sdpa(q, fk, fv, mask=mask)
+    want, _, _, other = capi.sdpa(q, k, v, mask=mask)
+    assert name == other == "decode_split"
+    assert_bit_exact(out, want)

@@ -26,6 +26,16 @@ def test_workspace_of_wide_types_does_not_depend_on_the_pointers(dtype, with_att
     assert len(seen) == 1, seen
 
 
+@pytest.mark.parametrize("apart", [1 << 20, (1 << 34) - 8, 1 << 34, 80 * 2 * 8 * 131072 * 128, (1 << 40) + 4096])
+def test_one_token_attention_does_not_depend_on_how_far_apart_sequences_are(apart):
+    """The one-token kernel takes caches that hold all layers of a sequence together, whose sequences are 2^34 elements apart and more."""
+    q, k, out = torch.zeros(2, 32, 1, 128, dtype=torch.bfloat16), torch.zeros(2, 8, 1000, 128, dtype=torch.bfloat16), torch.zeros(2, 32, 1, 128, dtype=torch.bfloat16)
+    a = capi.sdpa_args(q, k, k, out)
+    want = capi.lib().paras_sdpa_workspace(C.byref(a))
+    a.k_strides[0] = a.v_strides[0] = apart
+    assert capi.lib().paras_sdpa_kernel_name(C.byref(a)) == b"decode_split" and capi.lib().paras_sdpa_workspace(C.byref(a)) == want
+
+
 @pytest.fixture(scope="module")
 def deal(tmp_path_factory):
     """sdpa_flash_deal.h as a library of its own (plain C++, no HIP)."""
