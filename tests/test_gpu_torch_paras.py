@@ -1072,6 +1072,33 @@ def test_negated_views_are_read_negated(device):
     assert torch.equal(into.cpu(), -x)
 
 
+@pytest.mark.parametrize("rank", [4, 5, 6, 7, 8])
+def test_dimensions_that_do_not_fold(rank, device):
+    """Up to four dimensions go to the kernels in small arguments, five to eight in general ones: copies of every element width, row by row
+    and element by element, sums and products of 16-bit rows, rotate_half.  The dimensions are in the reverse order, so no two are one."""
+    from torch_paras import nn as paras_nn
+    shape = (2, 3, 2, 3, 2, 2, 3, 32)[-rank:]
+    base = torch.randn(shape)
+    rows = lambda t: t.permute(*range(rank - 2, -1, -1), rank - 1)
+    elements = lambda t: t.permute(*range(rank - 1, -1, -1))
+    for view in (rows, elements):
+        v = view(base)
+        assert all(v.stride(d) != v.stride(d + 1) * v.size(d + 1) for d in range(rank - 1))
+        for dt in (torch.uint8, torch.bfloat16, torch.float16, torch.float32, torch.float64):
+            t = (50 * base.abs()).clamp(max=255).to(dt)
+            assert torch.equal(view(t.to(device)).contiguous().cpu(), view(t).contiguous()), dt
+            into = torch.zeros(shape, dtype=dt).to(device)
+            view(into).copy_(view(t).contiguous().to(device))
+            assert torch.equal(into.cpu(), t), dt
+    for dt in (torch.bfloat16, torch.float16):
+        a, b, row = base.to(dt), torch.randn(shape).to(dt), torch.randn(shape[-1]).to(dt)
+        for other in (rows(b), rows(b).contiguous(), row, b.reshape(rows(b).shape)):
+            on = rows(b.to(device)) if other.shape == rows(b).shape and not other.is_contiguous() else other.to(device)
+            for fn, code in ((torch.add, O.OP_ADD), (torch.mul, O.OP_MUL)):
+                assert_bit_exact(fn(rows(a.to(device)), on).cpu(), O.binary(code, rows(a).contiguous(), other.contiguous()), f"{fn.__name__} {dt}")
+        assert_bit_exact(paras_nn.rotate_half(rows(a.to(device))).cpu(), O.rotate_half(rows(a).contiguous()), f"rotate_half {dt}")
+
+
 @pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])
 def test_rotate_half_of_views_is_that_of_their_copies(dtype, device):
     """Rows that lie anywhere (a projection's heads, slices of a fused one, repeated rows, one dimension of many) are read where they
