@@ -300,8 +300,8 @@ def test_swiglu_backward_every_gate_value(dtype):
 
 @pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])
 def test_swiglu_tiers_for_every_gate_and_many_values(dtype):
-    """The error bounds of the fp32 tier hold for every gate: each one with 24 random up and grad_out values of many magnitudes, so that
-    every distance from a rounding boundary turns up (any element that stood with a wrong rounding differs by a bit)."""
+    """Both tiers for every gate, each with 24 random up and grad_out values of many magnitudes: an element that stood with a wrong
+    rounding differs by a bit.  (Every distance from a rounding boundary: test_swiglu_bounds_of_the_fp32_tier.)"""
     g = torch.Generator().manual_seed(23)
     gate = torch.arange(-32768, 32768, dtype=torch.int32).to(torch.int16).view(dtype).repeat(24)
     gate = gate[gate.isfinite()]
@@ -311,6 +311,47 @@ def test_swiglu_tiers_for_every_gate_and_many_values(dtype):
     wgg, wgu = O.swiglu_backward(dy, gate, up)
     assert_bit_exact(gg, wgg, "grad_gate")
     assert_bit_exact(gu, wgu, "grad_up")
+
+
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])
+def test_swiglu_bounds_of_the_fp32_tier(dtype):
+    """The bounds say how near a rounding boundary an fp32 result may stand.  The result's place between boundaries depends on the gate and on
+    the significand of `up` alone (of grad_out for grad_up), so every gate of the fp32 tier's range is taken with every significand, at an
+    exponent that puts the result near 1.  grad_gate has two of them: all of grad_out's with one of up's each, and 16384 pairs where the bound is
+    the tightest, near -8, and where it grows, near the zero of silu' at -1.278.  Bit for bit against the oracle."""
+    bits = {torch.bfloat16: 7, torch.float16: 10}[dtype]
+    top = {torch.bfloat16: 120, torch.float16: 14}[dtype]
+    gate = torch.arange(-32768, 32768, dtype=torch.int32).to(torch.int16).view(dtype)
+    gate = gate[(gate >= -8) & (gate <= 60) & (gate != 0)]
+    g = torch.Generator().manual_seed(31)
+
+    def significands(n, count):
+        """Row r: `count` significands of the type, in an order of its own."""
+        every = 1 + torch.arange(1 << bits, dtype=torch.float64) / (1 << bits)
+        if count == 1 << bits:
+            return torch.stack([every.roll(int(k)) for k in torch.randint(1 << bits, (n,), generator=g)])
+        return every[torch.randint(1 << bits, (n, count), generator=g)]
+
+    def at(significand, exponent):
+        return torch.ldexp(significand, exponent.clamp(-top, top)[:, None]).to(dtype)
+
+    def check(gates, count):
+        x = gates.double()
+        s = torch.sigmoid(x)
+        near_one = -torch.log2((x * s).abs()).round().clamp(-top, top)
+        d_silu = (s * (1 + x * (1 - s))).abs().clamp_min(2.0 ** -20)
+        dy, up = at(significands(len(x), count), near_one), at(significands(len(x), count), near_one)
+        pair = at(significands(len(x), count), -near_one - torch.log2(d_silu).round())
+        every = gates[:, None].expand(-1, count).contiguous()
+        assert_bit_exact(capi.swiglu(dev(every), dev(up)), O.swiglu(every, up), "swiglu")
+        gg, gu = capi.swiglu_backward(dev(dy), dev(every), dev(pair))
+        wgg, wgu = O.swiglu_backward(dy, every, pair)
+        assert_bit_exact(gg, wgg, "grad_gate")
+        assert_bit_exact(gu, wgu, "grad_up")
+
+    for some in gate.split(8192):
+        check(some, 1 << bits)
+    check(gate[(gate < -7.5) | ((gate > -1.36) & (gate < -1.2))], 16384)
 
 
 @pytest.mark.parametrize("dtype", EXACT)
