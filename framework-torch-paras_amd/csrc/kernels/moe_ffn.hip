@@ -21,7 +21,6 @@
 // expert are contiguous in the routed order; m-tiles never straddle experts (the grid is sized for the
 // worst case and surplus workgroups exit).
 #include <hip/hip_runtime.h>
-#include <cmath>
 #include <cstdlib>
 #include <type_traits>
 
@@ -30,6 +29,7 @@
 #include "core/status.h"
 #include "kernels/gemm_flex.h"
 #include "kernels/gemm_tile.h"
+#include "kernels/moe_forms.h"
 #include "kernels/stream_rows.h"
 #include "kernels/swiglu_math.h"
 
@@ -213,9 +213,9 @@ struct SwigluQueue {
 };
 __device__ __forceinline__ unsigned scalar_of(unsigned v) { return static_cast<unsigned>(__builtin_amdgcn_readfirstlane(static_cast<int>(v))); }
 constexpr int kTileBand = 8;        // m-tiles whose column units an XCD walks through together: they share the experts' weights in its L2
-constexpr int kSuperM = 8, kSuperN = 4;
 constexpr int kStageElems = 256 * kBK;          // a stage of either operand: 256 rows of a k-tile
 static_assert(sizeof(SwigluQueue) <= kStageElems * 2, "a queue in a tile stage");
+static_assert(kBK == kFormStep, "moe_forms.h");
 
 // The weight rows of a 256-column tile that come as two groups of 128: a wave's 128 rows of the LDS tile are 64 rows of
 // group 0 and the 64 rows of group 1 with the same index, so that the accumulators of a gate column and of its up
@@ -851,66 +851,6 @@ int run_ffn_any(const void* x, const void* w_gate, const void* w_up, const void*
                        static_cast<std::uint16_t*>(out), T_, k, H);
     PARAS_HIP_TRY(hipGetLastError());
     return PARAS_OK;
-}
-
-// The tiles of a grouped product: rows, weight rows, stages, workgroups a CU holds, and for the gate-up product and the plain one the time
-// in us of 64 contraction steps on a CU that is full (`step`) and at least (`lat`).  The last two are grouped_gemm_direct_kernel, its tiles dealt in
-// super-tiles or one by one.
-struct GroupedForm { int m, n, stages, per_cu; double step[2], lat[2]; };
-constexpr GroupedForm kForms[] = {{128, 128, 2, 2, {0.91, 0.78}, {0.66, 0.47}}, {128, 128, 3, 1, {0.54, 0.36}, {0.13, 0.02}}, {64, 128, 2, 3, {0.74, 0.33}, {0.51, 0.42}},
-                                  {64, 128, 4, 1, {0.19, 0.24}, {0.35, 0.23}}, {32, 128, 4, 2, {0.30, 0.07}, {0.15, 0.16}}, {256, 256, 2, 1, {1.13, 0.97}, {0.32, 0.30}},
-                                  {256, 256, 2, 1, {1.13, 0.97}, {0.32, 0.30}}};
-constexpr int kFormCount = sizeof(kForms) / sizeof(kForms[0]), kDirectForm = kFormCount - 2, kOneByOne = kFormCount - 1;
-
-// Tiles of 256 rows where each of E experts has R / E rows on average and each row is sent on its own (a normal distribution).
-double tiles_256(long E, long R) {
-    const double rows = static_cast<double>(R) / E, spread = std::sqrt(2.0 * rows);
-    double n = 1.0 - std::exp(-rows);
-    for (double j = 256; j < rows + 3 * spread; j += 256) n += 0.5 * std::erfc((j + 0.5 - rows) / spread);
-    return E * n;
-}
-
-// The least estimated time, from three that overlap for the most part (the fourth root of the sum of their fourth powers): rounds of
-// workgroups times their contraction and stores, the way of the weights from memory, and that of all tiles' operands from the caches.  (How
-// the rows are spread over the experts is known on the device only: half an empty tile per expert, one tile where an expert has less than two
-// thirds of one.)  Fitted to 1800 timings of 150 layers (8 to 8192 tokens, 4 to 64 experts, H 512 to 4096, I 512 to 14336), over which the
-// choice is 2 % (gate-up) and 5 % (down) slower than the best form in the mean; always the same form is 15 % and 22 % at the least.  (256 x 256 tiles one
-// by one came later, for up to three rounds: of more the last is a small part.  One tile too many is a round, so their number is estimated by the
-// spread of the rows, with 3 % more, and a round is taken 5 % and 6 us longer than the contraction and stores, which is what separates 33 products near
-// the line: none over 4 % slower than the other forms would be, the mean 8 % faster.  36 layers of 500 to 8192 tokens: 0.3 % slower to 34 % faster, the mean 6 %.)
-int grouped_form(bool swiglu, long E, long R, long N, long K) {
-    const int w = swiglu ? 0 : 1;
-    const double start = swiglu ? 3.9 : 1.3, store = swiglu ? 15.4 : 9.4, rows = static_cast<double>(R) / E, used = R < E ? R : E;
-    const double memory = used * N * K * (swiglu ? 4.0 / 5.34e6 : 2.0 / 5.37e6), cached = swiglu ? 16.4e6 : 14.1e6;
-    auto fourth = [](double v) { return v * v * v * v; };
-    int best = 0;
-    double best_cost = 1e300;
-    for (int f = 0; f < kFormCount; ++f) {
-        const GroupedForm& t = kForms[f];
-        const long cols = swiglu ? t.n / 2 : t.n, units = (N + cols - 1) / cols, k_tiles = K / kBK, turns = (k_tiles + t.stages - 1) / t.stages * t.stages;
-        if (f == kOneByOne && static_cast<double>(R) / 256 * units > 3 * 256) continue;
-        const double m_tiles = f == kOneByOne ? tiles_256(E, R) : rows < 0.7 * t.m ? used : E * (rows / t.m + 0.5), tiles = m_tiles * units;
-        auto round = [&](double n) {
-            const double c = t.step[w] * n / t.per_cu;
-            return turns * (c > t.lat[w] ? c : t.lat[w]) + start + store * t.m * cols / 65536.0 * n;
-        };
-        double us;
-        if (f == kDirectForm) {          // super-tiles of 32 workgroups, dealt to the 8 XCDs
-            us = std::ceil(std::ceil(m_tiles / kSuperM) * std::ceil(static_cast<double>(units) / kSuperN) / 8) * round(1.0);
-        } else if (f == kOneByOne) {
-            us = 1.05 * std::ceil(1.03 * tiles / 256) * (round(1.0) + 6.0);
-        } else {
-            const double slots = 256.0 * t.per_cu, full = std::floor(tiles / slots), rest = std::ceil((tiles - full * slots) / 256.0);
-            us = full * round(t.per_cu) + (rest > 0 ? round(rest) : 0.0);
-        }
-        const double traffic = tiles * (t.m + t.n) * K * 2.0 / cached;
-        const double cost = fourth(us) + fourth(memory) + fourth(traffic);
-        if (cost < best_cost) {
-            best_cost = cost;
-            best = f;
-        }
-    }
-    return best;
 }
 
 template <typename T, bool kSwiglu>
