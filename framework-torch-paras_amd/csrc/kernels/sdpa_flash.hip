@@ -78,6 +78,7 @@
 #include "core/device_math.h"
 #include "core/status.h"
 #include "kernels/sdpa_flash_common.h"
+#include "kernels/sdpa_flash_deal.h"
 #include "kernels/sdpa_internal.h"
 
 namespace paras {
@@ -890,19 +891,9 @@ template <typename T, int D>
 int launch_t(FlashParams p, bool causal, int mask_kind, bool halves, hipStream_t s) {
     constexpr int kHalves = D > 128 ? 1 : 2;           // (the tiles of two halves of 256-element heads do not fit LDS)
     p.n_qblocks = (p.Lq + kBM - 1) / kBM;
-    const long BH = static_cast<long>(p.B) * p.Hq, heads = BH / 8;
+    const long BH = static_cast<long>(p.B) * p.Hq;
     p.head_group = BH % 16 == 0 ? 2 : 1;
-    if (causal && BH % 8 == 0) {
-        // Under the causal rule an XCD takes the longest query tiles of several heads first, as many as have 8 MB of keys and values between them:
-        // head by head, the last heads' longest tiles start late.  (By two heads, and this way: bf16 D64 B4 H16 S2048 58.4 -> 48.1 us, B2 H32
-        // S4096 181 -> 168, B1 H32 S8192 330 -> 322, B8 H8 S1024 23.8 -> 18.2, B1 H64 S700 16.0 -> 13.0; D128 B2 H32 S700 22.8 -> 20.0.
-        // More heads than that miss the L2: D256 B4 H16 S2532, 2.6 MB a head, by two 282, by eight 287.)
-        const long fit = (8L << 20) / (static_cast<long>(p.Lk) * D * 4 + 1);
-        long G = fit < heads ? fit : heads;
-        while (G > 2 && heads % G != 0) --G;
-        if (G > p.head_group) p.head_group = static_cast<int>(G);
-        if (heads % p.head_group != 0) p.head_group = 1;
-    }
+    if (causal && BH % 8 == 0) p.head_group = static_cast<int>(heads_together(BH / 8, p.n_qblocks, p.Lk, D));
     p.magic_group = magic_of(BH % 8 == 0 ? static_cast<long>(p.head_group) * p.n_qblocks : causal ? BH : p.n_qblocks);
     p.magic_heads = magic_of(p.head_group);
     p.magic_hq = magic_of(p.Hq);

@@ -1,4 +1,5 @@
-// How the query tiles of a causal problem are dealt to the persistent workgroups of sdpa_flash_wide.hip (host code, no HIP).
+// How the query tiles of a causal problem are dealt to the workgroups of sdpa_flash.hip (heads_together) and to the persistent ones of
+// sdpa_flash_wide.hip (deal_of).  Host code, no HIP.
 //
 // The items of a pool of workgroups (the chip, or an XCD where the heads are dealt to the XCDs) are numbered by groups of G heads, longest query
 // tiles first within a group, and dealt in rounds of one item per workgroup, every other round in reverse order.  A few heads at a time
@@ -6,6 +7,8 @@
 // (bf16 D128 B5 H8 S6175, 25 tiles of 25 heads for 32 workgroups: one head at a time 1.4 times the share, 436 us, five 1.02, 355; B5 H14 S3840, 1050 items for
 // 256: 2.0 times and 382 us, all 70 heads 1.03 and 256).
 #pragma once
+
+#include <initializer_list>
 
 namespace paras {
 namespace flash {
@@ -117,6 +120,29 @@ inline Deal deal_of(long BH, long nq, long blocks, double head_bytes) {
         if (cost < d.cost) d = {static_cast<int>(g), cost};
     }
     return d;
+}
+
+// The kernel of 32 queries per wavefront: an XCD has `heads` heads of nq query tiles of 128 and takes the longest tiles of so many of them first.  One or two heads at
+// a time, the last heads' longest tiles start late; of too many, keys and values are fetched again for every tile.  Over 110 problems, by one or two heads / this
+// way: D64 B4 H16 S2048 54.4 / 45.7 us, B8 H8 S1024 21.9 / 17.5, B5 H8 (one key head) S2072 47.7 / 35.2; D128 B2 H32 S700 22.3 / 20.1, B20 H64 S134 51.9 / 42.9; D256 B2 H32 S934
+// 70.2 / 59.9; the mean of all 0.945, none over 3 % slower.
+//   More heads come out even in the first rounds of workgroups (two to a CU, one at 256 elements) than in later ones, where their number counts as their bytes do
+// (D128 B29 H24 S308, 261 tiles: 1 head 53.0, 3 53.9, 29, which have 4.4 MB, 61.1; B7 H64 S602: 2 heads 75.0, 8 77.2, 14 81.2, 56 92.5).  A group divides the heads; where they
+// hardly divide, one half as large again will do (19 heads, D64 S1749: one 90.3, all 81.0).
+inline long heads_together(long heads, long nq, long Lk, long D) {
+    const bool   few = heads * nq <= (D == 64 ? 192 : D == 128 ? 144 : 96);
+    const double megabytes = D == 64 || (D == 128 && few) ? 8.0 : D == 128 ? 2.0 : 4.0;
+    const double fit = megabytes * 1048576.0 / (static_cast<double>(Lk) * static_cast<double>(D) * 4.0), many = (few ? 2048.0 : 1024.0) / static_cast<double>(D);
+    const double most = fit < many ? fit : many;
+    long at_most = 1, above = heads;                         // the largest divisor of `heads` up to `most` and the next
+    for (long g = 1; g * g <= heads; ++g)
+        if (heads % g == 0)
+            for (const long d : {g, heads / g}) {
+                if (static_cast<double>(d) <= most) at_most = d > at_most ? d : at_most;
+                else                                above = d < above ? d : above;
+            }
+    if (at_most <= 2 && 2.0 * static_cast<double>(at_most) < most && static_cast<double>(above) <= (D == 64 ? 2.0 : 1.5) * most) at_most = above;
+    return at_most == 1 && heads % 2 == 0 ? 2 : at_most;
 }
 
 }  // namespace flash
