@@ -231,9 +231,11 @@ __global__ __launch_bounds__(256 * kHalves, (D > 128 || kHalves > 1 ? 1 : 2)) vo
     };
 
     // (One fetch for all the arguments on the way to the first loads: left to itself the compiler fetches the pointers behind the
-    // quotients, a second way to memory in front of everything: 11.9 us for 11.7.)
-    asm volatile("" ::"s"(p.q), "s"(p.k), "s"(p.v), "s"(p.rep), "s"(p.magic_group), "s"(p.magic_heads), "s"(p.magic_hq), "s"(p.magic_rep), "s"(p.head_group));
-    if constexpr (kMask != 0) asm volatile("" ::"s"(p.mask), "s"(p.ms_b), "s"(p.ms_h), "s"(p.ms_q), "s"(p.ms_k));
+    // quotients, a second way to memory in front of everything: 11.9 us for 11.7.  Not with 256 elements, B2 H8 S6968 791 -> 796 us, nor where a
+    // mask's arguments join them in parts of the keys, B2 H3 S2055 padded 29.1 -> 30.1.)
+    if constexpr (kMask == 0 ? D <= 128 : !kParts)
+        asm volatile("" ::"s"(p.q), "s"(p.k), "s"(p.v), "s"(p.rep), "s"(p.magic_group), "s"(p.magic_heads), "s"(p.magic_hq), "s"(p.magic_rep), "s"(p.head_group));
+    if constexpr (kMask != 0 && !kParts) asm volatile("" ::"s"(p.mask), "s"(p.ms_b), "s"(p.ms_h), "s"(p.ms_q), "s"(p.ms_k));
     const int nq = p.n_qblocks;
     const int BH = p.B * p.Hq;
     int bh, qi;
