@@ -609,10 +609,11 @@ int wide_group(long B, long Hq, long Hkv, long Lq, long Lk, int head, int mask_k
     // W 688; B1 H16 S1661 30 / 40, W 208; B6 H16 S4585 897 / 825).
     //   Causal: by the cost of the deal (deal_of; 1 is an even one) times how much more of the triangle query tiles of 256 pad than those of 128 do, where that is
     // under 6 %.  How much it may be goes with the length (an item's fixed cost: cost 1.04, B10 H16 S1536 109 / 116 us, B5 H24 S2048 138 / 135; 1.07, B1 H40
-    // S4608 228 / 205), is more where the other kernel's tiles are few rounds and so come out ill themselves (1.08, B2 H32 S1536 51 / 49) and more where the heads
+    // S4608 228 / 205), is more where the other kernel's tiles are few rounds and so come out ill themselves (1.08, B2 H32 S1536 51 / 49), less where they are many and
+    // do not (cost 1.00, B6 H32 S2036, 6 rounds, 0.94 times the other kernel's time, B24 H32 S2271, 27 rounds, 1066 / 1118), and more where the heads
     // are not dealt to XCDs, whose caches do not help that kernel then (1.05, B3 H28 S1792 82 / 86, B5 H28 S2048 186 / 173; 1.09, B7 H36 S2558 523 / 446).
-    // Over 172 problems of 1400 to 8200 queries 2.3 % less than with a deal taken to be even wherever there were over 1024 items, 7.5 % less than with one head at a
-    // time and limits of 4096 queries and two items to a CU; none over 1 % slower than either in repeated runs.
+    // Over 148 problems of 1400 to 8400 queries whose heads are dealt to XCDs the faster of the two kernels is missed by 0.3 % in the mean, 5 % at most; of 38 whose heads
+    // are not, this one is ahead in 37.
     const long least = causal ? 1400 : 896;
     if (forced < 0 && (Lq < least || Lk < least)) return 0;        // (before the runtime is asked: small calls are bound by the host)
     int dev = 0, cus = 0;
@@ -624,8 +625,9 @@ int wide_group(long B, long Hq, long Hkv, long Lq, long Lk, int head, int mask_k
     const long blocks = workgroups_for(BH, items, cus);
     const Deal deal = deal_of(BH, static_cast<long>(nq), blocks, head_bytes(Hq, Hkv, Lk));
     const double cost = padding * deal.cost, thousands = 1e-3 * static_cast<double>(Lq);
-    const double most = BH % 8 == 0 && blocks % 8 == 0 ? std::fmin(0.94 + 0.0475 * thousands, 1.07) + (items < 2 * cus ? 0.07 : items < 3 * cus && Lq >= 4096 ? 0.05 : 0.0)
-                                                       : std::fmin(0.93 + 0.065 * thousands, 1.13) + (items > 4 * cus ? 0.06 : 0.0);
+    const double rounds = static_cast<double>(items) / static_cast<double>(cus);
+    const double most = BH % 8 == 0 && blocks % 8 == 0 ? std::fmin(0.96 + 0.03 * thousands, 1.09) - std::fmin(std::fmax(0.006 * (rounds - 7.0), -0.02), 0.08) + (rounds < 2.0 ? 0.04 : 0.0)
+                                                       : std::fmin(0.93 + 0.065 * thousands, 1.13) + (rounds > 2.5 ? 0.06 : 0.0);
     return forced > 0 || cost < most ? deal.group : 0;
 }
 
