@@ -50,7 +50,7 @@ __device__ __forceinline__ bool narrow_is_safe(float y, std::uint32_t ulps) {
 // at g = -8, where the rounding of the exponent's argument counts in full.  The product with `up` rounds once more (1
 // unit), and E units are less than E fp32 ulps of the result: 10 covers it.  Every ulp costs: with the 32 of a
 // bound by analysis, 0.8 % of fp16 results were evaluated again in fp64, and 40 % of the times that a wave came to an element
-// (8192 x 14336 in fp16: 166 us, with this bound and the redone elements of a vector taken together 120; bf16 113 either way).
+// (8192 x 14336 in fp16: 132 us, with this bound and the redone elements of a vector taken together 111; bf16 112 either way).
 constexpr std::uint32_t kSwigluUlps = 10;
 
 template <typename T>
@@ -146,10 +146,10 @@ __device__ __forceinline__ void swiglu4_from_acc(const V a0, const V a1, typenam
 // q crosses zero near g = -1.278: rho grows without bound there and those elements take the exact
 // tier.  One more unit for the last product; a relative error of E units is less than E fp32 ulps of the result,
 // which is what narrow_is_safe takes.  (The bounds by analysis were three times as wide, and so was the share of the elements
-// that came to the fp64 tier: 8192 x 14336 in fp16 272 us, with these 237.)  bf16, with 32 times fewer elements near a
-// boundary, keeps bounds of that width: the kernel is bound by memory, and with hardly a wave going to the fp64 tier the
-// waves of a CU stay in step and a forward and backward in turn take longer, 309 us at 8192 x 14336 for 293 with these (188.7 and 182.5
-// at 6553 x 11008).
+// that came to the fp64 tier: forward and backward of 8192 x 14336 in fp16 358 us, with these and the forward's 321.)  bf16, with 8 times fewer elements
+// near a boundary, keeps bounds of that width: with fp16's, a forward and backward in turn are level over 64 x 1024 to 4096 x 11008 and behind over more
+// (4096 x 14336 152.1 us for 150.8, 6553 x 11008 185.7 for 184.6, 8192 x 14336 303 for 298 on one card and 297.6 for 296.9 on another, 32000 x 3000
+// 246 for 244; why is not known).
 template <typename T> struct SwigluBwdUlps { static constexpr std::uint32_t kAll = 10, kGate = 12; static constexpr float kPerRho = 2.5f; };
 template <> struct SwigluBwdUlps<bf16_t> { static constexpr std::uint32_t kAll = 36, kGate = 36; static constexpr float kPerRho = 10.0f; };
 
