@@ -379,18 +379,6 @@ __global__ __launch_bounds__(kBlock) void rms_norm_bwd_dw_partial(
     partial[slab * H + j] = acc;
 }
 
-template <typename T>
-__global__ __launch_bounds__(kBlock) void rms_norm_bwd_dw_final(
-    const double* __restrict__ partial, typename Elem<T>::store_t* __restrict__ gw, long slabs,
-    long H) {
-    using E = Elem<T>;
-    const long j = static_cast<long>(blockIdx.x) * kBlock + threadIdx.x;
-    if (j >= H) return;
-    double acc = 0.0;
-    for (long s = 0; s < slabs; ++s) acc += partial[s * H + j];
-    gw[j] = E::from_f64(acc);
-}
-
 // The same in one pass, for what the 16-byte kernels below do not take (fp32 tensors, 16-bit rows that are not whole aligned
 // 16-byte pieces): a workgroup holds a row of g and x in registers, V adjacent elements at a time, and keeps the column sums
 // of its rows there too, so that g and x are read once instead of three times and there is a partial sum per resident workgroup
@@ -932,6 +920,148 @@ __global__ __launch_bounds__(256, 4) void rms_norm_bwd_small(
     }
 }
 
+// Few rows, any type, rows of up to kFewMax elements: dx and the column sums side by side in ONE launch.  The column sums need
+// nothing of the rows' dot products (rstd is the forward pass's), so the first workgroups of the grid take a group of columns
+// each, over all rows, and the others the rows; both read g and x, the second reader out of a cache.  No partial sums, no second
+// kernel.  What bounds it is latency: a launch, one row's loads, its reduction and its stores.  The kernels above deal 16 rows and
+// more to a workgroup, one after the other, so that partial sums stay few, and leave the chip idle behind a few workgroups:
+// bf16 184 x 14656 on 12 of them 62 us, 9.8 this way; 184 x 4096 16.9 and 3.8; fp32 33 x 1000 in three kernels 8.2 and 2.6.
+// A workgroup takes a row (P pieces of V elements per thread, in registers), or with kWaveRows each of its waves does.
+// V == 1: rows that are not whole aligned 16-byte pieces.  The columns of a group are one 128-byte line of a row (V == 1 and 16 bits:
+// 64 bytes), so a wave reads 8 rows (V == 1: two) at once; threads add every RL-th row, and the sums meet in a fixed order: lanes of a
+// wave by exchanges, waves in LDS.
+constexpr long kFewMax = 16384;
+template <typename T, int V, int P, bool kWaveRows>
+__global__ __launch_bounds__(1024) void rms_norm_bwd_few(
+    const typename Elem<T>::store_t* __restrict__ go, const typename Elem<T>::store_t* __restrict__ x,
+    const typename Elem<T>::store_t* __restrict__ w, const float* __restrict__ rstd,
+    typename Elem<T>::store_t* __restrict__ gx, typename Elem<T>::store_t* __restrict__ gw, int rows, int H, int col_groups) {
+    using E = Elem<T>;
+    using S = typename E::store_t;
+    typedef S vec __attribute__((ext_vector_type(V)));
+    constexpr int CL = V > 1 ? 8 : 32;           // lanes along the columns of a group
+    constexpr int kCols = CL * V;
+    __shared__ double sums[16 * kCols];          // columns: one set per wave; rows: one slot per wave
+    const int tid = threadIdx.x, lane = tid & (kWave - 1), wave = tid / kWave, waves = static_cast<int>(blockDim.x) / kWave;
+    auto load = [](const S* p, S (&v)[V]) __attribute__((always_inline)) {
+        if constexpr (V == 1) {
+            v[0] = *p;
+        } else {
+            const vec t = *reinterpret_cast<const vec*>(p);
+#pragma unroll
+            for (int c = 0; c < V; ++c) v[c] = t[c];
+        }
+    };
+    if (static_cast<int>(blockIdx.x) < col_groups) {
+        const int col = (static_cast<int>(blockIdx.x) * CL + (tid % CL)) * V;
+        const bool live = col < H;               // (whole pieces: V divides H)
+        const int RL = static_cast<int>(blockDim.x) / CL;
+        const long step = static_cast<long>(RL) * H;
+        double acc[V];
+#pragma unroll
+        for (int c = 0; c < V; ++c) acc[c] = 0.0;
+        if (live) {
+            int r = tid / CL;
+            long at = static_cast<long>(r) * H + col;
+            auto add = [&](const S (&g)[V], const S (&xx)[V], float rs) __attribute__((always_inline)) {
+                const double rr = static_cast<double>(rs);
+#pragma unroll
+                for (int c = 0; c < V; ++c) acc[c] = fma(E::to_f64(g[c]) * E::to_f64(xx[c]), rr, acc[c]);
+            };
+            constexpr int U = V == 1 ? 8 : 4;    // rows in flight per thread
+            for (; r + (U - 1) * RL < rows; r += U * RL, at += U * step) {
+                S g[U][V], xx[U][V];
+                float rs[U];
+#pragma unroll
+                for (int u = 0; u < U; ++u) {
+                    load(go + at + u * step, g[u]);
+                    load(x + at + u * step, xx[u]);
+                    rs[u] = rstd[r + u * RL];
+                }
+#pragma unroll
+                for (int u = 0; u < U; ++u) add(g[u], xx[u], rs[u]);
+            }
+            for (; r < rows; r += RL, at += step) {
+                S g[V], xx[V];
+                load(go + at, g);
+                load(x + at, xx);
+                add(g, xx, rstd[r]);
+            }
+        }
+#pragma unroll
+        for (int off = CL; off < kWave; off <<= 1)
+#pragma unroll
+            for (int c = 0; c < V; ++c) acc[c] += __shfl_xor(acc[c], off, kWave);
+        if (lane < CL) {
+#pragma unroll
+            for (int c = 0; c < V; ++c) sums[wave * kCols + lane * V + c] = acc[c];
+        }
+        __syncthreads();
+        const int j = static_cast<int>(blockIdx.x) * kCols + tid;
+        if (tid < kCols && j < H) {
+            double t = 0.0;
+            for (int i = 0; i < waves; ++i) t += sums[i * kCols + tid];
+            gw[j] = E::from_f64(t);
+        }
+        return;
+    }
+    const int mine = kWaveRows ? lane : tid, team = kWaveRows ? kWave : static_cast<int>(blockDim.x);
+    const int first = static_cast<int>(blockIdx.x) - col_groups;
+    const long r = kWaveRows ? static_cast<long>(first) * waves + wave : first;
+    if (kWaveRows && r >= rows) return;          // (no barrier on this way)
+    const S* gr = go + r * H;
+    const S* xr = x + r * H;
+    int at[P];                                   // pieces past the row's end read its first one and are not stored
+    bool live[P];
+    S g[P][V], xx[P][V], wv[P][V];
+#pragma unroll
+    for (int i = 0; i < P; ++i) {
+        const int j = (mine + i * team) * V;
+        live[i] = j < H;
+        at[i] = live[i] ? j : 0;
+        load(gr + at[i], g[i]);
+        load(xr + at[i], xx[i]);
+        load(w + at[i], wv[i]);
+    }
+    const double rr = static_cast<double>(rstd[r]);
+    double dot = 0.0;
+#pragma unroll
+    for (int i = 0; i < P; ++i)
+#pragma unroll
+        for (int c = 0; c < V; ++c)
+            if (live[i]) dot = fma(E::to_f64(g[i][c]) * E::to_f64(wv[i][c]), E::to_f64(xx[i][c]), dot);
+    dot = wave_sum(dot);
+    if constexpr (!kWaveRows) {
+        if (lane == 0) sums[wave] = dot;
+        __syncthreads();
+        dot = 0.0;
+        for (int i = 0; i < waves; ++i) dot += sums[i];
+    }
+    const double coef = rr * rr * rr / static_cast<double>(H);
+#pragma unroll
+    for (int i = 0; i < P; ++i) {
+        if (!live[i]) continue;
+        S* dst = gx + r * H + at[i];
+        auto value = [&](int c) __attribute__((always_inline)) {
+            const double xj = E::to_f64(xx[i][c]);
+            return fma(E::to_f64(g[i][c]) * E::to_f64(wv[i][c]), rr, -(coef * xj * dot));
+        };
+        if constexpr (V == 8) {
+            float y[8];
+#pragma unroll
+            for (int c = 0; c < 8; ++c) y[c] = static_cast<float>(value(c));
+            store16(dst, bwd_narrow_vec<T>(y));
+        } else if constexpr (V == 1) {
+            *dst = E::from_f64(value(0));
+        } else {
+            vec t;
+#pragma unroll
+            for (int c = 0; c < V; ++c) t[c] = E::from_f64(value(c));
+            *reinterpret_cast<vec*>(dst) = t;
+        }
+    }
+}
+
 // Column sums of the slabs in a fixed order: thread (column c of kDwFinalCols, lane l of
 // kDwFinalLanes) adds slabs l, l + kDwFinalLanes, ... and the lane sums meet in LDS in lane order.
 // A workgroup's columns are one 128-byte line of every slab row, so no line is fetched by two
@@ -1063,10 +1193,73 @@ int launch_fwd(const void* x, const void* w, void* out, float* rstd, long rows, 
     return PARAS_OK;
 }
 
+// Up to how many rows dx and the column sums are one launch (rms_norm_bwd_few): where that stops being faster than the kernels that
+// read g and x once.  us, those kernels and this one (bf16): 64 columns 787 rows 5.4 and 5.3, 1500 5.9 and 8.1; 512 columns 1500 rows 8.8 and
+// 8.3, 3000 9.8 and 15.6; 1024 columns 33 rows 10.8 and 3.2, 1500 15.2 and 10.0, 2500 16.0 and 15.2; 4096 columns 77 rows 16.5 and 3.4, 2000
+// 20.1 and 16.8; 8192 columns 2000 rows 31.6 and 30.2, 2500 32.6 and 39.7; 14656 columns 184 rows 62.2 and 9.8.  Rows that are not whole vectors:
+// bf16 257 columns 1500 rows 9.6 and 9.8; 4001 columns 2000 rows 29.8 and 22.6; fp32 777 columns 1500 rows 14.1 and 12.9, 2000 15.4 and 15.7.
+// Where the other way is three kernels at any size (fp64; fp32 beyond 8192 columns), whole vectors: fp32 5500 x 12160 357 and 253, fp64
+// 5500 x 1000 49 and 43, 5500 x 4096 205 and 177.
+template <typename T>
+long few_rows(bool whole, long H) {
+    constexpr bool k16 = sizeof(typename Elem<T>::store_t) == 2, k64 = sizeof(typename Elem<T>::store_t) == 8;
+    if (!whole)            return H <= 700 || k64 ? 1000 : k16 ? 2000 : 1500;
+    if (k16)               return H <= 128 ? 700 : H <= 512 ? 1500 : 2000;
+    return k64 || H > 8192 ? 5500 : 2000;
+}
+template <typename T>
+bool takes_few(const void* go, const void* x, const void* w, const void* gx, long rows, long H, bool* whole) {
+    *whole = H % Elem<T>::kVec == 0 && ((reinterpret_cast<uintptr_t>(go) | reinterpret_cast<uintptr_t>(x) | reinterpret_cast<uintptr_t>(w) |
+                                         reinterpret_cast<uintptr_t>(gx)) & 15) == 0;
+    if (H > kFewMax || rows > few_rows<T>(*whole, H)) return false;
+    // (its column sums read g and x while other workgroups write dx: not in place)
+    const auto lo = reinterpret_cast<uintptr_t>(gx), size = static_cast<uintptr_t>(rows * H) * sizeof(typename Elem<T>::store_t);
+    auto apart = [&](const void* p) { const auto at = reinterpret_cast<uintptr_t>(p); return at + size <= lo || lo + size <= at; };
+    return apart(go) && apart(x);
+}
+template <typename T>
+int launch_few(const void* go, const void* x, const void* w, const float* rstd, void* gx, void* gw, long rows, long H, bool whole, hipStream_t s) {
+    using S = typename Elem<T>::store_t;
+    constexpr int V = Elem<T>::kVec;
+    const int v = whole ? V : 1;
+    const long pieces = H / v;
+    const int cols = whole ? 8 * V : 32;
+    const long groups = (H + cols - 1) / cols;
+    // a wave per row up to 128 pieces; otherwise as many threads as pieces, in whole waves, and beyond 1024 pieces more per thread
+    const bool wave_rows = pieces <= 2 * kWave;
+    auto go_with = [&](auto kernel, int block) {
+        const int per_wg = wave_rows ? block / kWave : 1;
+        hipLaunchKernelGGL(kernel, dim3(static_cast<unsigned>(groups + (rows + per_wg - 1) / per_wg)), dim3(static_cast<unsigned>(block)), 0, s,
+                           static_cast<const S*>(go), static_cast<const S*>(x), static_cast<const S*>(w), rstd, static_cast<S*>(gx),
+                           static_cast<S*>(gw), static_cast<int>(rows), static_cast<int>(H), static_cast<int>(groups));
+    };
+    auto threads = [&](int per) {
+        const long t = ((pieces + per - 1) / per + kWave - 1) / kWave * kWave;
+        return static_cast<int>(t < 512 ? 512 : t);
+    };
+    if (whole) {
+        if (pieces <= kWave)                      go_with(rms_norm_bwd_few<T, V, 1, true>, 512);
+        else if (wave_rows)                       go_with(rms_norm_bwd_few<T, V, 2, true>, 512);
+        else if (pieces <= 1024)                  go_with(rms_norm_bwd_few<T, V, 1, false>, threads(1));
+        else if (pieces <= 2048)                  go_with(rms_norm_bwd_few<T, V, 2, false>, threads(2));
+        else if constexpr (V == 2)                go_with(rms_norm_bwd_few<T, V, 8, false>, threads(8));
+        else if constexpr (V == 4)                go_with(rms_norm_bwd_few<T, V, 4, false>, threads(4));
+    } else {
+        if (wave_rows)                            go_with(rms_norm_bwd_few<T, 1, 2, true>, 512);
+        else if (pieces <= 2048)                  go_with(rms_norm_bwd_few<T, 1, 2, false>, threads(2));
+        else if (pieces <= 8192)                  go_with(rms_norm_bwd_few<T, 1, 8, false>, threads(8));
+        else                                      go_with(rms_norm_bwd_few<T, 1, 16, false>, threads(16));
+    }
+    PARAS_HIP_TRY(hipGetLastError());
+    return PARAS_OK;
+}
+
 template <typename T>
 int launch_bwd(const void* go, const void* x, const void* w, const float* rstd, void* gx,
                void* gw, void* workspace, long rows, long H, hipStream_t s) {
     using S = typename Elem<T>::store_t;
+    bool whole = false;
+    if (takes_few<T>(go, x, w, gx, rows, H, &whole)) return launch_few<T>(go, x, w, rstd, gx, gw, rows, H, whole, s);
     long slabs = (rows + kDwSlabRows - 1) / kDwSlabRows;
     PARAS_REQUIRE(slabs <= 0x7fffffffL, "paras_rms_norm_bwd: too many rows");
     if constexpr (sizeof(S) == 2) {

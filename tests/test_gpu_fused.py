@@ -226,6 +226,60 @@ def test_rms_norm_backward_team_workgroups(shape, dtype):
     assert_bit_exact(gw, wgw, f"rms_norm grad_weight {rows}x{H}")
 
 
+# piece counts at the edges of a wave, two waves, a workgroup and two of them, whole vectors and not; rows on both sides of each limit
+FEW = {torch.bfloat16: [(1, 8), (3, 512), (700, 128), (701, 128), (1500, 512), (1501, 512), (9, 520), (65, 1024), (8, 1032), (2000, 1032), (2001, 1032),
+                        (5, 8192), (7, 8200), (2, 16384), (2001, 8200), (3, 1), (257, 127), (1000, 129), (1001, 129), (4, 2049), (6, 8193), (2, 16383)],
+       torch.float32: [(1, 4), (5, 256), (33, 260), (130, 512), (9, 516), (33, 1000), (2000, 520), (2001, 520), (3, 4096), (4, 4100), (7, 8196), (2, 16384),
+                       (2001, 8196), (3, 1), (1000, 127), (1001, 127), (5, 2049), (3, 16383), (1500, 701), (1501, 701)],
+       torch.float64: [(1, 2), (17, 128), (9, 130), (5, 258), (3, 2050), (4, 4098), (2, 16384), (5500, 64), (5501, 64), (33, 129), (1001, 129), (2, 16383)]}
+
+
+@pytest.mark.parametrize("dtype,shape", [(d, s) for d, ss in FEW.items() for s in ss])
+def test_rms_norm_backward_of_few_rows(dtype, shape):
+    """dx and the column sums in one launch, and the kernels past its limits.  fp64 sums in another order than the oracle's: bit-exact after
+    narrowing to 16 bits; the fp32 weight gradient and fp64 results differ by the last bits of sums of up to 16384 terms."""
+    rows, H = shape
+    torch.manual_seed(rows * 31 + H)
+    x, w, go = torch.randn(rows, H).to(dtype), (1 + 0.1 * torch.randn(H)).to(dtype), torch.randn(rows, H).to(dtype)
+    _, rstd = O.rms_norm(x, w, 1e-6)
+    gx, gw = capi.rms_norm_backward(dev(go), dev(x), dev(w), dev(rstd))
+    wgx, wgw = O.rms_norm_backward(go, x, w, rstd)
+    if dtype == torch.float64:          # 2^-53 a term of each sum, relative to the sum of the terms' sizes
+        assert ((gx.cpu() - wgx).norm() / wgx.norm()).item() < 1e-13
+        assert ((gw.cpu() - wgw).norm() / wgw.norm()).item() < 1e-13
+        return
+    assert_bit_exact(gx, wgx, f"rms_norm grad_input {rows}x{H}")
+    if dtype == torch.float32:
+        assert torch.allclose(gw.cpu(), wgw, rtol=1e-6, atol=1e-6)
+    else:
+        assert_bit_exact(gw, wgw, f"rms_norm grad_weight {rows}x{H}")
+
+
+@pytest.mark.parametrize("rows,H", [(40, 264), (2100, 264)])
+def test_rms_norm_backward_in_place_and_odd_rows(rows, H):
+    """dx written over grad_out (few rows are then not one launch), and few rows with NaN, infinities and zeros beside a one-pass problem
+    with the same ones."""
+    torch.manual_seed(rows)
+    x, w, go = torch.randn(rows, H).bfloat16(), (1 + 0.1 * torch.randn(H)).bfloat16(), torch.randn(rows, H).bfloat16()
+    go[3] = 0.0; go[4] = -0.0; x[5] *= 1e-30; go[6] = x[6]; x[7] *= 1e18; go[8] *= 1e30
+    _, rstd = O.rms_norm(x, w, 1e-6)
+    wgx, wgw = O.rms_norm_backward(go, x, w, rstd)
+    gd, xd, wd, rd = dev(go), dev(x), dev(w), dev(rstd)
+    gw = torch.empty_like(wd)
+    ws = torch.empty(capi.lib().paras_rms_norm_bwd_workspace(rows, H), dtype=torch.uint8, device="cuda")
+    capi.check(capi.lib().paras_rms_norm_bwd(gd.data_ptr(), xd.data_ptr(), wd.data_ptr(), rd.data_ptr(), gd.data_ptr(), gw.data_ptr(), ws.data_ptr(), rows, H,
+                                             capi.DT[torch.bfloat16], torch.cuda.current_stream().cuda_stream))
+    assert_bit_exact(gd, wgx, "grad_input over grad_out")
+    assert_bit_exact(gw, wgw, "grad_weight")
+    go[9, 5] = float("nan"); x[10, 7] = float("inf"); go[11, 3] = float("-inf"); go[11, 4] = float("inf")
+    _, rstd = O.rms_norm(x, w, 1e-6)
+    got, want = capi.rms_norm_backward(dev(go), dev(x), dev(w), dev(rstd)), O.rms_norm_backward(go, x, w, rstd)
+    for a, b in zip(got, want):
+        a = a.cpu()
+        assert torch.equal(a.isnan(), b.isnan())
+        assert torch.equal(a[~a.isnan()].view(torch.int16), b[~b.isnan()].view(torch.int16))
+
+
 def test_rms_norm_backward_general_path_with_more_than_a_million_rows():
     """fp32 takes the three-kernel path, whose partial column sums are laid out one slab of 16 rows
     per workgroup along grid x: more than 65535 slabs (1,048,560 rows) must work."""
