@@ -230,5 +230,91 @@ __device__ __forceinline__ void mainloop(OA& oa, OB& ob, int k_count, std::uint1
     __builtin_amdgcn_s_waitcnt(0x0F70);         // vmcnt(0): no request may outlive the workgroup's LDS
 }
 
+// The results' way out.  A lane holds four columns of 16 rows apart per block: stored from there a wave's store is 16 pieces of 32 bytes, and
+// a tile's stores come all at once, from every CU in the same few us, with nothing beside them on a CU that holds one workgroup.  So each wave lays its
+// rows, narrowed, into one of the stages that nobody reads any more and stores them from there in whole rows, 16 bytes a lane.
+// `kChunks` 16-byte pieces a row, in an order turned by the row (16 rows apart by a power of two would be one bank).
+typedef __attribute__((address_space(3))) std::uint16_t lds_u16;
+typedef __attribute__((address_space(3))) u32x2 lds_u32x2;
+typedef __attribute__((address_space(3))) u32x4 lds_u32x4;
+template <int NJ> struct RowsOut {
+    static constexpr int kChunks = 2 * NJ;
+    __device__ static __forceinline__ int place(int row, int chunk) { return (chunk + (row & 15)) % kChunks; }
+    // columns 4*kq .. + 3 of block j of `row`
+    __device__ static __forceinline__ void lay(lds_u16* out, int row, int j, int kq, u32x2 v) {
+        *(lds_u32x2*)(out + row * (16 * NJ) + place(row, 2 * j + (kq >> 1)) * 8 + (kq & 1) * 4) = v;
+    }
+    __device__ static __forceinline__ u32x4 piece(lds_u16* out, int row, int chunk) {
+        return *(lds_u32x4*)(out + row * (16 * NJ) + place(row, chunk) * 8);
+    }
+};
+
+// Values narrowed by the conversion instructions, NaNs among them, to what the host's types make of a NaN.
+template <typename T> __device__ __forceinline__ std::uint32_t host_nan(std::uint32_t two) {
+    constexpr std::uint32_t kInf = __is_same(T, bf16_t) ? 0x7F80u : 0x7C00u;
+    auto one = [](std::uint32_t v) { return (v & 0x7FFFu) <= kInf ? v : __is_same(T, bf16_t) ? 0x7FC0u : (v & 0x8000u) | 0x7E00u; };
+    return one(two & 0xFFFFu) | one(two >> 16) << 16;
+}
+
+// Rows of a wave, laid out by RowsOut, to memory: `dst` is its first row and column, `rows` x `cols` of it exist (<= 0: none), in rows of `ld` elements.
+// `wide`: those are whole aligned 16-byte pieces.  `nan_here`: NaNs may be among them.
+template <typename T, int MI, int NJ>
+__device__ __forceinline__ void store_rows(lds_u16* out, std::uint16_t* dst, long ld, long rows, long cols, bool wide, bool nan_here) {
+    using Out = RowsOut<NJ>;
+    constexpr int kAll = 16 * MI * Out::kChunks, kTurns = (kAll + 63) / 64;
+    constexpr int kAhead = kTurns % 8 == 0 ? 8 : kTurns % 7 == 0 ? 7 : kTurns % 6 == 0 ? 6 : kTurns % 5 == 0 ? 5 : kTurns % 4 == 0 ? 4 : 1;
+    const int lane = threadIdx.x & 63;
+    if (wide && !nan_here && rows >= 16 * MI && cols >= 16 * NJ) {
+#pragma unroll 1
+        for (int t = 0; t < kTurns; t += kAhead) {
+            u32x4 v[kAhead];
+#pragma unroll
+            for (int u = 0; u < kAhead; ++u) {
+                const int c = (t + u) * 64 + lane;
+                v[u] = Out::piece(out, c / Out::kChunks, c % Out::kChunks);
+            }
+#pragma unroll
+            for (int u = 0; u < kAhead; ++u) {
+                const int c = (t + u) * 64 + lane;
+                if (kAll % 64 == 0 || c < kAll) *reinterpret_cast<u32x4*>(dst + (c / Out::kChunks) * ld + (c % Out::kChunks) * 8) = v[u];
+            }
+        }
+        return;
+    }
+#pragma unroll 1
+    for (int t = 0; t < kTurns; ++t) {
+        const int c = t * 64 + lane, row = c / Out::kChunks, col = (c % Out::kChunks) * 8;
+        if (c >= kAll || row >= rows || col >= cols) continue;
+        u32x4 v = Out::piece(out, row, c % Out::kChunks);
+        if (nan_here) {
+#pragma unroll
+            for (int u = 0; u < 4; ++u) v[u] = host_nan<T>(v[u]);
+        }
+        std::uint16_t* d = dst + row * ld + col;
+        if (wide && col + 7 < cols) {
+            *reinterpret_cast<u32x4*>(d) = v;
+        } else {
+#pragma unroll
+            for (int e = 0; e < 8; ++e)
+                if (col + e < cols) d[e] = static_cast<std::uint16_t>(v[e >> 1] >> (16 * (e & 1)));
+        }
+    }
+}
+
+// An accumulator, moved out of its register here and no earlier: all at once there is no room for them.  (`kWay`: the two sides of a branch
+// say something different, or the compiler moves what they have in common in front of it.)
+template <int kWay> __device__ __forceinline__ float4v in_turn(float4v& acc) {
+    if constexpr (kWay == 0) asm volatile("; plain" : "+a"(acc) : : "memory");
+    else if constexpr (kWay == 1) asm volatile("; scaled" : "+a"(acc) : : "memory");
+    else                     asm volatile("; part" : "+a"(acc) : : "memory");
+    return acc;
+}
+
+template <typename T> __device__ __forceinline__ u32x2 pack4(const float4v v) {
+    using El = Elem<T>;
+    return u32x2{El::from_f32_finite(v[0]) | (static_cast<std::uint32_t>(El::from_f32_finite(v[1])) << 16),
+                 El::from_f32_finite(v[2]) | (static_cast<std::uint32_t>(El::from_f32_finite(v[3])) << 16)};
+}
+
 }  // namespace flex
 }  // namespace paras

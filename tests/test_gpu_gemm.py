@@ -602,3 +602,37 @@ def test_rows_of_result_and_addend_beyond_31_bits(K, a_rows, b_rows, dtype):
     half_ulp = {torch.bfloat16: 2.0 ** -8, torch.float16: 2.0 ** -11}[dtype]
     assert bool(((c[:, :N].double() - want).abs() <= half_ulp * 1.01 * want.abs() + (4 * math.sqrt(K) + 8) * 2.0 ** -24).all())
     assert bool((c[:, N:] == 7).all())
+
+
+# one problem for each tile form and layout, edges cut short in both directions (N % 4 == 0; K % 64 == 8, 16 ... or few steps)
+TILES = [(0, (6437, 2104, 528)), (0, (2483, 4712, 576)), (0, (7082, 792, 536)), (0, (6536, 536, 528)), (0, (7119, 392, 64)), (0, (6977, 400, 136)), (0, (683, 5488, 64)),
+         (0, (5661, 144, 200)), (0, (5700, 136, 64)), (0, (33, 72, 64)), (0, (36, 72, 208)), (0, (130, 5528, 64)), (0, (2709, 4520, 520)), (0, (2389, 4344, 520)), (0, (1189, 7000, 528)),
+         (1, (1645, 7336, 520)), (1, (7683, 1160, 520)), (1, (1185, 5008, 528)), (1, (6805, 520, 528)), (1, (455, 6200, 64)), (1, (470, 6232, 136)), (1, (662, 5464, 64)),
+         (1, (4246, 200, 200)), (1, (34, 72, 200)), (1, (134, 5528, 72)),
+         (2, (1544, 7272, 528)), (2, (4840, 1840, 528)), (2, (7192, 816, 520)), (2, (520, 6552, 536)), (2, (7016, 408, 64)), (2, (400, 7128, 144)), (2, (5576, 136, 64)), (2, (136, 5616, 64))]
+
+
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])
+@pytest.mark.parametrize("layout,shape", TILES)
+def test_every_tile_form_stores_its_rows(layout, shape, dtype):
+    """Results in rows that lie apart, with the columns and rows beside them left alone: whole 16-byte pieces, and from an address and a stride
+    that are not; plain, and with an addend whose rows are and are not 8-byte pieces.  Bar: half a 16-bit ulp of the result, plus fp32 sums."""
+    M, N, K = shape
+    g = torch.Generator(device="cuda").manual_seed(M + N + K)
+    x, y = torch.randn(M, K, generator=g, device="cuda").to(dtype), (torch.randn(N, K, generator=g, device="cuda") / math.sqrt(K)).to(dtype)
+    a, b = x.T.contiguous() if layout == 2 else x, y.T.contiguous() if layout else y
+    add = torch.randn(M, N + 5, generator=g, device="cuda").to(dtype)
+    prod = x.double() @ y.double().T
+    half_ulp = {torch.bfloat16: 2.0 ** -8, torch.float16: 2.0 ** -11}[dtype]
+    for off, ldc, lda_, alpha in ((8, N + 16, None, 1.0), (1, N + 9, None, 1.0), (8, N + 16, N + 5, 0.5), (3, N + 8, 0, 1.0), (8, N + 16, N + 4, 1.0)):
+        buf = torch.full(((M + 1) * ldc + 16,), 7.0, device="cuda", dtype=dtype)
+        used = add.reshape(-1)[:M * (N + 4)].reshape(M, N + 4) if lda_ == N + 4 else add
+        problem = capi.GemmArgs(a.data_ptr(), b.data_ptr(), used.data_ptr() if lda_ is not None else None, buf.data_ptr() + 2 * off, M, N, K, a.stride(0), b.stride(0), ldc,
+                                lda_ or 0, 1, 0, 0, 0, 0, alpha, 2.0, capi.DT[dtype], int(layout == 2), int(layout > 0))
+        capi.check(capi.lib().paras_gemm(C.byref(problem), None, 0, torch.cuda.current_stream().cuda_stream))
+        want = alpha * prod
+        if lda_ is not None:
+            want = want + 2.0 * (used[:1, :N] if lda_ == 0 else used[:, :N]).double()
+        rows = buf[off:off + M * ldc].reshape(M, ldc)
+        assert bool(((rows[:, :N].double() - want).abs() <= half_ulp * 1.01 * want.abs() + (4 * math.sqrt(K) + 16) * 2.0 ** -24).all()), (off, lda_)
+        assert bool((rows[:, N:] == 7).all()) and bool((buf[:off] == 7).all()) and bool((buf[off + M * ldc:] == 7).all()), (off, lda_)
