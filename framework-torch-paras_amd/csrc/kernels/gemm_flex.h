@@ -136,6 +136,115 @@ template <int W, bool R> struct Operand {
     }
 };
 
+// Waits for all but `n` of this wave's loads in flight and for its LDS reads, and meets the others.
+template <int n> __device__ __forceinline__ void meet() {
+    __builtin_amdgcn_s_waitcnt(0x0070 | (n & 15) | ((n >> 4) << 14));     // vmcnt(n) lgkmcnt(0)
+    asm volatile("s_barrier" ::: "memory");     // (a fence of the compiler's own would wait for every direct load in flight)
+}
+
+// mainloop (below) for the largest tiles, whose two stages fill LDS.  Requests for a tile can go out once its stage is read, and with both operands
+// freed together that is one k-step out of two: a request per four MFMAs there, none in the other, and what comes from HBM instead of the last-level cache is
+// late.  Here B's fragments of both k-steps are read in the k-step before the tile, each into the registers that its predecessor has
+// just been multiplied from, so B's stage is free a k-step earlier than A's: B is requested in the first k-step and A in the second, a
+// request per eight MFMAs throughout.  It is the even pace that counts: with the same waits and distances but four MFMAs between requests it is slower than with one
+// barrier.  bf16, x W^T, 256 x 256 tiles, one barrier and this: 4096 x 4096 x 4096 with its operands in HBM 103.8 and 97.8 us, 16384 x 4096 x 4096 401 and 385,
+// 8192 x 4096 x 16384 805 and 738, 8192^3 753 and 733; with everything in the caches level (4096^3 94.4 and 94.0).
+template <typename T, int MI, int NJ, typename OA, typename OB>
+__device__ __forceinline__ void mainloop_paced(OA& oa, OB& ob, int k_count, std::uint16_t* const (&sa)[2], std::uint16_t* const (&sb)[2],
+                                               float4v (&acc)[MI][NJ]) {
+    constexpr int S = MI * NJ;          // MFMAs per k-step
+    i16x8 af[2][MI], bf[2][NJ];
+    const int k_tiles = (k_count + kBK - 1) / kBK;
+    auto request_all = [&](int kt, std::uint16_t* ta, std::uint16_t* tb) {
+        if (kt == k_tiles - 1) {
+            oa.last_tile(k_count - kt * kBK);
+            ob.last_tile(k_count - kt * kBK);
+        }
+        const auto ra = oa.rsrc(kt, k_tiles);
+        const auto rb = ob.rsrc(kt, k_tiles);
+#pragma unroll
+        for (int c = 0; c < NJ; ++c) ob.request(rb, tb, c);
+#pragma unroll
+        for (int c = 0; c < MI; ++c) oa.request(ra, ta, c);
+    };
+#pragma unroll
+    for (int i = 0; i < MI; ++i)
+#pragma unroll
+        for (int j = 0; j < NJ; ++j) acc[i][j] = float4v{0.f, 0.f, 0.f, 0.f};
+    auto pin = [&] {          // orders the accumulators' other uses against the written-out MFMAs
+#pragma unroll
+        for (int i = 0; i < MI; ++i)
+#pragma unroll
+            for (int j = 0; j < NJ; ++j) asm volatile("" : "+a"(acc[i][j]));
+    };
+    pin();
+    constexpr int kFree = 2 * MI;       // MFMAs into a tile until its last fragment of B, asked for at its start, is there in every wave
+    auto tile = [&](int kt, std::uint16_t* ca, std::uint16_t* cb, std::uint16_t* na, std::uint16_t* nb) {
+        if (kt + 2 == k_tiles - 1) {
+            oa.last_tile(k_count - (kt + 2) * kBK);
+            ob.last_tile(k_count - (kt + 2) * kBK);
+        }
+        const auto ra = oa.rsrc(kt + 2, k_tiles);
+        const auto rb = ob.rsrc(kt + 2, k_tiles);
+#pragma unroll
+        for (int j = 0; j < NJ; ++j)
+#pragma unroll
+            for (int i = 0; i < MI; ++i) {
+                const int slot = j * MI + i;
+                if (slot == kFree) {
+                    __builtin_amdgcn_s_waitcnt(0xC07F);         // lgkmcnt(0): the loads stay in flight
+                    asm volatile("s_barrier" ::: "memory");
+                }
+                mma<T>(acc[i][j], bf[0][j], af[0][i]);
+                if (slot == MI / 2) bf[1][NJ - 1] = ob.frag(cb, NJ - 1, 1);
+#pragma unroll
+                for (int c = 0; c < MI; ++c)
+                    if (kFree + (c * (S - kFree) * 7) / (8 * MI) == slot) af[1][c] = oa.frag(ca, c, 1);
+#pragma unroll
+                for (int c = 0; c < NJ; ++c)
+                    if (kFree + 2 + (c * (S - kFree - 2)) / NJ == slot) ob.request(rb, cb, c);
+                __builtin_amdgcn_sched_barrier(0);
+            }
+        meet<NJ>();                     // the next tile has landed, A's stage is read; B's requests are on their way
+#pragma unroll
+        for (int j = 0; j < NJ; ++j)
+#pragma unroll
+            for (int i = 0; i < MI; ++i) {
+                const int slot = j * MI + i;
+                mma<T>(acc[i][j], bf[1][j], af[1][i]);
+#pragma unroll
+                for (int c = 0; c < MI + NJ; ++c)
+                    if ((c * S * 7) / (8 * (MI + NJ)) == slot) {
+                        if (c < NJ) bf[0][c] = ob.frag(nb, c, 0);
+                        else        af[0][c - NJ] = oa.frag(na, c - NJ, 0);
+                    }
+                if (i == MI / 2 && j > 0) bf[1][j - 1] = ob.frag(nb, j - 1, 1);
+#pragma unroll
+                for (int c = 0; c < MI; ++c)
+                    if ((c * S) / MI == slot) oa.request(ra, ca, c);
+                __builtin_amdgcn_sched_barrier(0);
+            }
+    };
+    request_all(0, sa[0], sb[0]);
+    request_all(1, sa[1], sb[1]);
+    meet<MI + NJ>();
+#pragma unroll
+    for (int f = 0; f < NJ; ++f) {
+        bf[0][f] = ob.frag(sb[0], f, 0);
+        if (f < NJ - 1) bf[1][f] = ob.frag(sb[0], f, 1);
+    }
+#pragma unroll
+    for (int f = 0; f < MI; ++f) af[0][f] = oa.frag(sa[0], f, 0);
+    // (In whole turns of the stages, with one way out: a tile past the last one multiplies cleared stages.)
+    for (int kt = 0; kt < k_tiles; kt += 2) {
+        tile(kt, sa[0], sb[0], sa[1], sb[1]);
+        tile(kt + 1, sa[1], sb[1], sa[0], sb[0]);
+    }
+    asm volatile("s_nop 15\n\ts_nop 15" ::: "memory");      // the last products are on their way to the registers the epilogue reads
+    pin();
+    __builtin_amdgcn_s_waitcnt(0x0F70);         // vmcnt(0): no request may outlive the workgroup's LDS
+}
+
 // acc[i][j]: the B fragment is the instruction's first operand, so lane (l16 = lane % 16, kq = lane / 16)
 // holds row i*16 + l16 of the wave's rows and columns j*16 + 4*kq .. + 3 of its columns.
 // (The ST stages are separate arrays named at compile time: an LDS read waits for every direct load in flight
@@ -144,6 +253,10 @@ template <int W, bool R> struct Operand {
 template <typename T, int MI, int NJ, int ST, typename OA, typename OB>
 __device__ __forceinline__ void mainloop(OA& oa, OB& ob, int k_count, std::uint16_t* const (&sa)[ST], std::uint16_t* const (&sb)[ST],
                                          float4v (&acc)[MI][NJ]) {
+    if constexpr (ST == 2 && MI >= 6 && NJ >= 7) {
+        mainloop_paced<T, MI, NJ>(oa, ob, k_count, sa, sb, acc);
+        return;
+    }
     constexpr int C = MI + NJ;          // requests per wave and tile, and fragments per k-step
     constexpr int S = MI * NJ;          // MFMAs per k-step
     static_assert(ST >= 2 && (ST - 1) * C < 64, "the tiles in flight have to fit the load counter");
@@ -166,12 +279,6 @@ __device__ __forceinline__ void mainloop(OA& oa, OB& ob, int k_count, std::uint1
     auto read_frag = [&](const std::uint16_t* ta, const std::uint16_t* tb, int buf, int f, int ks) {
         if (f < MI) af[buf][f] = oa.frag(ta, f, ks);
         else        bf[buf][f - MI] = ob.frag(tb, f - MI, ks);
-    };
-    // this wave's part of the next tile has landed (those of `ahead` tiles after it may be under way), its reads of this one are done
-    auto meet = [](auto ahead) {
-        constexpr int n = decltype(ahead)::value * C;
-        __builtin_amdgcn_s_waitcnt(0x0070 | (n & 15) | ((n >> 4) << 14));     // vmcnt(n) lgkmcnt(0)
-        asm volatile("s_barrier" ::: "memory");     // (a fence of the compiler's own would wait for every direct load in flight)
     };
 #pragma unroll
     for (int i = 0; i < MI; ++i)
@@ -199,7 +306,7 @@ __device__ __forceinline__ void mainloop(OA& oa, OB& ob, int k_count, std::uint1
         const auto rb = ob.rsrc(kt + ST, k_tiles);
 #pragma unroll
         for (int ks = 0; ks < 2; ++ks) {
-            if (ks == 1) meet(std::integral_constant<int, ST - 2>{});
+            if (ks == 1) meet<(ST - 2) * C>();         // this wave's part of the next tile has landed, its reads of this one are done
 #pragma unroll
             for (int j = 0; j < NJ; ++j)
 #pragma unroll
@@ -217,7 +324,7 @@ __device__ __forceinline__ void mainloop(OA& oa, OB& ob, int k_count, std::uint1
     };
 #pragma unroll
     for (int u = 0; u < ST; ++u) request_all(u, sa[u], sb[u]);
-    meet(std::integral_constant<int, ST - 1>{});
+    meet<(ST - 1) * C>();
 #pragma unroll
     for (int f = 0; f < C; ++f) read_frag(sa[0], sb[0], 0, f, 0);
     // (In whole turns of the stages, with one way out: tiles past the last one multiply cleared stages.)
