@@ -348,9 +348,8 @@ template <int NJ> struct RowsOut {
     static constexpr int kChunks = 2 * NJ;
     __device__ static __forceinline__ int place(int row, int chunk) { return (chunk + (row & 15)) % kChunks; }
     // columns 4*kq .. + 3 of block j of `row`
-    __device__ static __forceinline__ void lay(lds_u16* out, int row, int j, int kq, u32x2 v) {
-        *(lds_u32x2*)(out + row * (16 * NJ) + place(row, 2 * j + (kq >> 1)) * 8 + (kq & 1) * 4) = v;
-    }
+    __device__ static __forceinline__ int at(int row, int j, int kq) { return row * (16 * NJ) + place(row, 2 * j + (kq >> 1)) * 8 + (kq & 1) * 4; }
+    __device__ static __forceinline__ void lay(lds_u16* out, int row, int j, int kq, u32x2 v) { *(lds_u32x2*)(out + at(row, j, kq)) = v; }
     __device__ static __forceinline__ u32x4 piece(lds_u16* out, int row, int chunk) {
         return *(lds_u32x4*)(out + row * (16 * NJ) + place(row, chunk) * 8);
     }

@@ -204,17 +204,18 @@ __device__ __forceinline__ void static_for(F&& f) {
     static_for_impl(std::make_integer_sequence<int, N>{}, static_cast<F&&>(f));
 }
 
-// A wave's queue of SwiGLU values that left the common tier (four of one lane per entry): laid over one
-// of the four tile stages once the contraction is done.
+// A wave's queue of SwiGLU values that left the common tier (four of one lane per entry): laid over the second half of one
+// of the four tile stages once the contraction is done (the first half is for the wave's rows on their way out).
 struct SwigluQueue {
-    static constexpr unsigned kEntries = 896;
+    static constexpr unsigned kEntries = 448;
     unsigned where[kEntries];       // (row in the tile) << 16 | column in the column unit
     flex::float4v gate[kEntries], up[kEntries];
 };
 __device__ __forceinline__ unsigned scalar_of(unsigned v) { return static_cast<unsigned>(__builtin_amdgcn_readfirstlane(static_cast<int>(v))); }
 constexpr int kTileBand = 8;        // m-tiles whose column units an XCD walks through together: they share the experts' weights in its L2
 constexpr int kStageElems = 256 * kBK;          // a stage of either operand: 256 rows of a k-tile
-static_assert(sizeof(SwigluQueue) <= kStageElems * 2, "a queue in a tile stage");
+constexpr int kQueueAt = 128 * 64;               // elements: the rows of a wave, 64 columns each
+static_assert(sizeof(SwigluQueue) <= (kStageElems - kQueueAt) * 2, "a queue in a tile stage");
 static_assert(kBK == kFormStep, "moe_forms.h");
 
 // The weight rows of a 256-column tile that come as two groups of 128: a wave's 128 rows of the LDS tile are 64 rows of
@@ -223,8 +224,8 @@ static_assert(kBK == kFormStep, "moe_forms.h");
 struct TwoGroups : flex::Operand<8, false> {
     const char* base2;
     struct Rsrc { __amdgpu_buffer_rsrc_t g[2]; };
-    // b, b2: row 0 of the groups; rows_left[g] rows of group g exist (<= 0: none)
-    __device__ __forceinline__ void aim(const std::uint16_t* b, const std::uint16_t* b2, long K, long rows_left, long second, int w) {
+    // b, b2: row 0 of the groups, of each of which rows_left exist (<= 0: none)
+    __device__ __forceinline__ void aim(const std::uint16_t* b, const std::uint16_t* b2, long K, long rows_left, int w) {
         const int lane = threadIdx.x & 63, l16 = lane & 15, kq = lane >> 4;
         base = reinterpret_cast<const char*>(b);
         base2 = reinterpret_cast<const char*>(b2);
@@ -233,7 +234,7 @@ struct TwoGroups : flex::Operand<8, false> {
 #pragma unroll
         for (int i = 0; i < 8; ++i) {
             const int r = (i * 4 + flex::wave_id()) * 8 + (lane >> 3);
-            const long row = (r >> 7) * 64 + ((r >> 4) & 3) * 16 + (r & 15) + ((i & 2) ? second : 0);
+            const long row = (r >> 7) * 64 + ((r >> 4) & 3) * 16 + (r & 15);
             off[i] = static_cast<std::uint32_t>(row * K * 2 + ((lane & 7) ^ (lane >> 3)) * 16);
         }
 #pragma unroll
@@ -389,30 +390,12 @@ __global__ __launch_bounds__(flex::kThreads, 1) void grouped_gemm_direct_kernel(
 #pragma unroll
         for (int ks = 0; ks < 2; ++ks) oa.fb[ks] = (w * 16 * W + l16) * kBK + ((ks * 4 + kq) ^ (l16 & 7)) * 8;
     };
-    TwoGroups ob;
+    typename std::conditional<kSwiglu, TwoGroups, flex::Operand<8, false>>::type ob;
     {
-        const long first = (static_cast<long>(e) * p.Nw + n0) * p.K;
-        ob.aim(p.b + first, p.b2 + first, p.K, p.Nw - n0, kSwiglu ? 0 : kBN, wn);
+        const long first = static_cast<long>(e) * p.Nw * p.K;
+        if constexpr (kSwiglu) ob.aim(p.b + first + n0 * p.K, p.b2 + first + n0 * p.K, p.K, p.Nw - n0, wn);
+        else                   ob.init(p.b + first, p.K, p.Nw, n0, 0, p.K, wn);
     }
-    // four values of one output row, narrowed
-    auto put4 = [&](long prow, long col, const flex::float4v v, bool nan_here) __attribute__((always_inline)) {
-        if (prow >= row_end || col >= p.N) return;
-        std::uint16_t o[4];
-#pragma unroll
-        for (int r = 0; r < 4; ++r) o[r] = __builtin_expect(nan_here, 0) ? El::from_f32(v[r]) : El::from_f32_finite(v[r]);
-        if (col + 3 < p.N) {        // (N is a multiple of 64 here and the rows are 16-byte aligned)
-            u32x2 w2;
-            w2[0] = o[0] | (static_cast<std::uint32_t>(o[1]) << 16);
-            w2[1] = o[2] | (static_cast<std::uint32_t>(o[3]) << 16);
-            *reinterpret_cast<u32x2*>(p.c + prow * p.N + col) = w2;
-        } else {
-#pragma unroll
-            for (int r = 0; r < 4; ++r)
-                if (col + r < p.N) p.c[prow * p.N + col + r] = o[r];
-        }
-    };
-    auto any_nan = [&](float probe) { return __builtin_amdgcn_ballot_w64(probe != probe) != 0; };
-
     // The tile with 32 MI of its rows: an expert's last tile takes the fewest that hold its rows, with the same sums in the
     // same order (64 rows about a third of a full tile's time, 128 rows two thirds).
     auto tile = [&](auto mi) __attribute__((always_inline)) {
@@ -433,7 +416,10 @@ __global__ __launch_bounds__(flex::kThreads, 1) void grouped_gemm_direct_kernel(
         int t = threadIdx.x;
         asm volatile("" : "+v"(t));
         const int lane = t & 63, wave = t >> 6, l16 = t & 15, kq = (t >> 4) & 3, wm = t >> 7, wn = (t >> 6) & 1;
-        SwigluQueue& q = *reinterpret_cast<SwigluQueue*>(wave == 0 ? a0 : (wave == 1 ? a1 : (wave == 2 ? b0 : b1)));
+        std::uint16_t* const stage = wave == 0 ? a0 : (wave == 1 ? a1 : (wave == 2 ? b0 : b1));
+        SwigluQueue& q = *reinterpret_cast<SwigluQueue*>(stage + kQueueAt);
+        flex::lds_u16* const out = (flex::lds_u16*)stage;
+        using Out = flex::RowsOut<4>;
         const unsigned long long lanes_below = (1ull << lane) - 1ull;
         unsigned queued = 0;      // uniform
         auto work_off = [&]() __attribute__((always_inline)) {
@@ -441,40 +427,25 @@ __global__ __launch_bounds__(flex::kThreads, 1) void grouped_gemm_direct_kernel(
                 const unsigned e = idx >> 2, r = idx & 3, where = q.where[e];
                 const float a0 = reinterpret_cast<const float*>(&q.gate[e])[r];
                 const float a1 = reinterpret_cast<const float*>(&q.up[e])[r];
-                const long qcol = n0 + (where & 0xFFFFu) + r;
-                const std::uint16_t v = swiglu_from_acc<T>(a0, a1);
-                if (qcol < p.N) p.c[(row0 + (where >> 16)) * p.N + qcol] = v;
+                out[where + r] = swiglu_from_acc<T>(a0, a1);
             }
             queued = 0;
         };
+        const long rows_left = row_end - row0 - wm * 16 * MI, cols_left = p.N - n0 - wn * 64;
         static_for<MI>([&](auto I) __attribute__((always_inline)) {
             constexpr int i = decltype(I)::value;
-            const int trow = wm * 16 * MI + i * 16 + l16;
-            const long prow = row0 + trow;
 #pragma unroll
             for (int jb = 0; jb < 4; ++jb) {
-                const int tcol = wn * 64 + jb * 16 + 4 * kq;
-                const long col = n0 + tcol;
-                const bool live = prow < row_end && col < p.N;
+                const int row = i * 16 + l16, at = Out::at(row, jb, kq);
+                const bool live = row < rows_left && jb * 16 + 4 * kq < cols_left;
                 std::uint16_t o[4];
                 const bool ok = swiglu4_common_tier<T>(acc[i][jb], acc[i][4 + jb], o);
-                if (live && ok) {
-                    if (col + 3 < p.N) {
-                        u32x2 w2;
-                        w2[0] = o[0] | (static_cast<std::uint32_t>(o[1]) << 16);
-                        w2[1] = o[2] | (static_cast<std::uint32_t>(o[3]) << 16);
-                        *reinterpret_cast<u32x2*>(p.c + prow * p.N + col) = w2;
-                    } else {
-#pragma unroll
-                        for (int r = 0; r < 4; ++r)
-                            if (col + r < p.N) p.c[prow * p.N + col + r] = o[r];
-                    }
-                }
+                *(flex::lds_u32x2*)(out + at) = u32x2{o[0] | (static_cast<std::uint32_t>(o[1]) << 16), o[2] | (static_cast<std::uint32_t>(o[3]) << 16)};
                 const unsigned long long left = __builtin_amdgcn_ballot_w64(live && !ok);
                 if (left != 0) {
                     if (live && !ok) {
                         const unsigned slot = queued + static_cast<unsigned>(__builtin_popcountll(left & lanes_below));
-                        q.where[slot] = (static_cast<unsigned>(trow) << 16) | static_cast<unsigned>(tcol);
+                        q.where[slot] = static_cast<unsigned>(at);
                         q.gate[slot] = acc[i][jb];
                         q.up[slot] = acc[i][4 + jb];
                     }
@@ -484,26 +455,25 @@ __global__ __launch_bounds__(flex::kThreads, 1) void grouped_gemm_direct_kernel(
             // a row block queues 4 x 64 entries at most
             if (i == MI - 1 || queued > SwigluQueue::kEntries - 256) work_off();
         });
+        flex::store_rows<T, MI, 4>(out, p.c + (row0 + wm * 16 * MI) * p.N + n0 + wn * 64, p.N, rows_left, cols_left, true, false);
         return;
-    }
-    // (row blocks as constants of the front end: the optimiser's unroller gives up on a loop of 128
-    // SwiGLU values with their exact tier, and the accumulators would move to scratch memory)
-    static_for<MI>([&](auto I) __attribute__((always_inline)) {
-        constexpr int i = decltype(I)::value;
-        const long prow = row0 + wm * 16 * MI + i * 16 + l16;
+    } else {
+        flex::lds_u16* const out = (flex::lds_u16*)(wave == 0 ? a0 : (wave == 1 ? a1 : (wave == 2 ? b0 : b1)));
+        __syncthreads();
         float probe = 0.f;
+        static_for<MI>([&](auto I) __attribute__((always_inline)) {
+            constexpr int i = decltype(I)::value;
 #pragma unroll
-        for (int j = 0; j < 8; ++j)
-#pragma unroll
-            for (int r = 0; r < 4; ++r) probe += acc[i][j][r];
-        const bool nan_here = any_nan(probe);
-#pragma unroll
-        for (int jb = 0; jb < 4; ++jb) {
-            const long col = n0 + wn * 64 + jb * 16 + 4 * kq;
-            put4(prow, col, acc[i][jb], nan_here);
-            put4(prow, col + kBN, acc[i][4 + jb], nan_here);
-        }
-    });
+            for (int j = 0; j < 8; ++j) {
+                const flex::float4v v = flex::in_turn<0>(acc[i][j]);
+                probe += (v[0] + v[1]) + (v[2] + v[3]);
+                flex::RowsOut<8>::lay(out, i * 16 + l16, j, kq, flex::pack4<T>(v));
+            }
+        });
+        const bool nan_here = __builtin_amdgcn_ballot_w64(probe != probe) != 0;      // (an infinity minus an infinity counts as well)
+        const long r0 = row0 + wm * 16 * MI, c0 = n0 + wn * 128;
+        flex::store_rows<T, MI, 8>(out, p.c + r0 * p.N + c0, p.N, row_end - r0, p.N - c0, true, nan_here);
+    }
     };      // tile
     const long rows = row_end - row0;
     if (rows > 192)      tile(std::integral_constant<int, 8>{});
@@ -549,7 +519,6 @@ template <int NJ> struct GateUp : flex::Operand<NJ, false> {
 
 template <typename T, bool kSwiglu, int MI, int NJ, int ST>
 __global__ __launch_bounds__(flex::kThreads, (MI * NJ >= 32 || ST * (MI + NJ) > 20 ? 1 : 2)) void grouped_tile_kernel(const FfnGemmParams p) {
-    using El = Elem<T>;
     using OA = flex::Operand<MI, false>;
     using OB = typename std::conditional<kSwiglu, GateUp<NJ>, flex::Operand<NJ, false>>::type;
     constexpr int kBM = 32 * MI, kCols = kSwiglu ? 16 * NJ : 32 * NJ;
@@ -609,16 +578,17 @@ __global__ __launch_bounds__(flex::kThreads, (MI * NJ >= 32 || ST * (MI + NJ) > 
     else if constexpr (ST == 3) flex::mainloop<T, MI, NJ, 3>(oa, ob, K, {a0, a1, a2}, {b0, b1, b2}, acc);
     else                        flex::mainloop<T, MI, NJ, 4>(oa, ob, K, {a0, a1, a2, a3}, {b0, b1, b2, b3}, acc);
 
-    auto put = [&](long prow, long col, const std::uint16_t (&o)[4]) __attribute__((always_inline)) {
-        if (prow >= row_end || col >= p.N) return;          // (N is a multiple of 64 here and the rows are 16-byte aligned)
-        u32x2 w2;
-        w2[0] = o[0] | (static_cast<std::uint32_t>(o[1]) << 16);
-        w2[1] = o[2] | (static_cast<std::uint32_t>(o[3]) << 16);
-        *reinterpret_cast<u32x2*>(p.c + prow * p.N + col) = w2;
-    };
+    // (N is a multiple of 64 here and the rows are 16-byte aligned)
+    constexpr int OJ = kSwiglu ? NJ / 2 : NJ;               // column blocks of the result per wave
+    using Out = flex::RowsOut<OJ>;
+    static_assert(16 * MI * 16 * OJ <= OA::kElems && 16 * MI * 16 * OJ <= OB::kElems, "a wave's rows in a stage");
+    flex::lds_u16* const out = wave == 0 ? (flex::lds_u16*)a0 : wave == 1 ? (flex::lds_u16*)a1 : wave == 2 ? (flex::lds_u16*)b0 : (flex::lds_u16*)b1;
+    const long r0 = row0 + wm * 16 * MI, c0 = n0 + wn * 16 * OJ;
+    __syncthreads();                                        // (no wave's requests are on their way to the stages)
+    float probe = 0.f;
 #pragma unroll
     for (int i = 0; i < MI; ++i) {
-        const long prow = row0 + wm * 16 * MI + i * 16 + l16;
+        const long prow = r0 + i * 16 + l16;
         if constexpr (kSwiglu) {
 #pragma unroll
             for (int j = 0; j < NJ / 2; ++j) {
@@ -636,24 +606,19 @@ __global__ __launch_bounds__(flex::kThreads, (MI * NJ >= 32 || ST * (MI + NJ) > 
                         o[3] = r == 3 ? v : o[3];
                     }
                 }
-                put(prow, n0 + wn * 8 * NJ + j * 16 + 4 * kq, o);
+                Out::lay(out, i * 16 + l16, j, kq, u32x2{o[0] | (static_cast<std::uint32_t>(o[1]) << 16), o[2] | (static_cast<std::uint32_t>(o[3]) << 16)});
             }
         } else {
-            float probe = 0.f;
-#pragma unroll
-            for (int j = 0; j < NJ; ++j)
-#pragma unroll
-                for (int r = 0; r < 4; ++r) probe += acc[i][j][r];
-            const bool nan_here = __builtin_amdgcn_ballot_w64(probe != probe) != 0;      // (an infinity minus an infinity counts as well)
 #pragma unroll
             for (int j = 0; j < NJ; ++j) {
-                std::uint16_t o[4];
-#pragma unroll
-                for (int r = 0; r < 4; ++r) o[r] = __builtin_expect(nan_here, 0) ? El::from_f32(acc[i][j][r]) : El::from_f32_finite(acc[i][j][r]);
-                put(prow, n0 + wn * 16 * NJ + j * 16 + 4 * kq, o);
+                const flex::float4v v = acc[i][j];
+                probe += (v[0] + v[1]) + (v[2] + v[3]);
+                Out::lay(out, i * 16 + l16, j, kq, flex::pack4<T>(v));
             }
         }
     }
+    const bool nan_here = !kSwiglu && __builtin_amdgcn_ballot_w64(probe != probe) != 0;      // (an infinity minus an infinity counts as well)
+    flex::store_rows<T, MI, OJ>(out, p.c + r0 * p.N + c0, p.N, row_end - r0, p.N - c0, true, nan_here);
 }
 
 // ---- few rows per expert (decode-time batches): the layer is bound by streaming every active
