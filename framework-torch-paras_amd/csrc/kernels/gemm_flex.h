@@ -20,7 +20,8 @@
 // What bounds it is the number of stages where a CU holds one or two workgroups of small tiles: a tile of 64 x 64 is 512
 // cycles of MFMA and LDS work, and its operands are 1500 cycles away.  Waits are for the next tile's requests only, the later ones stay
 // in flight (64 x 128 tiles, x W^T in bf16, two stages -> four: 1500 x 1024 x 4096 29.6 -> 23.1 us, 2040 x 1024 x 3584 29.5 -> 22.1,
-// 232 x 7168 x 2048 25.6 -> 17.8; 192 x 128, three stages: 1500 x 4096 x 4096 60.8 -> 50.2).  256-row tiles fill LDS with two stages and are
+// 232 x 7168 x 2048 25.6 -> 17.8; 192 x 128, three
+// stages: 1500 x 4096 x 4096 60.8 -> 50.2; four: with the weights from HBM 53.2 -> 52.0).  256-row tiles fill LDS with two stages and are
 // bound by the matrix cores' power.
 //
 // Direct loads fill LDS in lane order, so rows cannot be padded apart; instead the 16-byte chunks of a

@@ -160,26 +160,34 @@ __global__ __launch_bounds__(kThreads, (MI * NJ >= 32 || ST * (MI + NJ) > 20 ? 1
 template <typename T, bool AR, bool BR>
 void launch_tile(int tile, const Params& p, unsigned grid, hipStream_t s) {
     const dim3 g(grid), t(kThreads);
-    if constexpr (!AR && !BR) {          // (the permuted units of a tile that lies along its rows need widths of 64 or 128)
+    if constexpr (!AR) {                 // (a tile that lies along its rows permutes 32-byte units in groups of four: its width is 32 or a multiple of 64)
         switch (tile) {
-            case 12: hipLaunchKernelGGL((gemm_flex_kernel<T, 8, 7, 2, AR, BR>), g, t, 0, s, p); return;
-            case 13: hipLaunchKernelGGL((gemm_flex_kernel<T, 7, 7, 2, AR, BR>), g, t, 0, s, p); return;
-            case 14: hipLaunchKernelGGL((gemm_flex_kernel<T, 6, 7, 2, AR, BR>), g, t, 0, s, p); return;
+            case 13: hipLaunchKernelGGL((gemm_flex_kernel<T, 3, 4, 4, AR, BR>), g, t, 0, s, p); return;
+            case 14: hipLaunchKernelGGL((gemm_flex_kernel<T, 3, 4, 2, AR, BR>), g, t, 0, s, p); return;
+            case 15: hipLaunchKernelGGL((gemm_flex_kernel<T, 3, 2, 4, AR, BR>), g, t, 0, s, p); return;
+            case 16: hipLaunchKernelGGL((gemm_flex_kernel<T, 5, 4, 2, AR, BR>), g, t, 0, s, p); return;
+        }
+        if constexpr (!BR) {
+            switch (tile) {
+                case 17: hipLaunchKernelGGL((gemm_flex_kernel<T, 8, 7, 2, AR, BR>), g, t, 0, s, p); return;
+                case 18: hipLaunchKernelGGL((gemm_flex_kernel<T, 6, 7, 2, AR, BR>), g, t, 0, s, p); return;
+            }
         }
     }
     switch (tile) {
         case 0: hipLaunchKernelGGL((gemm_flex_kernel<T, 8, 8, 2, AR, BR>), g, t, 0, s, p); break;
         case 1: hipLaunchKernelGGL((gemm_flex_kernel<T, 6, 8, 2, AR, BR>), g, t, 0, s, p); break;
         case 2: hipLaunchKernelGGL((gemm_flex_kernel<T, 6, 6, 3, AR, BR>), g, t, 0, s, p); break;
-        case 3: hipLaunchKernelGGL((gemm_flex_kernel<T, 6, 4, 3, AR, BR>), g, t, 0, s, p); break;
+        case 3: hipLaunchKernelGGL((gemm_flex_kernel<T, 6, 4, 4, AR, BR>), g, t, 0, s, p); break;
         case 4: hipLaunchKernelGGL((gemm_flex_kernel<T, 4, 4, 2, AR, BR>), g, t, 0, s, p); break;
-        case 5: hipLaunchKernelGGL((gemm_flex_kernel<T, 4, 4, 3, AR, BR>), g, t, 0, s, p); break;
+        case 5: hipLaunchKernelGGL((gemm_flex_kernel<T, 4, 4, 4, AR, BR>), g, t, 0, s, p); break;
         case 6: hipLaunchKernelGGL((gemm_flex_kernel<T, 2, 4, 2, AR, BR>), g, t, 0, s, p); break;
         case 7: hipLaunchKernelGGL((gemm_flex_kernel<T, 2, 4, 4, AR, BR>), g, t, 0, s, p); break;
-        case 8: hipLaunchKernelGGL((gemm_flex_kernel<T, 2, 2, 2, AR, BR>), g, t, 0, s, p); break;
-        case 9: hipLaunchKernelGGL((gemm_flex_kernel<T, 2, 2, 3, AR, BR>), g, t, 0, s, p); break;
-        case 10: hipLaunchKernelGGL((gemm_flex_kernel<T, 2, 2, 4, AR, BR>), g, t, 0, s, p); break;
-        default: hipLaunchKernelGGL((gemm_flex_kernel<T, 1, 4, 4, AR, BR>), g, t, 0, s, p); break;
+        case 8: hipLaunchKernelGGL((gemm_flex_kernel<T, 2, 2, 3, AR, BR>), g, t, 0, s, p); break;
+        case 9: hipLaunchKernelGGL((gemm_flex_kernel<T, 2, 2, 4, AR, BR>), g, t, 0, s, p); break;
+        case 10: hipLaunchKernelGGL((gemm_flex_kernel<T, 4, 2, 3, AR, BR>), g, t, 0, s, p); break;
+        case 11: hipLaunchKernelGGL((gemm_flex_kernel<T, 1, 2, 4, AR, BR>), g, t, 0, s, p); break;
+        default: hipLaunchKernelGGL((gemm_flex_kernel<T, 6, 4, 2, AR, BR>), g, t, 0, s, p); break;
     }
 }
 

@@ -609,7 +609,15 @@ TILES = [(0, (6437, 2104, 528)), (0, (2483, 4712, 576)), (0, (7082, 792, 536)), 
          (0, (5661, 144, 200)), (0, (5700, 136, 64)), (0, (33, 72, 64)), (0, (36, 72, 208)), (0, (130, 5528, 64)), (0, (2709, 4520, 520)), (0, (2389, 4344, 520)), (0, (1189, 7000, 528)),
          (1, (1645, 7336, 520)), (1, (7683, 1160, 520)), (1, (1185, 5008, 528)), (1, (6805, 520, 528)), (1, (455, 6200, 64)), (1, (470, 6232, 136)), (1, (662, 5464, 64)),
          (1, (4246, 200, 200)), (1, (34, 72, 200)), (1, (134, 5528, 72)),
-         (2, (1544, 7272, 528)), (2, (4840, 1840, 528)), (2, (7192, 816, 520)), (2, (520, 6552, 536)), (2, (7016, 408, 64)), (2, (400, 7128, 144)), (2, (5576, 136, 64)), (2, (136, 5616, 64))]
+         (2, (1544, 7272, 528)), (2, (4840, 1840, 528)), (2, (7192, 816, 520)), (2, (520, 6552, 536)), (2, (7016, 408, 64)), (2, (400, 7128, 144)), (2, (5576, 136, 64)), (2, (136, 5616, 64)),
+         (0, (2321, 5616, 528)), (0, (4932, 2040, 560)), (0, (1180, 6544, 528)), (0, (2732, 2224, 64)), (0, (2544, 1160, 408)), (0, (1049, 1800, 64)), (0, (584, 2312, 408)),
+         (0, (737, 648, 64)), (0, (694, 712, 200)), (0, (1292, 1176, 64)), (0, (33, 72, 88)), (0, (3050, 3256, 64)), (0, (2514, 776, 392)), (0, (1155, 1672, 64)),
+         (0, (1220, 792, 64)), (0, (3006, 1296, 64)), (0, (5569, 2056, 528)), (0, (7152, 1168, 536)), (0, (644, 5392, 2040)),
+         (1, (5466, 2128, 536)), (1, (6224, 1360, 544)), (1, (3493, 2320, 520)), (1, (519, 7256, 920)), (1, (2543, 2440, 64)), (1, (2614, 1176, 392)), (1, (1409, 1360, 64)),
+         (1, (408, 4176, 400)), (1, (618, 784, 64)), (1, (898, 520, 208)), (1, (1102, 904, 64)), (1, (34, 72, 64)), (1, (2886, 3472, 64)), (1, (836, 2328, 208)),
+         (1, (1228, 1616, 64)), (1, (599, 1608, 200)), (1, (2705, 1456, 64)),
+         (2, (8152, 1360, 520)), (2, (1624, 5400, 520)), (2, (3656, 2224, 520)), (2, (2056, 1928, 672)), (2, (2904, 2104, 64)), (2, (2104, 984, 392)), (2, (1040, 1808, 64)),
+         (2, (784, 2384, 400)), (2, (792, 648, 64)), (2, (808, 600, 208)), (2, (904, 1104, 64)), (2, (40, 72, 64)), (2, (2552, 1584, 64))]
 
 
 @pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])
