@@ -99,6 +99,13 @@ template <> struct Elem<f16_t> {
     __device__ static __forceinline__ std::uint16_t from_f64(double v) { return f32_to_f16_bits_host(static_cast<float>(v)); }
 };
 
+// Values narrowed by the conversion instructions, NaNs among them, to what the host's types make of a NaN.
+template <typename T> __device__ __forceinline__ std::uint32_t host_nan(std::uint32_t two) {
+    constexpr std::uint32_t kInf = __is_same(T, bf16_t) ? 0x7F80u : 0x7C00u;
+    auto one = [](std::uint32_t v) { return (v & 0x7FFFu) <= kInf ? v : __is_same(T, bf16_t) ? 0x7FC0u : (v & 0x8000u) | 0x7E00u; };
+    return one(two & 0xFFFFu) | one(two >> 16) << 16;
+}
+
 // ---- wavefront reductions ----------------------------------------------------
 // Butterfly over all 64 lanes; every lane ends with the full result.
 template <typename T, typename Op>

@@ -13,6 +13,7 @@
 #include "core/device_context.h"
 #include "core/device_math.h"
 #include "core/status.h"
+#include "kernels/few_dims.h"
 #include "kernels/swiglu_math.h"
 
 namespace paras {
@@ -53,32 +54,14 @@ __device__ __forceinline__ void offsets(const Strided& s, long flat, bool small,
     *d_o = b;
 }
 
-// Up to four dimensions and 2^32 elements, in 112 bytes: a launch whose arguments take more costs the host 0.7 us more, 3.4 for 2.7 (a decode step's
-// new keys and values written into the cache).  Strides in elements of W.
-struct FewDims {
-    const void* src;
-    void* dst;
-    unsigned n;
-    int ndim;
-    unsigned sizes[4];
-    long src_strides[4], dst_strides[4];
-};
-static_assert(sizeof(FewDims) <= 112, "see above");
-bool few_dims(const Strided& s, long n) { return s.ndim <= 4 && n <= 0xFFFFFFFFL; }
-
-template <typename W>
-__global__ __launch_bounds__(kBlock) void copy_few_dims_kernel(const FewDims s) {
-    for (unsigned long i = static_cast<unsigned long>(blockIdx.x) * kBlock + threadIdx.x; i < s.n; i += static_cast<unsigned long>(gridDim.x) * kBlock) {
-        unsigned left = static_cast<unsigned>(i);
-        long a = 0, b = 0;
-        for (int d = s.ndim - 1; d >= 0; --d) {
-            const unsigned q = left / s.sizes[d], c = left - q * s.sizes[d];
-            left = q;
-            a += c * s.src_strides[d];
-            b += c * s.dst_strides[d];
-        }
-        static_cast<W*>(s.dst)[b] = static_cast<const W*>(s.src)[a];
-    }
+template <typename W, int ND>
+__global__ __launch_bounds__(kBlock) void copy_few_dims_kernel(const W* __restrict__ src, W* __restrict__ dst, unsigned n, unsigned s1, unsigned s2, unsigned s3, unsigned a0,
+                                                               unsigned a1, unsigned a2, unsigned a3, unsigned b0, unsigned b1, unsigned b2, unsigned b3) {
+    const unsigned i = blockIdx.x * kBlock + threadIdx.x;
+    if (i >= n) return;
+    std::uint64_t a, b;
+    place_of<ND>(i, s1, s2, s3, a0, a1, a2, a3, b0, b1, b2, b3, a, b);
+    dst[b] = src[a];
 }
 
 template <typename W>
@@ -332,6 +315,55 @@ __global__ __launch_bounds__(kBlock) void binary_strided_kernel(int op, const ty
     }
 }
 
+// Sum, difference or product of eight 16-bit pairs, alpha = 1, as binary_one gives it.  The operation is the kernel's: with all four of them and alpha in one kernel, eight
+// times over, its code is several KB that a small call waits for more than for its data.
+template <typename T, int kOp> __device__ __forceinline__ u32x4 binary_unit8(const u32x4 av, const u32x4 bv) {
+    using E = Elem<T>;
+    u32x4 o;
+    float probe = 0.f;                      // (an infinity minus an infinity counts as a NaN as well)
+#pragma unroll
+    for (int w = 0; w < 4; ++w) {
+        std::uint32_t two = 0;
+#pragma unroll
+        for (int h = 0; h < 2; ++h) {
+            const float x = E::to_f32(static_cast<std::uint16_t>(av[w] >> (16 * h))), y = E::to_f32(static_cast<std::uint16_t>(bv[w] >> (16 * h)));
+            const float r = kOp == kOpAdd ? x + y : kOp == kOpSub ? x - y : x * y;
+            probe += r;
+            two |= static_cast<std::uint32_t>(E::from_f32_finite(r)) << (16 * h);
+        }
+        o[w] = two;
+    }
+    if (__builtin_amdgcn_ballot_w64(probe != probe) != 0) {
+        asm volatile("" ::: "memory");      // not to be evaluated ahead of the branch
+#pragma unroll
+        for (int w = 0; w < 4; ++w) o[w] = host_nan<T>(o[w]);
+    }
+    return o;
+}
+
+// out and a dense, b dense (`brow` = nvec) or a row of `brow` vectors repeated.
+template <typename T, int kOp>
+__global__ __launch_bounds__(kBlock) void binary_unit_vec16_kernel(const std::uint16_t* __restrict__ a, const std::uint16_t* __restrict__ b, std::uint16_t* __restrict__ out,
+                                                                   unsigned nvec, unsigned brow) {
+    const unsigned i = blockIdx.x * kBlock + threadIdx.x;
+    if (i >= nvec) return;
+    const u32x4 av = load16_nt(a + i * 8UL);
+    const u32x4 bv = brow == nvec ? load16_nt(b + i * 8UL) : load16(b + i % brow * 8UL);
+    store16_nt(out + i * 8UL, binary_unit8<T, kOp>(av, bv));
+}
+
+// Rows of both operands in whole 16-byte pieces, anywhere (a projection's heads seen as [B, h, S, D], times cos / sin repeated over them); strides in pieces (Dims, place_of).
+template <typename T, int kOp, int ND>
+__global__ __launch_bounds__(kBlock) void binary_unit_rows_kernel(const std::uint16_t* __restrict__ a, const std::uint16_t* __restrict__ b, std::uint16_t* __restrict__ out,
+                                                                  unsigned nvec, unsigned s1, unsigned s2, unsigned s3, unsigned a0, unsigned a1, unsigned a2, unsigned b0,
+                                                                  unsigned b1, unsigned b2) {
+    const unsigned i = blockIdx.x * kBlock + threadIdx.x;
+    if (i >= nvec) return;
+    std::uint64_t ao, bo;
+    place_of<ND>(i, s1, s2, s3, a0, a1, a2, 1, b0, b1, b2, 1, ao, bo);
+    store16(out + i * 8UL, binary_unit8<T, kOp>(load16(a + ao * 8), load16(b + bo * 8)));
+}
+
 // 16-bit tensors, out and a dense, b dense or one value or one row repeated (period `brow` vectors,
 // 0 = one value): eight elements per thread
 template <typename T>
@@ -420,17 +452,19 @@ unsigned grid_for(long n) {
 
 template <typename W>
 void copy_same(const void* src, void* dst, long n, const Strided& s, hipStream_t st) {
-    const dim3 g(grid_for(n)), b(kBlock);
-    if (few_dims(s, n)) {
-        FewDims f{src, dst, static_cast<unsigned>(n), s.ndim, {}, {}, {}};
-        for (int d = 0; d < s.ndim; ++d) {
-            f.sizes[d] = static_cast<unsigned>(s.sizes[d]);
-            f.src_strides[d] = s.src_strides[d];
-            f.dst_strides[d] = s.dst_strides[d];
-        }
-        hipLaunchKernelGGL((copy_few_dims_kernel<W>), g, b, 0, st, f);
+    const dim3 b(kBlock);
+    Dims d;
+    if (few_dims(s.ndim, s.sizes, s.src_strides, s.dst_strides, n, 1, &d)) {
+        auto launch = [&](auto dims) {
+            hipLaunchKernelGGL((copy_few_dims_kernel<W, decltype(dims)::value>), dim3(static_cast<unsigned>((n + kBlock - 1) / kBlock)), b, 0, st, static_cast<const W*>(src),
+                               static_cast<W*>(dst), static_cast<unsigned>(n), d.sizes[1], d.sizes[2], d.sizes[3], d.a[0], d.a[1], d.a[2], d.a[3], d.b[0], d.b[1], d.b[2], d.b[3]);
+        };
+        if (s.ndim <= 2)      launch(std::integral_constant<int, 2>{});         // (fewer: in front there is one of size 1)
+        else if (s.ndim == 3) launch(std::integral_constant<int, 3>{});
+        else                  launch(std::integral_constant<int, 4>{});
         return;
     }
+    const dim3 g(grid_for(n));
     hipLaunchKernelGGL((copy_same_kernel<W>), g, b, 0, st, static_cast<const W*>(src), static_cast<W*>(dst), n, s);
 }
 
@@ -702,6 +736,21 @@ int paras_binary_strided(int op, const void* a, const void* b, void* out, int nd
     if (rc != PARAS_OK) return rc;
     const dim3 g(grid_for(n)), blk(kBlock);
     if (dtype == PARAS_BF16 || dtype == PARAS_F16) {
+        // (add, sub and mul with alpha = 1, what a model's layers ask for, on kernels of their own)
+        const bool unit = alpha == 1.0 && op != kOpDiv && n / 8 < (1L << 31);
+        auto by_op = [&](auto with) {
+            if (dtype == PARAS_BF16) {
+                if (op == kOpAdd)      with(bf16_t{}, std::integral_constant<int, kOpAdd>{});
+                else if (op == kOpSub) with(bf16_t{}, std::integral_constant<int, kOpSub>{});
+                else                   with(bf16_t{}, std::integral_constant<int, kOpMul>{});
+            } else {
+                if (op == kOpAdd)      with(f16_t{}, std::integral_constant<int, kOpAdd>{});
+                else if (op == kOpSub) with(f16_t{}, std::integral_constant<int, kOpSub>{});
+                else                   with(f16_t{}, std::integral_constant<int, kOpMul>{});
+            }
+        };
+        const auto *a16 = static_cast<const uint16_t*>(a), *b16 = static_cast<const uint16_t*>(b);
+        auto* out16 = static_cast<uint16_t*>(out);
         // a dense; b dense, a single value, or a trailing block repeated over the leading dims
         long brow = -1;
         if (s.ndim <= 1 && (s.ndim == 0 || s.src_strides[0] == 1)) {
@@ -715,7 +764,12 @@ int paras_binary_strided(int op, const void* a, const void* b, void* out, int nd
         if (brow >= 0 && aligned && n % 8 == 0 && brow % 8 == 0) {
             const long nvec = n / 8;
             const dim3 gv(static_cast<unsigned>((nvec + kBlock - 1) / kBlock));
-            if (dtype == PARAS_BF16)
+            if (unit && brow > 0)
+                by_op([&](auto t, auto o) {
+                    hipLaunchKernelGGL((binary_unit_vec16_kernel<decltype(t), decltype(o)::value>), gv, blk, 0, st, a16, b16, out16, static_cast<unsigned>(nvec),
+                                       static_cast<unsigned>(brow / 8));
+                });
+            else if (dtype == PARAS_BF16)
                 hipLaunchKernelGGL((binary_vec16_kernel<bf16_t>), gv, blk, 0, st, op, static_cast<const uint16_t*>(a), static_cast<const uint16_t*>(b), static_cast<uint16_t*>(out), nvec, brow / 8, alpha);
             else
                 hipLaunchKernelGGL((binary_vec16_kernel<f16_t>), gv, blk, 0, st, op, static_cast<const uint16_t*>(a), static_cast<const uint16_t*>(b), static_cast<uint16_t*>(out), nvec, brow / 8, alpha);
@@ -727,6 +781,21 @@ int paras_binary_strided(int op, const void* a, const void* b, void* out, int nd
         for (int d = 0; rows && d < last; ++d) rows = s.src_strides[d] % 8 == 0 && s.dst_strides[d] % 8 == 0;
         if (rows) {
             const unsigned nvec = static_cast<unsigned>(n / 8);
+            Dims d;
+            if (unit && few_dims(s.ndim, s.sizes, s.src_strides, s.dst_strides, n / 8, 8, &d)) {
+                const dim3 gv((nvec + kBlock - 1) / kBlock);
+                by_op([&](auto t, auto o) {
+                    auto launch = [&](auto dims) {
+                        hipLaunchKernelGGL((binary_unit_rows_kernel<decltype(t), decltype(o)::value, decltype(dims)::value>), gv, blk, 0, st, a16, b16, out16, nvec, d.sizes[1],
+                                           d.sizes[2], d.sizes[3], d.a[0], d.a[1], d.a[2], d.b[0], d.b[1], d.b[2]);
+                    };
+                    if (s.ndim == 2)      launch(std::integral_constant<int, 2>{});
+                    else if (s.ndim == 3) launch(std::integral_constant<int, 3>{});
+                    else                  launch(std::integral_constant<int, 4>{});
+                });
+                PARAS_HIP_TRY(hipGetLastError());
+                return PARAS_OK;
+            }
             auto launch = [&](auto dims) {
                 constexpr int ND = decltype(dims)::value;
                 BinaryRows<ND> v{static_cast<const uint16_t*>(a), static_cast<const uint16_t*>(b), static_cast<uint16_t*>(out), nvec, op, s.ndim, {}, {}, {}, alpha};

@@ -356,13 +356,6 @@ template <int NJ> struct RowsOut {
     }
 };
 
-// Values narrowed by the conversion instructions, NaNs among them, to what the host's types make of a NaN.
-template <typename T> __device__ __forceinline__ std::uint32_t host_nan(std::uint32_t two) {
-    constexpr std::uint32_t kInf = __is_same(T, bf16_t) ? 0x7F80u : 0x7C00u;
-    auto one = [](std::uint32_t v) { return (v & 0x7FFFu) <= kInf ? v : __is_same(T, bf16_t) ? 0x7FC0u : (v & 0x8000u) | 0x7E00u; };
-    return one(two & 0xFFFFu) | one(two >> 16) << 16;
-}
-
 // Rows of a wave, laid out by RowsOut, to memory: `dst` is its first row and column, `rows` x `cols` of it exist (<= 0: none), in rows of `ld` elements.
 // `wide`: those are whole aligned 16-byte pieces.  `nan_here`: NaNs may be among them.
 template <typename T, int MI, int NJ>

@@ -14,6 +14,7 @@
 #include "core/device_context.h"
 #include "core/device_math.h"
 #include "core/status.h"
+#include "kernels/few_dims.h"
 #include "kernels/swiglu_math.h"
 
 namespace paras {
@@ -262,20 +263,30 @@ __global__ __launch_bounds__(kBlock) void rotate_half_vec16(const std::uint16_t*
 }
 
 // The same for rows of D contiguous elements that lie anywhere: a projection's heads seen as [B, h, S, D], which were copied
-// together first (bf16 [1, 32, 1500, 128] and [1, 8, 1500, 128], transposed views: 22.3 us, 12.6 this way).
-// (Up to four dimensions: the arguments stay within 112 bytes; more cost a launch 0.7 us more of the host's time, 3.4 for 2.7.)
-template <int ND> struct RowDims {
+// together first (bf16 [1, 32, 1500, 128] and [1, 8, 1500, 128], transposed views: 22.3 us, 12.6 this way).  Strides in pieces (few_dims.h).
+template <int ND>
+__global__ __launch_bounds__(kBlock) void rotate_half_few_dims(const std::uint16_t* __restrict__ x, std::uint16_t* __restrict__ out, unsigned nvec, int backward, int nan_kind,
+                                                               unsigned s1, unsigned s2, unsigned s3, unsigned a0, unsigned a1, unsigned a2) {
+    const unsigned i = blockIdx.x * kBlock + threadIdx.x;
+    if (i >= nvec) return;
+    const unsigned half = s3 / 2, row = i / s3, col = i - row * s3;
+    const bool first = col < half;
+    std::uint64_t at, unused;
+    place_of<ND>(row * s3 + (first ? col + half : col - half), s1, s2, s3, a0, a1, a2, 1, 0, 0, 0, 0, at, unused);
+    u32x4 v = load16(x + at * 8);
+    rotate_piece(v, backward ? !first : first, nan_kind);
+    store16(out + i * 8UL, v);
+}
+struct RowDims {
     const std::uint16_t* x;
     std::uint16_t* out;
     unsigned nvec;
     int ndim;                    // the last dim is the row, in vectors
     int backward, nan_kind;
-    unsigned sizes[ND];
-    long strides[ND];            // elements
+    unsigned sizes[8];
+    long strides[8];             // elements
 };
-static_assert(sizeof(RowDims<4>) <= 112, "see above");
-template <int ND>
-__global__ __launch_bounds__(kBlock) void rotate_half_rows_vec16(const RowDims<ND> s) {
+__global__ __launch_bounds__(kBlock) void rotate_half_rows_vec16(const RowDims s) {
     const unsigned i = blockIdx.x * kBlock + threadIdx.x;
     if (i >= s.nvec) return;
     const unsigned half = s.sizes[s.ndim - 1] / 2;
@@ -445,7 +456,7 @@ int paras_rotate_half_strided(const void* x, void* out, int ndim, const int64_t*
     PARAS_REQUIRE(dtype == PARAS_BF16 || dtype == PARAS_F16, "paras_rotate_half_strided: 16-bit dtypes only");
     PARAS_REQUIRE(ndim >= 1 && ndim <= 8 && sizes && strides, "paras_rotate_half_strided: 1 to 8 dimensions");
     PARAS_REQUIRE(sizes[ndim - 1] % 16 == 0 && strides[ndim - 1] == 1, "paras_rotate_half_strided: rows of a multiple of 16 contiguous elements");
-    RowDims<8> d{};
+    RowDims d{};
     long n = 1;
     for (int k = 0; k < ndim; ++k) {
         PARAS_REQUIRE(sizes[k] >= 0 && (k == ndim - 1 || strides[k] % 8 == 0), "paras_rotate_half_strided: rows that begin on 16 bytes");
@@ -472,15 +483,19 @@ int paras_rotate_half_strided(const void* x, void* out, int ndim, const int64_t*
     d.backward = backward;
     d.nan_kind = dtype == PARAS_BF16 ? 1 : 2;
     const dim3 grid((d.nvec + kBlock - 1) / kBlock), block(kBlock);
-    if (d.ndim <= 4) {
-        RowDims<4> few{d.x, d.out, d.nvec, d.ndim, d.backward, d.nan_kind, {}, {}};
-        for (int k = 0; k < d.ndim; ++k) {
-            few.sizes[k] = d.sizes[k];
-            few.strides[k] = d.strides[k];
-        }
-        hipLaunchKernelGGL((rotate_half_rows_vec16<4>), grid, block, 0, s, few);
+    Dims few;
+    long row_sizes[8];
+    for (int k = 0; k < d.ndim; ++k) row_sizes[k] = k + 1 < d.ndim ? static_cast<long>(d.sizes[k]) : static_cast<long>(d.sizes[k]) * 8;
+    if (few_dims(d.ndim, row_sizes, d.strides, d.strides, n / 8, 8, &few)) {
+        auto launch = [&](auto dims) {
+            hipLaunchKernelGGL((rotate_half_few_dims<decltype(dims)::value>), grid, block, 0, s, d.x, d.out, d.nvec, backward, d.nan_kind, few.sizes[1], few.sizes[2],
+                               few.sizes[3], few.a[0], few.a[1], few.a[2]);
+        };
+        if (d.ndim <= 2)      launch(std::integral_constant<int, 2>{});             // (a lone row: in front of it a dimension of size 1)
+        else if (d.ndim == 3) launch(std::integral_constant<int, 3>{});
+        else                  launch(std::integral_constant<int, 4>{});
     } else {
-        hipLaunchKernelGGL((rotate_half_rows_vec16<8>), grid, block, 0, s, d);
+        hipLaunchKernelGGL(rotate_half_rows_vec16, grid, block, 0, s, d);
     }
     PARAS_HIP_TRY(hipGetLastError());
     return PARAS_OK;

@@ -1100,6 +1100,31 @@ def test_dimensions_that_do_not_fold(rank, device):
 
 
 @pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])
+def test_sums_differences_and_products_of_few_dimensions(dtype, device):
+    """Dense operands, a row or a block repeated, rows that lie anywhere in two to four dimensions, at one piece, a workgroup's pieces and some more; sizes with NaNs,
+    infinities that cancel, zeros of both signs, overflow and underflow.  The host's bits."""
+    def values(*shape):
+        t = torch.randn(shape) * torch.tensor([1.0, 1e-3, 3e4, 2.0]).repeat(shape[-1] // 4)
+        flat = t.reshape(-1)
+        for i, v in enumerate((math.nan, math.inf, -math.inf, 0.0, -0.0, -math.nan)):
+            flat[(7 * i + 3) % flat.numel()] = v
+        return t.to(dtype)
+    pairs = [(values(8), values(8)), (values(256 * 8), values(256 * 8).flip(0).contiguous()), (values(3, 257, 8), values(257, 8)), (values(5, 40), values(40)),
+             (values(9, 24).T.contiguous().T[:, :16], values(9, 16)), (values(2, 9, 6, 16).transpose(1, 2), values(9, 16)), (values(7, 48)[:, 8:24], values(7, 48)[:, 32:]),
+             (values(2, 9, 6, 16).transpose(1, 2), values(2, 6, 9, 16)), (values(3, 5, 7, 16).permute(2, 1, 0, 3), values(5, 3, 16)), (values(4, 1, 8).expand(4, 6, 8), values(6, 4, 8).transpose(0, 1))]
+    for a, b in pairs:
+        for fn, code in ((torch.add, O.OP_ADD), (torch.sub, O.OP_SUB), (torch.mul, O.OP_MUL)):
+            want = O.binary(code, a.contiguous(), b.expand(a.shape).contiguous())
+            assert_bit_exact(fn(a.to(device) if a.is_contiguous() else _view_on(a, device), b.to(device) if b.is_contiguous() else _view_on(b, device)).cpu(), want, f"{fn.__name__} {tuple(a.shape)}")
+
+
+def _view_on(t, device):
+    """t's values in the same layout on the device: a view into a copy of its storage."""
+    whole = torch.empty(0, dtype=t.dtype).set_(t.untyped_storage())
+    return whole.to(device).as_strided(t.size(), t.stride(), t.storage_offset())
+
+
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])
 def test_rotate_half_of_views_is_that_of_their_copies(dtype, device):
     """Rows that lie anywhere (a projection's heads, slices of a fused one, repeated rows, one dimension of many) are read where they
     are; NaNs, infinities and zeros keep the host's bits; views the kernel cannot read that way are copied as before."""
