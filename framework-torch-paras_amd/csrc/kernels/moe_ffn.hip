@@ -491,7 +491,7 @@ template <int NJ> struct GateUp : flex::Operand<NJ, false> {
     const char* base2;
     struct Rsrc { __amdgpu_buffer_rsrc_t g[2]; };
     __device__ __forceinline__ void aim(const std::uint16_t* gate, const std::uint16_t* up, long K, long rows_left, int w) {
-        static_assert(NJ % 4 == 0, "a request of 32 rows belongs to one of the two");
+        static_assert(NJ % 4 == 0 || NJ == 2, "the rows that a wave requests at once belong to one of the two");
         const int lane = threadIdx.x & 63, l16 = lane & 15, kq = lane >> 4;
         this->base = reinterpret_cast<const char*>(gate);
         base2 = reinterpret_cast<const char*>(up);
@@ -509,11 +509,12 @@ template <int NJ> struct GateUp : flex::Operand<NJ, false> {
     __device__ __forceinline__ Rsrc rsrc(int kt, int k_tiles) const {
         const long l = this->left - kt * this->step;
         const int n = static_cast<int>(static_cast<std::uint32_t>(l < 0 || kt >= k_tiles ? 0 : (l > flex::kMaxExtent ? flex::kMaxExtent : l)));
-        return {{__builtin_amdgcn_make_buffer_rsrc(const_cast<char*>(this->base + kt * this->step), 0, n, 0x00020000),
+        const char* first = NJ == 2 && flex::wave_id() >= 2 ? base2 : this->base;          // (NJ == 2: half of the waves' requests are for one matrix, half for the other)
+        return {{__builtin_amdgcn_make_buffer_rsrc(const_cast<char*>(first + kt * this->step), 0, n, 0x00020000),
                  __builtin_amdgcn_make_buffer_rsrc(const_cast<char*>(base2 + kt * this->step), 0, n, 0x00020000)}};
     }
     __device__ __forceinline__ void request(const Rsrc& r, std::uint16_t* tile, int i) const {
-        flex::Operand<NJ, false>::request((2 * i) % NJ >= NJ / 2 ? r.g[1] : r.g[0], tile, i);
+        flex::Operand<NJ, false>::request(NJ > 2 && (2 * i) % NJ >= NJ / 2 ? r.g[1] : r.g[0], tile, i);
     }
 };
 
@@ -820,7 +821,7 @@ int run_ffn_any(const void* x, const void* w_gate, const void* w_up, const void*
 
 template <typename T, bool kSwiglu>
 void launch_form(int form, FfnGemmParams g, hipStream_t s) {
-    const GroupedForm f = kForms[form];
+    const GroupedForm f = kAllForms[form];
     const long cols = kSwiglu ? f.n / 2 : f.n;
     g.mt_total = static_cast<int>((g.R + f.m - 1) / f.m + (g.R < g.E ? g.R : g.E));      // an upper bound: workgroups past the last tile return
     g.n_units = static_cast<int>((g.N + cols - 1) / cols);
@@ -832,6 +833,20 @@ void launch_form(int form, FfnGemmParams g, hipStream_t s) {
         case 2: hipLaunchKernelGGL((grouped_tile_kernel<T, kSwiglu, 2, 4, 2>), grid, block, 0, s, g); break;
         case 3: hipLaunchKernelGGL((grouped_tile_kernel<T, kSwiglu, 2, 4, 4>), grid, block, 0, s, g); break;
         case 4: hipLaunchKernelGGL((grouped_tile_kernel<T, kSwiglu, 1, 4, 4>), grid, block, 0, s, g); break;
+        case 7: hipLaunchKernelGGL((grouped_tile_kernel<T, kSwiglu, 1, 2, 4>), grid, block, 0, s, g); break;
+        case 8: hipLaunchKernelGGL((grouped_tile_kernel<T, kSwiglu, 2, 2, 4>), grid, block, 0, s, g); break;
+        case 9: hipLaunchKernelGGL((grouped_tile_kernel<T, kSwiglu, 3, 2, 4>), grid, block, 0, s, g); break;
+        case 10: hipLaunchKernelGGL((grouped_tile_kernel<T, kSwiglu, 3, 4, 2>), grid, block, 0, s, g); break;
+        case 11: hipLaunchKernelGGL((grouped_tile_kernel<T, kSwiglu, 6, 4, 2>), grid, block, 0, s, g); break;
+        case 12:
+            if constexpr (kSwiglu) hipLaunchKernelGGL((grouped_tile_kernel<T, kSwiglu, 5, 4, 2>), grid, block, 0, s, g);
+            break;
+        case 13:
+            if constexpr (!kSwiglu) hipLaunchKernelGGL((grouped_tile_kernel<T, kSwiglu, 6, 8, 2>), grid, block, 0, s, g);
+            break;
+        case 14:
+            if constexpr (!kSwiglu) hipLaunchKernelGGL((grouped_tile_kernel<T, kSwiglu, 4, 8, 3>), grid, block, 0, s, g);
+            break;
         default: {
             g.ngt = form == kOneByOne ? 1 : 0;
             const long wgs = form == kOneByOne ? (static_cast<long>(g.mt_total) * g.n_units + 7) / 8 * 8 : (supers + 7) / 8 * 8 * kSuperM * kSuperN;
@@ -874,7 +889,7 @@ int run_ffn_tiles(const void* x, const void* w_gate, const void* w_up, const voi
     g1.a_bytes = T_ * H * 2;
     g1.K = H; g1.N = I; g1.Nw = I; g1.R = R; g1.E = E; g1.k = k;
     division_by(static_cast<unsigned>(k), &g1.div_m, &g1.div_s);
-    if (by_form) launch_form<T, true>(grouped_form(true, E, R, I, H), g1, s);
+    if (by_form) launch_form<T, true>(grouped_tiles(true, E, R, I, H), g1, s);
     else         launch_register_staged<T, true>(g1, s);
     PARAS_HIP_TRY(hipGetLastError());
 
@@ -886,7 +901,7 @@ int run_ffn_tiles(const void* x, const void* w_gate, const void* w_up, const voi
     g2.order = nullptr;
     g2.offsets = offsets;
     g2.K = I; g2.N = H; g2.Nw = H; g2.R = R; g2.E = E; g2.k = k;
-    if (by_form) launch_form<T, false>(grouped_form(false, E, R, H, I), g2, s);
+    if (by_form) launch_form<T, false>(grouped_tiles(false, E, R, H, I), g2, s);
     else         launch_register_staged<T, false>(g2, s);
     PARAS_HIP_TRY(hipGetLastError());
 

@@ -79,4 +79,75 @@ inline int grouped_form(bool swiglu, long E, long R, long N, long K) {
     return best;
 }
 
+// All tiles of the grouped products: those above in their order, then what grouped_tile_kernel has besides.  (A time of zero: not for that product.)
+inline constexpr GroupedForm kAllForms[] = {{128, 128, 2, 2, {0.519, 0.476}, {0.607, 0.611}}, {128, 128, 3, 1, {0.312, 0.306}, {0.164, 0.131}},
+                                             {64, 128, 2, 3, {0.594, 0.789}, {0.472, 0.526}}, {64, 128, 4, 1, {0.183, 0.227}, {0.215, 0.251}},
+                                             {32, 128, 4, 2, {0.372, 0.042}, {0.218, 0.461}}, {256, 256, 2, 1, {0.614, 0.812}, {0.539, 0.137}},
+                                             {256, 256, 2, 1, {0.767, 0.288}, {0.403, 0.706}}, {32, 64, 4, 3, {0.256, 0.409}, {0.211, 0.204}},
+                                             {64, 64, 4, 2, {0.229, 0.318}, {0.211, 0.224}}, {96, 64, 4, 2, {0.201, 0.181}, {0.286, 0.377}},
+                                             {96, 128, 2, 2, {0.478, 0.601}, {0.545, 0.547}}, {192, 128, 2, 2, {0.453, 0.788}, {0.737, 0.663}},
+                                             {160, 128, 2, 2, {0.696, 0.0}, {0.575, 0.0}}, {192, 256, 2, 1, {0.0, 0.636}, {0.0, 0.574}},
+                                             {128, 256, 3, 1, {0.0, 0.533}, {0.0, 0.223}}};
+constexpr int kAllFormCount = sizeof(kAllForms) / sizeof(kAllForms[0]);
+
+// Tiles of m rows, as tiles_256; where an expert fills more than six, half a tile each is what is lost.
+inline double tiles_of_rows(long E, long R, int m) {
+    const double rows = static_cast<double>(R) / E;
+    if (rows > 6.0 * m) return E * (rows / m + 0.5);
+    const double spread = std::sqrt(2.0 * rows);
+    double n = 1.0 - std::exp(-rows);
+    for (double j = m; j < rows + 3 * spread; j += m) n += 0.5 * std::erfc((j + 0.5 - rows) / spread);
+    return E * n;
+}
+
+// The tiles that a product runs on: the least estimated time, as above, of all forms, of grouped_gemm_direct_kernel's two dealings the one that grouped_form
+// takes, and none where it takes neither.  The number of an expert's tiles is a matter of chance, and one tile more can be a round more: the time is a mean over the
+// expected number and half a tile per square root of an expert less and more.  grouped_form's own choice stays unless another one is estimated to be a tenth (gate-up) or a
+// sixteenth (down) faster.  Fitted to 50000 timings of 1806 layers (4 to 64 experts, 8 to 16384 routed rows, H 512 to 4096, I 512 to
+// 14336, weights from HBM): 2.0 % (gate-up) and 2.3 % (down) of a layer's time faster in the mean than grouped_form alone, 7.5 % and 4.2 % where the choice is another one; 7
+// and 8 layers are more than 4 % slower, of what was measured another 1.9 % and 0.9 % could be had.  What the further forms bring.  32 x 64 with four stages, three to a CU, is for
+// products whose tiles are too few for 256 CUs: down of 230 tokens, top-2, 8 experts, 640 x 4096, 26.8 us on 32 x 128, 19.5.  192 x 128 and 160 x 128 with two stages,
+// two to a CU, hide each other's SwiGLU and stores, which 256 x 256 tiles do one CU at a time, and waste less of an expert's last tile: gate-up of 2167 tokens,
+// top-4, 32 experts, 1856 x 1280, 181 us on 256 x 256, 166.  192 x 256 and 128 x 256: down of 1156 tokens, top-2, 8 experts, 3520 x 14272, and of 910,
+// 3008 x 10496 (with the gate-up product's change layers 1201 -> 860 and 596 -> 467).  Where the tiles are about as many as the CUs hold, chance decides: gate-up of 3221 tokens, top-2, 8
+// experts, 1088 x 832 came to 520 tiles of 192 x 128 for 512 places, layer 75 -> 93.
+inline int grouped_tiles(bool swiglu, long E, long R, long N, long K) {
+    const int w = swiglu ? 0 : 1, base = grouped_form(swiglu, E, R, N, K);
+    const double start = swiglu ? 1.460 : 0.634, store = swiglu ? 30.08 : 7.54, beside = swiglu ? 0.586 : 0.601;          // us; `beside`: with other workgroups on the CU
+    const double from_memory = swiglu ? 20.11e6 : 22595.85e6, from_caches = swiglu ? 30.70e6 : 458704.40e6;                 // bytes per us
+    const double supers = swiglu ? 0.995 : 0.838, one_by_one = swiglu ? 1.010 : 0.666, ahead = swiglu ? 0.90 : 0.94;
+    const double memory = static_cast<double>(R < E ? R : E) * N * K * (swiglu ? 4.0 : 2.0) / from_memory, chance = 0.5 * std::sqrt(static_cast<double>(E));
+    auto fourth = [](double v) { return v * v * v * v; };
+    double by_rows[9] = {};           // row tiles of 32, 64 ... 256
+    int best = 0;
+    double best_cost = 1e300;
+    for (int f = 0; f < kAllFormCount; ++f) {
+        const GroupedForm& t = kAllForms[f];
+        const bool direct = f == kDirectForm || f == kOneByOne;
+        if (t.step[w] == 0.0 || (direct && f != base)) continue;
+        const long cols = swiglu ? t.n / 2 : t.n, units = (N + cols - 1) / cols, k_tiles = K / kFormStep, turns = (k_tiles + t.stages - 1) / t.stages * t.stages;
+        double& m_tiles = by_rows[t.m / 32];
+        if (m_tiles == 0.0) m_tiles = tiles_of_rows(E, R, t.m);
+        const double stores = store * t.m * cols / 65536.0 * (t.per_cu > 1 ? beside : 1.0), slots = 256.0 * t.per_cu;
+        auto round = [&](double n) {
+            const double c = t.step[w] * n / t.per_cu;
+            return turns * (c > t.lat[w] ? c : t.lat[w]) + start + stores * n;
+        };
+        const double one_round = round(t.per_cu);
+        auto rounds = [&](double m) {
+            if (f == kDirectForm) return supers * std::ceil(std::ceil(m / kSuperM) * std::ceil(static_cast<double>(units) / kSuperN) / 8) * one_round;
+            if (f == kOneByOne) return one_by_one * std::ceil(m * units / 256) * one_round;
+            const double full = std::floor(m * units / slots), rest = std::ceil((m * units - full * slots) / 256.0);
+            return full * one_round + (rest > 0 ? round(rest) : 0.0);
+        };
+        const double us = 0.25 * rounds(m_tiles > 1.0 + chance ? m_tiles - chance : 1.0) + 0.5 * rounds(m_tiles) + 0.25 * rounds(m_tiles + chance);
+        const double cost = (fourth(us) + fourth(memory) + fourth(m_tiles * units * (t.m + t.n) * K * 2.0 / from_caches)) * (f == base ? fourth(ahead) : 1.0);
+        if (cost < best_cost) {
+            best_cost = cost;
+            best = f;
+        }
+    }
+    return best;
+}
+
 }  // namespace paras

@@ -461,10 +461,14 @@ TILE_SHAPES = [(1843, 70, 6, 192, 256), (2055, 32, 4, 192, 192), (1188, 70, 6, 1
                (727, 70, 6, 576, 192), (163, 70, 6, 192, 128), (159, 70, 6, 320, 768), (2778, 70, 6, 960, 448), (45, 4, 1, 256, 320), (2769, 70, 6, 192, 512),
                (2756, 4, 1, 768, 320), (2978, 8, 2, 960, 128), (2581, 8, 2, 320, 256), (2861, 32, 4, 960, 128), (1834, 32, 4, 192, 896),
                (2006, 70, 6, 704, 384), (1796, 32, 4, 1472, 576)]
+# (with those, every form of grouped_tiles that the gate-up and that the down product have)
+FURTHER_TILE_SHAPES = [(43, 70, 6, 192, 384), (63, 8, 2, 64, 1024), (288, 8, 2, 64, 1152), (577, 32, 4, 576, 64), (587, 4, 1, 832, 1216), (828, 4, 1, 1344, 1472), (858, 4, 1, 1536, 448),
+                       (1299, 4, 1, 1536, 576), (1828, 32, 4, 960, 768), (2548, 4, 1, 1472, 1344), (2604, 32, 4, 960, 512), (2757, 8, 2, 960, 1024), (46, 70, 6, 896, 192), (287, 8, 2, 64, 1408),
+                       (1109, 32, 4, 1088, 960), (1967, 8, 2, 1408, 960)]
 
 
 @pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])
-@pytest.mark.parametrize("shape", TILE_SHAPES)
+@pytest.mark.parametrize("shape", TILE_SHAPES + FURTHER_TILE_SHAPES)
 def test_ffn_tiles_of_every_form(shape, dtype):
     """Experts of a few to a few hundred rows, uneven: one that most tokens choose, some that nobody does, more experts than a
     wave has lanes; gates far from zero (SwiGLU's exact tier), a NaN, an infinite and an all-zero token.  Sampled tokens against the

@@ -37,3 +37,22 @@ def test_every_form_is_chosen_by_a_shape_of_the_gpu_tests(form):
     chosen = [(form(1, E, T * k, I, H), form(0, E, T * k, H, I)) for T, E, k, H, I in TILE_SHAPES]
     assert {f for pair in chosen for f in pair} == set(range(7)), chosen
     assert ONE_BY_ONE in {g for g, _ in chosen} and ONE_BY_ONE in {d for _, d in chosen}, chosen
+
+
+def test_every_tile_of_both_products_is_chosen_by_a_shape_of_the_gpu_tests(tmp_path):
+    """TILE_SHAPES and FURTHER_TILE_SHAPES of test_gpu_moe.py reach all that grouped_tiles chooses among, and sizes from one row to the largest get a form that the product has."""
+    from test_gpu_moe import FURTHER_TILE_SHAPES, TILE_SHAPES
+    (tmp_path / "tiles.cpp").write_text('#include "kernels/moe_forms.h"\n'
+                                        'extern "C" int tiles(int swiglu, long E, long R, long N, long K) { return paras::grouped_tiles(swiglu != 0, E, R, N, K); }\n'
+                                        'extern "C" int has(int swiglu, int form) { return form >= 0 && form < paras::kAllFormCount && paras::kAllForms[form].step[swiglu ? 0 : 1] > 0; }\n')
+    subprocess.run(["g++", "-O2", "-std=c++17", "-shared", "-fPIC", f"-I{capi.PKG / 'csrc'}", str(tmp_path / "tiles.cpp"), "-o", str(tmp_path / "tiles.so")], check=True)
+    lib = C.CDLL(str(tmp_path / "tiles.so"))
+    lib.tiles.argtypes = [C.c_int] + [C.c_long] * 4
+    shapes = TILE_SHAPES + FURTHER_TILE_SHAPES
+    assert {lib.tiles(1, E, T * k, I, H) for T, E, k, H, I in shapes} >= {f for f in range(15) if lib.has(1, f)}
+    assert {lib.tiles(0, E, T * k, H, I) for T, E, k, H, I in shapes} >= {f for f in range(15) if lib.has(0, f)}
+    for E in (1, 3, 64, 4096):
+        for R in (1, 31, 32, 33, 1000, 16384, 1 << 24):
+            for N, K in ((64, 64), (64, 14336), (14336, 64), (4096, 4096), (1 << 20, 1 << 20)):
+                for swiglu in (0, 1):
+                    assert lib.has(swiglu, lib.tiles(swiglu, E, R, N, K)), (swiglu, E, R, N, K)
