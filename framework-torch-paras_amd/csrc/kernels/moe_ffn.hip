@@ -701,33 +701,54 @@ __global__ __launch_bounds__(stream::kThreads, 4) void grouped_few_rows_kernel(c
     else                 few_rows<T, kSwiglu, 4>(p, e, row_lo, row_hi, lds, kept);
 }
 
-// out[t, :] = T( sum_slot T( y[inv[t*k+slot], :] * T(w[t, slot]) ) ), 8 columns per lane.
-template <typename T>
-__global__ __launch_bounds__(kThreads) void moe_combine_kernel(const std::uint16_t* __restrict__ y,
-                                                              const float* __restrict__ topw,
-                                                              const long* __restrict__ inv_order,
-                                                              std::uint16_t* __restrict__ out, long T_, int k, long H) {
+// out[t, :] = T( sum_slot T( y[inv[t*k+slot], :] * T(w[t, slot]) ) ), 8 columns per lane, the sum in double.  KC slots at a time, which divides k: their places and
+// weights are asked for together, and then their rows, so a lane waits for two trips to memory and not for two per slot.  (A product of two 16-bit values is
+// exact in fp32, or rounded as from double; so is the sum of two.  One slot after the other with 64-bit divisions for the place, in double throughout,
+// and this: 8192 tokens, top-2, 4096 columns 44.0 and 36.5 us; 555, top-6, 2496 9.2 and 7.0; 2344, top-1, 1088 5.3 and 4.5.)
+template <typename T, int KC, bool kAll>
+__global__ __launch_bounds__(kThreads) void moe_combine_kernel(const std::uint16_t* __restrict__ y, const float* __restrict__ topw, const long* __restrict__ inv_order,
+                                                              std::uint16_t* __restrict__ out, unsigned total, unsigned hv, int k) {
     using El = Elem<T>;
-    const long hv = H / 8;
-    const long total = T_ * hv;
-    for (long i = static_cast<long>(blockIdx.x) * kThreads + threadIdx.x; i < total;
-         i += static_cast<long>(gridDim.x) * kThreads) {
-        const long t = i / hv, c = (i % hv) * 8;
-        double acc[8] = {0, 0, 0, 0, 0, 0, 0, 0};
-        for (int s = 0; s < k; ++s) {
-            const long prow = inv_order[t * k + s];
-            const double w = El::to_f64(El::from_f32(topw[t * k + s]));  // w.to(T)
-            const u32x4 v = load16(y + prow * H + c);
-            const std::uint16_t* ve = reinterpret_cast<const std::uint16_t*>(&v);
+    typedef typename std::conditional<(kAll && KC <= 2), float, double>::type sum_t;
+    for (unsigned i = blockIdx.x * kThreads + threadIdx.x; i < total; i += gridDim.x * kThreads) {
+        const unsigned t = i / hv, c = i - t * hv;
+        const long first = static_cast<long>(t) * k;
+        sum_t acc[8] = {};
+        for (int s = 0; s < (kAll ? KC : k); s += KC) {
+            float w[KC];
+            u32x4 v[KC];
 #pragma unroll
-            for (int j = 0; j < 8; ++j) acc[j] += El::to_f64(El::from_f64(El::to_f64(ve[j]) * w));
+            for (int u = 0; u < KC; ++u) w[u] = El::to_f32(El::from_f32(topw[first + s + u]));        // w.to(T)
+#pragma unroll
+            for (int u = 0; u < KC; ++u) v[u] = load16(y + (inv_order[first + s + u] * hv + c) * 8);
+#pragma unroll
+            for (int u = 0; u < KC; ++u)
+#pragma unroll
+                for (int j = 0; j < 8; ++j) acc[j] += static_cast<sum_t>(El::to_f32(El::from_f32(El::to_f32(static_cast<std::uint16_t>(v[u][j >> 1] >> (16 * (j & 1)))) * w[u])));
         }
         u32x4 o;
-        std::uint16_t* oe = reinterpret_cast<std::uint16_t*>(&o);
 #pragma unroll
-        for (int j = 0; j < 8; ++j) oe[j] = El::from_f64(acc[j]);
-        store16(out + t * H + c, o);
+        for (int j = 0; j < 4; ++j)
+            o[j] = El::from_f32(static_cast<float>(acc[2 * j])) | static_cast<std::uint32_t>(El::from_f32(static_cast<float>(acc[2 * j + 1]))) << 16;
+        store16(out + static_cast<std::uint64_t>(i) * 8, o);
     }
+}
+
+template <typename T>
+void launch_combine(const std::uint16_t* y, const float* topw, const long* inv_order, void* out, long tokens, int k, long H, hipStream_t s) {
+    const unsigned hv = static_cast<unsigned>(H / 8), total = static_cast<unsigned>(tokens * (H / 8));          // (paras_moe_ffn: T H < 2^32)
+    const unsigned blocks = (total + kThreads - 1) / kThreads;
+    auto launch = [&](auto slots, auto all) {
+        hipLaunchKernelGGL((moe_combine_kernel<T, decltype(slots)::value, decltype(all)::value>), dim3(blocks), dim3(kThreads), 0, s, y, topw, inv_order,
+                           static_cast<std::uint16_t*>(out), total, hv, k);
+    };
+    if (k == 1)          launch(std::integral_constant<int, 1>{}, std::true_type{});
+    else if (k == 2)     launch(std::integral_constant<int, 2>{}, std::true_type{});
+    else if (k == 4)     launch(std::integral_constant<int, 4>{}, std::true_type{});
+    else if (k % 4 == 0) launch(std::integral_constant<int, 4>{}, std::false_type{});
+    else if (k % 3 == 0) launch(std::integral_constant<int, 3>{}, std::false_type{});
+    else if (k % 2 == 0) launch(std::integral_constant<int, 2>{}, std::false_type{});
+    else                 launch(std::integral_constant<int, 1>{}, std::false_type{});
 }
 
 // ---- sizes the MFMA tiles do not take (hidden or intermediate size not a multiple of 64) -------
@@ -905,11 +926,7 @@ int run_ffn_tiles(const void* x, const void* w_gate, const void* w_up, const voi
     else         launch_register_staged<T, false>(g2, s);
     PARAS_HIP_TRY(hipGetLastError());
 
-    const long total = T_ * (H / 8);
-    long blocks = (total + kThreads - 1) / kThreads;
-    if (blocks > 256L * 16) blocks = 256L * 16;
-    hipLaunchKernelGGL((moe_combine_kernel<T>), dim3(static_cast<unsigned>(blocks)), dim3(kThreads), 0, s, y, topw,
-                       inv_order, static_cast<std::uint16_t*>(out), T_, k, H);
+    launch_combine<T>(y, topw, inv_order, out, T_, k, H, s);
     PARAS_HIP_TRY(hipGetLastError());
     return PARAS_OK;
 }
@@ -950,11 +967,7 @@ int run_ffn_few_rows(const void* x, const void* w_gate, const void* w_up, const 
     hipLaunchKernelGGL((grouped_few_rows_kernel<T, false>), dim3(static_cast<unsigned>((H / 16 + each - 1) / each), static_cast<unsigned>(E)),
                        dim3(stream::kThreads), 0, s, g2);
     PARAS_HIP_TRY(hipGetLastError());
-    const long total = T_ * (H / 8);
-    long blocks = (total + kThreads - 1) / kThreads;
-    if (blocks > 256L * 16) blocks = 256L * 16;
-    hipLaunchKernelGGL((moe_combine_kernel<T>), dim3(static_cast<unsigned>(blocks)), dim3(kThreads), 0, s, y, topw,
-                       inv_order, static_cast<std::uint16_t*>(out), T_, k, H);
+    launch_combine<T>(y, topw, inv_order, out, T_, k, H, s);
     PARAS_HIP_TRY(hipGetLastError());
     return PARAS_OK;
 }
