@@ -429,7 +429,11 @@ bool few_rows_by_tiles(long M, long N, long batch) {
 // eight of 128 x 512 x 64 4.1 / 4.3; two of 100 x 128 x 128 4.0 / 4.0, 128 of 33 x 512 x 64 6.0 / 6.0.  Where the tiles want the contraction in parts and the caller has no workspace for
 // them, and for paras_gemm_nt, the few-row kernels stay up to kSkinnyMaxM rows.
 bool few_rows_up_to(long M, long N, long K, long batch, bool parts_or_whole) {
-    if (M <= kFewRowsM) return true;
+    // (17 to 32 rows read four times the activations that 8 do, for each block of weight rows: over a long contraction, and where the weight rows are few, 32 x 64 and
+    // 64 x 64 tiles in parts are ahead.  This kernel and those, us: 32 x 4096 x 14336 32.4 / 26.5, 24 x 2048 x 7168 13.5 / 12.1, 20 x 320 x 9600 13.4 / 10.3,
+    // 32 x 1024 x 14336 24.3 / 14.0, 17 x 64 x 14336 17.4 / 10.1; 32 x 1024 x 4096 8.8 / 9.0, 32 x 7168 x 2048 9.9 / 11.7, 17 x 8192 x 6400 24.2 / 25.9,
+    // 20 x 14336 x 8192 46.6 / 53.3; 16 x 4096 x 14336 26.0 / 25.9, 16 x 2048 x 7168 11.4 / 11.8)
+    if (M <= kFewRowsM) return M <= 16 || K < 6144 || N > 4096 || batch > 1 || !parts_or_whole;
     return M <= kSkinnyMaxM && (!parts_or_whole || (K <= 64 && M * N * batch <= 1 << 19) || (M <= 64 && M * K <= 36000 && N * batch <= 4096));
 }
 

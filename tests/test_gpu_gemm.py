@@ -644,3 +644,16 @@ def test_every_tile_form_stores_its_rows(layout, shape, dtype):
         rows = buf[off:off + M * ldc].reshape(M, ldc)
         assert bool(((rows[:, :N].double() - want).abs() <= half_ulp * 1.01 * want.abs() + (4 * math.sqrt(K) + 16) * 2.0 ** -24).all()), (off, lda_)
         assert bool((rows[:, N:] == 7).all()) and bool((buf[:off] == 7).all()) and bool((buf[off + M * ldc:] == 7).all()), (off, lda_)
+
+
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])
+@pytest.mark.parametrize("M,N,K", [(16, 328, 6144), (17, 328, 6080), (17, 328, 6144), (17, 64, 9600), (24, 8, 6208), (31, 1032, 14336), (32, 4096, 6144), (32, 4104, 6144)])
+def test_few_rows_of_a_long_contraction(M, N, K, dtype):
+    """On both sides of where tiles in parts take over from the kernel of a few rows.  Bar: half a 16-bit ulp of the result, plus fp32 sums."""
+    x, y = torch.randn(M, K, device="cuda").to(dtype), (torch.randn(N, K, device="cuda") / math.sqrt(K)).to(dtype)
+    add = torch.randn(N, device="cuda").to(dtype)
+    half_ulp = {torch.bfloat16: 2.0 ** -8, torch.float16: 2.0 ** -11}[dtype]
+    for bias in (None, add):
+        want = x.double() @ y.double().T + (0 if bias is None else bias.double())
+        got = capi.gemm(x, y, bias).double()
+        assert bool(((got - want).abs() <= half_ulp * 1.01 * want.abs() + (4 * math.sqrt(K) + 16) * 2.0 ** -24).all())
