@@ -20,6 +20,7 @@
 #include "core/device_context.h"
 #include "core/device_math.h"
 #include "core/status.h"
+#include "kernels/rms_norm_few.h"
 #include "kernels/swiglu_math.h"
 
 namespace paras {
@@ -930,7 +931,6 @@ __global__ __launch_bounds__(256, 4) void rms_norm_bwd_small(
 // V == 1: rows that are not whole aligned 16-byte pieces.  The columns of a group are one 128-byte line of a row (V == 1 and 16 bits:
 // 64 bytes), so a wave reads 8 rows (V == 1: two) at once; threads add every RL-th row, and the sums meet in a fixed order: lanes of a
 // wave by exchanges, waves in LDS.
-constexpr long kFewMax = 16384;
 template <typename T, int V, int P, bool kWaveRows>
 __global__ __launch_bounds__(1024) void rms_norm_bwd_few(
     const typename Elem<T>::store_t* __restrict__ go, const typename Elem<T>::store_t* __restrict__ x,
@@ -1193,30 +1193,6 @@ int launch_fwd(const void* x, const void* w, void* out, float* rstd, long rows, 
     return PARAS_OK;
 }
 
-// Up to how many rows dx and the column sums are one launch (rms_norm_bwd_few): where that stops being faster than the kernels that
-// read g and x once.  us, those kernels and this one (bf16): 64 columns 787 rows 5.4 and 5.3, 1500 5.9 and 8.1; 512 columns 1500 rows 8.8 and
-// 8.3, 3000 9.8 and 15.6; 1024 columns 33 rows 10.8 and 3.2, 1500 15.2 and 10.0, 2500 16.0 and 15.2; 4096 columns 77 rows 16.5 and 3.4, 2000
-// 20.1 and 16.8; 8192 columns 2000 rows 31.6 and 30.2, 2500 32.6 and 39.7; 14656 columns 184 rows 62.2 and 9.8.  Rows that are not whole vectors:
-// bf16 257 columns 1500 rows 9.6 and 9.8; 4001 columns 2000 rows 29.8 and 22.6; fp32 777 columns 1500 rows 14.1 and 12.9, 2000 15.4 and 15.7.
-// Where the other way is three kernels at any size (fp64; fp32 beyond 8192 columns), whole vectors: fp32 5500 x 12160 357 and 253, fp64
-// 5500 x 1000 49 and 43, 5500 x 4096 205 and 177.
-template <typename T>
-long few_rows(bool whole, long H) {
-    constexpr bool k16 = sizeof(typename Elem<T>::store_t) == 2, k64 = sizeof(typename Elem<T>::store_t) == 8;
-    if (!whole)            return H <= 700 || k64 ? 1000 : k16 ? 2000 : 1500;
-    if (k16)               return H <= 128 ? 700 : H <= 512 ? 1500 : 2000;
-    return k64 || H > 8192 ? 5500 : 2000;
-}
-template <typename T>
-bool takes_few(const void* go, const void* x, const void* w, const void* gx, long rows, long H, bool* whole) {
-    *whole = H % Elem<T>::kVec == 0 && ((reinterpret_cast<uintptr_t>(go) | reinterpret_cast<uintptr_t>(x) | reinterpret_cast<uintptr_t>(w) |
-                                         reinterpret_cast<uintptr_t>(gx)) & 15) == 0;
-    if (H > kFewMax || rows > few_rows<T>(*whole, H)) return false;
-    // (its column sums read g and x while other workgroups write dx: not in place)
-    const auto lo = reinterpret_cast<uintptr_t>(gx), size = static_cast<uintptr_t>(rows * H) * sizeof(typename Elem<T>::store_t);
-    auto apart = [&](const void* p) { const auto at = reinterpret_cast<uintptr_t>(p); return at + size <= lo || lo + size <= at; };
-    return apart(go) && apart(x);
-}
 template <typename T>
 int launch_few(const void* go, const void* x, const void* w, const float* rstd, void* gx, void* gw, long rows, long H, bool whole, hipStream_t s) {
     using S = typename Elem<T>::store_t;
@@ -1259,7 +1235,7 @@ int launch_bwd(const void* go, const void* x, const void* w, const float* rstd, 
                void* gw, void* workspace, long rows, long H, hipStream_t s) {
     using S = typename Elem<T>::store_t;
     bool whole = false;
-    if (takes_few<T>(go, x, w, gx, rows, H, &whole)) return launch_few<T>(go, x, w, rstd, gx, gw, rows, H, whole, s);
+    if (takes_few(static_cast<int>(sizeof(S)), go, x, w, rstd, gx, gw, rows, H, &whole)) return launch_few<T>(go, x, w, rstd, gx, gw, rows, H, whole, s);
     long slabs = (rows + kDwSlabRows - 1) / kDwSlabRows;
     PARAS_REQUIRE(slabs <= 0x7fffffffL, "paras_rms_norm_bwd: too many rows");
     if constexpr (sizeof(S) == 2) {

@@ -280,6 +280,26 @@ def test_rms_norm_backward_in_place_and_odd_rows(rows, H):
         assert torch.equal(a[~a.isnan()].view(torch.int16), b[~b.isnan()].view(torch.int16))
 
 
+@pytest.mark.parametrize("dtype", EXACT)
+@pytest.mark.parametrize("rows,H,over", [(300, 264, "w"), (300, 1000, "w"), (700, 1024, "w"), (40, 4001, "w"), (1, 4096, "go"), (1, 1000, "x"), (1, 4096, "w")])
+def test_rms_norm_backward_writes_the_weight_gradient_over_an_input(rows, H, over, dtype):
+    """w is read in a launch before the one that writes dw; with one row so are grad_out and x."""
+    torch.manual_seed(rows + H)
+    x, w, go = torch.randn(rows, H).to(dtype), (1 + 0.1 * torch.randn(H)).to(dtype), torch.randn(rows, H).to(dtype)
+    _, rstd = O.rms_norm(x, w, 1e-6)
+    wgx, wgw = O.rms_norm_backward(go, x, w, rstd)
+    t = {"go": dev(go), "x": dev(x), "w": dev(w)}
+    rd, gx = dev(rstd), torch.empty(rows, H, dtype=dtype, device="cuda")
+    ws = torch.empty(capi.lib().paras_rms_norm_bwd_workspace(rows, H), dtype=torch.uint8, device="cuda")
+    capi.check(capi.lib().paras_rms_norm_bwd(t["go"].data_ptr(), t["x"].data_ptr(), t["w"].data_ptr(), rd.data_ptr(), gx.data_ptr(), t[over].data_ptr(), ws.data_ptr(), rows, H,
+                                             capi.DT[dtype], torch.cuda.current_stream().cuda_stream))
+    assert_bit_exact(gx, wgx, "grad_input")
+    if dtype == torch.float32:
+        assert torch.allclose(t[over].reshape(-1).cpu(), wgw, rtol=1e-6, atol=1e-6)   # slab-wise column sums
+    else:
+        assert_bit_exact(t[over].reshape(-1), wgw, "grad_weight")
+
+
 def test_rms_norm_backward_general_path_with_more_than_a_million_rows():
     """fp32 takes the three-kernel path, whose partial column sums are laid out one slab of 16 rows
     per workgroup along grid x: more than 65535 slabs (1,048,560 rows) must work."""
