@@ -52,3 +52,21 @@ def test_results_that_share_memory_with_anything_else_are_not_one_launch(takes, 
 @pytest.mark.parametrize("elem", [2, 4, 8])
 def test_inputs_may_share_memory(takes, elem):
     assert takes(elem, 1 << 30, 1 << 30, 1 << 30, 1 << 30, 2 << 30, 3 << 30, 40, 264) == 2
+
+
+# (element size, rows, columns, us of the kernels that read g and x once, us of one launch)
+MEASURED = [(2, 400, 8, 5.2, 4.4), (2, 600, 8, 5.3, 5.8), (2, 700, 64, 5.3, 5.3), (2, 1000, 64, 5.4, 6.2), (2, 400, 72, 5.3, 4.2), (2, 600, 72, 5.3, 5.6), (2, 600, 136, 6.1, 5.5), (2, 700, 136, 6.2, 6.7),
+            (2, 1000, 136, 6.3, 9.3), (2, 1500, 136, 6.7, 11.8), (2, 1000, 192, 6.1, 6.2), (2, 1250, 192, 6.5, 7.4), (2, 600, 200, 6.1, 5.7), (2, 750, 200, 6.2, 7.4), (2, 1000, 256, 6.5, 6.3),
+            (2, 1500, 256, 6.8, 8.2), (2, 900, 264, 7.8, 7.6), (2, 1000, 264, 8.0, 8.9), (2, 1250, 384, 8.9, 7.7), (2, 1500, 360, 9.3, 10.7), (2, 1500, 488, 9.6, 10.8), (2, 1750, 584, 15.7, 14.8),
+            (2, 2000, 584, 15.8, 18.5), (2, 2000, 632, 15.9, 14.1), (2, 2000, 1024, 15.4, 12.9), (2, 800, 33, 7.3, 6.6), (2, 1000, 65, 8.0, 9.4), (2, 1000, 385, 9.1, 8.1), (2, 2000, 2001, 22.4, 15.4),
+            (4, 1500, 36, 8.0, 7.2), (4, 2000, 36, 8.3, 10.2), (4, 2000, 64, 8.2, 6.7), (4, 1250, 132, 8.4, 7.2), (4, 1500, 164, 9.1, 10.0), (4, 1800, 292, 11.9, 11.0), (4, 2000, 292, 12.2, 12.8),
+            (4, 2000, 516, 13.6, 13.3), (4, 2000, 1000, 16.2, 14.4), (4, 5500, 8196, 236.6, 186.2), (4, 800, 33, 7.4, 7.1), (4, 1000, 33, 7.6, 8.6), (4, 1000, 129, 7.9, 7.4), (4, 1500, 777, 14.0, 12.8),
+            (8, 1500, 34, 8.3, 5.6), (8, 2000, 34, 8.7, 11.0), (8, 2000, 64, 8.7, 7.0), (8, 4000, 64, 12.9, 14.5), (8, 2500, 128, 12.2, 13.2), (8, 2000, 130, 11.7, 12.6), (8, 4000, 256, 16.3, 20.4),
+            (8, 3000, 448, 17.2, 15.4), (8, 5500, 512, 26.2, 30.8), (8, 2500, 642, 19.2, 19.9), (8, 5500, 672, 34.5, 29.7), (8, 5500, 1026, 53.2, 48.7), (8, 5500, 2000, 100.8, 61.9), (8, 500, 193, 7.9, 7.1),
+            (8, 1000, 193, 10.0, 13.5), (8, 1000, 769, 14.5, 15.0), (8, 1000, 2001, 21.7, 17.2)]
+
+
+@pytest.mark.parametrize("elem,rows,H,several,one", MEASURED)
+def test_one_launch_where_that_was_measured_to_be_no_slower(takes, elem, rows, H, several, one):
+    taken = takes(elem, *((i + 1) << 32 for i in range(6)), rows, H) != 0
+    assert (one if taken else several) <= 1.02 * min(several, one)
