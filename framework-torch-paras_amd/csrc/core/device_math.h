@@ -159,6 +159,14 @@ __device__ __forceinline__ void lds_barrier() {
     __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "workgroup", "local");
 }
 
+// What the lanes of one wave hand each other through LDS, between the writes and the reads.  Hardware keeps a wave's LDS accesses in order; this keeps the
+// compiler from moving a lane's read ahead of its own writes where it sees that their addresses differ.  No instruction.
+__device__ __forceinline__ void lds_exchange_in_wave() {
+    __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront", "local");
+    __builtin_amdgcn_wave_barrier();
+    __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront", "local");
+}
+
 // ---- 16-byte global access ---------------------------------------------------
 __device__ __forceinline__ u32x4 load16(const void* p) {
     return *reinterpret_cast<const u32x4*>(p);

@@ -364,6 +364,7 @@ __device__ __forceinline__ void store_rows(lds_u16* out, std::uint16_t* dst, lon
     constexpr int kAll = 16 * MI * Out::kChunks, kTurns = (kAll + 63) / 64;
     constexpr int kAhead = kTurns % 8 == 0 ? 8 : kTurns % 7 == 0 ? 7 : kTurns % 6 == 0 ? 6 : kTurns % 5 == 0 ? 5 : kTurns % 4 == 0 ? 4 : 1;
     const int lane = threadIdx.x & 63;
+    lds_exchange_in_wave();
     if (wide && !nan_here && rows >= 16 * MI && cols >= 16 * NJ) {
 #pragma unroll 1
         for (int t = 0; t < kTurns; t += kAhead) {

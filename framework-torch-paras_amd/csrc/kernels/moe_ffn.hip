@@ -423,12 +423,14 @@ __global__ __launch_bounds__(flex::kThreads, 1) void grouped_gemm_direct_kernel(
         const unsigned long long lanes_below = (1ull << lane) - 1ull;
         unsigned queued = 0;      // uniform
         auto work_off = [&]() __attribute__((always_inline)) {
+            lds_exchange_in_wave();
             for (unsigned idx = lane; idx < 4 * queued; idx += 64) {
                 const unsigned e = idx >> 2, r = idx & 3, where = q.where[e];
                 const float a0 = reinterpret_cast<const float*>(&q.gate[e])[r];
                 const float a1 = reinterpret_cast<const float*>(&q.up[e])[r];
                 out[where + r] = swiglu_from_acc<T>(a0, a1);
             }
+            lds_exchange_in_wave();
             queued = 0;
         };
         const long rows_left = row_end - row0 - wm * 16 * MI, cols_left = p.N - n0 - wn * 64;
