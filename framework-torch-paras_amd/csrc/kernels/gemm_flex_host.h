@@ -6,6 +6,8 @@
 #include <cstddef>
 #include <cstdint>
 
+#include "kernels/gemm_flex_plan.h"
+
 namespace paras {
 namespace flex {
 
@@ -21,13 +23,6 @@ struct Problem {
     bool a_rows, b_rows;        // the operand is contiguous along its rows, not along the contraction (a_rows only with b_rows)
     bool bf16;
 };
-constexpr int kTile128x128 = 4;      // the index of its two-stage form in the tile table
-struct Plan {
-    int  tile = 0;              // index into the tile table
-    int  splits = 1;            // parts of the contraction
-    long k_per_split = 0;
-};
-
 bool takes(const Problem& q);                       // sizes and alignments the kernel can read
 Plan plan(const Problem& q, bool may_split);
 inline size_t workspace(const Problem& q, const Plan& p) {

@@ -604,7 +604,7 @@ def test_rows_of_result_and_addend_beyond_31_bits(K, a_rows, b_rows, dtype):
     assert bool((c[:, N:] == 7).all())
 
 
-# one problem for each tile form and layout, edges cut short in both directions (N % 4 == 0; K % 64 == 8, 16 ... or few steps)
+# problems of x W^T (0), dy W (1) and dy^T x (2) that reach each tile form, whole (test_gemm_forms_cpu.py); edges cut short in both directions (N % 4 == 0; K % 64 == 8, 16 ... or few steps)
 TILES = [(0, (6437, 2104, 528)), (0, (2483, 4712, 576)), (0, (7082, 792, 536)), (0, (6536, 536, 528)), (0, (7119, 392, 64)), (0, (6977, 400, 136)), (0, (683, 5488, 64)),
          (0, (5661, 144, 200)), (0, (5700, 136, 64)), (0, (33, 72, 64)), (0, (36, 72, 208)), (0, (130, 5528, 64)), (0, (2709, 4520, 520)), (0, (2389, 4344, 520)), (0, (1189, 7000, 528)),
          (1, (1645, 7336, 520)), (1, (7683, 1160, 520)), (1, (1185, 5008, 528)), (1, (6805, 520, 528)), (1, (455, 6200, 64)), (1, (470, 6232, 136)), (1, (662, 5464, 64)),
@@ -644,6 +644,46 @@ def test_every_tile_form_stores_its_rows(layout, shape, dtype):
         rows = buf[off:off + M * ldc].reshape(M, ldc)
         assert bool(((rows[:, :N].double() - want).abs() <= half_ulp * 1.01 * want.abs() + (4 * math.sqrt(K) + 16) * 2.0 ** -24).all()), (off, lda_)
         assert bool((rows[:, N:] == 7).all()) and bool((buf[:off] == 7).all()) and bool((buf[off + M * ldc:] == 7).all()), (off, lda_)
+
+
+# problems whose contraction comes in parts, the last of them short, for each tile form that is split (test_gemm_forms_cpu.py); edges cut short in both directions
+PARTS = [(0, (193, 6504, 10216)), (0, (139, 4464, 14440)), (0, (2050, 136, 12320)), (0, (1889, 72, 14408)), (0, (193, 2992, 10280)), (0, (1367, 72, 13496)), (0, (36, 2712, 9336)),
+         (0, (34, 1232, 9640)), (0, (33, 136, 5272)), (0, (33, 176, 6760)), (0, (620, 72, 7016)), (0, (34, 72, 1048)), (0, (66, 1832, 6568)), (0, (65, 1840, 13960)),
+         (0, (65, 280, 6696)), (0, (199, 2952, 11560)), (0, (131, 4112, 10912)), (1, (195, 2768, 13408)), (1, (131, 5424, 7728)), (1, (2063, 136, 12296)), (1, (2712, 72, 9496)),
+         (1, (1833, 72, 6176)), (1, (34, 2712, 5432)), (1, (584, 72, 5488)), (1, (34, 272, 5032)), (1, (33, 272, 6424)), (1, (292, 72, 4872)), (1, (33, 72, 776)), (1, (898, 72, 7824)),
+         (1, (1370, 72, 10488)), (1, (68, 264, 6760)), (2, (208, 5384, 7867)), (2, (72, 5552, 14555)), (2, (2744, 136, 8331)), (2, (136, 1848, 6267)), (2, (80, 5656, 10259)),
+         (2, (2704, 72, 4259)), (2, (40, 2864, 7179)), (2, (72, 392, 13360)), (2, (40, 184, 5251)), (2, (40, 216, 6819)), (2, (72, 584, 4664)), (2, (40, 72, 1032)),
+         (2, (152, 1840, 8211))]
+
+
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])
+@pytest.mark.parametrize("layout,shape", PARTS)
+def test_every_tile_form_in_parts(layout, shape, dtype):
+    """fp32 parts in a workspace (not a byte past it), added and narrowed into rows that lie apart, plain and with an addend; two products in one call.
+    Bar: half a 16-bit ulp of the result, plus fp32 sums."""
+    M, N, K = shape
+    g = torch.Generator(device="cuda").manual_seed(M + N + K)
+    half_ulp = {torch.bfloat16: 2.0 ** -8, torch.float16: 2.0 ** -11}[dtype]
+    for batch, ldc, alpha, ld_add in ((1, N + 16, 1.0, None), (1, N + 9, 0.5, N + 5), (2, N + 8, 1.0, 0)):
+        x = torch.randn(batch, M, K, generator=g, device="cuda").to(dtype)
+        y = (torch.randn(batch, N, K, generator=g, device="cuda") / math.sqrt(K)).to(dtype)
+        a, b = x.transpose(1, 2).contiguous() if layout == 2 else x, y.transpose(1, 2).contiguous() if layout else y
+        add = torch.randn(M, N + 5, generator=g, device="cuda").to(dtype)
+        buf = torch.full((batch, M, ldc), 7.0, device="cuda", dtype=dtype)
+        problem = capi.GemmArgs(a.data_ptr(), b.data_ptr(), None if ld_add is None else add.data_ptr(), buf.data_ptr(), M, N, K, a.stride(1), b.stride(1), ldc, ld_add or 0, batch,
+                                a.stride(0), b.stride(0), buf.stride(0), 0, alpha, 2.0, capi.DT[dtype], int(layout == 2), int(layout > 0))
+        n = capi.lib().paras_gemm_workspace(C.byref(problem))
+        if batch == 1:
+            assert n >= 2 * 4 * M * N and n % (4 * M * N) == 0
+        ws = torch.full((n // 4 + 64,), 7.0, device="cuda")
+        capi.check(capi.lib().paras_gemm(C.byref(problem), ws.data_ptr(), n, torch.cuda.current_stream().cuda_stream))
+        assert bool((ws[n // 4:] == 7).all())
+        for i in range(batch):
+            want = alpha * (x[i].double() @ y[i].double().T)
+            if ld_add is not None:
+                want = want + 2.0 * (add[:1, :N] if ld_add == 0 else add[:, :N]).double()
+            assert bool(((buf[i, :, :N].double() - want).abs() <= half_ulp * 1.01 * want.abs() + (4 * math.sqrt(K) + 16) * 2.0 ** -24).all()), (batch, ld_add)
+        assert bool((buf[:, :, N:] == 7).all())
 
 
 @pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])
