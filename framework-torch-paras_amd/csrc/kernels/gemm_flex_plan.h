@@ -44,8 +44,8 @@ constexpr int kCus = 256;
 //
 // The search is on the way of every call, and a small product's launch costs a few us: the forms' constants are the compiler's
 // (no division by a variable but two per number of parts), and forms and numbers of parts are left out whose least possible time is no
-// better than one found.  The same plan as the search through all of them; host time of that and of this: 48 x 1024 x 1024 1.4 and 0.17 us,
-// 128 x 2048 x 2048 2.0 and 0.41, 1024 x 1024 x 4096 2.1 and 0.19, 8192^3 0.37 and 0.05.
+// better than one found.  The same plan as the search through all of them; host time of that and of this: 48 x 1024 x 1024 0.50 and 0.18 us,
+// 128 x 2048 x 2048 0.68 and 0.36, 1024 x 1024 x 4096 0.67 and 0.25, 8192^3 0.15 and 0.08; 900 problems of 33 to 8192 rows 0.20 in the mean.
 struct Search {
     int M, N, batch, k_tiles;
     bool may_split;
@@ -64,6 +64,7 @@ struct Search {
     }
     template <int t, bool record> void consider() {
         constexpr Tile tl = kTiles[t];
+        if (tl.m >= 128 && M <= 64 && batch == 1 && k_tiles <= 256) return;       // (half as many rows: not behind)
         constexpr int slots = kCus * tl.per_cu;
         constexpr double area = tl.m * tl.n / 65536.0, whole = area * (tl.per_cu > 1 ? 0.475 : 1.0) * 10.06, in_parts = area * (tl.per_cu > 1 ? 0.475 : 1.0) * 5.67;
         const double each = tl.step / tl.per_cu * k_step, lat = tl.lat * k_lat;
@@ -76,11 +77,11 @@ struct Search {
             want(i, wanted);
             const int n_parts = parts[i], turns = static_cast<unsigned>(per[i] + (tl.stages - 1)) / tl.stages * tl.stages;
             const double finish = n_parts > 1 ? 2.5 + mn * n_parts * 1.574e-6 : 0.0;
-            if (least + finish >= found) break;
-            if ((turns * lat + kStart) * kBelow + finish >= found) continue;
+            const double stores = n_parts > 1 ? in_parts : whole;
+            if (least + finish >= found || (kStart + in_parts) * kBelow + finish >= found) break;       // (more parts are more to add)
+            if ((turns * (each > lat ? each : lat) + kStart + stores) * kBelow + finish >= found) continue;      // a workgroup's own time
             const int wgs = tiles * n_parts, full = static_cast<unsigned>(wgs) / slots;
             const int rest = static_cast<unsigned>(wgs - full * slots + kCus - 1) / kCus;
-            const double stores = n_parts > 1 ? in_parts : whole;
             auto round = [&](double n) {
                 const double c = each * n;
                 return turns * (c > lat ? c : lat) + kStart + stores * n;
