@@ -14,9 +14,9 @@
 // contraction dim, which is exactly the 8-element-per-lane operand layout of
 // v_mfma_f32_32x32x16, so neither operand needs a transpose.
 //
-// Tiling: 32 to 256 routed rows x 128 or 256 weight rows (gate and up rows of the same columns for GEMM 1), k-tile 64, four
+// Tiling: 32 to 256 routed rows x 64 to 256 weight rows (gate and up rows of the same columns for GEMM 1), k-tile 64, four
 // waves on v_mfma_f32_16x16x32 with loads straight to LDS (gemm_flex.h; grouped_tile_kernel, grouped_gemm_direct_kernel), the
-// tile chosen by an estimate (grouped_form); few rows per expert on kernels that stream the weights (grouped_few_rows_kernel); an x
+// tile chosen by an estimate (grouped_tiles); few rows per expert on kernels that stream the weights (grouped_few_rows_kernel); an x
 // beyond a 32-bit byte offset on register-staged 256-row tiles (gemm_tile.h; grouped_gemm_kernel).  Rows of one
 // expert are contiguous in the routed order; m-tiles never straddle experts (the grid is sized for the
 // worst case and surplus workgroups exit).

@@ -464,7 +464,7 @@ TILE_SHAPES = [(1843, 70, 6, 192, 256), (2055, 32, 4, 192, 192), (1188, 70, 6, 1
 # (with those, every form of grouped_tiles that the gate-up and that the down product have)
 FURTHER_TILE_SHAPES = [(43, 70, 6, 192, 384), (63, 8, 2, 64, 1024), (288, 8, 2, 64, 1152), (577, 32, 4, 576, 64), (587, 4, 1, 832, 1216), (828, 4, 1, 1344, 1472), (858, 4, 1, 1536, 448),
                        (1299, 4, 1, 1536, 576), (1828, 32, 4, 960, 768), (2548, 4, 1, 1472, 1344), (2604, 32, 4, 960, 512), (2757, 8, 2, 960, 1024), (46, 70, 6, 896, 192), (287, 8, 2, 64, 1408),
-                       (1109, 32, 4, 1088, 960), (1967, 8, 2, 1408, 960)]
+                       (1109, 32, 4, 1088, 960), (1967, 8, 2, 1408, 960), (603, 16, 2, 64, 1664)]
 
 
 @pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])
