@@ -42,7 +42,7 @@ struct DenseParams {
                                 // result (row of a, row of b) belongs at c[row of b][row of a], and the addend likewise
 };
 
-// ---- up to 32 rows: the decode-time projections, bound by streaming the weights once.  A workgroup owns 16 NBG
+// ---- up to 32 rows (from 17 on over contractions of less than 6144 or more than 4096 weight rows: few_rows_up_to): the decode-time projections, bound by streaming the weights once.  A workgroup owns 16 NBG
 // weight rows and its eight waves split the contraction (stream_rows.h); 8 XQ activation rows at most.
 using stream::Mma16;
 
@@ -140,7 +140,7 @@ __global__ __launch_bounds__(stream::kThreads, 4) void stream_gemm_nt_kernel(con
 // a 16x16 result holds activation row l%16 and weight rows 4*(l/16) .. +3.
 constexpr int kSkinnyWaves = 8;
 constexpr int kSkinnyMaxM = 128;
-constexpr int kFewRowsM = 32;            // the staged tiles take over from here (few_rows_up_to)
+constexpr int kFewRowsM = 32;            // the staged tiles take over from here, and from 17 rows on over long contractions (few_rows_up_to)
 
 template <typename T, int MB, int NB>   // MB = 16-row blocks of activations, NB = 16-row blocks of weights per workgroup
 __global__ __launch_bounds__(kSkinnyWaves * 64) void skinny_gemm_nt_kernel(const DenseParams p) {
@@ -417,7 +417,7 @@ __global__ __launch_bounds__(256) void skinny_splitk_finish_kernel(const DensePa
 // Few rows but many columns (a vocabulary projection, a fused gate-up projection at M = 64 ... 128):
 // from about 200 tiles of 128 x 128 the tile kernel streams the weights faster than the few-row
 // kernels do (M = 128, N = 128256, K = 4096: 267 against 649 us; N = 28672: 75 against 106 us; at
-// N = 6144 the few-row kernels win, 47 against 67 us).  Up to 32 rows the few-row kernels stay.
+// N = 6144 the few-row kernels win, 47 against 67 us).  Up to 32 rows few_rows_up_to decides alone.
 bool few_rows_by_tiles(long M, long N, long batch) {
     return M > 32 && M <= kSkinnyMaxM && (N + gemm::kBN - 1) / gemm::kBN * batch >= 192;
 }

@@ -14,9 +14,9 @@ struct Plan {
     long k_per_split = 0;
 };
 
-// Per tile form: rows, columns, stages, workgroups a CU holds at once, and in us the time of one tile of 64
-// contraction steps on a CU that is full (`step`) and at least, on a CU with fewer workgroups (`lat`: a
-// barrier and the way from L2).
+// Per tile form: rows, columns, stages, workgroups a CU holds at once, and what a fit makes of one tile of 64
+// contraction steps, in us: on a CU that is full (`step`), and at least, on a CU with fewer workgroups (`lat`: a
+// barrier and the way from L2).  Coefficients of the estimate below, whose sum was fitted and counts; each by itself is no time or rate of the chip.
 struct Tile { int m, n, stages, per_cu; double step, lat; };
 constexpr Tile kTiles[] = {{256, 256, 2, 1, 0.827, 0.304}, {192, 256, 2, 1, 0.743, 0.052}, {192, 192, 3, 1, 0.682, 0.258}, {192, 128, 4, 1, 0.525, 0.562},
                            {128, 128, 2, 2, 0.849, 0.859}, {128, 128, 4, 1, 0.399, 0.472}, {64, 128, 2, 3, 0.916, 0.653}, {64, 128, 4, 1, 0.338, 0.230},
@@ -40,7 +40,8 @@ constexpr int kCus = 256;
 // as much per flop as a 128 x 128 one, but with 192 of them for 256 CUs a quarter of the chip idles (3000 x 4096 x 4096 85.7 us, with 256 tiles of
 // 192 x 256 78.3); a small problem has few workgroups per CU, and then more
 // stages stand in for the other workgroups' loads (821 x 1024 x 3584 64 x 64: two stages in four parts 21 us, four stages 14.5 whole);
-// what is still too few tiles is cut up along the contraction (1500 x 4096 x 14336: 192 x 128 whole 160 us, 256 x 224 in two parts 147).
+// what is still too few tiles is cut up along the contraction (1500 x 4096 x 14336, with the second
+// kernel: 192 x 256 in two parts 141 us, 256 x 224 159; 192 x 128 whole 164).
 //
 // The search is on the way of every call, and a small product's launch costs a few us: the forms' constants are the compiler's
 // (no division by a variable but two per number of parts), and forms and numbers of parts are left out whose least possible time is no

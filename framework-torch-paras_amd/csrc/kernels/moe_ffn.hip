@@ -208,7 +208,7 @@ __device__ __forceinline__ void static_for(F&& f) {
 // of the four tile stages once the contraction is done (the first half is for the wave's rows on their way out).
 struct SwigluQueue {
     static constexpr unsigned kEntries = 448;
-    unsigned where[kEntries];       // (row in the tile) << 16 | column in the column unit
+    unsigned where[kEntries];       // the first of the four in the wave's rows (RowsOut)
     flex::float4v gate[kEntries], up[kEntries];
 };
 __device__ __forceinline__ unsigned scalar_of(unsigned v) { return static_cast<unsigned>(__builtin_amdgcn_readfirstlane(static_cast<int>(v))); }
@@ -302,9 +302,9 @@ template <typename Tiles> __device__ __forceinline__ TileOf find_tile(const FfnG
 // The same on the four-wave 256 x 256 tile of v_mfma_f32_16x16x32 whose loads go straight to LDS (gemm_flex.h): what the
 // layer runs on when the experts are big enough for 256-row tiles.  Tile coordinates and the search for the
 // m-tile's expert as above; the routed rows are gathered by the addresses the lanes fetch from.  A lane of accumulator
-// block (i, j) holds row i*16 + lane%16 and columns 4*(lane/16) .. + 3 of column block j (group j / 4, columns
-// wn*64 + (j % 4)*16 of it), so gate and up of one output sit in blocks j and j + 4 of the same lane and an output row
-// gets 8-byte stores.  Bound by the matrix cores' power and the LDS reads.
+// block (i, j) holds row i*16 + lane%16 and columns 4*(lane/16) .. + 3 of column block j; of the gate-up product that is group j / 4
+// (TwoGroups), columns wn*64 + (j % 4)*16 of it, so gate and up of one output sit in blocks j and j + 4 of the same lane.  Results leave through LDS in
+// whole rows (RowsOut).  Bound by the matrix cores' power and the LDS reads.
 template <typename T, bool kSwiglu>
 __global__ __launch_bounds__(flex::kThreads, 1) void grouped_gemm_direct_kernel(const FfnGemmParams p) {
     using El = Elem<T>;

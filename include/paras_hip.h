@@ -359,9 +359,10 @@ PARAS_API int paras_moe_ffn(const void* x, const void* w_gate, const void* w_up,
 /* (a bias) over the M rows.  All four float dtypes.  bf16 / f16 with K a       */
 /* multiple of 8, 16-byte aligned operands and leading dimensions and batch    */
 /* strides that are multiples of 8 run on the MFMA kernels (fp32 accumulation, */
-/* one rounding; up to 32 rows, 128 by paras_gemm_nt, on kernels that stream    */
-/* the weights, K a multiple of 64); fp32 tensors on the fp32 MFMA kernel (full */
-/* fp32 multiplies, any K and alignment); everything else -- fp64 tensors,     */
+/* one rounding; up to 16 rows, 32 where K < 6144 or N > 4096, 128 by          */
+/* paras_gemm_nt, on kernels that stream the weights, K a multiple of 64);     */
+/* fp32 tensors on the fp32 MFMA kernel (full fp32 multiplies, any K and       */
+/* alignment); everything else -- fp64 tensors,                                */
 /* 16-bit ones with other K or alignments -- on a general kernel (fp32         */
 /* accumulation, fp64 for fp64 tensors), so no product needs a host path.      */
 /* ------------------------------------------------------------------------- */
