@@ -228,10 +228,12 @@ def test_rms_norm_backward_team_workgroups(shape, dtype):
 
 # piece counts at the edges of a wave, two waves, a workgroup and two of them, whole vectors and not; rows on both sides of each limit
 FEW = {torch.bfloat16: [(1, 8), (3, 512), (700, 128), (701, 128), (1500, 512), (1501, 512), (9, 520), (65, 1024), (8, 1032), (2000, 1032), (2001, 1032),
-                        (5, 8192), (7, 8200), (2, 16384), (2001, 8200), (3, 1), (257, 127), (1000, 129), (1001, 129), (4, 2049), (6, 8193), (2, 16383)],
+                        (5, 8192), (7, 8200), (2, 16384), (2001, 8200), (3, 1), (257, 127), (1000, 129), (1001, 129), (4, 2049), (6, 8193), (2, 16383),
+                        (450, 72), (451, 72), (600, 136), (601, 136), (1000, 256), (1001, 256), (900, 264), (901, 264), (1250, 512), (1251, 512), (1750, 584), (1751, 584), (800, 33), (801, 33)],
        torch.float32: [(1, 4), (5, 256), (33, 260), (130, 512), (9, 516), (33, 1000), (2000, 520), (2001, 520), (3, 4096), (4, 4100), (7, 8196), (2, 16384),
-                       (2001, 8196), (3, 1), (1000, 127), (1001, 127), (5, 2049), (3, 16383), (1500, 701), (1501, 701)],
-       torch.float64: [(1, 2), (17, 128), (9, 130), (5, 258), (3, 2050), (4, 4098), (2, 16384), (5500, 64), (5501, 64), (33, 129), (1001, 129), (2, 16383)]}
+                       (2001, 8196), (3, 1), (1000, 127), (1001, 127), (5, 2049), (3, 16383), (1500, 701), (1501, 701), (1700, 36), (1701, 36), (1350, 132), (1351, 132), (1800, 260), (1801, 260), (800, 65), (801, 65)],
+       torch.float64: [(1, 2), (17, 128), (9, 130), (5, 258), (3, 2050), (4, 4098), (2, 16384), (5500, 64), (5501, 64), (33, 129), (1001, 129), (2, 16383),
+                       (1500, 34), (1501, 34), (2200, 128), (2201, 128), (3000, 192), (3001, 192), (2000, 386), (2001, 386), (550, 129), (551, 129), (700, 257), (701, 257), (900, 641), (901, 641)]}
 
 
 @pytest.mark.parametrize("dtype,shape", [(d, s) for d, ss in FEW.items() for s in ss])
